@@ -1229,9 +1229,10 @@ int ffk_linear_ws_try(const ffk_linear_desc* d, hipStream_t st, int* status) {
     if (d->variant == FFK_LINEAR_STAGED) return 0;
     bool chan_major = false, v_tiles = false, tails = false;
     int mask_tile = -1;
-    // a trailing pair-bias tile (score-operand tiles of <= 4 heads) rides on the launch without a weight slot
+    // a trailing pair-bias tile (score-operand tiles of <= 4 heads) rides on the launch without a weight slot; it may be
+    // the only tile (a chunked attention computes its bias before the first slab, with the bits of the riding one)
     int n_slot_tiles = d->n_tiles, bias_tile = -1;
-    if (d->n_tiles >= 2 && d->tiles[d->n_tiles - 1].kind == FFK_TILE_BIAS) {
+    if (d->tiles[d->n_tiles - 1].kind == FFK_TILE_BIAS) {
         const ffk_tile& t = d->tiles[d->n_tiles - 1];
         auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
         if (d->K != 128 || d->a_chanmajor || d->a2 || t.ncols < 1 || t.ncols > 4 || t.bias || t.resid || t.gate || t.rowmask ||

@@ -118,6 +118,28 @@ def fits_fused(K, dtype):
     return K <= 256 and K % 32 == 0
 
 
+def pad_to_tiles(m, z, msa_mask, pair_mask, pad_s=True):
+    """m [1, s, r, c_m], z [1, r, r, c_z] and their masks, zero-padded to whole 32-row tiles along the residue axis and
+    (``pad_s``) the sequence axis; bf16 tensors whose extents are no multiples of 32, everything else as it came.
+
+    The padding is masked: no un-padded result reads it.  It exists because the fast kernels work on whole tiles: the
+    weights-stationary projections write attention operands in accumulator order for rows of whole 32-key tiles, the
+    triangle multiplication's output stage and the fused outer product want r % 8 == 0 and r % 32 == 0.  The rows added
+    (at most 31 of each axis: 13 % of the pair positions at 391 residues) cost less than the LDS-staged kernels a ragged
+    extent would take at every size measured: 8 blocks at N_seq = 125, N_res = 391 18.1 -> 10.9 ms.  fp32 runs on the
+    staged kernels at any extent, so padding would only add work there."""
+    s, r = m.shape[1], m.shape[2]
+    if m.dtype != torch.bfloat16:
+        return m, z, msa_mask, pair_mask
+    ds, dr = (round_up(s, 32) - s if pad_s else 0), round_up(r, 32) - r
+    if ds == 0 and dr == 0:
+        return m, z, msa_mask, pair_mask
+    pad = torch.nn.functional.pad
+    if dr:
+        z, pair_mask = pad(z, (0, 0, 0, dr, 0, dr)), pad(pair_mask, (0, dr, 0, dr))
+    return pad(m, (0, 0, 0, dr, 0, ds)), z, pad(msa_mask, (0, dr, 0, ds)), pair_mask
+
+
 # ------------------------------------------------------------------------- linear ----
 def linear(x2, w_pk, b_pk, N, *, act=FFK_ACT_NONE, out=None, resid=None, ln=None):
     """out[M, N] = act(LN(x2)[M, K] @ W^T + b) (+ resid).  ``w_pk`` is [>=N (padded to 128), K]."""
@@ -251,8 +273,9 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     # rows of a bias buffer the caller leaves to this function (bias_in_launch with bias_t None) end in one unused tile
     # when the projection launch writes them: with 2^n key tiles per row every query-tile row would start in the same
     # memory channel (-2 % per triangle-attention launch at N = 1024, measured three times on one box)
-    will_ride = (bias_in_launch and acc_order and C == 128 and H <= 4 and slab >= B2 and _PAIR_BIAS_RIDES
-                 and (not gate_in_out or hasattr(w_pk, "without_gate")))
+    can_ride = (bias_in_launch and acc_order and C == 128 and H <= 4 and _PAIR_BIAS_RIDES
+                and (not gate_in_out or hasattr(w_pk, "without_gate")))
+    will_ride = can_ride and slab >= B2
     bias_padded = will_ride and _BIAS_ROW_PAD and bias_t is None
     if bias_in_launch:
         ntp = NT + (1 if bias_padded else 0)
@@ -270,6 +293,12 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     # has pushed x out by the time the bias pass reads it (measured: -0.65 % block time at N = 1024).
     if rides:
         pass
+    elif can_ride and N < 1024:
+        # In slabs: the same kernel with the bias as its only tile, so that slabs change no bit of the result.  Longer rows
+        # keep the bias pass of its own, which streams x twice as fast (16 M rows at N = 4096: 0.9 against 1.9 ms).
+        _lib.fused_linear(x, w_pk, [bias_tile], M=M, K=C, a_inner=a_inner, a_so=a_so, a_si=a_si, ln=ln,
+                          w_row_off=4 * tpg * 128)
+        bias_tile = None
     elif bias_tile is not None and acc_order and C in (64, 128):
         _pair_bias_launch(bias_t, x, ln, w_pk[4 * tpg * 128:], pb_scratch, N=N, C=C, H=H, a_inner=a_inner,
                           a_so=a_so, a_si=a_si, scale=LOG2E)
@@ -473,6 +502,9 @@ def outer_product_mean(m, mask, z, out, *, s, r, C, Cz, ln, wab_pk, bab_pk, wo, 
     dt, dev = m.dtype, m.device
     es = es_of(dt)
     spad = round_up(s, vec_of(dt))
+    fused = wo_ed is not None and dt == torch.bfloat16 and Cz == 128 and r % 32 == 0 and s <= 128
+    if fused:       # the fused kernel's sequence extents; the zero sequences add nothing to a sum
+        spad = 64 if s <= 64 else 128
     ab = alloc((2, r * 32, spad), dt, dev, zero=spad != s)
     tile = make_tile(ab, bias=bab_pk, ncols=64, inner=s, s_o=32 * spad, s_i=1, s_h=r * 32 * spad, s_d=spad,
                      rowmask=mask, m_so=1, m_si=r)
@@ -485,7 +517,7 @@ def outer_product_mean(m, mask, z, out, *, s, r, C, Cz, ln, wab_pk, bab_pk, wo, 
         _lib.bgemm_nt(mt, mt, nrm, M=r, N=r, K=spad, lda=spad, ldb=spad, out_f32=True)
         return nrm
     nrm = _mask_derived(mask, ("opm_norm", s, r, spad), normaliser)
-    if wo_ed is not None and dt == torch.bfloat16 and Cz == 128 and r % 32 == 0 and spad in (64, 128):
+    if fused:
         # fused core: the [r, r, 1024] outer product never leaves the chip
         _lib.opm_fused(out, z, ab[0], ab[1], wo_ed, bo, nrm, r=r, spad=spad, eps=eps, xtail=xtail)
         return out

@@ -36,7 +36,7 @@ class _BlockRecompute(torch.autograd.Function):
     def forward(ctx, block, msa_mask, pair_mask, drops, _grad_anchor, m, z):
         ctx.block, ctx.masks, ctx.drops = block, (msa_mask, pair_mask), drops
         ctx.save_for_backward(m, z)
-        return block._core(m.contiguous(), z.contiguous(), msa_mask, pair_mask, inplace=False, drops=drops)
+        return block._core_any(m.contiguous(), z.contiguous(), msa_mask, pair_mask, inplace=False, drops=drops)
 
     @staticmethod
     def backward(ctx, dm, dz):
@@ -68,7 +68,7 @@ class Evoformer(nn.Module):
     def _core(self, m, z, msa_mask, pair_mask, inplace: bool, tails=(None, None), drops=None):
         """``tails = (m_tail, z_tail)``: int8 tails of m / z as extended residual streams (the stack's bf16 mode),
         or None for the plain stream of the reference.  ``drops``: None, or the dropout multipliers of a training-mode
-        pass (``_draw_drops``; out-of-place only)."""
+        pass (``_draw_drops``)."""
         F_.check_nonempty("Evoformer", m, z)
         mt, zt = tails
         if self.is_multimer:
@@ -76,19 +76,35 @@ class Evoformer(nn.Module):
             # pair tensor it leaves, the pair stack runs last
             z_new = z if inplace else torch.empty_like(z)
             self.communication._run(m, msa_mask, z, z_new, zt)
-            m = self.msa.inplace(m, z_new, msa_mask, mt) if inplace else self.msa.forward(m, z_new, msa_mask, mt, drops=drops)
+            m = self.msa.inplace(m, z_new, msa_mask, mt, drops=drops) if inplace else self.msa.forward(m, z_new, msa_mask, mt, drops=drops)
             self.pair.inplace([z_new], pair_mask, zt, drops=drops)
             return m, z_new
         if inplace:
-            m = self.msa.inplace(m, z, msa_mask, mt)
+            m = self.msa.inplace(m, z, msa_mask, mt, drops=drops)
             self.communication._run(m, msa_mask, z, z, zt)
-            self.pair.inplace([z], pair_mask, zt)
+            self.pair.inplace([z], pair_mask, zt, drops=drops)
             return m, z
         m = self.msa.forward(m, z, msa_mask, mt, drops=drops)
         z_new = torch.empty_like(z)
         self.communication._run(m, msa_mask, z, z_new, zt)
         self.pair.inplace([z_new], pair_mask, zt, drops=drops)
         return m, z_new
+
+    def _core_any(self, m, z, msa_mask, pair_mask, inplace: bool, drops=None):
+        """``_core`` at any extents: ragged bf16 tensors run zero-padded to whole tiles (``_fused.pad_to_tiles``)."""
+        s, r = m.shape[1], m.shape[2]
+        mp, zp, mk, pk = F_.pad_to_tiles(m, z, msa_mask, pair_mask)
+        if mp is m and zp is z:
+            return self._core(m, z, msa_mask, pair_mask, inplace, drops=drops)
+        if drops and zp is not z:
+            # multipliers of the padding rows: any will do
+            drops = {k: F.pad(v, (0, 0, 0, zp.shape[1] - r) if v.shape[1] == 1 else (0, 0, 0, 0, 0, zp.shape[1] - r))
+                     for k, v in drops.items()}
+        mp, zp = self._core(mp, zp, mk, pk, inplace=inplace or (mp is not m and zp is not z), drops=drops)
+        mp, zp = mp[:, :s, :r], zp[:, :r, :r]
+        if inplace:
+            return m.copy_(mp) if mp.data_ptr() != m.data_ptr() else m, z.copy_(zp) if zp.data_ptr() != z.data_ptr() else z
+        return mp.contiguous(), zp.contiguous()
 
     def _core_train(self, m, z, msa_mask, pair_mask, drops=None):
         """The differentiable block (evoformer.py:64-76) on the un-padded tensors: every update is out of place and
@@ -156,7 +172,7 @@ class Evoformer(nn.Module):
                 m, z = m[:, :, :r, :], z[:, :r, :r, :]
             return self._leave(*self._run_grad(m, z, msa_mask.unsqueeze(0), pair_mask.unsqueeze(0)))
         m, z = self._enter(m, z, r)
-        m, z = self._core(m, z, msa_mask.unsqueeze(0), pair_mask.unsqueeze(0), inplace=not self.first_block)
+        m, z = self._core_any(m, z, msa_mask.unsqueeze(0), pair_mask.unsqueeze(0), inplace=not self.first_block)
         return self._leave(m, z)
 
     def inplace(self, m, z, msa_mask: torch.Tensor, pair_mask: torch.Tensor, chunk_size: Optional[int] = None,
@@ -170,7 +186,7 @@ class Evoformer(nn.Module):
                 mm, zz = mm.contiguous(), zz.contiguous()
         else:
             mm, zz = self._enter(m[0], z[0], r)
-        mm, zz = self._core(mm, zz, msa_mask.unsqueeze(0), pair_mask.unsqueeze(0), inplace=True)
+        mm, zz = self._core_any(mm, zz, msa_mask.unsqueeze(0), pair_mask.unsqueeze(0), inplace=True)
         m[0], z[0] = self._leave(mm, zz)
         return m, z
 
@@ -195,8 +211,11 @@ class EvoformerStack(nn.Module):
         self.linear = Linear(c_m, c_s)
 
     def _run(self, m, z, msa_mask, pair_mask, inplace_first: bool):
-        mm, zz = m.unsqueeze(0), z.unsqueeze(0)
-        mk, pk = msa_mask.unsqueeze(0), pair_mask.unsqueeze(0)
+        F_.check_nonempty("EvoformerStack", m, z)
+        s, r = m.shape[0], m.shape[1]
+        m0, z0 = m.unsqueeze(0), z.unsqueeze(0)
+        mm, zz, mk, pk = F_.pad_to_tiles(m0, z0, msa_mask.unsqueeze(0), pair_mask.unsqueeze(0))
+        own_m, own_z = mm is not m0, zz is not z0        # padded copies may be overwritten
         tails = (None, None)
         if self.extended_residual and mm.dtype == torch.bfloat16 and mm.is_cuda:
             # zero tails: the inputs are exact bf16 values; the tails die with this call, the bf16 tensors they
@@ -207,8 +226,14 @@ class EvoformerStack(nn.Module):
             for i, b in enumerate(self.blocks):
                 if self.clear_cache_between_blocks:
                     torch.cuda.empty_cache()
-                mm, zz = b._core(mm.contiguous(), zz.contiguous(), mk, pk, inplace=(inplace_first or i > 0), tails=tails)
-        return mm.squeeze(0), zz.squeeze(0)
+                mm, zz = b._core(mm.contiguous(), zz.contiguous(), mk, pk, inplace=(inplace_first or i > 0 or (own_m and own_z)),
+                                 tails=tails)
+        mm, zz = mm.squeeze(0), zz.squeeze(0)
+        if own_m:
+            mm = m.copy_(mm[:s, :r]) if inplace_first else mm[:s, :r].contiguous()
+        if own_z:
+            zz = z.copy_(zz[:r, :r]) if inplace_first else zz[:r, :r].contiguous()
+        return mm, zz
 
     def _run_train(self, m, z, msa_mask, pair_mask):
         """The differentiable stack: plain residual stream, blocks re-run in the backward pass in groups of

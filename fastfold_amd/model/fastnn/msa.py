@@ -169,8 +169,8 @@ class MSACore(nn.Module):
         self.MSATransition._run(out, out, xtail)
         return out
 
-    def inplace(self, node, pair, node_mask, xtail=None):
-        self.MSARowAttentionWithPairBias._run(node, pair, node_mask, node, xtail)
+    def inplace(self, node, pair, node_mask, xtail=None, drops=None):
+        self.MSARowAttentionWithPairBias._run(node, pair, node_mask, node, xtail, drop=(drops or {}).get("row"))
         self.MSAColumnAttention._run(node, node_mask, node, xtail)
         self.MSATransition._run(node, node, xtail)
         return node
@@ -294,14 +294,24 @@ class ExtraMSAStack(nn.Module):
                                              last_block=(block_id == no_blocks - 1), is_multimer=is_multimer))
 
     def _run(self, m, z, msa_mask, pair_mask, inplace_first: bool):
-        mm, zz = m.unsqueeze(0).contiguous(), z.unsqueeze(0).contiguous()
-        mk, pk = msa_mask.unsqueeze(0), pair_mask.unsqueeze(0)
+        m0, z0 = m.unsqueeze(0).contiguous(), z.unsqueeze(0).contiguous()
+        mm, zz, mk, pk = m0, z0, msa_mask.unsqueeze(0), pair_mask.unsqueeze(0)
+        if not _needs_grad(self, m, z):       # the global attention takes any number of sequences
+            mm, zz, mk, pk = F_.pad_to_tiles(m0, z0, mk, pk, pad_s=False)
+        own = zz is not z0
         with F_.mask_cache():
             for i, b in enumerate(self.blocks):
-                mm, zz = b._core(mm, zz, mk, pk, inplace=(inplace_first or i > 0))
+                mm, zz = b._core(mm, zz, mk, pk, inplace=(inplace_first or i > 0 or own))
                 if self.clear_cache_between_blocks:
                     torch.cuda.empty_cache()
-        return zz.squeeze(0)
+        zz = zz.squeeze(0)
+        if own:
+            r = z.shape[0]
+            if inplace_first:
+                m.copy_(mm[0, :, :r])
+                return z.copy_(zz[:r, :r])
+            return zz[:r, :r].contiguous()
+        return zz
 
     def forward(self, m: torch.Tensor, z: torch.Tensor, chunk_size: int, msa_mask: Optional[torch.Tensor] = None,
                 pair_mask: Optional[torch.Tensor] = None, _mask_trans: bool = True) -> torch.Tensor:

@@ -207,13 +207,19 @@ class TemplatePairStack(nn.Module):
                 outs.append(self.layer_norm(z[0]))
             return torch.stack(outs, 0)
         out = t if (inplace and t.is_contiguous()) else torch.empty_like(t, memory_format=torch.contiguous_format)
+        r = t.shape[1]
+        dr = F_.round_up(r, 32) - r if t.dtype == torch.bfloat16 else 0       # whole tiles, see pad_to_tiles
+        if dr:
+            mask = F.pad(mask, (0, dr, 0, dr))
         for i in range(t.shape[0]):
             with F_.mask_cache():
                 z = t[i:i + 1].contiguous()
+                if dr:
+                    z = F.pad(z, (0, 0, 0, dr, 0, dr))
                 own = z.data_ptr() != t[i].data_ptr()          # a fresh copy may be overwritten
                 for k, b in enumerate(self.blocks):
                     z = b._core(z, mask[i:i + 1], inplace=(inplace or own or k > 0))
-            out[i] = self.layer_norm(z[0])
+            out[i] = self.layer_norm(z[0, :r, :r])
         return out
 
     def forward(self, t: torch.tensor, mask: torch.tensor, chunk_size: int, _mask_trans: bool = True):
