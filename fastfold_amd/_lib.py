@@ -8,6 +8,7 @@ launch stream is torch's current HIP stream.
 """
 import ctypes
 import os
+import threading
 from ctypes import c_int, c_int64, c_float, c_void_p, c_char_p
 
 import torch
@@ -33,6 +34,13 @@ SIGNATURES = {
 }
 
 _lib = None
+
+
+class _ThreadState(threading.local):
+    recorder = None          # see fastfold_amd/_plan.py
+
+
+_STATE = _ThreadState()
 
 
 def load(path: str = None):
@@ -107,6 +115,8 @@ def time_kernel(name, enable=True):
 def call(name: str, *args):
     """Calls an entry point; raises RuntimeError with the library's message on failure."""
     lib = load()
+    if _STATE.recorder is not None:
+        _STATE.recorder.note(name, args)
     rec = _TIMED.get(name)
     if rec is not None:
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -360,6 +370,15 @@ def gated_out_fused(out, x, gamma, beta, wg, bg, o, wo, bo, *, M, C, inner, s_o,
 def key_bias(keybias, tileflags, mask, *, B, N, mask_sb=0, mask_sn=1):
     call("ffk_key_bias", ptr(keybias), ptr(tileflags), ptr(mask), B, N, mask_sb, mask_sn,
          dtype_tag(mask.dtype) if mask is not None else FFK_F32, stream_ptr())
+
+
+SIGNATURES["ffk_fill_zero"] = [_P, _L, _P]
+SIGNATURES["ffk_run_plan"] = [_P, _L, _P, _L, _P]
+
+
+def fill_zero(t):
+    """Zeroes a contiguous tensor whose size is a multiple of 16 bytes."""
+    call("ffk_fill_zero", t.data_ptr(), t.numel() * t.element_size(), stream_ptr())
 
 
 SIGNATURES["ffk_global_attention_core"] = [_P, _P, _P, _P, _P, _F, _P, _P, _P, _L, _L, _L, _L, _L, _L, _L, _L, _L,

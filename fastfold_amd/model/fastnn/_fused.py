@@ -8,10 +8,11 @@ weight version).  Row-addressing conventions are those of ``ffk_fused_linear``: 
 import contextlib
 import math
 import os
+import threading
 
 import torch
 
-from fastfold_amd import _lib
+from fastfold_amd import _lib, _plan
 from fastfold_amd._lib import (FFK_ACT_NONE, FFK_ACT_RELU, FFK_ACT_SIGMOID, FFK_TILE_ACC, FFK_TILE_BIAS, FFK_TILE_QK,
                                FFK_TILE_STRIDED, FFK_TILE_V, LOG2E, make_tile)
 
@@ -32,7 +33,19 @@ def round_up(x, m):
 
 
 def alloc(shape, dtype, device, zero=False):
-    return (torch.zeros if zero else torch.empty)(shape, dtype=dtype, device=device)
+    """A scratch tensor of the launch sequences below."""
+    t = _plan.alloc(torch.empty(shape, dtype=dtype, device=device))
+    if zero:
+        if t.numel() * t.element_size() % 16:
+            raise RuntimeError("alloc: zeroed scratch must be a multiple of 16 bytes, got %s" % (tuple(t.shape),))
+        _lib.fill_zero(t)
+    return t
+
+
+def switches():
+    """Everything besides shapes and dtypes that the launch sequences below depend on."""
+    return (_WS_BUDGET_DEFAULT, _WS_BUDGET_CHUNKED, _FUSED_TRANSITION, _TRIMUL_CHAN_PAD, _PAIR_BIAS_RIDES, _BIAS_ROW_PAD,
+            _GATE_IN_OUT_STAGE, _GATE_IN_OUT_MIN_N, _GATE_IN_OUT_WIDTHS)
 
 
 def pack_rows(mats, dtype, device):
@@ -68,7 +81,16 @@ def check_nonempty(who, *ts):
 
 # ---- values derived from a mask only (key bias + tile flags of an attention, the normaliser of the outer
 # product mean) are the same in every block of a stack: inside `mask_cache()` they are computed once ----
-_MASK_CACHE = None
+class _MaskCache(threading.local):
+    entries = None           # of the calling thread, while in a mask_cache()
+
+
+_MASK_CACHE = _MaskCache()
+
+
+def mask_scope():
+    """The running ``mask_cache``, or one for the caller's block alone."""
+    return mask_cache() if _MASK_CACHE.entries is None else contextlib.nullcontext()
 
 
 @contextlib.contextmanager
@@ -76,24 +98,24 @@ def mask_cache():
     """While active, launches whose result depends only on a mask tensor are done once per distinct
     (storage, view geometry, version) and reused.  Entries keep their mask alive, so its memory cannot be
     handed to another tensor while the entry exists; the cache dies with the context."""
-    global _MASK_CACHE
-    prev, _MASK_CACHE = _MASK_CACHE, []
+    prev, _MASK_CACHE.entries = _MASK_CACHE.entries, []
     try:
         yield
     finally:
-        _MASK_CACHE = prev
+        _MASK_CACHE.entries = prev
 
 
 def _mask_derived(mask, what, build):
-    if _MASK_CACHE is None:
+    entries = _MASK_CACHE.entries
+    if entries is None:
         return build()
     key = (what, mask.data_ptr(), mask._version, tuple(mask.shape), tuple(mask.stride()), mask.dtype)
-    for k, _, v in _MASK_CACHE:
+    for k, _, v in entries:
         if k == key:
             return v
     v = build()
-    if len(_MASK_CACHE) < 32:          # a stack needs about ten; bounded whatever the caller does
-        _MASK_CACHE.append((key, mask, v))
+    if len(entries) < 32:              # a stack needs about ten; bounded whatever the caller does
+        entries.append((key, mask, v))
     return v
 
 
@@ -110,6 +132,8 @@ class PairBiasScratch:
 def _pair_bias_launch(bias_t, x, ln, w, scratch, **kw):
     if scratch is None:
         scratch = PairBiasScratch(x.shape[-1], x.device)
+    if not scratch.ready:
+        _plan.note_build()
     _lib.pair_bias(bias_t, x, ln[0], ln[1], None if scratch.ready else w, scratch.buf, **kw)
     scratch.ready = True
 
@@ -190,7 +214,7 @@ def transition(x, out, *, ln, w1_pk, b1_pk, w2, b2, hidden, budget, xtail=None):
         _lib.transition_fused(out, x, ln[0], ln[1], w1_pk, b1_pk, w2, b2, M=M, C=C, hidden=hidden, xtail=xtail)
         return out
     rows = max(128, min(M, (budget // (hidden * es)) // 128 * 128))
-    hid = torch.empty(min(rows, M), hidden, dtype=dt, device=dev)
+    hid = alloc((min(rows, M), hidden), dt, dev)
     nt = hidden // 128
     for r0 in range(0, M, rows):
         n = min(rows, M - r0)
@@ -206,6 +230,17 @@ def transition(x, out, *, ln, w1_pk, b1_pk, w2, b2, hidden, budget, xtail=None):
 
 
 # ---------------------------------------------------------------------- attention ----
+def key_bias(mask, device, *, B2, N, mask_sb, mask_sn):
+    """(additive key bias, key-tile flags) of an attention over B2 rows of N keys; from a mask once per ``mask_cache``."""
+    def build():
+        NT = (N + 31) // 32
+        kb = torch.empty(B2, NT * 32, dtype=torch.float32, device=device)
+        flags = torch.empty(B2, NT, dtype=torch.int32, device=device)
+        _lib.key_bias(kb, flags, mask, B=B2, N=N, mask_sb=mask_sb, mask_sn=mask_sn)
+        return kb, flags
+    return build() if mask is None else _mask_derived(mask, ("key_bias", B2, N, mask_sb, mask_sn), build)
+
+
 def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_pk, out_bias_pk, c_out,
               mask, mask_sb, mask_sn, bias_t=None, bias_in_launch=False, pb_scratch=None, head_dim=32, budget=None, o_map=None, xtail=None,
               drop=None):
@@ -264,8 +299,8 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
                    and resid.data_ptr() == x.data_ptr() and a_so % 16 == 0 and a_si % 16 == 0)
     gate = None
     if not gate_in_out:
-        gate = torch.empty((slab, H, NT, 1024) if acc_order else (slab * N, HC), dtype=dt, device=dev)
-    o = torch.empty(slab * N, HC, dtype=dt, device=dev)
+        gate = alloc((slab, H, NT, 1024) if acc_order else (slab * N, HC), dt, dev)
+    o = alloc((slab * N, HC), dt, dev)
     tpg = HC // 128
     qscale = LOG2E / math.sqrt(float(head_dim))
     tkw = dict(inner=N, s_o=H * NT * 1024, s_h=NT * 1024)
@@ -307,12 +342,7 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
         _lib.fused_linear(x, w_pk, [bias_tile], M=M, K=C, a_inner=a_inner, a_so=a_so, a_si=a_si, ln=ln,
                           w_row_off=4 * tpg * 128)
         bias_tile = None
-    def key_bias():
-        kb = torch.empty(B2, NT * 32, dtype=torch.float32, device=dev)
-        flags = torch.empty(B2, NT, dtype=torch.int32, device=dev)
-        _lib.key_bias(kb, flags, mask, B=B2, N=N, mask_sb=mask_sb, mask_sn=mask_sn)
-        return kb, flags
-    kb, flags = _mask_derived(mask, ("key_bias", B2, N, mask_sb, mask_sn), key_bias) if mask is not None else key_bias()
+    kb, flags = key_bias(mask, dev, B2=B2, N=N, mask_sb=mask_sb, mask_sn=mask_sn)
     for b0 in range(0, B2, slab):
         nb = min(slab, B2 - b0)
         Ms = nb * N
@@ -452,7 +482,7 @@ def triangle_multiplication(z, out, *, r, C, c, incoming, ln1, w_pk, b_pk, n_glu
     cs = r * kpad + _TRIMUL_CHAN_PAD
     lr = alloc((2, c, cs), dt, dev, zero)
     dual = dual_pk is not None and drop is None and trimul_gate_in_output_stage(dt, r, C, c)
-    g = None if dual else torch.empty(M, C, dtype=dt, device=dev)
+    g = None if dual else alloc((M, C), dt, dev)
     tiles = []
     if incoming:      # logical row (a, b) reads z[b, a]
         a_map, m_so, m_si = (r, C, r * C), 1, r
@@ -464,14 +494,19 @@ def triangle_multiplication(z, out, *, r, C, c, incoming, ln1, w_pk, b_pk, n_glu
             tiles.append(make_tile(lr.data_ptr() + (side * c + t * 64) * cs * es,
                                    bias=b_pk.data_ptr() + ti * 128 * es, glu=1, ncols=64, inner=r, s_o=kpad, s_i=1,
                                    s_h=32 * cs, s_d=cs, rowmask=mask, m_so=m_so, m_si=m_si))
+    gates = []
     for t in range((C + 127) // 128 if not dual else 0):
-        kw = dict(inner=r, s_o=C, s_i=r * C) if incoming else dict(inner=M, s_i=C)
-        tiles.append(make_tile(g.data_ptr() + t * 128 * es, bias=b_pk.data_ptr() + (n_glu + t) * 128 * es,
-                               act=FFK_ACT_SIGMOID, ncols=min(128, C - t * 128), **kw))
+        kw = dict(inner=r, s_o=C, s_i=r * C) if incoming and drop is None else dict(inner=M, s_i=C)
+        gates.append(make_tile(g.data_ptr() + t * 128 * es, bias=b_pk.data_ptr() + (n_glu + t) * 128 * es,
+                               act=FFK_ACT_SIGMOID, ncols=min(128, C - t * 128),
+                               gate=None if drop is None else drop.data_ptr() + t * 128 * es,
+                               gate_ld=0 if drop is None else C, gate_rows=0 if drop is None else r, **kw))
+    if drop is None:
+        tiles, gates = tiles + gates, []
     _lib.fused_linear(z, w_pk, tiles, M=M, K=C, a_inner=a_map[0], a_so=a_map[1], a_si=a_map[2], ln=ln1)
-    if drop is not None:
-        g.view(r, r, C).mul_(drop[None])
-    p = torch.empty(c, cs, dtype=dt, device=dev)
+    if gates:      # with dropout multipliers of row m % r: the gate's rows in the order of z, whatever the first launch's is
+        _lib.fused_linear(z, w_pk, gates, M=M, K=C, ln=ln1, w_row_off=n_glu * 128)
+    p = alloc((c, cs), dt, dev)
     _lib.bgemm_nt(lr[0], lr[1], p, M=r, N=r, K=kpad, lda=kpad, ldb=kpad, batch=c, a_bs=cs, b_bs=cs,
                   o_bs=cs, s_i=kpad)
     del lr
@@ -495,6 +530,20 @@ def triangle_multiplication(z, out, *, r, C, c, incoming, ln1, w_pk, b_pk, n_glu
 
 
 # ------------------------------------------------------------------ outer product mean ----
+def opm_normaliser(mask):
+    """fp32 [r, r]: sum over the sequences of mask[s, i] mask[s, j]; once per ``mask_cache``."""
+    s, r = mask.shape
+
+    def build():
+        spad = round_up(s, vec_of(mask.dtype))
+        mt = torch.zeros(r, spad, dtype=mask.dtype, device=mask.device)
+        mt[:, :s] = mask.t()
+        nrm = torch.empty(r, r, dtype=torch.float32, device=mask.device)
+        _lib.bgemm_nt(mt, mt, nrm, M=r, N=r, K=spad, lda=spad, ldb=spad, out_f32=True)
+        return nrm
+    return _mask_derived(mask, ("opm_norm", s, r), build)
+
+
 def outer_product_mean(m, mask, z, out, *, s, r, C, Cz, ln, wab_pk, bab_pk, wo, bo, budget, eps=1e-3, wo_ed=None,
                        xtail=None):
     """out = z + (Wo vec(sum_s a[s,i,:] (x) b[s,j,:]) + bo) / (sum_s mask[s,i] mask[s,j] + eps),
@@ -510,19 +559,13 @@ def outer_product_mean(m, mask, z, out, *, s, r, C, Cz, ln, wab_pk, bab_pk, wo, 
                      rowmask=mask, m_so=1, m_si=r)
     # logical row (i, s') reads m[s', i]
     _lib.fused_linear(m, wab_pk, [tile], M=s * r, K=C, a_inner=s, a_so=C, a_si=r * C, ln=ln)
-    def normaliser():
-        mt = torch.zeros(r, spad, dtype=dt, device=dev)
-        mt[:, :s] = mask.t()
-        nrm = torch.empty(r, r, dtype=torch.float32, device=dev)
-        _lib.bgemm_nt(mt, mt, nrm, M=r, N=r, K=spad, lda=spad, ldb=spad, out_f32=True)
-        return nrm
-    nrm = _mask_derived(mask, ("opm_norm", s, r, spad), normaliser)
+    nrm = opm_normaliser(mask)
     if fused:
         # fused core: the [r, r, 1024] outer product never leaves the chip
         _lib.opm_fused(out, z, ab[0], ab[1], wo_ed, bo, nrm, r=r, spad=spad, eps=eps, xtail=xtail)
         return out
     ci = max(1, min(r, budget // (r * 1024 * es)))
-    O = torch.empty(ci * r, 1024, dtype=dt, device=dev)
+    O = alloc((ci * r, 1024), dt, dev)
     for i0 in range(0, r, ci):
         n = min(ci, r - i0)
         _lib.bgemm_nt(ab.data_ptr() + i0 * 32 * spad * es, ab[1], O, M=32 * n, N=32 * r, K=spad, lda=spad, ldb=spad,
@@ -545,13 +588,13 @@ def global_attention(x, out, resid, *, S, R, C, H, D, x_ss, x_sr, out_ss, out_sr
     HD = H * D
     if not fits_fused(C, dt) or not fits_fused(HD, dt) or HD > 128 or c_out % vec_of(dt) != 0:
         raise RuntimeError("global_attention: unsupported widths C=%d, H*D=%d, out=%d" % (C, HD, c_out))
-    o = torch.empty(R, HD, dtype=dt, device=dev)
+    o = alloc((R, HD), dt, dev)
     _lib.global_attention_core(o, x, mask, None if ln is None else ln[0], None if ln is None else ln[1], wq, wk, wv,
                                S=S, R=R, C=C, H=H, D=D, m_ss=x_ss, m_sr=x_sr, mask_ss=mask_ss, mask_sr=mask_sr,
                                scaling=D ** -0.5, eps=eps)
     # gate and output projection, a bounded number of sequences at a time
     sc = max(1, min(S, budget // max(1, R * HD * es)))
-    tmp = torch.empty(sc * R, HD, dtype=dt, device=dev)
+    tmp = alloc((sc * R, HD), dt, dev)
     for s0 in range(0, S, sc):
         n = min(sc, S - s0)
         M = n * R

@@ -9,6 +9,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from fastfold_amd.model.fastnn.kernel import LayerNorm
+from fastfold_amd import _plan
 from . import _fused as F_
 from .ops import (ChunkMSAColumnGlobalAttention, ChunkTransition, OutProductMean, SelfAttention, Transition,
                   _PackMixin, _budget, _check_tail, _ln_pair, _mask_like, _needs_grad, _no_grad_guard)
@@ -42,6 +43,7 @@ class MSARowAttentionWithPairBias(nn.Module, _PackMixin):
 
     def _run(self, M_raw, Z, M_mask, out, xtail=None, drop=None):
         """``drop``: None or the [1, 1, r, C] dropout multipliers of a training-mode call (drawn by the caller)."""
+        _plan.scope()
         F_.check_cuda(M_raw, Z, M_mask)
         _no_grad_guard(self, M_raw, Z)
         dt, dev = M_raw.dtype, M_raw.device
@@ -107,6 +109,7 @@ class MSAColumnAttention(nn.Module, _PackMixin):
         self.attention = SelfAttention(qkv_dim=d_node, c=c, n_head=n_head, out_dim=d_node, gating=True)
 
     def _run(self, M_raw, M_mask, out, xtail=None):
+        _plan.scope()
         F_.check_cuda(M_raw, M_mask)
         _no_grad_guard(self, M_raw)
         dt, dev = M_raw.dtype, M_raw.device
@@ -163,17 +166,17 @@ class MSACore(nn.Module):
             node = self.MSAColumnAttention(node, node_mask)
             return self.MSATransition(node)
         node = node.contiguous()
-        out = torch.empty_like(node)
-        self.MSARowAttentionWithPairBias._run(node, pair, node_mask, out, xtail, drop=drop)
+        return self._into(node, pair, node_mask, torch.empty_like(node), xtail, drops)
+
+    def inplace(self, node, pair, node_mask, xtail=None, drops=None):
+        return self._into(node, pair, node_mask, node, xtail, drops)
+
+    def _into(self, node, pair, node_mask, out, xtail=None, drops=None):
+        """The updated node tensor in ``out`` (which may be ``node``)."""
+        self.MSARowAttentionWithPairBias._run(node, pair, node_mask, out, xtail, drop=(drops or {}).get("row"))
         self.MSAColumnAttention._run(out, node_mask, out, xtail)
         self.MSATransition._run(out, out, xtail)
         return out
-
-    def inplace(self, node, pair, node_mask, xtail=None, drops=None):
-        self.MSARowAttentionWithPairBias._run(node, pair, node_mask, node, xtail, drop=(drops or {}).get("row"))
-        self.MSAColumnAttention._run(node, node_mask, node, xtail)
-        self.MSATransition._run(node, node, xtail)
-        return node
 
 
 class ExtraMSACore(nn.Module):
@@ -192,19 +195,20 @@ class ExtraMSACore(nn.Module):
             node = self.MSAColumnAttention(node, node_mask)
             return self.MSATransition(node)
         node = node.contiguous()
-        out = torch.empty_like(node)
-        self.MSARowAttentionWithPairBias._run(node, pair, node_mask, out)
-        self.MSAColumnAttention._run(out, node_mask, out)
-        self.MSATransition._run(out, out)
-        return out
+        return self._into(node, pair, node_mask, torch.empty_like(node))
 
     def inplace(self, node, pair, node_mask):
         """``node`` is a one-element list; ``pair`` a tensor (msa.py:176-187)."""
         node[0] = node[0].contiguous()
-        self.MSARowAttentionWithPairBias._run(node[0], pair, node_mask, node[0])
-        self.MSAColumnAttention._run(node[0], node_mask, node[0])
-        self.MSATransition._run(node[0], node[0])
+        self._into(node[0], pair, node_mask, node[0])
         return node
+
+    def _into(self, node, pair, node_mask, out):
+        """The updated node tensor in ``out`` (which may be ``node``)."""
+        self.MSARowAttentionWithPairBias._run(node, pair, node_mask, out)
+        self.MSAColumnAttention._run(out, node_mask, out)
+        self.MSATransition._run(out, out)
+        return out
 
 
 class ExtraMSABlock(nn.Module):
@@ -233,23 +237,30 @@ class ExtraMSABlock(nn.Module):
             m = self.msa_stack(m, z, msa_mask)
             z = self.communication(m, msa_mask, z)
             return m, self.pair_stack(z, pair_mask)
+        F_.check_cuda(m, z, msa_mask, pair_mask)
+        _no_grad_guard(self, m, z)
+        m_out, z_out = (m, z) if inplace else (torch.empty_like(m), torch.empty_like(z))
+        s, r = m.shape[1], m.shape[2]
+        msa_mask, pair_mask = _mask_like(msa_mask, m), _mask_like(pair_mask, z)
+        with F_.mask_scope():
+            mm, pm = msa_mask[0], pair_mask[0]
+            tensors = [m, z, m_out, z_out, mm, pm, *F_.key_bias(mm, m.device, B2=s, N=r, mask_sb=r, mask_sn=1),
+                       *F_.key_bias(pm, m.device, B2=r, N=r, mask_sb=r, mask_sn=1),
+                       *F_.key_bias(pm, m.device, B2=r, N=r, mask_sb=1, mask_sn=r), F_.opm_normaliser(mm)]
+            _plan.run(self, (m.shape, z.shape, mm.shape, pm.shape, m.dtype, m.device, inplace, self.is_multimer, _budget(), F_.switches()), tensors,
+                      lambda: self._sequence(m, z, m_out, z_out, msa_mask, pair_mask))
+        return m_out, z_out
+
+    def _sequence(self, m, z, m_out, z_out, msa_mask, pair_mask):
         if self.is_multimer:
             # msa.py:252-258, 321-332: outer product mean first, the MSA stack reads the pair tensor it leaves,
             # the pair stack runs last
-            z_new = z if inplace else torch.empty_like(z)
-            self.communication._run(m, msa_mask, z, z_new)
-            m = self.msa_stack.inplace([m], z_new, msa_mask)[0] if inplace else self.msa_stack.forward(m, z_new, msa_mask)
-            self.pair_stack.inplace([z_new], pair_mask)
-            return m, z_new
-        if inplace:
-            m = self.msa_stack.inplace([m], z, msa_mask)[0]
-            self.communication._run(m, msa_mask, z, z)
-            self.pair_stack.inplace([z], pair_mask)
-            return m, z
-        m = self.msa_stack.forward(m, z, msa_mask)
-        z = self.communication.forward(m, msa_mask, z)
-        self.pair_stack.inplace([z], pair_mask)
-        return m, z
+            self.communication._run(m, msa_mask, z, z_out)
+            self.msa_stack._into(m, z_out, msa_mask, m_out)
+        else:
+            self.msa_stack._into(m, z, msa_mask, m_out)
+            self.communication._run(m_out, msa_mask, z, z_out)
+        self.pair_stack.inplace([z_out], pair_mask)
 
     def _enter(self, m, z, s, r):
         if self.first_block:

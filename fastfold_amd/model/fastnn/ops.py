@@ -14,7 +14,7 @@ import os
 import torch
 import torch.nn as nn
 
-from fastfold_amd import _lib
+from fastfold_amd import _lib, _plan
 from fastfold_amd.model.fastnn.kernel import LayerNorm
 from . import _fused as F_
 from .initializer import glorot_uniform_af
@@ -46,7 +46,8 @@ class _PackMixin:
     ``invalidate_packed()`` on the module (or any parent, via ``module.apply``) after such a write."""
 
     def invalidate_packed(self):
-        self.__dict__.pop("_pack_cache", None)
+        if self.__dict__.pop("_pack_cache", None):
+            _plan.invalidate()
 
     def _apply(self, fn, *args, **kwargs):
         self.invalidate_packed()
@@ -61,6 +62,7 @@ class _PackMixin:
         ver = tuple((p.data_ptr(), p._version, p.dtype) for p in params)
         ent = cache.get(key)
         if ent is None or ent[0] != ver:
+            _plan.note_build()
             with torch.no_grad():
                 ent = (ver, build())
             cache[key] = ent
@@ -400,6 +402,7 @@ class Transition(nn.Module, _PackMixin):
         self.linear2 = Linear(n * d, d, initializer='zeros')
 
     def _run(self, src, out, xtail=None):
+        _plan.scope()
         F_.check_cuda(src)
         _no_grad_guard(self, src)
         dt, dev = src.dtype, src.device
@@ -449,6 +452,7 @@ class OutProductMean(nn.Module, _PackMixin):
         self.n_feat_proj = n_feat_proj
 
     def _run(self, M, M_mask, Z_raw, out, xtail=None):
+        _plan.scope()
         F_.check_cuda(M, M_mask, Z_raw)
         _no_grad_guard(self, M, Z_raw)
         if self.n_feat_proj != 32:
@@ -695,6 +699,7 @@ class ChunkMSAColumnGlobalAttention(nn.Module):
         self.global_attention = GlobalAttention(qkv_dim=d_node, c=c, n_head=n_head, out_dim=d_node)
 
     def _run(self, M_raw, M_mask, out):
+        _plan.scope()
         F_.check_cuda(M_raw, M_mask)
         _no_grad_guard(self, M_raw)
         if M_raw.dim() != 4 or M_raw.shape[0] != 1:
@@ -748,6 +753,7 @@ class _TriangleMultiplication(nn.Module, _PackMixin):
 
     def _run(self, Z_raw, Z_mask, out, xtail=None, drop=None):
         """``drop``: None or the [1, 1, r, C] dropout multipliers of a training-mode call (drawn by the caller)."""
+        _plan.scope()
         F_.check_cuda(Z_raw, Z_mask)
         _no_grad_guard(self, Z_raw)
         dt, dev = Z_raw.dtype, Z_raw.device
@@ -842,6 +848,7 @@ class _TriangleAttention(nn.Module, _PackMixin):
     def _run(self, Z_raw, Z_mask, out, xtail=None, drop=None):
         """``drop``: None or the dropout multipliers of a training-mode call, [1, 1, r, C] (starting node) or
         [1, r, 1, C] (ending node)."""
+        _plan.scope()
         F_.check_cuda(Z_raw, Z_mask)
         _no_grad_guard(self, Z_raw)
         dt, dev = Z_raw.dtype, Z_raw.device

@@ -14,11 +14,11 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from fastfold_amd.model.fastnn.kernel import LayerNorm
-from fastfold_amd import _lib
+from fastfold_amd import _lib, _plan
 from . import _fused as F_
 from .ops import (AsyncChunkTriangleMultiplicationIncoming, AsyncChunkTriangleMultiplicationOutgoing,
                   ChunkTransition, ChunkTriangleAttentionEndingNode, ChunkTriangleAttentionStartingNode, Linear,
-                  _PackMixin, _needs_grad, _no_grad_guard)
+                  _PackMixin, _budget, _mask_like, _needs_grad, _no_grad_guard)
 
 
 class _PointwiseProjections(nn.Module):
@@ -146,13 +146,25 @@ class TemplatePairBlock(nn.Module):
             z = self.TriangleMultiplicationOutgoing(z, mask)
             z = self.TriangleMultiplicationIncoming(z, mask)
             return self.PairTransition(z)
+        F_.check_cuda(z, mask)
+        _no_grad_guard(self, z)
         out = z if inplace else torch.empty_like(z)
+        r = z.shape[1]
+        mask = _mask_like(mask, z)
+        with F_.mask_scope():
+            pm = mask[0]
+            tensors = [z, out, pm, *F_.key_bias(pm, z.device, B2=r, N=r, mask_sb=r, mask_sn=1),
+                       *F_.key_bias(pm, z.device, B2=r, N=r, mask_sb=1, mask_sn=r)]
+            _plan.run(self, (z.shape, pm.shape, z.dtype, z.device, inplace, _budget(), F_.switches()), tensors,
+                      lambda: self._sequence(z, mask, out))
+        return out
+
+    def _sequence(self, z, mask, out):
         self.TriangleAttentionStartingNode._run(z, mask, out)
         self.TriangleAttentionEndingNode._run(out, mask, out)
         self.TriangleMultiplicationOutgoing._run(out, mask, out)
         self.TriangleMultiplicationIncoming._run(out, mask, out)
         self.PairTransition._run(out, out)
-        return out
 
     def _enter(self, z, r):
         if z.dim() != 4 or z.shape[0] != 1:

@@ -461,6 +461,25 @@ int ffk_pointwise_attention_core(void* o, const void* q, const void* kv, const f
 int ffk_key_bias(float* keybias, int32_t* tileflags, const void* mask, int64_t B, int64_t N,
                  int64_t mask_sb, int64_t mask_sn, int dtype, void* stream);
 
+/* Zeroes `bytes` (a multiple of 16) at a 16-byte aligned address with a kernel: padding rows and columns of operand
+ * buffers, in code that may be captured into a graph. */
+int ffk_fill_zero(void* p, int64_t bytes, void* stream);
+
+/* ------------------------------------------------------------------------------------
+ * Launch plans: replays a recorded sequence of entry points with other buffers.  A plan is a byte string of operations,
+ *   { int32 op, n_slots, n_relocs, 0;  n_relocs x { int32 slot, base; int64 offset };  n_slots x 8 bytes of arguments }
+ * one after the other.  The arguments of an operation are its entry point's, in order and without the stream, one 8-byte
+ * slot each (pointers as addresses, integers as int64, floats in the low four bytes) - or, for the entry points that take
+ * a descriptor, the descriptor itself.  A relocation replaces slot `slot` by bases[base] + offset.  The call does what the
+ * calls would do one by one, and stops at the first that fails.  No counterpart in the reference.
+ */
+enum {
+    FFK_OP_FUSED_LINEAR = 0, FFK_OP_BGEMM_NT = 1, FFK_OP_ATTENTION_FWD = 2, FFK_OP_PAIR_BIAS = 3, FFK_OP_OPM_FUSED = 4,
+    FFK_OP_TRANSITION_FUSED = 5, FFK_OP_GATED_OUT_FUSED = 6, FFK_OP_GLOBAL_ATTENTION_CORE = 7, FFK_OP_LAYERNORM_FWD = 8,
+    FFK_OP_FILL_ZERO = 9, FFK_OP_COUNT = 10
+};
+int ffk_run_plan(const void* plan, int64_t bytes, const uint64_t* bases, int64_t n_bases, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
