@@ -412,3 +412,71 @@ def pointwise_attention_core(o, q, kv, bias, *, P, H, D, NT, kv_st, kv_sp, v_off
         raise RuntimeError("pointwise_attention_core: out_scale must be one fp32 value on the device")
     call("ffk_pointwise_attention_core", ptr(o), ptr(q), ptr(kv), ptr(bias), ptr(out_scale), P, H, D, NT, kv_st, kv_sp, v_off,
          dtype_tag(q.dtype), stream_ptr())
+
+
+# ----------------------------------------------------------------- backward pass of a block ----
+SIGNATURES["ffk_attention_fwd_lse"] = [_P] * 9 + [_L, _L, _L, _L, _L, _I, _I, _P]
+SIGNATURES["ffk_attention_bwd_rows"] = [_P] * 4 + [_L] + [_P] * 11 + [_L] * 6 + [_F, _F, _I, _I, _P]
+SIGNATURES["ffk_weight_grad"] = [_P, _L, _P, _L, _L, _P, _P, _P, _P] + [_L] * 14 + [_I, _I, _P]
+SIGNATURES["ffk_slice_sum"] = [_P, _P] + [_L] * 7 + [_I, _P]
+SIGNATURES["ffk_layernorm_bwd_rows"] = [_P] * 10 + [_L, _L, _F, _I, _P]
+SIGNATURES["ffk_scale_rows"] = [_P, _P, _P, _L, _L, _L, _L, _L, _I, _F, _I, _P]
+SIGNATURES["ffk_att_gate_bwd"] = [_P] * 9 + [_L] * 5 + [_I, _P]
+SIGNATURES["ffk_trimul_gate_bwd"] = [_P] * 6 + [_L] * 5 + [_I, _P]
+SIGNATURES["ffk_glu_bwd"] = [_P] * 6 + [_L] * 8 + [_I, _P]
+SIGNATURES["ffk_bias_cols"] = [_P, _P, _L, _L, _L, _L, _I, _P]
+FFK_WGRAD_READ, FFK_WGRAD_WRITE = 1, 2
+FFK_ACT_GATE_POS = 3
+FFK_LN_BWD_BLOCKS = 1024
+
+
+def attention_fwd_lse(out, lse, q_t, k_t, v_t, bias_t, keybias, tileflags, *, B2, H, N, bias_padded=False):
+    call("ffk_attention_fwd_lse", ptr(out), ptr(lse), ptr(q_t), ptr(k_t), ptr(v_t), ptr(bias_t), ptr(keybias), ptr(tileflags),
+         None, B2, H, N, N, 32, FFK_ATT_BIAS_PADDED if bias_padded else 0, dtype_tag(q_t.dtype), stream_ptr())
+
+
+def attention_bwd_rows(dq, dk, dv, dbias, lse, dsum, q_t, q_v, k_t, k_v, v_t, bias_t, keybias, do_t, do_v, *, B2, H, N, s_b, s_h,
+                       s_n, dq_scale, dk_scale, dtype, dbias_parts=0, bias_padded=False):
+    call("ffk_attention_bwd_rows", ptr(dq), ptr(dk), ptr(dv), ptr(dbias), dbias_parts, ptr(lse), ptr(dsum), ptr(q_t), ptr(q_v),
+         ptr(k_t), ptr(k_v), ptr(v_t), ptr(bias_t), ptr(keybias), ptr(do_t), ptr(do_v), B2, H, N, s_b, s_h, s_n, dq_scale,
+         dk_scale, FFK_ATT_BIAS_PADDED if bias_padded else 0, dtype_tag(dtype), stream_ptr())
+
+
+def weight_grad(out, colsum, ws, y, x, *, M, N, K, slices, dtype, y_map, x_map, n_out=None, cs_first=0, cs_count=None,
+                o_map=None, acc=None, flags=0):
+    """``y_map`` / ``x_map``: (inner, s_o, s_i) of the operand rows; ``o_map``: (inner, s_o, s_i, s_k) of the output."""
+    o_map = (N, 0, K, 1) if o_map is None else o_map
+    call("ffk_weight_grad", ptr(out), N if n_out is None else n_out, ptr(colsum), cs_first, N if cs_count is None else cs_count,
+         ptr(acc), ptr(ws), ptr(y), ptr(x), M, N, K, slices, *y_map, *x_map, *o_map, flags, dtype_tag(dtype), stream_ptr())
+
+
+def slice_sum(out, part, *, slices, N, K, o_map, dtype):
+    call("ffk_slice_sum", ptr(out), ptr(part), slices, N, K, *o_map, dtype_tag(dtype), stream_ptr())
+
+
+def layernorm_bwd_rows(dx, xn, dgamma, dbeta, ws, dy, x, gamma, beta, resid, *, rows, C, dtype, eps=1e-5):
+    call("ffk_layernorm_bwd_rows", ptr(dx), ptr(xn), ptr(dgamma), ptr(dbeta), ptr(ws), ptr(dy), ptr(x), ptr(gamma), ptr(beta),
+         ptr(resid), rows, C, eps, dtype_tag(dtype), stream_ptr())
+
+
+def scale_rows(out, x, mul, *, rows, C, inner, m_so, m_si, mode, dtype, eps=0.0):
+    call("ffk_scale_rows", ptr(out), ptr(x), ptr(mul), rows, C, inner, m_so, m_si, mode, eps, dtype_tag(dtype), stream_ptr())
+
+
+def att_gate_bwd(go, dgpre, do_t, do_v, dsum, dgo, gpre, gbias, o, *, B2, N, H, g_ld, dg_ld, dtype):
+    call("ffk_att_gate_bwd", ptr(go), ptr(dgpre), ptr(do_t), ptr(do_v), ptr(dsum), ptr(dgo), ptr(gpre), ptr(gbias), ptr(o), B2, N,
+         H, g_ld, dg_ld, dtype_tag(dtype), stream_ptr())
+
+
+def trimul_gate_bwd(dab, dgpre, dz, drop, ab, gpre, *, rows, C, period, g_ld, dg_ld, dtype):
+    call("ffk_trimul_gate_bwd", ptr(dab), ptr(dgpre), ptr(dz), ptr(drop), ptr(ab), ptr(gpre), rows, C, period, g_ld, dg_ld,
+         dtype_tag(dtype), stream_ptr())
+
+
+def glu_bwd(dproj, dgate, dl, l, gate, mask, *, R, C, cs, kpad, d_ld, g_ld, r_i, r_k, dtype):
+    call("ffk_glu_bwd", ptr(dproj), ptr(dgate), ptr(dl), ptr(l), ptr(gate), ptr(mask), R, C, cs, kpad, d_ld, g_ld, r_i, r_k,
+         dtype_tag(dtype), stream_ptr())
+
+
+def bias_cols(out, dbias, *, parts, rows, H, ld, dtype):
+    call("ffk_bias_cols", ptr(out), ptr(dbias), parts, rows, H, ld, dtype_tag(dtype), stream_ptr())

@@ -22,7 +22,9 @@ import torch
 from . import _lib
 
 OPS = ["ffk_fused_linear", "ffk_bgemm_nt", "ffk_attention_fwd", "ffk_pair_bias", "ffk_opm_fused", "ffk_transition_fused",
-       "ffk_gated_out_fused", "ffk_global_attention_core", "ffk_layernorm_fwd", "ffk_fill_zero"]     # order of FFK_OP_*
+       "ffk_gated_out_fused", "ffk_global_attention_core", "ffk_layernorm_fwd", "ffk_fill_zero", "ffk_attention_fwd_lse",
+       "ffk_attention_bwd_rows", "ffk_transpose_batched", "ffk_weight_grad", "ffk_layernorm_bwd_rows", "ffk_scale_rows",
+       "ffk_att_gate_bwd", "ffk_trimul_gate_bwd", "ffk_glu_bwd", "ffk_bias_cols", "ffk_slice_sum"]   # order of FFK_OP_*
 _CODE = {name: i for i, name in enumerate(OPS)}
 _MAX_PLANS = 16               # per module: shapes in use at a time
 _ALIGN = 512                  # of scratch buffers, as torch's allocator aligns its blocks
@@ -73,22 +75,27 @@ class _Recorder:
         self.bound = [(t.data_ptr(), t.data_ptr() + t.numel() * t.element_size(), i + 2) for i, t in enumerate(tensors)
                       if t is not None]
         self.keep = [(t.data_ptr(), t.data_ptr() + t.numel() * t.element_size()) for t in keep]
-        self.temps = []
-        self.bump = self.peak = 0
+        self.temps, self.held = [], []
+        self.bump = self.peak = self.floor = 0
         self.out = []
         self.failed = None
 
     def alloc(self, t):
-        size = t.numel() * t.element_size()
-        size = -(-size // _ALIGN) * _ALIGN if size < _LARGE else -(-size // _PAGE) * _PAGE + _STAGGER
-        self.temps.append((t.data_ptr(), t.data_ptr() + size, self.bump))
+        used = t.numel() * t.element_size()
+        size = -(-used // _ALIGN) * _ALIGN if used < _LARGE else -(-used // _PAGE) * _PAGE + _STAGGER
+        self.temps.append((t.data_ptr(), t.data_ptr() + used, self.bump))
         self.bump += size
         self.peak = max(self.peak, self.bump)
 
     def scope(self):
         """A sub-module begins: the scratch of the one before is dead."""
-        self.temps = []
-        self.bump = 0
+        self.temps = list(self.held)
+        self.bump = self.floor
+
+    def hold(self):
+        """What has been allocated so far stays alive until the end of the sequence."""
+        self.held = list(self.temps)
+        self.floor = self.bump
 
     def _reloc(self, p):
         for lo, hi, off in reversed(self.temps):       # the youngest first: memory freed in between may have been reused
@@ -213,6 +220,12 @@ def scope():
         rec.scope()
 
 
+def hold():
+    rec = _lib._STATE.recorder
+    if rec is not None:
+        rec.hold()
+
+
 def run(owner, key, tensors, sequence):
     """Executes ``sequence()`` - launches on the current stream that work on ``tensors`` (a list, entries may be None; the
     first is not), on scratch from ``alloc`` and on the weights of the module ``owner`` - or replays its plan.  ``key``
@@ -228,6 +241,8 @@ def run(owner, key, tensors, sequence):
         if plan.blob is None:
             return sequence()
         return plan.run(tensors)
+    if any(p.dtype != tensors[0].dtype for d in st.watch.params for p in d.values() if p is not None):
+        return sequence()        # parameters of another dtype are converted on the way, into memory no recording knows
     before = builds
     rec = _lib._STATE.recorder = _Recorder(tensors, st.watch.tensors())
     try:

@@ -100,7 +100,7 @@ template <typename T, bool HAS_BIAS>
 __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention_kernel(
     T* __restrict__ out, const T* __restrict__ q_t, const T* __restrict__ k_t, const T* __restrict__ v_t,
     const T* __restrict__ bias_t, const float* __restrict__ keybias, const int* __restrict__ tileflags,
-    const T* __restrict__ gate, int B2, int H, int Nq, int Nk, int flags) {
+    const T* __restrict__ gate, float* __restrict__ lse, int B2, int H, int Nq, int Nk, int flags) {
     typedef Mma<T> MM;
     typedef typename MM::Frag Frag;
     constexpr int NF = 16 / MM::KLANE;            // fragments per 16-element lane slice (bf16 2, fp32 4)
@@ -384,6 +384,9 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
     // rows whose keys are all masked have l == 0 and produce zeros
     const float l_tot = l_run + lane_xor<32>(l_run);
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+    // log-sum-exp of the row (log2 domain) for the backward kernels; an all-masked row's makes every exp2(s - lse) zero
+    if (lse && live && half == 0)
+        lse[(bh * QT + qt) * 32 + l32] = l_tot > 0.0f ? __builtin_amdgcn_logf(l_tot) - negm[0] : 3.0e38f;
     if (live && q < Nq) {
         T gv[4][4];
         if (gate) {
@@ -555,7 +558,8 @@ __global__ void key_bias_kernel(float* kb, int* flags, const T* mask, long N, lo
 
 template <typename T, bool HAS_BIAS>
 int launch_attention_b(void* out, const void* q, const void* k, const void* v, const void* bias, const float* kb,
-                       const int* flags, const void* gate, long B2, long H, long Nq, long Nk, int aflags, hipStream_t st) {
+                       const int* flags, const void* gate, float* lse, long B2, long H, long Nq, long Nk, int aflags,
+                       hipStream_t st) {
     const size_t smem = (3 * (size_t)(HAS_BIAS ? 8 : 4) * 1024 + ATT_THREADS * 16) * sizeof(T) + 16;   // operand ring + gate + redo flag
     static FfkLdsReservation lds_reserved;
     {
@@ -566,16 +570,17 @@ int launch_attention_b(void* out, const void* q, const void* k, const void* v, c
     FFK_REQUIRE(items < (1L << 31) - 8, FFK_ERR_SHAPE, "ffk_attention_fwd: %ld workgroups exceed the grid limit", items);
     dim3 grid((unsigned)(8 * ffk_cdiv(items, 8)));
     attention_kernel<T, HAS_BIAS><<<grid, ATT_THREADS, smem, st>>>((T*)out, (const T*)q, (const T*)k, (const T*)v,
-                                                                  (const T*)bias, kb, flags, (const T*)gate, (int)B2,
+                                                                  (const T*)bias, kb, flags, (const T*)gate, lse, (int)B2,
                                                                   (int)H, (int)Nq, (int)Nk, aflags);
     return ffk_check_launch("ffk_attention_fwd");
 }
 
 template <typename T>
 int launch_attention(void* out, const void* q, const void* k, const void* v, const void* bias, const float* kb,
-                     const int* flags, const void* gate, long B2, long H, long Nq, long Nk, int aflags, hipStream_t st) {
-    return bias ? launch_attention_b<T, true>(out, q, k, v, bias, kb, flags, gate, B2, H, Nq, Nk, aflags, st)
-                : launch_attention_b<T, false>(out, q, k, v, nullptr, kb, flags, gate, B2, H, Nq, Nk, aflags, st);
+                     const int* flags, const void* gate, float* lse, long B2, long H, long Nq, long Nk, int aflags,
+                     hipStream_t st) {
+    return bias ? launch_attention_b<T, true>(out, q, k, v, bias, kb, flags, gate, lse, B2, H, Nq, Nk, aflags, st)
+                : launch_attention_b<T, false>(out, q, k, v, nullptr, kb, flags, gate, lse, B2, H, Nq, Nk, aflags, st);
 }
 
 }  // namespace
@@ -583,6 +588,12 @@ int launch_attention(void* out, const void* q, const void* k, const void* v, con
 extern "C" int ffk_attention_fwd(void* out, const void* q_t, const void* k_t, const void* v_t, const void* bias_t,
                                  const float* keybias, const int32_t* tileflags, const void* gate, int64_t B2, int64_t H, int64_t Nq,
                                  int64_t Nk, int64_t D, int flags, int dtype, void* stream) {
+    return ffk_attention_fwd_lse(out, nullptr, q_t, k_t, v_t, bias_t, keybias, tileflags, gate, B2, H, Nq, Nk, D, flags, dtype, stream);
+}
+
+extern "C" int ffk_attention_fwd_lse(void* out, float* lse, const void* q_t, const void* k_t, const void* v_t, const void* bias_t,
+                                     const float* keybias, const int32_t* tileflags, const void* gate, int64_t B2, int64_t H,
+                                     int64_t Nq, int64_t Nk, int64_t D, int flags, int dtype, void* stream) {
     FFK_REQUIRE(out && q_t && k_t && v_t && keybias && tileflags, FFK_ERR_NULL, "ffk_attention_fwd: null pointer");
     FFK_REQUIRE(B2 > 0 && B2 < 131072 && H > 0 && H < 65536 && Nq > 0 && Nk > 0 && Nq < (1 << 24) && Nk < (1 << 24),
                 FFK_ERR_SHAPE, "ffk_attention_fwd: bad shape B2=%ld H=%ld Nq=%ld Nk=%ld", (long)B2, (long)H, (long)Nq,
@@ -594,8 +605,8 @@ extern "C" int ffk_attention_fwd(void* out, const void* q_t, const void* k_t, co
                 "ffk_attention_fwd: head dimension %ld (32, 64 or 128; narrower heads arrive zero-padded to 32)", (long)D);
     hipStream_t st = (hipStream_t)stream;
     if (D != 32) {
-        FFK_REQUIRE(!gate && !(flags & (FFK_ATT_BIAS_PADDED | FFK_ATT_HALF_K)), FFK_ERR_UNSUPPORTED,
-                    "ffk_attention_fwd: the gate, padded bias rows and the narrow-head flag are built for head dimension 32 only");
+        FFK_REQUIRE(!gate && !lse && !(flags & (FFK_ATT_BIAS_PADDED | FFK_ATT_HALF_K)), FFK_ERR_UNSUPPORTED,
+                    "ffk_attention_fwd: the gate, the log-sum-exp, padded bias rows and the narrow-head flag are built for head dimension 32 only");
         if (dtype == FFK_BF16)
             return D == 64 ? launch_attention_wide<bf16_t, 2>(out, q_t, k_t, v_t, bias_t, keybias, tileflags, B2, H, Nq, Nk, st)
                            : launch_attention_wide<bf16_t, 4>(out, q_t, k_t, v_t, bias_t, keybias, tileflags, B2, H, Nq, Nk, st);
@@ -605,8 +616,8 @@ extern "C" int ffk_attention_fwd(void* out, const void* q_t, const void* k_t, co
         return ffk_fail(FFK_ERR_DTYPE, "ffk_attention_fwd: unsupported dtype tag %d", dtype);
     }
     switch (dtype) {
-        case FFK_BF16: return launch_attention<bf16_t>(out, q_t, k_t, v_t, bias_t, keybias, tileflags, gate, B2, H, Nq, Nk, flags, st);
-        case FFK_F32: return launch_attention<float>(out, q_t, k_t, v_t, bias_t, keybias, tileflags, gate, B2, H, Nq, Nk, flags, st);
+        case FFK_BF16: return launch_attention<bf16_t>(out, q_t, k_t, v_t, bias_t, keybias, tileflags, gate, lse, B2, H, Nq, Nk, flags, st);
+        case FFK_F32: return launch_attention<float>(out, q_t, k_t, v_t, bias_t, keybias, tileflags, gate, lse, B2, H, Nq, Nk, flags, st);
         default: return ffk_fail(FFK_ERR_DTYPE, "ffk_attention_fwd: unsupported dtype tag %d", dtype);
     }
 }

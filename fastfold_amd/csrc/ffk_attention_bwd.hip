@@ -28,6 +28,7 @@
 // as the forward pass); waves load their tiles straight from global memory - this pair of kernels serves the
 // autograd path of the stand-alone operator, not the inference block, and is not tuned beyond that.
 #include "ffk_common.h"
+#include <initializer_list>
 
 namespace {
 
@@ -83,13 +84,29 @@ __device__ __forceinline__ long bwd_logical_block() {
     return (long)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
 }
 
+// Where a gradient goes: element (b2, head, token, d) at b2 * s_b + head * s_h + token * s_n + d.
+struct OutMap {
+    long s_b, s_h, s_n;
+};
+
+template <typename T>
+__device__ __forceinline__ void store4(T* o, const float* f) {          // four consecutive elements, 4-element aligned
+    T r[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = DT<T>::from_f(f[e]);
+    if (sizeof(T) == 2) *reinterpret_cast<u32x2*>(o) = *reinterpret_cast<const u32x2*>(r);
+    else *reinterpret_cast<u32x4*>(o) = *reinterpret_cast<const u32x4*>(r);
+}
+
 // ------------------------------------------------------------------------------ dq ----
-template <typename T, int DP, bool HAS_BIAS>
+// STATS: the row statistics are computed here (a walk over the keys of its own) and written for the other kernels; otherwise
+// the forward pass has left the log-sum-exp and the gate's backward kernel sum_d do o.
+template <typename T, int DP, bool HAS_BIAS, bool STATS>
 __global__ __launch_bounds__(256) void attention_bwd_dq_kernel(
     T* __restrict__ dq, float* __restrict__ lse, float* __restrict__ dsum, const T* __restrict__ q_qk,
     const T* __restrict__ k_qk, const T* __restrict__ k_acc, const T* __restrict__ v_qk, const T* __restrict__ bias_t,
     const float* __restrict__ keybias, const T* __restrict__ do_qk, const T* __restrict__ o_qk, int B2, int H, int Nq,
-    int Nk, float dq_scale, long part_q, long part_k) {
+    int Nk, float dq_scale, long part_q, long part_k, OutMap om, int bias_pad) {
     typedef Mma<T> MM;
     typedef typename MM::Frag Frag;
     constexpr int NF = 16 / MM::KLANE;
@@ -106,14 +123,17 @@ __global__ __launch_bounds__(256) void attention_bwd_dq_kernel(
     float dpart = 0.0f;
 #pragma unroll
     for (int p = 0; p < DP; ++p) {
-        Tile16<T> of;
         qf[p].load(q_qk + p * part_q + ((bh * QT + qt) << 10) + lane * 16);
         dof[p].load(do_qk + p * part_q + ((bh * QT + qt) << 10) + lane * 16);
-        of.load(o_qk + p * part_q + ((bh * QT + qt) << 10) + lane * 16);
+        if (STATS) {
+            Tile16<T> of;
+            of.load(o_qk + p * part_q + ((bh * QT + qt) << 10) + lane * 16);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) dpart += dof[p].f(j) * of.f(j);
+            for (int j = 0; j < 16; ++j) dpart += dof[p].f(j) * of.f(j);
+        }
     }
-    const float D = dpart + lane_xor<32>(dpart);             // this lane's query: sum_d do o
+    // this lane's query: sum_d do o
+    const float D = STATS ? dpart + lane_xor<32>(dpart) : dsum[(bh * QT + qt) * 32 + l32];
     const float* mp = keybias + (long)b2 * KT * 32 + 4 * half;
 
     Frag ident[NF];
@@ -134,7 +154,7 @@ __global__ __launch_bounds__(256) void attention_bwd_dq_kernel(
         }
         if (HAS_BIAS) {
             Tile16<T> bc;
-            bc.load(bias_t + ((((long)h * QT + qt) * KT + kt) << 10) + lane * 16);
+            bc.load(bias_t + ((((long)h * QT + qt) * (KT + bias_pad) + kt) << 10) + lane * 16);
 #pragma unroll
             for (int i = 0; i < NF; ++i) MM::mma(s, bc.frag(i), ident[i]);
         }
@@ -146,27 +166,32 @@ __global__ __launch_bounds__(256) void attention_bwd_dq_kernel(
         }
     };
 
-    // first walk: row maximum and sum
-    float m_run = REF_FLOOR, l_run = 0.0f;
-    for (int kt = 0; kt < KT; ++kt) {
-        f32x16 s;
-        score(kt, s);
-        float mt = fmaxf(s[0], s[1]);
+    float L;
+    if (STATS) {
+        // first walk: row maximum and sum
+        float m_run = REF_FLOOR, l_run = 0.0f;
+        for (int kt = 0; kt < KT; ++kt) {
+            f32x16 s;
+            score(kt, s);
+            float mt = fmaxf(s[0], s[1]);
 #pragma unroll
-        for (int v = 2; v < 16; ++v) mt = fmaxf(mt, s[v]);
-        mt = fmaxf(mt, lane_xor<32>(mt));
-        const float m_new = fmaxf(m_run, mt);
-        float ts = 0.0f;
+            for (int v = 2; v < 16; ++v) mt = fmaxf(mt, s[v]);
+            mt = fmaxf(mt, lane_xor<32>(mt));
+            const float m_new = fmaxf(m_run, mt);
+            float ts = 0.0f;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) ts += fast_exp2(s[v] - m_new);
-        l_run = l_run * fast_exp2(m_run - m_new) + ts;
-        m_run = m_new;
-    }
-    const float l_tot = l_run + lane_xor<32>(l_run);
-    const float L = l_tot > 0.0f ? m_run + __builtin_amdgcn_logf(l_tot) : NO_ROW;   // v_log_f32 is log2
-    if (half == 0) {
-        lse[(bh * QT + qt) * 32 + l32] = L;
-        dsum[(bh * QT + qt) * 32 + l32] = D;
+            for (int v = 0; v < 16; ++v) ts += fast_exp2(s[v] - m_new);
+            l_run = l_run * fast_exp2(m_run - m_new) + ts;
+            m_run = m_new;
+        }
+        const float l_tot = l_run + lane_xor<32>(l_run);
+        L = l_tot > 0.0f ? m_run + __builtin_amdgcn_logf(l_tot) : NO_ROW;   // v_log_f32 is log2
+        if (half == 0) {
+            lse[(bh * QT + qt) * 32 + l32] = L;
+            dsum[(bh * QT + qt) * 32 + l32] = D;
+        }
+    } else {
+        L = lse[(bh * QT + qt) * 32 + l32];
     }
 
     // second walk: dq^T += k^T . dS^T
@@ -203,13 +228,16 @@ __global__ __launch_bounds__(256) void attention_bwd_dq_kernel(
     }
     const int q = qt * 32 + l32;
     if (q < Nq) {
-        T* o = dq + (bh * Nq + q) * (32 * DP) + 4 * half;
+        T* o = dq + (long)b2 * om.s_b + (long)h * om.s_h + (long)q * om.s_n + 4 * half;
 #pragma unroll
         for (int p = 0; p < DP; ++p)
 #pragma unroll
-            for (int g = 0; g < 4; ++g)
+            for (int g = 0; g < 4; ++g) {
+                float f[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[32 * p + 8 * g + e] = DT<T>::from_f(acc[p][4 * g + e] * dq_scale);
+                for (int e = 0; e < 4; ++e) f[e] = acc[p][4 * g + e] * dq_scale;
+                store4(o + 32 * p + 8 * g, f);
+            }
     }
 }
 
@@ -220,7 +248,7 @@ __global__ __launch_bounds__(256) void attention_bwd_dkv_kernel(
     const T* __restrict__ q_acc, const T* __restrict__ k_qk, const T* __restrict__ v_qk, const T* __restrict__ bias_t,
     const float* __restrict__ keybias, const T* __restrict__ do_qk, const T* __restrict__ do_acc,
     const float* __restrict__ lse, const float* __restrict__ dsum, int B2, int H, int Nq, int Nk, float dk_scale,
-    long part_q, long part_k) {
+    long part_q, long part_k, OutMap om, int bias_pad) {
     typedef Mma<T> MM;
     typedef typename MM::Frag Frag;
     constexpr int NF = 16 / MM::KLANE;
@@ -268,7 +296,7 @@ __global__ __launch_bounds__(256) void attention_bwd_dkv_kernel(
         }
         if (bias_t) {                                                           // S += I . bias (rows = queries)
             Tile16<T> bc;
-            bc.load(bias_t + ((((long)h * QT + qt) * KT + kt) << 10) + lane * 16);
+            bc.load(bias_t + ((((long)h * QT + qt) * (KT + bias_pad) + kt) << 10) + lane * 16);
 #pragma unroll
             for (int i = 0; i < NF; ++i) MM::mma(s, ident[i], bc.frag(i));
         }
@@ -304,17 +332,20 @@ __global__ __launch_bounds__(256) void attention_bwd_dkv_kernel(
         }
     }
     if (key < Nk) {
-        T* ok = dk + (bh * Nk + key) * (32 * DP) + 4 * half;
-        T* ov = dv + (bh * Nk + key) * (32 * DP) + 4 * half;
+        const long o = (long)b2 * om.s_b + (long)h * om.s_h + (long)key * om.s_n + 4 * half;
 #pragma unroll
         for (int pp = 0; pp < DP; ++pp)
 #pragma unroll
-            for (int g = 0; g < 4; ++g)
+            for (int g = 0; g < 4; ++g) {
+                float fk[4], fv[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    ok[32 * pp + 8 * g + e] = DT<T>::from_f(acc_k[pp][4 * g + e] * dk_scale);
-                    ov[32 * pp + 8 * g + e] = DT<T>::from_f(acc_v[pp][4 * g + e]);
+                    fk[e] = acc_k[pp][4 * g + e] * dk_scale;
+                    fv[e] = acc_v[pp][4 * g + e];
                 }
+                store4(dk + o + 32 * pp + 8 * g, fk);
+                store4(dv + o + 32 * pp + 8 * g, fv);
+            }
     }
 }
 
@@ -325,7 +356,7 @@ __global__ __launch_bounds__(256) void attention_bwd_dbias_kernel(
     float* __restrict__ dbias, const T* __restrict__ q_qk, const T* __restrict__ k_qk, const T* __restrict__ v_qk,
     const T* __restrict__ bias_t, const float* __restrict__ keybias, const T* __restrict__ do_qk,
     const float* __restrict__ lse, const float* __restrict__ dsum, int B2, int H, int Nq, int Nk, int NS,
-    long part_q, long part_k) {
+    long part_q, long part_k, int bias_pad, int partial) {
     typedef Mma<T> MM;
     typedef typename MM::Frag Frag;
     constexpr int NF = 16 / MM::KLANE;
@@ -344,7 +375,7 @@ __global__ __launch_bounds__(256) void attention_bwd_dbias_kernel(
 #pragma unroll
     for (int i = 0; i < NF; ++i) ident[i] = identity_frag<T>(i, l32, half);
     Tile16<T> bc;
-    bc.load(bias_t + ((((long)h * QT + qt) * KT + kt) << 10) + lane * 16);
+    bc.load(bias_t + ((((long)h * QT + qt) * (KT + bias_pad) + kt) << 10) + lane * 16);
     f32x16 sb;                                                  // the bias tile in accumulator order, once
 #pragma unroll
     for (int v = 0; v < 16; ++v) sb[v] = 0.0f;
@@ -389,49 +420,56 @@ __global__ __launch_bounds__(256) void attention_bwd_dbias_kernel(
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const int qrow = qt * 32 + acc_row(v, lane);
-            if (qrow < Nq) atomicAdd(dbias + ((long)h * Nq + qrow) * Nk + key, acc[v]);
+            if (qrow >= Nq) continue;
+            if (partial) dbias[(((long)slice * H + h) * Nq + qrow) * Nk + key] = acc[v];
+            else atomicAdd(dbias + ((long)h * Nq + qrow) * Nk + key, acc[v]);
         }
     }
 }
 
-template <typename T, int DP>
+// Slices of the batch rows of the pair-bias gradient: enough for ~ 8 waves per SIMD, at least 8 rows each.
+long dbias_slices(long B2, long H, long QT, long KT) {
+    const long tiles = H * QT * KT;
+    long ns = (8L * 1024 + tiles - 1) / tiles;
+    if (ns > (B2 + 7) / 8) ns = (B2 + 7) / 8;
+    return ns < 1 ? 1 : ns;
+}
+
+template <typename T, int DP, bool STATS>
 int launch_bwd(void* dq, void* dk, void* dv, float* dbias, float* lse, float* dsum, const void* q_qk, const void* q_acc,
                const void* k_qk, const void* k_acc, const void* v_qk, const void* bias_t,
                const float* keybias, const void* do_qk, const void* do_acc, const void* o_qk, long B2, long H, long Nq,
-               long Nk, float dq_scale, float dk_scale, hipStream_t st) {
+               long Nk, float dq_scale, float dk_scale, OutMap mq, OutMap mk, int bias_pad, long dbias_parts, hipStream_t st) {
     const long QT = (Nq + 31) / 32, KT = (Nk + 31) / 32;
     const long part_q = B2 * H * QT * 1024, part_k = B2 * H * KT * 1024;
     const long g1 = 8 * ((B2 * H * QT + 31) / 32), g2 = 8 * ((B2 * H * KT + 31) / 32);      // blocks of four waves, a multiple of 8
     FFK_REQUIRE(g1 < (1L << 31) && g2 < (1L << 31), FFK_ERR_SHAPE, "ffk_attention_bwd: too many tiles for one launch");
     if (bias_t) {
-        attention_bwd_dq_kernel<T, DP, true><<<(unsigned)g1, 256, 0, st>>>((T*)dq, lse, dsum, (const T*)q_qk, (const T*)k_qk,
-                                                                         (const T*)k_acc, (const T*)v_qk, (const T*)bias_t, keybias,
-                                                                         (const T*)do_qk, (const T*)o_qk, (int)B2, (int)H, (int)Nq,
-                                                                         (int)Nk, dq_scale, part_q, part_k);
+        attention_bwd_dq_kernel<T, DP, true, STATS><<<(unsigned)g1, 256, 0, st>>>((T*)dq, lse, dsum, (const T*)q_qk, (const T*)k_qk,
+                                                                                (const T*)k_acc, (const T*)v_qk, (const T*)bias_t, keybias,
+                                                                                (const T*)do_qk, (const T*)o_qk, (int)B2, (int)H, (int)Nq,
+                                                                                (int)Nk, dq_scale, part_q, part_k, mq, bias_pad);
     } else {
-        attention_bwd_dq_kernel<T, DP, false><<<(unsigned)g1, 256, 0, st>>>((T*)dq, lse, dsum, (const T*)q_qk, (const T*)k_qk,
-                                                                          (const T*)k_acc, (const T*)v_qk, nullptr, keybias,
-                                                                          (const T*)do_qk, (const T*)o_qk, (int)B2, (int)H, (int)Nq,
-                                                                          (int)Nk, dq_scale, part_q, part_k);
+        attention_bwd_dq_kernel<T, DP, false, STATS><<<(unsigned)g1, 256, 0, st>>>((T*)dq, lse, dsum, (const T*)q_qk, (const T*)k_qk,
+                                                                                 (const T*)k_acc, (const T*)v_qk, nullptr, keybias,
+                                                                                 (const T*)do_qk, (const T*)o_qk, (int)B2, (int)H, (int)Nq,
+                                                                                 (int)Nk, dq_scale, part_q, part_k, mq, 0);
     }
     int rc = ffk_check_launch("ffk_attention_bwd");
     if (rc != FFK_OK) return rc;
     attention_bwd_dkv_kernel<T, DP><<<(unsigned)g2, 256, 0, st>>>((T*)dk, (T*)dv, (const T*)q_qk, (const T*)q_acc,
                                                                 (const T*)k_qk, (const T*)v_qk, (const T*)bias_t, keybias,
                                                                 (const T*)do_qk, (const T*)do_acc, lse, dsum, (int)B2, (int)H,
-                                                                (int)Nq, (int)Nk, dk_scale, part_q, part_k);
+                                                                (int)Nq, (int)Nk, dk_scale, part_q, part_k, mk, bias_pad);
     rc = ffk_check_launch("ffk_attention_bwd");
     if (rc != FFK_OK || !dbias) return rc;
-    // enough slices of the batch rows for ~ 8 waves per SIMD, at least 8 rows per slice
-    const long tiles = H * QT * KT;
-    long ns = (8L * 1024 + tiles - 1) / tiles;
-    if (ns > (B2 + 7) / 8) ns = (B2 + 7) / 8;
-    if (ns < 1) ns = 1;
-    const long g3 = 8 * ((ns * tiles + 31) / 32);
+    const long ns = dbias_parts > 0 ? dbias_parts : dbias_slices(B2, H, QT, KT);
+    const long g3 = 8 * ((ns * H * QT * KT + 31) / 32);
     FFK_REQUIRE(g3 < (1L << 31), FFK_ERR_SHAPE, "ffk_attention_bwd: too many tiles for one launch");
     attention_bwd_dbias_kernel<T, DP><<<(unsigned)g3, 256, 0, st>>>(dbias, (const T*)q_qk, (const T*)k_qk, (const T*)v_qk,
                                                                   (const T*)bias_t, keybias, (const T*)do_qk, lse, dsum,
-                                                                  (int)B2, (int)H, (int)Nq, (int)Nk, (int)ns, part_q, part_k);
+                                                                  (int)B2, (int)H, (int)Nq, (int)Nk, (int)ns, part_q, part_k, bias_pad,
+                                                                  dbias_parts > 0 ? 1 : 0);
     return ffk_check_launch("ffk_attention_bwd");
 }
 
@@ -455,16 +493,45 @@ extern "C" int ffk_attention_bwd(void* dq, void* dk, void* dv, float* dbias, flo
                     ffk_aligned16(o_qk) && (!bias_t || ffk_aligned16(bias_t)),
                 FFK_ERR_ALIGN, "ffk_attention_bwd: buffers must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
+    const OutMap mq = {H * Nq * D, Nq * D, D}, mk = {H * Nk * D, Nk * D, D};
 #define FFK_BWD_ARGS dq, dk, dv, dbias, lse, dsum, q_qk, q_acc, k_qk, k_acc, v_qk, bias_t, keybias, do_qk, do_acc, o_qk, \
-                     B2, H, Nq, Nk, dq_scale, dk_scale, st
+                     B2, H, Nq, Nk, dq_scale, dk_scale, mq, mk, 0, 0, st
     switch (dtype) {
         case FFK_BF16:
-            return D == 32 ? launch_bwd<bf16_t, 1>(FFK_BWD_ARGS)
-                           : (D == 64 ? launch_bwd<bf16_t, 2>(FFK_BWD_ARGS) : launch_bwd<bf16_t, 4>(FFK_BWD_ARGS));
+            return D == 32 ? launch_bwd<bf16_t, 1, true>(FFK_BWD_ARGS)
+                           : (D == 64 ? launch_bwd<bf16_t, 2, true>(FFK_BWD_ARGS) : launch_bwd<bf16_t, 4, true>(FFK_BWD_ARGS));
         case FFK_F32:
-            return D == 32 ? launch_bwd<float, 1>(FFK_BWD_ARGS)
-                           : (D == 64 ? launch_bwd<float, 2>(FFK_BWD_ARGS) : launch_bwd<float, 4>(FFK_BWD_ARGS));
+            return D == 32 ? launch_bwd<float, 1, true>(FFK_BWD_ARGS)
+                           : (D == 64 ? launch_bwd<float, 2, true>(FFK_BWD_ARGS) : launch_bwd<float, 4, true>(FFK_BWD_ARGS));
         default: return ffk_fail(FFK_ERR_DTYPE, "ffk_attention_bwd: unsupported dtype tag %d", dtype);
     }
 #undef FFK_BWD_ARGS
+}
+
+extern "C" int ffk_attention_bwd_rows(void* dq, void* dk, void* dv, float* dbias, int64_t dbias_parts, const float* lse,
+                                      const float* dsum, const void* q_t, const void* q_v, const void* k_t, const void* k_v,
+                                      const void* v_t, const void* bias_t, const float* keybias, const void* do_t, const void* do_v,
+                                      int64_t B2, int64_t H, int64_t N, int64_t s_b, int64_t s_h, int64_t s_n, float dq_scale,
+                                      float dk_scale, int flags, int dtype, void* stream) {
+    FFK_REQUIRE(dq && dk && dv && lse && dsum && q_t && q_v && k_t && k_v && v_t && keybias && do_t && do_v, FFK_ERR_NULL,
+                "ffk_attention_bwd_rows: null pointer");
+    FFK_REQUIRE(!dbias || (bias_t && dbias_parts > 0 && dbias_parts <= B2), FFK_ERR_NULL,
+                "ffk_attention_bwd_rows: dbias needs bias_t and a number of partial sums between 1 and B2");
+    FFK_REQUIRE(B2 > 0 && B2 < 131072 && H > 0 && H < 65536 && N > 0 && N < (1 << 24), FFK_ERR_SHAPE,
+                "ffk_attention_bwd_rows: bad shape B2=%ld H=%ld N=%ld", (long)B2, (long)H, (long)N);
+    for (const void* p : {(const void*)dq, (const void*)dk, (const void*)dv, (const void*)lse, (const void*)dsum, q_t, q_v, k_t, k_v,
+                          v_t, bias_t, (const void*)keybias, do_t, do_v})
+        FFK_REQUIRE(ffk_aligned16(p), FFK_ERR_ALIGN, "ffk_attention_bwd_rows: buffers must be 16-byte aligned");
+    FFK_REQUIRE(s_b % 4 == 0 && s_h % 4 == 0 && s_n % 4 == 0, FFK_ERR_ALIGN, "ffk_attention_bwd_rows: strides must be multiples of 4 elements");
+    const OutMap om = {s_b, s_h, s_n};
+    const int pad = (flags & FFK_ATT_BIAS_PADDED) ? 1 : 0;
+    hipStream_t st = (hipStream_t)stream;
+    // with the statistics given neither is written
+    switch (dtype) {
+        case FFK_BF16: return launch_bwd<bf16_t, 1, false>(dq, dk, dv, dbias, (float*)lse, (float*)dsum, q_t, q_v, k_t, k_v, v_t, bias_t,
+                                                           keybias, do_t, do_v, nullptr, B2, H, N, N, dq_scale, dk_scale, om, om, pad, dbias_parts, st);
+        case FFK_F32: return launch_bwd<float, 1, false>(dq, dk, dv, dbias, (float*)lse, (float*)dsum, q_t, q_v, k_t, k_v, v_t, bias_t,
+                                                         keybias, do_t, do_v, nullptr, B2, H, N, N, dq_scale, dk_scale, om, om, pad, dbias_parts, st);
+        default: return ffk_fail(FFK_ERR_DTYPE, "ffk_attention_bwd_rows: unsupported dtype tag %d", dtype);
+    }
 }

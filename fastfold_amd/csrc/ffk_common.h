@@ -177,6 +177,8 @@ __device__ __forceinline__ float sigmoid_f(float x) {
     // 1 / (1 + 2^(-x*log2e))
     return fast_rcp(1.0f + fast_exp2(-1.4426950408889634f * x));
 }
+// factor of a tile's gate operand: the gate itself, or 1 where it is positive (FFK_ACT_GATE_POS)
+__device__ __forceinline__ float gate_factor(float g, int act) { return act == FFK_ACT_GATE_POS ? (g > 0.0f ? 1.0f : 0.0f) : g; }
 template <typename T> __device__ __forceinline__ float exp_for(float x);
 template <> __device__ __forceinline__ float exp_for<float>(float x) { return expf(x); }
 template <> __device__ __forceinline__ float exp_for<bf16_t>(float x) { return fast_exp2(1.4426950408889634f * x); }

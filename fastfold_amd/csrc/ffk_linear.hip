@@ -370,7 +370,7 @@ __global__ __launch_bounds__(THREADS, 4) void fused_linear_kernel(const LinArgs 
                     if (gate) {
 #pragma unroll
                         for (int e = 0; e < VEC; ++e)
-                            x[j].e[e] = DT<T>::from_f(DT<T>::to_f(x[j].e[e]) * DT<T>::to_f(gv[j].e[e]));
+                            x[j].e[e] = DT<T>::from_f(DT<T>::to_f(x[j].e[e]) * gate_factor(DT<T>::to_f(gv[j].e[e]), t.act));
                     }
                     if constexpr (XS_OK) {
                         if (xtail) {
@@ -410,7 +410,7 @@ __global__ __launch_bounds__(THREADS, 4) void fused_linear_kernel(const LinArgs 
                     } else {
                         oo = tab.off[r] + (long)(c >> 5) * t.s_h + (c & 31);
                     }
-                    if (gate) y = DT<T>::to_f(DT<T>::from_f(y * DT<T>::to_f(gate[(t.gate_rows > 0 ? (m0 + r) % t.gate_rows : (m0 + r)) * t.gate_ld + c])));
+                    if (gate) y = DT<T>::to_f(DT<T>::from_f(y * gate_factor(DT<T>::to_f(gate[(t.gate_rows > 0 ? (m0 + r) % t.gate_rows : (m0 + r)) * t.gate_ld + c]), t.act)));
                     if constexpr (XS_OK) {
                         if (xtail) {
                             xs_round(y + xs_value(resid[oo], xtail[oo]), &out[oo], &xtail[oo]);

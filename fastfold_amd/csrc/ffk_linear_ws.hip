@@ -116,7 +116,7 @@ __device__ __forceinline__ void unpack8(const T* p, float* f) {
 // STRIDED tiles: weight rows were loaded through tau, registers hold channels 16*half + v.
 // ACC / QK tiles: natural weight order, registers hold channels 8a + 4*half + b.
 // sb: this slot's 32 (GLU: 64) bias values in LDS (fp32); rmask: the row's mask value.
-template <bool GLU, bool XT>
+template <bool GLU, bool XT, bool POS>
 __device__ __forceinline__ void ws_store_rows_compact(const WsSlot& t, const f32x16& acc, const f32x16& accg, const float* sb,
                                               bool valid, unsigned mc, unsigned hi, unsigned lo, float rmask, int half) {
     const bool strided = t.kind == FFK_TILE_STRIDED;
@@ -196,7 +196,7 @@ __device__ __forceinline__ void ws_store_rows_compact(const WsSlot& t, const f32
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
                         float u = (float)y[8 * j + e];
-                        if (gate) u = (float)(T)(u * (float)reinterpret_cast<const T*>(&gv[j])[e]);
+                        if (gate) u = (float)(T)(u * gate_factor((float)reinterpret_cast<const T*>(&gv[j])[e], POS ? t.act : FFK_ACT_NONE));
                         f[e] += u;
                     }
                     u32x4 hv;
@@ -216,7 +216,7 @@ __device__ __forceinline__ void ws_store_rows_compact(const WsSlot& t, const f32
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     float f = (float)y[8 * j + e];
-                    if (gate) f = (float)(T)(f * (float)gh[e]);
+                    if (gate) f = (float)(T)(f * gate_factor((float)gh[e], POS ? t.act : FFK_ACT_NONE));
                     if (resid) f += (float)rh[e];
                     y[8 * j + e] = (T)f;
                 }
@@ -377,7 +377,7 @@ __device__ __forceinline__ void ws_store_rows(const WsSlot& t, const f32x16& acc
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
                         float u = (float)y[8 * j + e];
-                        if (gate) u = (float)(T)(u * (float)reinterpret_cast<const T*>(&gv[j])[e]);
+                        if (gate) u = (float)(T)(u * gate_factor((float)reinterpret_cast<const T*>(&gv[j])[e], t.act));
                         f[e] += u;
                     }
                     u32x4 hv;
@@ -397,7 +397,7 @@ __device__ __forceinline__ void ws_store_rows(const WsSlot& t, const f32x16& acc
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     float f = (float)y[8 * j + e];
-                    if (gate) f = (float)(T)(f * (float)gh[e]);
+                    if (gate) f = (float)(T)(f * gate_factor((float)gh[e], t.act));
                     if (resid) f += (float)rh[e];
                     y[8 * j + e] = (T)f;
                 }
@@ -572,6 +572,7 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
     constexpr int WS_KS = G::KS, WS_AP = G::AP, WS_BM = G::BM, WS_RG = G::RG, LPR = G::LPR, RPP = G::RPP;
     constexpr bool ALLOW_GLU = NS >= 2 && WS_K <= 128;
     constexpr bool LEAN = NS == 2 && WS_K <= 128 && !DUAL;   // straight-line epilogues where the registers allow them
+    constexpr bool POS = NS == 2 && !XT;                   // variants that take FFK_ACT_GATE_POS (the others have no register for it)
     constexpr int AFC = WS_K == 128 ? 8 : 4;               // A fragments held at a time (register budget)
     const ffk_linear_desc& d = args.d;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -1083,8 +1084,8 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
                             }
                             ws_store_rows_folded<XT>(t, acc, accg, sb, s_c1 + s_wrow[s], rstd, -rstd * mean, rstd_g, -rstd_g * mean_g,
                                                  valid, c_hi, c_lo, half, a2r, a2v, n32 & 15);
-                        } else if (ALLOW_GLU && glu) ws_store_rows_compact<true, XT>(t, acc, accg, sb, valid, mc, c_hi, c_lo, rmask, half);
-                        else ws_store_rows_compact<false, XT>(t, acc, accg, sb, valid, mc, c_hi, c_lo, rmask, half);
+                        } else if (ALLOW_GLU && glu) ws_store_rows_compact<true, XT, POS>(t, acc, accg, sb, valid, mc, c_hi, c_lo, rmask, half);
+                        else ws_store_rows_compact<false, XT, POS>(t, acc, accg, sb, valid, mc, c_hi, c_lo, rmask, half);
                     } else {
                         const float* sm = t.masked ? smk : nullptr;
                         if (ALLOW_GLU && glu) ws_store_cols_compact<true>(t, acc, accg, sb, sm, m0g, M, l32, half);
@@ -1268,6 +1269,8 @@ int ffk_linear_ws_try(const ffk_linear_desc* d, hipStream_t st, int* status) {
             return 0;
     }
     if (bias_tile >= 0 && (tails || chan_major)) return 0;   // built into the plain K = 128 variants only
+    for (int i = 0; i < n_slot_tiles; ++i)
+        if (d->tiles[i].act == FFK_ACT_GATE_POS && (tails || args.plan.max_slots > 2)) return 0;
     if (k256) {
         for (int i = 0; i < d->n_tiles; ++i)
             if (d->tiles[i].glu) return 0;                   // GLU units are only built for K = 128

@@ -60,6 +60,17 @@ const OpEntry OPS[] = {
     args_op<ffk_global_attention_core>(),
     args_op<ffk_layernorm_fwd>(),
     args_op<ffk_fill_zero>(),
+    args_op<ffk_attention_fwd_lse>(),
+    args_op<ffk_attention_bwd_rows>(),
+    args_op<ffk_transpose_batched>(),
+    args_op<ffk_weight_grad>(),
+    args_op<ffk_layernorm_bwd_rows>(),
+    args_op<ffk_scale_rows>(),
+    args_op<ffk_att_gate_bwd>(),
+    args_op<ffk_trimul_gate_bwd>(),
+    args_op<ffk_glu_bwd>(),
+    args_op<ffk_bias_cols>(),
+    args_op<ffk_slice_sum>(),
 };
 constexpr int N_OPS = (int)(sizeof(OPS) / sizeof(OPS[0]));
 static_assert(N_OPS == FFK_OP_COUNT, "one entry per operation code");

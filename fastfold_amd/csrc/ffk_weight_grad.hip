@@ -1,0 +1,325 @@
+// Weight gradients (see ffk_weight_grad in include/ffk.h):  out[n][k] = sum_m y[m][n] x[m][k]  and the column sums of y,
+// for activations of 10^4 .. 10^6 rows and weights of a few hundred rows and columns.
+//
+// The product contracts over the rows of two row-major operands, and its output alone (a few 128 x 128 tiles) cannot fill
+// the chip: the rows are cut into slices, one workgroup multiplies one slice for one output tile into fp32 accumulators and
+// leaves them in a workspace, and a second launch adds the slices in a fixed order (no atomics: the same gradients every
+// time) and rounds once.  Workgroups are ordered slice by slice and each XCD takes a contiguous part of that order, so the
+// tiles that read the same rows run behind one L2.
+//
+//   bf16   v_mfma_f32_32x32x16_bf16 wants eight consecutive rows of one column per lane.  A thread fetches an 8 x 8 block
+//          (eight 16-byte loads, whole 256-byte row pieces per 16 lanes), transposes it in registers (32 byte permutes) and
+//          stores eight columns of eight rows; in LDS a column is 64 rows = 128 bytes, its eight 16-byte chunks XOR-swizzled
+//          with the column index so that neither the stores (columns 8 apart) nor the fragment reads (adjacent columns) meet
+//          in one bank group.  The permutes cost a fifth of the MFMA time.
+//   fp32   v_mfma_f32_32x32x2_f32 takes one element per lane: rows stay as they are.
+// Bound: the reads of y and x (from HBM or the last-level cache).  65 536 x 640 by 65 536 x 128, bf16: library slab GEMM +
+// reduction 75 + 24 us, this pair 29 + 6 us.
+#include "ffk_common.h"
+#include <type_traits>
+
+namespace {
+
+constexpr int WG_THREADS = 256;
+constexpr int WG_T = 128;                   // output tile: 128 columns of y by 128 columns of x
+
+struct WgArgs {
+    const void* y;
+    const void* x;
+    float* part;                            // [slices][N * K]
+    float* csum;                            // [slices][N], or nullptr
+    long y_so, y_si, x_so, x_si;
+    unsigned y_inner, x_inner;
+    int M, N, K, slices, rows_per_slice;    // rows_per_slice: a multiple of 64
+};
+
+__device__ __forceinline__ long wg_row(unsigned m, unsigned inner, long so, long si, bool flat) {
+    const unsigned hi = flat ? 0u : m / inner;
+    return (long)hi * so + (long)(m - hi * inner) * si;
+}
+
+template <typename T>
+__global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs a) {
+    constexpr bool BF = std::is_same<T, bf16_t>::value;
+    constexpr int MB = BF ? 64 : 32;                       // rows per step
+    constexpr int BUF = BF ? WG_T * 128 : MB * 640;        // bytes of one operand's buffer
+    constexpr int NP = BF ? 8 : 4;                         // 16-byte loads per thread and step
+    extern __shared__ __align__(16) unsigned char smem[];  // [2 buffers][y | x]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, half = lane >> 5;
+    const int tn = (a.N + WG_T - 1) / WG_T, tk = (a.K + WG_T - 1) / WG_T;
+    const unsigned per_xcd = gridDim.x >> 3;
+    const unsigned item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (item >= (unsigned)(tn * tk) * (unsigned)a.slices) return;
+    const int n0 = (int)(item % tn) * WG_T, k0 = (int)((item / tn) % tk) * WG_T, slice = (int)(item / (tn * tk));
+    const int m_begin = slice * a.rows_per_slice;
+    const int m_end = m_begin + a.rows_per_slice < a.M ? m_begin + a.rows_per_slice : a.M;
+    const bool y_flat = a.y_inner >= (unsigned)a.M, x_flat = a.x_inner >= (unsigned)a.M;
+
+    // bf16: threads 0 .. 127 fetch y, 128 .. 255 x, an 8 x 8 block each.  fp32: every thread half of its vectors from each.
+    Vec16<T> pre[NP * (BF ? 1 : 2)];
+    const int bt = BF ? (tid & 127) : tid;
+    const int cb = BF ? (bt & 15) : (bt & 31);             // column block (8 or 4 columns)
+    const int rb = BF ? (bt >> 4) : (bt >> 5);             // row block
+    const bool is_x = BF && tid >= 128;
+    auto fetch = [&](int m0) {
+        if constexpr (BF) {
+            const T* base = (const T*)(is_x ? a.x : a.y);
+            int col = (is_x ? k0 : n0) + cb * 8;
+            const int cols = is_x ? a.K : a.N;
+            col = col < cols ? col : cols - 8;             // clamped columns are never stored
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int m = m0 + rb * 8 + e;
+                const unsigned mc = (unsigned)(m < m_end ? m : m_end - 1);
+                const long off = is_x ? wg_row(mc, a.x_inner, a.x_so, a.x_si, x_flat) : wg_row(mc, a.y_inner, a.y_so, a.y_si, y_flat);
+                pre[e] = ld16(base + off + col);
+                if (m >= m_end && !is_x) pre[e] = Vec16<T>{};        // rows past the end add nothing
+            }
+        } else {
+            int cy = n0 + cb * 4, cx = k0 + cb * 4;
+            cy = cy < a.N ? cy : a.N - 4;
+            cx = cx < a.K ? cx : a.K - 4;
+#pragma unroll
+            for (int e = 0; e < NP; ++e) {
+                const int m = m0 + rb + 8 * e;
+                const unsigned mc = (unsigned)(m < m_end ? m : m_end - 1);
+                pre[e] = ld16((const T*)a.y + wg_row(mc, a.y_inner, a.y_so, a.y_si, y_flat) + cy);
+                pre[NP + e] = ld16((const T*)a.x + wg_row(mc, a.x_inner, a.x_so, a.x_si, x_flat) + cx);
+                if (m >= m_end) pre[e] = Vec16<T>{};
+            }
+        }
+    };
+    auto commit = [&](int buf) {
+        unsigned char* sb = smem + buf * 2 * BUF;
+        if constexpr (BF) {
+            unsigned char* so = sb + (is_x ? BUF : 0);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {                  // columns 2 d and 2 d + 1 of the block
+                u32x4 lo, hi;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t r0 = reinterpret_cast<const u32x4*>(&pre[2 * j])[0][d], r1 = reinterpret_cast<const u32x4*>(&pre[2 * j + 1])[0][d];
+                    lo[j] = __builtin_amdgcn_perm(r1, r0, 0x05040100u);
+                    hi[j] = __builtin_amdgcn_perm(r1, r0, 0x07060302u);
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int n = cb * 8 + 2 * d + h;
+                    *reinterpret_cast<u32x4*>(so + n * 128 + (((rb ^ n ^ (n >> 3)) & 7) << 4)) = h ? hi : lo;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < NP; ++e) {
+                *reinterpret_cast<Vec16<T>*>(sb + (rb + 8 * e) * 640 + cb * 16) = pre[e];
+                *reinterpret_cast<Vec16<T>*>(sb + BUF + (rb + 8 * e) * 640 + cb * 16) = pre[NP + e];
+            }
+        }
+    };
+
+    const int wn = wave >> 1, wk = wave & 1;               // the wave's 64 x 64 quarter of the tile
+    const bool sums = a.csum != nullptr && k0 == 0 && wk == 0;
+    float cs[2] = {0.0f, 0.0f};
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+
+    fetch(m_begin);
+    commit(0);
+    lds_barrier();
+    int buf = 0;
+    for (int m0 = m_begin; m0 < m_end; m0 += MB) {
+        const bool more = m0 + MB < m_end;
+        if (more) fetch(m0 + MB);                          // in flight during the products
+        const unsigned char* sy = smem + buf * 2 * BUF;
+        const unsigned char* sx = sy + BUF;
+        if constexpr (BF) {
+#pragma unroll
+            for (int ks = 0; ks < MB / 16; ++ks) {
+                bf16x8 fy[2], fx[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int n = wn * 64 + i * 32 + l32, k = wk * 64 + i * 32 + l32;
+                    fy[i] = *reinterpret_cast<const bf16x8*>(sy + n * 128 + ((((2 * ks + half) ^ n ^ (n >> 3)) & 7) << 4));
+                    fx[i] = *reinterpret_cast<const bf16x8*>(sx + k * 128 + ((((2 * ks + half) ^ k ^ (k >> 3)) & 7) << 4));
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) Mma<bf16_t>::mma(acc[i][j], fy[i], fx[j]);
+                if (sums) {
+                    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+                    const bf16x2 ones = {(bf16_t)1.0f, (bf16_t)1.0f};
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const bf16x2 pr = {fy[i][2 * e], fy[i][2 * e + 1]};
+                            cs[i] = __builtin_amdgcn_fdot2_f32_bf16(pr, ones, cs[i], false);
+                        }
+                }
+            }
+        } else {
+#pragma unroll 4
+            for (int ks = 0; ks < MB / 2; ++ks) {
+                float fy[2], fx[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    fy[i] = *reinterpret_cast<const float*>(sy + (2 * ks + half) * 640 + (wn * 64 + i * 32 + l32) * 4);
+                    fx[i] = *reinterpret_cast<const float*>(sx + (2 * ks + half) * 640 + (wk * 64 + i * 32 + l32) * 4);
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fy[i], fx[j], acc[i][j], 0, 0, 0);
+                if (sums) {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) cs[i] += fy[i];
+                }
+            }
+        }
+        if (!more) break;
+        commit(buf ^ 1);                                   // the other buffer: its last readers passed the barrier below
+        lds_barrier();
+        buf ^= 1;
+    }
+    float* part = a.part + (long)slice * a.N * a.K;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int k = k0 + wk * 64 + j * 32 + l32;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int n = n0 + wn * 64 + i * 32 + acc_row(v, lane);
+                if (n < a.N && k < a.K) part[(long)n * a.K + k] = acc[i][j][v];
+            }
+        }
+    if (sums) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float s = cs[i] + lane_xor<32>(cs[i]);
+            const int n = n0 + wn * 64 + i * 32 + l32;
+            if (half == 0 && n < a.N) a.csum[(long)slice * a.N + n] = s;
+        }
+    }
+}
+
+// sum over the slices of part[s][i], plus acc[i] if READ: to acc[i] if WRITE, else to out.  Four adjacent values per lane, the
+// slices spread over the four waves.  Element i = (row n, column k) of out is at (n / inner) * o_so + (n % inner) * o_si + k * o_sk.
+template <typename OT>
+__global__ __launch_bounds__(256) void slice_sum_kernel(OT* __restrict__ out, const float* __restrict__ part, float* acc, int flags,
+                                                        int slices, long n, int K, unsigned inner, long o_so, long o_si, long o_sk,
+                                                        long pitch) {
+    __shared__ f32x4 red[3][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const long i = ((long)blockIdx.x * 64 + lane) * 4;
+    f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (i < n) {
+#pragma unroll 4
+        for (int sl = wave; sl < slices; sl += 4) s += *reinterpret_cast<const f32x4*>(part + (long)sl * pitch + i);
+    }
+    if (wave) red[wave - 1][lane] = s;
+    __syncthreads();
+    if (wave || i >= n) return;
+    s = (s + red[0][lane]) + (red[1][lane] + red[2][lane]);
+    if (flags & FFK_WGRAD_READ) s += *reinterpret_cast<const f32x4*>(acc + i);
+    if (flags & FFK_WGRAD_WRITE) {
+        *reinterpret_cast<f32x4*>(acc + i) = s;
+        return;
+    }
+    const unsigned row = (unsigned)(i / K), k = (unsigned)(i - (long)row * K), hi = row / inner;      // K % 4 == 0
+    OT* o = out + (long)hi * o_so + (long)(row - hi * inner) * o_si + (long)k * o_sk;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e * o_sk] = DT<OT>::from_f(s[e]);
+}
+
+template <typename T>
+int slice_sum(T* out, const float* part, float* acc, int flags, long slices, long n, int K, unsigned inner, long so, long si, long sk,
+              long pitch, hipStream_t st) {
+    slice_sum_kernel<T><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(out, part, acc, flags, (int)slices, n, K, inner, so, si, sk, pitch);
+    return ffk_check_launch("ffk_weight_grad");
+}
+
+template <typename T>
+int launch_weight_grad(const WgArgs& a, void* out, long n_out, void* colsum, long cs_first, long cs_count, float* acc, long o_inner, long o_so, long o_si, long o_sk, int flags,
+                       hipStream_t st) {
+    const size_t smem = std::is_same<T, bf16_t>::value ? 4 * (size_t)WG_T * 128 : 4 * (size_t)32 * 640;
+    static FfkLdsReservation lds_reserved;
+    int rc = ffk_reserve_lds(lds_reserved, (const void*)weight_grad_kernel<T>, smem, "ffk_weight_grad");
+    if (rc != FFK_OK) return rc;
+    const long items = (long)ffk_cdiv(a.N, WG_T) * ffk_cdiv(a.K, WG_T) * a.slices;
+    FFK_REQUIRE(items < (1L << 31) - 8, FFK_ERR_SHAPE, "ffk_weight_grad: %ld workgroups exceed the grid limit", items);
+    weight_grad_kernel<T><<<(unsigned)(8 * ffk_cdiv(items, 8)), WG_THREADS, smem, st>>>(a);
+    rc = ffk_check_launch("ffk_weight_grad");
+    if (rc != FFK_OK) return rc;
+    const long nk = (long)a.N * a.K;
+    rc = slice_sum<T>((T*)out, a.part, acc, flags, a.slices, n_out * a.K, a.K, (unsigned)o_inner, o_so, o_si, o_sk, nk, st);
+    if (rc != FFK_OK || !a.csum) return rc;
+    return slice_sum<T>((T*)colsum, a.csum + cs_first, acc ? acc + n_out * a.K : nullptr, flags, a.slices, cs_count, (int)cs_count, 1u, 0, 0, 1,
+                        a.N, st);
+}
+
+}  // namespace
+
+extern "C" int ffk_weight_grad(void* out, int64_t n_out, void* colsum, int64_t cs_first, int64_t cs_count, float* acc, float* ws,
+                               const void* y, const void* x, int64_t M, int64_t N, int64_t K, int64_t slices, int64_t y_inner, int64_t y_so, int64_t y_si, int64_t x_inner, int64_t x_so,
+                               int64_t x_si, int64_t o_inner, int64_t o_so, int64_t o_si, int64_t o_sk, int flags, int dtype,
+                               void* stream) {
+    FFK_REQUIRE(out && ws && y && x && (acc || flags == 0), FFK_ERR_NULL, "ffk_weight_grad: null pointer");
+    FFK_REQUIRE(M > 0 && M < (1L << 31) - 128 && N > 0 && N % 8 == 0 && K > 0 && K % 8 == 0 && N < (1 << 20) && K < (1 << 20) &&
+                    slices > 0 && slices <= 65536 && y_inner > 0 && x_inner > 0 && o_inner > 0 && N * K < (1L << 32),
+                FFK_ERR_SHAPE, "ffk_weight_grad: bad shape M=%ld N=%ld K=%ld slices=%ld", (long)M, (long)N, (long)K, (long)slices);
+    FFK_REQUIRE(n_out > 0 && n_out <= N && (!colsum || (cs_first >= 0 && cs_first % 4 == 0 && cs_count > 0 && cs_count % 4 == 0 && cs_first + cs_count <= N)),
+                FFK_ERR_SHAPE, "ffk_weight_grad: rows %ld and column sums [%ld, +%ld) of %ld", (long)n_out, (long)cs_first, (long)cs_count, (long)N);
+    const int vec = dtype == FFK_F32 ? 4 : 8;
+    FFK_REQUIRE(ffk_aligned16(ws) && ffk_aligned16(acc) && ffk_aligned16(y) && ffk_aligned16(x) && y_so % vec == 0 && y_si % vec == 0 && x_so % vec == 0 &&
+                    x_si % vec == 0,
+                FFK_ERR_ALIGN, "ffk_weight_grad: operand rows must be 16-byte aligned");
+    WgArgs a;
+    a.y = y;
+    a.x = x;
+    a.part = ws;
+    a.csum = colsum ? ws + slices * N * K : nullptr;
+    a.y_so = y_so;
+    a.y_si = y_si;
+    a.x_so = x_so;
+    a.x_si = x_si;
+    a.y_inner = (unsigned)(y_inner < M ? y_inner : M);
+    a.x_inner = (unsigned)(x_inner < M ? x_inner : M);
+    a.M = (int)M;
+    a.N = (int)N;
+    a.K = (int)K;
+    a.slices = (int)slices;
+    a.rows_per_slice = (int)(((M + slices - 1) / slices + 63) / 64 * 64);
+    FFK_REQUIRE((slices - 1) * (int64_t)a.rows_per_slice < M, FFK_ERR_SHAPE,
+                "ffk_weight_grad: %ld slices of 64-row steps leave empty slices of %ld rows", (long)slices, (long)M);
+    hipStream_t st = (hipStream_t)stream;
+    switch (dtype) {
+        case FFK_BF16: return launch_weight_grad<bf16_t>(a, out, n_out, colsum, cs_first, cs_count, acc, o_inner, o_so, o_si, o_sk, flags, st);
+        case FFK_F32: return launch_weight_grad<float>(a, out, n_out, colsum, cs_first, cs_count, acc, o_inner, o_so, o_si, o_sk, flags, st);
+        default: return ffk_fail(FFK_ERR_DTYPE, "ffk_weight_grad: unsupported dtype tag %d", dtype);
+    }
+}
+
+extern "C" int ffk_slice_sum(void* out, const float* part, int64_t slices, int64_t N, int64_t K, int64_t o_inner, int64_t o_so,
+                             int64_t o_si, int64_t o_sk, int dtype, void* stream) {
+    FFK_REQUIRE(out && part, FFK_ERR_NULL, "ffk_slice_sum: null pointer");
+    FFK_REQUIRE(slices > 0 && slices <= 65536 && N > 0 && K > 0 && K % 4 == 0 && N < (1L << 31) && K < (1L << 31) && o_inner > 0 &&
+                    N * K < (1L << 38),
+                FFK_ERR_SHAPE, "ffk_slice_sum: bad shape slices=%ld N=%ld K=%ld", (long)slices, (long)N, (long)K);
+    FFK_REQUIRE(ffk_aligned16(part), FFK_ERR_ALIGN, "ffk_slice_sum: the partial sums must be 16-byte aligned");
+    hipStream_t st = (hipStream_t)stream;
+    const unsigned inner = (unsigned)(o_inner < N ? o_inner : N);
+    switch (dtype) {
+        case FFK_BF16: return slice_sum<bf16_t>((bf16_t*)out, part, nullptr, 0, slices, N * K, (int)K, inner, o_so, o_si, o_sk, N * K, st);
+        case FFK_F32: return slice_sum<float>((float*)out, part, nullptr, 0, slices, N * K, (int)K, inner, o_so, o_si, o_sk, N * K, st);
+        default: return ffk_fail(FFK_ERR_DTYPE, "ffk_slice_sum: unsupported dtype tag %d", dtype);
+    }
+}

@@ -16,6 +16,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from fastfold_amd import _plan
+from . import _backward
 from . import _fused as F_
 from .msa import MSACore
 from .ops import Linear, OutProductMean, _budget, _mask_like, _needs_grad, _no_grad_guard
@@ -47,6 +48,26 @@ class _BlockRecompute(torch.autograd.Function):
             mo, zo = ctx.block._core_train(m_, z_, *ctx.masks, drops=ctx.drops if ctx.drops is not None else {})
         torch.autograd.backward((mo, zo), (dm, dz))        # parameter gradients accumulate here, as under checkpointing
         return None, None, None, None, None, m_.grad, z_.grad
+
+
+class _BlockGrad(torch.autograd.Function):
+    """One Evoformer block as its own checkpoint, forward and backward as launch sequences (``_backward.block_backward``): the
+    forward pass keeps the two inputs and the dropout multipliers (drawn by the caller), the backward pass returns the gradients
+    of the inputs and of every parameter."""
+
+    @staticmethod
+    def forward(ctx, block, msa_mask, pair_mask, drops, m, z, *params):
+        ctx.block, ctx.masks, ctx.drops, ctx.params = block, (msa_mask, pair_mask), drops, params
+        ctx.save_for_backward(m, z)
+        return block._core_any(m.contiguous(), z.contiguous(), msa_mask, pair_mask, inplace=False, drops=drops)
+
+    @staticmethod
+    def backward(ctx, dm, dz):
+        m, z = ctx.saved_tensors
+        dm, dz, grads = ctx.block._backward(m, z, *ctx.masks, dm, dz, ctx.drops)
+        need = ctx.needs_input_grad
+        grads = [g.to(p.dtype) if need[6 + i] else None for i, (p, g) in enumerate(zip(ctx.params, grads))]
+        return (None, None, None, None, dm if need[4] else None, dz if need[5] else None, *grads)
 
 
 class Evoformer(nn.Module):
@@ -129,6 +150,47 @@ class Evoformer(nn.Module):
         z = self.communication(m, msa_mask, z)
         return m, self.pair(z, pair_mask, drops=drops)
 
+    def _backward(self, m, z, msa_mask, pair_mask, dm, dz, drops):
+        """Gradients of a pass of this block on the un-padded tensors: (dm, dz, [one per ``_backward.parameters``]).  Extents
+        that are no multiples of 32 run zero-padded (a masked position has no gradient and gives none)."""
+        s, r = m.shape[1], m.shape[2]
+        ds, dr = F_.round_up(s, 32) - s, F_.round_up(r, 32) - r
+        with torch.no_grad():
+            m, z, dm, dz = m.contiguous(), z.contiguous(), dm.to(m.dtype).contiguous(), dz.to(z.dtype).contiguous()
+            msa_mask, pair_mask = _mask_like(msa_mask, m), _mask_like(pair_mask, z)
+            if ds or dr:
+                m, dm = (F.pad(t, (0, 0, 0, dr, 0, ds)) for t in (m, dm))
+                msa_mask = F.pad(msa_mask, (0, dr, 0, ds))
+            if dr:
+                z, dz = (F.pad(t, (0, 0, 0, dr, 0, dr)) for t in (z, dz))
+                pair_mask = F.pad(pair_mask, (0, dr, 0, dr))
+                drops = {k: F.pad(v, (0, 0, 0, dr) if v.shape[1] == 1 else (0, 0, 0, 0, 0, dr)) for k, v in (drops or {}).items()}
+            dm_in, dz_in = torch.empty_like(m), torch.empty_like(z)
+            st = self.__dict__.get("_grad_layout")
+            params = _backward.parameters(self)
+            if st is None or [id(p) for p in st.params] != [id(p) for p in params]:
+                st = _backward.Grads(params)
+                self.__dict__["_grad_layout"] = st
+            g = st.bind(torch.empty(st.numel, dtype=m.dtype, device=m.device))
+            sp, rp = m.shape[1], m.shape[2]
+            with F_.mask_scope():
+                mm, pm = msa_mask[0], pair_mask[0]
+                derived = [F_.key_bias(mm, m.device, B2=sp, N=rp, mask_sb=rp, mask_sn=1),
+                           F_.key_bias(mm, m.device, B2=rp, N=sp, mask_sb=1, mask_sn=rp),
+                           F_.key_bias(pm, m.device, B2=rp, N=rp, mask_sb=rp, mask_sn=1),
+                           F_.key_bias(pm, m.device, B2=rp, N=rp, mask_sb=1, mask_sn=rp), F_.opm_normaliser(mm)]
+                drop = [(drops or {}).get(k) for k in ("row", "tmo", "tmi", "tas", "tae")]
+                tensors = [m, z, dm, dz, dm_in, dz_in, g.flat, mm, pm, *(t for pair in derived[:4] for t in pair), derived[4], *drop]
+                key = ("backward", m.shape, z.shape, mm.shape, pm.shape, m.dtype, m.device, self.is_multimer, _budget(),
+                       F_.switches(), tuple(t is None for t in drop))
+                _plan.run(self, key, tensors, lambda: _backward.block_backward(
+                    self, m, z, msa_mask, pair_mask, dm, dz, dm_in, dz_in, g, drops, derived=derived, budget=_budget()))
+            if ds or dr:
+                dm_in = dm_in[:, :s, :r].contiguous()
+            if dr:
+                dz_in = dz_in[:, :r, :r].contiguous()
+        return dm_in, dz_in, g.views()
+
     def _draw_drops(self, m, z):
         """Dropout multipliers (0 or 1 / (1 - p)) of one training-mode pass of this block, one tensor per update that
         the reference drops (msa.py:70-73; triangle.py:66-75,122-131,168-173,215-222): shared along the rows, except for
@@ -151,6 +213,9 @@ class Evoformer(nn.Module):
         """The block under autograd, on the un-padded [1, ...] tensors."""
         if not self.recompute_in_backward:
             return self._core_train(m, z, msa_mask, pair_mask)
+        if m.dtype in (torch.bfloat16, torch.float32) and z.dtype == m.dtype and m.shape[-1] == 256 and z.shape[-1] == 128 \
+                and _backward.supported(self):
+            return _BlockGrad.apply(self, msa_mask, pair_mask, self._draw_drops(m, z), m, z, *_backward.parameters(self))
         anchor = torch.empty(0, device=m.device, requires_grad=True)     # outputs need a gradient even when m and z do not
         return _BlockRecompute.apply(self, msa_mask, pair_mask, self._draw_drops(m, z), anchor, m, z)
 

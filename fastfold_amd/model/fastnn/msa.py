@@ -10,6 +10,7 @@ import torch.nn.functional as F
 
 from fastfold_amd.model.fastnn.kernel import LayerNorm
 from fastfold_amd import _plan
+from . import _backward
 from . import _fused as F_
 from .ops import (ChunkMSAColumnGlobalAttention, ChunkTransition, OutProductMean, SelfAttention, Transition,
                   _PackMixin, _budget, _check_tail, _ln_pair, _mask_like, _needs_grad, _no_grad_guard)
@@ -70,15 +71,19 @@ class MSARowAttentionWithPairBias(nn.Module, _PackMixin):
         return out
 
     def _train(self, M_raw, Z, M_mask, drop=None):
-        """msa.py:60-74, operator by operator.  ``drop``: dropout multipliers drawn by the caller; None = drawn here."""
+        """msa.py:60-74; operator by operator where no backward sequence covers the widths.  ``drop``: dropout multipliers drawn
+        by the caller; None = drawn here in training mode."""
         from .kernel import bias_dropout_add
+        if drop is None and self.training and self.p_drop > 0:
+            drop = F.dropout(torch.ones_like(M_raw[:, 0:1, :, :]), p=self.p_drop, training=True)
+        y = _backward.row_attention(self, M_raw, Z, M_mask, drop)
+        if y is not None:
+            return y
         M = self.layernormM(M_raw)
         b = F.linear(self.layernormZ(Z), self.linear_b_weights.to(Z.dtype))
         M = self.attention(M, M_mask, (b, None))
-        if drop is not None:
-            return bias_dropout_add(M, self.out_bias, drop, M_raw, prob=0.0, training=False)
-        dropout_mask = torch.ones_like(M[:, 0:1, :, :])
-        return bias_dropout_add(M, self.out_bias, dropout_mask, M_raw, prob=self.p_drop, training=self.training)
+        drop = torch.ones_like(M[:, 0:1, :, :]) if drop is None else drop
+        return bias_dropout_add(M, self.out_bias, drop, M_raw, prob=0.0, training=False)
 
     def forward(self, M_raw, Z, M_mask):
         if _needs_grad(self, M_raw, Z):
@@ -129,7 +134,10 @@ class MSAColumnAttention(nn.Module, _PackMixin):
         return out
 
     def _train(self, M_raw, M_mask):
-        """msa.py:92-104, operator by operator."""
+        """msa.py:92-104; operator by operator where no backward sequence covers the widths."""
+        y = _backward.column_attention(self, M_raw, M_mask)
+        if y is not None:
+            return y
         M = self.layernormM(M_raw.transpose(-2, -3))
         M = self.attention(M, M_mask.transpose(-1, -2))
         return M_raw + M.transpose(-2, -3)

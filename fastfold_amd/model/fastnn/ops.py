@@ -16,6 +16,7 @@ import torch.nn as nn
 
 from fastfold_amd import _lib, _plan
 from fastfold_amd.model.fastnn.kernel import LayerNorm
+from . import _backward
 from . import _fused as F_
 from .initializer import glorot_uniform_af
 from .kernel import layouts
@@ -420,7 +421,10 @@ class Transition(nn.Module, _PackMixin):
         return out
 
     def _train(self, src):
-        """ops.py:79-82, operator by operator."""
+        """ops.py:79-82; operator by operator where no backward sequence covers the widths."""
+        y = _backward.transition(self, src)
+        if y is not None:
+            return y
         x = self.norm(src)
         return src + self.linear2(torch.relu(self.linear1(x)))
 
@@ -480,7 +484,11 @@ class OutProductMean(nn.Module, _PackMixin):
         return out
 
     def _train(self, M, M_mask, Z_raw):
-        """ops.py:141-173 (the un-chunked branch); the normaliser is kept in fp32."""
+        """ops.py:141-173 (the un-chunked branch; the normaliser is kept in fp32), operator by operator where no backward
+        sequence covers the widths."""
+        y = _backward.outer_product_mean(self, M, M_mask, Z_raw, _budget())
+        if y is not None:
+            return y
         M = self.layernormM(M)
         mask = M_mask.unsqueeze(-1).to(M.dtype)
         left = mask * self.linear_a(M)
@@ -751,6 +759,12 @@ class _TriangleMultiplication(nn.Module, _PackMixin):
         self.output_bias = nn.parameter.Parameter(data=torch.zeros((d_pair,)), requires_grad=True)
         self.p_drop = p_drop
 
+    def _drop(self, Z):
+        """Dropout multipliers of a training-mode call, shared along the rows; None in eval mode."""
+        if not (self.training and self.p_drop > 0):
+            return None
+        return torch.nn.functional.dropout(torch.ones_like(Z[:, 0:1, :, :]), p=self.p_drop, training=True)
+
     def _run(self, Z_raw, Z_mask, out, xtail=None, drop=None):
         """``drop``: None or the [1, 1, r, C] dropout multipliers of a training-mode call (drawn by the caller)."""
         _plan.scope()
@@ -788,9 +802,13 @@ class _TriangleMultiplication(nn.Module, _PackMixin):
         return out
 
     def _train(self, Z_raw, Z_mask, drop=None):
-        """triangle.py:41-75 / :97-131, operator by operator.  ``drop``: dropout multipliers drawn by the caller
+        """triangle.py:41-75 / :97-131; operator by operator where no backward sequence covers the widths.  ``drop``: dropout multipliers drawn by the caller
         ([1, 1, r, C]); None = drawn here in training mode."""
         from .kernel import bias_ele_dropout_residual
+        drop = self._drop(Z_raw) if drop is None else drop
+        y = _backward.triangle_multiplication(self, Z_raw, Z_mask, drop)
+        if y is not None:
+            return y
         Z = self.layernorm1(Z_raw)
         lr = Z_mask.unsqueeze(-1).to(Z.dtype) * self.left_right_projection(Z)
         lr = lr * torch.sigmoid(self.left_right_gate(Z))
@@ -802,11 +820,8 @@ class _TriangleMultiplication(nn.Module, _PackMixin):
         left, right = _ToChanMajorFn.apply(lr.contiguous(), self._incoming)
         p = _FromChanMajorFn.apply(_TriContractFn.apply(left, right, r), r)
         ab = self.output_projection(self.layernorm2(p))
-        if drop is not None:
-            return bias_ele_dropout_residual(ab, self.output_bias, g, drop, Z_raw, prob=0.0, training=False)
-        dropout_mask = torch.ones_like(Z[:, 0:1, :, :])
-        return bias_ele_dropout_residual(ab, self.output_bias, g, dropout_mask, Z_raw, prob=self.p_drop,
-                                         training=self.training)
+        drop = torch.ones_like(Z[:, 0:1, :, :]) if drop is None else drop
+        return bias_ele_dropout_residual(ab, self.output_bias, g, drop, Z_raw, prob=0.0, training=False)
 
     def forward(self, Z_raw, Z_mask):
         if _needs_grad(self, Z_raw):
@@ -845,6 +860,13 @@ class _TriangleAttention(nn.Module, _PackMixin):
                                        last_bias_fuse=True)
         self.out_bias = nn.parameter.Parameter(data=torch.zeros((d_pair,)), requires_grad=True)
 
+    def _drop(self, Z):
+        """Dropout multipliers of a training-mode call, shared along the rows (ending node: the columns); None in eval mode."""
+        if not (self.training and self.p_drop > 0):
+            return None
+        like = Z[:, :, 0:1, :] if self._ending else Z[:, 0:1, :, :]
+        return torch.nn.functional.dropout(torch.ones_like(like), p=self.p_drop, training=True)
+
     def _run(self, Z_raw, Z_mask, out, xtail=None, drop=None):
         """``drop``: None or the dropout multipliers of a training-mode call, [1, 1, r, C] (starting node) or
         [1, r, 1, C] (ending node)."""
@@ -875,8 +897,12 @@ class _TriangleAttention(nn.Module, _PackMixin):
 
     def _train(self, Z_raw, Z_mask, drop=None):
         """triangle.py:156-173 (starting node) / :202-222 (ending node: the same on the transposed pair tensor, with
-        the dropout mask shared along the other axis)."""
+        the dropout mask shared along the other axis); operator by operator where no backward sequence covers the widths."""
         from .kernel import bias_dropout_add
+        drop = self._drop(Z_raw) if drop is None else drop
+        y = _backward.triangle_attention(self, Z_raw, Z_mask, drop)
+        if y is not None:
+            return y
         Z = Z_raw.transpose(-2, -3) if self._ending else Z_raw
         mask = Z_mask.transpose(-1, -2) if self._ending else Z_mask
         Z = self.layernorm1(Z)
@@ -884,12 +910,9 @@ class _TriangleAttention(nn.Module, _PackMixin):
         Z = self.attention(Z, mask, (b, None))
         if self._ending:
             Z = Z.transpose(-2, -3)
-            dropout_mask = torch.ones_like(Z[:, :, 0:1, :])
-        else:
-            dropout_mask = torch.ones_like(Z[:, 0:1, :, :])
-        if drop is not None:
-            return bias_dropout_add(Z, self.out_bias, drop, Z_raw, prob=0.0, training=False)
-        return bias_dropout_add(Z, self.out_bias, dropout_mask, Z_raw, prob=self.p_drop, training=self.training)
+        if drop is None:
+            drop = torch.ones_like(Z[:, :, 0:1, :] if self._ending else Z[:, 0:1, :, :])
+        return bias_dropout_add(Z, self.out_bias, drop, Z_raw, prob=0.0, training=False)
 
     def forward(self, Z_raw, Z_mask):
         if _needs_grad(self, Z_raw):

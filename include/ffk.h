@@ -154,7 +154,9 @@ int ffk_bias_ele_dropout_res(void* out, const void* ab, const void* bias, const 
  * 79-82,143-155,305-324,393-399,404-412,659-670 and msa.py:61-72.
  */
 enum { FFK_TILE_STRIDED = 0, FFK_TILE_QK = 1, FFK_TILE_V = 2, FFK_TILE_BIAS = 3, FFK_TILE_ACC = 4 };
-enum { FFK_ACT_NONE = 0, FFK_ACT_RELU = 1, FFK_ACT_SIGMOID = 2 };
+/* GATE_POS: no activation; the gate operand is taken as 1 where it is positive and 0 elsewhere (derivative of a ReLU whose
+   output the gate is) */
+enum { FFK_ACT_NONE = 0, FFK_ACT_RELU = 1, FFK_ACT_SIGMOID = 2, FFK_ACT_GATE_POS = 3 };
 enum { FFK_LINEAR_AUTO = 0, FFK_LINEAR_STAGED = 1 };
 #define FFK_MAX_TILES 10
 
@@ -292,6 +294,12 @@ enum { FFK_ATT_GATE_TILED = 1, FFK_ATT_BIAS_PADDED = 2, FFK_ATT_HALF_K = 4 };
 int ffk_attention_fwd(void* out, const void* q_t, const void* k_t, const void* v_t,
                       const void* bias_t, const float* keybias, const int32_t* tileflags, const void* gate,
                       int64_t B2, int64_t H, int64_t Nq, int64_t Nk, int64_t D, int flags, int dtype, void* stream);
+
+/* The same with the log-sum-exp of every row (log2 domain, 3e38 for a row without a valid key) in
+ * lse[((b2 * H + h) * ceil(Nq/32)) * 32 + q] for the backward pass; lse may be NULL, and must be for D != 32. */
+int ffk_attention_fwd_lse(void* out, float* lse, const void* q_t, const void* k_t, const void* v_t, const void* bias_t,
+                          const float* keybias, const int32_t* tileflags, const void* gate, int64_t B2, int64_t H, int64_t Nq,
+                          int64_t Nk, int64_t D, int flags, int dtype, void* stream);
 
 /* Backward of ffk_attention_fwd without a gate (the autograd path of fused_attention_core):
  *     given do = d loss / d out, computes dq, dk, dv and (optionally) dbias of
@@ -461,6 +469,77 @@ int ffk_pointwise_attention_core(void* o, const void* q, const void* kv, const f
 int ffk_key_bias(float* keybias, int32_t* tileflags, const void* mask, int64_t B, int64_t N,
                  int64_t mask_sb, int64_t mask_sn, int dtype, void* stream);
 
+/* ------------------------------------------------------------------------------------
+ * Backward pass of a block.  The reference differentiates its modules operator by operator through autograd
+ * (fastfold/utils/checkpointing.py:55-73 re-runs a block and back-propagates through it); these entry points are the pieces of
+ * the same gradients as passes over whole activations.  dtype f32 or bf16 throughout, fp32 arithmetic; no atomics, so equal
+ * inputs give equal gradients.
+ *
+ * out[n][k] = sum_m y[m][n] x[m][k]  and, optionally, colsum[n] = sum_m y[m][n].
+ *   row m of y / x : (m / inner) * so + (m % inner) * si;  N and K multiples of 8
+ *   ws             : fp32 scratch, slices * (N * K + N) elements; the rows are cut into `slices` slices of a multiple of 64 rows
+ *   element (n, k) of out : (n / o_inner) * o_so + (n % o_inner) * o_si + k * o_sk, of the operands' dtype; rows n < n_out are
+ *                    stored
+ *   colsum         : sums of the columns [cs_first, cs_first + cs_count), or NULL
+ *   acc            : for rows that come in several calls: fp32 [n_out * K + cs_count], added to what this call sums (FFK_WGRAD_READ)
+ *                    and written instead of out and colsum (FFK_WGRAD_WRITE); NULL with flags 0
+ */
+enum { FFK_WGRAD_READ = 1, FFK_WGRAD_WRITE = 2 };
+int ffk_weight_grad(void* out, int64_t n_out, void* colsum, int64_t cs_first, int64_t cs_count, float* acc, float* ws,
+                    const void* y, const void* x, int64_t M, int64_t N, int64_t K, int64_t slices, int64_t y_inner, int64_t y_so, int64_t y_si, int64_t x_inner, int64_t x_so,
+                    int64_t x_si, int64_t o_inner, int64_t o_so, int64_t o_si, int64_t o_sk, int flags, int dtype,
+                    void* stream);
+
+/* out[n][k] = sum over the slices of part[slice][n][k] (fp32, contiguous, K a multiple of 4), addressed like the output above. */
+int ffk_slice_sum(void* out, const float* part, int64_t slices, int64_t N, int64_t K, int64_t o_inner, int64_t o_so,
+                  int64_t o_si, int64_t o_sk, int dtype, void* stream);
+
+/* dx = resid + (gradient of LayerNorm(x) for the cotangent dy), xn = LayerNorm(x) (optional), dgamma and dbeta.  Rows of C = 64,
+ * 128 or 256 channels, contiguous; resid may be NULL, dx may alias dy or resid; ws: fp32, FFK_LN_BWD_BLOCKS * 2 * C. */
+#define FFK_LN_BWD_BLOCKS 1024
+int ffk_layernorm_bwd_rows(void* dx, void* xn, void* dgamma, void* dbeta, float* ws, const void* dy, const void* x,
+                           const void* gamma, const void* beta, const void* resid, int64_t rows, int64_t C, float eps,
+                           int dtype, void* stream);
+
+/* out[m][c] = x[m][c] * mul, the multiplier of row m at (m / inner) * m_so + (m % inner) * m_si: mode 0 a row of C multipliers,
+ * mode 1 one multiplier, mode 2 one fp32 divisor (x / (mul + eps)).  out may alias x. */
+int ffk_scale_rows(void* out, const void* x, const void* mul, int64_t rows, int64_t C, int64_t inner, int64_t m_so,
+                   int64_t m_si, int mode, float eps, int dtype, void* stream);
+
+/* Gate of an attention, s = sigmoid(gpre + gbias), rows m = b2 * N + n of H * 32 channels (gpre with row pitch g_ld):
+ *   go = s o;  dgpre = dgo o s (1 - s) (row pitch dg_ld);  do = dgo s as FFK_TILE_ACC tiles (do_t) and FFK_TILE_V tiles (do_v),
+ *   tokens past N zero;  dsum[((b2 * H + h) * ceil(N / 32)) * 32 + n] = sum_d do o */
+int ffk_att_gate_bwd(void* go, void* dgpre, void* do_t, void* do_v, float* dsum, const void* dgo, const void* gpre,
+                     const void* gbias, const void* o, int64_t B2, int64_t N, int64_t H, int64_t g_ld, int64_t dg_ld,
+                     int dtype, void* stream);
+
+/* Output gate of a triangle multiplication, s = sigmoid(gpre), d = dz * drop[m % period] (drop may be NULL):
+ *   dab = d s;  dgpre = d ab s (1 - s) */
+int ffk_trimul_gate_bwd(void* dab, void* dgpre, const void* dz, const void* drop, const void* ab, const void* gpre,
+                        int64_t rows, int64_t C, int64_t period, int64_t g_ld, int64_t dg_ld, int dtype, void* stream);
+
+/* Gated projections l = mask proj sigmoid(gate) of one side of a triangle multiplication, l and its cotangent dl channel-major
+ * ([c][i][k], planes cs apart, rows kpad):  dproj = dl mask s;  dgate = dl l (1 - s).  Row (i, k) of gate (pitch g_ld), mask and
+ * the outputs (pitch d_ld) is row i * r_i + k * r_k. */
+int ffk_glu_bwd(void* dproj, void* dgate, const void* dl, const void* l, const void* gate, const void* mask, int64_t R,
+                int64_t C, int64_t cs, int64_t kpad, int64_t d_ld, int64_t g_ld, int64_t r_i, int64_t r_k, int dtype,
+                void* stream);
+
+/* Backward of an attention (head dimension 32, N queries and keys) whose forward pass left lse (ffk_attention_fwd_lse) and whose
+ * gate's backward pass left dsum and do: as ffk_attention_bwd, with dq, dk, dv written to rows, element (b2, h, n, d) at
+ * b2 * s_b + h * s_h + n * s_n + d.  q_t, k_t are a pair of equal order (FFK_TILE_QK or FFK_TILE_ACC), do_t and v_t another;
+ * q_v, k_v, do_v are FFK_TILE_V.  dbias (NULL: none): fp32 [dbias_parts][H][N][N] partial sums over the batch rows, not added
+ * up.  flags: FFK_ATT_BIAS_PADDED or 0. */
+int ffk_attention_bwd_rows(void* dq, void* dk, void* dv, float* dbias, int64_t dbias_parts, const float* lse,
+                           const float* dsum, const void* q_t, const void* q_v, const void* k_t, const void* k_v,
+                           const void* v_t, const void* bias_t, const float* keybias, const void* do_t, const void* do_v,
+                           int64_t B2, int64_t H, int64_t N, int64_t s_b, int64_t s_h, int64_t s_n, float dq_scale,
+                           float dk_scale, int flags, int dtype, void* stream);
+
+/* out[m][h] = sum over `parts` of dbias[part][h][m] for h < H, 0 for h = H .. 31 (row pitch ld): a pair-bias gradient as 32
+ * columns of a product's operand. */
+int ffk_bias_cols(void* out, const float* dbias, int64_t parts, int64_t rows, int64_t H, int64_t ld, int dtype, void* stream);
+
 /* Zeroes `bytes` (a multiple of 16) at a 16-byte aligned address with a kernel: padding rows and columns of operand
  * buffers, in code that may be captured into a graph. */
 int ffk_fill_zero(void* p, int64_t bytes, void* stream);
@@ -476,7 +555,9 @@ int ffk_fill_zero(void* p, int64_t bytes, void* stream);
 enum {
     FFK_OP_FUSED_LINEAR = 0, FFK_OP_BGEMM_NT = 1, FFK_OP_ATTENTION_FWD = 2, FFK_OP_PAIR_BIAS = 3, FFK_OP_OPM_FUSED = 4,
     FFK_OP_TRANSITION_FUSED = 5, FFK_OP_GATED_OUT_FUSED = 6, FFK_OP_GLOBAL_ATTENTION_CORE = 7, FFK_OP_LAYERNORM_FWD = 8,
-    FFK_OP_FILL_ZERO = 9, FFK_OP_COUNT = 10
+    FFK_OP_FILL_ZERO = 9, FFK_OP_ATTENTION_FWD_LSE = 10, FFK_OP_ATTENTION_BWD_ROWS = 11, FFK_OP_TRANSPOSE_BATCHED = 12,
+    FFK_OP_WEIGHT_GRAD = 13, FFK_OP_LAYERNORM_BWD_ROWS = 14, FFK_OP_SCALE_ROWS = 15, FFK_OP_ATT_GATE_BWD = 16,
+    FFK_OP_TRIMUL_GATE_BWD = 17, FFK_OP_GLU_BWD = 18, FFK_OP_BIAS_COLS = 19, FFK_OP_SLICE_SUM = 20, FFK_OP_COUNT = 21
 };
 int ffk_run_plan(const void* plan, int64_t bytes, const uint64_t* bases, int64_t n_bases, void* stream);
 

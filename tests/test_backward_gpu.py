@@ -1,0 +1,108 @@
+"""The pieces of a block's backward pass against float64 on the CPU, and the block-level sequence against the modules on their own
+(multimer order, pieces of the outer product mean)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DT = [torch.float32, torch.bfloat16]
+
+
+def _rel(a, b):
+    return float((a.double().cpu() - b.double().cpu()).norm() / b.double().cpu().norm())
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("M,N,K,slices", [(1, 8, 8, 1), (63, 32, 128, 1), (64, 128, 128, 1), (65, 136, 264, 2), (1000, 544, 128, 4),
+                                          (4096, 128, 1024, 16), (129, 256, 32, 3)])
+def test_weight_grad(dev, dtype, M, N, K, slices):
+    from fastfold_amd import _lib
+    g = torch.Generator().manual_seed(M + N)
+    y, x = torch.randn(M, N + 8, generator=g).to(dev, dtype), torch.randn(M, K, generator=g).to(dev, dtype)
+    ws = torch.empty(slices * N * (K + 1), device=dev)
+    n_out = N - 4
+    out, cs = torch.full((N, K), 7.0, device=dev, dtype=dtype), torch.empty(4, device=dev, dtype=dtype)
+    kw = dict(M=M, N=N, K=K, slices=slices, dtype=dtype, y_map=(M, 0, N + 8), x_map=(M, 0, K), n_out=n_out, cs_first=4, cs_count=4)
+    _lib.weight_grad(out, cs, ws, y, x, **kw)
+    ref = y[:, :N].double().cpu().t() @ x.double().cpu()
+    tol = 1e-5 if dtype == torch.float32 else 6e-3
+    assert _rel(out[:n_out], ref[:n_out]) < tol and bool((out[n_out:] == 7.0).all())
+    assert _rel(cs, y[:, 4:8].double().cpu().sum(0)) < tol
+    # rows through a map (pairs of rows exchanged) and the output transposed
+    if M % 2 == 0:
+        perm = torch.arange(M).view(2, M // 2).t().reshape(-1)
+        o2 = torch.empty(K, N, device=dev, dtype=dtype)
+        _lib.weight_grad(o2, None, ws, y, x, **dict(kw, y_map=(2, N + 8, (M // 2) * (N + 8)), n_out=None, o_map=(N, 0, 1, N)))
+        assert _rel(o2.t(), y[perm.to(dev), :N].double().cpu().t() @ x.double().cpu()) < tol
+    # two calls through an accumulator
+    acc = torch.empty(n_out * K + 4, device=dev)
+    _lib.weight_grad(out, cs, ws, y, x, **dict(kw, acc=acc, flags=_lib.FFK_WGRAD_WRITE))
+    _lib.weight_grad(out, cs, ws, y, x, **dict(kw, acc=acc, flags=_lib.FFK_WGRAD_READ))
+    assert _rel(out[:n_out], 2 * ref[:n_out]) < tol and _rel(cs, 2 * y[:, 4:8].double().cpu().sum(0)) < tol
+    with pytest.raises(RuntimeError):
+        _lib.weight_grad(out, cs, ws, y, x, **dict(kw, slices=M // 64 + 2))          # an empty slice
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("rows,C", [(1, 64), (33, 128), (5000, 256), (70001, 128)])
+def test_layernorm_bwd_rows(dev, dtype, rows, C):
+    from fastfold_amd import _lib
+    g = torch.Generator().manual_seed(rows)
+    x, dy, res = (torch.randn(rows, C, generator=g).to(dev, dtype) for _ in range(3))
+    gam, bet = (1 + 0.1 * torch.randn(C, generator=g)).to(dev, dtype), torch.randn(C, generator=g).to(dev, dtype)
+    dx, xn, dg, db = torch.empty_like(x), torch.empty_like(x), torch.empty_like(gam), torch.empty_like(gam)
+    ws = torch.empty(_lib.FFK_LN_BWD_BLOCKS * 2 * C, device=dev)
+    _lib.layernorm_bwd_rows(dx, xn, dg, db, ws, dy, x, gam, bet, res, rows=rows, C=C, dtype=dtype)
+    xr, gr, br = (t.double().cpu().requires_grad_() for t in (x, gam, bet))
+    y = torch.nn.functional.layer_norm(xr, (C,), gr, br, 1e-5)
+    y.backward(dy.double().cpu())
+    tol = 2e-5 if dtype == torch.float32 else 6e-3
+    assert _rel(dx, xr.grad + res.double().cpu()) < tol and _rel(xn, y.detach()) < tol
+    assert _rel(dg, gr.grad) < tol and _rel(db, br.grad) < tol
+    d2 = dx.clone()
+    _lib.layernorm_bwd_rows(d2, None, dg, db, ws, dy, x, gam, None, None, rows=rows, C=C, dtype=dtype)
+    assert _rel(d2, xr.grad) < tol
+
+
+def _block(dev, dtype, multimer):
+    from fastfold_amd.model.fastnn import Evoformer
+    g = torch.Generator().manual_seed(2)
+    blk = Evoformer(256, 128, True, True, is_multimer=multimer)
+    with torch.no_grad():
+        for n, p in blk.named_parameters():
+            w = torch.randn(p.shape, generator=g) * (0.1 if p.dim() == 1 else p.shape[-1] ** -0.5)
+            p.copy_(1 + w if "norm" in n and n.endswith("weight") else w)
+    return blk.to(dev, dtype).eval()
+
+
+@pytest.mark.parametrize("multimer", [False, True])
+@pytest.mark.parametrize("s,r,chunk", [(32, 64, None), (40, 33, None), (32, 64, 4)])
+def test_block_sequence_equals_the_modules(dev, multimer, s, r, chunk, monkeypatch):
+    """The block-level sequence (run twice: recorded and replayed) against autograd over the modules, fp32, with a masked tail; and
+    with the outer product mean cut into pieces of a few residues."""
+    from fastfold_amd.model.fastnn import _fused, set_chunk_size
+    blk = _block(dev, torch.float32, multimer)
+    g = torch.Generator().manual_seed(5)
+    m, z = torch.randn(1, s, r, 256, generator=g).to(dev), torch.randn(1, r, r, 128, generator=g).to(dev)
+    res = torch.ones(r, device=dev)
+    res[r - 3:] = 0
+    mm, pm = torch.ones(1, s, 1, device=dev) * res, (res[:, None] * res)[None]
+    cot = torch.randn(1, s, r, 256, generator=g).to(dev) * mm[..., None], torch.randn(1, r, r, 128, generator=g).to(dev) * pm[..., None]
+
+    def grads(fn):
+        a, b = m.clone().requires_grad_(), z.clone().requires_grad_()
+        for p in blk.parameters():
+            p.grad = None
+        torch.autograd.backward(fn(a, b), cot)
+        return [a.grad, b.grad] + [p.grad.clone() for p in blk.parameters()]
+    want = grads(lambda a, b: blk._core_train(a, b, mm, pm, drops={}))
+    if chunk:
+        monkeypatch.setattr(_fused, "_WS_BUDGET_CHUNKED", 12 * r * 2048 * 4)
+        set_chunk_size(chunk)
+    try:
+        for _ in range(2):
+            got = grads(lambda a, b: blk._run_grad(a, b, mm, pm))
+            for n, x, y in zip(["m", "z"] + [n for n, _ in blk.named_parameters()], got, want):
+                if float(y.norm()) > 1e-3:
+                    assert _rel(x, y) < 2e-5, n
+    finally:
+        set_chunk_size(None)

@@ -130,3 +130,35 @@ def test_malformed_plans_are_refused():
     assert run(struct.pack("<iiii", 9, 2, 1, 0) + struct.pack("<iiq", 0, 7, 0) + b"\0" * 16) == 2      # no such buffer
     assert run(struct.pack("<iiii", 9, 2, 1, 0) + struct.pack("<iiq", 0, 1, 0) + b"\0" * 16) == 2      # a null buffer
     assert run(struct.pack("<iiii", 9, 2, 0, 0) + struct.pack("<Qq", 0, 16)) == 3        # the entry point's own check
+
+
+@gpu
+@pytest.mark.parametrize("s,r", [(12, 40), (16, 64)])
+def test_replay_under_memory_of_any_content(dev, s, r):
+    """Forward and backward of a block with freshly filled memory around (zeros, NaN): recorded and replayed passes give the
+    same bits, so no launch reads scratch it has not written and no replay takes a neighbour's buffer."""
+    from fastfold_amd.model.fastnn import Evoformer
+    st = _stack(dev, torch.bfloat16, 1)
+    blk = Evoformer(256, 128, True, True).to(dev, torch.bfloat16)
+    blk.load_state_dict(st.blocks[0].state_dict())
+    blk.train()
+    m, z, mm, pm = _inputs(dev, torch.bfloat16, s, r, 3)
+    cot = torch.randn(s, r, 256, device=dev).bfloat16(), torch.randn(r, r, 128, device=dev).bfloat16()
+    want = None
+    for fill in (0.0, float("nan"), float("nan"), float("nan")):
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        junk = [torch.full((n,), fill, device=dev) for n in [1 << 25] * 2 + [1 << 18] * 64 + [1 << 12] * 200]
+        del junk
+        torch.manual_seed(5)
+        a, b = m.clone().requires_grad_(), z.clone().requires_grad_()
+        for p in blk.parameters():
+            p.grad = None
+        out = blk(a, b, mm, pm)
+        torch.autograd.backward(out, cot)
+        got = [*out, a.grad, b.grad, *(p.grad for p in blk.parameters())]
+        got = [t.detach().clone() for t in got]
+        assert all(bool(torch.isfinite(t).all()) for t in got)
+        if want is not None:
+            assert all(torch.equal(x, y) for x, y in zip(got, want))
+        want = got
