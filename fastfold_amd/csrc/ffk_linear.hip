@@ -28,6 +28,7 @@ template <> struct LinCfg<float> {
 
 struct LinArgs {
     ffk_linear_desc d;
+    int tiles_per;       // N-tiles of one workgroup: blockIdx.y takes the tiles blockIdx.y * tiles_per ...
 };
 
 // Row tables.  Splitting a logical row into (hi, lo) = divmod(m, inner) needs an integer
@@ -128,9 +129,11 @@ __global__ __launch_bounds__(THREADS, 4) void fused_linear_kernel(const LinArgs 
     constexpr int WVEC = NT * BK / VEC / THREADS;  // 16-byte vectors per thread per chunk (= 4)
     Vec16<T> wreg[WVEC];
     const int kchunks = K / BK;
-    const int total_chunks = d.n_tiles * kchunks;
+    const int nt_first = blockIdx.y * args.tiles_per;
+    const int nt_end = nt_first + args.tiles_per < d.n_tiles ? nt_first + args.tiles_per : d.n_tiles;
+    const int total_chunks = (nt_end - nt_first) * kchunks;
     auto w_fetch = [&](int chunk) {
-        const int nt = chunk / kchunks, kc = chunk - nt * kchunks;
+        const int ct = chunk / kchunks, kc = chunk - ct * kchunks, nt = nt_first + ct;
 #pragma unroll
         for (int i = 0; i < WVEC; ++i) {
             const int v = tid + THREADS * i;
@@ -251,7 +254,7 @@ __global__ __launch_bounds__(THREADS, 4) void fused_linear_kernel(const LinArgs 
     // ---- main loop over N-tiles ----
     const unsigned char* a_frag_base = sA + (wm * 32 + l32) * AP + half * (MM::KLANE * ES);
     int chunk = 0;
-    for (int nt = 0; nt < d.n_tiles; ++nt) {
+    for (int nt = nt_first; nt < nt_end; ++nt) {
         f32x16 acc[CT];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
@@ -480,7 +483,20 @@ int launch_linear(const ffk_linear_desc& d, hipStream_t st) {
     }
     LinArgs a;
     a.d = d;
-    dim3 grid(ffk_cdiv(d.M, Cfg::BM));
+    // Few rows: the N-tiles are spread over several workgroups (which then each stage and normalise the same rows, from L2)
+    // until there are two workgroups per CU; from there on one workgroup per slab is as fast and reads its rows once.  One
+    // workgroup walking eight tiles over 64 of 4 096 rows keeps a quarter of the chip busy for 79 us (fp32, K = 128); spread
+    // out it takes 24 us, 125 -> 28 us at 2 048 rows of K = 256, 89 -> 69 us at 16 384 rows.  A launch that writes over its
+    // own input keeps one workgroup per slab, which has read its rows before it stores any.
+    const int slabs = ffk_cdiv(d.M, Cfg::BM);
+    int split = slabs >= 512 ? 1 : ffk_cdiv(512, slabs);
+    const char* a0 = (const char*)d.a;
+    for (int i = 0; i < d.n_tiles; ++i) {
+        const char* o = (const char*)d.tiles[i].out;
+        if (o >= a0 && o < a0 + (size_t)d.M * d.K * ES) split = 1;
+    }
+    a.tiles_per = ffk_cdiv(d.n_tiles, split < d.n_tiles ? split : d.n_tiles);
+    dim3 grid(slabs, ffk_cdiv(d.n_tiles, a.tiles_per));
     fused_linear_kernel<T><<<grid, THREADS, smem, st>>>(a);
     return ffk_check_launch("ffk_fused_linear");
 }

@@ -511,3 +511,19 @@ def test_periodic_gate_rows(dev, dtype, K, N, P):
     y = 1.0 / (1.0 + np.exp(-ops_np.linear(_np(a), _np(w), _np(b))))
     ref = y.reshape(S, P, N) * _np(gate)[None]
     assert _rel(_np(out).reshape(S, P, N), ref) < TOL[dtype]
+
+
+@pytest.mark.parametrize("M,nt", [(1, 3), (65, 5), (64 * 511, 2), (64 * 512, 2)])
+def test_tiles_spread_over_workgroups(dev, M, nt):
+    """Few rows: several workgroups share a slab, each with some of the N-tiles (also an uneven share of them)."""
+    from fastfold_amd import _lib
+    F = torch.nn.functional
+    g = torch.Generator().manual_seed(M + nt)
+    K, N = 64, 128 * nt
+    x, w, b = (torch.randn(*sh, generator=g).to(dev) for sh in ((M, K), (N, K), (N,)))
+    ln = (torch.rand(K, generator=g).to(dev) + 0.5, torch.randn(K, generator=g).to(dev))
+    out = torch.full((M, N), float("nan"), device=dev)
+    tiles = [_lib.make_tile(out.data_ptr() + 512 * i, inner=M, s_i=N, bias=b.data_ptr() + 512 * i) for i in range(nt)]
+    _lib.fused_linear(x, w, tiles, M=M, K=K, ln=ln)
+    ref = F.linear(F.layer_norm(x, (K,), *ln), w, b)
+    torch.testing.assert_close(out, ref, rtol=1e-4, atol=2e-4)
