@@ -25,6 +25,7 @@ int ffk_fail(int code, const char* fmt, ...);
 int ffk_linear_slab_launch(const ffk_linear_desc* d, hipStream_t st);   // ffk_linear_slab.hip
 int ffk_bgemm_big_try(const ffk_bgemm_desc* d, hipStream_t st, int* status);    // ffk_bgemm_big.hip
 int ffk_linear_ws_try(const ffk_linear_desc* d, hipStream_t st, int* status);   // ffk_linear_ws.hip
+int ffk_linear_ws32_try(const ffk_linear_desc* d, hipStream_t st, int* status); // ffk_linear_ws32.hip
 
 // Dynamic-LDS reservation of one kernel: hipFuncSetAttribute is needed once per device (again only if a
 // later launch asks for more).  A function-scope `static FfkLdsReservation` (zero-initialised) remembers, per
@@ -183,6 +184,47 @@ template <typename T> __device__ __forceinline__ float exp_for(float x);
 template <> __device__ __forceinline__ float exp_for<float>(float x) { return expf(x); }
 template <> __device__ __forceinline__ float exp_for<bf16_t>(float x) { return fast_exp2(1.4426950408889634f * x); }
 template <> __device__ __forceinline__ float exp_for<f16_t>(float x) { return fast_exp2(1.4426950408889634f * x); }
+
+// Four sums over LPR (32 or 64) adjacent lanes at once; lane l gets the sum of s[l & 3].  Exchanging two values for one in the
+// first two steps takes 14 instructions where four butterflies take 32 and more.
+template <int LPR> __device__ __forceinline__ float ffk_sum4(const float (&s)[4]) {
+    const bool b1 = __lane_id() & 1, b2 = __lane_id() & 2;
+    const float a = (b1 ? s[1] : s[0]) + lane_xor<1>(b1 ? s[0] : s[1]);
+    const float b = (b1 ? s[3] : s[2]) + lane_xor<1>(b1 ? s[2] : s[3]);
+    float c = (b2 ? b : a) + lane_xor<2>(b2 ? a : b);
+    int x = __builtin_bit_cast(int, c);
+    c += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(x, x, 0x124, 0xF, 0xF, false));     // row_ror:4
+    x = __builtin_bit_cast(int, c);
+    c += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(x, x, 0x128, 0xF, 0xF, false));     // row_ror:8
+    c += lane_xor<16>(c);
+    if (LPR == 64) c += lane_xor<32>(c);
+    return c;
+}
+template <int I> __device__ __forceinline__ float ffk_quad(float v) {          // value of lane I of the quad
+    const int x = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(x, x, I * 0x55, 0xF, 0xF, false));
+}
+// LayerNorm of four rows of 4 * LPR fp32 values, one 16-byte piece of each per lane (both fused linear kernels: the same bits
+// from either; mean first, then the squares of the differences).
+template <int LPR> __device__ __forceinline__ void ffk_ln_rows4(f32x4* x, const f32x4& gam, const f32x4& bet, float eps) {
+    float s[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] = (x[i][0] + x[i][1]) + (x[i][2] + x[i][3]);
+    const float mu = ffk_sum4<LPR>(s) * (1.0f / (4 * LPR));
+    const float m[4] = {ffk_quad<0>(mu), ffk_quad<1>(mu), ffk_quad<2>(mu), ffk_quad<3>(mu)};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[i][e] -= m[i];
+        s[i] = __builtin_fmaf(x[i][0], x[i][0], x[i][1] * x[i][1]) + __builtin_fmaf(x[i][2], x[i][2], x[i][3] * x[i][3]);
+    }
+    const float rs = rsqrtf(__builtin_fmaf(ffk_sum4<LPR>(s), 1.0f / (4 * LPR), eps));
+    const float r[4] = {ffk_quad<0>(rs), ffk_quad<1>(rs), ffk_quad<2>(rs), ffk_quad<3>(rs)};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[i][e] = __builtin_fmaf(x[i][e] * r[i], gam[e], bet[e]);
+}
 
 // ------------------------------------------------- extended residual stream ----
 // A residual stream that is rounded to bf16 after every one of the ~300 updates of a 48-block stack drifts by

@@ -157,6 +157,7 @@ __global__ __launch_bounds__(THREADS, 4) void fused_linear_kernel(const LinArgs 
     // Loads below are unconditional (row / column indices are clamped to valid ones instead of
     // being predicated) so that a batch of four is in flight at once; only the LDS stores are guarded.
     // Rows beyond M hold a copy of row M-1: their results are never stored.
+    bool ln_done = false;
     if (!d.a_chanmajor) {
         const int vpr = K / VEC;                   // 16-byte vectors per row
         int cs = 3;
@@ -165,6 +166,14 @@ __global__ __launch_bounds__(THREADS, 4) void fused_linear_kernel(const LinArgs 
         const int c = c_raw < vpr ? c_raw : vpr - 1;
         const int r_first = tid >> cs, rstep = THREADS >> cs;
         const int n_it = BM / rstep;
+        [[maybe_unused]] f32x4 gam, bet;
+        if constexpr (ES == 4) {
+            ln_done = d.ln_gamma && (K == 128 || K == 256) && ((reinterpret_cast<uintptr_t>(d.ln_gamma) | reinterpret_cast<uintptr_t>(d.ln_beta)) & 15) == 0;
+            if (ln_done) {
+                gam = *reinterpret_cast<const f32x4*>((const float*)d.ln_gamma + c * 4);
+                bet = *reinterpret_cast<const f32x4*>((const float*)d.ln_beta + c * 4);
+            }
+        }
         for (int i0 = 0; i0 < n_it; i0 += 4) {
             Vec16<T> buf[4];
 #pragma unroll
@@ -172,6 +181,17 @@ __global__ __launch_bounds__(THREADS, 4) void fused_linear_kernel(const LinArgs 
                 int r = r_first + (i0 + j) * rstep;
                 r = r < BM ? r : BM - 1;
                 buf[j] = ld16(A + tab.off[r] + c * VEC);
+            }
+            if constexpr (ES == 4) {               // whole rows of 32 / 64 lanes: normalised on the way
+                if (ln_done) {
+                    f32x4 x[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) x[j] = *reinterpret_cast<f32x4*>(&buf[j]);
+                    if (K == 128) ffk_ln_rows4<32>(x, gam, bet, d.ln_eps);
+                    else ffk_ln_rows4<64>(x, gam, bet, d.ln_eps);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4*>(&buf[j]) = x[j];
+                }
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -216,7 +236,7 @@ __global__ __launch_bounds__(THREADS, 4) void fused_linear_kernel(const LinArgs 
     lds_barrier();
 
     // ---- LayerNorm prologue, in place ----
-    if (d.ln_gamma) {
+    if (d.ln_gamma && !ln_done) {
         constexpr int TPR = THREADS / BM;          // threads per row (adjacent lanes)
         const int r = tid / TPR, j = tid % TPR;
         const int vpr = K / VEC;
@@ -560,6 +580,7 @@ extern "C" int ffk_fused_linear(const ffk_linear_desc* d, void* stream) {
     {
         int status = FFK_OK;
         if (ffk_linear_ws_try(d, (hipStream_t)stream, &status)) return status;
+        if (ffk_linear_ws32_try(d, (hipStream_t)stream, &status)) return status;
     }
     FFK_REQUIRE(!d->a2, FFK_ERR_UNSUPPORTED,
                 "ffk_fused_linear: a second operand needs bf16, K = 128, a channel-major first operand and GLU tiles only");

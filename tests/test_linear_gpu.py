@@ -527,3 +527,40 @@ def test_tiles_spread_over_workgroups(dev, M, nt):
     _lib.fused_linear(x, w, tiles, M=M, K=K, ln=ln)
     ref = F.linear(F.layer_norm(x, (K,), *ln), w, b)
     torch.testing.assert_close(out, ref, rtol=1e-4, atol=2e-4)
+
+
+@pytest.mark.parametrize("case", ["attention", "glu", "plain"])
+def test_fp32_weights_stationary_matches_staged(dev, case):
+    """Long fp32 launches: ragged last slabs, operand tiles of a row length that is no multiple of 32, channel-major GLU tiles beside
+    plain ones, gate, residual and a partly filled last tile; the staged kernel normalises and multiplies in the same order."""
+    from fastfold_amd import _lib
+    g = torch.Generator().manual_seed(3)
+    rnd = lambda *sh: torch.randn(*sh, generator=g).to(dev)
+    r, K, nt = {"attention": (97, 128, 9), "glu": (176, 128, 5), "plain": (97, 256, 4)}[case]
+    M = r * r
+    x, w, b = rnd(M, K), rnd(nt * 128, K) / K ** 0.5, rnd(nt * 128)
+    ln, mask = (rnd(K), rnd(K)), (rnd(r) > 0).float()
+    gate, resid, NT = rnd(M, 512), rnd(M, 512), (r + 31) // 32
+    got = []
+    for staged in (True, False):
+        bp = lambda i: b.data_ptr() + 512 * i
+        if case == "attention":
+            outs = [torch.zeros(r, 4, NT, 1024, device=dev) for _ in range(8)] + [torch.zeros(4, NT, NT, 1024, device=dev)]
+            kinds = [_lib.FFK_TILE_QK, _lib.FFK_TILE_V, _lib.FFK_TILE_ACC, _lib.FFK_TILE_V] * 2
+            tiles = [_lib.make_tile(o, kind=k, inner=r, s_o=4 * NT * 1024, s_h=NT * 1024, bias=bp(i), scale=0.5 + i, act=i % 3,
+                                    rowmask=mask if i > 5 else None, m_si=1) for i, (o, k) in enumerate(zip(outs, kinds))]
+            tiles.append(_lib.make_tile(outs[8], kind=_lib.FFK_TILE_BIAS, inner=r, s_o=NT * 1024, s_h=NT * NT * 1024, ncols=4, bias=bp(8)))
+        elif case == "glu":
+            outs = [torch.zeros(256, M, device=dev), torch.zeros(M, 128, device=dev)]
+            tiles = [_lib.make_tile(outs[0].data_ptr() + 256 * i * M, inner=r, s_o=r, s_i=1, s_h=32 * M, s_d=M, glu=1, ncols=64,
+                                    bias=bp(i), rowmask=mask, m_so=1) for i in range(4)]
+            tiles.append(_lib.make_tile(outs[1], inner=M, s_i=128, bias=bp(4), act=_lib.FFK_ACT_SIGMOID))
+        else:
+            outs = [torch.zeros(M, 512, device=dev)]
+            tiles = [_lib.make_tile(outs[0].data_ptr() + 512 * i, inner=M, s_i=512, bias=bp(i), ncols=128 if i < 3 else 36,
+                                    gate=gate.data_ptr() + 512 * i if i % 2 else None, gate_ld=512,
+                                    resid=resid.data_ptr() + 512 * i if i else None) for i in range(nt)]
+        _lib.fused_linear(x, w, tiles, M=M, K=K, ln=ln, staged=staged)
+        got.append(outs)
+    for a, c in zip(*got):
+        assert torch.isfinite(a).all() and float((a - c).abs().max()) <= 1e-5 * float(a.abs().max())
