@@ -1,28 +1,35 @@
 // Batched NT GEMM with a K loop (see ffk_bgemm_nt in include/ffk.h).
 //
-// 128x128 output tile per workgroup, 4 wavefronts in a 2x2 grid, each owning 64x64 as
-// 2x2 MFMA 32x32 tiles.  A and B K-chunks (128 bytes of K per row) stream through a
-// double-buffered LDS ring with register prefetch.  As in the fused linear kernel the MFMA
-// computes C^T (rows of B are the M-operand) so that a lane holds 4 consecutive n of one
-// row m, and the tile is staged through LDS for 16-byte stores.
+// A workgroup's 4 wavefronts compute one output tile.  K-chunks of A and B stream through a double-buffered LDS ring with
+// register prefetch.  As in the fused linear kernel the MFMA computes C^T (rows of B are the M-operand) so that a lane holds
+// 4 consecutive n of one row m, and the tile is staged through LDS for 16-byte stores.  Three tiles (see launch_tile):
+//   128 x 128, chunks of 128 bytes, 64 x 64 per wave       (four 32 x 32 products per two fragments of each operand)
+//    64 x  64, chunks of 256 bytes, 32 x 32 per wave
+//    32 x  32, chunks of 4 x 128 bytes, each wave takes one quarter of K (fp32, K >= 512)
+// Every tile gives the same bits (callers cut their rows into pieces as memory allows, and pieces take other tiles): products are
+// added in ascending order of K, for fp32 and K >= 512 within quarters of K, as ((q0 + q1) + q2) + q3.
 #include "ffk_common.h"
 #include <type_traits>
 
 namespace {
 
-constexpr int BT = 128;
 constexpr int THREADS = 256;
+constexpr int BG_QUARTERS = 512;                   // K from which fp32 products are added in quarters of K
 
-template <typename T, typename OT>
-__global__ __launch_bounds__(THREADS) void bgemm_nt_kernel(const ffk_bgemm_desc d) {
+template <typename T, typename OT, int BT>
+__global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_desc d) {
     typedef Mma<T> MM;
     constexpr int VEC = DT<T>::VEC;
     constexpr int ES = sizeof(T);
     constexpr int OES = sizeof(OT);
     constexpr int OVEC = 16 / OES;
     constexpr bool XS_OK = std::is_same<OT, bf16_t>::value;     // outputs that may carry a residual tail
-    constexpr int BK = 128 / ES;                   // K elements per chunk (128 bytes per row)
-    constexpr int P = 128 + 16;                    // ring row pitch (bytes)
+    constexpr int WT = BT == 128 ? 2 : 1;          // 32 x 32 blocks per wave and dimension
+    constexpr bool KSPLIT = BT == 32;
+    constexpr bool QUARTERS = std::is_same<T, float>::value;    // sums in quarters of K possible
+    constexpr int BKB = 128 * 128 / BT;            // bytes of K per row and chunk
+    constexpr int BK = BKB / ES;
+    constexpr int P = BKB + 16;                    // ring row pitch (bytes)
     constexpr int SLOT = BT * P;
     constexpr int CP = BT * OES + 16;              // staged C pitch [m][n]
     constexpr int NV = BT * (BK / VEC) / THREADS;  // 16-byte vectors per thread per operand chunk (= 4)
@@ -33,7 +40,7 @@ __global__ __launch_bounds__(THREADS) void bgemm_nt_kernel(const ffk_bgemm_desc 
     unsigned char* sC = smem;                      // aliases the ring after the K loop
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = KSPLIT ? 0 : wave >> 1, wn = KSPLIT ? 0 : wave & 1;
     const int l32 = lane & 31, half = lane >> 5;
     const int M = d.M, N = d.N, K = d.K;
     // Workgroup -> tile.  Consecutive workgroup ids go to the eight XCDs in turn, each with its own L2.
@@ -53,13 +60,17 @@ __global__ __launch_bounds__(THREADS) void bgemm_nt_kernel(const ffk_bgemm_desc 
     const T* A = (const T*)d.a + (long)bz * d.a_bs;
     const T* B = (const T*)d.b + (long)bz * d.b_bs;
 
+    const int kq = QUARTERS && K >= BG_QUARTERS ? (K + 255) / 256 * 64 : K;     // length of a quarter (whole chunks)
+    auto k_of = [&](int kc, int c) {               // K index of vector c of a chunk row
+        return KSPLIT ? c / (BK / VEC / 4) * kq + kc * (BK / 4) + c % (BK / VEC / 4) * VEC : kc * BK + c * VEC;
+    };
     Vec16<T> ra[NV], rb[NV];
     auto fetch = [&](int kc) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int v = tid + THREADS * i;
             const int r = v / (BK / VEC), c = v % (BK / VEC);
-            const int k = kc * BK + c * VEC;
+            const int k = k_of(kc, c);
             long ma = m0 + r;
             if (ma >= M) ma = M - 1;
             long nb = n0 + r;
@@ -76,7 +87,7 @@ __global__ __launch_bounds__(THREADS) void bgemm_nt_kernel(const ffk_bgemm_desc 
         for (int i = 0; i < NV; ++i) {
             const int v = tid + THREADS * i;
             const int r = v / (BK / VEC), c = v % (BK / VEC);
-            const bool tail = kc * BK + c * VEC >= K;
+            const bool tail = k_of(kc, c) >= K;
             Vec16<T> xa = ra[i], xb = rb[i];
             if (tail) {
 #pragma unroll
@@ -87,38 +98,83 @@ __global__ __launch_bounds__(THREADS) void bgemm_nt_kernel(const ffk_bgemm_desc 
         }
     };
 
-    f32x16 acc[2][2];   // [ni][mi]
+    f32x16 acc[WT][WT];   // [ni][mi]
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < WT; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < WT; ++b)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
 
-    const int kchunks = (K + BK - 1) / BK;
+    f32x16 sum[QUARTERS && !KSPLIT ? WT : 1][QUARTERS && !KSPLIT ? WT : 1];       // of the finished quarters
+    int quarter = 0;
+    auto end_quarter = [&]() {
+#pragma unroll
+        for (int a = 0; a < WT; ++a)
+#pragma unroll
+            for (int b = 0; b < WT; ++b)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) sum[a][b][v] = quarter ? sum[a][b][v] + acc[a][b][v] : acc[a][b][v];
+        ++quarter;
+    };
+    const int kchunks = KSPLIT ? kq / (BK / 4) : (K + BK - 1) / BK;
     fetch(0);
     for (int kc = 0; kc < kchunks; ++kc) {
+        if constexpr (QUARTERS && !KSPLIT) {
+            if (kc * BK == (quarter + 1) * kq) {
+                end_quarter();
+#pragma unroll
+                for (int a = 0; a < WT; ++a)
+#pragma unroll
+                    for (int b = 0; b < WT; ++b)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
+            }
+        }
         const int slot = kc & 1;
         commit(slot, kc);
         lds_barrier();
         if (kc + 1 < kchunks) fetch(kc + 1);
-        const unsigned char* pa = sA + slot * SLOT + (wm * 64 + l32) * P + half * (MM::KLANE * ES);
-        const unsigned char* pb = sB + slot * SLOT + (wn * 64 + l32) * P + half * (MM::KLANE * ES);
+        const unsigned char* pa = sA + slot * SLOT + (wm * WT * 32 + l32) * P + half * (MM::KLANE * ES);
+        const unsigned char* pb = sB + slot * SLOT + (wn * WT * 32 + l32) * P + half * (MM::KLANE * ES);
 #pragma unroll
-        for (int ks = 0; ks < BK / MM::KSTEP; ++ks) {
-            typename MM::Frag fa[2], fb[2];
+        for (int k0 = 0; k0 < BK / MM::KSTEP / (KSPLIT ? 4 : 1); ++k0) {
+            const int ks = KSPLIT ? wave * (BK / MM::KSTEP / 4) + k0 : k0;
+            typename MM::Frag fa[WT], fb[WT];
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
+            for (int i = 0; i < WT; ++i) {
                 fa[i] = *reinterpret_cast<const typename MM::Frag*>(pa + i * 32 * P + ks * MM::KSTEP * ES);
                 fb[i] = *reinterpret_cast<const typename MM::Frag*>(pb + i * 32 * P + ks * MM::KSTEP * ES);
             }
 #pragma unroll
-            for (int ni = 0; ni < 2; ++ni)
+            for (int ni = 0; ni < WT; ++ni)
 #pragma unroll
-                for (int mi = 0; mi < 2; ++mi) MM::mma(acc[ni][mi], fb[ni], fa[mi]);
+                for (int mi = 0; mi < WT; ++mi) MM::mma(acc[ni][mi], fb[ni], fa[mi]);
+        }
+    }
+    if constexpr (QUARTERS && !KSPLIT) {
+        if (quarter) {
+            end_quarter();
+#pragma unroll
+            for (int a = 0; a < WT; ++a)
+#pragma unroll
+                for (int b = 0; b < WT; ++b) acc[a][b] = sum[a][b];
         }
     }
     lds_barrier();
+    if constexpr (KSPLIT) {                        // wave 0 adds the quarters
+        float* red = reinterpret_cast<float*>(smem);
+        if (wave) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) red[((wave - 1) * 16 + v) * 64 + lane] = acc[0][0][v];
+        }
+        lds_barrier();
+        if (wave == 0) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[0][0][v] = ((acc[0][0][v] + red[v * 64 + lane]) + red[(16 + v) * 64 + lane]) + red[(32 + v) * 64 + lane];
+        }
+        lds_barrier();
+    }
 
     // row offsets of this tile, one integer division per row (kept in LDS for phase 2)
     __shared__ long s_off[BT];
@@ -134,36 +190,38 @@ __global__ __launch_bounds__(THREADS) void bgemm_nt_kernel(const ffk_bgemm_desc 
     // (bias / rowdiv are fetched with clamped indices, i.e. without per-lane branches, so the loads
     // are issued back to back; out-of-range values are computed but never stored)
     const T* bias = (const T*)d.bias;
-    float bv[2][4][4];
+    if (!KSPLIT || wave == 0) {
+        float bv[WT][4][4];
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
+        for (int ni = 0; ni < WT; ++ni)
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                long n = n0 + wn * 64 + ni * 32 + 8 * g + 4 * half + e;
-                n = n < N ? n : N - 1;
-                bv[ni][g][e] = bias ? DT<T>::to_f(bias[n]) : 0.0f;
-            }
-#pragma unroll
-    for (int mi = 0; mi < 2; ++mi) {
-        const int mr = wm * 64 + mi * 32 + l32;
-        long m = m0 + mr;
-        m = m < M ? m : M - 1;
-        float rdiv = 1.0f;
-        if (d.rowdiv) rdiv = 1.0f / (d.rowdiv[(long)bz * M + m] + d.div_eps);
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int nc = wn * 64 + ni * 32 + 8 * g + 4 * half;
-                OT* dst = reinterpret_cast<OT*>(sC + mr * CP + nc * OES);
+            for (int g = 0; g < 4; ++g)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    float x = acc[ni][mi][4 * g + e] + bv[ni][g][e];
-                    if (d.act == FFK_ACT_RELU) x = relu_f(x);
-                    else if (d.act == FFK_ACT_SIGMOID) x = sigmoid_f(x);
-                    dst[e] = DT<OT>::from_f(x * d.scale * rdiv);
+                    long n = n0 + wn * WT * 32 + ni * 32 + 8 * g + 4 * half + e;
+                    n = n < N ? n : N - 1;
+                    bv[ni][g][e] = bias ? DT<T>::to_f(bias[n]) : 0.0f;
+                }
+#pragma unroll
+        for (int mi = 0; mi < WT; ++mi) {
+            const int mr = wm * WT * 32 + mi * 32 + l32;
+            long m = m0 + mr;
+            m = m < M ? m : M - 1;
+            float rdiv = 1.0f;
+            if (d.rowdiv) rdiv = 1.0f / (d.rowdiv[(long)bz * M + m] + d.div_eps);
+#pragma unroll
+            for (int ni = 0; ni < WT; ++ni) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const int nc = wn * WT * 32 + ni * 32 + 8 * g + 4 * half;
+                    OT* dst = reinterpret_cast<OT*>(sC + mr * CP + nc * OES);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float x = acc[ni][mi][4 * g + e] + bv[ni][g][e];
+                        if (d.act == FFK_ACT_RELU) x = relu_f(x);
+                        else if (d.act == FFK_ACT_SIGMOID) x = sigmoid_f(x);
+                        dst[e] = DT<OT>::from_f(x * d.scale * rdiv);
+                    }
                 }
             }
         }
@@ -178,21 +236,22 @@ __global__ __launch_bounds__(THREADS) void bgemm_nt_kernel(const ffk_bgemm_desc 
     if constexpr (XS_OK) xtail = d.xtail ? (int8_t*)d.xtail + (long)bz * d.o_bs : nullptr;
     if (d.s_d == 1) {
         constexpr int VPR = BT / OVEC;
-        constexpr int N_IT = BT * VPR / THREADS;
+        constexpr int N_V = BT * VPR, N_IT = (N_V + THREADS - 1) / THREADS, NB = N_IT < 4 ? N_IT : 4;
         // vector path when every row pitch / base keeps 16-byte alignment and N is a multiple of the vector
         const bool vec_ok = (N % OVEC) == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0 &&
                             (!resid || (reinterpret_cast<uintptr_t>(resid) & 15u) == 0) && (d.s_o % OVEC) == 0 &&
                             (d.s_i % OVEC) == 0 && (d.s_h % OVEC) == 0;
         if (vec_ok) {
             const long n_last = N - OVEC;
+            const bool live = N_V >= THREADS || tid < N_V;
 #pragma unroll 1
-            for (int i0 = 0; i0 < N_IT; i0 += 4) {
-                Vec16<OT> x[4], rv[4];
-                u32x2 tv[4];
-                long o[4];
+            for (int i0 = 0; i0 < N_IT; i0 += NB) {
+                Vec16<OT> x[NB], rv[NB];
+                u32x2 tv[NB];
+                long o[NB];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int v = tid + THREADS * (i0 + j);
+                for (int j = 0; j < NB; ++j) {
+                    const int v = N_V >= THREADS ? tid + THREADS * (i0 + j) : tid % N_V;       // the repetitions store nothing
                     const int r = v / VPR, c = (v % VPR) * OVEC;
                     long n = n0 + c;
                     n = n <= n_last ? n : n_last;
@@ -202,8 +261,8 @@ __global__ __launch_bounds__(THREADS) void bgemm_nt_kernel(const ffk_bgemm_desc 
                     if (xtail) tv[j] = *reinterpret_cast<const u32x2*>(xtail + o[j]);
                 }
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int v = tid + THREADS * (i0 + j);
+                for (int j = 0; j < NB; ++j) {
+                    const int v = N_V >= THREADS ? tid + THREADS * (i0 + j) : tid % N_V;       // the repetitions store nothing
                     const int r = v / VPR, c = (v % VPR) * OVEC;
                     if constexpr (XS_OK) {
                         if (xtail) {
@@ -214,7 +273,7 @@ __global__ __launch_bounds__(THREADS) void bgemm_nt_kernel(const ffk_bgemm_desc 
                             u32x4 hv;
                             u32x2 tn;
                             xs_encode8(f, hv, tn);
-                            if (m0 + r < M && n0 + c < N) {
+                            if (live && m0 + r < M && n0 + c < N) {
                                 *reinterpret_cast<u32x4*>(out + o[j]) = hv;
                                 *reinterpret_cast<u32x2*>(xtail + o[j]) = tn;
                             }
@@ -226,7 +285,7 @@ __global__ __launch_bounds__(THREADS) void bgemm_nt_kernel(const ffk_bgemm_desc 
                         for (int e = 0; e < OVEC; ++e)
                             x[j].e[e] = DT<OT>::from_f(DT<OT>::to_f(x[j].e[e]) + DT<OT>::to_f(rv[j].e[e]));
                     }
-                    if (m0 + r < M && n0 + c < N) st16(out + o[j], x[j]);
+                    if (live && m0 + r < M && n0 + c < N) st16(out + o[j], x[j]);
                 }
             }
         } else {
@@ -259,21 +318,49 @@ __global__ __launch_bounds__(THREADS) void bgemm_nt_kernel(const ffk_bgemm_desc 
     }
 }
 
-template <typename T, typename OT>
-int launch_bgemm(const ffk_bgemm_desc& d, hipStream_t st) {
-    size_t ring = 4 * (size_t)BT * (128 + 16);
+template <typename T, typename OT, int BT>
+int launch_tile(const ffk_bgemm_desc& d, hipStream_t st) {
+    size_t ring = 4 * (size_t)BT * (128 * 128 / BT + 16);
     size_t ct = (size_t)BT * (BT * sizeof(OT) + 16);
     const size_t smem = ring > ct ? ring : ct;
     static FfkLdsReservation lds_reserved;
     {
-        const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)bgemm_nt_kernel<T, OT>, smem, "ffk_bgemm_nt");
+        const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)bgemm_nt_kernel<T, OT, BT>, smem, "ffk_bgemm_nt");
         if (rc_lds != FFK_OK) return rc_lds;
     }
     const long tiles = (long)ffk_cdiv(d.M, BT) * ffk_cdiv(d.N, BT) * d.batch;
     FFK_REQUIRE(tiles < (1L << 31) - 8, FFK_ERR_SHAPE, "ffk_bgemm_nt: %ld output tiles exceed the grid limit", tiles);
     dim3 grid((unsigned)(d.batch >= 8 ? 8 * ffk_cdiv(tiles, 8) : tiles));
-    bgemm_nt_kernel<T, OT><<<grid, THREADS, smem, st>>>(d);
+    bgemm_nt_kernel<T, OT, BT><<<grid, THREADS, smem, st>>>(d);
     return ffk_check_launch("ffk_bgemm_nt");
+}
+
+// Which tile: the launch takes about  start + rounds * (each + per_k * K)  microseconds, rounds = tiles / 256 CUs rounded up.  The
+// constants are fitted to measured launches of 32 .. 24 576 rows, 32 .. 5 120 columns and K = 16 .. 1 024: a small tile pays its
+// latencies over less work, but a large one leaves CUs without a tile (fp32, 2 048 x 256, K = 1 024: 81 us with 16 tiles of 128,
+// 28 us with 128 of 64, 18.7 us with 512 of 32; bf16: 14.0 us with 16 of 256 x 128, 9.8 us with 128 of 64) or works on padding
+// (128 products of 64 x 64 x 64 in fp32: 12.4, 5.7, 6.3 us).  0: the large tiles of the other kernel, if it takes the launch.
+int pick_tile(const ffk_bgemm_desc& d, bool large) {
+    auto cost = [&](int bm, int bn, double start, double each, double per_k) {
+        return start + ffk_cdiv((long)ffk_cdiv(d.M, bm) * ffk_cdiv(d.N, bn) * d.batch, 256) * (each + per_k * d.K);
+    };
+    const bool f = d.dtype == FFK_F32;
+    const double c128 = f ? cost(128, 128, 2.0, 6.8, 0.0645) : cost(128, 128, 3.5, 5.0, 0.0060);
+    const double c64 = f ? cost(64, 64, 3.0, 2.3, 0.0182) : cost(64, 64, 3.0, 1.9, 0.0035);
+    if (large && (c64 >= c128 || c64 >= cost(256, d.N <= 128 ? 128 : 256, 4.7, 0.0, 0.0095))) return 0;
+    if (f && d.K >= BG_QUARTERS) {
+        const double c32 = cost(32, 32, 2.5, 2.1, 0.0060);
+        if (c32 < c64 && c32 < c128) return 32;
+    }
+    return c64 < c128 ? 64 : 128;
+}
+
+template <typename T, typename OT>
+int launch_bgemm(const ffk_bgemm_desc& d, int tile, hipStream_t st) {
+    if constexpr (sizeof(T) == 4) {
+        if (tile == 32) return launch_tile<T, OT, 32>(d, st);
+    }
+    return tile == 64 ? launch_tile<T, OT, 64>(d, st) : launch_tile<T, OT, 128>(d, st);
 }
 
 }  // namespace
@@ -294,14 +381,16 @@ extern "C" int ffk_bgemm_nt(const ffk_bgemm_desc* d, void* stream) {
                     d->a_bs % vec == 0 && d->b_bs % vec == 0,
                 FFK_ERR_ALIGN, "ffk_bgemm_nt: operand rows must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
-    {
+    int tile = pick_tile(*d, d->dtype == FFK_BF16);
+    if (tile == 0) {
         int status = FFK_OK;
         if (ffk_bgemm_big_try(d, st, &status)) return status;
+        tile = pick_tile(*d, false);
     }
     if (d->dtype == FFK_BF16) {
-        return d->out_f32 ? launch_bgemm<bf16_t, float>(*d, st) : launch_bgemm<bf16_t, bf16_t>(*d, st);
+        return d->out_f32 ? launch_bgemm<bf16_t, float>(*d, tile, st) : launch_bgemm<bf16_t, bf16_t>(*d, tile, st);
     } else if (d->dtype == FFK_F32) {
-        return launch_bgemm<float, float>(*d, st);
+        return launch_bgemm<float, float>(*d, tile, st);
     }
     return ffk_fail(FFK_ERR_DTYPE, "ffk_bgemm_nt: unsupported dtype tag %d", d->dtype);
 }

@@ -23,7 +23,7 @@ template <typename T> __device__ __forceinline__ Vec16<T> pack(const float* f) {
 // dx = resid + LayerNorm'(x)^T dy and, optionally, xn = LayerNorm(x) for the weight gradient behind it.  A row is LPR = C / VEC
 // adjacent lanes with one 16-byte vector each; mean and rstd are recomputed from the row (it is read anyway, and nothing has
 // to be kept from the forward pass).  A thread sums its columns of dgamma / dbeta over the rows it sees; the workgroup adds
-// them in LDS and leaves one partial row per workgroup, which slice_sum-like reduction follows in ln_finish_kernel: no
+// them in LDS and leaves one partial row per workgroup, which ln_finish_kernel adds up: no
 // atomics, the same result every time.
 template <typename T, int C>
 __global__ __launch_bounds__(TR_THREADS) void ln_bwd_rows_kernel(T* dx, T* __restrict__ xn, float* __restrict__ part,
@@ -107,22 +107,33 @@ __global__ __launch_bounds__(TR_THREADS) void ln_bwd_rows_kernel(T* dx, T* __res
         part[(long)blockIdx.x * 2 * C + i] = (red[i] + red[2 * C + i]) + (red[4 * C + i] + red[6 * C + i]);
 }
 
-// dgamma[c] / dbeta[c] = sum of the partial rows: a workgroup per 32 columns, eight groups of 32 lanes over the partial rows
+// dgamma[c] / dbeta[c] = sum of the partial rows: a workgroup per 16 columns, 64 groups of four lanes over the partial rows (a
+// workgroup per 32 columns with eight groups walked 128 rows one load after the other: 34 us at C = 256, now ... us)
 template <typename T>
 __global__ __launch_bounds__(256) void ln_finish_kernel(T* __restrict__ dgamma, T* __restrict__ dbeta, const float* __restrict__ part,
                                                         int blocks, int C) {
-    __shared__ float red[8][32];
-    const int l = threadIdx.x & 31, gpr = threadIdx.x >> 5;
-    const int col = blockIdx.x * 32 + l;
-    float s = 0.0f;
-    for (int b = gpr; b < blocks; b += 8) s += part[(long)b * 2 * C + col];
-    red[gpr][l] = s;
+    __shared__ f32x4 red[256];
+    const int tid = threadIdx.x, col = blockIdx.x * 16 + (tid & 3) * 4;
+    f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+    for (int b = tid >> 2; b < blocks; b += 64) s += *reinterpret_cast<const f32x4*>(part + (long)b * 2 * C + col);
+    red[tid] = s;
     __syncthreads();
-    if (gpr) return;
+    if (tid < 64) {
+        s = (red[tid] + red[tid + 64]) + (red[tid + 128] + red[tid + 192]);
 #pragma unroll
-    for (int j = 1; j < 8; ++j) s += red[j][l];
-    if (col < C) dgamma[col] = DT<T>::from_f(s);
-    else dbeta[col - C] = DT<T>::from_f(s);
+        for (int e = 0; e < 4; ++e) {
+            float v = s[e];
+#pragma unroll
+            for (int w = 4; w < 64; w <<= 1) v += __shfl_xor(v, w, 64);
+            s[e] = v;
+        }
+        if (tid < 4) {
+            T* out = col < C ? dgamma + col : dbeta + (col - C);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[e] = DT<T>::from_f(s[e]);
+        }
+    }
 }
 
 // --------------------------------------------------------------------------------------------- row scaling ----
@@ -372,7 +383,7 @@ int ln_bwd_launch(T* dx, T* xn, T* dgamma, T* dbeta, float* ws, const T* dy, con
 #undef FFK_LN_BWD
     int rc = ffk_check_launch("ffk_layernorm_bwd_rows");
     if (rc != FFK_OK) return rc;
-    ln_finish_kernel<T><<<2 * C / 32, 256, 0, st>>>(dgamma, dbeta, ws, blocks, C);
+    ln_finish_kernel<T><<<2 * C / 16, 256, 0, st>>>(dgamma, dbeta, ws, blocks, C);
     return ffk_check_launch("ffk_layernorm_bwd_rows");
 }
 

@@ -211,39 +211,55 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
     }
 }
 
-// sum over the slices of part[s][i], plus acc[i] if READ: to acc[i] if WRITE, else to out.  Four adjacent values per lane, the
-// slices spread over the four waves.  Element i = (row n, column k) of out is at (n / inner) * o_so + (n % inner) * o_si + k * o_sk.
+// One sum over slices: of part[s][i] over s, plus acc[i] if READ: to acc[i] if WRITE, else to out.  Element i = (row n, column k) of
+// out is at (n / inner) * o_so + (n % inner) * o_si + k * o_sk.
+struct SliceSum {
+    void* out;
+    const float* part;
+    float* acc;
+    long n, pitch, o_so, o_si, o_sk;
+    int K;
+    unsigned inner, blocks;                              // workgroups of 256 values
+};
+
+// Four adjacent values per lane, the slices spread over the four waves.  The matrix and its column sums go in one launch (a
+// launch of its own took the few hundred column sums 5 us): workgroups from a.blocks on belong to b.
 template <typename OT>
-__global__ __launch_bounds__(256) void slice_sum_kernel(OT* __restrict__ out, const float* __restrict__ part, float* acc, int flags,
-                                                        int slices, long n, int K, unsigned inner, long o_so, long o_si, long o_sk,
-                                                        long pitch) {
+__global__ __launch_bounds__(256) void slice_sum_kernel(const SliceSum a, const SliceSum b, int flags, int slices) {
     __shared__ f32x4 red[3][64];
+    const bool second = blockIdx.x >= a.blocks;
+    const SliceSum& q = second ? b : a;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long i = ((long)blockIdx.x * 64 + lane) * 4;
+    const long i = ((long)(blockIdx.x - (second ? a.blocks : 0u)) * 64 + lane) * 4;
     f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (i < n) {
-#pragma unroll 4
-        for (int sl = wave; sl < slices; sl += 4) s += *reinterpret_cast<const f32x4*>(part + (long)sl * pitch + i);
+    if (i < q.n) {
+        const float* p = q.part + i;
+        const long pitch = q.pitch;
+#pragma unroll 8
+        for (int sl = wave; sl < slices; sl += 4) s += *reinterpret_cast<const f32x4*>(p + (long)sl * pitch);
     }
     if (wave) red[wave - 1][lane] = s;
     __syncthreads();
-    if (wave || i >= n) return;
+    if (wave || i >= q.n) return;
     s = (s + red[0][lane]) + (red[1][lane] + red[2][lane]);
-    if (flags & FFK_WGRAD_READ) s += *reinterpret_cast<const f32x4*>(acc + i);
+    if (flags & FFK_WGRAD_READ) s += *reinterpret_cast<const f32x4*>(q.acc + i);
     if (flags & FFK_WGRAD_WRITE) {
-        *reinterpret_cast<f32x4*>(acc + i) = s;
+        *reinterpret_cast<f32x4*>(q.acc + i) = s;
         return;
     }
-    const unsigned row = (unsigned)(i / K), k = (unsigned)(i - (long)row * K), hi = row / inner;      // K % 4 == 0
-    OT* o = out + (long)hi * o_so + (long)(row - hi * inner) * o_si + (long)k * o_sk;
+    const unsigned row = (unsigned)(i / q.K), k = (unsigned)(i - (long)row * q.K), hi = row / q.inner;      // K % 4 == 0
+    OT* o = (OT*)q.out + (long)hi * q.o_so + (long)(row - hi * q.inner) * q.o_si + (long)k * q.o_sk;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e * o_sk] = DT<OT>::from_f(s[e]);
+    for (int e = 0; e < 4; ++e) o[e * q.o_sk] = DT<OT>::from_f(s[e]);
+}
+
+SliceSum slice_sum(void* out, const float* part, float* acc, long n, int K, long inner, long so, long si, long sk, long pitch) {
+    return SliceSum{out, part, acc, n, pitch, so, si, sk, K, (unsigned)inner, (unsigned)((n + 255) / 256)};
 }
 
 template <typename T>
-int slice_sum(T* out, const float* part, float* acc, int flags, long slices, long n, int K, unsigned inner, long so, long si, long sk,
-              long pitch, hipStream_t st) {
-    slice_sum_kernel<T><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(out, part, acc, flags, (int)slices, n, K, inner, so, si, sk, pitch);
+int slice_sum_launch(const SliceSum& a, const SliceSum& b, int flags, long slices, hipStream_t st) {
+    slice_sum_kernel<T><<<a.blocks + b.blocks, 256, 0, st>>>(a, b, flags, (int)slices);
     return ffk_check_launch("ffk_weight_grad");
 }
 
@@ -260,10 +276,10 @@ int launch_weight_grad(const WgArgs& a, void* out, long n_out, void* colsum, lon
     rc = ffk_check_launch("ffk_weight_grad");
     if (rc != FFK_OK) return rc;
     const long nk = (long)a.N * a.K;
-    rc = slice_sum<T>((T*)out, a.part, acc, flags, a.slices, n_out * a.K, a.K, (unsigned)o_inner, o_so, o_si, o_sk, nk, st);
-    if (rc != FFK_OK || !a.csum) return rc;
-    return slice_sum<T>((T*)colsum, a.csum + cs_first, acc ? acc + n_out * a.K : nullptr, flags, a.slices, cs_count, (int)cs_count, 1u, 0, 0, 1,
-                        a.N, st);
+    const SliceSum m = slice_sum(out, a.part, acc, n_out * a.K, a.K, o_inner, o_so, o_si, o_sk, nk);
+    SliceSum c{};
+    if (a.csum) c = slice_sum(colsum, a.csum + cs_first, acc ? acc + n_out * a.K : nullptr, cs_count, (int)cs_count, 1, 0, 0, 1, a.N);
+    return slice_sum_launch<T>(m, c, flags, a.slices, st);
 }
 
 }  // namespace
@@ -316,10 +332,10 @@ extern "C" int ffk_slice_sum(void* out, const float* part, int64_t slices, int64
                 FFK_ERR_SHAPE, "ffk_slice_sum: bad shape slices=%ld N=%ld K=%ld", (long)slices, (long)N, (long)K);
     FFK_REQUIRE(ffk_aligned16(part), FFK_ERR_ALIGN, "ffk_slice_sum: the partial sums must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
-    const unsigned inner = (unsigned)(o_inner < N ? o_inner : N);
+    const SliceSum q = slice_sum(out, part, nullptr, N * K, (int)K, o_inner < N ? o_inner : N, o_so, o_si, o_sk, N * K);
     switch (dtype) {
-        case FFK_BF16: return slice_sum<bf16_t>((bf16_t*)out, part, nullptr, 0, slices, N * K, (int)K, inner, o_so, o_si, o_sk, N * K, st);
-        case FFK_F32: return slice_sum<float>((float*)out, part, nullptr, 0, slices, N * K, (int)K, inner, o_so, o_si, o_sk, N * K, st);
+        case FFK_BF16: return slice_sum_launch<bf16_t>(q, SliceSum{}, 0, slices, st);
+        case FFK_F32: return slice_sum_launch<float>(q, SliceSum{}, 0, slices, st);
         default: return ffk_fail(FFK_ERR_DTYPE, "ffk_slice_sum: unsupported dtype tag %d", dtype);
     }
 }

@@ -159,6 +159,23 @@ def test_attention_moving_reference(dev, dtype, tol, slope):
     assert _rel(got, ref) < tol
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("C,M,N,K,resid", [(9, 33, 65, 40, False), (1, 40, 200, 24, True), (3, 70, 36, 1032, True), (1, 2051, 132, 520, True),
+                                           (9, 129, 257, 8, False), (2, 500, 500, 136, False)])
+def test_bgemm_tiles(dev, C, M, N, K, resid, dtype):
+    """Sizes that take each output tile (32, 64, 128) with partly filled tiles and chunks of K, in place on a residual or not."""
+    from fastfold_amd import _lib
+    g = torch.Generator().manual_seed(C * M + N + K)
+    a, b = torch.randn(C, M, K, generator=g).to(dev, dtype), torch.randn(C, N, K, generator=g).to(dev, dtype)
+    out = torch.randn(C, M, N, generator=g).to(dev, dtype) if resid else torch.full((C, M, N), float("nan"), dtype=dtype, device=dev)
+    bias = torch.randn(N, generator=g).to(dev, dtype)
+    ref = np.einsum("cmk,cnk->cmn", _np(a), _np(b)) + _np(bias) + (_np(out) if resid else 0)
+    _lib.bgemm_nt(a, b, out, M=M, N=N, K=K, lda=K, ldb=K, batch=C, a_bs=M * K, b_bs=N * K, o_bs=M * N, bias=bias,
+                  resid=out if resid else None)
+    got = _np(out)
+    assert np.isfinite(got).all() and np.abs(got - ref).max() < (2e-6 if dtype is torch.float32 else 8e-3) * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-5), (torch.bfloat16, 1e-2)])
 @pytest.mark.parametrize("r", [52, 128, 200])
 def test_bgemm_trimul_contraction(dev, dtype, tol, r):
