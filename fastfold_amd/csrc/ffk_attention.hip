@@ -96,7 +96,12 @@ __device__ __forceinline__ typename Mma<T>::Frag identity_frag(int i, int l32, i
 constexpr int ATT_WAVES = 8;
 constexpr int ATT_THREADS = 64 * ATT_WAVES;
 
-template <typename T, bool HAS_BIAS>
+// HD < 32: heads of 16 or 8 channels, packed two or four to an operand tile (head h is channels HD * (h % G) .. of tile h / G).
+// A wave takes its head's share of the packed tiles: the one fragment of k its channels lie in (for HD = 8 with the other head's
+// half of q zeroed), and the accumulator registers of its channels from the product with v, whose other rows it drops - the
+// kernel is bound by exp2 and by what it reads, and padding such heads to 32 channels made q, k, v and the gate two to four
+// times as large (extra-MSA row attention, 1 024 x 384, 8 heads of 8: projection 142 -> ... us, core 162 -> ... us).
+template <typename T, bool HAS_BIAS, int HD>
 __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention_kernel(
     T* __restrict__ out, const T* __restrict__ q_t, const T* __restrict__ k_t, const T* __restrict__ v_t,
     const T* __restrict__ bias_t, const float* __restrict__ keybias, const int* __restrict__ tileflags,
@@ -125,16 +130,27 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
     const unsigned total = (unsigned)NQG * H * NZ, per_xcd = (total + 7) >> 3;
     const unsigned item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (item >= total) return;                    // whole workgroup leaves together
-    const int wg_q = item % NQG, wg_z = (item / NQG) % NZ;
-    const int h = (item / NQG) / NZ;
+    constexpr int G = 32 / HD;                    // heads per operand tile; those of one tile and batch-row pair run together
+    const int wg_q = item % NQG, rest = item / NQG;
+    const int wg_z = (rest / G) % NZ;
+    const int ht = (rest / G) / NZ, Ht = H / G, h = ht * G + rest % G;
+    const int c0 = HD * (rest % G);               // first channel of the head in its tile
     const int b2_raw = wg_z * 2 + bsel, qt_raw = wg_q * 4 + qsel;
     const bool live = b2_raw < B2 && qt_raw < QT;      // dead waves still help loading and keep the barriers
     const int b2 = b2_raw < B2 ? b2_raw : B2 - 1;
     const int qt = qt_raw < QT ? qt_raw : QT - 1;
-    const long bh = (long)b2 * H + h;
+    const long bh = (long)b2 * Ht + ht;
 
     Ops16<T> qf;
     qf.load(q_t + ((bh * QT + qt) << 10) + lane * 16);
+    if constexpr (HD < 32) {                      // v[0]: the fragment with the head's channels
+        if (c0 >= 16) qf.v[0] = qf.v[1];
+        if constexpr (HD == 8) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if ((e >> 2) != ((c0 >> 3) & 1)) qf.v[0].e[e] = DT<T>::from_f(0.0f);
+        }
+    }
     const float* mp = keybias + (long)b2 * KT * 32 + 4 * half;
     const int* fl = tileflags + (long)b2 * KT;
 
@@ -153,7 +169,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
         if (tile < 4) {
             int bb = wg_z * 2 + (tile & 1);
             bb = bb < B2 ? bb : B2 - 1;
-            base = (tile < 2 ? k_t : v_t) + ((((long)bb * H + h) * KT) << 10);
+            base = (tile < 2 ? k_t : v_t) + ((((long)bb * Ht + ht) * KT) << 10);
         } else {
             int qq = wg_q * 4 + (tile - 4);
             qq = qq < QT ? qq : QT - 1;
@@ -167,7 +183,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
     // gate values of this lane's 16 outputs, fetched now so that their latency is hidden by the loop
     const int q = qt * 32 + l32;
     const int qc = q < Nq ? q : Nq - 1;
-    const long rowo = ((long)b2 * Nq + qc) * (H * 32) + h * 32 + 4 * half;
+    const long rowo = ((long)b2 * Nq + qc) * (H * HD) + ht * 32 + 4 * half;
     // They wait in LDS (each lane's own 16 values), not in registers.
     T* gate_lds = lds + NSLOT * NTILES * 1024 + tid * 16;
     if (gate) {
@@ -279,14 +295,15 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
         f32x16 s;
         auto score_tile = [&]() {
             Ops16<T> kc, bc;
-            kc.load_lds(buf + bsel * 1024, lane);
+            if constexpr (HD == 32) kc.load_lds(buf + bsel * 1024, lane);
+            else kc.v[0] = ld16(buf + bsel * 1024 + ((c0 >> 4) * 64 + lane) * VEC);
             if (HAS_BIAS) bc.load_lds(buf + (4 + qsel) * 1024, lane);
             s = negm;
             // FFK_ATT_HALF_K: elements 8 .. 15 of every lane's sixteen are zero padding in q and k (narrow heads): the
             // second half of the score product adds nothing and is skipped
 #pragma unroll
             for (int i = 0; i < NF / 2; ++i) MM::mma(s, kc.frag(i), qf.frag(i));
-            if (!(flags & FFK_ATT_HALF_K)) {
+            if (HD == 32 && !(flags & FFK_ATT_HALF_K)) {
 #pragma unroll
                 for (int i = NF / 2; i < NF; ++i) MM::mma(s, kc.frag(i), qf.frag(i));
             }
@@ -396,6 +413,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
         }
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
+            if (HD < 32 && (8 * g < c0 || 8 * g >= c0 + HD)) continue;        // another head's channels
             T r4[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -556,31 +574,31 @@ __global__ void key_bias_kernel(float* kb, int* flags, const T* mask, long N, lo
     }
 }
 
-template <typename T, bool HAS_BIAS>
+template <typename T, bool HAS_BIAS, int HD>
 int launch_attention_b(void* out, const void* q, const void* k, const void* v, const void* bias, const float* kb,
                        const int* flags, const void* gate, float* lse, long B2, long H, long Nq, long Nk, int aflags,
                        hipStream_t st) {
     const size_t smem = (3 * (size_t)(HAS_BIAS ? 8 : 4) * 1024 + ATT_THREADS * 16) * sizeof(T) + 16;   // operand ring + gate + redo flag
     static FfkLdsReservation lds_reserved;
     {
-        const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)attention_kernel<T, HAS_BIAS>, smem, "ffk_attention_fwd");
+        const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)attention_kernel<T, HAS_BIAS, HD>, smem, "ffk_attention_fwd");
         if (rc_lds != FFK_OK) return rc_lds;
     }
     const long items = (long)ffk_cdiv((Nq + 31) / 32, 4) * H * ffk_cdiv(B2, 2);
     FFK_REQUIRE(items < (1L << 31) - 8, FFK_ERR_SHAPE, "ffk_attention_fwd: %ld workgroups exceed the grid limit", items);
     dim3 grid((unsigned)(8 * ffk_cdiv(items, 8)));
-    attention_kernel<T, HAS_BIAS><<<grid, ATT_THREADS, smem, st>>>((T*)out, (const T*)q, (const T*)k, (const T*)v,
+    attention_kernel<T, HAS_BIAS, HD><<<grid, ATT_THREADS, smem, st>>>((T*)out, (const T*)q, (const T*)k, (const T*)v,
                                                                   (const T*)bias, kb, flags, (const T*)gate, lse, (int)B2,
                                                                   (int)H, (int)Nq, (int)Nk, aflags);
     return ffk_check_launch("ffk_attention_fwd");
 }
 
-template <typename T>
+template <typename T, int HD = 32>
 int launch_attention(void* out, const void* q, const void* k, const void* v, const void* bias, const float* kb,
                      const int* flags, const void* gate, float* lse, long B2, long H, long Nq, long Nk, int aflags,
                      hipStream_t st) {
-    return bias ? launch_attention_b<T, true>(out, q, k, v, bias, kb, flags, gate, lse, B2, H, Nq, Nk, aflags, st)
-                : launch_attention_b<T, false>(out, q, k, v, nullptr, kb, flags, gate, lse, B2, H, Nq, Nk, aflags, st);
+    return bias ? launch_attention_b<T, true, HD>(out, q, k, v, bias, kb, flags, gate, lse, B2, H, Nq, Nk, aflags, st)
+                : launch_attention_b<T, false, HD>(out, q, k, v, nullptr, kb, flags, gate, lse, B2, H, Nq, Nk, aflags, st);
 }
 
 }  // namespace
@@ -601,9 +619,15 @@ extern "C" int ffk_attention_fwd_lse(void* out, float* lse, const void* q_t, con
     FFK_REQUIRE(ffk_aligned16(out) && ffk_aligned16(q_t) && ffk_aligned16(k_t) && ffk_aligned16(v_t) &&
                     ffk_aligned16(keybias) && (!bias_t || ffk_aligned16(bias_t)) && (!gate || ffk_aligned16(gate)),
                 FFK_ERR_ALIGN, "ffk_attention_fwd: buffers must be 16-byte aligned");
-    FFK_REQUIRE(D == 32 || D == 64 || D == 128, FFK_ERR_SHAPE,
-                "ffk_attention_fwd: head dimension %ld (32, 64 or 128; narrower heads arrive zero-padded to 32)", (long)D);
+    FFK_REQUIRE(D == 8 || D == 16 || D == 32 || D == 64 || D == 128, FFK_ERR_SHAPE,
+                "ffk_attention_fwd: head dimension %ld (8 and 16 packed into 32-channel tiles, 32, 64 or 128)", (long)D);
     hipStream_t st = (hipStream_t)stream;
+    if (D < 32) {
+        FFK_REQUIRE(dtype == FFK_BF16 && H * D % 32 == 0 && !lse && (!gate || (flags & FFK_ATT_GATE_TILED)) && !(flags & FFK_ATT_HALF_K),
+                    FFK_ERR_UNSUPPORTED, "ffk_attention_fwd: packed heads need bf16, whole tiles, a tiled gate or none, and no log-sum-exp");
+        return D == 16 ? launch_attention<bf16_t, 16>(out, q_t, k_t, v_t, bias_t, keybias, tileflags, gate, lse, B2, H, Nq, Nk, flags, st)
+                       : launch_attention<bf16_t, 8>(out, q_t, k_t, v_t, bias_t, keybias, tileflags, gate, lse, B2, H, Nq, Nk, flags, st);
+    }
     if (D != 32) {
         FFK_REQUIRE(!gate && !lse && !(flags & (FFK_ATT_BIAS_PADDED | FFK_ATT_HALF_K)), FFK_ERR_UNSUPPORTED,
                     "ffk_attention_fwd: the gate, the log-sum-exp, padded bias rows and the narrow-head flag are built for head dimension 32 only");

@@ -244,8 +244,9 @@ def key_bias(mask, device, *, B2, N, mask_sb, mask_sn):
 def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_pk, out_bias_pk, c_out,
               mask, mask_sb, mask_sn, bias_t=None, bias_in_launch=False, pb_scratch=None, head_dim=32, budget=None, o_map=None, xtail=None,
               drop=None):
-    """Gated multi-head attention over N tokens for each of B2 batch rows.  The kernels work on 32-wide
-    heads; a narrower head (``head_dim`` < 32) arrives zero-padded to 32 channels in ``w_pk`` / ``wo_pk``,
+    """Gated multi-head attention over N tokens for each of B2 batch rows.  The kernels work on 32-channel tiles.  Heads of
+    8 or 16 channels lie side by side in them (``w_pk.packed_heads``) where the operands are written in accumulator order;
+    elsewhere, and at other widths, a narrower head (``head_dim`` < 32) arrives zero-padded to 32 channels in ``w_pk`` / ``wo_pk``,
     which changes neither the scores nor the used output channels - only the score scale is its own.
 
     x holds the C-channel rows addressed by ``a_map = (inner, s_o, s_i)`` with ``inner`` either B2 * N (plain
@@ -265,9 +266,6 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     """
     dt, dev = x.dtype, x.device
     es = es_of(dt)
-    HC = H * 32
-    if HC % 128 != 0:
-        raise RuntimeError("attention: n_head * 32 must be a multiple of 128 (got %d heads)" % H)
     M = B2 * N
     NT = (N + 31) // 32
     zero = (N % 32) != 0
@@ -275,15 +273,24 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     o_inner, o_so, o_si = a_map if o_map is None else o_map
     if a_inner not in (M, N) or o_inner != a_inner:
         raise RuntimeError("attention: row maps with inner=%d / %d fit neither B2 * N nor N" % (a_inner, o_inner))
-    per_row = 5 * H * NT * 1024 * es
-    slab = B2 if budget is None else min(B2, max(2, (budget // per_row) // 2 * 2))
-    q_t = alloc((slab, H, NT, 1024), dt, dev, zero)
-    k_t = alloc((slab, H, NT, 1024), dt, dev, zero)
-    v_t = alloc((slab, H, NT, 1024), dt, dev, zero)
     # With bf16, 128 input channels and whole key tiles the projection runs on the weights-stationary
     # kernel, which writes q, k and the gate in accumulator order straight from its registers.
     acc_order = dt == torch.bfloat16 and C in (64, 128, 256) and N % 32 == 0
     qk_kind = FFK_TILE_ACC if acc_order else FFK_TILE_QK
+    # Packed heads: nothing is written or read for padding (extra-MSA stack, 8 heads of 8 channels: a quarter of the operand
+    # bytes; template stack, 4 heads of 16: half of them).
+    packed = acc_order and hasattr(w_pk, "packed_heads")
+    if packed:
+        w_pk, gate_bias_pk, wo_pk = w_pk.packed_heads
+    HC = H * head_dim if packed else H * 32
+    if HC % 128 != 0 and not packed:
+        raise RuntimeError("attention: n_head * 32 must be a multiple of 128 (got %d heads)" % H)
+    HT = HC // 32                                  # operand tiles per batch row and 32 tokens
+    per_row = 5 * HT * NT * 1024 * es
+    slab = B2 if budget is None else min(B2, max(2, (budget // per_row) // 2 * 2))
+    q_t = alloc((slab, HT, NT, 1024), dt, dev, zero)
+    k_t = alloc((slab, HT, NT, 1024), dt, dev, zero)
+    v_t = alloc((slab, HT, NT, 1024), dt, dev, zero)
     # Where the update goes back into the tensor the gate is computed from (every attention of the Evoformer block),
     # the gate is not a tensor at all: the output stage computes sigmoid(Wg LN(x) + bg) from the rows of x it reads as
     # residual anyway and multiplies the heads' outputs by it on their way into the output projection
@@ -295,15 +302,15 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     # Shorter rows were not measured and keep the gate tensor.  The choice depends on the row length and the width only, never on the number of
     # batch rows: a subset of the batch rows must give the bits of the full call.
     gate_in_out = (_GATE_IN_OUT_STAGE and drop is None and N >= _GATE_IN_OUT_MIN_N and C in _GATE_IN_OUT_WIDTHS and acc_order
-                   and ln is not None and HC == C and c_out == C and resid is not None and o_map is None
+                   and ln is not None and not packed and HC == C and c_out == C and resid is not None and o_map is None
                    and resid.data_ptr() == x.data_ptr() and a_so % 16 == 0 and a_si % 16 == 0)
     gate = None
     if not gate_in_out:
-        gate = alloc((slab, H, NT, 1024) if acc_order else (slab * N, HC), dt, dev)
+        gate = alloc((slab, HT, NT, 1024) if acc_order else (slab * N, HC), dt, dev)
     o = alloc((slab * N, HC), dt, dev)
-    tpg = HC // 128
+    tpg = (HC + 127) // 128
     qscale = LOG2E / math.sqrt(float(head_dim))
-    tkw = dict(inner=N, s_o=H * NT * 1024, s_h=NT * 1024)
+    tkw = dict(inner=N, s_o=HT * NT * 1024, s_h=NT * 1024, ncols=min(128, HC))
     bias_tile = None
     # rows of a bias buffer the caller leaves to this function (bias_in_launch with bias_t None) end in one unused tile
     # when the projection launch writes them: with 2^n key tiles per row every query-tile row would start in the same
@@ -371,7 +378,7 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
                               w_row_off=t0 * 128, a_off=off)
         _lib.attention_fwd(o, q_t, k_t, v_t, bias_t, kb[b0:b0 + nb], flags[b0:b0 + nb], gate, B2=nb, H=H, Nq=N, Nk=N,
                            gate_tiled=acc_order, bias_padded=bias_padded,
-                           half_k=head_dim <= (16 if acc_order else 8))
+                           D=head_dim if packed else 32, half_k=not packed and head_dim <= (16 if acc_order else 8))
         if gate_in_out:
             # packed rows of w_pk: q, k, v, gate blocks of HC rows each; o holds the slab's rows in logical order
             _lib.gated_out_fused(out.data_ptr() + o_off * es, x.data_ptr() + off * es, ln[0], ln[1],

@@ -563,6 +563,13 @@ class SelfAttention(nn.Module, _PackMixin):
                 # the same without the gate block ([q; k; v; extra]): the projection launch of an attention whose gate
                 # is computed in the output stage finds the extra (pair-bias) rows right behind v
                 w.without_gate = torch.cat([w[:3 * hc], extra], 0).contiguous()
+            if c in (8, 16) and H * c in (64, 128, 256) and dtype == torch.bfloat16:
+                # heads side by side, every block in whole 128-row tiles (see attention)
+                mats = [*self.to_qkv.weight.detach().unflatten(0, (3, H * c)), self.gating_linear.weight]
+                w.packed_heads = (torch.cat([F_.pack_rows([m], dtype, device) for m in mats]
+                                            + ([] if extra_rows is None else [extra])).contiguous(),
+                                  F_.pack_vec([self.gating_bias], dtype, device),
+                                  F_.pack_rows([self.o_linear.weight], dtype, device))
             return (w, F_.pack_vec([_pad_heads(self.gating_bias, H, c, 0)], dtype, device),
                     F_.pack_rows([_pad_heads(self.o_linear.weight, H, c, 1)], dtype, device))
         return self._packed(key, params, build)

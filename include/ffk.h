@@ -283,6 +283,8 @@ int ffk_bgemm_nt(const ffk_bgemm_desc* desc, void* stream);
  *   gate     : multiplicative gate (already sigmoid-ed) or NULL: [B2*Nq, H*32] row-major, or with
  *              FFK_ATT_GATE_TILED in flags [B2][H][ceil(Nq/32)][1024] in FFK_TILE_ACC order
  *   out      : [B2*Nq, H*D] row-major
+ * D = 8 / 16 (bf16): 32 / D heads lie side by side in an operand tile; q_t, k_t (FFK_TILE_ACC order), v_t and a tiled gate are
+ * [B2][H*D/32][ceil(N/32)][1024], head h being channels D * (h % (32/D)) .. of tile h / (32/D); bias_t is per head as above.
  * D = 64 / 128: the head is cut into D / 32 parts of 32 channels; q_t, k_t (FFK_TILE_QK order) and v_t hold one
  * [B2][H][ceil(N/32)][1024] block per part, part-major ([D/32][B2][H][...]: part p = channels 32p .. 32p+31 of
  * every head), q still carries d^-1/2 * log2(e) with d = D; gate must be NULL.

@@ -330,3 +330,26 @@ def test_extra_stack_extreme_shapes(dev, s, r, tail):
             assert np.abs(gz[:nv, :nv] - rz[:nv, :nv]).max() <= 1e-4 * max(1.0, float(np.abs(rz).max()))
         else:
             assert _rel_l2(gz[:nv, :nv], rz[:nv, :nv]) <= 2e-2
+
+
+@pytest.mark.parametrize("c,H,C", [(8, 8, 64), (16, 4, 64), (16, 8, 128)])
+@pytest.mark.parametrize("B2,N", [(1, 32), (3, 160)])
+def test_packed_narrow_heads(dev, c, H, C, B2, N):
+    """Heads of 8 and 16 channels side by side in the operand tiles (bf16), with and without a bias, against the padded fp32 path."""
+    from fastfold_amd.model.fastnn.ops import SelfAttention
+    g = torch.Generator().manual_seed(c * H + N)
+    att = SelfAttention(C, c, H, C).to(dev).eval()
+    with torch.no_grad():
+        for p in att.parameters():
+            p.copy_(torch.randn(p.shape, generator=g) * (p.shape[-1] ** -0.5 if p.dim() > 1 else 1.0))
+        x = torch.randn(1, B2, N, C, generator=g).to(dev)
+        mask = (torch.rand(1, B2, N, generator=g) > 0.2).float().to(dev)
+        mask[..., 0], mask[0, -1] = 1, 0                      # some keys masked; all keys of the last row
+        bias = torch.randn(1, N, N, H, generator=g).to(dev)
+        half = copy.deepcopy(att).bfloat16()
+        for b in (None, (bias, None)):
+            ref = att(x, mask, b)
+            got = half(x.bfloat16(), mask.bfloat16(), None if b is None else (bias.bfloat16(), None))
+            rows = slice(0, max(1, B2 - 1))
+            assert torch.isfinite(got).all()
+            assert float((got.float() - ref)[:, rows].norm() / ref[:, rows].norm()) < 2e-2
