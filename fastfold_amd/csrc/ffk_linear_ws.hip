@@ -39,42 +39,56 @@ template <int K> struct WsGeo {
 
 typedef bf16_t T;
 
-struct WsPlan {
-    int wrow[WS_WAVES][WS_NS];   // first weight row of the slot
-    int tile[WS_WAVES][WS_NS];   // descriptor tile the slot belongs to, -1 = unused
-    int chan[WS_WAVES][WS_NS];   // first output channel (within the tile) of the slot's unit
-    int glu[WS_WAVES][WS_NS];    // 0 plain, 1 value half of a GLU unit (gate half in the next slot), 2 gate half
-    int rg_first[WS_WAVES], rg_step[WS_WAVES];   // row groups of a slab this wave works on
-    int row_perm;                // 1: rows of a group are read through tau (launch has channel-major tiles)
-    int mask_tile;               // first tile with a row mask (all masked tiles share its mask), -1 = none
-    int max_slots;               // largest number of slots any wave holds
-    int resid_a2;                // 1: every residual is the second operand itself (same rows): taken from its LDS slab
-    int bias_tile;               // index of a trailing FFK_TILE_BIAS tile (<= 4 heads, K = 128), -1 = none: it takes no
-                                 // weight slot - its few dot products per row are 16 x 16 x 32 MFMAs on the slab in LDS
-};
-
-struct WsArgs {
-    ffk_linear_desc d;
-    WsPlan plan;
-};
-
-// What the epilogue of one slot needs, copied out of the tile descriptor once per kernel so that it
-// lives in scalar registers (reading descriptor fields inside the loops costs a scalar load plus a
-// full wait each time).  Channel offsets of the slot's unit are folded into the pointers.
+// A weight slot: 32 rows of the weights and everything its epilogue needs, laid out by the host so that a wave reads it in
+// one piece (a chain of scalar loads - plan, tile, pointers - cost a launch 0.8 us per link before the first row was requested).
+// Channel offsets of the slot's unit are folded into the pointers.
 struct WsSlot {
     T* out;
     const T* resid;
     const T* gate;
+    const T* bias;           // of the slot's 32 rows, or nullptr
     int8_t* xtail;           // tail bytes of resid / out as an extended residual stream, or nullptr
     long s_o, s_i, s_d, gate_ld;
     unsigned inner;
     unsigned gate_rows;      // 0, or the period of the gate's row index
     int ncols_left;          // valid channels from the unit's first channel on
-    int kind, act;
+    int wrow;                // first weight row of the slot, -1 = unused
     float scale;
-    bool masked;
-    bool has_bias;
+    signed char kind, act;
+    signed char glu;         // 0 plain, 1 value half of a GLU unit (gate half in the next slot), 2 gate half
+    bool masked, has_bias, by_rows;
+    bool tau;                // weight rows through ws_tau
+    bool sig;                // bias pre-multiplied for ws_sigmoid_pre
 };
+
+struct WsArgs {
+    const T* a;
+    const T* w;
+    const T* a2;
+    const void* ln_gamma;
+    const void* ln_beta;
+    int a_so, a_si, a_cs, a2_so, a2_si;
+    int M, n_tiles, a_inner, a2_inner;
+    float ln_eps;
+    // the waves form `groups` groups holding the same slots; the waves of a group take every rg_step-th row group of a slab
+    int groups, rg_step;
+    int row_perm;                // 1: rows of a group are read through tau (launch has channel-major tiles)
+    int max_slots;               // largest number of slots any wave holds
+    int resid_a2;                // 1: every residual is the second operand itself (same rows): taken from its LDS slab
+    // row mask of the launch (all masked tiles share it), or nullptr
+    const T* rowmask;
+    int m_so, m_si;
+    unsigned m_inner;
+    // trailing FFK_TILE_BIAS tile (<= 4 heads, K = 128), pb_heads = 0: none.  It takes no weight slot - its few dot products per row
+    // are 16 x 16 x 32 MFMAs on the slab in LDS
+    int pb_heads, pb_wrow;
+    unsigned pb_inner;
+    T* pb_out;
+    int pb_so, pb_sh;
+    float pb_scale;
+    WsSlot slot[WS_WAVES][WS_NS];    // [group][slot]
+};
+static_assert(sizeof(WsArgs) <= 4096, "kernel arguments");
 
 // sigmoid(acc + b) with the bias table entry pre-multiplied:  bs = -log2(e) * b
 __device__ __forceinline__ float ws_sigmoid_pre(float acc, float bs) {
@@ -178,7 +192,7 @@ __device__ __forceinline__ void ws_store_rows_compact(const WsSlot& t, const f32
         if (t.gate || t.resid) {
             // every load first (clamped, unconditional), then combine and store
             u32x4 gv[2], rv[2];
-            const T* gate = t.gate ? t.gate + (long)(t.gate_rows ? mc % t.gate_rows : mc) * t.gate_ld + cl : nullptr;
+            const T* gate = t.gate ? t.gate + (long)(int)(t.gate_rows ? mc % t.gate_rows : mc) * t.gate_ld + cl : nullptr;
             const T* resid = t.resid ? t.resid + off : nullptr;
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
@@ -359,7 +373,7 @@ __device__ __forceinline__ void ws_store_rows(const WsSlot& t, const f32x16& acc
         if (t.gate || t.resid) {
             // every load first (clamped, unconditional), then combine and store
             u32x4 gv[2], rv[2];
-            const T* gate = t.gate ? t.gate + (long)(t.gate_rows ? mc % t.gate_rows : mc) * t.gate_ld + cl : nullptr;
+            const T* gate = t.gate ? t.gate + (long)(int)(t.gate_rows ? mc % t.gate_rows : mc) * t.gate_ld + cl : nullptr;
             const T* resid = t.resid ? t.resid + off : nullptr;
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
@@ -574,7 +588,7 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
     constexpr bool LEAN = NS == 2 && WS_K <= 128 && !DUAL;   // straight-line epilogues where the registers allow them
     constexpr bool POS = NS == 2 && !XT;                   // variants that take FFK_ACT_GATE_POS (the others have no register for it)
     constexpr int AFC = WS_K == 128 ? 8 : 4;               // A fragments held at a time (register budget)
-    const ffk_linear_desc& d = args.d;
+    const WsArgs& d = args;
     extern __shared__ __align__(16) unsigned char smem[];
     unsigned char* s_a = smem;                                                 // [2][WS_BM][WS_AP]
     float* s_mask = reinterpret_cast<float*>(smem + 2 * WS_BM * WS_AP);        // [2][WS_BM]
@@ -592,49 +606,18 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
     const int M = d.M;
-    const T* A = (const T*)d.a;
-    const T* W = (const T*)d.w;
+    const T* A = d.a;
+    const T* W = d.w;
 
     // ---- this wave's weight slots, resident in registers ----
-    int s_tile[NS], s_chan[NS], s_glu[NS], s_wrow[NS];
     WsSlot sp[NS];
-    bool by_rows[NS];
-    int s_wl[NS];
     bf16x8 wf[NS][WS_KS];
+    const int grp = wave & (args.groups - 1);            // groups: a power of two
+    const int rg_first = wave / args.groups, rg_step = args.rg_step;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        s_tile[s] = args.plan.tile[wave][s];
-        s_chan[s] = args.plan.chan[wave][s];
-        s_glu[s] = args.plan.glu[wave][s];
-        s_wrow[s] = s_tile[s] >= 0 ? args.plan.wrow[wave][s] : 0;
-        // [row][channel] tiles take their weight rows through tau (16 consecutive channels per lane)
-        const ffk_tile& ts = d.tiles[s_tile[s] >= 0 ? s_tile[s] : 0];
-        const int wl = ts.kind == FFK_TILE_STRIDED && ts.s_d == 1 ? ws_tau(l32) : l32;
-        {
-            const long coff = (long)(s_chan[s] >> 5) * ts.s_h;
-            sp[s].out = (T*)ts.out + coff;
-            sp[s].resid = ts.resid ? (const T*)ts.resid + coff : nullptr;
-            sp[s].gate = ts.gate ? (const T*)ts.gate + s_chan[s] : nullptr;
-            sp[s].xtail = XT && ts.xtail ? (int8_t*)ts.xtail + coff : nullptr;
-            sp[s].s_o = ts.s_o;
-            sp[s].s_i = ts.s_i;
-            sp[s].s_d = ts.s_d;
-            sp[s].gate_ld = ts.gate_ld;
-            sp[s].gate_rows = (unsigned)ts.gate_rows;
-            sp[s].inner = (unsigned)ts.inner;
-            sp[s].ncols_left = ts.ncols - s_chan[s];
-            sp[s].kind = ts.kind;
-            sp[s].act = ts.act;
-            sp[s].scale = ts.scale;
-            sp[s].masked = ts.rowmask != nullptr;
-            sp[s].has_bias = ts.bias != nullptr;
-            by_rows[s] = ws_by_rows(ts);
-        }
-        s_wl[s] = wl;
-    }
-    const int rg_first = args.plan.rg_first[wave], rg_step = args.plan.rg_step[wave];
+    for (int s = 0; s < NS; ++s) sp[s] = args.slot[grp][s];
     // launches with channel-major tiles read the rows of a group through tau (16 consecutive rows per lane)
-    const int n32 = args.plan.row_perm ? ws_tau(l32) : l32;
+    const int n32 = args.row_perm ? ws_tau(l32) : l32;
 
     // ---- slab streaming: thread -> (row tid / LPR + RPP * i, 8 channels starting at 8 * (tid % LPR)) ----
     const int c8 = tid % LPR, r0 = tid / LPR;
@@ -643,10 +626,9 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
     const bool folded = DUAL;
     const bool ln = d.ln_gamma != nullptr && !folded;
     // row mask of the launch (all masked tiles share it): fetched with the slab, kept in LDS as fp32
-    const int mt = args.plan.mask_tile;
-    const T* rm = mt >= 0 ? (const T*)d.tiles[mt].rowmask : nullptr;
-    const unsigned m_inner = mt >= 0 ? (unsigned)d.tiles[mt].inner : 1u;
-    const long m_so = mt >= 0 ? d.tiles[mt].m_so : 0, m_si = mt >= 0 ? d.tiles[mt].m_si : 0;
+    const T* rm = args.rowmask;
+    const unsigned m_inner = args.m_inner;
+    const int m_so = args.m_so, m_si = args.m_si;
     // plain row-major operands (inner >= M) need no division per fetched vector
     const bool a_flat = d.a_inner >= M, a2_flat = DUAL && d.a2_inner >= M, m_flat = m_inner >= (unsigned)M;
     Vec16<T> pre[4];
@@ -670,7 +652,7 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
                 long m = (long)slab * WS_BM + i * 32 + (tid >> 4);
                 m = m < M ? m : M - 1;
                 const unsigned hi = a2_flat ? 0u : (unsigned)m / (unsigned)d.a2_inner, lo = (unsigned)m - hi * (unsigned)d.a2_inner;
-                const T* gp = (const T*)d.a2 + (long)hi * d.a2_so + (long)lo * d.a2_si + a2_col * 8;
+                const T* gp = d.a2 + (long)hi * d.a2_so + (long)lo * d.a2_si + a2_col * 8;
                 const unsigned dst = lds_a2 + tobuf * (WS_BM * 256) + (i * WS_THREADS + wave * 64) * 16;
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
@@ -787,7 +769,7 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
 
     const int nslabs = (M + WS_BM - 1) / WS_BM;
     int slab = blockIdx.x;                               // grid <= nslabs
-    const int pb_tile = PB ? args.plan.bias_tile : -1;
+    const int pb_heads = PB ? args.pb_heads : 0;
     fetch(slab, 0);                                      // the first slab travels while the weights are fetched
     // ---- weights: every wave reads the 32 rows of its slots as whole lines (a lane's fragments are 16-byte pieces
     // 32 bytes apart in one row, 32 rows per request: fetched that way every request touches 32 lines and uses a
@@ -810,35 +792,22 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
             for (int pc = 0; pc < NP; ++pc)
 #pragma unroll
                 for (int i = 0; i < NI; ++i)
-                    wf[sl][pc * NI + i] = MM::ld(W + (long)(s_wrow[sl] + i * (64 / LR) + lrow) * WS_K + pc * PW + lcol * 8);
+                    wf[sl][pc * NI + i] = MM::ld(W + (long)((sp[sl].wrow >= 0 ? sp[sl].wrow : 0) + i * (64 / LR) + lrow) * WS_K + pc * PW + lcol * 8);
         // tables the epilogues and the commits read from LDS (no global loads there); the barrier in front of the first
-        // commit publishes them
-        for (int i = tid; i < d.n_tiles * 128; i += WS_THREADS) {
-            const ffk_tile& tb = d.tiles[i >> 7];
-            const T* bp = (const T*)tb.bias;
-            // gate halves of a GLU unit ([p 32 | g 32 | p 32 | g 32]) and sigmoid tiles: pre-multiplied for ws_sigmoid_pre
-            const bool sig = tb.glu ? ((i >> 5) & 1) != 0 : tb.act == FFK_ACT_SIGMOID;
-            const float b = bp ? (float)bp[i & 127] : 0.0f;
-            s_bias[i] = sig ? -1.4426950408889634f * b : b;
+        // commit publishes them.  All are requested together with the weights and stored when these have arrived.
+        float tb[NS], tc[2];
+        T tg[2] = {(T)0.0f, (T)0.0f}, tw = (T)0.0f;
+#pragma unroll
+        for (int sl = 0; sl < NS; ++sl) tb[sl] = sp[sl].wrow >= 0 && sp[sl].bias ? (float)sp[sl].bias[l32] : 0.0f;
+        if (ln && tid < WS_K) {
+            tg[0] = ((const T*)d.ln_gamma)[tid];
+            tg[1] = ((const T*)d.ln_beta)[tid];
         }
-
-        {
-            if (folded) {
-                for (int i = tid; i < d.n_tiles * 128; i += WS_THREADS) s_c1[i] = ((const float*)d.ln_gamma)[i];
-            }
-            if (ln && !CM && tid < WS_K) {
-                s_ln1[tid] = ((const T*)d.ln_gamma)[tid];
-                s_ln1[WS_K + tid] = ((const T*)d.ln_beta)[tid];
-            }
-            if (ln && CM && tid < WS_K) {
-                s_cmln[tid] = (float)((const T*)d.ln_gamma)[tid];
-                s_cmln[WS_K + tid] = (float)((const T*)d.ln_beta)[tid];
-            }
-        }
-        if (PB && pb_tile >= 0) {
-            const int heads = d.tiles[pb_tile].ncols;
-            for (int i = tid; i < 4 * WS_K; i += WS_THREADS)
-                s_wb[i] = (i / WS_K) < heads ? W[(long)(pb_tile * 128 + i / WS_K) * WS_K + (i % WS_K)] : (T)0.0f;
+        if (PB && pb_heads && tid < pb_heads * WS_K) tw = W[(long)args.pb_wrow * WS_K + tid];     // 4 * WS_K == WS_THREADS
+        if (folded) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                tc[i] = tid + i * WS_THREADS < d.n_tiles * 128 ? ((const float*)d.ln_gamma)[tid + i * WS_THREADS] : 0.0f;
         }
 #pragma unroll
         for (int sl = 0; sl < NS; ++sl)
@@ -849,11 +818,32 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
                     const int row = i * (64 / LR) + lrow;
                     *reinterpret_cast<bf16x8*>(stage + row * (PW * 2) + ((lcol ^ (row & (LR - 1))) * 16)) = wf[sl][pc * NI + i];
                 }
+                // [row][channel] tiles take their weight rows through tau (16 consecutive channels per lane)
+                const int wl = sp[sl].tau ? ws_tau(l32) : l32;
 #pragma unroll
                 for (int k = 0; k < NI; ++k)
                     wf[sl][pc * NI + k] = *reinterpret_cast<const bf16x8*>(
-                        stage + s_wl[sl] * (PW * 2) + (((2 * k + half) ^ (s_wl[sl] & (LR - 1))) * 16));
+                        stage + wl * (PW * 2) + (((2 * k + half) ^ (wl & (LR - 1))) * 16));
             }
+#pragma unroll
+        for (int sl = 0; sl < NS; ++sl)                   // (waves of a group write the same values)
+            if (half == 0 && sp[sl].wrow >= 0) s_bias[sp[sl].wrow + l32] = sp[sl].sig ? -1.4426950408889634f * tb[sl] : tb[sl];
+        if (ln && tid < WS_K) {
+            if (CM) {
+                s_cmln[tid] = (float)tg[0];
+                s_cmln[WS_K + tid] = (float)tg[1];
+            } else {
+                s_ln1[tid] = tg[0];
+                s_ln1[WS_K + tid] = tg[1];
+            }
+        }
+        if (PB && pb_heads && tid < 4 * WS_K) s_wb[tid] = tw;
+        if (folded) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                if (tid + i * WS_THREADS < FFK_MAX_TILES * 128) s_c1[tid + i * WS_THREADS] = tc[i];
+            for (int i = tid + 2 * WS_THREADS; i < d.n_tiles * 128; i += WS_THREADS) s_c1[i] = ((const float*)d.ln_gamma)[i];
+        }
     }
     lds_barrier();                                       // every wave is done with the staging area
     commit(0);
@@ -863,13 +853,12 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
         const bool more = slab + (int)gridDim.x < nslabs;
         if (more) fetch(slab + (int)gridDim.x, buf ^ 1);  // in flight during the products below
         const unsigned char* sa = s_a + buf * (WS_BM * WS_AP);
-        if (PB && pb_tile >= 0) {
+        if (PB && pb_heads) {
             // pair bias of this slab on the matrix pipe: wave w takes the rows 16 w .. 16 w + 15 as the N operand of
             // four 16 x 16 x 32 products against the (at most four) head weight rows, zero rows up to 16 (M operand).
             // The rows are the operand as the other products see it (normalised, rounded to bf16), so the value
             // equals a further output column group of four channels.  Result layout: lane = row, register v = head
             // (4 * (lane / 16) + v: only the first sixteen lanes hold real heads).
-            const ffk_tile& tb = d.tiles[pb_tile];
             const int r16 = lane & 15, kq = lane >> 4;
             const unsigned char* xr = sa + (wave * 16 + r16) * WS_AP + kq * 16;
             const T* wr = s_wb + (r16 & 3) * WS_K + kq * 8;
@@ -886,11 +875,11 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
             }
             const long pm = (long)slab * WS_BM + wave * 16 + r16;
             if (kq == 0 && pm < M) {
-                const unsigned hi = (unsigned)pm / (unsigned)tb.inner, lo = (unsigned)pm - hi * (unsigned)tb.inner;
-                T* po = (T*)tb.out + (long)(hi >> 5) * tb.s_o + (long)(lo >> 5) * 1024 + qk_tile_off((int)(lo & 31), (int)(hi & 31));
+                const unsigned hi = (unsigned)pm / args.pb_inner, lo = (unsigned)pm - hi * args.pb_inner;
+                T* po = args.pb_out + (long)(int)(hi >> 5) * args.pb_so + (long)(lo >> 5) * 1024 + qk_tile_off((int)(lo & 31), (int)(hi & 31));
 #pragma unroll
                 for (int hd = 0; hd < 4; ++hd)
-                    if (hd < tb.ncols) po[(long)hd * tb.s_h] = (T)(pacc[hd] * tb.scale);
+                    if (hd < pb_heads) po[(long)hd * args.pb_sh] = (T)(pacc[hd] * args.pb_scale);
             }
         }
         for (int rg = rg_first; rg < WS_RG; rg += rg_step) {
@@ -906,18 +895,18 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
             const float* smk = s_mask + buf * WS_BM + rg * 32;
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
-                if (s_tile[s] < 0 || s_glu[s] == 2) continue;
+                if (sp[s].wrow < 0 || sp[s].glu == 2) continue;
                 const WsSlot& t = sp[s];
-                const bool glu = s_glu[s] == 1;
+                const bool glu = sp[s].glu == 1;
                 const int sg = s + 1 < NS ? s + 1 : s;             // gate slot of a GLU unit (constant after unrolling)
-                const float* sb = s_bias + s_wrow[s];
+                const float* sb = s_bias + sp[s].wrow;
                 // The A fragments are re-read from LDS for every slot: keeping them across the epilogue of
                 // the previous slot costs 32 registers, and a single spilled register puts a scratch
                 // reload with a full vector-memory wait into every epilogue.
                 int reread = 0;
                 asm volatile("" : "+v"(reread));                   // opaque zero: keeps the compiler from reusing the loads
                 if constexpr (LEAN) {
-                    const bool rows = by_rows[s];
+                    const bool rows = sp[s].by_rows;
                     // One straight-line body per (store order, GLU or not): the gate accumulator only exists
                     // where it is used, and no accumulator has to be copied or cleared where paths would join.
                     auto slot_body = [&](auto rows_tag, auto glu_tag) {
@@ -995,7 +984,7 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
 #pragma unroll
                     for (int v = 0; v < 16; ++v) acc[v] = accg[v] = 0.0f;
                     float st1 = 0.0f, st2 = 0.0f, su1 = 0.0f, su2 = 0.0f;   // row statistics of the two operands (DUAL)
-                    const bool rows = by_rows[s];
+                    const bool rows = sp[s].by_rows;
                     if (DUAL && ALLOW_GLU && glu) {
                         // gate half: fragments of the second operand's row (row % 16 == l32 % 16 picks the swizzle)
                         const unsigned a2row = (unsigned)(buf * (WS_BM * 256) + (rg * 32 + n32) * 256 + ((half ^ (n32 & 15)) << 4));
@@ -1078,11 +1067,11 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
                             const float rstd_g = -1.4426950408889634f * rsqrtf(fmaxf(su2 * (1.0f / WS_K) - mean_g * mean_g, 0.0f) + d.ln_eps);
                             const unsigned char* a2r = nullptr;
                             int a2v = 0;
-                            if (args.plan.resid_a2 && t.resid) {
+                            if (args.resid_a2 && t.resid) {
                                 a2r = s_a2 + buf * (WS_BM * 256) + (rg * 32 + n32) * 256;
-                                a2v = (int)(t.resid - (const T*)d.a2) / 8 + 2 * half;
+                                a2v = (int)(t.resid - d.a2) / 8 + 2 * half;
                             }
-                            ws_store_rows_folded<XT>(t, acc, accg, sb, s_c1 + s_wrow[s], rstd, -rstd * mean, rstd_g, -rstd_g * mean_g,
+                            ws_store_rows_folded<XT>(t, acc, accg, sb, s_c1 + sp[s].wrow, rstd, -rstd * mean, rstd_g, -rstd_g * mean_g,
                                                  valid, c_hi, c_lo, half, a2r, a2v, n32 & 15);
                         } else if (ALLOW_GLU && glu) ws_store_rows_compact<true, XT, POS>(t, acc, accg, sb, valid, mc, c_hi, c_lo, rmask, half);
                         else ws_store_rows_compact<false, XT, POS>(t, acc, accg, sb, valid, mc, c_hi, c_lo, rmask, half);
@@ -1125,11 +1114,11 @@ bool ws_tile_ok(const ffk_linear_desc& d, const ffk_tile& t) {
 // Distributes the 32-row weight units over the waves.  The waves form G = 8 / R groups; the R waves
 // of a group hold the same units and take every R-th row group of a slab (R as large as the units
 // allow, so that few units still use all eight waves).  Returns false if the units do not fit.
-bool ws_make_plan(const ffk_linear_desc& d, WsPlan& p, int rg_per_slab, int max_ns) {
+bool ws_make_plan(const ffk_linear_desc& d, int n_tiles, WsArgs& p, int rg_per_slab, int max_ns) {
     struct Unit { int tile, chan, wrow, slots; };
     Unit units[FFK_MAX_TILES * 4];
     int nu = 0;
-    for (int i = 0; i < d.n_tiles; ++i) {
+    for (int i = 0; i < n_tiles; ++i) {
         const ffk_tile& t = d.tiles[i];
         const int n = (t.ncols + 31) / 32;
         for (int u = 0; u < n; ++u) {
@@ -1173,29 +1162,42 @@ bool ws_make_plan(const ffk_linear_desc& d, WsPlan& p, int rg_per_slab, int max_
         for (int sl = 0; sl < WS_NS; ++sl) n += assign[g][sl] != -1;
         p.max_slots = n > p.max_slots ? n : p.max_slots;
     }
-    for (int w = 0; w < WS_WAVES; ++w) {
-        const int g = w % G;
-        p.rg_first[w] = w / G;
-        p.rg_step[w] = R;
-        for (int s = 0; s < WS_NS; ++s) {
-            const int a = assign[g][s];
-            if (a == -1) {
-                p.tile[w][s] = -1;
-                p.wrow[w][s] = p.chan[w][s] = p.glu[w][s] = 0;
-            } else if (a >= 0) {
-                p.tile[w][s] = units[a].tile;
-                p.wrow[w][s] = units[a].wrow;
-                p.chan[w][s] = units[a].chan;
-                p.glu[w][s] = units[a].slots == 2 ? 1 : 0;
-            } else {
-                const Unit& u = units[-2 - a];
-                p.tile[w][s] = u.tile;
-                p.wrow[w][s] = u.wrow + 32;
-                p.chan[w][s] = u.chan;
-                p.glu[w][s] = 2;
-            }
+    p.groups = G;
+    p.rg_step = R;
+    for (int g = 0; g < G; ++g)
+        for (int sl = 0; sl < WS_NS; ++sl) {
+            WsSlot& q = p.slot[g][sl];
+            q = WsSlot{};
+            q.wrow = -1;
+            const int a = assign[g][sl];
+            if (a == -1) continue;
+            const Unit& u = units[a >= 0 ? a : -2 - a];
+            const ffk_tile& t = d.tiles[u.tile];
+            const long coff = (long)(u.chan >> 5) * t.s_h;
+            q.wrow = u.wrow + (a >= 0 ? 0 : 32);
+            q.glu = (signed char)(a < 0 ? 2 : u.slots == 2 ? 1 : 0);
+            q.out = (T*)t.out + coff;
+            q.resid = t.resid ? (const T*)t.resid + coff : nullptr;
+            q.gate = t.gate ? (const T*)t.gate + u.chan : nullptr;
+            q.bias = t.bias ? (const T*)t.bias + (q.wrow & 127) : nullptr;
+            q.xtail = t.xtail ? (int8_t*)t.xtail + coff : nullptr;
+            q.s_o = (int)t.s_o;
+            q.s_i = (int)t.s_i;
+            q.s_d = (int)t.s_d;
+            q.gate_ld = (int)t.gate_ld;
+            q.inner = (unsigned)t.inner;
+            q.gate_rows = (unsigned)t.gate_rows;
+            q.ncols_left = t.ncols - u.chan;
+            q.scale = t.scale;
+            q.kind = (signed char)t.kind;
+            q.act = (signed char)t.act;
+            q.masked = t.rowmask != nullptr;
+            q.has_bias = t.bias != nullptr;
+            q.by_rows = ws_by_rows(t);
+            q.tau = t.kind == FFK_TILE_STRIDED && t.s_d == 1;
+            // gate halves of a GLU unit and sigmoid tiles
+            q.sig = t.glu ? q.glu == 2 : t.act == FFK_ACT_SIGMOID;
         }
-    }
     return true;
 }
 
@@ -1211,7 +1213,7 @@ int ws_launch(const WsArgs& args, hipStream_t st) {
         const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)linear_ws_kernel<NS, K, CM, DUAL, XT>, smem, "ffk_fused_linear");
         if (rc_lds != FFK_OK) return rc_lds;
     }
-    const int nslabs = ffk_cdiv(args.d.M, WS_BM);
+    const int nslabs = ffk_cdiv(args.M, WS_BM);
     const int grid = nslabs < WS_MAX_GRID ? nslabs : WS_MAX_GRID;
     linear_ws_kernel<NS, K, CM, DUAL, XT><<<grid, WS_THREADS, smem, st>>>(args);
     return ffk_check_launch("ffk_fused_linear");
@@ -1228,6 +1230,12 @@ int ffk_linear_ws_try(const ffk_linear_desc* d, hipStream_t st, int* status) {
     if (d->a2 && d->K != 128) return 0;                          // the second operand is built for K = 128
     const bool k256 = d->K == 256;
     if (d->variant == FFK_LINEAR_STAGED) return 0;
+    auto i32 = [](int64_t v) { return v >= -0x7fffffffL && v <= 0x7fffffffL; };      // the kernel's strides have 32 bits
+    if (!i32(d->a_so) || !i32(d->a_si) || !i32(d->a_cs) || !i32(d->a2_so) || !i32(d->a2_si)) return 0;
+    for (int i = 0; i < d->n_tiles; ++i) {
+        const ffk_tile& t = d->tiles[i];
+        if (!i32(t.s_o) || !i32(t.s_i) || !i32(t.s_d) || !i32(t.s_h) || !i32(t.gate_ld) || !i32(t.m_so) || !i32(t.m_si)) return 0;
+    }
     bool chan_major = false, v_tiles = false, tails = false;
     int mask_tile = -1;
     // a trailing pair-bias tile (score-operand tiles of <= 4 heads) rides on the launch without a weight slot; it may be
@@ -1261,28 +1269,56 @@ int ffk_linear_ws_try(const ffk_linear_desc* d, hipStream_t st, int* status) {
     if (chan_major && v_tiles) return 0;          // they need different row orders within a group
     WsArgs args;
     const bool k64 = d->K == 64;
-    {
-        ffk_linear_desc slots = *d;                   // the plan covers the tiles that take weight slots
-        slots.n_tiles = n_slot_tiles;
-        if (!ws_make_plan(slots, args.plan, k256 ? WsGeo<256>::RG : (k64 ? WsGeo<64>::RG : WsGeo<128>::RG),
-                          k256 ? 2 : (k64 ? 4 : 3)))
-            return 0;
-    }
+    if (!ws_make_plan(*d, n_slot_tiles, args, k256 ? WsGeo<256>::RG : (k64 ? WsGeo<64>::RG : WsGeo<128>::RG), k256 ? 2 : (k64 ? 4 : 3)))
+        return 0;
     if (bias_tile >= 0 && (tails || chan_major)) return 0;   // built into the plain K = 128 variants only
     for (int i = 0; i < n_slot_tiles; ++i)
-        if (d->tiles[i].act == FFK_ACT_GATE_POS && (tails || args.plan.max_slots > 2)) return 0;
+        if (d->tiles[i].act == FFK_ACT_GATE_POS && (tails || args.max_slots > 2)) return 0;
     if (k256) {
         for (int i = 0; i < d->n_tiles; ++i)
             if (d->tiles[i].glu) return 0;                   // GLU units are only built for K = 128
     }
-    args.plan.row_perm = chan_major ? 1 : 0;
-    args.plan.mask_tile = mask_tile;
-    args.plan.resid_a2 = 0;
-    args.plan.bias_tile = bias_tile;
-    args.d = *d;
+    args.a = (const T*)d->a;
+    args.w = (const T*)d->w;
+    args.a2 = (const T*)d->a2;
+    args.ln_gamma = d->ln_gamma;
+    args.ln_beta = d->ln_beta;
+    args.a_so = (int)d->a_so;
+    args.a_si = (int)d->a_si;
+    args.a_cs = (int)d->a_cs;
+    args.a2_so = (int)d->a2_so;
+    args.a2_si = (int)d->a2_si;
+    args.M = d->M;
+    args.n_tiles = d->n_tiles;
+    args.a_inner = d->a_inner;
+    args.a2_inner = d->a2_inner;
+    args.ln_eps = d->ln_eps;
+    args.row_perm = chan_major ? 1 : 0;
+    args.resid_a2 = 0;
+    args.rowmask = nullptr;
+    args.m_so = args.m_si = 0;
+    args.m_inner = 1;
+    if (mask_tile >= 0) {
+        const ffk_tile& t = d->tiles[mask_tile];
+        args.rowmask = (const T*)t.rowmask;
+        args.m_so = (int)t.m_so;
+        args.m_si = (int)t.m_si;
+        args.m_inner = (unsigned)t.inner;
+    }
+    args.pb_heads = 0;
+    if (bias_tile >= 0) {
+        const ffk_tile& t = d->tiles[bias_tile];
+        args.pb_heads = t.ncols;
+        args.pb_wrow = bias_tile * 128;
+        args.pb_inner = (unsigned)t.inner;
+        args.pb_out = (T*)t.out;
+        args.pb_so = (int)t.s_o;
+        args.pb_sh = (int)t.s_h;
+        args.pb_scale = t.scale;
+    }
     if (d->a2) {
         // second operand: every unit must be a GLU unit stored [row][channel], first operand channel-major
-        if (!d->a_chanmajor || args.plan.max_slots > 2 || mask_tile >= 0 || d->a2_si % 8 || d->a2_so % 8) return 0;
+        if (!d->a_chanmajor || args.max_slots > 2 || mask_tile >= 0 || d->a2_si % 8 || d->a2_so % 8) return 0;
         bool resid_a2 = true;
         for (int i = 0; i < d->n_tiles; ++i) {
             const ffk_tile& t = d->tiles[i];
@@ -1295,21 +1331,21 @@ int ffk_linear_ws_try(const ffk_linear_desc* d, hipStream_t st, int* status) {
                 t.inner != d->a2_inner || t.s_h != 32 || t.s_d != 1)
                 resid_a2 = false;
         }
-        args.plan.resid_a2 = resid_a2 ? 1 : 0;
+        args.resid_a2 = resid_a2 ? 1 : 0;
         *status = tails ? ws_launch<2, 128, true, true, true>(args, st) : ws_launch<2, 128, true, true>(args, st);
     } else if (tails) {
         // residual tails: built for the output projections of the attentions (one plain tile group, two slots)
-        if (d->a_chanmajor || args.plan.max_slots > 2 || k64) return 0;
+        if (d->a_chanmajor || args.max_slots > 2 || k64) return 0;
         *status = k256 ? ws_launch<2, 256, false, false, true>(args, st) : ws_launch<2, 128, false, false, true>(args, st);
     } else if (d->a_chanmajor) {
-        if (args.plan.max_slots > 2 || mask_tile >= 0) return 0;
+        if (args.max_slots > 2 || mask_tile >= 0) return 0;
         *status = k64 ? ws_launch<2, 64, true>(args, st) : ws_launch<2, 128, true>(args, st);
     } else if (k256) {
         *status = ws_launch<2, 256, false>(args, st);
     } else if (k64) {
-        *status = args.plan.max_slots <= 2 ? ws_launch<2, 64, false>(args, st) : ws_launch<4, 64, false>(args, st);
+        *status = args.max_slots <= 2 ? ws_launch<2, 64, false>(args, st) : ws_launch<4, 64, false>(args, st);
     } else {
-        *status = args.plan.max_slots <= 2 ? ws_launch<2, 128, false>(args, st) : ws_launch<3, 128, false>(args, st);
+        *status = args.max_slots <= 2 ? ws_launch<2, 128, false>(args, st) : ws_launch<3, 128, false>(args, st);
     }
     return 1;
 }
