@@ -135,6 +135,7 @@ def call(name: str, *args):
 FFK_TILE_STRIDED, FFK_TILE_QK, FFK_TILE_V, FFK_TILE_BIAS, FFK_TILE_ACC = 0, 1, 2, 3, 4
 FFK_ACT_NONE, FFK_ACT_RELU, FFK_ACT_SIGMOID = 0, 1, 2
 FFK_MAX_TILES = 10
+WS_TILES = 8               # 128-column tiles the weights-stationary projection kernels take in one launch (two groups of 16 units)
 LOG2E = 1.4426950408889634
 
 

@@ -57,6 +57,7 @@ struct WsSlot {
     signed char kind, act;
     signed char glu;         // 0 plain, 1 value half of a GLU unit (gate half in the next slot), 2 gate half
     bool masked, has_bias, by_rows;
+    signed char rg_first, rg_mask;   // row groups of a slab this wave takes for the slot: those with rg & rg_mask == rg_first
     bool tau;                // weight rows through ws_tau
     bool sig;                // bias pre-multiplied for ws_sigmoid_pre
 };
@@ -70,8 +71,7 @@ struct WsArgs {
     int a_so, a_si, a_cs, a2_so, a2_si;
     int M, n_tiles, a_inner, a2_inner;
     float ln_eps;
-    // the waves form `groups` groups holding the same slots; the waves of a group take every rg_step-th row group of a slab
-    int groups, rg_step;
+    int col_groups;              // sets of workgroups (blockIdx.y), each with slots of its own over all rows
     int row_perm;                // 1: rows of a group are read through tau (launch has channel-major tiles)
     int max_slots;               // largest number of slots any wave holds
     int resid_a2;                // 1: every residual is the second operand itself (same rows): taken from its LDS slab
@@ -86,7 +86,7 @@ struct WsArgs {
     T* pb_out;
     int pb_so, pb_sh;
     float pb_scale;
-    WsSlot slot[WS_WAVES][WS_NS];    // [group][slot]
+    WsSlot slot[WS_WAVES * WS_NS];   // [column group][wave][slot]
 };
 static_assert(sizeof(WsArgs) <= 4096, "kernel arguments");
 
@@ -612,10 +612,8 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
     // ---- this wave's weight slots, resident in registers ----
     WsSlot sp[NS];
     bf16x8 wf[NS][WS_KS];
-    const int grp = wave & (args.groups - 1);            // groups: a power of two
-    const int rg_first = wave / args.groups, rg_step = args.rg_step;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) sp[s] = args.slot[grp][s];
+    for (int s = 0; s < NS; ++s) sp[s] = args.slot[((int)blockIdx.y * WS_WAVES + wave) * NS + s];
     // launches with channel-major tiles read the rows of a group through tau (16 consecutive rows per lane)
     const int n32 = args.row_perm ? ws_tau(l32) : l32;
 
@@ -853,7 +851,7 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
         const bool more = slab + (int)gridDim.x < nslabs;
         if (more) fetch(slab + (int)gridDim.x, buf ^ 1);  // in flight during the products below
         const unsigned char* sa = s_a + buf * (WS_BM * WS_AP);
-        if (PB && pb_heads) {
+        if (PB && pb_heads && blockIdx.y == 0) {
             // pair bias of this slab on the matrix pipe: wave w takes the rows 16 w .. 16 w + 15 as the N operand of
             // four 16 x 16 x 32 products against the (at most four) head weight rows, zero rows up to 16 (M operand).
             // The rows are the operand as the other products see it (normalised, rounded to bf16), so the value
@@ -882,7 +880,9 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
                     if (hd < pb_heads) po[(long)hd * args.pb_sh] = (T)(pacc[hd] * args.pb_scale);
             }
         }
-        for (int rg = rg_first; rg < WS_RG; rg += rg_step) {
+        int rg_by = 1;
+        asm volatile("" : "+s"(rg_by));                    // opaque: a known trip count makes the compiler keep addresses it spills for
+        for (int rg = 0; rg < WS_RG; rg += rg_by) {
             const long m0g = (long)slab * WS_BM + rg * 32;
             if (m0g >= M) break;
             const unsigned char* ap = sa + (rg * 32 + n32) * WS_AP + half * 16;
@@ -895,7 +895,7 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
             const float* smk = s_mask + buf * WS_BM + rg * 32;
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
-                if (sp[s].wrow < 0 || sp[s].glu == 2) continue;
+                if (sp[s].wrow < 0 || sp[s].glu == 2 || (rg & sp[s].rg_mask) != sp[s].rg_first) continue;
                 const WsSlot& t = sp[s];
                 const bool glu = sp[s].glu == 1;
                 const int sg = s + 1 < NS ? s + 1 : s;             // gate slot of a GLU unit (constant after unrolling)
@@ -1111,24 +1111,75 @@ bool ws_tile_ok(const ffk_linear_desc& d, const ffk_tile& t) {
     return d.M % 16 == 0 && t.inner % 16 == 0 && t.s_i == 1 && t.s_o % 8 == 0 && t.s_h % 8 == 0 && t.s_d % 8 == 0;
 }
 
-// Distributes the 32-row weight units over the waves.  The waves form G = 8 / R groups; the R waves
-// of a group hold the same units and take every R-th row group of a slab (R as large as the units
-// allow, so that few units still use all eight waves).  Returns false if the units do not fit.
+WsSlot ws_slot(const ffk_linear_desc& d, int tile, int chan, int wrow, int glu, int rg_first, int rg_step) {
+    const ffk_tile& t = d.tiles[tile];
+    const long coff = (long)(chan >> 5) * t.s_h;
+    WsSlot q{};
+    q.wrow = wrow;
+    q.glu = (signed char)glu;
+    q.out = (T*)t.out + coff;
+    q.resid = t.resid ? (const T*)t.resid + coff : nullptr;
+    q.gate = t.gate ? (const T*)t.gate + chan : nullptr;
+    q.bias = t.bias ? (const T*)t.bias + (wrow & 127) : nullptr;
+    q.xtail = t.xtail ? (int8_t*)t.xtail + coff : nullptr;
+    q.s_o = t.s_o;
+    q.s_i = t.s_i;
+    q.s_d = t.s_d;
+    q.gate_ld = t.gate_ld;
+    q.inner = (unsigned)t.inner;
+    q.gate_rows = (unsigned)t.gate_rows;
+    q.ncols_left = t.ncols - chan;
+    q.scale = t.scale;
+    q.kind = (signed char)t.kind;
+    q.act = (signed char)t.act;
+    q.masked = t.rowmask != nullptr;
+    q.has_bias = t.bias != nullptr;
+    q.by_rows = ws_by_rows(t);
+    q.tau = t.kind == FFK_TILE_STRIDED && t.s_d == 1;
+    q.sig = t.glu ? glu == 2 : t.act == FFK_ACT_SIGMOID;     // gate halves of a GLU unit and sigmoid tiles
+    q.rg_first = (signed char)rg_first;
+    q.rg_mask = (signed char)(rg_step - 1);
+    return q;
+}
+
+// Distributes the 32-row weight units over the waves; false if they do not fit.  Plain units, up to 16 of them: unit i goes to
+// wave i % 8 as its first or second slot; a round of at most four units is given to two or more waves each, which take every
+// second (or fourth ..) row group of a slab, so that any multiple of four units loads the waves equally.  Up to 32 plain units
+// are two column groups of 16: one launch pays for its start (6 .. 7 us) once.  Otherwise (GLU units) the waves form G = 8 / R
+// groups; the R waves of a group hold the same units and take every R-th row group (R as large as the units allow).
 bool ws_make_plan(const ffk_linear_desc& d, int n_tiles, WsArgs& p, int rg_per_slab, int max_ns) {
     struct Unit { int tile, chan, wrow, slots; };
     Unit units[FFK_MAX_TILES * 4];
     int nu = 0;
+    bool plain = true;
     for (int i = 0; i < n_tiles; ++i) {
         const ffk_tile& t = d.tiles[i];
         const int n = (t.ncols + 31) / 32;
-        for (int u = 0; u < n; ++u) {
-            Unit x;
-            x.tile = i;
-            x.chan = u * 32;
-            x.wrow = i * 128 + (t.glu ? u * 64 : u * 32);
-            x.slots = t.glu ? 2 : 1;
-            units[nu++] = x;
-        }
+        plain = plain && !t.glu;
+        for (int u = 0; u < n; ++u) units[nu++] = {i, u * 32, i * 128 + (t.glu ? u * 64 : u * 32), t.glu ? 2 : 1};
+    }
+    for (auto& q : p.slot) {
+        q = WsSlot{};
+        q.wrow = -1;
+    }
+    p.col_groups = 1;
+    if (plain && nu <= 32) {
+        p.max_slots = 2;
+        p.col_groups = nu <= 16 ? 1 : 2;
+        const int per = (nu + p.col_groups - 1) / p.col_groups;
+        for (int cg = 0; cg < p.col_groups; ++cg)
+            for (int sl = 0; sl < 2; ++sl) {
+                const int first = cg * per + 8 * sl;
+                int n = (cg + 1) * per < nu ? (cg + 1) * per - first : nu - first;
+                n = n > 8 ? 8 : n;
+                int R = 1;
+                while (n > 0 && 2 * R * n <= WS_WAVES && 2 * R <= rg_per_slab) R *= 2;
+                for (int w = 0; w < n * R; ++w) {
+                    const Unit& u = units[first + w % n];
+                    p.slot[(cg * WS_WAVES + w) * 2 + sl] = ws_slot(d, u.tile, u.chan, u.wrow, 0, w / n, R);
+                }
+            }
+        return true;
     }
     int assign[WS_WAVES][WS_NS];
     int G = 0, R = 0;
@@ -1156,47 +1207,19 @@ bool ws_make_plan(const ffk_linear_desc& d, int n_tiles, WsArgs& p, int rg_per_s
         if (fits) break;
     }
     if (R < 1) return false;
-    p.max_slots = 0;
+    p.max_slots = 2;
     for (int g = 0; g < G; ++g) {
         int n = 0;
         for (int sl = 0; sl < WS_NS; ++sl) n += assign[g][sl] != -1;
         p.max_slots = n > p.max_slots ? n : p.max_slots;
     }
-    p.groups = G;
-    p.rg_step = R;
-    for (int g = 0; g < G; ++g)
-        for (int sl = 0; sl < WS_NS; ++sl) {
-            WsSlot& q = p.slot[g][sl];
-            q = WsSlot{};
-            q.wrow = -1;
-            const int a = assign[g][sl];
+    if (p.max_slots > 2) p.max_slots = max_ns;                     // the slots a wave of the launched kernel has
+    for (int w = 0; w < WS_WAVES; ++w)
+        for (int sl = 0; sl < p.max_slots; ++sl) {
+            const int a = assign[w % G][sl];
             if (a == -1) continue;
             const Unit& u = units[a >= 0 ? a : -2 - a];
-            const ffk_tile& t = d.tiles[u.tile];
-            const long coff = (long)(u.chan >> 5) * t.s_h;
-            q.wrow = u.wrow + (a >= 0 ? 0 : 32);
-            q.glu = (signed char)(a < 0 ? 2 : u.slots == 2 ? 1 : 0);
-            q.out = (T*)t.out + coff;
-            q.resid = t.resid ? (const T*)t.resid + coff : nullptr;
-            q.gate = t.gate ? (const T*)t.gate + u.chan : nullptr;
-            q.bias = t.bias ? (const T*)t.bias + (q.wrow & 127) : nullptr;
-            q.xtail = t.xtail ? (int8_t*)t.xtail + coff : nullptr;
-            q.s_o = (int)t.s_o;
-            q.s_i = (int)t.s_i;
-            q.s_d = (int)t.s_d;
-            q.gate_ld = (int)t.gate_ld;
-            q.inner = (unsigned)t.inner;
-            q.gate_rows = (unsigned)t.gate_rows;
-            q.ncols_left = t.ncols - u.chan;
-            q.scale = t.scale;
-            q.kind = (signed char)t.kind;
-            q.act = (signed char)t.act;
-            q.masked = t.rowmask != nullptr;
-            q.has_bias = t.bias != nullptr;
-            q.by_rows = ws_by_rows(t);
-            q.tau = t.kind == FFK_TILE_STRIDED && t.s_d == 1;
-            // gate halves of a GLU unit and sigmoid tiles
-            q.sig = t.glu ? q.glu == 2 : t.act == FFK_ACT_SIGMOID;
+            p.slot[w * p.max_slots + sl] = ws_slot(d, u.tile, u.chan, u.wrow + (a >= 0 ? 0 : 32), a < 0 ? 2 : u.slots == 2 ? 1 : 0, w / G, R);
         }
     return true;
 }
@@ -1213,9 +1236,8 @@ int ws_launch(const WsArgs& args, hipStream_t st) {
         const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)linear_ws_kernel<NS, K, CM, DUAL, XT>, smem, "ffk_fused_linear");
         if (rc_lds != FFK_OK) return rc_lds;
     }
-    const int nslabs = ffk_cdiv(args.M, WS_BM);
-    const int grid = nslabs < WS_MAX_GRID ? nslabs : WS_MAX_GRID;
-    linear_ws_kernel<NS, K, CM, DUAL, XT><<<grid, WS_THREADS, smem, st>>>(args);
+    const int nslabs = ffk_cdiv(args.M, WS_BM), most = WS_MAX_GRID / args.col_groups;
+    linear_ws_kernel<NS, K, CM, DUAL, XT><<<dim3(nslabs < most ? nslabs : most, args.col_groups), WS_THREADS, smem, st>>>(args);
     return ffk_check_launch("ffk_fused_linear");
 }
 

@@ -29,14 +29,13 @@ def _plain(rows, width):
     return rows, 0, width
 
 
-def _rows(x, w, out, *, M, K, N, a_map=None, ln=None, bias=None, act=0, gate=None, gate_ld=0, w_row=0, out_ld=None, per=None):
+def _rows(x, w, out, *, M, K, N, a_map=None, ln=None, bias=None, act=0, gate=None, gate_ld=0, w_row=0, out_ld=None):
     """out[M, N] (row pitch ``out_ld``) = act(LN(x) W^T + b) over the rows ``a_map`` of x."""
     es = es_of(x.dtype)
     ld = N if out_ld is None else out_ld
     inner, so, si = _plain(M, K) if a_map is None else a_map
     nt = (N + 127) // 128
-    # the weights-stationary kernel holds 16 (K = 256) or 24 (K = 128) 32-channel units per launch
-    per = per or (4 if K == 256 else 6)
+    per = _lib.WS_TILES
     for t0 in range(0, nt, per):
         tiles = [make_tile(out.data_ptr() + t * 128 * es, bias=None if bias is None else bias.data_ptr() + t * 128 * es,
                            act=act, gate=None if gate is None else gate.data_ptr() + t * 128 * es, gate_ld=gate_ld,
@@ -195,7 +194,7 @@ def transition_backward(tr, x, dy, dx, g):
     h = alloc((M, H), dt, dev)
     _rows(x, w1, h, M=M, K=C, N=H, ln=ln, bias=b1, act=FFK_ACT_RELU)
     dh = alloc((M, H), dt, dev)
-    _rows(dy, w2t, dh, M=M, K=C, N=H, act=FFK_ACT_GATE_POS, gate=h, gate_ld=H, per=4)
+    _rows(dy, w2t, dh, M=M, K=C, N=H, act=FFK_ACT_GATE_POS, gate=h, gate_ld=H)
     dn, xn = alloc((M, C), dt, dev), alloc((M, C), dt, dev)
     _lib.bgemm_nt(dh, w1t, dn, M=M, N=C, K=H, lda=H, ldb=H)
     _wgrad(g[tr.linear2.weight], g[tr.linear2.bias], dy, h, M=M, N=C, K=H, dtype=dt, device=dev)
@@ -247,7 +246,7 @@ def attention_backward(owner, att, ln_mod, x, dy, dx, g, out_bias, *, B2, N, a_m
         first.append(make_tile(bias_t, kind=FFK_TILE_BIAS, inner=N, s_o=(NT + 1) * 1024, s_h=NT * (NT + 1) * 1024, ncols=H, scale=LOG2E))
     gates = [make_tile(gpre.data_ptr() + t * 128 * es, inner=M, s_i=HC) for t in range(HC // 128)]
     second = [*op_tiles("v_t", FFK_TILE_ACC), *op_tiles("v_v", FFK_TILE_V), *gates]
-    per = 4 if C == 256 else _lib.FFK_MAX_TILES          # 16 units of 32 channels per launch at K = 256
+    per = _lib.WS_TILES if C == 256 else _lib.FFK_MAX_TILES
     for w, ts in ((w_qk, first), (w_vg, second)):
         for t0 in range(0, len(ts), per):
             _lib.fused_linear(x, w, ts[t0:t0 + per], w_row_off=t0 * 128, **akw)

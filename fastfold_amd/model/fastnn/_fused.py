@@ -218,7 +218,7 @@ def transition(x, out, *, ln, w1_pk, b1_pk, w2, b2, hidden, budget, xtail=None):
     nt = hidden // 128
     for r0 in range(0, M, rows):
         n = min(rows, M - r0)
-        per = 4 if (dt == torch.bfloat16 and C == 256) else _lib.FFK_MAX_TILES
+        per = _lib.WS_TILES if dt == torch.bfloat16 else _lib.FFK_MAX_TILES
         for t0 in range(0, nt, per):
             tiles = [make_tile(hid.data_ptr() + t * 128 * es, bias=b1_pk.data_ptr() + t * 128 * es, inner=n,
                                s_i=hidden, act=FFK_ACT_RELU)
@@ -369,8 +369,7 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
                                        inner=Ms, s_i=HC, act=FFK_ACT_SIGMOID))
         if bias_tile is not None:      # single slab: the bias rides on the projection launch
             tiles.append(bias_tile)
-        # the weights-stationary kernel holds at most 16 (K = 256) or 24 (K = 128) 32-channel units per launch
-        per = (3 if gate_in_out else 4) if (acc_order and C == 256) else len(tiles)
+        per = _lib.WS_TILES if (acc_order and C == 256) else len(tiles)
         for t0 in range(0, len(tiles), per):
             # a bias tile riding behind q, k, v (no gate tiles) takes its weight rows from the gate-less packing
             wp = w_pk.without_gate if (gate_in_out and bias_tile is not None) else w_pk

@@ -564,3 +564,21 @@ def test_fp32_weights_stationary_matches_staged(dev, case):
         got.append(outs)
     for a, c in zip(*got):
         assert torch.isfinite(a).all() and float((a - c).abs().max()) <= 1e-5 * float(a.abs().max())
+
+
+@pytest.mark.parametrize("K", [64, 128, 256])
+@pytest.mark.parametrize("N,M", [(96, 33), (288, 129), (416, 700), (544, 1000), (1024, 130)])
+def test_weights_stationary_unit_shares(dev, K, N, M):
+    """Unit counts that are shared by several waves (3 of 9, 13), fill a column group (16 of 17) or two of them (32)."""
+    from fastfold_amd import _lib
+    F = torch.nn.functional
+    g = torch.Generator().manual_seed(N + K)
+    x, w, b = (torch.randn(*sh, generator=g).to(dev, torch.bfloat16) for sh in ((M, K), (N, K), (N,)))
+    ln = (torch.rand(K, generator=g).to(dev, torch.bfloat16) + 0.5, torch.randn(K, generator=g).to(dev, torch.bfloat16))
+    nt = (N + 127) // 128
+    wp, bp = _pack(w, nt), F.pad(b, (0, nt * 128 - N))
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
+    tiles = [_lib.make_tile(out.data_ptr() + 256 * i, inner=M, s_i=N, bias=bp.data_ptr() + 256 * i, ncols=min(128, N - 128 * i)) for i in range(nt)]
+    _lib.fused_linear(x, wp, tiles, M=M, K=K, ln=ln)
+    ref = F.linear(F.layer_norm(x.float(), (K,), ln[0].float(), ln[1].float()), w.float(), b.float())
+    assert torch.isfinite(out).all() and float((out.float() - ref).norm() / ref.norm()) < 6e-3
