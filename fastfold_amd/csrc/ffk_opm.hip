@@ -3,8 +3,8 @@
 //     O_ij[d, e]   = sum_s a[s, i, d] * b[s, j, e]                       (32 x 32 per residue pair)
 // without ever writing the [r, r, 1024] outer product to memory.
 //
-// A workgroup (8 wavefronts) owns 8 i x 32 j = 256 residue pairs and walks the 32 values of e in 16
-// chunks of two.  Per chunk:
+// A workgroup (8 wavefronts) owns TI i x 32 j residue pairs, TI = 8 or 4, and walks the 32 values of e in 16
+// chunks of two.  Per chunk (TI = 8):
 //   phase A  (outer product)  wave w multiplies its own i = i0 + w: rows (d) x columns (j, e in chunk),
 //            K = s.  Its a-fragments stay in registers for the whole tile; the b rows of the chunk come
 //            from LDS.  The 32 x 32 results are rounded to bf16 and written to LDS as rows of
@@ -13,19 +13,19 @@
 //            wave owns 2 x 2 of them; accumulators live in registers across all chunks.
 // b and W2 chunks arrive by direct global -> LDS loads (XOR-swizzled unpadded rows) one iteration
 // ahead; phase B of chunk q - 1 and phase A of chunk q run between the same pair of barriers, so there
-// is one barrier per chunk.  The weight is expected pre-permuted to k2 = e * 32 + d order.
+// is one barrier per chunk.  With TI = 4 two waves share an i (one column tile each) and a wave owns 1 x 2 output tiles: half
+// the work per chunk and twice the workgroups, for launches that leave CUs empty (see ffk_opm_fused).  The weight is expected pre-permuted to k2 = e * 32 + d order.
 #include "ffk_common.h"
 
 namespace {
 
 typedef bf16_t T;
 constexpr int OP_THREADS = 512;
-constexpr int OP_TI = 8, OP_TJ = 32;            // pairs per workgroup: 8 i x 32 j
+constexpr int OP_TJ = 32;                        // pairs per workgroup: TI i x 32 j
 constexpr int OP_EC = 2;                         // values of e per chunk
 constexpr int OP_NCHUNK = 32 / OP_EC;            // 16
 constexpr int OP_K2C = OP_EC * 32;               // k2 elements per chunk (64)
 constexpr int OP_PA = OP_K2C * 2 + 16;           // A2 row pitch in bytes (padded: written by ds_write)
-constexpr int OP_A2 = OP_TI * OP_TJ * OP_PA;     // one A2 buffer
 constexpr int OP_W2SLOT = 128 * OP_K2C * 2;      // W2 chunk: 128 rows of 128 bytes (16 KB)
 
 __device__ __forceinline__ int op_tau(int i) { return ((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3); }
@@ -35,12 +35,14 @@ __device__ __forceinline__ void op_load_lds(const T* src, unsigned char* dst_wav
                                      (__attribute__((address_space(3))) void*)dst_wave, 16, 0, 0);
 }
 
-template <int KS1>   // MFMA K steps of the outer product: spad / 16 (4 or 8)
+template <int KS1, int OP_TI>   // MFMA K steps of the outer product: spad / 16 (4 or 8)
 __global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict__ out, const T* __restrict__ resid, int8_t* __restrict__ xtail,
                                                                  const T* __restrict__ at, const T* __restrict__ bt,
                                                                  const T* __restrict__ w2p, const T* __restrict__ bias,
                                                                  const float* __restrict__ norm, int r, float eps) {
     typedef Mma<T> MM;
+    constexpr int OP_A2 = OP_TI * OP_TJ * OP_PA;         // one A2 buffer
+    constexpr int MT = OP_TI / 4, WI = 8 / OP_TI, NCT = 2 / WI;    // m-tiles per wave (phase B), waves per i, column tiles per wave (phase A)
     constexpr int SPAD = KS1 * 16;                       // K of the outer product
     constexpr int BROW = SPAD * 2;                       // bytes per b row (128 or 256)
     constexpr int BCOLS = BROW / 16;                     // 16-byte columns per b row (8 or 16)
@@ -57,10 +59,11 @@ __global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict_
     const int tiles_j = r / OP_TJ;
     const int i0 = (blockIdx.x / tiles_j) * OP_TI, j0 = (blockIdx.x % tiles_j) * OP_TJ;
 
+    const int iw = wave / WI, ctw = (wave % WI) * NCT;   // phase A: this wave's i and first column tile
     // ---- a fragments of this wave's i (rows d through tau: registers of the result hold d = 16 half + v) ----
     bf16x8 af[KS1];
     {
-        const T* ap = at + ((long)(i0 + wave) * 32 + op_tau(l32)) * SPAD + half * 8;
+        const T* ap = at + ((long)(i0 + iw) * 32 + op_tau(l32)) * SPAD + half * 8;
 #pragma unroll
         for (int ks = 0; ks < KS1; ++ks) af[ks] = MM::ld(ap + ks * 16);
     }
@@ -90,11 +93,11 @@ __global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict_
         for (int i = 0; i < 2; ++i) op_load_lds(wsrc[i] + q * OP_K2C, ws + i * (OP_THREADS * 16));
     };
 
-    // ---- phase B roles: m-tiles 2 * (wave % 4) + {0, 1}, c-tiles 2 * (wave / 4) + {0, 1} ----
-    const int mt0 = 2 * (wave & 3), ct0 = 2 * (wave >> 2);
-    f32x16 acc2[2][2];   // [m][c]
+    // ---- phase B roles: m-tiles MT * (wave % 4) .., c-tiles 2 * (wave / 4) + {0, 1} ----
+    const int mt0 = MT * (wave & 3), ct0 = 2 * (wave >> 2);
+    f32x16 acc2[MT][2];   // [m][c]
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < MT; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
@@ -111,16 +114,16 @@ __global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict_
     int woff[4];                                         // W2 fragment of c-tile 0: row l32, column 2 ks + half
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) woff[ks] = l32 * 128 + (((2 * ks + half) ^ ((l32 >> 1) & 7)) << 4);
-    // A2 write position of phase A: pair (wave, 16 ct + l32 / 2), k2 = (l32 & 1) * 32 + 16 half
-    const int a2w = (wave * 32 + (l32 >> 1)) * OP_PA + ((l32 & 1) * 32 + 16 * half) * 2;
+    // A2 write position of phase A: pair (iw, 16 ct + l32 / 2), k2 = (l32 & 1) * 32 + 16 half
+    const int a2w = (iw * 32 + (l32 >> 1)) * OP_PA + ((l32 & 1) * 32 + 16 * half) * 2;
     // A2 fragment of phase B: pair row mt * 32 + l32, k2 = 16 ks + 8 half
     const int a2r = l32 * OP_PA + half * 16;
 
     // The epilogue's operands (residual, its tail, the normaliser) are requested during the third chunk, not in the
     // epilogue: with one workgroup per CU (154 KB of LDS) nothing else would cover their latency - four dependent round
     // trips took 8 of a workgroup's 42 microseconds.  The wait at the top of the next chunk covers them.
-    u32x4 e_rv[2][2][2], e_tv[2][2];
-    float e_norm[2];
+    u32x4 e_rv[MT][2][2], e_tv[MT][2];
+    float e_norm[MT];
     const int pf_q = 2 + (int)((blockIdx.x >> 3) % 12u);   // spread over the chunks: the workgroups of a launch run in step
     fetch(0);
     for (int q = 0; q <= OP_NCHUNK; ++q) {
@@ -129,7 +132,7 @@ __global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict_
         if (q + 1 < OP_NCHUNK) fetch(q + 1);
         if (q == pf_q) {
 #pragma unroll
-            for (int m = 0; m < 2; ++m) {
+            for (int m = 0; m < MT; ++m) {
                 const long pr = (long)(i0 + mt0 + m) * r + j0 + l32;
                 e_norm[m] = norm[pr];
 #pragma unroll
@@ -147,13 +150,13 @@ __global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict_
             const unsigned char* w2 = s_w2 + ((q - 1) % 3) * OP_W2SLOT;
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
-                bf16x8 fa[2], fw[2];
+                bf16x8 fa[MT], fw[2];
 #pragma unroll
-                for (int m = 0; m < 2; ++m) fa[m] = *reinterpret_cast<const bf16x8*>(a2 + (mt0 + m) * 32 * OP_PA + a2r + ks * 32);
+                for (int m = 0; m < MT; ++m) fa[m] = *reinterpret_cast<const bf16x8*>(a2 + (mt0 + m) * 32 * OP_PA + a2r + ks * 32);
 #pragma unroll
                 for (int c = 0; c < 2; ++c) fw[c] = *reinterpret_cast<const bf16x8*>(w2 + (ct0 + c) * 32 * 128 + woff[ks]);
 #pragma unroll
-                for (int m = 0; m < 2; ++m)
+                for (int m = 0; m < MT; ++m)
 #pragma unroll
                     for (int c = 0; c < 2; ++c) MM::mma(acc2[m][c], fw[c], fa[m]);
             }
@@ -163,7 +166,8 @@ __global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict_
             const unsigned char* bs = s_b + (q & 1) * BSLOT;
             unsigned char* a2 = s_a2 + (q & 1) * OP_A2;
 #pragma unroll
-            for (int ct = 0; ct < 2; ++ct) {
+            for (int c1 = 0; c1 < NCT; ++c1) {
+                const int ct = ctw + c1;
                 f32x16 o;
 #pragma unroll
                 for (int v = 0; v < 16; ++v) o[v] = 0.0f;
@@ -182,7 +186,7 @@ __global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict_
 
     // ---- epilogue: lane = pair, registers = 16 consecutive channels ----
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
+    for (int m = 0; m < MT; ++m) {
         const long pr = (long)(i0 + mt0 + m) * r + j0 + l32;
         const float inv = 1.0f / (e_norm[m] + eps);
 #pragma unroll
@@ -218,17 +222,17 @@ __global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict_
     }
 }
 
-template <int KS1>
+template <int KS1, int OP_TI>
 int opm_launch(T* out, const T* resid, int8_t* xtail, const T* at, const T* bt, const T* w2p, const T* bias, const float* norm, int r,
                float eps, hipStream_t st) {
-    const size_t smem = 2 * (size_t)OP_A2 + 3 * OP_W2SLOT + 2 * (size_t)(OP_TJ * OP_EC * KS1 * 32);
+    const size_t smem = 2 * (size_t)(OP_TI * OP_TJ * OP_PA) + 3 * OP_W2SLOT + 2 * (size_t)(OP_TJ * OP_EC * KS1 * 32);
     static FfkLdsReservation lds_reserved;
     {
-        const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)opm_fused_kernel<KS1>, smem, "ffk_opm_fused");
+        const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)opm_fused_kernel<KS1, OP_TI>, smem, "ffk_opm_fused");
         if (rc_lds != FFK_OK) return rc_lds;
     }
     const unsigned grid = (unsigned)((r / OP_TI) * (r / OP_TJ));
-    opm_fused_kernel<KS1><<<grid, OP_THREADS, smem, st>>>(out, resid, xtail, at, bt, w2p, bias, norm, r, eps);
+    opm_fused_kernel<KS1, OP_TI><<<grid, OP_THREADS, smem, st>>>(out, resid, xtail, at, bt, w2p, bias, norm, r, eps);
     return ffk_check_launch("ffk_opm_fused");
 }
 
@@ -244,7 +248,11 @@ extern "C" int ffk_opm_fused(void* out, const void* resid, void* xtail, const vo
                     ffk_aligned16(bias) && ffk_aligned16(xtail),
                 FFK_ERR_ALIGN, "ffk_opm_fused: buffers must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
-    if (spad == 128)
-        return opm_launch<8>((T*)out, (const T*)resid, (int8_t*)xtail, (const T*)a_t, (const T*)b_t, (const T*)w2p, (const T*)bias, norm, (int)r, eps, st);
-    return opm_launch<4>((T*)out, (const T*)resid, (int8_t*)xtail, (const T*)a_t, (const T*)b_t, (const T*)w2p, (const T*)bias, norm, (int)r, eps, st);
+    // Four i per workgroup while these give no CU a second one (a workgroup's time is mostly its 17 barriers: r = 96, 128
+    // sequences: 36 workgroups of eight 31.4 us, 72 of four 21.3 us; r = 160: 33.9 and 24.0 us; r = 192: 35.2 and 44.0 us).
+    const bool small = (r / 4) * (r / OP_TJ) <= 256;
+#define FFK_OPM(KS1, TI) opm_launch<KS1, TI>((T*)out, (const T*)resid, (int8_t*)xtail, (const T*)a_t, (const T*)b_t, (const T*)w2p, (const T*)bias, norm, (int)r, eps, st)
+    if (spad == 128) return small ? FFK_OPM(8, 4) : FFK_OPM(8, 8);
+    return small ? FFK_OPM(4, 4) : FFK_OPM(4, 8);
+#undef FFK_OPM
 }
