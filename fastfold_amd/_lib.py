@@ -25,6 +25,7 @@ _P, _I, _L, _F = c_void_p, c_int, c_int64, c_float
 SIGNATURES = {
     "ffk_softmax_fwd": [_P, _P, _P, _P, _L, _L, _L, _L, _L, _I, _P],
     "ffk_softmax_bwd": [_P, _P, _P, _L, _L, _I, _P],
+    "ffk_softmax_bwd_bias": [_P, _P, _P, _L, _P, _P, _L, _L, _L, _L, _I, _P],
     "ffk_layernorm_fwd": [_P, _P, _P, _P, _P, _P, _L, _L, _F, _I, _P],
     "ffk_layernorm_bwd": [_P, _P, _P, _P, _P, _P, _P, _P, _L, _L, _I, _P],
     "ffk_bias_sigmoid_mul": [_P, _P, _P, _P, _L, _L, _I, _P],
@@ -324,6 +325,41 @@ def tile_pack(x, kind, scale=1.0):
             call("ffk_tile_pack", ptr(out[p]), x.data_ptr() + p * 32 * x.element_size(), B2, H, N, min(D, 32),
                  x.stride(0), x.stride(1), x.stride(2), float(scale), kind, dtype_tag(x.dtype), stream_ptr())
     return out[0] if D <= 32 else out
+
+
+FFK_PACK_JOBS = 4
+
+
+class PackJob(ctypes.Structure):
+    """Mirror of ``ffk_pack_job`` (include/ffk.h)."""
+    _fields_ = [("src", c_void_p), ("qk", c_void_p), ("acc", c_void_p), ("other", c_void_p), ("dsum", c_void_p),
+                ("s_b", c_int64), ("s_h", c_int64), ("s_n", c_int64), ("o_sb", c_int64), ("o_sh", c_int64), ("o_sn", c_int64),
+                ("scale", c_float), ("tiled", c_int)]
+
+
+class PackDesc(ctypes.Structure):
+    """Mirror of ``ffk_pack_desc`` (include/ffk.h)."""
+    _fields_ = [("job", PackJob * FFK_PACK_JOBS), ("bias", c_void_p), ("bias_t", c_void_p), ("bias_scale", c_float),
+                ("n", c_int), ("B2", c_int), ("H", c_int), ("N", c_int), ("D", c_int), ("dtype", c_int), ("reserved", c_int)]
+
+
+SIGNATURES["ffk_attention_pack"] = [ctypes.POINTER(PackDesc), _P]
+
+
+def attention_pack(jobs, *, B2, H, N, D, dtype, bias=None, bias_t=None, bias_scale=1.0):
+    """``jobs``: tuples (src, scale, qk, acc, dsum, other); ``src`` and ``other`` are [B2, H, N, D] views with contiguous
+    channels, or ``src`` the [B2, H, ceil(N/32), 1024] FFK_TILE_QK tiles of an earlier call."""
+    d = PackDesc(bias=ptr(bias), bias_t=ptr(bias_t), bias_scale=bias_scale, n=len(jobs), B2=B2, H=H, N=N, D=D, dtype=dtype_tag(dtype))
+    for j, (src, scale, qk, acc, dsum, other) in zip(d.job, jobs):
+        tiled = src.shape[-1] == 1024
+        # raw pointers: the operands may be strided views (their strides go along), which ``ptr`` would refuse
+        j.src, j.qk, j.acc, j.dsum, j.scale, j.tiled = src.data_ptr(), ptr(qk), ptr(acc), ptr(dsum), scale, int(tiled)
+        if not tiled:
+            j.s_b, j.s_h, j.s_n = src.stride()[:3]
+        if other is not None:
+            j.other = other.data_ptr()
+            j.o_sb, j.o_sh, j.o_sn = other.stride()[:3]
+    call("ffk_attention_pack", ctypes.byref(d), stream_ptr())
 
 
 SIGNATURES["ffk_pair_bias"] = [_P, _P, _P, _P, _P, _P, _L, _L, _L, _L, _L, _L, _F, _F, _I, _P]

@@ -42,6 +42,14 @@ template <typename T> struct Tile16 {         // the 16 elements one lane owns o
 #pragma unroll
         for (int i = 0; i < NV; ++i) v[i] = ld16(p + i * DT<T>::VEC);
     }
+    // Both operands of a product over the tiles' minor index may take that index in any common order: access i of the lanes of
+    // row `row` covers elements 16 i' + VEC (2 i'' + half) .. of it (bf16: i' = i, so that one access of the wave is a
+    // contiguous KB; in the order of load() it is every other 16 bytes of two).  p: the tile + row * 16.
+    __device__ __forceinline__ void load_rows(const T* p, int half) {
+        constexpr int PER = NV / 2;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) v[i] = ld16(p + (i / PER) * 512 + ((i % PER) * 2 + half) * DT<T>::VEC);
+    }
     __device__ __forceinline__ float f(int j) const { return DT<T>::to_f(v[j / DT<T>::VEC].e[j % DT<T>::VEC]); }
     __device__ __forceinline__ typename Mma<T>::Frag frag(int i) const {
         return *reinterpret_cast<const typename Mma<T>::Frag*>(
@@ -70,9 +78,10 @@ template <> struct NFrag<float> {
 
 template <typename T>
 __device__ __forceinline__ typename Mma<T>::Frag identity_frag(int i, int l32, int half) {
+    constexpr int PER = 8 / Mma<T>::KLANE;                      // the order of Tile16::load_rows
     typename Mma<T>::Frag f;
 #pragma unroll
-    for (int t = 0; t < Mma<T>::KLANE; ++t) f[t] = (T)((16 * half + i * Mma<T>::KLANE + t) == l32 ? 1.0f : 0.0f);
+    for (int t = 0; t < Mma<T>::KLANE; ++t) f[t] = (T)((16 * (i / PER) + ((i % PER) * 2 + half) * Mma<T>::KLANE + t) == l32 ? 1.0f : 0.0f);
     return f;
 }
 
@@ -102,7 +111,7 @@ __device__ __forceinline__ void store4(T* o, const float* f) {          // four 
 // STATS: the row statistics are computed here (a walk over the keys of its own) and written for the other kernels; otherwise
 // the forward pass has left the log-sum-exp and the gate's backward kernel sum_d do o.
 template <typename T, int DP, bool HAS_BIAS, bool STATS>
-__global__ __launch_bounds__(256) void attention_bwd_dq_kernel(
+__global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 4 : 1) void attention_bwd_dq_kernel(
     T* __restrict__ dq, float* __restrict__ lse, float* __restrict__ dsum, const T* __restrict__ q_qk,
     const T* __restrict__ k_qk, const T* __restrict__ k_acc, const T* __restrict__ v_qk, const T* __restrict__ bias_t,
     const float* __restrict__ keybias, const T* __restrict__ do_qk, const T* __restrict__ o_qk, int B2, int H, int Nq,
@@ -123,11 +132,11 @@ __global__ __launch_bounds__(256) void attention_bwd_dq_kernel(
     float dpart = 0.0f;
 #pragma unroll
     for (int p = 0; p < DP; ++p) {
-        qf[p].load(q_qk + p * part_q + ((bh * QT + qt) << 10) + lane * 16);
-        dof[p].load(do_qk + p * part_q + ((bh * QT + qt) << 10) + lane * 16);
+        qf[p].load_rows(q_qk + p * part_q + ((bh * QT + qt) << 10) + l32 * 16, half);
+        dof[p].load_rows(do_qk + p * part_q + ((bh * QT + qt) << 10) + l32 * 16, half);
         if (STATS) {
             Tile16<T> of;
-            of.load(o_qk + p * part_q + ((bh * QT + qt) << 10) + lane * 16);
+            of.load_rows(o_qk + p * part_q + ((bh * QT + qt) << 10) + l32 * 16, half);
 #pragma unroll
             for (int j = 0; j < 16; ++j) dpart += dof[p].f(j) * of.f(j);
         }
@@ -148,13 +157,13 @@ __global__ __launch_bounds__(256) void attention_bwd_dq_kernel(
 #pragma unroll
         for (int p = 0; p < DP; ++p) {
             Tile16<T> kc;
-            kc.load(k_qk + p * part_k + ((bh * KT + kt) << 10) + lane * 16);
+            kc.load_rows(k_qk + p * part_k + ((bh * KT + kt) << 10) + l32 * 16, half);
 #pragma unroll
             for (int i = 0; i < NF; ++i) MM::mma(s, kc.frag(i), qf[p].frag(i));
         }
         if (HAS_BIAS) {
             Tile16<T> bc;
-            bc.load(bias_t + ((((long)h * QT + qt) * (KT + bias_pad) + kt) << 10) + lane * 16);
+            bc.load_rows(bias_t + ((((long)h * QT + qt) * (KT + bias_pad) + kt) << 10) + l32 * 16, half);
 #pragma unroll
             for (int i = 0; i < NF; ++i) MM::mma(s, bc.frag(i), ident[i]);
         }
@@ -194,37 +203,69 @@ __global__ __launch_bounds__(256) void attention_bwd_dq_kernel(
         L = lse[(bh * QT + qt) * 32 + l32];
     }
 
-    // second walk: dq^T += k^T . dS^T
+    // second walk: dq^T += k^T . dS^T.  What a step reads is requested for the next step as soon as its registers are free
+    // (a step later it is there; waiting for each tile where it is used took 57 us at 128 x 8 heads of 256 x 256 logits).
+    // The scores start at key bias - log-sum-exp and dP at -D, so that the products leave the exponent and dP - D themselves.
     f32x16 acc[DP];
 #pragma unroll
     for (int p = 0; p < DP; ++p)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[p][v] = 0.0f;
-    for (int kt = 0; kt < KT; ++kt) {
-        f32x16 s, dp;
-        score(kt, s);
+    Tile16<T> kc[DP], vq[DP], ka[DP], bc;
+    f32x4 mk[4];
+    const T* bias_row = HAS_BIAS ? bias_t + ((((long)h * QT + qt) * (KT + bias_pad)) << 10) + l32 * 16 : nullptr;
+    const long krow = (bh * KT) << 10;
+    auto load_mask = [&](int kt) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) dp[v] = 0.0f;
+        for (int g = 0; g < 4; ++g) mk[g] = *reinterpret_cast<const f32x4*>(mp + kt * 32 + 8 * g);
+    };
+    auto load_scores = [&](int kt) {
 #pragma unroll
         for (int p = 0; p < DP; ++p) {
-            Tile16<T> vq;
-            vq.load(v_qk + p * part_k + ((bh * KT + kt) << 10) + lane * 16);
-#pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(dp, vq.frag(i), dof[p].frag(i));      // dP^T[key, q] = v[key] . do[q]
+            kc[p].load_rows(k_qk + p * part_k + krow + ((long)kt << 10) + l32 * 16, half);
+            vq[p].load_rows(v_qk + p * part_k + krow + ((long)kt << 10) + l32 * 16, half);
         }
+        if (HAS_BIAS) bc.load_rows(bias_row + ((long)kt << 10), half);
+    };
+    auto load_acc = [&](int kt) {
+#pragma unroll
+        for (int p = 0; p < DP; ++p) ka[p].load(k_acc + p * part_k + krow + ((long)kt << 10) + lane * 16);
+    };
+    load_mask(0);
+    load_scores(0);
+    load_acc(0);
+    for (int kt = 0; kt < KT; ++kt) {
+        const int next = kt + 1 < KT ? kt + 1 : kt;
+        f32x16 s, dp;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            s[v] = mk[v >> 2][v & 3] - L;
+            dp[v] = -D;
+        }
+#pragma unroll
+        for (int p = 0; p < DP; ++p) {
+#pragma unroll
+            for (int i = 0; i < NF; ++i) MM::mma(s, kc[p].frag(i), qf[p].frag(i));
+#pragma unroll
+            for (int i = 0; i < NF; ++i) MM::mma(dp, vq[p].frag(i), dof[p].frag(i));   // dP^T[key, q] = v[key] . do[q]
+        }
+        if (HAS_BIAS) {
+#pragma unroll
+            for (int i = 0; i < NF; ++i) MM::mma(s, bc.frag(i), ident[i]);
+        }
+        load_scores(next);
         float ds[16];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) ds[v] = fast_exp2(s[v] - L) * (dp[v] - D);
+        for (int v = 0; v < 16; ++v) ds[v] = fast_exp2(s[v]) * dp[v];
         Frag dsf[NF];
 #pragma unroll
         for (int i = 0; i < NF; ++i) dsf[i] = NFrag<T>::make(ds + i * MM::KLANE);
+        load_mask(next);                                       // late: the registers are those of the scores
 #pragma unroll
-        for (int p = 0; p < DP; ++p) {
-            Tile16<T> ka;
-            ka.load(k_acc + p * part_k + ((bh * KT + kt) << 10) + lane * 16);
+        for (int p = 0; p < DP; ++p)
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(acc[p], ka.frag(i), dsf[i]);
-        }
+            for (int i = 0; i < NF; ++i) MM::mma(acc[p], ka[p].frag(i), dsf[i]);
+        load_acc(next);
     }
     const int q = qt * 32 + l32;
     if (q < Nq) {
@@ -243,7 +284,7 @@ __global__ __launch_bounds__(256) void attention_bwd_dq_kernel(
 
 // ------------------------------------------------------------------------- dk, dv ----
 template <typename T, int DP>
-__global__ __launch_bounds__(256) void attention_bwd_dkv_kernel(
+__global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 3 : 1) void attention_bwd_dkv_kernel(
     T* __restrict__ dk, T* __restrict__ dv, const T* __restrict__ q_qk,
     const T* __restrict__ q_acc, const T* __restrict__ k_qk, const T* __restrict__ v_qk, const T* __restrict__ bias_t,
     const float* __restrict__ keybias, const T* __restrict__ do_qk, const T* __restrict__ do_acc,
@@ -264,8 +305,8 @@ __global__ __launch_bounds__(256) void attention_bwd_dkv_kernel(
     Tile16<T> kf[DP], vf[DP];                      // this lane's key (column l32): k and v rows as N operands
 #pragma unroll
     for (int p = 0; p < DP; ++p) {
-        kf[p].load(k_qk + p * part_k + ((bh * KT + kt) << 10) + lane * 16);
-        vf[p].load(v_qk + p * part_k + ((bh * KT + kt) << 10) + lane * 16);
+        kf[p].load_rows(k_qk + p * part_k + ((bh * KT + kt) << 10) + l32 * 16, half);
+        vf[p].load_rows(v_qk + p * part_k + ((bh * KT + kt) << 10) + l32 * 16, half);
     }
     const int key = kt * 32 + l32;
     const float kb = keybias[(long)b2 * KT * 32 + key];     // 0, masked (-1e9 log2e) or padding (hugely negative)
@@ -280,39 +321,63 @@ __global__ __launch_bounds__(256) void attention_bwd_dkv_kernel(
     for (int p = 0; p < DP; ++p)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc_k[p][v] = acc_v[p][v] = 0.0f;
-    for (int qt = 0; qt < QT; ++qt) {
-        f32x16 s, dp;
+    // as in the dq kernel: each operand is requested for the next step once its registers are free
+    Tile16<T> qc[DP], doc[DP], qa[DP], doa[DP], bc;
+    f32x4 L4[4], D4[4];
+    const long qrow = (bh * QT) << 10;
+    const float* lp = lse + bh * QT * 32 + 4 * half;
+    const float* dpz = dsum + bh * QT * 32 + 4 * half;
+    const T* bias_col = bias_t ? bias_t + ((((long)h * QT) * (KT + bias_pad) + kt) << 10) + l32 * 16 : nullptr;
+    auto load_rows = [&](int qt) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) s[v] = dp[v] = 0.0f;
+        for (int g = 0; g < 4; ++g) {
+            L4[g] = *reinterpret_cast<const f32x4*>(lp + qt * 32 + 8 * g);
+            D4[g] = *reinterpret_cast<const f32x4*>(dpz + qt * 32 + 8 * g);
+        }
+    };
+    auto load_scores = [&](int qt) {
 #pragma unroll
         for (int p = 0; p < DP; ++p) {
-            Tile16<T> qc, doc;
-            qc.load(q_qk + p * part_q + ((bh * QT + qt) << 10) + lane * 16);
-            doc.load(do_qk + p * part_q + ((bh * QT + qt) << 10) + lane * 16);
+            qc[p].load_rows(q_qk + p * part_q + qrow + ((long)qt << 10) + l32 * 16, half);
+            doc[p].load_rows(do_qk + p * part_q + qrow + ((long)qt << 10) + l32 * 16, half);
+        }
+        if (bias_t) bc.load_rows(bias_col + (((long)qt * (KT + bias_pad)) << 10), half);
+    };
+    auto load_acc = [&](int qt) {
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(s, qc.frag(i), kf[p].frag(i));       // S[q, key], log2 domain
+        for (int p = 0; p < DP; ++p) {
+            qa[p].load(q_acc + p * part_q + qrow + ((long)qt << 10) + lane * 16);
+            doa[p].load(do_acc + p * part_q + qrow + ((long)qt << 10) + lane * 16);
+        }
+    };
+    load_rows(0);
+    load_scores(0);
+    load_acc(0);
+    for (int qt = 0; qt < QT; ++qt) {
+        const int next = qt + 1 < QT ? qt + 1 : qt;
+        f32x16 s, dp;
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(dp, doc.frag(i), vf[p].frag(i));     // dP[q, key] = do[q] . v[key]
+        for (int v = 0; v < 16; ++v) {
+            s[v] = kb - L4[v >> 2][v & 3];
+            dp[v] = -D4[v >> 2][v & 3];
+        }
+#pragma unroll
+        for (int p = 0; p < DP; ++p) {
+#pragma unroll
+            for (int i = 0; i < NF; ++i) MM::mma(s, qc[p].frag(i), kf[p].frag(i));       // S[q, key], log2 domain
+#pragma unroll
+            for (int i = 0; i < NF; ++i) MM::mma(dp, doc[p].frag(i), vf[p].frag(i));     // dP[q, key] = do[q] . v[key]
         }
         if (bias_t) {                                                           // S += I . bias (rows = queries)
-            Tile16<T> bc;
-            bc.load(bias_t + ((((long)h * QT + qt) * (KT + bias_pad) + kt) << 10) + lane * 16);
 #pragma unroll
             for (int i = 0; i < NF; ++i) MM::mma(s, ident[i], bc.frag(i));
         }
-        const float* lp = lse + (bh * QT + qt) * 32 + 4 * half;
-        const float* dpz = dsum + (bh * QT + qt) * 32 + 4 * half;
+        load_scores(next);
         float p[16], ds[16];
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const f32x4 L4 = *reinterpret_cast<const f32x4*>(lp + 8 * g);
-            const f32x4 D4 = *reinterpret_cast<const f32x4*>(dpz + 8 * g);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int v = 4 * g + e;
-                p[v] = fast_exp2(s[v] + kb - L4[e]);
-                ds[v] = p[v] * (dp[v] - D4[e]);
-            }
+        for (int v = 0; v < 16; ++v) {
+            p[v] = fast_exp2(s[v]);
+            ds[v] = p[v] * dp[v];
         }
         Frag pfr[NF], dsf[NF];
 #pragma unroll
@@ -320,16 +385,15 @@ __global__ __launch_bounds__(256) void attention_bwd_dkv_kernel(
             pfr[i] = NFrag<T>::make(p + i * MM::KLANE);
             dsf[i] = NFrag<T>::make(ds + i * MM::KLANE);
         }
+        load_rows(next);                                   // late: the 32 registers are those of the scores
 #pragma unroll
         for (int pp = 0; pp < DP; ++pp) {
-            Tile16<T> qa, doa;
-            qa.load(q_acc + pp * part_q + ((bh * QT + qt) << 10) + lane * 16);
-            doa.load(do_acc + pp * part_q + ((bh * QT + qt) << 10) + lane * 16);
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(acc_v[pp], doa.frag(i), pfr[i]);   // dv^T += do^T . P
+            for (int i = 0; i < NF; ++i) MM::mma(acc_v[pp], doa[pp].frag(i), pfr[i]);   // dv^T += do^T . P
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(acc_k[pp], qa.frag(i), dsf[i]);    // dk^T += q^T . dS
+            for (int i = 0; i < NF; ++i) MM::mma(acc_k[pp], qa[pp].frag(i), dsf[i]);    // dk^T += q^T . dS
         }
+        load_acc(next);
     }
     if (key < Nk) {
         const long o = (long)b2 * om.s_b + (long)h * om.s_h + (long)key * om.s_n + 4 * half;
@@ -352,7 +416,7 @@ __global__ __launch_bounds__(256) void attention_bwd_dkv_kernel(
 // ---------------------------------------------------------------------------- dbias ----
 // dbias[h, q, key] += sum over the batch rows b2 = slice, slice + NS, ... of dS[b2, h, q, key].
 template <typename T, int DP>
-__global__ __launch_bounds__(256) void attention_bwd_dbias_kernel(
+__global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 4 : 1) void attention_bwd_dbias_kernel(
     float* __restrict__ dbias, const T* __restrict__ q_qk, const T* __restrict__ k_qk, const T* __restrict__ v_qk,
     const T* __restrict__ bias_t, const float* __restrict__ keybias, const T* __restrict__ do_qk,
     const float* __restrict__ lse, const float* __restrict__ dsum, int B2, int H, int Nq, int Nk, int NS,
@@ -375,7 +439,7 @@ __global__ __launch_bounds__(256) void attention_bwd_dbias_kernel(
 #pragma unroll
     for (int i = 0; i < NF; ++i) ident[i] = identity_frag<T>(i, l32, half);
     Tile16<T> bc;
-    bc.load(bias_t + ((((long)h * QT + qt) * (KT + bias_pad) + kt) << 10) + lane * 16);
+    bc.load_rows(bias_t + ((((long)h * QT + qt) * (KT + bias_pad) + kt) << 10) + l32 * 16, half);
     f32x16 sb;                                                  // the bias tile in accumulator order, once
 #pragma unroll
     for (int v = 0; v < 16; ++v) sb[v] = 0.0f;
@@ -385,36 +449,52 @@ __global__ __launch_bounds__(256) void attention_bwd_dbias_kernel(
     f32x16 acc;
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
-    for (int b2 = slice; b2 < B2; b2 += NS) {
+    // as in the dq kernel: each operand is requested for the next batch row once its registers are free
+    Tile16<T> qc[DP], doc[DP], kf[DP], vf[DP];
+    f32x4 L4[4], D4[4];
+    float kb;
+    auto load_rows = [&](int b2) {
         const long bh = (long)b2 * H + h;
-        const float kb = keybias[(long)b2 * KT * 32 + key];
-        f32x16 s = sb, dp;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) dp[v] = 0.0f;
-#pragma unroll
-        for (int p = 0; p < DP; ++p) {
-            Tile16<T> qc, doc, kf, vf;
-            qc.load(q_qk + p * part_q + ((bh * QT + qt) << 10) + lane * 16);
-            doc.load(do_qk + p * part_q + ((bh * QT + qt) << 10) + lane * 16);
-            kf.load(k_qk + p * part_k + ((bh * KT + kt) << 10) + lane * 16);
-            vf.load(v_qk + p * part_k + ((bh * KT + kt) << 10) + lane * 16);
-#pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(s, qc.frag(i), kf.frag(i));
-#pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(dp, doc.frag(i), vf.frag(i));
-        }
+        kb = keybias[(long)b2 * KT * 32 + key];
         const float* lp = lse + (bh * QT + qt) * 32 + 4 * half;
         const float* dpz = dsum + (bh * QT + qt) * 32 + 4 * half;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const f32x4 L4 = *reinterpret_cast<const f32x4*>(lp + 8 * g);
-            const f32x4 D4 = *reinterpret_cast<const f32x4*>(dpz + 8 * g);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int v = 4 * g + e;
-                acc[v] += fast_exp2(s[v] + kb - L4[e]) * (dp[v] - D4[e]);
-            }
+            L4[g] = *reinterpret_cast<const f32x4*>(lp + 8 * g);
+            D4[g] = *reinterpret_cast<const f32x4*>(dpz + 8 * g);
         }
+    };
+    auto load_scores = [&](int b2) {
+        const long bh = (long)b2 * H + h;
+#pragma unroll
+        for (int p = 0; p < DP; ++p) {
+            qc[p].load_rows(q_qk + p * part_q + ((bh * QT + qt) << 10) + l32 * 16, half);
+            kf[p].load_rows(k_qk + p * part_k + ((bh * KT + kt) << 10) + l32 * 16, half);
+            doc[p].load_rows(do_qk + p * part_q + ((bh * QT + qt) << 10) + l32 * 16, half);
+            vf[p].load_rows(v_qk + p * part_k + ((bh * KT + kt) << 10) + l32 * 16, half);
+        }
+    };
+    load_rows(slice);                                          // slice < NS <= B2
+    load_scores(slice);
+    for (int b2 = slice; b2 < B2; b2 += NS) {
+        const int next = b2 + NS < B2 ? b2 + NS : b2;
+        f32x16 s, dp;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            s[v] = sb[v] + (kb - L4[v >> 2][v & 3]);
+            dp[v] = -D4[v >> 2][v & 3];
+        }
+        load_rows(next);
+#pragma unroll
+        for (int p = 0; p < DP; ++p) {
+#pragma unroll
+            for (int i = 0; i < NF; ++i) MM::mma(s, qc[p].frag(i), kf[p].frag(i));
+#pragma unroll
+            for (int i = 0; i < NF; ++i) MM::mma(dp, doc[p].frag(i), vf[p].frag(i));
+        }
+        load_scores(next);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[v] += fast_exp2(s[v]) * dp[v];
     }
     if (key < Nk) {
 #pragma unroll

@@ -6,6 +6,8 @@
 // xor-shuffles inside the lane group; all arithmetic is fp32.
 #include "ffk_common.h"
 #include <stdlib.h>
+#include <initializer_list>
+#include <type_traits>
 
 thread_local char ffk_err_buf[512] = "";
 
@@ -52,6 +54,46 @@ static bool row_geom(long nvec, RowGeom* g) {
     return true;
 }
 
+// Rows that 16-byte vectors cannot cut (an odd length puts every row at another offset) keep the same shape with accesses of
+// two elements or one: a row is read once, all of a lane's accesses in flight together, and stays in registers.
+#define FFK_ROW_GEOMETRIES_NARROW(X) X(16, 2) X(16, 4) X(32, 4) X(64, 4) X(64, 8) X(64, 16)
+static bool row_geom_narrow(long nacc, RowGeom* g) {
+    int lpr = 16;
+    while (lpr < 64 && (long)lpr * 4 < nacc) lpr <<= 1;
+    const long per = (nacc + lpr - 1) / lpr;
+    if (per > 16) return false;
+    g->lpr = lpr;
+    g->vpl = per <= 2 && lpr == 16 ? 2 : per <= 4 ? 4 : per <= 8 ? 8 : 16;
+    return true;
+}
+
+// Two elements or one, streamed (non-temporal) or cached; a full vector goes through ld16 / st16.
+template <typename T, int VW> struct RowAcc {
+    struct alignas(VW * sizeof(T)) V {
+        T e[VW];
+    };
+    typedef typename std::conditional<VW * sizeof(T) == 2, uint16_t,
+                                      typename std::conditional<VW * sizeof(T) == 4, uint32_t, u32x2>::type>::type Raw;
+    static __device__ __forceinline__ V ld(const T* p) { return __builtin_bit_cast(V, *reinterpret_cast<const Raw*>(p)); }
+    static __device__ __forceinline__ V ld_nt(const T* p) { return ld(p); }   // a line is shared by several accesses
+    static __device__ __forceinline__ void st_nt(T* p, const V& v) { *reinterpret_cast<Raw*>(p) = __builtin_bit_cast(Raw, v); }
+};
+template <typename T> struct RowAccVec {
+    typedef Vec16<T> V;
+    static __device__ __forceinline__ V ld(const T* p) { return ld16(p); }
+    static __device__ __forceinline__ V ld_nt(const T* p) { return ld16_nt(p); }
+    static __device__ __forceinline__ void st_nt(T* p, const V& v) { st16_nt(p, v); }
+};
+template <> struct RowAcc<float, 4> : RowAccVec<float> {};
+template <> struct RowAcc<bf16_t, 8> : RowAccVec<bf16_t> {};
+template <> struct RowAcc<f16_t, 8> : RowAccVec<f16_t> {};
+
+static bool row_aligned(size_t bytes, std::initializer_list<const void*> ps) {
+    for (const void* q : ps)
+        if (reinterpret_cast<uintptr_t>(q) % bytes) return false;
+    return true;
+}
+
 static int row_grid(long rows, int lpr) {
     long rows_per_block = (long)WAVES_PER_BLOCK * (64 / lpr);
     long blocks = (rows + rows_per_block - 1) / rows_per_block;
@@ -84,45 +126,45 @@ template <> __device__ __forceinline__ const float* sm_ones_row<float>() { retur
 template <> __device__ __forceinline__ const bf16_t* sm_ones_row<bf16_t>() { return reinterpret_cast<const bf16_t*>(sm_ones_bf16.w); }
 template <> __device__ __forceinline__ const f16_t* sm_ones_row<f16_t>() { return reinterpret_cast<const f16_t*>(sm_ones_f16.w); }
 // RAGGED = false: the row is exactly LPR * VPL vectors, every vector offset is an immediate (one address per lane).
-template <typename T, int LPR, int VPL, bool RAGGED>
+template <typename T, int VW, int LPR, int VPL, bool RAGGED>
 __global__ __launch_bounds__(64 * SM_WAVES) void softmax_vec_kernel(T* out, const T* x,   // out may alias x
                                                                   const T* __restrict__ mask,
                                                                   const T* __restrict__ bias, unsigned rows, int cols,
                                                                   unsigned hq) {
-    constexpr int VEC = DT<T>::VEC;
+    typedef RowAcc<T, VW> A;
     constexpr int RPW = 64 / LPR;
     constexpr bool F32 = sizeof(T) == 4;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int sub = lane / LPR;
     const int j = lane % LPR;
-    const int nvec = RAGGED ? cols / VEC : LPR * VPL;
-    const int rowlen = RAGGED ? cols : LPR * VPL * VEC;
+    const int nvec = RAGGED ? cols / VW : LPR * VPL;
+    const int rowlen = RAGGED ? cols : LPR * VPL * VW;
     const unsigned stride = gridDim.x * SM_WAVES * RPW;
     for (unsigned base = (blockIdx.x * SM_WAVES + wave) * RPW; base < rows; base += stride) {
         const unsigned row = base + sub;
         const bool valid = row < rows;
         const unsigned rc = valid ? row : rows - 1;
         const unsigned b2 = rc / hq;                             // 32-bit: rows < 2^31 is checked by the entry point
-        const T* xr = x + (long)rc * rowlen + j * VEC;
-        const T* br = (bias ? bias + (long)(rc - b2 * hq) * rowlen : reinterpret_cast<const T*>(sm_zero_row)) + j * VEC;
-        const T* mr = (mask ? mask + (long)b2 * rowlen : sm_ones_row<T>()) + j * VEC;
-        Vec16<T> xv[VPL], bv[VPL], mv[VPL];
+        const T* xr = x + (long)rc * rowlen + j * VW;
+        const T* br = (bias ? bias + (long)(rc - b2 * hq) * rowlen : reinterpret_cast<const T*>(sm_zero_row)) + j * VW;
+        const T* mr = (mask ? mask + (long)b2 * rowlen : sm_ones_row<T>()) + j * VW;
+        typename A::V xv[VPL], bv[VPL], mv[VPL];
 #pragma unroll
         for (int i = 0; i < VPL; ++i) {
-            int vo = i * LPR * VEC;
-            if (RAGGED) vo = j + i * LPR < nvec ? vo : (nvec - 1 - j) * VEC;   // clamped: the copy is ignored below
-            xv[i] = ld16_nt(xr + vo);
-            bv[i] = ld16(br + vo);
-            mv[i] = ld16(mr + vo);
+            int vo = i * LPR * VW;
+            if (RAGGED) vo = j + i * LPR < nvec ? vo : (nvec - 1 - j) * VW;   // clamped: the copy is ignored below
+            xv[i] = A::ld_nt(xr + vo);
+            bv[i] = A::ld(br + vo);
+            mv[i] = A::ld(mr + vo);
         }
-        float v[VPL][VEC];
+        float v[VPL][VW];
         float mx = -INFINITY;
 #pragma unroll
         for (int i = 0; i < VPL; ++i) {
             const bool in = !RAGGED || j + i * LPR < nvec;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) {
+            for (int e = 0; e < VW; ++e) {
                 float f = DT<T>::to_f(xv[i].e[e]) + DT<T>::to_f(bv[i].e[e]);
                 if (DT<T>::to_f(mv[i].e[e]) == 0.0f) f = MASK_FILL;
                 if (RAGGED) f = in ? f : -INFINITY;
@@ -136,7 +178,7 @@ __global__ __launch_bounds__(64 * SM_WAVES) void softmax_vec_kernel(T* out, cons
 #pragma unroll
             for (int i = 0; i < VPL; ++i)
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) {
+                for (int e = 0; e < VW; ++e) {
                     v[i][e] = expf(v[i][e] - mx);
                     sum += v[i][e];
                 }
@@ -145,20 +187,20 @@ __global__ __launch_bounds__(64 * SM_WAVES) void softmax_vec_kernel(T* out, cons
 #pragma unroll
             for (int i = 0; i < VPL; ++i)
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) {
+                for (int e = 0; e < VW; ++e) {
                     v[i][e] = fast_exp2(__builtin_fmaf(v[i][e], 1.4426950408889634f, -mxl));
                     sum += v[i][e];
                 }
         }
         sum = group_sum(sum, LPR);
         const float inv = F32 ? 1.0f / sum : fast_rcp(sum);
-        T* orow = out + (long)rc * rowlen + j * VEC;
+        T* orow = out + (long)rc * rowlen + j * VW;
 #pragma unroll
         for (int i = 0; i < VPL; ++i) {
-            Vec16<T> ov;
+            typename A::V ov;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) ov.e[e] = DT<T>::from_f(v[i][e] * inv);
-            if (valid && (!RAGGED || j + i * LPR < nvec)) st16_nt(orow + i * LPR * VEC, ov);
+            for (int e = 0; e < VW; ++e) ov.e[e] = DT<T>::from_f(v[i][e] * inv);
+            if (valid && (!RAGGED || j + i * LPR < nvec)) A::st_nt(orow + i * LPR * VW, ov);
         }
     }
 }
@@ -193,6 +235,105 @@ __global__ __launch_bounds__(BLOCK) void softmax_generic_kernel(T* out, const T*
     }
 }
 
+// Backward: dx = (dy - sum y dy) y over rows of up to LPR * VPL accesses, each tensor read once and dx written once; three
+// passes of 134 MB at [1, 128, 8, 256, 256] bf16 bound it (one wave per row with two-byte loads in two walks: 152 us).
+// BIAS: the gradient of a bias shared by the B2 batch rows is dx summed over them.  A workgroup then owns 64 / LPR rows of
+// one (b1, h, q) range, its waves take the batch rows in turn (blockIdx.y: slices of them) and keep fp32 sums of dx in
+// registers, folded through LDS at the end: reading dx again for the sum was a fourth pass (25 us of a library reduction).
+// One slice writes the bias gradient itself, several leave fp32 parts for softmax_dbias_kernel.
+template <typename T, int VW, int LPR, int VPL, bool BIAS>
+__global__ __launch_bounds__(64 * SM_WAVES) void softmax_bwd_vec_kernel(T* __restrict__ dx, T* __restrict__ dbias,
+                                                                      float* __restrict__ part, const T* __restrict__ dy,
+                                                                      const T* __restrict__ y, unsigned rows, int cols,
+                                                                      unsigned B2, unsigned hq) {
+    typedef RowAcc<T, VW> A;
+    constexpr int RPW = 64 / LPR;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int sub = lane / LPR, j = lane % LPR;
+    const int nacc = cols / VW;
+    float acc[VPL][VW];
+    auto step = [&](unsigned row, bool valid) {
+        const long o = (long)row * cols + j * VW;
+        typename A::V gv[VPL], yv[VPL];
+#pragma unroll
+        for (int i = 0; i < VPL; ++i) {
+            const int vo = j + i * LPR < nacc ? i * LPR * VW : (nacc - 1 - j) * VW;      // clamped: ignored below
+            gv[i] = A::ld_nt(dy + o + vo);
+            yv[i] = A::ld_nt(y + o + vo);
+        }
+        float dot = 0.0f;
+#pragma unroll
+        for (int i = 0; i < VPL; ++i) {
+            float d = 0.0f;
+#pragma unroll
+            for (int e = 0; e < VW; ++e) d += DT<T>::to_f(yv[i].e[e]) * DT<T>::to_f(gv[i].e[e]);
+            dot += j + i * LPR < nacc ? d : 0.0f;
+        }
+        dot = group_sum(dot, LPR);
+#pragma unroll
+        for (int i = 0; i < VPL; ++i) {
+            typename A::V ov;
+#pragma unroll
+            for (int e = 0; e < VW; ++e) {
+                const float v = (DT<T>::to_f(gv[i].e[e]) - dot) * DT<T>::to_f(yv[i].e[e]);
+                if (BIAS) acc[i][e] += v;
+                ov.e[e] = DT<T>::from_f(v);
+            }
+            if (valid && j + i * LPR < nacc) A::st_nt(dx + o + i * LPR * VW, ov);
+        }
+    };
+    if constexpr (!BIAS) {
+        const unsigned stride = gridDim.x * SM_WAVES * RPW;
+        for (unsigned base = (blockIdx.x * SM_WAVES + wave) * RPW; base < rows; base += stride) {
+            const unsigned row = base + sub;
+            step(row < rows ? row : rows - 1, row < rows);
+        }
+    } else {
+        __shared__ float red[SM_WAVES][64 * VW];
+#pragma unroll
+        for (int i = 0; i < VPL; ++i)
+#pragma unroll
+            for (int e = 0; e < VW; ++e) acc[i][e] = 0.0f;
+        // rows: those of the bias, B1 * hq
+        const unsigned r = blockIdx.x * RPW + sub;
+        const bool valid = r < rows;
+        const unsigned rc = valid ? r : rows - 1, b1 = rc / hq;
+        const unsigned first = b1 * B2 * hq + (rc - b1 * hq);
+        for (unsigned b2 = blockIdx.y * SM_WAVES + wave; b2 < B2; b2 += gridDim.y * SM_WAVES) step(first + b2 * hq, valid);
+#pragma unroll
+        for (int i = 0; i < VPL; ++i) {
+#pragma unroll
+            for (int e = 0; e < VW; ++e) red[wave][lane * VW + e] = acc[i][e];
+            __syncthreads();
+            // wave w folds and writes the lanes' element w (, w + SM_WAVES ...) of this access
+#pragma unroll
+            for (int e = wave; e < VW; e += SM_WAVES) {
+                float t = 0.0f;
+#pragma unroll
+                for (int w = 0; w < SM_WAVES; ++w) t += red[w][lane * VW + e];
+                const int c = (j + i * LPR) * VW + e;
+                if (valid && j + i * LPR < nacc) {
+                    if (gridDim.y == 1) dbias[(long)r * cols + c] = DT<T>::from_f(t);
+                    else part[((long)blockIdx.y * rows + r) * cols + c] = t;
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// The slices' parts of the bias gradient added up.
+template <typename T>
+__global__ __launch_bounds__(BLOCK) void softmax_dbias_kernel(T* __restrict__ dbias, const float* __restrict__ part, long n, int slices) {
+    for (long i = (long)blockIdx.x * BLOCK + threadIdx.x; i < n; i += (long)gridDim.x * BLOCK) {
+        float t = 0.0f;
+#pragma unroll 4
+        for (int s = 0; s < slices; ++s) t += part[s * n + i];
+        dbias[i] = DT<T>::from_f(t);
+    }
+}
+
+// Rows longer than the geometries above: one wave per row, two walks over it.
 template <typename T>
 __global__ __launch_bounds__(BLOCK) void softmax_bwd_kernel(T* dx, const T* dy, const T* y, long rows, int cols) {
     const int lane = threadIdx.x & 63;
@@ -208,6 +349,66 @@ __global__ __launch_bounds__(BLOCK) void softmax_bwd_kernel(T* dx, const T* dy, 
         for (int c = lane; c < cols; c += 64)
             o[c] = DT<T>::from_f((DT<T>::to_f(gr[c]) - dot) * DT<T>::to_f(yr[c]));
     }
+}
+
+// dbias of such rows: dx read again and summed over the batch rows (dx[b1][b2][n] -> dbias[b1][n], n = hq * cols).
+template <typename T>
+__global__ __launch_bounds__(BLOCK) void softmax_dbias_long_kernel(T* __restrict__ dbias, const T* __restrict__ dx, long total, long n,
+                                                                 long B2) {
+    for (long i = (long)blockIdx.x * BLOCK + threadIdx.x; i < total; i += (long)gridDim.x * BLOCK) {
+        const long b1 = i / n;
+        const T* p = dx + b1 * B2 * n + (i - b1 * n);
+        float t = 0.0f;
+#pragma unroll 8
+        for (long b2 = 0; b2 < B2; ++b2) t += DT<T>::to_f(p[b2 * n]);
+        dbias[i] = DT<T>::from_f(t);
+    }
+}
+
+// B1 == 0: no bias, `rows` rows; otherwise dx is [B1, B2, hq, cols] and dbias [B1, hq, cols].
+template <typename T>
+int softmax_bwd_launch(T* dx, T* dbias, float* part, int slices, const T* dy, const T* y, long B1, long B2, long hq, long rows,
+                       long cols, hipStream_t st) {
+    constexpr int VEC = DT<T>::VEC;
+    RowGeom g;
+    const long brows = B1 * hq;
+    const bool small = rows < (1L << 31) - (1L << 24);
+    auto grid = [&](int lpr) {
+        const long rpw = 64 / lpr;
+        if (B1) return dim3((unsigned)((brows + rpw - 1) / rpw), (unsigned)slices);
+        const long need = (rows + SM_WAVES * rpw - 1) / (SM_WAVES * rpw);
+        return dim3((unsigned)(need < 256L * 8 ? need : 256L * 8));
+    };
+    bool done = false;
+#define FFK_SMB_RUN(VW, L, V)                                                                                                \
+    if (!done && g.lpr == L && g.vpl == V) {                                                                                 \
+        if (B1) softmax_bwd_vec_kernel<T, VW, L, V, true><<<grid(L), 64 * SM_WAVES, 0, st>>>(dx, dbias, part, dy, y, (unsigned)brows, (int)cols, (unsigned)B2, (unsigned)hq); \
+        else softmax_bwd_vec_kernel<T, VW, L, V, false><<<grid(L), 64 * SM_WAVES, 0, st>>>(dx, dbias, part, dy, y, (unsigned)rows, (int)cols, 1u, 1u); \
+        done = true;                                                                                                         \
+    }
+#define FFK_SMB_CASE(L, V) FFK_SMB_RUN(VEC, L, V)
+#define FFK_SMB_CASE2(L, V) FFK_SMB_RUN(2, L, V)
+#define FFK_SMB_CASE1(L, V) FFK_SMB_RUN(1, L, V)
+    if (small && cols % VEC == 0 && row_aligned(16, {dx, dy, y}) && row_geom(cols / VEC, &g)) {
+        FFK_ROW_GEOMETRIES(FFK_SMB_CASE)
+    } else if (small && cols % 2 == 0 && row_aligned(2 * sizeof(T), {dx, dy, y}) && row_geom_narrow(cols / 2, &g)) {
+        FFK_ROW_GEOMETRIES_NARROW(FFK_SMB_CASE2)
+    } else if (small && row_geom_narrow(cols, &g)) {
+        FFK_ROW_GEOMETRIES_NARROW(FFK_SMB_CASE1)
+    }
+#undef FFK_SMB_CASE
+#undef FFK_SMB_CASE2
+#undef FFK_SMB_CASE1
+#undef FFK_SMB_RUN
+    const char* what = B1 ? "ffk_softmax_bwd_bias" : "ffk_softmax_bwd";
+    if (!done) softmax_bwd_kernel<T><<<row_grid(rows, 64), BLOCK, 0, st>>>(dx, dy, y, rows, (int)cols);
+    int rc = ffk_check_launch(what);
+    if (rc != FFK_OK || !B1 || (done && slices == 1)) return rc;
+    const long n = brows * cols, blocks = (n + BLOCK - 1) / BLOCK;
+    const unsigned fgrid = (unsigned)(blocks < 256L * 16 ? blocks : 256L * 16);
+    if (done) softmax_dbias_kernel<T><<<fgrid, BLOCK, 0, st>>>(dbias, part, n, slices);
+    else softmax_dbias_long_kernel<T><<<fgrid, BLOCK, 0, st>>>(dbias, dx, n, hq * cols, B2);
+    return ffk_check_launch(what);
 }
 
 template <typename T>
@@ -226,15 +427,38 @@ int softmax_launch(T* out, const T* x, const T* mask, const T* bias, long rows, 
 #define FFK_SM_CASE(L, V)                                                                                         \
     if (g.lpr == L && g.vpl == V) {                                                                               \
         if (cols == (long)L * V * VEC)                                                                            \
-            softmax_vec_kernel<T, L, V, false><<<grid, 64 * SM_WAVES, 0, st>>>(out, x, mask, bias, (unsigned)rows, (int)cols, (unsigned)hq); \
+            softmax_vec_kernel<T, VEC, L, V, false><<<grid, 64 * SM_WAVES, 0, st>>>(out, x, mask, bias, (unsigned)rows, (int)cols, (unsigned)hq); \
         else                                                                                                      \
-            softmax_vec_kernel<T, L, V, true><<<grid, 64 * SM_WAVES, 0, st>>>(out, x, mask, bias, (unsigned)rows, (int)cols, (unsigned)hq); \
+            softmax_vec_kernel<T, VEC, L, V, true><<<grid, 64 * SM_WAVES, 0, st>>>(out, x, mask, bias, (unsigned)rows, (int)cols, (unsigned)hq); \
         return ffk_check_launch("ffk_softmax_fwd");                                                               \
     }
         FFK_ROW_GEOMETRIES(FFK_SM_CASE)
 #undef FFK_SM_CASE
         return ffk_fail(FFK_ERR_UNSUPPORTED, "ffk_softmax_fwd: no kernel for the row geometry (%d lanes, %d vectors)", g.lpr, g.vpl);
-    } else {
+    }
+    // rows of another length or alignment: accesses of two elements, or one, of the same kernel (one wave per row with two-byte
+    // loads walked a row three times and exponentiated it twice)
+    auto grid = [&](int lpr) {
+        const long rows_per_block = (long)SM_WAVES * (64 / lpr), need = (rows + rows_per_block - 1) / rows_per_block;
+        return dim3((unsigned)(need < 256L * 8 ? need : 256L * 8));
+    };
+    const bool small = rows < (1L << 31) - (1L << 24);
+#define FFK_SM_NARROW(VW, L, V)                                                                                           \
+    if (g.lpr == L && g.vpl == V) {                                                                                       \
+        softmax_vec_kernel<T, VW, L, V, true><<<grid(L), 64 * SM_WAVES, 0, st>>>(out, x, mask, bias, (unsigned)rows, (int)cols, (unsigned)hq); \
+        return ffk_check_launch("ffk_softmax_fwd");                                                                       \
+    }
+#define FFK_SM_CASE2(L, V) FFK_SM_NARROW(2, L, V)
+#define FFK_SM_CASE1(L, V) FFK_SM_NARROW(1, L, V)
+    if (small && cols % 2 == 0 && row_aligned(2 * sizeof(T), {out, x, mask, bias}) && row_geom_narrow(cols / 2, &g)) {
+        FFK_ROW_GEOMETRIES_NARROW(FFK_SM_CASE2)
+    } else if (small && row_geom_narrow(cols, &g)) {
+        FFK_ROW_GEOMETRIES_NARROW(FFK_SM_CASE1)
+    }
+#undef FFK_SM_CASE1
+#undef FFK_SM_CASE2
+#undef FFK_SM_NARROW
+    {
         dim3 grid(row_grid(rows, 64));
         softmax_generic_kernel<T><<<grid, BLOCK, 0, st>>>(out, x, mask, bias, rows, (int)cols, hq);
     }
@@ -732,14 +956,27 @@ extern "C" int ffk_softmax_bwd(void* dx, const void* dy, const void* y, int64_t 
     FFK_REQUIRE(rows > 0 && cols > 0 && cols < (1L << 30), FFK_ERR_SHAPE, "ffk_softmax_bwd: bad shape [%ld,%ld]",
                 (long)rows, (long)cols);
     hipStream_t st = (hipStream_t)stream;
-    dim3 grid(row_grid(rows, 64));
     switch (dtype) {
-        case FFK_F32: softmax_bwd_kernel<float><<<grid, BLOCK, 0, st>>>((float*)dx, (const float*)dy, (const float*)y, rows, (int)cols); break;
-        case FFK_BF16: softmax_bwd_kernel<bf16_t><<<grid, BLOCK, 0, st>>>((bf16_t*)dx, (const bf16_t*)dy, (const bf16_t*)y, rows, (int)cols); break;
-        case FFK_F16: softmax_bwd_kernel<f16_t><<<grid, BLOCK, 0, st>>>((f16_t*)dx, (const f16_t*)dy, (const f16_t*)y, rows, (int)cols); break;
+        case FFK_F32: return softmax_bwd_launch<float>((float*)dx, nullptr, nullptr, 1, (const float*)dy, (const float*)y, 0, 0, 0, rows, cols, st);
+        case FFK_BF16: return softmax_bwd_launch<bf16_t>((bf16_t*)dx, nullptr, nullptr, 1, (const bf16_t*)dy, (const bf16_t*)y, 0, 0, 0, rows, cols, st);
+        case FFK_F16: return softmax_bwd_launch<f16_t>((f16_t*)dx, nullptr, nullptr, 1, (const f16_t*)dy, (const f16_t*)y, 0, 0, 0, rows, cols, st);
         default: return ffk_fail(FFK_ERR_DTYPE, "ffk_softmax_bwd: unsupported dtype tag %d", dtype);
     }
-    return ffk_check_launch("ffk_softmax_bwd");
+}
+
+extern "C" int ffk_softmax_bwd_bias(void* dx, void* dbias, float* ws, int64_t slices, const void* dy, const void* y, int64_t B1,
+                                    int64_t B2, int64_t HQ, int64_t cols, int dtype, void* stream) {
+    FFK_REQUIRE(dx && dbias && dy && y && (ws || slices == 1), FFK_ERR_NULL, "ffk_softmax_bwd_bias: null pointer");
+    FFK_REQUIRE(B1 > 0 && B2 > 0 && HQ > 0 && cols > 0 && cols < (1L << 30) && slices > 0 && slices < 65536, FFK_ERR_SHAPE,
+                "ffk_softmax_bwd_bias: bad shape [%ld,%ld,%ld,%ld], %ld slices", (long)B1, (long)B2, (long)HQ, (long)cols, (long)slices);
+    hipStream_t st = (hipStream_t)stream;
+    const long rows = B1 * B2 * HQ;
+    switch (dtype) {
+        case FFK_F32: return softmax_bwd_launch<float>((float*)dx, (float*)dbias, ws, (int)slices, (const float*)dy, (const float*)y, B1, B2, HQ, rows, cols, st);
+        case FFK_BF16: return softmax_bwd_launch<bf16_t>((bf16_t*)dx, (bf16_t*)dbias, ws, (int)slices, (const bf16_t*)dy, (const bf16_t*)y, B1, B2, HQ, rows, cols, st);
+        case FFK_F16: return softmax_bwd_launch<f16_t>((f16_t*)dx, (f16_t*)dbias, ws, (int)slices, (const f16_t*)dy, (const f16_t*)y, B1, B2, HQ, rows, cols, st);
+        default: return ffk_fail(FFK_ERR_DTYPE, "ffk_softmax_bwd_bias: unsupported dtype tag %d", dtype);
+    }
 }
 
 extern "C" int ffk_layernorm_fwd(void* out, float* mean, float* rstd, const void* x, const void* gamma,

@@ -38,51 +38,76 @@ __global__ __launch_bounds__(TR_THREADS) void ln_bwd_rows_kernel(T* dx, T* __res
     if (xn) unpack<T>(ld16(beta + c), b);
 #pragma unroll
     for (int e = 0; e < V; ++e) dg[e] = db[e] = 0.0f;
-    for (long r0 = (long)blockIdx.x * RPB; r0 < rows; r0 += (long)gridDim.x * RPB) {
-        const long r = r0 + tid / LPR;
-        const bool ok = r < rows;
-        const long o = (ok ? r : rows - 1) * C + c;
-        float xv[V], dv[V], rv[V];
-        const Vec16<T> vx = ld16(x + o), vd = ld16(dy + o);
-        Vec16<T> vr{};
-        if (resid) vr = ld16(resid + o);
-        unpack<T>(vx, xv);
-        unpack<T>(vd, dv);
-        unpack<T>(vr, rv);
-        float s = 0.0f;
+    // RU rows per thread at a time: their loads go out together, and the reductions - a chain of two, the statistics of the
+    // gradient need only the centred row - run side by side
+    constexpr int RU = 2;
+    for (long r0 = (long)blockIdx.x * RPB; r0 < rows; r0 += (long)gridDim.x * RPB * RU) {
+        Vec16<T> vx[RU], vd[RU], vr[RU];
+        bool ok[RU];
+        long o[RU];
 #pragma unroll
-        for (int e = 0; e < V; ++e) s += xv[e];
-        const float mu = group_sum(s, LPR) * (1.0f / C);
-        float q = 0.0f;
-#pragma unroll
-        for (int e = 0; e < V; ++e) {
-            xv[e] -= mu;
-            q += xv[e] * xv[e];
+        for (int u = 0; u < RU; ++u) {
+            const long r = r0 + (long)u * gridDim.x * RPB + tid / LPR;
+            ok[u] = r < rows;
+            o[u] = (ok[u] ? r : rows - 1) * C + c;
+            vx[u] = ld16(x + o[u]);
+            vd[u] = ld16(dy + o[u]);
+            vr[u] = Vec16<T>{};
+            if (resid) vr[u] = ld16(resid + o[u]);
         }
-        const float rs = rsqrtf(group_sum(q, LPR) * (1.0f / C) + eps);
-        float s1 = 0.0f, s2 = 0.0f;
+        float mu[RU], rs[RU], s1[RU], s2[RU];
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
-            xv[e] *= rs;                                        // normalised
-            const float t = dv[e] * g[e];
-            s1 += t;
-            s2 += t * xv[e];
+        for (int u = 0; u < RU; ++u) {
+            float xv[V], s = 0.0f;
+            unpack<T>(vx[u], xv);
+#pragma unroll
+            for (int e = 0; e < V; ++e) s += xv[e];
+            mu[u] = s;
         }
-        s1 = group_sum(s1, LPR) * (1.0f / C);
-        s2 = group_sum(s2, LPR) * (1.0f / C);
-        float out[V], xo[V];
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
-            out[e] = rv[e] + rs * (dv[e] * g[e] - s1 - xv[e] * s2);
-            xo[e] = xv[e] * g[e] + (xn ? b[e] : 0.0f);
-            if (ok) {
-                dg[e] += dv[e] * xv[e];
-                db[e] += dv[e];
+        for (int u = 0; u < RU; ++u) mu[u] = group_sum(mu[u], LPR) * (1.0f / C);
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            float xv[V], dv[V], q = 0.0f, t1 = 0.0f, t2 = 0.0f;
+            unpack<T>(vx[u], xv);
+            unpack<T>(vd[u], dv);
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                const float xc = xv[e] - mu[u], t = dv[e] * g[e];
+                q += xc * xc;
+                t1 += t;
+                t2 += t * xc;
             }
+            rs[u] = q;
+            s1[u] = t1;
+            s2[u] = t2;
         }
-        if (ok) {
-            st16(dx + o, pack<T>(out));
-            if (xn) st16(xn + o, pack<T>(xo));
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            rs[u] = rsqrtf(group_sum(rs[u], LPR) * (1.0f / C) + eps);
+            s1[u] = group_sum(s1[u], LPR) * (1.0f / C);
+            s2[u] = group_sum(s2[u], LPR) * rs[u] * (1.0f / C);
+        }
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            float xv[V], dv[V], rv[V], out[V], xo[V];
+            unpack<T>(vx[u], xv);
+            unpack<T>(vd[u], dv);
+            unpack<T>(vr[u], rv);
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                const float xh = (xv[e] - mu[u]) * rs[u];
+                out[e] = rv[e] + rs[u] * (dv[e] * g[e] - s1[u] - xh * s2[u]);
+                xo[e] = xh * g[e] + (xn ? b[e] : 0.0f);
+                if (ok[u]) {
+                    dg[e] += dv[e] * xh;
+                    db[e] += dv[e];
+                }
+            }
+            if (ok[u]) {
+                st16(dx + o[u], pack<T>(out));
+                if (xn) st16(xn + o[u], pack<T>(xo));
+            }
         }
     }
     // lanes of a wave that own the same columns: LPR .. 64 apart
@@ -108,7 +133,7 @@ __global__ __launch_bounds__(TR_THREADS) void ln_bwd_rows_kernel(T* dx, T* __res
 }
 
 // dgamma[c] / dbeta[c] = sum of the partial rows: a workgroup per 16 columns, 64 groups of four lanes over the partial rows (a
-// workgroup per 32 columns with eight groups walked 128 rows one load after the other: 34 us at C = 256, now ... us)
+// workgroup per 32 columns with eight groups walked 128 rows one load after the other: 34 us at C = 256, now 4.6)
 template <typename T>
 __global__ __launch_bounds__(256) void ln_finish_kernel(T* __restrict__ dgamma, T* __restrict__ dbeta, const float* __restrict__ part,
                                                         int blocks, int C) {

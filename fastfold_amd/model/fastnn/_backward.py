@@ -265,7 +265,7 @@ def attention_backward(owner, att, ln_mod, x, dy, dx, g, out_bias, *, B2, N, a_m
     dsum = alloc((B2 * H * N,), torch.float32, dev)
     at = cat.data_ptr()
     _lib.att_gate_bwd(go, at + 3 * HC * es, do_t, do_v, dsum, dgo, gpre, gb, o, B2=B2, N=N, H=H, g_ld=HC, dg_ld=Kd, dtype=dt)
-    parts = max(1, min((8192 + H * NT * NT - 1) // (H * NT * NT), (B2 + 7) // 8)) if bias_t is not None else 0
+    parts = max(1, min((4096 + H * NT * NT - 1) // (H * NT * NT), (B2 + 7) // 8)) if bias_t is not None else 0
     dbias = alloc((parts, H, N, N), torch.float32, dev) if parts else None
     _lib.attention_bwd_rows(at, at + HC * es, at + 2 * HC * es, dbias, lse, dsum, tiles["q_t"], tiles["q_v"], tiles["k_t"],
                             tiles["k_v"], tiles["v_t"], bias_t, kb, do_t, do_v, B2=B2, H=H, N=N, s_b=N * Kd, s_h=32, s_n=Kd,

@@ -20,7 +20,7 @@ from .... import _lib
 from . import layouts
 
 
-def _attention_core(q, k, v, mask=None, bias=None):
+def _check(q, k, v, mask, bias):
     for t in (q, k, v, mask, bias):          # any strides: the operands are re-tiled as they lie
         if t is not None and not t.is_cuda:
             raise RuntimeError("fastfold_amd: tensor must be a CUDA/HIP tensor (got %s)" % t.device)
@@ -37,44 +37,110 @@ def _attention_core(q, k, v, mask=None, bias=None):
         raise RuntimeError("fused_attention_core: mask must be [b1, b2, n], got %s" % (tuple(mask.shape),))
     if bias is not None and tuple(bias.shape) != (b1, h, n, n):
         raise RuntimeError("fused_attention_core: bias must be [b1, h, n, n], got %s" % (tuple(bias.shape),))
-    # zero channels past d add nothing to q.k and give zero output channels, which are dropped at the end
-    dk = max(d, 32)                        # head width the kernel sees
-    out = torch.empty(b1, b2, n, h * dk, dtype=q.dtype, device=q.device)
-    if out.numel() == 0:
-        return out.view(b1, b2, n, h, dk)[..., :d].reshape(b1, b2, n, h * d)
+
+
+def _key_bias(kb, fl, mask, b2, n, dt, dev):
+    mk = mask.to(dt).contiguous() if mask is not None else torch.ones(b2, n, dtype=dt, device=dev)
+    _lib.key_bias(kb, fl, mk, B=b2, N=n, mask_sb=n, mask_sn=1)
+
+
+def _attention_core_wide(q, k, v, mask, bias):
+    """Head dims 64 and 128."""
+    b1, b2, h, n, d = q.shape
+    out = torch.empty(b1, b2, n, h * d, dtype=q.dtype, device=q.device)
     nt = layouts.n_tiles(n)
-    scale = _lib.LOG2E / math.sqrt(d)      # the kernel exponentiates in base 2
     kb = torch.empty(b2, nt * 32, dtype=torch.float32, device=q.device)
     fl = torch.empty(b2, nt, dtype=torch.int32, device=q.device)
     for i in range(b1):
-        mk = mask[i].to(q.dtype).contiguous() if mask is not None else torch.ones(b2, n, dtype=q.dtype, device=q.device)
-        _lib.key_bias(kb, fl, mk, B=b2, N=n, mask_sb=n, mask_sn=1)
+        _key_bias(kb, fl, None if mask is None else mask[i], b2, n, q.dtype, q.device)
         bt = layouts.tile_bias((bias[i].float() * _lib.LOG2E).to(q.dtype)) if bias is not None else None
-        _lib.attention_fwd(out[i].view(b2 * n, h * dk), _lib.tile_pack(q[i], _lib.FFK_TILE_QK, scale),
+        _lib.attention_fwd(out[i].view(b2 * n, h * d), _lib.tile_pack(q[i], _lib.FFK_TILE_QK, _lib.LOG2E / math.sqrt(d)),
                            _lib.tile_pack(k[i], _lib.FFK_TILE_QK), _lib.tile_pack(v[i], _lib.FFK_TILE_V), bt, kb, fl,
-                           None, B2=b2, H=h, Nq=n, Nk=n, D=dk)
-    if d < 32:
-        return out.view(b1, b2, n, h, 32)[..., :d].reshape(b1, b2, n, h * d)
+                           None, B2=b2, H=h, Nq=n, Nk=n, D=d)
     return out
 
 
-def _attention_core_backward(q, k, v, mask, bias, out, dout, need_dbias):
-    """dq, dk, dv (shapes of q, k, v) and dbias ([b1, h, n, n] or None) through ``ffk_attention_bwd``."""
+def _attention_core(q, k, v, mask=None, bias=None, keep=False):
+    """Head dims 8, 16 and 32.  ``keep``: also what the backward pass reads - the q and k tiles, the rows' log-sum-exp, the key
+    bias of the mask and the bias tiles, one set per b1."""
+    b1, b2, h, n, d = q.shape
+    dt, dev = q.dtype, q.device
+    nt = layouts.n_tiles(n)
+    # zero channels past d add nothing to q.k and give zero output channels, which are dropped at the end
+    out = torch.empty(b1, b2, n, h * 32, dtype=dt, device=dev)
+    kept = b1 if keep else 1
+    qk = torch.empty(kept, 2, b2, h, nt, 1024, dtype=dt, device=dev)
+    vt = torch.empty(b2, h, nt, 1024, dtype=dt, device=dev)
+    bt = torch.empty(kept, h, nt, nt, 1024, dtype=dt, device=dev) if bias is not None else None
+    kb = torch.empty(kept, b2, nt * 32, dtype=torch.float32, device=dev)
+    fl = torch.empty(b2, nt, dtype=torch.int32, device=dev)
+    lse = torch.empty(b1, b2 * h * nt * 32, dtype=torch.float32, device=dev) if keep else None
+    q, k, v = (t if t.stride(-1) == 1 else t.contiguous() for t in (q, k, v))
+    for i in range(b1):
+        s = i if keep else 0
+        bi, bscale = None, 1.0
+        if bias is not None:                  # the kernel exponentiates in base 2
+            bi, bscale = ((bias[i].contiguous(), _lib.LOG2E) if bias.dtype == dt
+                          else ((bias[i].float() * _lib.LOG2E).to(dt).contiguous(), 1.0))
+        _key_bias(kb[s], fl, None if mask is None else mask[i], b2, n, dt, dev)
+        _lib.attention_pack([(q[i], _lib.LOG2E / math.sqrt(d), qk[s, 0], None, None, None), (k[i], 1.0, qk[s, 1], None, None, None),
+                             (v[i], 1.0, None, vt, None, None)],
+                            B2=b2, H=h, N=n, D=d, dtype=dt, bias=bi, bias_t=None if bt is None else bt[s], bias_scale=bscale)
+        _lib.attention_fwd_lse(out[i].view(b2 * n, h * 32), None if lse is None else lse[i], qk[s, 0], qk[s, 1], vt,
+                               None if bt is None else bt[s], kb[s], fl, B2=b2, H=h, N=n)
+    if d < 32:
+        out = out.view(b1, b2, n, h, 32)[..., :d].reshape(b1, b2, n, h * d)
+    return (out, qk, kb, bt, lse) if keep else out
+
+
+def _attention_core_backward(qk, v, kb, bt, lse, out, dout, need_dbias):
+    """dq, dk, dv (shape of v) and dbias ([b1, h, n, n] or None) for head dims up to 32, from what the forward pass kept."""
+    b1, b2, h, n, d = v.shape
+    dt, dev = v.dtype, v.device
+    nt = layouts.n_tiles(n)
+    dq, dk, dv = (torch.empty(b1, b2, h, n, 32, dtype=dt, device=dev) for _ in range(3))
+    q_acc, k_acc, v_qk, do_qk, do_acc = torch.empty(5, b2, h, nt, 1024, dtype=dt, device=dev)
+    dsum = torch.empty(b2 * h * nt * 32, dtype=torch.float32, device=dev)
+    parts, dbias = 0, None
+    if need_dbias and bt is not None:
+        # partial sums over slices of the batch rows, at least eight each: the four waves per SIMD that are resident together
+        parts = max(1, min(-(-4096 // (h * nt * nt)), (b2 + 7) // 8))
+        part = torch.empty(parts, h, n, n, dtype=torch.float32, device=dev)
+        dbias = torch.empty(b1, h, n, n, dtype=dt, device=dev)
+    v = v if v.stride(-1) == 1 else v.contiguous()
+    for i in range(b1):
+        do_ = dout[i].view(b2, n, h, d).permute(0, 2, 1, 3)          # [b2, h, n, d] views: re-tiled as they lie
+        o_ = out[i].view(b2, n, h, d).permute(0, 2, 1, 3)
+        _lib.attention_pack([(qk[i, 0], 1.0, None, q_acc, None, None), (qk[i, 1], 1.0, None, k_acc, None, None),
+                             (v[i], 1.0, v_qk, None, None, None), (do_, 1.0, do_qk, do_acc, dsum, o_)],
+                            B2=b2, H=h, N=n, D=d, dtype=dt)
+        _lib.attention_bwd_rows(dq[i], dk[i], dv[i], part if parts else None, lse[i], dsum, qk[i, 0], q_acc, qk[i, 1], k_acc, v_qk,
+                                None if bt is None else bt[i], kb[i], do_qk, do_acc, B2=b2, H=h, N=n, s_b=h * n * 32, s_h=n * 32,
+                                s_n=32, dq_scale=1.0 / math.sqrt(d), dk_scale=1.0 / _lib.LOG2E, dtype=dt, dbias_parts=parts)
+        if parts and h * n * n % 4 == 0:
+            _lib.slice_sum(dbias[i], part, slices=parts, N=1, K=h * n * n, o_map=(1, 0, 0, 1), dtype=dt)
+        elif parts:
+            torch.sum(part, 0, out=dbias[i]) if dt == torch.float32 else dbias[i].copy_(part.sum(0))
+    if d < 32:
+        dq, dk, dv = (t[..., :d] for t in (dq, dk, dv))
+    return dq, dk, dv, dbias
+
+
+def _attention_core_backward_wide(q, k, v, mask, bias, out, dout, need_dbias):
+    """The same for head dims 64 and 128, through ``ffk_attention_bwd``."""
     b1, b2, h, n, d = q.shape
     dt, dev = q.dtype, q.device
     QK, ACC = _lib.FFK_TILE_QK, _lib.FFK_TILE_V
     nt = layouts.n_tiles(n)
-    dk_ = max(d, 32)
     scale = _lib.LOG2E / math.sqrt(d)
-    dq, dk, dv = (torch.empty(b1, b2, h, n, dk_, dtype=dt, device=dev) for _ in range(3))
+    dq, dk, dv = (torch.empty(b1, b2, h, n, d, dtype=dt, device=dev) for _ in range(3))
     dbias = torch.zeros(b1, h, n, n, dtype=torch.float32, device=dev) if (need_dbias and bias is not None) else None
     kb = torch.empty(b2, nt * 32, dtype=torch.float32, device=dev)
     fl = torch.empty(b2, nt, dtype=torch.int32, device=dev)
     lse = torch.empty(b2 * h * nt * 32, dtype=torch.float32, device=dev)
     dsum = torch.empty_like(lse)
     for i in range(b1):
-        mk = mask[i].to(dt).contiguous() if mask is not None else torch.ones(b2, n, dtype=dt, device=dev)
-        _lib.key_bias(kb, fl, mk, B=b2, N=n, mask_sb=n, mask_sn=1)
+        _key_bias(kb, fl, None if mask is None else mask[i], b2, n, dt, dev)
         bt = layouts.tile_bias((bias[i].float() * _lib.LOG2E).to(dt)) if bias is not None else None
         do_ = dout[i].view(b2, n, h, d).permute(0, 2, 1, 3)          # [b2, h, n, d] views: re-tiled as they lie
         o_ = out[i].view(b2, n, h, d).permute(0, 2, 1, 3)
@@ -83,9 +149,7 @@ def _attention_core_backward(q, k, v, mask, bias, out, dout, need_dbias):
                            _lib.tile_pack(k[i], QK), _lib.tile_pack(k[i], ACC), _lib.tile_pack(v[i], QK),
                            bt, kb,
                            _lib.tile_pack(do_, QK), _lib.tile_pack(do_, ACC), _lib.tile_pack(o_, QK),
-                           B2=b2, H=h, Nq=n, Nk=n, D=dk_, dq_scale=1.0 / math.sqrt(d), dk_scale=1.0 / _lib.LOG2E)
-    if d < 32:
-        dq, dk, dv = (t[..., :d] for t in (dq, dk, dv))
+                           B2=b2, H=h, Nq=n, Nk=n, D=d, dq_scale=1.0 / math.sqrt(d), dk_scale=1.0 / _lib.LOG2E)
     return dq, dk, dv, (None if dbias is None else dbias.to(dt))
 
 
@@ -96,16 +160,28 @@ class FusedAttenionCoreFunc(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, mask=None, bias=None):
-        out = _attention_core(q, k, v, mask, bias)
-        if any(t is not None and t.requires_grad for t in (q, k, v, bias)):
-            ctx.save_for_backward(q, k, v, mask, bias, out)
+        _check(q, k, v, mask, bias)
+        grads = any(t is not None and t.requires_grad for t in (q, k, v, bias))
+        b1, b2, h, n, d = q.shape
+        ctx.wide = d > 32
+        if q.numel() == 0:
+            return torch.empty(b1, b2, n, h * d, dtype=q.dtype, device=q.device)
+        if ctx.wide:
+            out = _attention_core_wide(q, k, v, mask, bias)
+            if grads:
+                ctx.save_for_backward(q, k, v, mask, bias, out)
+        elif grads:
+            out, qk, kb, bt, lse = _attention_core(q, k, v, mask, bias, keep=True)
+            ctx.save_for_backward(qk, v, kb, bt, lse, out)
+        else:
+            out = _attention_core(q, k, v, mask, bias)
         return out
 
     @staticmethod
     def backward(ctx, dout):
-        q, k, v, mask, bias, out = ctx.saved_tensors
-        dq, dk, dv, dbias = _attention_core_backward(q, k, v, mask, bias, out.contiguous(), dout.contiguous(),
-                                                     bias is not None and ctx.needs_input_grad[4])
+        back = _attention_core_backward_wide if ctx.wide else _attention_core_backward
+        saved = ctx.saved_tensors
+        dq, dk, dv, dbias = back(*saved[:-1], saved[-1].contiguous(), dout.contiguous(), ctx.needs_input_grad[4])
         return dq, dk, dv, None, dbias
 
 

@@ -61,9 +61,22 @@ class FusedSoftmaxFunc(torch.autograd.Function):
         (output,) = ctx.saved_tensors
         _lib.check_device(grad_output, output)
         grad_input = torch.empty_like(output)
-        _lib.call("ffk_softmax_bwd", _lib.ptr(grad_input), _lib.ptr(grad_output), _lib.ptr(output),
-                  ctx.rows, ctx.cols, _lib.dtype_tag(output.dtype), _lib.stream_ptr())
-        grad_bias = torch.sum(grad_input, dim=1, keepdim=True) if ctx.use_bias else None
+        grad_bias = None
+        if not (ctx.use_bias and ctx.needs_input_grad[2]) or output.numel() == 0:
+            _lib.call("ffk_softmax_bwd", _lib.ptr(grad_input), _lib.ptr(grad_output), _lib.ptr(output),
+                      ctx.rows, ctx.cols, _lib.dtype_tag(output.dtype), _lib.stream_ptr())
+            if ctx.use_bias and ctx.needs_input_grad[2]:
+                grad_bias = torch.sum(grad_input, dim=1, keepdim=True)
+        else:
+            B1, B2, H, Nq, Nk = output.shape
+            rows = B1 * H * Nq
+            grad_bias = torch.empty(B1, 1, H, Nq, Nk, dtype=output.dtype, device=output.device)
+            # a workgroup owns up to eight rows of the bias: batch rows in slices until there are two workgroups per CU,
+            # sixteen batch rows at least (the slices' fp32 sums stay below a tenth of the tensors' bytes)
+            slices = max(1, min(B2 // 16, -(-4096 // rows)))
+            ws = torch.empty(slices * rows * Nk, dtype=torch.float32, device=output.device) if slices > 1 else None
+            _lib.call("ffk_softmax_bwd_bias", _lib.ptr(grad_input), _lib.ptr(grad_bias), _lib.ptr(ws), slices,
+                      _lib.ptr(grad_output), _lib.ptr(output), B1, B2, H * Nq, Nk, _lib.dtype_tag(output.dtype), _lib.stream_ptr())
         return grad_input, None, grad_bias
 
 

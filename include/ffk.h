@@ -60,6 +60,13 @@ int ffk_softmax_fwd(void* out, const void* x, const void* mask, const void* bias
 int ffk_softmax_bwd(void* dx, const void* dy, const void* y, int64_t rows, int64_t cols,
                     int dtype, void* stream);
 
+/* The same for a softmax with a bias shared by the batch rows: dx, dy, y [B1][B2][HQ][cols], and the bias gradient
+ * dbias[B1][HQ][cols] = dx summed over B2 (in fp32, before dx is rounded).  The batch rows are cut into `slices`; with more
+ * than one, ws holds slices * B1 * HQ * cols floats.
+ * Replaces: softmax_cuda_kernel.cu:252-334,524-614 and the sum over dim 1 of kernel/softmax.py:56. */
+int ffk_softmax_bwd_bias(void* dx, void* dbias, float* ws, int64_t slices, const void* dy, const void* y, int64_t B1,
+                         int64_t B2, int64_t HQ, int64_t cols, int dtype, void* stream);
+
 /* Measurement aid with no counterpart in the reference: a plain streaming copy of `bytes` (a multiple of 16) with the
  * access pattern of the row kernels (16-byte non-temporal loads and stores, a grid like theirs).  bench.py times it
  * beside the fused softmax and LayerNorm: it is what a read-once / write-once stream of the same size reaches on the
@@ -338,6 +345,30 @@ int ffk_attention_bwd(void* dq, void* dk, void* dv, float* dbias, float* lse, fl
  * (fastfold/model/fastnn/ops.py:303-306; kernel/attention_core.py:24-31), which here has to end in tile order. */
 int ffk_tile_pack(void* dst, const void* src, int64_t B2, int64_t H, int64_t N, int64_t D, int64_t s_b, int64_t s_h,
                   int64_t s_n, float scale, int kind, int dtype, void* stream);
+
+/* The same for several operands of one attention in one launch.  Operand i is job[i].src (strided as above, or with `tiled`
+ * the FFK_TILE_QK tiles of an earlier call), times `scale`, written in FFK_TILE_QK order to qk and in FFK_TILE_V order to acc
+ * (either may be NULL).  With dsum, the row sums over d of src * other (before the factor; fp32,
+ * dsum[((b2 * H + h) * ceil(N/32)) * 32 + n], rows past N zero) - the sum_d do.o of the backward pass.
+ * bias (optional): [H][N][N] contiguous, times bias_scale, to bias_t in FFK_TILE_BIAS order.  bf16 and fp32. */
+#define FFK_PACK_JOBS 4
+typedef struct {
+    const void* src;
+    void *qk, *acc;
+    const void* other;
+    float* dsum;
+    int64_t s_b, s_h, s_n, o_sb, o_sh, o_sn;
+    float scale;
+    int tiled;
+} ffk_pack_job;
+typedef struct {
+    ffk_pack_job job[FFK_PACK_JOBS];
+    const void* bias;
+    void* bias_t;
+    float bias_scale;
+    int n, B2, H, N, D, dtype, reserved;
+} ffk_pack_desc;
+int ffk_attention_pack(const ffk_pack_desc* desc, void* stream);
 
 /* Batched 2-D transposition with strides (all strides in elements):
  *     out[b][y][x] = in[b][x][y]      for b < B, x < X, y < Y,

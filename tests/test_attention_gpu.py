@@ -390,3 +390,32 @@ def test_tile_pack_matches_the_torch_layout_helpers(dev, dtype, b2, h, n, d):
             ref = (x32.float() * scale).to(dtype) if scale != 1.0 else x32
             assert torch.equal(_lib.tile_pack(x, _lib.FFK_TILE_QK, scale).view(-1), layouts.tile_qk(ref).reshape(-1))
             assert torch.equal(_lib.tile_pack(x, _lib.FFK_TILE_V, scale).view(-1), layouts.tile_v(ref).reshape(-1))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("b2,h,n,d", [(1, 1, 1, 8), (2, 3, 33, 16), (3, 2, 64, 32), (2, 2, 95, 32), (1, 5, 160, 32)])
+def test_attention_pack_matches_the_torch_layout_helpers(dev, dtype, b2, h, n, d):
+    """ffk_attention_pack against the pad / view / permute formulation of the same tiles, bit for bit: plain and strided
+    sources, tiles re-tiled, the factor, both orders at once, the row sums of a product, the bias tiles."""
+    from fastfold_amd import _lib
+    from fastfold_amd.model.fastnn.kernel import layouts
+    g = torch.Generator().manual_seed(n + d)
+    x = torch.randn(b2, h, n, d, generator=g).to(dev, dtype)
+    y = torch.randn(b2, n, h, d, generator=g).to(dev, dtype).permute(0, 2, 1, 3)          # strided, as the output of a core is
+    bias = torch.randn(h, n, n, generator=g).to(dev, dtype)
+    nt = (n + 31) // 32
+
+    def pad(t):
+        return torch.nn.functional.pad(t.float(), (0, 32 - d)).to(dtype)
+    xq, yq, ya, xa = (torch.empty(b2, h, nt, 1024, dtype=dtype, device=dev) for _ in range(4))
+    dsum = torch.empty(b2, h, nt * 32, dtype=torch.float32, device=dev)
+    bt = torch.empty(h, nt, nt, 1024, dtype=dtype, device=dev)
+    _lib.attention_pack([(x, 0.3, xq, None, None, None), (y, 1.0, yq, ya, dsum, x)], B2=b2, H=h, N=n, D=d, dtype=dtype, bias=bias,
+                        bias_t=bt, bias_scale=1.5)
+    _lib.attention_pack([(xq, 1.0, None, xa, None, None)], B2=b2, H=h, N=n, D=d, dtype=dtype)
+    xs = pad((x.float() * 0.3).to(dtype))
+    assert torch.equal(xq.view(-1), layouts.tile_qk(xs).reshape(-1)) and torch.equal(xa.view(-1), layouts.tile_v(xs).reshape(-1))
+    assert torch.equal(yq.view(-1), layouts.tile_qk(pad(y)).reshape(-1)) and torch.equal(ya.view(-1), layouts.tile_v(pad(y)).reshape(-1))
+    assert torch.equal(bt.view(-1), layouts.tile_bias((bias.float() * 1.5).to(dtype)).reshape(-1))
+    ref = (x.double() * y.double()).sum(-1)
+    assert float((dsum[..., :n] - ref).abs().max()) < 1e-4 and float(dsum[..., n:].abs().sum()) == 0.0

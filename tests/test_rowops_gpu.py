@@ -36,6 +36,37 @@ def test_fused_softmax_reference_cases(dev, seq, dtype):
             assert float(out[0, :, :, :, :][(m_[0] == 0)[:, None, None, :].expand_as(out[0])].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b1,b2,h,nq,cols", [(1, 3, 2, 5, 24), (2, 7, 1, 9, 33), (1, 40, 2, 6, 64), (1, 5, 3, 7, 77), (1, 4, 2, 3, 130),
+                                             (1, 64, 4, 24, 24), (1, 33, 2, 8, 257), (1, 9, 1, 2, 770), (1, 2, 1, 3, 1023),
+                                             (1, 3, 1, 2, 1025), (1, 2, 1, 2, 4104), (2, 3, 2, 4, 2048)])
+def test_fused_softmax_rows_and_bias_gradient(dev, dtype, b1, b2, h, nq, cols):
+    """Every access width of the row kernels (vectors, two elements, one element, rows beyond the register geometries), the
+    bias gradient with one slice of the batch rows and with several, against float64 autograd of the formula."""
+    from fastfold_amd.model.fastnn.kernel import fused_softmax
+    g = torch.Generator().manual_seed(cols + b2)
+    x = (2 * torch.randn(b1, b2, h, nq, cols, generator=g)).to(dev, dtype)
+    mask = (torch.rand(b1, b2, cols, generator=g) > 0.2).to(dev, dtype)
+    mask[..., 1] = 1
+    bias = torch.randn(b1, 1, h, nq, cols, generator=g).to(dev, dtype)
+    dy = torch.randn(b1, b2, h, nq, cols, generator=g).to(dev, dtype)
+    xr, br = (t.double().cpu().requires_grad_(True) for t in (x, bias))
+    ref = torch.softmax((xr + br).masked_fill(mask.cpu()[:, :, None, None, :] == 0, -1e9), -1)
+    ref.backward(dy.double().cpu())
+    xf, bf = x.clone().requires_grad_(True), bias.clone().requires_grad_(True)
+    out = fused_softmax(xf, mask, bf)
+    out.backward(dy)
+    tol = {torch.float32: 2e-6, torch.bfloat16: 1e-2, torch.float16: 2e-3}[dtype]
+
+    def rel(a, b):
+        return float((a.detach().double().cpu() - b).norm() / b.norm())
+    assert rel(out, ref.detach()) < tol
+    assert rel(xf.grad, xr.grad) < 2 * tol and rel(bf.grad, br.grad) < 2 * tol
+    xg = x.clone().requires_grad_(True)
+    fused_softmax(xg, mask, bias).backward(dy)              # without a bias gradient
+    assert rel(xg.grad, xr.grad) < 2 * tol
+
+
 def test_fused_softmax_inplace_and_backward(dev):
     from fastfold_amd.model.fastnn.kernel import fused_softmax
     from fastfold_amd.model.fastnn.kernel.softmax import fused_softmax_
