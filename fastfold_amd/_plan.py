@@ -7,7 +7,8 @@ the foreign call - at about 20 microseconds of host time each, 0.57 ms for a blo
 and from then on replays it: the 48-block trunk at N_seq = 128, N_res = 77 went from 30.6 to 4.6 ms of host time.
 
 A plan holds no results.  Every pointer of a recorded launch is one of
-  * a caller's buffer (activations, masks and what is derived from them), patched on each replay,
+  * a caller's buffer (activations, masks and what is derived from them), patched on each replay - of calls in which the same
+    buffers coincide as in the recorded one,
   * scratch, laid out in one allocation that each replay makes for itself on its own stream,
   * a packed weight or parameter, which the plan keeps alive; a plan is dropped as soon as a parameter of its module has
     changed (another tensor, or another version of it), exactly as the packed weights are.
@@ -226,16 +227,32 @@ def hold():
         rec.hold()
 
 
+def _sharing(tensors):
+    """Which of the tensors share memory, and how: () or one (position, position of another, bytes between their starts) per
+    tensor that begins inside memory another one has begun in.  A recording knows a buffer by its address only, so a plan fits
+    no call in which other buffers coincide (one mask passed for both, a cotangent that is the input itself)."""
+    spans = sorted((t.data_ptr(), i, t.nbytes) for i, t in enumerate(tensors) if t is not None)
+    out, start, first, end = [], 0, 0, 0
+    for lo, i, n in spans:
+        if lo < end:
+            out.append((i, first, lo - start))
+        else:
+            start, first = lo, i
+        end = max(end, lo + n)
+    return tuple(out)
+
+
 def run(owner, key, tensors, sequence):
     """Executes ``sequence()`` - launches on the current stream that work on ``tensors`` (a list, entries may be None; the
     first is not), on scratch from ``alloc`` and on the weights of the module ``owner`` - or replays its plan.  ``key``
-    names everything else the launches depend on (shapes, dtypes, switches)."""
+    names everything else the launches depend on (shapes, dtypes, switches) but which of ``tensors`` share memory."""
     if _lib._TIMED or _lib._STATE.recorder is not None:        # launches are being timed one by one, or recorded already
         return sequence()
     st = owner.__dict__.get("_plan_state")
     if st is None or not st.watch.intact():
         st = owner.__dict__["_plan_state"] = _State(owner)
     version = st.watch.version()
+    key = (key, _sharing(tensors))
     plan = st.plans.get(key)
     if plan is not None and plan.version == version:
         if plan.blob is None:

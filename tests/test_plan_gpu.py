@@ -162,3 +162,42 @@ def test_replay_under_memory_of_any_content(dev, s, r):
         if want is not None:
             assert all(torch.equal(x, y) for x, y in zip(got, want))
         want = got
+
+
+@gpu
+@pytest.mark.parametrize("kind,dtype", [("evoformer", torch.float32), ("evoformer", torch.bfloat16), ("extra", torch.bfloat16),
+                                        ("backward", torch.float32)])
+def test_replay_with_other_buffers_shared(dev, kind, dtype):
+    """s == r, so that both masks have one shape: a block recorded with one tensor as both masks (and, backward, the input as
+    the cotangent), then called with two; and the other way round."""
+    from fastfold_amd.model.fastnn import Evoformer, ExtraMSABlock
+    n = 64
+    st = _stack(dev, dtype, 1)
+    if kind == "extra":
+        g = torch.Generator().manual_seed(2)
+        blk = ExtraMSABlock(64, 128, True, True)
+        with torch.no_grad():
+            for p in blk.parameters():
+                p.copy_(torch.randn(p.shape, generator=g) * 0.1)
+        blk = blk.to(dev, dtype).eval()
+    else:
+        blk = Evoformer(256, 128, True, True).to(dev, dtype).eval()
+        blk.load_state_dict(st.blocks[0].state_dict())
+    m, z, mm, pm = _inputs(dev, dtype, n, n, 7)
+    m = m[..., :64].contiguous() if kind == "extra" else m
+    ones = torch.ones_like(pm)
+    dm, dz = torch.randn_like(m), torch.randn_like(z)
+
+    def call(msa_mask, pair_mask, own_cotangent):
+        if kind != "backward":
+            with torch.no_grad():
+                return blk(m, z, msa_mask, pair_mask)
+        with torch.no_grad():
+            a, b = m[None], z[None]
+            cot = (a, b) if own_cotangent else (dm[None], dz[None])
+            da, db, grads = blk._backward(a, b, msa_mask[None], pair_mask[None], *cot, None)
+            return [da, db, *grads]
+    for args in [(ones, ones, True)] * 3 + [(mm, pm, False)] * 3 + [(ones, ones, True), (mm, pm, True), (pm, mm, False)]:
+        got = call(*args)
+        want = _in_python(lambda: call(*args))
+        assert all(torch.equal(x, y) for x, y in zip(got, want))
