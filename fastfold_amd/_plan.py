@@ -239,7 +239,7 @@ def _sharing(tensors):
         else:
             start, first = lo, i
         end = max(end, lo + n)
-    return tuple(out)
+    return tuple(sorted(out))            # in the order of the list, whatever the addresses
 
 
 def run(owner, key, tensors, sequence):

@@ -60,3 +60,17 @@ def test_a_plan_recorded_with_shared_buffers_serves_no_others(library, form):
     for tensors in (shared, other, shared, other, other[::-1], shared):
         assert _call(library, owner, tensors) == _ptrs(tensors)
     assert library.replays == 4                # all but the first call of each pattern (the reversed one has that of ``other``)
+    for tensors in ([a, b, a, b], [b, a, b, a], [x, a, x, a]):         # one pattern, whichever buffer lies first in memory
+        assert _call(library, owner, tensors, "pairs") == _ptrs(tensors)
+    assert library.replays == 6
+
+
+def test_values_derived_from_a_mask_without_a_version_counter():
+    """Tensors made under ``torch.inference_mode`` have none: built once per mask inside a cache, like the others."""
+    from fastfold_amd.model.fastnn import _fused as F_
+    with torch.inference_mode():
+        masks = [torch.ones(4, 4), torch.ones(4, 4)]
+        masks.append(masks[0].t())
+        with F_.mask_cache():
+            got = [F_._mask_derived(m, "twice", lambda m=m: 2 * m) for m in masks + masks]
+    assert all(got[i] is got[i + 3] for i in range(3)) and len({id(t) for t in got}) == 3
