@@ -109,7 +109,10 @@ def _mask_derived(mask, what, build):
     entries = _MASK_CACHE.entries
     if entries is None:
         return build()
-    key = (what, mask.data_ptr(), mask._version, tuple(mask.shape), tuple(mask.stride()), mask.dtype)
+    # tensors made under torch.inference_mode have no version counter; a cache lives within one call of a stack or block,
+    # during which nobody writes the masks it was given
+    version = None if mask.is_inference() else mask._version
+    key = (what, mask.data_ptr(), version, tuple(mask.shape), tuple(mask.stride()), mask.dtype)
     for k, _, v in entries:
         if k == key:
             return v

@@ -86,3 +86,28 @@ def test_feeder_stacks_at_ragged_extents(dev, s, r):
         lst = [t.clone()]
         half.inplace(lst, pm[None], None)
         assert torch.equal(lst[0], out)
+
+
+@pytest.mark.parametrize("r", [32, 45])
+def test_under_inference_mode(dev, r):
+    """Stacks and single blocks with masks from outside and with masks made under ``torch.inference_mode``, which have no version
+    counter (the padded ones of a ragged bf16 call are always such): the bits of the call under ``torch.no_grad``."""
+    from fastfold_amd.model.fastnn import Evoformer, EvoformerStack, ExtraMSABlock, ExtraMSAStack, TemplatePairStack
+    m, z, mm, pm = _inputs(dev, 33, r, 256, 3)
+    e = m[..., :64].contiguous()
+    t = torch.randn(2, r, r, 64, device=dev).bfloat16()
+    mods = [(_init(mod, dev).bfloat16(), call) for mod, call in (
+        (EvoformerStack(256, 128, 384, 2, 1), lambda f, a, b: f(m, z, a, b)),
+        (Evoformer(256, 128, True, True), lambda f, a, b: f(m, z, a, b)),
+        (ExtraMSAStack(64, 128, 2), lambda f, a, b: (f(e, z, None, a, b),)),
+        (ExtraMSABlock(64, 128, True, True), lambda f, a, b: f(e, z, a, b)),
+        (TemplatePairStack(64, 16, 64, 2, 4, 2, 0.25, None), lambda f, a, b: (f(t, b[None], None),)))]
+    for mod, call in mods:
+        with torch.no_grad():
+            want = call(mod, mm, pm)
+        with torch.inference_mode():
+            for a, b in ((mm, pm), (mm.clone(), pm.clone()), (mm.clone(), pm.clone())):
+                got = call(mod, a, b)
+                assert all(torch.equal(x, y) for x, y in zip(got, want)), type(mod).__name__
+        with torch.no_grad():
+            assert all(torch.equal(x, y) for x, y in zip(call(mod, mm, pm), want))
