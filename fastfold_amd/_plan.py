@@ -16,6 +16,7 @@ A sequence that issues anything else is not planned and keeps running in Python.
 """
 import ctypes
 import struct
+import threading
 from collections import OrderedDict
 
 import torch
@@ -198,7 +199,20 @@ class _State:
 
     def __init__(self, owner):
         self.watch = _Watch(owner)
-        self.plans = OrderedDict()
+        self.plans = OrderedDict()               # the one used longest ago first
+        self.lock = threading.Lock()             # of the order and the size of ``plans``
+
+    def touch(self, key):
+        with self.lock:
+            if key in self.plans:                # another thread may have dropped it since
+                self.plans.move_to_end(key)
+
+    def store(self, key, plan):
+        with self.lock:
+            self.plans[key] = plan
+            self.plans.move_to_end(key)
+            while len(self.plans) > _MAX_PLANS:
+                self.plans.popitem(last=False)
 
     def __deepcopy__(self, memo):
         return None
@@ -255,6 +269,7 @@ def run(owner, key, tensors, sequence):
     key = (key, _sharing(tensors))
     plan = st.plans.get(key)
     if plan is not None and plan.version == version:
+        st.touch(key)
         if plan.blob is None:
             return sequence()
         return plan.run(tensors)
@@ -268,7 +283,4 @@ def run(owner, key, tensors, sequence):
         _lib._STATE.recorder = None
     if builds != before:
         return           # weights were packed on the way: their memory was not known when the recording began
-    st.plans.pop(key, None)
-    st.plans[key] = _Plan(version, None if rec.failed else b"".join(rec.out), rec.peak, st.watch.tensors())
-    if len(st.plans) > _MAX_PLANS:
-        st.plans.popitem(last=False)
+    st.store(key, _Plan(version, None if rec.failed else b"".join(rec.out), rec.peak, st.watch.tensors()))

@@ -65,6 +65,18 @@ def test_a_plan_recorded_with_shared_buffers_serves_no_others(library, form):
     assert library.replays == 6
 
 
+def test_the_plan_dropped_is_the_one_used_longest_ago(library):
+    owner, x = torch.nn.Linear(2, 2), torch.zeros(8)
+    for k in range(_plan._MAX_PLANS):
+        _call(library, owner, [x], k)
+    for k in range(_plan._MAX_PLANS, _plan._MAX_PLANS + 4):
+        _call(library, owner, [x], 0)                 # used in between
+        _call(library, owner, [x], k)
+    assert library.replays == 4
+    plans = owner.__dict__["_plan_state"].plans
+    assert [k[0] for k in plans] == [*range(5, _plan._MAX_PLANS + 3), 0, _plan._MAX_PLANS + 3]
+
+
 def test_values_derived_from_a_mask_without_a_version_counter():
     """Tensors made under ``torch.inference_mode`` have none: built once per mask inside a cache, like the others."""
     from fastfold_amd.model.fastnn import _fused as F_
