@@ -341,7 +341,8 @@ class ExtraMSAStack(nn.Module):
 
     def inplace(self, m, z, chunk_size: int, msa_mask: Optional[torch.Tensor] = None,
                 pair_mask: Optional[torch.Tensor] = None, _mask_trans: bool = True):
-        """``m`` / ``z`` are one-element lists; returns the list ``z`` as the reference does (msa.py:433-464)."""
+        """``m`` / ``z`` are one-element lists; returns the list ``z`` as the reference does (msa.py:433-464).  In bf16 at a
+        residue extent that is no multiple of 32 the call holds zero-padded copies of both beside them."""
         msa_mask, pair_mask = self._masks(m[0], z[0], msa_mask, pair_mask)
         contiguous = m[0].is_contiguous() and z[0].is_contiguous()
         z[0] = self._run(m[0], z[0], msa_mask, pair_mask, inplace_first=contiguous)

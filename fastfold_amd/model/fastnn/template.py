@@ -240,6 +240,7 @@ class TemplatePairStack(nn.Module):
         return self._run(t, mask, inplace=False)
 
     def inplace(self, t, mask: torch.tensor, chunk_size: int, _mask_trans: bool = True):
-        """``t`` is a one-element list whose tensor is overwritten (template.py:404-434)."""
+        """``t`` is a one-element list whose tensor is overwritten (template.py:404-434).  In bf16 at an extent that is no
+        multiple of 32 the call holds a zero-padded copy of one template at a time beside it."""
         t[0] = self._run(t[0], mask, inplace=True)
         return t

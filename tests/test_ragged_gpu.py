@@ -111,3 +111,33 @@ def test_under_inference_mode(dev, r):
                 assert all(torch.equal(x, y) for x, y in zip(got, want)), type(mod).__name__
         with torch.no_grad():
             assert all(torch.equal(x, y) for x, y in zip(call(mod, mm, pm), want))
+
+
+@pytest.mark.parametrize("kind", ["trunk", "extra"])
+def test_in_place_memory_at_ragged_extents(dev, kind, monkeypatch):
+    """The padded copies of an in-place call take no more than the un-padded run takes in gate tensors and unfused scratch (5 %
+    of the peak beyond the inputs), and no more than themselves beyond the peak at the next whole tile."""
+    from fastfold_amd.model.fastnn import EvoformerStack, ExtraMSAStack, _fused, set_chunk_size
+    s, r = 64, 1270
+    mod = _init(EvoformerStack(256, 128, 384, 1, 1) if kind == "trunk" else ExtraMSAStack(64, 128, 1), dev).bfloat16()
+    c_m = 256 if kind == "trunk" else 64
+
+    def peak(r):
+        m, z, mm, pm = _inputs(dev, s, r, c_m, 3)
+        with torch.no_grad():
+            for _ in range(2):                                   # packs the weights; measured
+                torch.cuda.synchronize()
+                base = torch.cuda.memory_allocated()
+                torch.cuda.reset_peak_memory_stats()
+                mod.inplace([m], [z], mm, pm) if kind == "trunk" else mod.inplace([m], [z], None, mm, pm)
+        torch.cuda.synchronize()
+        return torch.cuda.max_memory_allocated() - base
+    set_chunk_size(64)
+    try:
+        padded, whole = peak(r), peak(1280)
+        monkeypatch.setattr(_fused, "pad_to_tiles", lambda m, z, mk, pk, pad_s=True: (m, z, mk, pk))
+        as_it_is = peak(r)
+    finally:
+        set_chunk_size(None)
+    assert padded <= 1.05 * as_it_is, (padded, as_it_is)
+    assert padded <= whole + 1.02 * 2 * (s * 1280 * c_m + 1280 * 1280 * 128), (padded, whole)
