@@ -432,27 +432,43 @@ def _over(n):
     return round_up(n, 32) - n
 
 
+def kept(t, like):
+    """A mask or dropout multiplier as an autograd function keeps it: in the type of ``like``, contiguous.  Through
+    ``save_for_backward``, so that a change of it between the passes is noticed; a tensor made under ``torch.inference_mode``
+    cannot be saved and is copied."""
+    if t is None:
+        return None
+    t = t.to(like.dtype).contiguous()
+    return t.clone() if t.is_inference() else t
+
+
 class _Module(torch.autograd.Function):
     """A sub-module under autograd: the fused forward launches, and the backward sequence above at extents padded to whole tiles.
-    ``forward(ctx, step, n_inputs, *inputs, *parameters)``; ``step`` knows the module and its masks and dropout multipliers."""
+    ``forward(ctx, step, (n_inputs, n_kept), *inputs, *kept, *parameters)``: ``kept`` are the masks and dropout multipliers."""
 
     @staticmethod
-    def forward(ctx, step, n, *args):
+    def forward(ctx, step, counts, *args):
+        n, k = counts
         inputs = [t.contiguous() for t in args[:n]]
-        ctx.step, ctx.n, ctx.params = step, n, args[n:]
-        ctx.save_for_backward(*inputs)
-        return step.forward(*inputs)
+        ctx.step, ctx.counts, ctx.params = step, counts, args[n + k:]
+        ctx.save_for_backward(*inputs, *args[n:])
+        return step.forward(*inputs, *args[n:n + k])
 
     @staticmethod
     def backward(ctx, dy):
+        n, k = ctx.counts
         g = Grads(list(ctx.params))
-        inputs = ctx.saved_tensors
+        saved = ctx.saved_tensors[:n + k]                 # raises if one of them, or a parameter, was changed in place
         g = g.bind(torch.empty(g.numel, dtype=dy.dtype, device=dy.device))
         with torch.no_grad():
-            dx = ctx.step.backward(dy.contiguous(), g, *inputs)
-        need = ctx.needs_input_grad
-        return (None, None, *(d if need[2 + i] else None for i, d in enumerate(dx)),
-                *(v.to(p.dtype) if need[2 + ctx.n + i] else None for i, (p, v) in enumerate(zip(ctx.params, g.views()))))
+            dx = ctx.step.backward(dy.contiguous(), g, *saved)
+        need = ctx.needs_input_grad[2:]
+        return (None, None, *(d if need[i] else None for i, d in enumerate(dx)), *(None for _ in range(k)),
+                *(v.to(p.dtype) if need[n + k + i] else None for i, (p, v) in enumerate(zip(ctx.params, g.views()))))
+
+
+def _apply(step, inputs, extra, params):
+    return _Module.apply(step, (len(inputs), len(extra)), *inputs, *(kept(t, inputs[0]) for t in extra), *params)
 
 
 def _tiles(t):
@@ -475,39 +491,38 @@ class _TransitionStep:
 
 
 class _TriMulStep:
-    def __init__(self, tm, mask, drop):
-        self.mod, self.mask, self.drop = tm, mask, drop
+    def __init__(self, tm):
+        self.mod = tm
 
-    def forward(self, z):
+    def forward(self, z, mask, drop):
         r = z.shape[1]
         d, _ = _tiles(z)
-        z, mask, drop = _pad(z, d, d), _pad(self.mask.to(z.dtype), d, d).contiguous(), self.drop
+        z, mask = _pad(z, d, d), _pad(mask, d, d)
         if drop is not None:
             drop = _pad(drop, *((d, 0) if drop.shape[1] == r and drop.shape[2] == 1 else (0, d)))
         return self.mod._run(z, mask, torch.empty_like(z), drop=drop)[:, :r, :r].contiguous()
 
-    def backward(self, dy, g, z):
+    def backward(self, dy, g, z, mask, drop):
         r, C = z.shape[1], z.shape[3]
         d = _over(r)
-        zp, dyp, mask = _pad(z, d, d), _pad(dy, d, d), _pad(self.mask.to(z.dtype), d, d).contiguous()
+        zp, dyp, mask = _pad(z, d, d), _pad(dy, d, d), _pad(mask, d, d)
         dx = torch.empty_like(zp)
-        drop = None if self.drop is None else _pad(self.drop, 0, d).reshape(-1, C).contiguous()
+        drop = None if drop is None else _pad(drop, 0, d).reshape(-1, C).contiguous()
         triangle_multiplication_backward(self.mod, zp.view(-1, C), dyp.view(-1, C), dx.view(-1, C), g, r=r + d, mask=mask[0], drop=drop)
         return (dx[:, :r, :r].contiguous(),)
 
 
 class _TriAttStep(_TriMulStep):
-    def backward(self, dy, g, z):
+    def backward(self, dy, g, z, mask, drop):
         ta = self.mod
         r, C = z.shape[1], z.shape[3]
         d = _over(r)
         n = r + d
-        zp, dyp, mask = _pad(z, d, d), _pad(dy, d, d), _pad(self.mask.to(z.dtype), d, d).contiguous()
+        zp, dyp, mask = _pad(z, d, d), _pad(dy, d, d), _pad(mask, d, d)
         dx = torch.empty_like(zp)
         a_map, sb, sn, dmap = ((n, C, n * C), 1, n, (n, C, 0)) if ta._ending else ((n * n, 0, C), n, 1, (n, 0, C))
-        drop = None
-        if self.drop is not None:
-            drop = (_pad(self.drop, d, 0) if ta._ending else _pad(self.drop, 0, d)).reshape(-1, C).contiguous()
+        if drop is not None:
+            drop = (_pad(drop, d, 0) if ta._ending else _pad(drop, 0, d)).reshape(-1, C).contiguous()
         kb, flags = F_.key_bias(mask[0], z.device, B2=n, N=n, mask_sb=sb, mask_sn=sn)
         attention_backward(ta, ta.attention, ta.layernorm1, zp.view(-1, C), dyp.view(-1, C), dx.view(-1, C), g, ta.out_bias, B2=n, N=n,
                            a_map=a_map, kb=kb, flags=flags, linear_b=ta.linear_b, drop=drop, drop_map=dmap)
@@ -515,20 +530,20 @@ class _TriAttStep(_TriMulStep):
 
 
 class _ColumnStep:
-    def __init__(self, col, mask):
-        self.mod, self.mask = col, mask
+    def __init__(self, col):
+        self.mod = col
 
-    def forward(self, m):
+    def forward(self, m, mask):
         _, s, r, _ = m.shape
         ds, dr = _tiles(m)
-        m, mask = _pad(m, ds, dr), _pad(self.mask.to(m.dtype), ds, dr).contiguous()
+        m, mask = _pad(m, ds, dr), _pad(mask, ds, dr)
         return self.mod._run(m, mask, torch.empty_like(m))[:, :s, :r].contiguous()
 
-    def backward(self, dy, g, m):
+    def backward(self, dy, g, m, mask):
         col = self.mod
         _, s, r, C = m.shape
         ds, dr = _over(s), _over(r)
-        mp, dyp, mask = _pad(m, ds, dr), _pad(dy, ds, dr), _pad(self.mask.to(m.dtype), ds, dr).contiguous()
+        mp, dyp, mask = _pad(m, ds, dr), _pad(dy, ds, dr), _pad(mask, ds, dr)
         dx = torch.empty_like(mp)
         sp, rp = s + ds, r + dr
         kb, flags = F_.key_bias(mask[0], m.device, B2=rp, N=sp, mask_sb=1, mask_sn=rp)
@@ -538,45 +553,44 @@ class _ColumnStep:
 
 
 class _RowStep:
-    def __init__(self, row, mask, drop):
-        self.mod, self.mask, self.drop = row, mask, drop
+    def __init__(self, row):
+        self.mod = row
 
-    def forward(self, m, z):
+    def forward(self, m, z, mask, drop):
         _, s, r, _ = m.shape
         ds, dr = _tiles(m)
-        m, z, mask = _pad(m, ds, dr), _pad(z, dr, dr), _pad(self.mask.to(m.dtype), ds, dr).contiguous()
-        return self.mod._run(m, z, mask, torch.empty_like(m), drop=_pad(self.drop, 0, dr))[:, :s, :r].contiguous()
+        m, z, mask = _pad(m, ds, dr), _pad(z, dr, dr), _pad(mask, ds, dr)
+        return self.mod._run(m, z, mask, torch.empty_like(m), drop=_pad(drop, 0, dr))[:, :s, :r].contiguous()
 
-    def backward(self, dy, g, m, z):
+    def backward(self, dy, g, m, z, mask, drop):
         _, s, r, C = m.shape
         Cz = z.shape[-1]
         ds, dr = _over(s), _over(r)
-        mp, dyp, zp = _pad(m, ds, dr), _pad(dy, ds, dr), _pad(z, dr, dr)
-        mask = _pad(self.mask.to(m.dtype), ds, dr).contiguous()
+        mp, dyp, zp, mask = _pad(m, ds, dr), _pad(dy, ds, dr), _pad(z, dr, dr), _pad(mask, ds, dr)
         dm, dz = torch.empty_like(mp), torch.empty_like(zp)
         sp, rp = s + ds, r + dr
         kb, flags = F_.key_bias(mask[0], m.device, B2=sp, N=rp, mask_sb=rp, mask_sn=1)
-        drop = None if self.drop is None else _pad(self.drop, 0, dr).reshape(-1, C).contiguous()
+        drop = None if drop is None else _pad(drop, 0, dr).reshape(-1, C).contiguous()
         row_attention_backward(self.mod, mp.view(-1, C), zp.view(-1, Cz), dyp.view(-1, C), dm.view(-1, C), None, dz.view(-1, Cz), g, s=sp,
                                r=rp, kb=kb, flags=flags, drop=drop)
         return dm[:, :s, :r].contiguous(), dz[:, :r, :r].contiguous()
 
 
 class _OuterStep:
-    def __init__(self, opm, mask, budget):
-        self.mod, self.mask, self.budget = opm, mask, budget
+    def __init__(self, opm, budget):
+        self.mod, self.budget = opm, budget
 
-    def forward(self, m, z):
+    def forward(self, m, z, mask):
         r = z.shape[1]
         ds, dr = _tiles(m)
-        m, z, mask = _pad(m, ds, dr), _pad(z, dr, dr), _pad(self.mask.to(m.dtype), ds, dr).contiguous()
+        m, z, mask = _pad(m, ds, dr), _pad(z, dr, dr), _pad(mask, ds, dr)
         return self.mod._run(m, mask, z, torch.empty_like(z))[:, :r, :r].contiguous()
 
-    def backward(self, dy, g, m, z):
+    def backward(self, dy, g, m, z, mask):
         _, s, r, C = m.shape
         Cz = z.shape[-1]
         ds, dr = _over(s), _over(r)
-        mp, dyp, mask = _pad(m, ds, dr), _pad(dy, dr, dr), _pad(self.mask.to(m.dtype), ds, dr).contiguous()
+        mp, dyp, mask = _pad(m, ds, dr), _pad(dy, dr, dr), _pad(mask, ds, dr)
         dm = torch.empty_like(mp)
         outer_product_mean_backward(self.mod, mp.view(-1, C), mask[0], dyp.view(-1, Cz), None, dm.view(-1, C), g, s=s + ds, r=r + dr,
                                     nrm=F_.opm_normaliser(mask[0]), budget=self.budget)
@@ -584,33 +598,35 @@ class _OuterStep:
 
 
 def transition(tr, x):
-    return _Module.apply(_TransitionStep(tr), 1, x, *transition_parameters(tr)) if covers_transition(tr) and _dtype_ok(x) else None
+    return _apply(_TransitionStep(tr), (x,), (), transition_parameters(tr)) if covers_transition(tr) and _dtype_ok(x) else None
 
 
 def triangle_multiplication(tm, z, mask, drop):
     if not (covers_triangle_multiplication(tm) and _dtype_ok(z)):
         return None
-    return _Module.apply(_TriMulStep(tm, mask, drop), 1, z, *triangle_multiplication_parameters(tm))
+    return _apply(_TriMulStep(tm), (z,), (mask, drop), triangle_multiplication_parameters(tm))
 
 
 def triangle_attention(ta, z, mask, drop):
     if not (covers_triangle_attention(ta) and _dtype_ok(z)):
         return None
-    return _Module.apply(_TriAttStep(ta, mask, drop), 1, z, *triangle_attention_parameters(ta))
+    return _apply(_TriAttStep(ta), (z,), (mask, drop), triangle_attention_parameters(ta))
 
 
 def column_attention(col, m, mask):
-    return _Module.apply(_ColumnStep(col, mask), 1, m, *column_parameters(col)) if covers_column(col) and _dtype_ok(m) else None
+    return _apply(_ColumnStep(col), (m,), (mask,), column_parameters(col)) if covers_column(col) and _dtype_ok(m) else None
 
 
 def row_attention(row, m, z, mask, drop):
-    return _Module.apply(_RowStep(row, mask, drop), 2, m, z, *row_parameters(row)) if covers_row(row) and _dtype_ok(m, z) else None
+    if not (covers_row(row) and _dtype_ok(m, z)):
+        return None
+    return _apply(_RowStep(row), (m, z), (mask, drop), row_parameters(row))
 
 
 def outer_product_mean(opm, m, mask, z, budget):
     if not (covers_outer_product_mean(opm) and _dtype_ok(m, z)) or m.dim() != 4:
         return None
-    return _Module.apply(_OuterStep(opm, mask, budget), 2, m, z, *outer_product_mean_parameters(opm))
+    return _apply(_OuterStep(opm, budget), (m, z), (mask,), outer_product_mean_parameters(opm))
 
 
 # ------------------------------------------------------------------------------------------------- block ----

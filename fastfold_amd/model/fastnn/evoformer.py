@@ -28,46 +28,60 @@ def _private_copy(view, owner):
     return out.clone() if out.data_ptr() == owner.data_ptr() else out
 
 
+def _save(ctx, block, keys, m, z, msa_mask, pair_mask, multipliers):
+    """Keeps what the backward pass of a block reads; the multipliers as the dict ``drops`` (None without ``keys``).  All of it
+    through ``save_for_backward``: a mask that is changed in place between the passes is an error, not another gradient."""
+    ctx.block, ctx.keys = block, keys
+    ctx.save_for_backward(m, z, msa_mask, pair_mask, *multipliers)
+    return None if keys is None else dict(zip(keys, multipliers))
+
+
+def _saved(ctx):
+    m, z, msa_mask, pair_mask, *multipliers = ctx.saved_tensors
+    return m, z, (msa_mask, pair_mask), None if ctx.keys is None else dict(zip(ctx.keys, multipliers))
+
+
 class _BlockRecompute(torch.autograd.Function):
     """One Evoformer block as its own checkpoint: the forward pass runs the fused launches (nothing of it is kept but
-    the two inputs and the dropout multipliers, which are drawn here so that both passes see the same ones); the
+    the two inputs, the masks and the dropout multipliers, which the caller draws so that both passes see the same ones); the
     backward pass re-runs the block operator by operator with autograd on, the way block checkpointing re-runs it
     (fastfold/utils/checkpointing.py:55-73; evoformer.py:262-266), and back-propagates through that."""
 
     @staticmethod
-    def forward(ctx, block, msa_mask, pair_mask, drops, _grad_anchor, m, z):
-        ctx.block, ctx.masks, ctx.drops = block, (msa_mask, pair_mask), drops
-        ctx.save_for_backward(m, z)
+    def forward(ctx, block, keys, _grad_anchor, m, z, msa_mask, pair_mask, *multipliers):
+        drops = _save(ctx, block, keys, m, z, msa_mask, pair_mask, multipliers)
         return block._core_any(m.contiguous(), z.contiguous(), msa_mask, pair_mask, inplace=False, drops=drops)
 
     @staticmethod
     def backward(ctx, dm, dz):
-        m, z = ctx.saved_tensors
+        m, z, masks, drops = _saved(ctx)
         with torch.enable_grad():
             m_, z_ = m.detach().requires_grad_(True), z.detach().requires_grad_(True)
-            mo, zo = ctx.block._core_train(m_, z_, *ctx.masks, drops=ctx.drops if ctx.drops is not None else {})
+            mo, zo = ctx.block._core_train(m_, z_, *masks, drops=drops if drops is not None else {})
         torch.autograd.backward((mo, zo), (dm, dz))        # parameter gradients accumulate here, as under checkpointing
-        return None, None, None, None, None, m_.grad, z_.grad
+        return (None, None, None, m_.grad, z_.grad, None, None, *(None for _ in ctx.keys or ()))
 
 
 class _BlockGrad(torch.autograd.Function):
     """One Evoformer block as its own checkpoint, forward and backward as launch sequences (``_backward.block_backward``): the
-    forward pass keeps the two inputs and the dropout multipliers (drawn by the caller), the backward pass returns the gradients
-    of the inputs and of every parameter."""
+    forward pass keeps the two inputs, the masks and the dropout multipliers (drawn by the caller), the backward pass returns the
+    gradients of the inputs and of every parameter."""
 
     @staticmethod
-    def forward(ctx, block, msa_mask, pair_mask, drops, m, z, *params):
-        ctx.block, ctx.masks, ctx.drops, ctx.params = block, (msa_mask, pair_mask), drops, params
-        ctx.save_for_backward(m, z)
+    def forward(ctx, block, keys, m, z, msa_mask, pair_mask, *rest):
+        n = len(keys or ())
+        ctx.params = rest[n:]
+        drops = _save(ctx, block, keys, m, z, msa_mask, pair_mask, rest[:n])
         return block._core_any(m.contiguous(), z.contiguous(), msa_mask, pair_mask, inplace=False, drops=drops)
 
     @staticmethod
     def backward(ctx, dm, dz):
-        m, z = ctx.saved_tensors
-        dm, dz, grads = ctx.block._backward(m, z, *ctx.masks, dm, dz, ctx.drops)
+        m, z, masks, drops = _saved(ctx)
+        dm, dz, grads = ctx.block._backward(m, z, *masks, dm, dz, drops)
         need = ctx.needs_input_grad
-        grads = [g.to(p.dtype) if need[6 + i] else None for i, (p, g) in enumerate(zip(ctx.params, grads))]
-        return (None, None, None, None, dm if need[4] else None, dz if need[5] else None, *grads)
+        first = 6 + len(ctx.keys or ())
+        grads = [g.to(p.dtype) if need[first + i] else None for i, (p, g) in enumerate(zip(ctx.params, grads))]
+        return (None, None, dm if need[2] else None, dz if need[3] else None, None, None, *(None for _ in ctx.keys or ()), *grads)
 
 
 class Evoformer(nn.Module):
@@ -213,11 +227,14 @@ class Evoformer(nn.Module):
         """The block under autograd, on the un-padded [1, ...] tensors."""
         if not self.recompute_in_backward:
             return self._core_train(m, z, msa_mask, pair_mask)
+        msa_mask, pair_mask = _backward.kept(msa_mask, m), _backward.kept(pair_mask, z)
+        drops = self._draw_drops(m, z)
+        keys, multipliers = (None, ()) if drops is None else (tuple(drops), tuple(drops.values()))
         if m.dtype in (torch.bfloat16, torch.float32) and z.dtype == m.dtype and m.shape[-1] == 256 and z.shape[-1] == 128 \
                 and _backward.supported(self):
-            return _BlockGrad.apply(self, msa_mask, pair_mask, self._draw_drops(m, z), m, z, *_backward.parameters(self))
+            return _BlockGrad.apply(self, keys, m, z, msa_mask, pair_mask, *multipliers, *_backward.parameters(self))
         anchor = torch.empty(0, device=m.device, requires_grad=True)     # outputs need a gradient even when m and z do not
-        return _BlockRecompute.apply(self, msa_mask, pair_mask, self._draw_drops(m, z), anchor, m, z)
+        return _BlockRecompute.apply(self, keys, anchor, m, z, msa_mask, pair_mask, *multipliers)
 
     def _enter(self, m, z, r):
         if self.first_block:

@@ -106,3 +106,28 @@ def test_block_sequence_equals_the_modules(dev, multimer, s, r, chunk, monkeypat
                     assert _rel(x, y) < 2e-5, n
     finally:
         set_chunk_size(None)
+
+
+@pytest.mark.parametrize("dtype", DT)
+def test_masks_changed_between_the_passes_are_noticed(dev, dtype):
+    """As autograd does for the operators: a block and its modules on their own raise instead of another gradient."""
+    blk = _block(dev, dtype, False)
+    s = r = 32
+    m, z = torch.randn(1, s, r, 256, device=dev, dtype=dtype), torch.randn(1, r, r, 128, device=dev, dtype=dtype)
+    for call in (lambda a, b, mk, pk: blk(a[0], b[0], mk[0], pk[0]),
+                 lambda a, b, mk, pk: (blk.msa.MSARowAttentionWithPairBias(a, b, mk),),
+                 lambda a, b, mk, pk: (blk.msa.MSAColumnAttention(a, mk),),
+                 lambda a, b, mk, pk: (blk.communication(a, mk, b),),
+                 lambda a, b, mk, pk: (blk.pair.TriangleMultiplicationOutgoing(b, pk),),
+                 lambda a, b, mk, pk: (blk.pair.TriangleAttentionEndingNode(b, pk),)):
+        for change in (False, True):
+            mk, pk = torch.ones(1, s, r, device=dev, dtype=dtype), torch.ones(1, r, r, device=dev, dtype=dtype)
+            out = call(m.clone().requires_grad_(), z.clone().requires_grad_(), mk, pk)
+            cot = [torch.ones_like(t) for t in out]
+            if change:
+                mk.zero_()
+                pk.zero_()
+                with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+                    torch.autograd.backward(out, cot)
+            else:
+                torch.autograd.backward(out, cot)

@@ -83,3 +83,71 @@ def test_chan_major_copies_are_separate_and_padded():
     assert torch.equal(L[..., :6], left[0].permute(2, 0, 1)) and float(L[..., 6:].abs().max()) == 0.0
     Li = ops._chan_major(left, (2, 1, 0))                 # incoming: L[c, i, k] = left[k, i, c]
     assert torch.equal(Li[..., :6], left[0].permute(2, 1, 0))
+
+
+@pytest.mark.parametrize("what,noticed", [("mask", True), ("drop", True), ("parameter", True), ("input", True), ("cast mask", False),
+                                          ("inference mask", False)])
+def test_a_module_notices_what_changes_between_the_passes(what, noticed):
+    """The autograd function of the stand-alone modules keeps masks, dropout multipliers and parameters as autograd does: changed
+    in place before the backward pass they raise; a mask of another type, or one that cannot be saved, was copied."""
+    from fastfold_amd.model.fastnn import _backward
+
+    class Step:
+        def forward(self, x, mask, drop):
+            return x * mask * drop
+
+        def backward(self, dy, g, x, mask, drop):
+            return (dy * mask * drop,)
+    x, w, drop = torch.randn(4, requires_grad=True), torch.nn.Parameter(torch.randn(2)), torch.rand(4)
+    mask = torch.rand(4).to(torch.float64 if what == "cast mask" else torch.float32)
+    if what == "inference mask":
+        with torch.inference_mode():
+            mask = torch.rand(4)
+    want = mask.float() * drop
+    y = _backward._apply(Step(), (x,), (mask, drop), [w])
+    with torch.inference_mode(what == "inference mask"), torch.no_grad():
+        {"mask": mask, "cast mask": mask, "inference mask": mask, "drop": drop, "parameter": w, "input": x}[what].add_(1.0)
+    if noticed:
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            y.sum().backward()
+    else:
+        y.sum().backward()
+        assert torch.equal(x.grad, want)
+
+
+@pytest.mark.parametrize("keys", [None, (), ("row", "tmo")])
+def test_a_block_notices_masks_changed_between_the_passes(keys):
+    from fastfold_amd.model.fastnn import evoformer
+
+    class Block:
+        def _core_any(self, m, z, msa_mask, pair_mask, inplace, drops):
+            self.forward_drops = drops
+            return m * msa_mask, z * pair_mask
+
+        def _core_train(self, m, z, msa_mask, pair_mask, drops):
+            self.backward_drops = drops
+            return m * msa_mask, z * pair_mask
+
+        def _backward(self, m, z, msa_mask, pair_mask, dm, dz, drops):
+            self.backward_drops = drops
+            return dm * msa_mask, dz * pair_mask, [torch.ones(2)]
+    w = torch.nn.Parameter(torch.randn(2))
+    for changed in (None, 0, 1, 2):
+        for recompute in (False, True):
+            m, z = torch.randn(3, requires_grad=True), torch.randn(3, requires_grad=True)
+            masks, mult = [torch.rand(3), torch.rand(3)], [torch.rand(3) for _ in keys or ()]
+            blk = Block()
+            if recompute:
+                out = evoformer._BlockRecompute.apply(blk, keys, torch.empty(0, requires_grad=True), m, z, *masks, *mult)
+            else:
+                out = evoformer._BlockGrad.apply(blk, keys, m, z, *masks, *mult, w)
+            assert (blk.forward_drops is None) == (keys is None) and list(blk.forward_drops or ()) == list(keys or ())
+            kept = masks + mult
+            if changed is not None and changed < len(kept):
+                kept[changed].add_(1.0)
+                with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+                    torch.autograd.backward(out, (torch.ones(3), torch.ones(3)))
+                continue
+            torch.autograd.backward(out, (torch.ones(3), torch.ones(3)))
+            assert torch.equal(m.grad, masks[0]) and torch.equal(z.grad, masks[1])
+            assert all(torch.equal(a, b) for a, b in zip((blk.backward_drops or {}).values(), mult))
