@@ -13,6 +13,7 @@ products, and as much host time; the sequences below are about 150 launches, rec
 Rows are the logical rows of the sub-module (b, n) -> b * N + n; ``a_map = (inner, s_o, s_i)`` addresses them in the tensors of
 the natural order, so that the transposed attentions need no transposed copies.  Extents are multiples of 32 (the caller pads).
 """
+import functools
 import math
 
 import torch
@@ -135,10 +136,41 @@ def parameters(block):
             *triangle_attention_parameters(pair.TriangleAttentionEndingNode)]
 
 
-# Which modules the sequences below cover, by widths (the Evoformer's own; the narrower heads and rows of the feeder stacks are
-# differentiated operator by operator through autograd) and by the dtype of their input.
+# Which modules the sequences below cover: by widths (the Evoformer's own; the narrower heads and rows of the feeder stacks are
+# differentiated operator by operator through autograd), by the dtype of their input, and only with sub-modules as they were
+# constructed.  The sequences read the parameters of the sub-modules and never call them, so that a hook, a replaced forward or
+# an adapter in the place of a Linear would not be seen.
 def _dtype_ok(*ts):
     return ts[0].dtype in (torch.bfloat16, torch.float32) and all(t.dtype == ts[0].dtype and t.is_cuda for t in ts)
+
+
+@functools.lru_cache(maxsize=None)
+def _anatomy():
+    """The classes the sequences stand for and the names of their sub-modules."""
+    from . import msa, ops, triangle
+    att, tm, ta = {"to_qkv", "gating_linear", "o_linear"}, {"layernorm1", "layernorm2", "left_right_projection", "left_right_gate",
+                                                           "output_gate", "output_projection"}, {"layernorm1", "linear_b", "attention"}
+    return {ops.Linear: set(), ops.LayerNorm: set(), ops.SelfAttention: att,
+            ops.Transition: {"norm", "linear1", "linear2"}, ops.ChunkTransition: {"norm", "linear1", "linear2"},
+            ops.OutProductMean: {"layernormM", "linear_a", "linear_b", "o_linear"},
+            ops.AsyncChunkTriangleMultiplicationOutgoing: tm, ops.AsyncChunkTriangleMultiplicationIncoming: tm,
+            ops.ChunkTriangleAttentionStartingNode: ta, ops.ChunkTriangleAttentionEndingNode: ta,
+            msa.MSARowAttentionWithPairBias: {"layernormM", "layernormZ", "attention"}, msa.MSAColumnAttention: {"layernormM", "attention"},
+            msa.MSACore: {"MSARowAttentionWithPairBias", "MSAColumnAttention", "MSATransition"},
+            triangle.PairCore: {"TriangleMultiplicationOutgoing", "TriangleMultiplicationIncoming", "TriangleAttentionStartingNode",
+                                "TriangleAttentionEndingNode", "PairTransition"}}
+
+
+def _as_built(mod, anatomy):
+    return (mod._modules.keys() == anatomy.get(type(mod)) and "forward" not in mod.__dict__
+            and not (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks)
+            and getattr(mod, "eps", 1e-5) == 1e-5 and all(_as_built(c, anatomy) for c in mod._modules.values()))
+
+
+def as_built(mod):
+    """Whether everything below ``mod`` is as it was constructed and without hooks."""
+    anatomy = _anatomy()
+    return not torch.nn.modules.module._has_any_global_hook() and all(_as_built(c, anatomy) for c in mod._modules.values())
 
 
 def _covers_attention(att, d):
@@ -170,7 +202,7 @@ def covers_triangle_attention(ta):
 
 
 def supported(block):
-    """Whether ``block_backward`` covers this block."""
+    """Whether ``block_backward`` covers this block (if it is ``as_built``)."""
     msa, pair = block.msa, block.pair
     return (covers_row(msa.MSARowAttentionWithPairBias) and covers_column(msa.MSAColumnAttention)
             and covers_transition(msa.MSATransition) and covers_transition(pair.PairTransition)
@@ -598,33 +630,37 @@ class _OuterStep:
 
 
 def transition(tr, x):
-    return _apply(_TransitionStep(tr), (x,), (), transition_parameters(tr)) if covers_transition(tr) and _dtype_ok(x) else None
+    if not (as_built(tr) and covers_transition(tr) and _dtype_ok(x)):
+        return None
+    return _apply(_TransitionStep(tr), (x,), (), transition_parameters(tr))
 
 
 def triangle_multiplication(tm, z, mask, drop):
-    if not (covers_triangle_multiplication(tm) and _dtype_ok(z)):
+    if not (as_built(tm) and covers_triangle_multiplication(tm) and _dtype_ok(z)):
         return None
     return _apply(_TriMulStep(tm), (z,), (mask, drop), triangle_multiplication_parameters(tm))
 
 
 def triangle_attention(ta, z, mask, drop):
-    if not (covers_triangle_attention(ta) and _dtype_ok(z)):
+    if not (as_built(ta) and covers_triangle_attention(ta) and _dtype_ok(z)):
         return None
     return _apply(_TriAttStep(ta), (z,), (mask, drop), triangle_attention_parameters(ta))
 
 
 def column_attention(col, m, mask):
-    return _apply(_ColumnStep(col), (m,), (mask,), column_parameters(col)) if covers_column(col) and _dtype_ok(m) else None
+    if not (as_built(col) and covers_column(col) and _dtype_ok(m)):
+        return None
+    return _apply(_ColumnStep(col), (m,), (mask,), column_parameters(col))
 
 
 def row_attention(row, m, z, mask, drop):
-    if not (covers_row(row) and _dtype_ok(m, z)):
+    if not (as_built(row) and covers_row(row) and _dtype_ok(m, z)):
         return None
     return _apply(_RowStep(row), (m, z), (mask, drop), row_parameters(row))
 
 
 def outer_product_mean(opm, m, mask, z, budget):
-    if not (covers_outer_product_mean(opm) and _dtype_ok(m, z)) or m.dim() != 4:
+    if not (as_built(opm) and covers_outer_product_mean(opm) and _dtype_ok(m, z)) or m.dim() != 4:
         return None
     return _apply(_OuterStep(opm, budget), (m, z), (mask,), outer_product_mean_parameters(opm))
 

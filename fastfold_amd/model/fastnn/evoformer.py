@@ -14,6 +14,7 @@ from typing import Optional, Tuple
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.utils.checkpoint import checkpoint
 
 from fastfold_amd import _plan
 from . import _backward
@@ -227,6 +228,9 @@ class Evoformer(nn.Module):
         """The block under autograd, on the un-padded [1, ...] tensors."""
         if not self.recompute_in_backward:
             return self._core_train(m, z, msa_mask, pair_mask)
+        if not _backward.as_built(self):
+            # hooks or exchanged modules somewhere in the block: the fused launches would pass them by
+            return checkpoint(self._core_train, m, z, msa_mask, pair_mask, use_reentrant=False)
         msa_mask, pair_mask = _backward.kept(msa_mask, m), _backward.kept(pair_mask, z)
         drops = self._draw_drops(m, z)
         keys, multipliers = (None, ()) if drops is None else (tuple(drops), tuple(drops.values()))
@@ -330,7 +334,6 @@ class EvoformerStack(nn.Module):
     def _run_train(self, m, z, msa_mask, pair_mask):
         """The differentiable stack: plain residual stream, blocks re-run in the backward pass in groups of
         ``blocks_per_ckpt`` while the module is in training mode (evoformer.py:262-266)."""
-        from torch.utils.checkpoint import checkpoint
         mm, zz = m.unsqueeze(0), z.unsqueeze(0)
         mk, pk = msa_mask.unsqueeze(0), pair_mask.unsqueeze(0)
         blocks = list(self.blocks)

@@ -131,3 +131,53 @@ def test_masks_changed_between_the_passes_are_noticed(dev, dtype):
                     torch.autograd.backward(out, cot)
             else:
                 torch.autograd.backward(out, cot)
+
+
+class _LowRank(torch.nn.Module):
+    """An adapter in the place of a Linear: the Linear plus a product of two narrow matrices."""
+
+    def __init__(self, base):
+        super().__init__()
+        w = base.weight
+        g = torch.Generator().manual_seed(9)
+        self.base = base
+        self.a = torch.nn.Parameter(torch.randn(4, w.shape[1], generator=g).to(w) / 16)
+        self.b = torch.nn.Parameter(torch.randn(w.shape[0], 4, generator=g).to(w) / 16)
+
+    def forward(self, x):
+        return self.base(x) + x @ self.a.t() @ self.b.t()
+
+
+@pytest.mark.parametrize("what", ["hook", "adapter"])
+def test_hooks_and_adapters_are_part_of_the_module(dev, what):
+    """A scaling hook on an inner Linear, or a Linear replaced by an adapter, against the same change of the weights: outputs and
+    gradients of the module on its own and of the block around it, in float32."""
+    import copy
+    s, r = 8, 32
+    g = torch.Generator().manual_seed(5)
+    m, z = torch.randn(1, s, r, 256, generator=g).to(dev), torch.randn(1, r, r, 128, generator=g).to(dev)
+    mk, pk = torch.ones(1, s, r, device=dev), torch.ones(1, r, r, device=dev)
+    for call in (lambda b, x, y: (b.msa.MSATransition(x),), lambda b, x, y: b(x[0], y[0], mk[0], pk[0])):
+        blk = _block(dev, torch.float32, False)
+        ref = copy.deepcopy(blk)
+        tr, lin = blk.msa.MSATransition, ref.msa.MSATransition.linear2
+        with torch.no_grad():
+            if what == "hook":
+                tr.linear2.register_forward_hook(lambda mod, args, out: 2.0 * out)
+                lin.weight.mul_(2.0)
+                lin.bias.mul_(2.0)
+            else:
+                tr.linear2 = _LowRank(tr.linear2)
+                lin.weight.add_(tr.linear2.b @ tr.linear2.a)
+        got, want = [], []
+        for b, res in ((blk, got), (ref, want)):
+            x, y = m.clone().requires_grad_(), z.clone().requires_grad_()
+            out = call(b, x, y)
+            torch.autograd.backward(out, [torch.ones_like(t) for t in out])
+            res += [*(o.detach() for o in out), x.grad, b.msa.MSATransition.linear1.weight.grad]
+        # the composition and the launch sequence round differently: a hidden value next to zero may differ in sign (3e-3, see
+        # test_train_gpu.py); an ignored hook or adapter is an error of order one
+        for a, b in zip(got, want):
+            assert _rel(a, b) < 3e-3
+        if what == "adapter":
+            assert float(tr.linear2.a.grad.norm()) > 0 and float(tr.linear2.b.grad.norm()) > 0

@@ -151,3 +151,58 @@ def test_a_block_notices_masks_changed_between_the_passes(keys):
             torch.autograd.backward(out, (torch.ones(3), torch.ones(3)))
             assert torch.equal(m.grad, masks[0]) and torch.equal(z.grad, masks[1])
             assert all(torch.equal(a, b) for a, b in zip((blk.backward_drops or {}).values(), mult))
+
+
+@pytest.mark.parametrize("change", ["forward hook", "pre-hook", "backward hook", "global hook", "subclass", "own forward", "eps",
+                                    "another module", "a part more", "parametrization"])
+def test_only_untouched_modules_take_the_backward_sequences(change):
+    """The sequences read the parameters of the sub-modules and never call them: anything hung on one, or put in the place of one,
+    sends the module that contains it (and the block) through the modules themselves."""
+    from fastfold_amd.model.fastnn import Evoformer, _backward
+    blk = Evoformer(256, 128, True, True)
+    mods = [blk.msa.MSARowAttentionWithPairBias, blk.msa.MSAColumnAttention, blk.msa.MSATransition, blk.communication,
+            blk.pair.TriangleMultiplicationOutgoing, blk.pair.TriangleMultiplicationIncoming, blk.pair.TriangleAttentionStartingNode,
+            blk.pair.TriangleAttentionEndingNode, blk.pair.PairTransition]
+    leaf = blk.pair.TriangleAttentionEndingNode.attention.o_linear
+    norm = blk.pair.TriangleAttentionEndingNode.layernorm1
+    assert all(_backward.as_built(m) for m in mods) and _backward.as_built(blk) and _backward.supported(blk)
+    handle = None
+
+    class Adapted(type(leaf)):
+        pass
+    if change == "forward hook":
+        leaf.register_forward_hook(lambda m, a, y: None)
+    elif change == "pre-hook":
+        norm.register_forward_pre_hook(lambda m, a: None)
+    elif change == "backward hook":
+        leaf.register_full_backward_hook(lambda m, gi, go: None)
+    elif change == "global hook":
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda m, a, y: None)
+    elif change == "subclass":
+        leaf.__class__ = Adapted
+    elif change == "own forward":
+        leaf.forward = leaf.forward
+    elif change == "eps":
+        norm.eps = 1e-3
+    elif change == "another module":
+        blk.pair.TriangleAttentionEndingNode.attention.o_linear = torch.nn.Sequential(leaf)
+    elif change == "a part more":
+        leaf.add_module("adapter", torch.nn.Identity())
+    else:
+        torch.nn.utils.parametrizations.orthogonal(leaf)
+    try:
+        assert not _backward.as_built(mods[7]) and not _backward.as_built(blk)
+        assert [_backward.as_built(m) for m in mods[:7] + mods[8:]] == [change != "global hook"] * 8
+    finally:
+        if handle is not None:
+            handle.remove()
+
+
+def test_a_hook_on_the_module_itself_changes_nothing():
+    """It is called as a module, its hooks fire."""
+    from fastfold_amd.model.fastnn import Evoformer, _backward
+    blk = Evoformer(256, 128, True, True)
+    blk.register_forward_hook(lambda m, a, y: None)
+    assert _backward.as_built(blk)
+    blk.msa.MSATransition.register_forward_hook(lambda m, a, y: None)
+    assert _backward.as_built(blk.msa.MSATransition) and not _backward.as_built(blk)
