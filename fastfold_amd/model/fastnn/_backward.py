@@ -65,6 +65,12 @@ def _ln_back(dx, xn, g, ln_mod, ln, dy, x, resid, *, rows, C):
     _lib.layernorm_bwd_rows(dx, xn, g[ln_mod.weight], g[ln_mod.bias], ws, dy, x, ln[0], ln[1], resid, rows=rows, C=C, dtype=x.dtype)
 
 
+def distinct(params):
+    """Whether no parameter serves in two places: ``Grads`` has one piece for each place, and neither the sum of two nor, for a
+    place whose neighbours lie elsewhere, the memory one product writes."""
+    return len({id(p) for p in params}) == len(params)
+
+
 class Grads:
     """Gradients of a module's parameters as pieces of one flat tensor, in the order ``params`` lists them: neighbours in the
     list are neighbours in memory, so one product can write several (the projections of a concatenated operand)."""
@@ -211,7 +217,7 @@ def supported(block):
             and covers_triangle_multiplication(pair.TriangleMultiplicationIncoming)
             and covers_triangle_attention(pair.TriangleAttentionStartingNode)
             and covers_triangle_attention(pair.TriangleAttentionEndingNode)
-            and {id(p) for p in parameters(block)} == {id(p) for p in block.parameters()})
+            and distinct(parameters(block)) and {id(p) for p in parameters(block)} == {id(p) for p in block.parameters()})
 
 
 # -------------------------------------------------------------------------------------------- transition ----
@@ -500,6 +506,9 @@ class _Module(torch.autograd.Function):
 
 
 def _apply(step, inputs, extra, params):
+    """None: the module's operators have to do it."""
+    if not distinct(params):
+        return None
     return _Module.apply(step, (len(inputs), len(extra)), *inputs, *(kept(t, inputs[0]) for t in extra), *params)
 
 

@@ -181,3 +181,25 @@ def test_hooks_and_adapters_are_part_of_the_module(dev, what):
             assert _rel(a, b) < 3e-3
         if what == "adapter":
             assert float(tr.linear2.a.grad.norm()) > 0 and float(tr.linear2.b.grad.norm()) > 0
+
+
+def test_tied_parameters(dev):
+    """One weight in two places of a module and of a block: the gradient is the sum of those of two separate weights."""
+    import copy
+    s, r = 8, 32
+    g = torch.Generator().manual_seed(6)
+    m, z = torch.randn(1, s, r, 256, generator=g).to(dev), torch.randn(1, r, r, 128, generator=g).to(dev)
+    mk, pk = torch.ones(1, s, r, device=dev), torch.ones(1, r, r, device=dev)
+    for call in (lambda b, x, y: (b.communication(x, mk, y),), lambda b, x, y: b(x[0], y[0], mk[0], pk[0])):
+        apart = _block(dev, torch.float32, False)
+        with torch.no_grad():
+            apart.communication.linear_b.weight.copy_(apart.communication.linear_a.weight)
+        tied = copy.deepcopy(apart)
+        tied.communication.linear_b.weight = tied.communication.linear_a.weight
+        grads = []
+        for b in (apart, tied):
+            x, y = m.clone().requires_grad_(), z.clone().requires_grad_()
+            out = call(b, x, y)
+            torch.autograd.backward(out, [torch.ones_like(t) for t in out])
+            grads.append((x.grad, b.communication.linear_a.weight.grad, b.communication.linear_b.weight.grad))
+        assert _rel(grads[1][0], grads[0][0]) < 3e-3 and _rel(grads[1][1], grads[0][1] + grads[0][2]) < 3e-3

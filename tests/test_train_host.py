@@ -206,3 +206,19 @@ def test_a_hook_on_the_module_itself_changes_nothing():
     assert _backward.as_built(blk)
     blk.msa.MSATransition.register_forward_hook(lambda m, a, y: None)
     assert _backward.as_built(blk.msa.MSATransition) and not _backward.as_built(blk)
+
+
+def test_tied_parameters_do_not_take_the_backward_sequences():
+    """One parameter in two places (within a module, between the modules of a block): its two pieces of the flat gradient would
+    neither be added nor lie beside the neighbours one product writes with them."""
+    from fastfold_amd.model.fastnn import Evoformer, _backward
+    blk = Evoformer(256, 128, True, True)
+    blk.pair.TriangleMultiplicationIncoming.layernorm1 = blk.pair.TriangleMultiplicationOutgoing.layernorm1
+    assert not _backward.supported(blk)
+    opm = Evoformer(256, 128, True, True).communication
+    ps = _backward.outer_product_mean_parameters
+    assert _backward.distinct(ps(opm))
+    opm.linear_b.weight = opm.linear_a.weight
+    assert not _backward.distinct(ps(opm))
+    x = torch.zeros(2, requires_grad=True)
+    assert _backward._apply(None, (x,), (), ps(opm)) is None
