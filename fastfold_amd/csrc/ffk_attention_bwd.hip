@@ -578,6 +578,7 @@ extern "C" int ffk_attention_bwd(void* dq, void* dk, void* dv, float* dbias, flo
                      B2, H, Nq, Nk, dq_scale, dk_scale, mq, mk, 0, 0, st
     switch (dtype) {
         case FFK_BF16:
+            // D = 32 with the statistics found here is for callers of the library; this package has them from the forward pass
             return D == 32 ? launch_bwd<bf16_t, 1, true>(FFK_BWD_ARGS)
                            : (D == 64 ? launch_bwd<bf16_t, 2, true>(FFK_BWD_ARGS) : launch_bwd<bf16_t, 4, true>(FFK_BWD_ARGS));
         case FFK_F32:

@@ -359,6 +359,28 @@ def test_fused_attention_core_backward(dev, dtype, tol, b1, b2, h, n, d, use_bia
         assert float(k.grad[dead].abs().max()) == 0.0 and float(v.grad[dead].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 3e-2)])
+@pytest.mark.parametrize("b2,n,use_bias", [(1, 1, True), (3, 33, True), (2, 64, False), (17, 70, True)])
+def test_attention_bwd_entry_at_head_dimension_32(dev, dtype, tol, b2, n, use_bias):
+    """``ffk_attention_bwd`` takes head dimension 32 too (it finds the row statistics itself); inside the package such heads go to
+    ``ffk_attention_bwd_rows``, so this entry of the library has no other caller here."""
+    from fastfold_amd.model.fastnn.kernel import attention_core
+    h, d = 4, 32
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn(1, b2, h, n, d, generator=g).to(dev, dtype) for _ in range(3))
+    bias = torch.randn(1, h, n, n, generator=g).to(dev, dtype) if use_bias else None
+    mask = (torch.rand(1, b2, n, generator=g) > 0.25).to(dev, dtype)
+    mask[..., 0] = 1
+    dout = torch.randn(1, b2, n, h * d, generator=g).to(dev, dtype)
+    out = attention_core.fused_attention_core(q, k, v, mask, bias)
+    got = attention_core._attention_core_backward_wide(q, k, v, mask, bias, out, dout, use_bias)
+    leaves = [t.double().cpu().requires_grad_() for t in (q, k, v)] + ([bias.double().cpu().requires_grad_()] if use_bias else [])
+    _torch_attention_core(*leaves[:3], mask.double().cpu(), leaves[3] if use_bias else None).backward(dout.double().cpu())
+    for name, a, b in zip(("dq", "dk", "dv", "dbias"), got, leaves):
+        if float(b.grad.norm()) > 1e-6:            # one key: the softmax is constant
+            assert _rel(_np(a), b.grad.numpy()) < tol, name
+
+
 def test_fused_attention_core_backward_fully_masked_rows(dev):
     """A batch row whose keys are all masked gives zero output in the forward pass and zero gradients here."""
     from fastfold_amd.model.fastnn.kernel import fused_attention_core
