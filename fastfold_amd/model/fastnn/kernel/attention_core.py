@@ -5,8 +5,8 @@
 
 for q, k, v ``[b1, b2, h, n, d]``, mask ``[b1, b2, n]`` (0/1, over keys) and bias ``[b1, h, n, n]``.
 The logits are never materialised: the operands are re-tiled into the 32x32 MFMA order and handed to
-the flash attention kernel (``ffk_attention_fwd``); the backward pass (``ffk_attention_bwd``) recomputes them the
-same way.  The tuned kernel is the Evoformer's head dim (32); narrower heads (8 and 16, the extra-MSA and template
+the flash attention kernel (``ffk_attention_fwd``, ``ffk_attention_fwd_lse``); the backward pass (``ffk_attention_bwd_rows``, for
+wide heads ``ffk_attention_bwd``) recomputes them the same way.  The tuned kernel is the Evoformer's head dim (32); narrower heads (8 and 16, the extra-MSA and template
 stacks) are zero-padded to 32 channels, which changes neither the scores nor the used output channels; the other
 widths the reference's Triton kernel takes (64 and 128, triton/attention_core.py:142), which no module of the path
 uses, run on a plain one-wave-per-query-tile instantiation that cuts the head into 32-channel parts.
@@ -156,7 +156,7 @@ def _attention_core_backward_wide(q, k, v, mask, bias, out, dout, need_dbias):
 class FusedAttenionCoreFunc(torch.autograd.Function):
     """Name (including its spelling) as in the reference (attention_core.py:34).  The reference's function has no
     backward (training goes through matmul / fused_softmax / matmul there, fastnn/ops.py:310-322); this one has:
-    dq, dk, dv and dbias from ``ffk_attention_bwd``, which recomputes the logits tile by tile."""
+    dq, dk, dv and dbias from ``ffk_attention_bwd_rows`` and ``ffk_attention_bwd``, which recompute the logits tile by tile."""
 
     @staticmethod
     def forward(ctx, q, k, v, mask=None, bias=None):

@@ -3,8 +3,8 @@
 the ending node, outgoing and incoming triangle multiplication and the pair transition at the template
 width (c_t = 64, 4 heads of 16, multiplication width 64, transition factor 2), then a LayerNorm.
 
-The modules are the ones of the Evoformer pair stack at other widths: the attention kernel takes the
-16-wide heads zero-padded to 32 channels, the projections run on the generic kernel variants.
+The modules are the ones of the Evoformer pair stack at other widths: in bf16 the attention kernel takes the
+16-wide heads two to an operand tile, in fp32 zero-padded to 32 channels.
 As for ``Evoformer``, the reference's padding by one residue between blocks is kept as an interface only.
 """
 from typing import Optional

@@ -332,7 +332,7 @@ def _torch_attention_core(q, k, v, mask, bias):
                                                   (1, 3, 4, 77, 64, True), (2, 2, 4, 64, 128, True), (1, 2, 4, 45, 128, False),
                                                   (1, 19, 4, 70, 64, True)])
 def test_fused_attention_core_backward(dev, dtype, tol, b1, b2, h, n, d, use_bias):
-    """dq, dk, dv, dbias of the exported op (``ffk_attention_bwd``: logits recomputed tile by tile) against torch
+    """dq, dk, dv, dbias of the exported op (``ffk_attention_bwd_rows`` up to 32 channels, ``ffk_attention_bwd`` beyond) against torch
     autograd of the reference's formula in float64, with masked keys, a ragged last tile and the narrow heads."""
     from fastfold_amd.model.fastnn.kernel import fused_attention_core
     g = torch.Generator().manual_seed(b2 * n + d)
