@@ -131,7 +131,7 @@ def triangle_attention_parameters(ta):
 
 
 def parameters(block):
-    """Every parameter of the block once, grouped for ``Grads``."""
+    """Every parameter of the block (``as_built``), grouped for ``Grads``."""
     msa, pair = block.msa, block.pair
     return [*row_parameters(msa.MSARowAttentionWithPairBias), *column_parameters(msa.MSAColumnAttention),
             *transition_parameters(msa.MSATransition), *transition_parameters(pair.PairTransition),
@@ -152,31 +152,36 @@ def _dtype_ok(*ts):
 
 @functools.lru_cache(maxsize=None)
 def _anatomy():
-    """The classes the sequences stand for and the names of their sub-modules."""
+    """The classes the sequences stand for, with the names of their sub-modules and parameters."""
     from . import msa, ops, triangle
-    att, tm, ta = {"to_qkv", "gating_linear", "o_linear"}, {"layernorm1", "layernorm2", "left_right_projection", "left_right_gate",
-                                                           "output_gate", "output_projection"}, {"layernorm1", "linear_b", "attention"}
-    return {ops.Linear: set(), ops.LayerNorm: set(), ops.SelfAttention: att,
-            ops.Transition: {"norm", "linear1", "linear2"}, ops.ChunkTransition: {"norm", "linear1", "linear2"},
-            ops.OutProductMean: {"layernormM", "linear_a", "linear_b", "o_linear"},
+    wb, norm_linears = {"weight", "bias"}, {"norm", "linear1", "linear2"}
+    tm = {"layernorm1", "layernorm2", "left_right_projection", "left_right_gate", "output_gate", "output_projection"}, {"output_bias"}
+    ta = {"layernorm1", "linear_b", "attention"}, {"out_bias"}
+    return {ops.Linear: (set(), wb), ops.LayerNorm: (set(), wb),
+            ops.SelfAttention: ({"to_qkv", "gating_linear", "o_linear"}, {"gating_bias"}),
+            ops.Transition: (norm_linears, set()), ops.ChunkTransition: (norm_linears, set()),
+            ops.OutProductMean: ({"layernormM", "linear_a", "linear_b", "o_linear"}, set()),
             ops.AsyncChunkTriangleMultiplicationOutgoing: tm, ops.AsyncChunkTriangleMultiplicationIncoming: tm,
             ops.ChunkTriangleAttentionStartingNode: ta, ops.ChunkTriangleAttentionEndingNode: ta,
-            msa.MSARowAttentionWithPairBias: {"layernormM", "layernormZ", "attention"}, msa.MSAColumnAttention: {"layernormM", "attention"},
-            msa.MSACore: {"MSARowAttentionWithPairBias", "MSAColumnAttention", "MSATransition"},
-            triangle.PairCore: {"TriangleMultiplicationOutgoing", "TriangleMultiplicationIncoming", "TriangleAttentionStartingNode",
-                                "TriangleAttentionEndingNode", "PairTransition"}}
+            msa.MSARowAttentionWithPairBias: ({"layernormM", "layernormZ", "attention"}, {"linear_b_weights", "out_bias"}),
+            msa.MSAColumnAttention: ({"layernormM", "attention"}, set()),
+            msa.MSACore: ({"MSARowAttentionWithPairBias", "MSAColumnAttention", "MSATransition"}, set()),
+            triangle.PairCore: ({"TriangleMultiplicationOutgoing", "TriangleMultiplicationIncoming", "TriangleAttentionStartingNode",
+                                 "TriangleAttentionEndingNode", "PairTransition"}, set())}
 
 
 def _as_built(mod, anatomy):
-    return (mod._modules.keys() == anatomy.get(type(mod)) and "forward" not in mod.__dict__
-            and not (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks)
-            and getattr(mod, "eps", 1e-5) == 1e-5 and all(_as_built(c, anatomy) for c in mod._modules.values()))
+    d = mod.__dict__
+    parts, params = anatomy.get(type(mod), (None, None))
+    return (d["_modules"].keys() == parts and d["_parameters"].keys() == params and "forward" not in d
+            and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"])
+            and d.get("eps", 1e-5) == 1e-5 and all([_as_built(c, anatomy) for c in d["_modules"].values()]))
 
 
 def as_built(mod):
     """Whether everything below ``mod`` is as it was constructed and without hooks."""
     anatomy = _anatomy()
-    return not torch.nn.modules.module._has_any_global_hook() and all(_as_built(c, anatomy) for c in mod._modules.values())
+    return not torch.nn.modules.module._has_any_global_hook() and all([_as_built(c, anatomy) for c in mod._modules.values()])
 
 
 def _covers_attention(att, d):
@@ -207,8 +212,8 @@ def covers_triangle_attention(ta):
     return _covers_attention(ta.attention, ta.d_pair) and ta.n_head <= 4
 
 
-def supported(block):
-    """Whether ``block_backward`` covers this block (if it is ``as_built``)."""
+def supported(block, params):
+    """Whether ``block_backward`` covers this block (if it is ``as_built``); ``params``: its ``parameters``."""
     msa, pair = block.msa, block.pair
     return (covers_row(msa.MSARowAttentionWithPairBias) and covers_column(msa.MSAColumnAttention)
             and covers_transition(msa.MSATransition) and covers_transition(pair.PairTransition)
@@ -217,7 +222,7 @@ def supported(block):
             and covers_triangle_multiplication(pair.TriangleMultiplicationIncoming)
             and covers_triangle_attention(pair.TriangleAttentionStartingNode)
             and covers_triangle_attention(pair.TriangleAttentionEndingNode)
-            and distinct(parameters(block)) and {id(p) for p in parameters(block)} == {id(p) for p in block.parameters()})
+            and distinct(params))
 
 
 # -------------------------------------------------------------------------------------------- transition ----

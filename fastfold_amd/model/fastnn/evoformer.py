@@ -234,9 +234,10 @@ class Evoformer(nn.Module):
         msa_mask, pair_mask = _backward.kept(msa_mask, m), _backward.kept(pair_mask, z)
         drops = self._draw_drops(m, z)
         keys, multipliers = (None, ()) if drops is None else (tuple(drops), tuple(drops.values()))
-        if m.dtype in (torch.bfloat16, torch.float32) and z.dtype == m.dtype and m.shape[-1] == 256 and z.shape[-1] == 128 \
-                and _backward.supported(self):
-            return _BlockGrad.apply(self, keys, m, z, msa_mask, pair_mask, *multipliers, *_backward.parameters(self))
+        if m.dtype in (torch.bfloat16, torch.float32) and z.dtype == m.dtype and m.shape[-1] == 256 and z.shape[-1] == 128:
+            params = _backward.parameters(self)
+            if _backward.supported(self, params):
+                return _BlockGrad.apply(self, keys, m, z, msa_mask, pair_mask, *multipliers, *params)
         anchor = torch.empty(0, device=m.device, requires_grad=True)     # outputs need a gradient even when m and z do not
         return _BlockRecompute.apply(self, keys, anchor, m, z, msa_mask, pair_mask, *multipliers)
 

@@ -154,7 +154,7 @@ def test_a_block_notices_masks_changed_between_the_passes(keys):
 
 
 @pytest.mark.parametrize("change", ["forward hook", "pre-hook", "backward hook", "global hook", "subclass", "own forward", "eps",
-                                    "another module", "a part more", "parametrization"])
+                                    "another module", "a part more", "a parameter more", "parametrization"])
 def test_only_untouched_modules_take_the_backward_sequences(change):
     """The sequences read the parameters of the sub-modules and never call them: anything hung on one, or put in the place of one,
     sends the module that contains it (and the block) through the modules themselves."""
@@ -165,7 +165,9 @@ def test_only_untouched_modules_take_the_backward_sequences(change):
             blk.pair.TriangleAttentionEndingNode, blk.pair.PairTransition]
     leaf = blk.pair.TriangleAttentionEndingNode.attention.o_linear
     norm = blk.pair.TriangleAttentionEndingNode.layernorm1
-    assert all(_backward.as_built(m) for m in mods) and _backward.as_built(blk) and _backward.supported(blk)
+    assert all(_backward.as_built(m) for m in mods) and _backward.as_built(blk)
+    assert _backward.supported(blk, _backward.parameters(blk))
+    assert {id(p) for p in _backward.parameters(blk)} == {id(p) for p in blk.parameters()}
     handle = None
 
     class Adapted(type(leaf)):
@@ -186,6 +188,8 @@ def test_only_untouched_modules_take_the_backward_sequences(change):
         norm.eps = 1e-3
     elif change == "another module":
         blk.pair.TriangleAttentionEndingNode.attention.o_linear = torch.nn.Sequential(leaf)
+    elif change == "a parameter more":
+        leaf.extra = torch.nn.Parameter(torch.zeros(1))
     elif change == "a part more":
         leaf.add_module("adapter", torch.nn.Identity())
     else:
@@ -214,7 +218,7 @@ def test_tied_parameters_do_not_take_the_backward_sequences():
     from fastfold_amd.model.fastnn import Evoformer, _backward
     blk = Evoformer(256, 128, True, True)
     blk.pair.TriangleMultiplicationIncoming.layernorm1 = blk.pair.TriangleMultiplicationOutgoing.layernorm1
-    assert not _backward.supported(blk)
+    assert not _backward.supported(blk, _backward.parameters(blk))
     opm = Evoformer(256, 128, True, True).communication
     ps = _backward.outer_product_mean_parameters
     assert _backward.distinct(ps(opm))
