@@ -43,10 +43,11 @@ def _saved(ctx):
 
 
 class _BlockRecompute(torch.autograd.Function):
-    """One Evoformer block as its own checkpoint: the forward pass runs the fused launches (nothing of it is kept but
-    the two inputs, the masks and the dropout multipliers, which the caller draws so that both passes see the same ones); the
-    backward pass re-runs the block operator by operator with autograd on, the way block checkpointing re-runs it
-    (fastfold/utils/checkpointing.py:55-73; evoformer.py:262-266), and back-propagates through that."""
+    """One Evoformer block as its own checkpoint, for blocks ``_backward.block_backward`` does not cover: the forward pass runs
+    the fused launches (nothing of it is kept but the two inputs, the masks and the dropout multipliers, which the caller draws
+    so that both passes see the same ones); the backward pass re-runs the block module by module with autograd on, the way
+    block checkpointing re-runs it (fastfold/utils/checkpointing.py:55-73; evoformer.py:262-266), and back-propagates through
+    that."""
 
     @staticmethod
     def forward(ctx, block, keys, _grad_anchor, m, z, msa_mask, pair_mask, *multipliers):
@@ -87,9 +88,9 @@ class _BlockGrad(torch.autograd.Function):
 
 class Evoformer(nn.Module):
 
-    # A call that autograd has to see runs the fused forward and re-runs the block in the backward pass
-    # (_BlockRecompute).  False: the forward itself is the operator-by-operator composition, every intermediate is
-    # kept, and the backward pass re-runs nothing.
+    # A call that autograd has to see is its own checkpoint: it runs the fused forward and keeps the block's inputs
+    # (_BlockGrad, _BlockRecompute).  False: the forward is the chain of the block's modules, each of which keeps its own
+    # input, and the backward pass does not re-run the block.
     recompute_in_backward = True
 
     def __init__(self, c_m: int, c_z: int, first_block: bool, last_block: bool, is_multimer: bool = False):
