@@ -1,6 +1,7 @@
 """The differentiable path of the fastnn modules (what benchmark/perf.py's forward + backward mode and
-tests/test_train.py exercise in the reference): a call that autograd has to see runs the reference's own operator
-sequence, with the HIP LayerNorm / attention-core / elementwise kernels and their backward passes.
+tests/test_train.py exercise in the reference): a block that autograd has to see, and each of its modules on its own, runs
+its fused forward and a backward pass of launch sequences, other widths the reference's own operator sequence, with the HIP
+LayerNorm / attention-core / elementwise kernels and their backward passes.
 
 Gradients are checked against autograd through the CPU oracle in float64 (oracle.evoformer_ref, whose forward is
 pinned by the reference's golden vectors).  Parameter gradients are carried from the oracle's layout to the fastnn
@@ -111,11 +112,11 @@ def test_stack_gradients_fp32(dev, nb, s, r, tail):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_stack_gradients_with_checkpointing(dev, dtype):
-    """A training step in train() mode with the dropout probabilities forced to zero (so that it is comparable): the
-    blocks are re-run in the backward pass (blocks_per_ckpt = 1) and give the gradients of the un-checkpointed run -
-    to 1e-4 in fp32 (the pair-bias and LayerNorm parameter gradients are accumulated with floating-point atomics, so
-    not bit for bit); in bf16, where a last-bit difference there becomes a rounding step of 4e-3 further up, both runs
-    are held to the bf16 bound against the float64 oracle instead."""
+    """A training step in train() mode with the dropout probabilities forced to zero (so that it is comparable): blocks
+    that are their own checkpoints (blocks_per_ckpt = 1) give the gradients of the un-checkpointed run, the chain of
+    their modules - to 1e-4 in fp32 (the modules on their own round their outputs at other places of the stream); in
+    bf16, where such a difference is a rounding step of 4e-3 further up, both runs are held to the bf16 bound against
+    the float64 oracle instead."""
     nb, s, r = 2, 16, 48
     model = _oracle(32, nb)
     m, z, mm, pm = synth_inputs(32, s, r, mask_tail_frac=0.1)
@@ -312,10 +313,9 @@ def test_block_forward_backward_at_headline_size(dev):
 
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 3e-5), (torch.bfloat16, 2e-2)])
 def test_block_recompute_same_dropout_in_both_passes(dev, dtype, tol):
-    """A training-mode block under autograd runs the fused launches forward and re-runs itself operator by operator
-    in the backward pass (``_BlockRecompute``): with dropout active both passes must apply the SAME multipliers.  The
-    multipliers of one call are captured, and the fused forward is compared with the operator-by-operator block run
-    on them; the gradients of the call are those of that run."""
+    """A training-mode block under autograd is its own checkpoint: with dropout active its forward and its backward pass
+    must apply the SAME multipliers.  The multipliers of one call are captured, and the block is compared with the chain
+    of its modules run on them; the gradients of the call are those of that run."""
     from fastfold_amd.model.fastnn import Evoformer
     torch.manual_seed(4)
     s, r = 12, 40
@@ -350,7 +350,7 @@ def test_block_recompute_same_dropout_in_both_passes(dev, dtype, tol):
     mo2, zo2 = blk._core_train(m2.unsqueeze(0), z2.unsqueeze(0), mm.unsqueeze(0), pm.unsqueeze(0), drops=d)
     assert _rel(mo, mo2.squeeze(0)) <= tol and _rel(zo, zo2.squeeze(0)) <= tol, (_rel(mo, mo2.squeeze(0)), _rel(zo, zo2.squeeze(0)))
     (zo2.squeeze(0).float() * cot.float()).sum().backward()
-    gtol = 1e-4 if dtype == torch.float32 else 5e-2      # atomics in the parameter gradients; bf16: one rounding step
+    gtol = 1e-4 if dtype == torch.float32 else 5e-2      # sums in another order; bf16: one rounding step
     assert _rel(got[0], m2.grad) <= gtol and _rel(got[1], z2.grad) <= gtol
     assert len(pg) >= 70
     for n, p in blk.named_parameters():

@@ -1,7 +1,7 @@
 """The differentiable path of the modules around the Evoformer stack: extra-MSA stack (head-dim-8 row attention,
 global column attention), template pair stack, template point-wise attention, input and recycling embedders.
 
-As for the Evoformer stack, a call that autograd has to see runs the reference's operator sequence, and gradients
+A call that autograd has to see runs the reference's operator sequence here, and gradients
 are checked against autograd through the CPU oracle in float64.  Parameter gradients travel from the oracle's
 layout to the fastnn layout through the weight re-layout itself (it only copies and concatenates).
 
