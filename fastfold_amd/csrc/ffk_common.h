@@ -24,6 +24,7 @@ int ffk_fail(int code, const char* fmt, ...);
 
 int ffk_linear_slab_launch(const ffk_linear_desc* d, hipStream_t st);   // ffk_linear_slab.hip
 int ffk_bgemm_big_try(const ffk_bgemm_desc* d, hipStream_t st, int* status);    // ffk_bgemm_big.hip
+int ffk_linear_rm_try(const ffk_linear_desc* d, hipStream_t st, int* status);   // ffk_linear_rm.hip
 int ffk_linear_ws_try(const ffk_linear_desc* d, hipStream_t st, int* status);   // ffk_linear_ws.hip
 int ffk_linear_ws32_try(const ffk_linear_desc* d, hipStream_t st, int* status); // ffk_linear_ws32.hip
 

@@ -579,6 +579,7 @@ extern "C" int ffk_fused_linear(const ffk_linear_desc* d, void* stream) {
     }
     {
         int status = FFK_OK;
+        if (ffk_linear_rm_try(d, (hipStream_t)stream, &status)) return status;
         if (ffk_linear_ws_try(d, (hipStream_t)stream, &status)) return status;
         if (ffk_linear_ws32_try(d, (hipStream_t)stream, &status)) return status;
     }

@@ -582,3 +582,46 @@ def test_weights_stationary_unit_shares(dev, K, N, M):
     _lib.fused_linear(x, wp, tiles, M=M, K=K, ln=ln)
     ref = F.linear(F.layer_norm(x.float(), (K,), ln[0].float(), ln[1].float()), w.float(), b.float())
     assert torch.isfinite(out).all() and float((out.float() - ref).norm() / ref.norm()) < 6e-3
+
+
+@pytest.mark.parametrize("K", [64, 128, 256])
+@pytest.mark.parametrize("B2,N", [(1, 32), (3, 96), (70, 96), (300, 128), (5, 48), (9, 33), (1001, 33)])
+def test_row_major_layouts(dev, K, B2, N):
+    """Every epilogue of the row-major kernel from one row group to several rounds of its largest slabs, with groups that end in
+    the middle of an outer step (N = 48, 33), against the LDS-staged kernels: the same products, rounded once (2^-8)."""
+    from fastfold_amd import _lib
+    bf = torch.bfloat16
+    M, NT = B2 * N, (N + 31) // 32
+    g = torch.Generator().manual_seed(K + M)
+
+    def rnd(*s):
+        return torch.randn(*s, generator=g).to(dev, bf)
+    x, w, b = rnd(M, K), rnd(640, K) / K ** 0.5, rnd(640)
+    ln = (1 + 0.1 * rnd(K), 0.1 * rnd(K))
+    mask, gate = (torch.rand(B2, N, generator=g) > 0.2).to(dev, bf), rnd(17, 128)
+    resid, tail = rnd(M, 128), torch.randint(-128, 128, (M, 128), generator=g).to(dev, torch.int8)
+    resid[resid == 0] = 1.0                              # (0, negative tail) is no value: the pair would be below zero
+    got = []
+    for staged in (False, True):
+        bp = [b.data_ptr() + 256 * i for i in range(5)]
+        outs = [torch.zeros(B2, 4, NT, 1024, device=dev, dtype=bf) for _ in range(4)]
+        outs += [torch.zeros(M, 256, device=dev, dtype=bf), resid.clone(), tail.clone(), torch.zeros(M, 128, device=dev, dtype=bf)]
+        rows = [_lib.make_tile(outs[4].data_ptr() + 256 * i, bias=bp[i], act=_lib.FFK_ACT_RELU, inner=M, s_i=256, ncols=(128, 104)[i]) for i in range(2)]
+        if N % 32 == 0:
+            tk = dict(inner=N, s_o=4 * NT * 1024, s_h=NT * 1024)
+            rows += [_lib.make_tile(outs[0], kind=_lib.FFK_TILE_V, **tk), _lib.make_tile(outs[1], kind=_lib.FFK_TILE_QK, scale=0.25, **tk),
+                     _lib.make_tile(outs[2], kind=_lib.FFK_TILE_ACC, bias=bp[4], act=_lib.FFK_ACT_SIGMOID, **tk)]
+        _lib.fused_linear(x, w, rows, M=M, K=K, a_inner=N, a_so=N * K, a_si=K, ln=ln, staged=staged)
+        # residual with a tail in place, rows of the tensor taken column by column, a multiplier shared by every 17th row
+        _lib.fused_linear(x, w, [_lib.make_tile(outs[5], bias=bp[0], resid=outs[5], xtail=outs[6], gate=gate, gate_ld=128, gate_rows=17,
+                                                inner=N, s_o=128, s_i=B2 * 128)], M=M, K=K, staged=staged)
+        _lib.fused_linear(x, w, [_lib.make_tile(outs[7], resid=resid, inner=N, s_o=128, s_i=B2 * 128, ncols=72)], M=M, K=K, staged=staged)
+        if N % 16 == 0 and M % 16 == 0 and K != 256:
+            cm = torch.zeros(64, B2 * N + 16, device=dev, dtype=bf)
+            _lib.fused_linear(x, w, [_lib.make_tile(cm, glu=1, ncols=64, bias=bp[1], inner=N, s_o=N, s_i=1, s_h=32 * cm.shape[1], s_d=cm.shape[1],
+                                                    rowmask=mask, m_so=N, m_si=1)], M=M, K=K, ln=ln, staged=staged)
+            outs.append(cm)
+        got.append(outs)
+    got[0][6], got[1][6] = [((o[5].view(torch.int16).int() << 16) + (o[6].int() << 8)).view(torch.float32) for o in got]    # 24-bit values
+    for i, (a, c) in enumerate(zip(*got)):
+        assert torch.isfinite(a.float()).all() and _rel(_np(a), _np(c)) < 2 ** -7, i
