@@ -625,3 +625,42 @@ def test_row_major_layouts(dev, K, B2, N):
     got[0][6], got[1][6] = [((o[5].view(torch.int16).int() << 16) + (o[6].int() << 8)).view(torch.float32) for o in got]    # 24-bit values
     for i, (a, c) in enumerate(zip(*got)):
         assert torch.isfinite(a.float()).all() and _rel(_np(a), _np(c)) < 2 ** -7, i
+
+
+@pytest.mark.parametrize("K", [128, 256])
+@pytest.mark.parametrize("B,N", [(1, 1), (3, 37), (64, 64), (131, 96), (260, 128)])
+def test_fp32_row_layouts(dev, K, B, N):
+    """fp32 launches from one row to both sides of the persistent layout, row groups that end in the middle of an outer step and
+    channel-major operands and outputs of any extent, against the LDS-staged kernel (32-bit sums in another order: 1e-5)."""
+    from fastfold_amd import _lib
+    M = B * N
+    g = torch.Generator().manual_seed(K + M)
+
+    def rnd(*s):
+        return torch.randn(*s, generator=g).to(dev)
+    x, w, b = rnd(M, K), rnd(512, K) / K ** 0.5, rnd(512)
+    ln = (1 + 0.1 * rnd(K), 0.1 * rnd(K))
+    mask, gate, resid = (torch.rand(B, N, generator=g) > 0.2).to(dev, torch.float32), rnd(M, 128), rnd(M, 128)
+    kp = (N + 3) // 4 * 4
+    got = []
+    for staged in (False, True):
+        bp = [b.data_ptr() + 512 * i for i in range(4)]
+        plain, out, cm = torch.zeros(M, 512, device=dev), torch.zeros(M, 128, device=dev), torch.zeros(64, B * kp + 16, device=dev)
+        _lib.fused_linear(x, w, [_lib.make_tile(plain.data_ptr() + 512 * i, bias=bp[i], act=_lib.FFK_ACT_RELU, inner=M, s_i=512, ncols=(128, 128, 128, 36)[i])
+                                 for i in range(4)], M=M, K=K, ln=ln, staged=staged)
+        _lib.fused_linear(x, w, [_lib.make_tile(out, bias=bp[0], gate=gate, gate_ld=128, resid=resid, inner=N, s_o=128, s_i=B * 128)], M=M, K=K,
+                          a_inner=N, a_so=N * K, a_si=K, ln=ln, staged=staged)
+        outs = [plain, out]
+        if K == 128:
+            _lib.fused_linear(x, w, [_lib.make_tile(cm, glu=1, ncols=64, bias=bp[1], inner=N, s_o=kp, s_i=1, s_h=32 * cm.shape[1], s_d=cm.shape[1],
+                                                    rowmask=mask, m_so=N, m_si=1)], M=M, K=K, ln=ln, staged=staged)
+            xt = torch.zeros(K, B * kp + 4, device=dev)
+            for i in range(B):
+                xt[:, i * kp:i * kp + N] = x[i * N:(i + 1) * N].t()
+            back = torch.zeros(M, 128, device=dev)
+            _lib.fused_linear(xt, w, [_lib.make_tile(back, bias=bp[2], gate=gate, gate_ld=128, resid=resid, inner=M, s_i=128)], M=M, K=K,
+                              a_inner=N, a_so=kp, a_si=1, a_chanmajor=True, a_cs=xt.shape[1], ln=ln, staged=staged)
+            outs += [cm, back]
+        got.append(outs)
+    for i, (a, c) in enumerate(zip(*got)):
+        assert torch.isfinite(a).all() and float((a - c).abs().max()) <= 1e-5 * float(c.abs().max()), i
