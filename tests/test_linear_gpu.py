@@ -664,3 +664,29 @@ def test_fp32_row_layouts(dev, K, B, N):
         got.append(outs)
     for i, (a, c) in enumerate(zip(*got)):
         assert torch.isfinite(a).all() and float((a - c).abs().max()) <= 1e-5 * float(c.abs().max()), i
+
+
+@pytest.mark.parametrize("C", [128, 256])
+def test_transition_kernels_agree(dev, C):
+    """Rows of a launch get the same bits whichever kernel and workgroup size the row count selects (and so a piece of a
+    tensor those of the whole), with ragged last workgroups and residual tails, in place."""
+    from fastfold_amd import _lib
+    g = torch.Generator().manual_seed(C)
+
+    def rnd(*s):
+        return torch.randn(*s, generator=g).to(dev, torch.bfloat16)
+    M, H = 49300, 4 * C
+    x, tail = rnd(M, C), torch.randint(-128, 128, (M, C), generator=g).to(dev, torch.int8)
+    ln, w1, b1, w2, b2 = (1 + 0.1 * rnd(C), 0.1 * rnd(C)), rnd(H, C) / C ** 0.5, rnd(H), rnd(C, H) / H ** 0.5, rnd(C)
+
+    def run(n):
+        y, t = x[:n].clone(), tail[:n].clone()
+        _lib.transition_fused(y, y, ln[0], ln[1], w1, b1, w2, b2, M=n, C=C, hidden=H, xtail=t)
+        return y, t
+    whole = run(M)
+    h = torch.relu(torch.nn.functional.linear(torch.nn.functional.layer_norm(x.float(), (C,), ln[0].float(), ln[1].float()), w1.float(), b1.float()))
+    ref = x.float() + torch.nn.functional.linear(h, w2.float(), b2.float())
+    assert float((whole[0].float() - ref).norm() / ref.norm()) < 6e-3
+    for n in (1, 63, 64, 65 * 64 - 5, 64 * 256, 64 * 256 + 1, 128 * 256, 128 * 256 + 1):
+        y, t = run(n)
+        assert torch.equal(y, whole[0][:n]) and torch.equal(t, whole[1][:n]), n
