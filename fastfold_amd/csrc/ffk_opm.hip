@@ -3,7 +3,7 @@
 //     O_ij[d, e]   = sum_s a[s, i, d] * b[s, j, e]                       (32 x 32 per residue pair)
 // without ever writing the [r, r, 1024] outer product to memory.
 //
-// A workgroup (8 wavefronts) owns TI i x 32 j residue pairs, TI = 8 or 4, and walks the 32 values of e in 16
+// A workgroup owns TI i x 32 j residue pairs, TI = 8 or 4 (8 wavefronts) or 2 (4), and walks the 32 values of e in 16
 // chunks of two.  Per chunk (TI = 8):
 //   phase A  (outer product)  wave w multiplies its own i = i0 + w: rows (d) x columns (j, e in chunk),
 //            K = s.  Its a-fragments stay in registers for the whole tile; the b rows of the chunk come
@@ -13,14 +13,19 @@
 //            wave owns 2 x 2 of them; accumulators live in registers across all chunks.
 // b and W2 chunks arrive by direct global -> LDS loads (XOR-swizzled unpadded rows) one iteration
 // ahead; phase B of chunk q - 1 and phase A of chunk q run between the same pair of barriers, so there
-// is one barrier per chunk.  With TI = 4 two waves share an i (one column tile each) and a wave owns 1 x 2 output tiles: half
-// the work per chunk and twice the workgroups, for launches that leave CUs empty (see ffk_opm_fused).  The weight is expected pre-permuted to k2 = e * 32 + d order.
+// is one barrier per chunk.  With TI = 4 or 2 two waves share an i (one column tile each) and a wave owns 1 x 2 output tiles: less
+// work per chunk and more workgroups, for launches that leave CUs empty (see ffk_opm_fused).  The weight is expected pre-permuted
+// to k2 = e * 32 + d order.
+// What bounds it is the chain of a step: LDS reads, products, rounding, LDS writes, barrier (matrix pipe busy 45 % at r = 1 024
+// when each of them waited for the one before).  Operands requested a group ahead, the outer products rounded between the products
+// of the projection, and loads to LDS issued where the compiler does not order LDS reads behind them: r = 1 024, 128 sequences
+// 576 -> 536 us, 416 104 -> 99 us, 256 39.0 -> 37.0 us.
 #include "ffk_common.h"
+#include <type_traits>
 
 namespace {
 
 typedef bf16_t T;
-constexpr int OP_THREADS = 512;
 constexpr int OP_TJ = 32;                        // pairs per workgroup: TI i x 32 j
 constexpr int OP_EC = 2;                         // values of e per chunk
 constexpr int OP_NCHUNK = 32 / OP_EC;            // 16
@@ -30,19 +35,15 @@ constexpr int OP_W2SLOT = 128 * OP_K2C * 2;      // W2 chunk: 128 rows of 128 by
 
 __device__ __forceinline__ int op_tau(int i) { return ((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3); }
 
-__device__ __forceinline__ void op_load_lds(const T* src, unsigned char* dst_wave) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                     (__attribute__((address_space(3))) void*)dst_wave, 16, 0, 0);
-}
-
-template <int KS1, int OP_TI>   // MFMA K steps of the outer product: spad / 16 (4 or 8)
-__global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict__ out, const T* __restrict__ resid, int8_t* __restrict__ xtail,
+template <int KS1, int OP_TI, int WAVES>   // KS1: MFMA K steps of the outer product, spad / 16 (4 or 8)
+__global__ __launch_bounds__(64 * WAVES, WAVES / 4) void opm_fused_kernel(T* __restrict__ out, const T* __restrict__ resid, int8_t* __restrict__ xtail,
                                                                  const T* __restrict__ at, const T* __restrict__ bt,
                                                                  const T* __restrict__ w2p, const T* __restrict__ bias,
                                                                  const float* __restrict__ norm, int r, float eps) {
     typedef Mma<T> MM;
     constexpr int OP_A2 = OP_TI * OP_TJ * OP_PA;         // one A2 buffer
-    constexpr int MT = OP_TI / 4, WI = 8 / OP_TI, NCT = 2 / WI;    // m-tiles per wave (phase B), waves per i, column tiles per wave (phase A)
+    constexpr int OP_THREADS = 64 * WAVES, WM = WAVES / 2, WLD = OP_W2SLOT / 16 / OP_THREADS;
+    constexpr int MT = OP_TI / WM, WI = WAVES / OP_TI, NCT = 2 / WI;    // m-tiles per wave (phase B), waves per i, column tiles per wave (phase A)
     constexpr int SPAD = KS1 * 16;                       // K of the outer product
     constexpr int BROW = SPAD * 2;                       // bytes per b row (128 or 256)
     constexpr int BCOLS = BROW / 16;                     // 16-byte columns per b row (8 or 16)
@@ -78,23 +79,30 @@ __global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict_
         bsrc[i] = bt + ((long)(j0 + (rho >> 1)) * 32 + (rho & 1)) * SPAD + ((c ^ swz) * 8);
     }
     // W2 chunk: LDS row rho (0..127) holds weight row 32 * (rho / 32) + tau(rho % 32); 8 columns of 16 bytes
-    const T* wsrc[2];
+    const T* wsrc[WLD];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < WLD; ++i) {
         const int v = i * OP_THREADS + tid, rho = v >> 3, c = v & 7;
         wsrc[i] = w2p + (long)((rho & ~31) + op_tau(rho & 31)) * 1024 + ((c ^ ((rho >> 1) & 7)) * 8);
     }
-    auto fetch = [&](int q) {
-        unsigned char* bs = s_b + (q & 1) * BSLOT + wave * 1024;
+    const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
+    // asm: with loads to LDS that it knows of the compiler waits for every LDS read of the wave in front of each group of products
+    auto dma = [&](const T* src, unsigned dst) __attribute__((always_inline)) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_base + dst) : "memory", "m0");
+#pragma clang diagnostic pop
+    };
+    auto fetch = [&](int q) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < BLD; ++i) op_load_lds(bsrc[i] + (long)q * OP_EC * SPAD, bs + i * (OP_THREADS * 16));
-        unsigned char* ws = s_w2 + (q % 3) * OP_W2SLOT + wave * 1024;
+        for (int i = 0; i < BLD; ++i)
+            dma(bsrc[i] + (long)q * OP_EC * SPAD, 2 * OP_A2 + 3 * OP_W2SLOT + (q & 1) * BSLOT + (i * OP_THREADS + wave * 64) * 16);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) op_load_lds(wsrc[i] + q * OP_K2C, ws + i * (OP_THREADS * 16));
+        for (int i = 0; i < WLD; ++i) dma(wsrc[i] + q * OP_K2C, 2 * OP_A2 + (q % 3) * OP_W2SLOT + (i * OP_THREADS + wave * 64) * 16);
     };
 
-    // ---- phase B roles: m-tiles MT * (wave % 4) .., c-tiles 2 * (wave / 4) + {0, 1} ----
-    const int mt0 = MT * (wave & 3), ct0 = 2 * (wave >> 2);
+    // ---- phase B roles: m-tiles MT * (wave % WM) .., c-tiles 2 * (wave / WM) + {0, 1} ----
+    const int mt0 = MT * (wave % WM), ct0 = 2 * (wave / WM);
     f32x16 acc2[MT][2];   // [m][c]
 #pragma unroll
     for (int a = 0; a < MT; ++a)
@@ -125,10 +133,17 @@ __global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict_
     u32x4 e_rv[MT][2][2], e_tv[MT][2];
     float e_norm[MT];
     const int pf_q = 2 + (int)((blockIdx.x >> 3) % 12u);   // spread over the chunks: the workgroups of a launch run in step
-    fetch(0);
-    for (int q = 0; q <= OP_NCHUNK; ++q) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");    // chunk q has landed (this wave's part)
+    // A step: the outer products of chunk q (A) and the projection of chunk q - 1 (B).  All operands come through one ring of two
+    // groups of up to four fragments, requested a group ahead; the outer products are rounded and written between the products of
+    // the projection, so that neither an LDS latency nor the rounding stands alone between two barriers.
+    constexpr int AG = KS1 / 4, NA = NCT * AG;           // groups of the outer product
+    bf16x8 ring[2][4];
+    auto step = [&](int q, auto do_a, auto do_b) __attribute__((always_inline)) {
+        constexpr bool A = decltype(do_a)::value, B = decltype(do_b)::value;
+        constexpr int G0 = A ? 0 : NA, G1 = B ? NA + 4 : NA;
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");    // chunk q has landed (this wave's part), its A2 rows are written
         __builtin_amdgcn_s_barrier();                        // ... everyone's; A2 of chunk q - 1 is complete
+        asm volatile("" ::: "memory");
         if (q + 1 < OP_NCHUNK) fetch(q + 1);
         if (q == pf_q) {
 #pragma unroll
@@ -144,45 +159,73 @@ __global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict_
                 }
             }
         }
-        if (q > 0) {
-            // ---- phase B of chunk q - 1 ----
-            const unsigned char* a2 = s_a2 + ((q - 1) & 1) * OP_A2;
-            const unsigned char* w2 = s_w2 + ((q - 1) % 3) * OP_W2SLOT;
+        const unsigned char* bs = s_b + (q & 1) * BSLOT + ctw * 32 * BROW;
+        const unsigned char* a2 = s_a2 + ((q + 1) & 1) * OP_A2 + mt0 * 32 * OP_PA + a2r;
+        const unsigned char* w2 = s_w2 + ((q + 2) % 3) * OP_W2SLOT + ct0 * 32 * 128;
+        unsigned char* a2n = s_a2 + (q & 1) * OP_A2 + a2w + ctw * 16 * OP_PA;
+        f32x16 o[NCT];
+        auto request = [&](int g) __attribute__((always_inline)) {
+            bf16x8* f = ring[g & 1];
+            if (g < NA) {
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                bf16x8 fa[MT], fw[2];
+                for (int i = 0; i < 4; ++i) f[i] = *reinterpret_cast<const bf16x8*>(bs + g / AG * 32 * BROW + boff[g % AG * 4 + i]);
+            } else {
 #pragma unroll
-                for (int m = 0; m < MT; ++m) fa[m] = *reinterpret_cast<const bf16x8*>(a2 + (mt0 + m) * 32 * OP_PA + a2r + ks * 32);
+                for (int m = 0; m < MT; ++m) f[m] = *reinterpret_cast<const bf16x8*>(a2 + m * 32 * OP_PA + (g - NA) * 32);
 #pragma unroll
-                for (int c = 0; c < 2; ++c) fw[c] = *reinterpret_cast<const bf16x8*>(w2 + (ct0 + c) * 32 * 128 + woff[ks]);
+                for (int c = 0; c < 2; ++c) f[2 + c] = *reinterpret_cast<const bf16x8*>(w2 + c * 32 * 128 + woff[g - NA]);
+            }
+        };
+        // eight values of a column tile's result
+        auto hand_over = [&](int piece) __attribute__((always_inline)) {
+            typedef float f32x2 __attribute__((ext_vector_type(2)));
+            typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+            u32x4 y;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const f32x2 pr = {o[piece >> 1][8 * (piece & 1) + 2 * t], o[piece >> 1][8 * (piece & 1) + 2 * t + 1]};
+                y[t] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pr, bf16x2));
+            }
+            *reinterpret_cast<u32x4*>(a2n + (piece >> 1) * 16 * OP_PA + (piece & 1) * 16) = y;
+        };
+        if (A) {
+#pragma unroll
+            for (int c = 0; c < NCT; ++c)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) o[c][v] = 0.0f;
+        }
+        request(G0);
+#pragma unroll
+        for (int g = G0; g < G1; ++g) {
+            if (g + 1 < G1) request(g + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            const bf16x8* f = ring[g & 1];
+            if (g < NA) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) MM::mma(o[g / AG], af[g % AG * 4 + i], f[i]);
+            } else {
+                if (A && g - NA < 2 * NCT) hand_over(g - NA);
 #pragma unroll
                 for (int m = 0; m < MT; ++m)
 #pragma unroll
-                    for (int c = 0; c < 2; ++c) MM::mma(acc2[m][c], fw[c], fa[m]);
+                    for (int c = 0; c < 2; ++c) MM::mma(acc2[m][c], f[2 + c], f[m]);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if (q < OP_NCHUNK) {
-            // ---- phase A of chunk q: O[d, (j, e)] for this wave's i, two column tiles of 16 j x 2 e ----
-            const unsigned char* bs = s_b + (q & 1) * BSLOT;
-            unsigned char* a2 = s_a2 + (q & 1) * OP_A2;
+        if (A && !B) {
 #pragma unroll
-            for (int c1 = 0; c1 < NCT; ++c1) {
-                const int ct = ctw + c1;
-                f32x16 o;
-#pragma unroll
-                for (int v = 0; v < 16; ++v) o[v] = 0.0f;
-#pragma unroll
-                for (int ks = 0; ks < KS1; ++ks)
-                    MM::mma(o, af[ks], *reinterpret_cast<const bf16x8*>(bs + ct * 32 * BROW + boff[ks]));
-                T y[16];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) y[v] = (T)o[v];
-                unsigned char* p = a2 + a2w + ct * 16 * OP_PA;
-                *reinterpret_cast<u32x4*>(p) = *reinterpret_cast<const u32x4*>(&y[0]);
-                *reinterpret_cast<u32x4*>(p + 16) = *reinterpret_cast<const u32x4*>(&y[8]);
-            }
+            for (int p = 0; p < 2 * NCT; ++p) hand_over(p);
         }
-    }
+    };
+    typedef std::integral_constant<bool, true> Yes;
+    typedef std::integral_constant<bool, false> No;
+    fetch(0);
+    step(0, Yes(), No());
+    // Kernel arguments that only the epilogue reads would count as outstanding at the head of the loop, where a wait for a fragment
+    // would then be one for every LDS read of the wave
+    __builtin_amdgcn_s_waitcnt(0xc07f);                  // lgkmcnt(0)
+    for (int q = 1; q < OP_NCHUNK; ++q) step(q, Yes(), Yes());
+    step(OP_NCHUNK, No(), Yes());
 
     // ---- epilogue: lane = pair, registers = 16 consecutive channels ----
 #pragma unroll
@@ -222,17 +265,17 @@ __global__ __launch_bounds__(OP_THREADS, 2) void opm_fused_kernel(T* __restrict_
     }
 }
 
-template <int KS1, int OP_TI>
+template <int KS1, int OP_TI, int WAVES>
 int opm_launch(T* out, const T* resid, int8_t* xtail, const T* at, const T* bt, const T* w2p, const T* bias, const float* norm, int r,
                float eps, hipStream_t st) {
     const size_t smem = 2 * (size_t)(OP_TI * OP_TJ * OP_PA) + 3 * OP_W2SLOT + 2 * (size_t)(OP_TJ * OP_EC * KS1 * 32);
     static FfkLdsReservation lds_reserved;
     {
-        const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)opm_fused_kernel<KS1, OP_TI>, smem, "ffk_opm_fused");
+        const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)opm_fused_kernel<KS1, OP_TI, WAVES>, smem, "ffk_opm_fused");
         if (rc_lds != FFK_OK) return rc_lds;
     }
     const unsigned grid = (unsigned)((r / OP_TI) * (r / OP_TJ));
-    opm_fused_kernel<KS1, OP_TI><<<grid, OP_THREADS, smem, st>>>(out, resid, xtail, at, bt, w2p, bias, norm, r, eps);
+    opm_fused_kernel<KS1, OP_TI, WAVES><<<grid, 64 * WAVES, smem, st>>>(out, resid, xtail, at, bt, w2p, bias, norm, r, eps);
     return ffk_check_launch("ffk_opm_fused");
 }
 
@@ -248,11 +291,14 @@ extern "C" int ffk_opm_fused(void* out, const void* resid, void* xtail, const vo
                     ffk_aligned16(bias) && ffk_aligned16(xtail),
                 FFK_ERR_ALIGN, "ffk_opm_fused: buffers must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
-    // Four i per workgroup while these give no CU a second one (a workgroup's time is mostly its 17 barriers: r = 96, 128
-    // sequences: 36 workgroups of eight 31.4 us, 72 of four 21.3 us; r = 160: 33.9 and 24.0 us; r = 192: 35.2 and 44.0 us).
-    const bool small = (r / 4) * (r / OP_TJ) <= 256;
-#define FFK_OPM(KS1, TI) opm_launch<KS1, TI>((T*)out, (const T*)resid, (int8_t*)xtail, (const T*)a_t, (const T*)b_t, (const T*)w2p, (const T*)bias, norm, (int)r, eps, st)
-    if (spad == 128) return small ? FFK_OPM(8, 4) : FFK_OPM(8, 8);
-    return small ? FFK_OPM(4, 4) : FFK_OPM(4, 8);
+    // Two i and four waves per workgroup while no CU has two of these, then four i and eight waves, then eight i: a workgroup's time is
+    // mostly its 17 steps (0.65 us each with one wave per SIMD, 0.9 with two, 1.4 with twice the rows), so more and smaller workgroups
+    // win until they come in rounds.  128 sequences, TI = 2 / 4 / 8: r = 96 16.5 / 19.6 / 28.6 us, 128 17.9 / 20.9 / 29.3, 160
+    // 30.9 / 22.3 / 29.9, 192 45.2 / 38.6 / 30.5, 256 61 / 42.8 / 36.9.
+    const long tj = r / OP_TJ;
+    const int ti = (r / 2) * tj <= 256 ? 2 : (r / 4) * tj <= 256 ? 4 : 8;
+#define FFK_OPM(KS1, TI, W) opm_launch<KS1, TI, W>((T*)out, (const T*)resid, (int8_t*)xtail, (const T*)a_t, (const T*)b_t, (const T*)w2p, (const T*)bias, norm, (int)r, eps, st)
+    if (spad == 128) return ti == 2 ? FFK_OPM(8, 2, 4) : ti == 4 ? FFK_OPM(8, 4, 8) : FFK_OPM(8, 8, 8);
+    return ti == 2 ? FFK_OPM(4, 2, 4) : ti == 4 ? FFK_OPM(4, 4, 8) : FFK_OPM(4, 8, 8);
 #undef FFK_OPM
 }

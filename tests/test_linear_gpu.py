@@ -690,3 +690,32 @@ def test_transition_kernels_agree(dev, C):
     for n in (1, 63, 64, 65 * 64 - 5, 64 * 256, 64 * 256 + 1, 128 * 256, 128 * 256 + 1):
         y, t = run(n)
         assert torch.equal(y, whole[0][:n]) and torch.equal(t, whole[1][:n]), n
+
+
+@pytest.mark.parametrize("s", [64, 128])
+def test_opm_workgroup_sizes_agree(dev, s):
+    """A residue pair's update has the same bits whichever number of residues per workgroup the extent selects (two up to 128, four
+    at 160, eight from 192), with and without a tail."""
+    from fastfold_amd import _lib
+    g = torch.Generator().manual_seed(s)
+
+    def rnd(*sh):
+        return torch.randn(*sh, generator=g).to(dev, torch.bfloat16)
+    R = 192
+    z, ab, w, b = rnd(R, R, 128), rnd(2, R * 32, s), rnd(128, 1024) * 0.05, rnd(128)
+    nrm, tail = torch.rand(R, R, generator=g).to(dev) * s, torch.randint(-128, 128, (R, R, 128), generator=g).to(dev, torch.int8)
+
+    def run(r, xt):
+        zz, t = z[:r, :r].contiguous(), tail[:r, :r].clone(memory_format=torch.contiguous_format) if xt else None
+        out = torch.empty_like(zz)
+        _lib.opm_fused(out, zz, ab[0], ab[1], w, b, nrm[:r, :r].contiguous(), r=r, spad=s, eps=1e-3, xtail=t)
+        return out, t
+    for xt in (False, True):
+        whole = run(R, xt)
+        a, bb = (ab[i].float().view(R, 32, s) for i in range(2))
+        o = torch.einsum("ids,jes->ijed", a[:40].cpu(), bb[:40].cpu()).reshape(40, 40, 1024).to(torch.bfloat16).float()
+        ref = z[:40, :40].float().cpu() + (o @ w.float().cpu().t() + b.float().cpu()) / (nrm[:40, :40, None].cpu() + 1e-3)
+        assert float((whole[0][:40, :40].float().cpu() - ref).norm() / ref.norm()) < 6e-3
+        for r in (32, 128, 160):
+            y, t = run(r, xt)
+            assert torch.equal(y, whole[0][:r, :r]) and (not xt or torch.equal(t, whole[1][:r, :r])), (r, xt)
