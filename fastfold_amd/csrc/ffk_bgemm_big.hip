@@ -38,6 +38,19 @@ __device__ __forceinline__ void bg_load_lds(const T* src, unsigned char* dst_wav
                                      (__attribute__((address_space(3))) void*)dst_wave, 16, 0, 0);
 }
 
+// Tile of item idx of a batch, in bands of BG_BAND tiles along m, n outside m within a band.  Batched launches run a batch of large
+// matrices behind one L2, 32 tiles at a time: six by five or so of them read 11 panels of 256 rows, 16 by 2 (m first over all of
+// 4 096 rows) read 18, from memory, 2.5 TB/s of misses.  4 096 x 4 096 x 4 096: 1 020 TFLOP/s m first, 1 074 .. 1 097 bands of 4 or 2,
+// 1 105 of 8, 1 125 of 6; 3 072 1 090 against 1 100, 2 048 1 040 against 1 055; one band up to six tiles (1 536 rows).
+constexpr unsigned BG_BAND = 6;
+struct BgTile { unsigned m, n, bz; };
+__device__ __forceinline__ BgTile bg_tile(unsigned item, unsigned tiles_m, unsigned tiles_n, bool bands) {
+    const unsigned per = tiles_m * tiles_n, bz = item / per, idx = item - bz * per, h0 = bands && tiles_m > BG_BAND ? BG_BAND : tiles_m;
+    const unsigned band = idx / (h0 * tiles_n), in = idx - band * h0 * tiles_n, left = tiles_m - band * h0;
+    const unsigned h = left < h0 ? left : h0, n = in / h;
+    return {band * h0 + (in - n * h), n, bz};
+}
+
 template <int WTN>   // columns per wave: 128 (wide) or 64 (narrow)
 __global__ __launch_bounds__(BG_THREADS, 2) void bgemm_big_kernel(const ffk_bgemm_desc d) {
     typedef Mma<T> MM;
@@ -59,7 +72,7 @@ __global__ __launch_bounds__(BG_THREADS, 2) void bgemm_big_kernel(const ffk_bgem
     const int kchunks = K / BG_BK;
 
     // Persistent workgroups.  Tile t of this workgroup: batched launches give every XCD a contiguous
-    // eighth of the (batch, n-tile, m-tile) order (consecutive workgroup ids go to the eight XCDs in turn,
+    // eighth of the (batch, band, n-tile, m-tile) order (consecutive workgroup ids go to the eight XCDs in turn,
     // each with its own L2), so that all tiles of a batch run behind one L2; otherwise tiles are dealt
     // round-robin.  Returns false past the end.
     auto tile_at = [&](unsigned t, unsigned& item) {
@@ -84,10 +97,10 @@ __global__ __launch_bounds__(BG_THREADS, 2) void bgemm_big_kernel(const ffk_bgem
     int f_kc = 0;              // next chunk of it
     unsigned g_fetch = 0;      // running chunk count -> ring slot
     auto fetch_setup = [&](unsigned item) {
-        const long fm0 = (long)(item % tiles_m) * BM, fn0 = (long)((item / tiles_m) % tiles_n) * BN;
-        const int fbz = (item / tiles_m) / tiles_n;
-        const T* A = (const T*)d.a + (long)fbz * d.a_bs;
-        const T* B = (const T*)d.b + (long)fbz * d.b_bs;
+        const BgTile ft = bg_tile(item, tiles_m, tiles_n, d.batch >= 8);
+        const long fm0 = (long)ft.m * BM, fn0 = (long)ft.n * BN;
+        const T* A = (const T*)d.a + (long)ft.bz * d.a_bs;
+        const T* B = (const T*)d.b + (long)ft.bz * d.b_bs;
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
             const int row = i * 128 + wave * 16 + (lane >> 2);
@@ -241,8 +254,9 @@ __global__ __launch_bounds__(BG_THREADS, 2) void bgemm_big_kernel(const ffk_bgem
     };
     bool relaxed = false;      // previous tile was full: its stores are counted exactly
     for (unsigned t = 0; tile_at(t, item); ++t) {
-        const long m0 = (long)(item % tiles_m) * BM, n0 = (long)((item / tiles_m) % tiles_n) * BN;
-        const int bz = (item / tiles_m) / tiles_n;
+        const BgTile ct = bg_tile(item, tiles_m, tiles_n, d.batch >= 8);
+        const long m0 = (long)ct.m * BM, n0 = (long)ct.n * BN;
+        const int bz = (int)ct.bz;
         zero_acc();
         // One step = one chunk: wait, barrier, then the second K step of the chunk before (fragments fa1 / fb1), the
         // request for the chunk three ahead, and the first K step of this chunk.

@@ -220,6 +220,24 @@ def test_bgemm_large_tiles(dev, C, M, N, K):
     assert np.abs(got - ref).max() < 2e-2 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("C,M,N,K", [
+    (8, 1536, 272, 96),      # six tiles along m: one band
+    (8, 1537, 384, 96),      # one row more: a second band of one tile, 256 x 128 tiles
+    (9, 3073, 784, 128),     # 6 + 6 + 1 tiles, 468 of them: workgroups walk on into the next batch
+])
+def test_bgemm_bands(dev, C, M, N, K):
+    """The band order of batched launches visits every tile once: the bits of a launch per matrix, whose order has no bands."""
+    from fastfold_amd import _lib
+    g = torch.Generator().manual_seed(M)
+    a = torch.randn(C, M, K, generator=g).to(dev, torch.bfloat16)
+    b = torch.randn(C, N, K, generator=g).to(dev, torch.bfloat16)
+    outs = [torch.full((C, M, N), float("nan"), dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    _lib.bgemm_nt(a, b, outs[0], M=M, N=N, K=K, lda=K, ldb=K, batch=C, a_bs=M * K, b_bs=N * K, o_bs=M * N)
+    for c in range(C):
+        _lib.bgemm_nt(a[c], b[c], outs[1][c], M=M, N=N, K=K, lda=K, ldb=K)
+    assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-5), (torch.bfloat16, 1e-2)])
 @pytest.mark.parametrize("s,r", [(24, 10), (128, 9), (50, 33)])
 def test_bgemm_outer_product_and_projection(dev, dtype, tol, s, r):
