@@ -38,20 +38,23 @@ __device__ __forceinline__ void bg_load_lds(const T* src, unsigned char* dst_wav
                                      (__attribute__((address_space(3))) void*)dst_wave, 16, 0, 0);
 }
 
-// Tile of item idx of a batch, in bands of BG_BAND tiles along m, n outside m within a band.  Batched launches run a batch of large
-// matrices behind one L2, 32 tiles at a time: six by five or so of them read 11 panels of 256 rows, 16 by 2 (m first over all of
-// 4 096 rows) read 18, from memory, 2.5 TB/s of misses.  4 096 x 4 096 x 4 096: 1 020 TFLOP/s m first, 1 074 .. 1 097 bands of 4 or 2,
-// 1 105 of 8, 1 125 of 6; 3 072 1 090 against 1 100, 2 048 1 040 against 1 055; one band up to six tiles (1 536 rows).
-constexpr unsigned BG_BAND = 6;
+// Tile of item idx.  BANDS: bands of six tiles along m, n outside m within a band; else m first over all rows.  Batched launches run
+// a batch of large matrices behind one L2, 32 tiles at a time: six by five or so of them read 11 panels of 256 rows, 16 by 2 (m first
+// over 4 096 rows) read 18, from memory, 2.5 TB/s of misses.  4 096 x 4 096 x 4 096: 1 020 TFLOP/s m first, 1 074 .. 1 097 bands of 4
+// or 2, 1 105 of 8, 1 125 of 6; 3 072 1 090 against 1 100.  Up to eight tiles along m the launch is m first (2 048: 1 055 either way,
+// 1 792 3 % faster so; a kernel of its own, because the scalar registers of the bands cost 1 .. 2 % at 1 024).
+constexpr int BG_BAND = 6, BG_BAND_MIN = 9;
 struct BgTile { unsigned m, n, bz; };
-__device__ __forceinline__ BgTile bg_tile(unsigned item, unsigned tiles_m, unsigned tiles_n, bool bands) {
-    const unsigned per = tiles_m * tiles_n, bz = item / per, idx = item - bz * per, h0 = bands && tiles_m > BG_BAND ? BG_BAND : tiles_m;
-    const unsigned band = idx / (h0 * tiles_n), in = idx - band * h0 * tiles_n, left = tiles_m - band * h0;
-    const unsigned h = left < h0 ? left : h0, n = in / h;
-    return {band * h0 + (in - n * h), n, bz};
+template <bool BANDS>
+__device__ __forceinline__ BgTile bg_tile(unsigned item, unsigned tiles_m, unsigned tiles_n) {
+    if (!BANDS) return {item % tiles_m, (item / tiles_m) % tiles_n, (item / tiles_m) / tiles_n};
+    const unsigned per = tiles_m * tiles_n, bz = item / per, idx = item - bz * per;
+    const unsigned band = idx / (BG_BAND * tiles_n), in = idx - band * BG_BAND * tiles_n, left = tiles_m - band * BG_BAND;
+    const unsigned h = left < (unsigned)BG_BAND ? left : BG_BAND, n = in / h;
+    return {band * BG_BAND + (in - n * h), n, bz};
 }
 
-template <int WTN>   // columns per wave: 128 (wide) or 64 (narrow)
+template <int WTN, bool BANDS>   // columns per wave: 128 (wide) or 64 (narrow); order of the tiles
 __global__ __launch_bounds__(BG_THREADS, 2) void bgemm_big_kernel(const ffk_bgemm_desc d) {
     typedef Mma<T> MM;
     constexpr int BM = 256, BN = 2 * WTN;
@@ -72,7 +75,7 @@ __global__ __launch_bounds__(BG_THREADS, 2) void bgemm_big_kernel(const ffk_bgem
     const int kchunks = K / BG_BK;
 
     // Persistent workgroups.  Tile t of this workgroup: batched launches give every XCD a contiguous
-    // eighth of the (batch, band, n-tile, m-tile) order (consecutive workgroup ids go to the eight XCDs in turn,
+    // eighth of the (batch, [band,] n-tile, m-tile) order (consecutive workgroup ids go to the eight XCDs in turn,
     // each with its own L2), so that all tiles of a batch run behind one L2; otherwise tiles are dealt
     // round-robin.  Returns false past the end.
     auto tile_at = [&](unsigned t, unsigned& item) {
@@ -97,10 +100,11 @@ __global__ __launch_bounds__(BG_THREADS, 2) void bgemm_big_kernel(const ffk_bgem
     int f_kc = 0;              // next chunk of it
     unsigned g_fetch = 0;      // running chunk count -> ring slot
     auto fetch_setup = [&](unsigned item) {
-        const BgTile ft = bg_tile(item, tiles_m, tiles_n, d.batch >= 8);
+        const BgTile ft = bg_tile<BANDS>(item, tiles_m, tiles_n);
         const long fm0 = (long)ft.m * BM, fn0 = (long)ft.n * BN;
-        const T* A = (const T*)d.a + (long)ft.bz * d.a_bs;
-        const T* B = (const T*)d.b + (long)ft.bz * d.b_bs;
+        const int fbz = (int)ft.bz;
+        const T* A = (const T*)d.a + (long)fbz * d.a_bs;
+        const T* B = (const T*)d.b + (long)fbz * d.b_bs;
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
             const int row = i * 128 + wave * 16 + (lane >> 2);
@@ -254,7 +258,7 @@ __global__ __launch_bounds__(BG_THREADS, 2) void bgemm_big_kernel(const ffk_bgem
     };
     bool relaxed = false;      // previous tile was full: its stores are counted exactly
     for (unsigned t = 0; tile_at(t, item); ++t) {
-        const BgTile ct = bg_tile(item, tiles_m, tiles_n, d.batch >= 8);
+        const BgTile ct = bg_tile<BANDS>(item, tiles_m, tiles_n);
         const long m0 = (long)ct.m * BM, n0 = (long)ct.n * BN;
         const int bz = (int)ct.bz;
         zero_acc();
@@ -312,19 +316,19 @@ __global__ __launch_bounds__(BG_THREADS, 2) void bgemm_big_kernel(const ffk_bgem
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // the re-reads past the end
 }
 
-template <int WTN>
+template <int WTN, bool BANDS>
 int bg_launch(const ffk_bgemm_desc& d, hipStream_t st) {
     constexpr int BM = 256, BN = 2 * WTN;
     const size_t smem = (size_t)BG_SLOTS * (BM + BN) * 64;
     static FfkLdsReservation lds_reserved;
     {
-        const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)bgemm_big_kernel<WTN>, smem, "ffk_bgemm_nt");
+        const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)bgemm_big_kernel<WTN, BANDS>, smem, "ffk_bgemm_nt");
         if (rc_lds != FFK_OK) return rc_lds;
     }
     const long tiles = (long)ffk_cdiv(d.M, BM) * ffk_cdiv(d.N, BN) * d.batch;
     if (tiles >= (1L << 31) - 8) return ffk_fail(FFK_ERR_SHAPE, "ffk_bgemm_nt: %ld output tiles exceed the grid limit", tiles);
     const unsigned grid = (unsigned)(tiles < 256 ? 8 * ffk_cdiv(tiles, 8) : 256);   // persistent: one workgroup per CU
-    bgemm_big_kernel<WTN><<<grid, BG_THREADS, smem, st>>>(d);
+    bgemm_big_kernel<WTN, BANDS><<<grid, BG_THREADS, smem, st>>>(d);
     return ffk_check_launch("ffk_bgemm_nt");
 }
 
@@ -343,6 +347,8 @@ int ffk_bgemm_big_try(const ffk_bgemm_desc* d, hipStream_t st, int* status) {
     // 256 x 256 tiles, unless they would leave CUs without a tile while 256 x 128 tiles would not (small batched launches)
     const long wide_tiles = (long)ffk_cdiv(d->M, 256) * ffk_cdiv(d->N, 256) * d->batch;
     const bool narrow = d->N <= 128 || (wide_tiles < 256 && d->N % 128 == 0);
-    *status = narrow ? bg_launch<64>(*d, st) : bg_launch<128>(*d, st);
+    if (narrow) *status = bg_launch<64, false>(*d, st);
+    else if (d->batch >= 8 && ffk_cdiv(d->M, 256) >= BG_BAND_MIN) *status = bg_launch<128, true>(*d, st);
+    else *status = bg_launch<128, false>(*d, st);
     return 1;
 }

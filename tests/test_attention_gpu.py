@@ -221,9 +221,9 @@ def test_bgemm_large_tiles(dev, C, M, N, K):
 
 
 @pytest.mark.parametrize("C,M,N,K", [
-    (8, 1536, 272, 96),      # six tiles along m: one band
-    (8, 1537, 384, 96),      # one row more: a second band of one tile, 256 x 128 tiles
-    (9, 3073, 784, 128),     # 6 + 6 + 1 tiles, 468 of them: workgroups walk on into the next batch
+    (8, 2048, 272, 96),      # eight tiles along m: m first
+    (8, 2049, 272, 96),      # nine: bands of six and three, the last tile of one row
+    (9, 3073, 784, 128),     # 6 + 6 + 1 tiles, 468 in all: workgroups walk on into the next batch
 ])
 def test_bgemm_bands(dev, C, M, N, K):
     """The band order of batched launches visits every tile once: the bits of a launch per matrix, whose order has no bands."""
