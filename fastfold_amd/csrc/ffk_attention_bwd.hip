@@ -11,26 +11,29 @@
 //     dP    = do . v^T                 dS = P (dP - D)         (gradient w.r.t. the logits s)
 //     dq    = dS . k / sqrt(d)         dk = dS^T . q / sqrt(d)
 //     dv    = P^T . do                 dbias[h, q, k] = sum_b2 dS
-//   attention_bwd_dq_kernel   one wave per (b2, head, 32 queries): a walk over the key tiles accumulates dq^T = k^T . dS^T,
+//   attention_bwd_dq_kernel   one wave per (b2, head, NT tiles of 32 queries): a walk over the key tiles accumulates dq^T = k^T . dS^T,
 //                             the score tile transposed (keys along the MFMA rows) exactly as in the forward kernel,
 //                             so that dS^T is the N operand of that product as it stands.  Row log-sum-exp and D come
 //                             from the forward pass and the re-tiling (ffk_attention_bwd_rows) or from a walk before
 //                             it (ffk_attention_bwd, log2 domain), which leaves them for the other two kernels.
-//   attention_bwd_dkv_kernel  one wave per (b2, head, 32 keys): walks the query tiles with the score tile the other
+//   attention_bwd_dkv_kernel  one wave per (b2, head, NT tiles of 32 keys): walks the query tiles with the score tile the other
 //                             way round (queries along the MFMA rows, one key per lane), so that P and dS are the N
 //                             operands of  dv^T = do^T . P  and  dk^T = q^T . dS.
-//   attention_bwd_dbias_kernel  one wave per (head, query tile, key tile, slice of the batch rows): recomputes dS of
-//                             its tile for every batch row of the slice and sums in registers; the slices (what fills
+//   attention_bwd_dbias_kernel  one wave per (head, query tile, NT key tiles, slice of the batch rows): recomputes dS of
+//                             its tiles for every batch row of the slice and sums in registers; the slices (what fills
 //                             the chip when H * QT * KT alone is a few hundred tiles) are left as partial sums the
 //                             caller adds up (ffk_attention_bwd_rows) or added with one fp32 atomic per element.
 // They take the pair bias from the same operand tiles as the forward kernel: added to the scores by a product with
 // an identity operand, in the last two with the roles of the two operands exchanged (rows = queries).
 // Every operand arrives in the tile order its role needs.  Waves load their tiles straight from global memory, each
 // operand of the next step requested as soon as its registers are free, and no LDS is used: what bounds the kernels is
-// the latency of that chain and the exponentials, with three or four waves per SIMD to cover it.  128 x 8 heads of
-// 256 x 256 logits, bf16, before and after the early requests: dq 86 -> 45 us, dk / dv 71 -> 53, d bias 59 -> 43.
+// the latency of that chain and the exponentials, with three waves per SIMD to cover it, or two of two tiles each (NT = 2:
+// the operands of the walk are read once for both).  128 x 8 heads of 256 x 256 logits, bf16, one tile per wave and loads
+// that waited for each other, requested in time, two tiles per wave: dq 39.6, 38.8, 35.0 us, dk / dv 56.5, 56.2, 46.1,
+// d bias 41.5, 40.5, 32.1; fp32, the first two: dq 198, 174, dk / dv 232, 223, d bias 127, 121.
 #include "ffk_common.h"
 #include <initializer_list>
+#include <type_traits>
 
 namespace {
 
@@ -58,6 +61,13 @@ template <typename T> struct Tile16 {         // the 16 elements one lane owns o
             reinterpret_cast<const unsigned char*>(&v[0]) + i * sizeof(typename Mma<T>::Frag));
     }
 };
+
+// Requests above this point are issued above it: without it the compiler moves loads of the next step behind the branch back, in
+// front of their first use, to save registers, and every step waits for them (117 x 4 heads of 117 x 117: d bias 18.1 us, 14.4 with
+// it; dk / dv are left as they are by the compiler, and d bias in pairs, 32.1 us at 128 x 8 heads of 256, is 34.0 with it).
+template <bool HERE> __device__ __forceinline__ void issue_here() {
+    if (HERE) asm volatile("" ::: "memory");
+}
 
 // fragments (N operand) of 16 fp32 values held in accumulator order, rounded to the operand type
 template <typename T> struct NFrag;
@@ -112,8 +122,8 @@ __device__ __forceinline__ void store4(T* o, const float* f) {          // four 
 // ------------------------------------------------------------------------------ dq ----
 // STATS: the row statistics are computed here (a walk over the keys of its own) and written for the other kernels; otherwise
 // the forward pass has left the log-sum-exp and the gate's backward kernel sum_d do o.
-template <typename T, int DP, bool HAS_BIAS, bool STATS>
-__global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 4 : 1) void attention_bwd_dq_kernel(
+template <typename T, int DP, int NT, bool HAS_BIAS, bool STATS>
+__global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? (NT == 1 ? 3 : 2) : 1) void attention_bwd_dq_kernel(
     T* __restrict__ dq, float* __restrict__ lse, float* __restrict__ dsum, const T* __restrict__ q_qk,
     const T* __restrict__ k_qk, const T* __restrict__ k_acc, const T* __restrict__ v_qk, const T* __restrict__ bias_t,
     const float* __restrict__ keybias, const T* __restrict__ do_qk, const T* __restrict__ o_qk, int B2, int H, int Nq,
@@ -124,27 +134,35 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 4 : 1) void attent
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l32 = lane & 31, half = lane >> 5;
     const int QT = (Nq + 31) >> 5, KT = (Nk + 31) >> 5;
+    static_assert(NT == 1 || !STATS, "statistics: one query tile per wave");
+    const int QP = (QT + NT - 1) / NT;
     const long item = bwd_logical_block() * 4 + wave;
-    if (item >= (long)B2 * H * QT) return;
-    const int qt = (int)(item % QT);
-    const long bh = item / QT;
+    if (item >= (long)B2 * H * QP) return;
+    const int qt0 = (int)(item % QP) * NT;
+    const long bh = item / QP;
     const int h = (int)(bh % H), b2 = (int)(bh / H);
+    auto qtile = [&](int t) { return NT == 1 || qt0 + t < QT ? qt0 + t : QT - 1; };   // a tile past the last one is the last one again, not stored
+    const int qt = qt0;
 
-    Tile16<T> qf[DP], dof[DP];
+    Tile16<T> qf[NT][DP], dof[NT][DP];
     float dpart = 0.0f;
 #pragma unroll
-    for (int p = 0; p < DP; ++p) {
-        qf[p].load_rows(q_qk + p * part_q + ((bh * QT + qt) << 10) + l32 * 16, half);
-        dof[p].load_rows(do_qk + p * part_q + ((bh * QT + qt) << 10) + l32 * 16, half);
-        if (STATS) {
-            Tile16<T> of;
-            of.load_rows(o_qk + p * part_q + ((bh * QT + qt) << 10) + l32 * 16, half);
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int j = 0; j < 16; ++j) dpart += dof[p].f(j) * of.f(j);
+        for (int p = 0; p < DP; ++p) {
+            const long off = p * part_q + ((bh * QT + qtile(t)) << 10) + l32 * 16;
+            qf[t][p].load_rows(q_qk + off, half);
+            dof[t][p].load_rows(do_qk + off, half);
+            if (STATS) {
+                Tile16<T> of;
+                of.load_rows(o_qk + off, half);
+#pragma unroll
+                for (int j = 0; j < 16; ++j) dpart += dof[t][p].f(j) * of.f(j);
+            }
         }
-    }
-    // this lane's query: sum_d do o
-    const float D = STATS ? dpart + lane_xor<32>(dpart) : dsum[(bh * QT + qt) * 32 + l32];
+    float D[NT];                                               // this lane's queries: sum_d do o
+#pragma unroll
+    for (int t = 0; t < NT; ++t) D[t] = STATS ? dpart + lane_xor<32>(dpart) : dsum[(bh * QT + qtile(t)) * 32 + l32];
     const float* mp = keybias + (long)b2 * KT * 32 + 4 * half;
 
     Frag ident[NF];
@@ -161,7 +179,7 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 4 : 1) void attent
             Tile16<T> kc;
             kc.load_rows(k_qk + p * part_k + ((bh * KT + kt) << 10) + l32 * 16, half);
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(s, kc.frag(i), qf[p].frag(i));
+            for (int i = 0; i < NF; ++i) MM::mma(s, kc.frag(i), qf[0][p].frag(i));
         }
         if (HAS_BIAS) {
             Tile16<T> bc;
@@ -177,7 +195,7 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 4 : 1) void attent
         }
     };
 
-    float L;
+    float L[NT];
     if (STATS) {
         // first walk: row maximum and sum
         float m_run = REF_FLOOR, l_run = 0.0f;
@@ -196,26 +214,32 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 4 : 1) void attent
             m_run = m_new;
         }
         const float l_tot = l_run + lane_xor<32>(l_run);
-        L = l_tot > 0.0f ? m_run + __builtin_amdgcn_logf(l_tot) : NO_ROW;   // v_log_f32 is log2
+        L[0] = l_tot > 0.0f ? m_run + __builtin_amdgcn_logf(l_tot) : NO_ROW;   // v_log_f32 is log2
         if (half == 0) {
-            lse[(bh * QT + qt) * 32 + l32] = L;
-            dsum[(bh * QT + qt) * 32 + l32] = D;
+            lse[(bh * QT + qt) * 32 + l32] = L[0];
+            dsum[(bh * QT + qt) * 32 + l32] = D[0];
         }
     } else {
-        L = lse[(bh * QT + qt) * 32 + l32];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) L[t] = lse[(bh * QT + qtile(t)) * 32 + l32];
     }
 
     // second walk: dq^T += k^T . dS^T.  What a step reads is requested for the next step as soon as its registers are free
-    // (a step later it is there; waiting for each tile where it is used took 57 us at 128 x 8 heads of 256 x 256 logits).
+    // (a step later it is there; waiting for each tile where it is used took 57 us, NT = 1, at 128 x 8 heads of 256 x 256 logits).
     // The scores start at key bias - log-sum-exp and dP at -D, so that the products leave the exponent and dP - D themselves.
-    f32x16 acc[DP];
+    f32x16 acc[NT][DP];
 #pragma unroll
-    for (int p = 0; p < DP; ++p)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[p][v] = 0.0f;
-    Tile16<T> kc[DP], vq[DP], ka[DP], bc;
+        for (int p = 0; p < DP; ++p)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[t][p][v] = 0.0f;
+    Tile16<T> kc[DP], vq[DP], ka[DP], bc[NT];
     f32x4 mk[4];
-    const T* bias_row = HAS_BIAS ? bias_t + ((((long)h * QT + qt) * (KT + bias_pad)) << 10) + l32 * 16 : nullptr;
+    const T* bias_row[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+        bias_row[t] = HAS_BIAS ? bias_t + ((((long)h * QT + qtile(t)) * (KT + bias_pad)) << 10) + l32 * 16 : nullptr;
     const long krow = (bh * KT) << 10;
     auto load_mask = [&](int kt) {
 #pragma unroll
@@ -227,7 +251,10 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 4 : 1) void attent
             kc[p].load_rows(k_qk + p * part_k + krow + ((long)kt << 10) + l32 * 16, half);
             vq[p].load_rows(v_qk + p * part_k + krow + ((long)kt << 10) + l32 * 16, half);
         }
-        if (HAS_BIAS) bc.load_rows(bias_row + ((long)kt << 10), half);
+        if (HAS_BIAS) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) bc[t].load_rows(bias_row[t] + ((long)kt << 10), half);
+        }
     };
     auto load_acc = [&](int kt) {
 #pragma unroll
@@ -238,39 +265,52 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 4 : 1) void attent
     load_acc(0);
     for (int kt = 0; kt < KT; ++kt) {
         const int next = kt + 1 < KT ? kt + 1 : kt;
-        f32x16 s, dp;
+        f32x16 s[NT], dp[NT];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            s[v] = mk[v >> 2][v & 3] - L;
-            dp[v] = -D;
-        }
+        for (int t = 0; t < NT; ++t) {
 #pragma unroll
-        for (int p = 0; p < DP; ++p) {
+            for (int v = 0; v < 16; ++v) {
+                s[t][v] = mk[v >> 2][v & 3] - L[t];
+                dp[t][v] = -D[t];
+            }
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(s, kc[p].frag(i), qf[p].frag(i));
+            for (int p = 0; p < DP; ++p) {
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(dp, vq[p].frag(i), dof[p].frag(i));   // dP^T[key, q] = v[key] . do[q]
-        }
-        if (HAS_BIAS) {
+                for (int i = 0; i < NF; ++i) MM::mma(s[t], kc[p].frag(i), qf[t][p].frag(i));
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(s, bc.frag(i), ident[i]);
+                for (int i = 0; i < NF; ++i) MM::mma(dp[t], vq[p].frag(i), dof[t][p].frag(i));   // dP^T[key, q] = v[key] . do[q]
+            }
+            if (HAS_BIAS) {
+#pragma unroll
+                for (int i = 0; i < NF; ++i) MM::mma(s[t], bc[t].frag(i), ident[i]);
+            }
         }
         load_scores(next);
-        float ds[16];
+        issue_here<DP == 1>();
+        Frag dsf[NT][NF];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) ds[v] = fast_exp2(s[v]) * dp[v];
-        Frag dsf[NF];
+        for (int t = 0; t < NT; ++t) {
+            float ds[16];
 #pragma unroll
-        for (int i = 0; i < NF; ++i) dsf[i] = NFrag<T>::make(ds + i * MM::KLANE);
+            for (int v = 0; v < 16; ++v) ds[v] = fast_exp2(s[t][v]) * dp[t][v];
+#pragma unroll
+            for (int i = 0; i < NF; ++i) dsf[t][i] = NFrag<T>::make(ds + i * MM::KLANE);
+        }
         load_mask(next);                                       // late: the registers are those of the scores
+        issue_here<DP == 1>();
 #pragma unroll
-        for (int p = 0; p < DP; ++p)
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(acc[p], ka[p].frag(i), dsf[i]);
+            for (int p = 0; p < DP; ++p)
+#pragma unroll
+                for (int i = 0; i < NF; ++i) MM::mma(acc[t][p], ka[p].frag(i), dsf[t][i]);
         load_acc(next);
+        issue_here<DP == 1>();
     }
-    const int q = qt * 32 + l32;
-    if (q < Nq) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int q = (qt0 + t) * 32 + l32;
+        if (q >= Nq) continue;
         T* o = dq + (long)b2 * om.s_b + (long)h * om.s_h + (long)q * om.s_n + 4 * half;
 #pragma unroll
         for (int p = 0; p < DP; ++p)
@@ -278,15 +318,15 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 4 : 1) void attent
             for (int g = 0; g < 4; ++g) {
                 float f[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) f[e] = acc[p][4 * g + e] * dq_scale;
+                for (int e = 0; e < 4; ++e) f[e] = acc[t][p][4 * g + e] * dq_scale;
                 store4(o + 32 * p + 8 * g, f);
             }
     }
 }
 
 // ------------------------------------------------------------------------- dk, dv ----
-template <typename T, int DP>
-__global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 3 : 1) void attention_bwd_dkv_kernel(
+template <typename T, int DP, int NT>
+__global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? (NT == 1 ? 3 : 2) : 1) void attention_bwd_dkv_kernel(
     T* __restrict__ dk, T* __restrict__ dv, const T* __restrict__ q_qk,
     const T* __restrict__ q_acc, const T* __restrict__ k_qk, const T* __restrict__ v_qk, const T* __restrict__ bias_t,
     const float* __restrict__ keybias, const T* __restrict__ do_qk, const T* __restrict__ do_acc,
@@ -298,38 +338,47 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 3 : 1) void attent
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l32 = lane & 31, half = lane >> 5;
     const int QT = (Nq + 31) >> 5, KT = (Nk + 31) >> 5;
+    const int KP = (KT + NT - 1) / NT;
     const long item = bwd_logical_block() * 4 + wave;
-    if (item >= (long)B2 * H * KT) return;
-    const int kt = (int)(item % KT);
-    const long bh = item / KT;
+    if (item >= (long)B2 * H * KP) return;
+    const int kt0 = (int)(item % KP) * NT;
+    const long bh = item / KP;
     const int h = (int)(bh % H), b2 = (int)(bh / H);
+    auto ktile = [&](int t) { return NT == 1 || kt0 + t < KT ? kt0 + t : KT - 1; };   // a tile past the last one is the last one again, not stored
 
-    Tile16<T> kf[DP], vf[DP];                      // this lane's key (column l32): k and v rows as N operands
+    Tile16<T> kf[NT][DP], vf[NT][DP];              // this lane's keys (column l32): k and v rows as N operands
+    float kb[NT];                                  // 0, masked (-1e9 log2e) or padding (hugely negative)
 #pragma unroll
-    for (int p = 0; p < DP; ++p) {
-        kf[p].load_rows(k_qk + p * part_k + ((bh * KT + kt) << 10) + l32 * 16, half);
-        vf[p].load_rows(v_qk + p * part_k + ((bh * KT + kt) << 10) + l32 * 16, half);
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+        for (int p = 0; p < DP; ++p) {
+            kf[t][p].load_rows(k_qk + p * part_k + ((bh * KT + ktile(t)) << 10) + l32 * 16, half);
+            vf[t][p].load_rows(v_qk + p * part_k + ((bh * KT + ktile(t)) << 10) + l32 * 16, half);
+        }
+        kb[t] = keybias[((long)b2 * KT + ktile(t)) * 32 + l32];
     }
-    const int key = kt * 32 + l32;
-    const float kb = keybias[(long)b2 * KT * 32 + key];     // 0, masked (-1e9 log2e) or padding (hugely negative)
     Frag ident[NF];
     if (bias_t) {
 #pragma unroll
         for (int i = 0; i < NF; ++i) ident[i] = identity_frag<T>(i, l32, half);
     }
 
-    f32x16 acc_k[DP], acc_v[DP];
+    f32x16 acc_k[NT][DP], acc_v[NT][DP];
 #pragma unroll
-    for (int p = 0; p < DP; ++p)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc_k[p][v] = acc_v[p][v] = 0.0f;
+        for (int p = 0; p < DP; ++p)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc_k[t][p][v] = acc_v[t][p][v] = 0.0f;
     // as in the dq kernel: each operand is requested for the next step once its registers are free
-    Tile16<T> qc[DP], doc[DP], qa[DP], doa[DP], bc;
+    Tile16<T> qc[DP], doc[DP], qa[DP], doa[DP], bc[NT];
     f32x4 L4[4], D4[4];
     const long qrow = (bh * QT) << 10;
     const float* lp = lse + bh * QT * 32 + 4 * half;
     const float* dpz = dsum + bh * QT * 32 + 4 * half;
-    const T* bias_col = bias_t ? bias_t + ((((long)h * QT) * (KT + bias_pad) + kt) << 10) + l32 * 16 : nullptr;
+    const T* bias_col[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) bias_col[t] = bias_t ? bias_t + ((((long)h * QT) * (KT + bias_pad) + ktile(t)) << 10) + l32 * 16 : nullptr;
     auto load_rows = [&](int qt) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
@@ -343,7 +392,10 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 3 : 1) void attent
             qc[p].load_rows(q_qk + p * part_q + qrow + ((long)qt << 10) + l32 * 16, half);
             doc[p].load_rows(do_qk + p * part_q + qrow + ((long)qt << 10) + l32 * 16, half);
         }
-        if (bias_t) bc.load_rows(bias_col + (((long)qt * (KT + bias_pad)) << 10), half);
+        if (bias_t) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) bc[t].load_rows(bias_col[t] + (((long)qt * (KT + bias_pad)) << 10), half);
+        }
     };
     auto load_acc = [&](int qt) {
 #pragma unroll
@@ -357,47 +409,58 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 3 : 1) void attent
     load_acc(0);
     for (int qt = 0; qt < QT; ++qt) {
         const int next = qt + 1 < QT ? qt + 1 : qt;
-        f32x16 s, dp;
+        f32x16 s[NT], dp[NT];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            s[v] = kb - L4[v >> 2][v & 3];
-            dp[v] = -D4[v >> 2][v & 3];
-        }
+        for (int t = 0; t < NT; ++t) {
 #pragma unroll
-        for (int p = 0; p < DP; ++p) {
+            for (int v = 0; v < 16; ++v) {
+                s[t][v] = kb[t] - L4[v >> 2][v & 3];
+                dp[t][v] = -D4[v >> 2][v & 3];
+            }
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(s, qc[p].frag(i), kf[p].frag(i));       // S[q, key], log2 domain
+            for (int p = 0; p < DP; ++p) {
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(dp, doc[p].frag(i), vf[p].frag(i));     // dP[q, key] = do[q] . v[key]
-        }
-        if (bias_t) {                                                           // S += I . bias (rows = queries)
+                for (int i = 0; i < NF; ++i) MM::mma(s[t], qc[p].frag(i), kf[t][p].frag(i));       // S[q, key], log2 domain
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(s, ident[i], bc.frag(i));
+                for (int i = 0; i < NF; ++i) MM::mma(dp[t], doc[p].frag(i), vf[t][p].frag(i));     // dP[q, key] = do[q] . v[key]
+            }
+            if (bias_t) {                                                           // S += I . bias (rows = queries)
+#pragma unroll
+                for (int i = 0; i < NF; ++i) MM::mma(s[t], ident[i], bc[t].frag(i));
+            }
         }
         load_scores(next);
-        float p[16], ds[16];
+        Frag pfr[NT][NF], dsf[NT][NF];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            p[v] = fast_exp2(s[v]);
-            ds[v] = p[v] * dp[v];
-        }
-        Frag pfr[NF], dsf[NF];
+        for (int t = 0; t < NT; ++t) {
+            float p[16], ds[16];
 #pragma unroll
-        for (int i = 0; i < NF; ++i) {
-            pfr[i] = NFrag<T>::make(p + i * MM::KLANE);
-            dsf[i] = NFrag<T>::make(ds + i * MM::KLANE);
+            for (int v = 0; v < 16; ++v) {
+                p[v] = fast_exp2(s[t][v]);
+                ds[v] = p[v] * dp[t][v];
+            }
+#pragma unroll
+            for (int i = 0; i < NF; ++i) {
+                pfr[t][i] = NFrag<T>::make(p + i * MM::KLANE);
+                dsf[t][i] = NFrag<T>::make(ds + i * MM::KLANE);
+            }
         }
         load_rows(next);                                   // late: the 32 registers are those of the scores
 #pragma unroll
-        for (int pp = 0; pp < DP; ++pp) {
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(acc_v[pp], doa[pp].frag(i), pfr[i]);   // dv^T += do^T . P
+            for (int pp = 0; pp < DP; ++pp) {
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(acc_k[pp], qa[pp].frag(i), dsf[i]);    // dk^T += q^T . dS
-        }
+                for (int i = 0; i < NF; ++i) MM::mma(acc_v[t][pp], doa[pp].frag(i), pfr[t][i]);   // dv^T += do^T . P
+#pragma unroll
+                for (int i = 0; i < NF; ++i) MM::mma(acc_k[t][pp], qa[pp].frag(i), dsf[t][i]);    // dk^T += q^T . dS
+            }
         load_acc(next);
     }
-    if (key < Nk) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int key = (kt0 + t) * 32 + l32;
+        if (key >= Nk) continue;
         const long o = (long)b2 * om.s_b + (long)h * om.s_h + (long)key * om.s_n + 4 * half;
 #pragma unroll
         for (int pp = 0; pp < DP; ++pp)
@@ -406,8 +469,8 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 3 : 1) void attent
                 float fk[4], fv[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    fk[e] = acc_k[pp][4 * g + e] * dk_scale;
-                    fv[e] = acc_v[pp][4 * g + e];
+                    fk[e] = acc_k[t][pp][4 * g + e] * dk_scale;
+                    fv[e] = acc_v[t][pp][4 * g + e];
                 }
                 store4(dk + o + 32 * pp + 8 * g, fk);
                 store4(dv + o + 32 * pp + 8 * g, fv);
@@ -417,8 +480,8 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 3 : 1) void attent
 
 // ---------------------------------------------------------------------------- dbias ----
 // dbias[h, q, key] += sum over the batch rows b2 = slice, slice + NS, ... of dS[b2, h, q, key].
-template <typename T, int DP>
-__global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 4 : 1) void attention_bwd_dbias_kernel(
+template <typename T, int DP, int NT>
+__global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? (NT == 1 ? 3 : 2) : 1) void attention_bwd_dbias_kernel(
     float* __restrict__ dbias, const T* __restrict__ q_qk, const T* __restrict__ k_qk, const T* __restrict__ v_qk,
     const T* __restrict__ bias_t, const float* __restrict__ keybias, const T* __restrict__ do_qk,
     const float* __restrict__ lse, const float* __restrict__ dsum, int B2, int H, int Nq, int Nk, int NS,
@@ -426,38 +489,37 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 4 : 1) void attent
     typedef Mma<T> MM;
     typedef typename MM::Frag Frag;
     constexpr int NF = 16 / MM::KLANE;
+    constexpr bool PIN = DP == 1 && (sizeof(T) == 4 || NT == 1);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l32 = lane & 31, half = lane >> 5;
     const int QT = (Nq + 31) >> 5, KT = (Nk + 31) >> 5;
+    const int KP = (KT + NT - 1) / NT;
     const long item = bwd_logical_block() * 4 + wave;          // key tile fastest: a block's waves share q and do
-    if (item >= (long)NS * H * QT * KT) return;
-    const int kt = (int)(item % KT);
-    const int qt = (int)((item / KT) % QT);
-    const int h = (int)((item / ((long)KT * QT)) % H);
-    const int slice = (int)(item / ((long)KT * QT * H));
-    const int key = kt * 32 + l32;
+    if (item >= (long)NS * H * QT * KP) return;
+    const int kt0 = (int)(item % KP) * NT;
+    const int qt = (int)((item / KP) % QT);
+    const int h = (int)((item / ((long)KP * QT)) % H);
+    const int slice = (int)(item / ((long)KP * QT * H));
+    auto ktile = [&](int t) { return NT == 1 || kt0 + t < KT ? kt0 + t : KT - 1; };   // a tile past the last one is the last one again, not stored
 
-    Frag ident[NF];
+    f32x16 sb[NT], acc[NT];                                     // the bias tile in accumulator order, once; the sums
 #pragma unroll
-    for (int i = 0; i < NF; ++i) ident[i] = identity_frag<T>(i, l32, half);
-    Tile16<T> bc;
-    bc.load_rows(bias_t + ((((long)h * QT + qt) * (KT + bias_pad) + kt) << 10) + l32 * 16, half);
-    f32x16 sb;                                                  // the bias tile in accumulator order, once
+    for (int t = 0; t < NT; ++t) {
+        Tile16<T> bc;
+        bc.load_rows(bias_t + ((((long)h * QT + qt) * (KT + bias_pad) + ktile(t)) << 10) + l32 * 16, half);
 #pragma unroll
-    for (int v = 0; v < 16; ++v) sb[v] = 0.0f;
+        for (int v = 0; v < 16; ++v) sb[t][v] = acc[t][v] = 0.0f;
 #pragma unroll
-    for (int i = 0; i < NF; ++i) MM::mma(sb, ident[i], bc.frag(i));
-
-    f32x16 acc;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+        for (int i = 0; i < NF; ++i) MM::mma(sb[t], identity_frag<T>(i, l32, half), bc.frag(i));
+    }
     // as in the dq kernel: each operand is requested for the next batch row once its registers are free
-    Tile16<T> qc[DP], doc[DP], kf[DP], vf[DP];
+    Tile16<T> qc[DP], doc[DP], kf[NT][DP], vf[NT][DP];
     f32x4 L4[4], D4[4];
-    float kb;
+    float kb[NT];
     auto load_rows = [&](int b2) {
         const long bh = (long)b2 * H + h;
-        kb = keybias[(long)b2 * KT * 32 + key];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) kb[t] = keybias[((long)b2 * KT + ktile(t)) * 32 + l32];
         const float* lp = lse + (bh * QT + qt) * 32 + 4 * half;
         const float* dpz = dsum + (bh * QT + qt) * 32 + 4 * half;
 #pragma unroll
@@ -471,40 +533,53 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? 4 : 1) void attent
 #pragma unroll
         for (int p = 0; p < DP; ++p) {
             qc[p].load_rows(q_qk + p * part_q + ((bh * QT + qt) << 10) + l32 * 16, half);
-            kf[p].load_rows(k_qk + p * part_k + ((bh * KT + kt) << 10) + l32 * 16, half);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) kf[t][p].load_rows(k_qk + p * part_k + ((bh * KT + ktile(t)) << 10) + l32 * 16, half);
             doc[p].load_rows(do_qk + p * part_q + ((bh * QT + qt) << 10) + l32 * 16, half);
-            vf[p].load_rows(v_qk + p * part_k + ((bh * KT + kt) << 10) + l32 * 16, half);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) vf[t][p].load_rows(v_qk + p * part_k + ((bh * KT + ktile(t)) << 10) + l32 * 16, half);
         }
     };
     load_rows(slice);                                          // slice < NS <= B2
     load_scores(slice);
     for (int b2 = slice; b2 < B2; b2 += NS) {
         const int next = b2 + NS < B2 ? b2 + NS : b2;
-        f32x16 s, dp;
+        f32x16 s[NT], dp[NT];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            s[v] = sb[v] + (kb - L4[v >> 2][v & 3]);
-            dp[v] = -D4[v >> 2][v & 3];
-        }
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                s[t][v] = sb[t][v] + (kb[t] - L4[v >> 2][v & 3]);
+                dp[t][v] = -D4[v >> 2][v & 3];
+            }
         load_rows(next);
+        issue_here<PIN>();
 #pragma unroll
-        for (int p = 0; p < DP; ++p) {
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(s, qc[p].frag(i), kf[p].frag(i));
+            for (int p = 0; p < DP; ++p) {
 #pragma unroll
-            for (int i = 0; i < NF; ++i) MM::mma(dp, doc[p].frag(i), vf[p].frag(i));
-        }
+                for (int i = 0; i < NF; ++i) MM::mma(s[t], qc[p].frag(i), kf[t][p].frag(i));
+#pragma unroll
+                for (int i = 0; i < NF; ++i) MM::mma(dp[t], doc[p].frag(i), vf[t][p].frag(i));
+            }
         load_scores(next);
+        issue_here<PIN>();
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[v] += fast_exp2(s[v]) * dp[v];
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[t][v] += fast_exp2(s[t][v]) * dp[t][v];
     }
-    if (key < Nk) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int key = (kt0 + t) * 32 + l32;
+        if (key >= Nk) continue;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const int qrow = qt * 32 + acc_row(v, lane);
             if (qrow >= Nq) continue;
-            if (partial) dbias[(((long)slice * H + h) * Nq + qrow) * Nk + key] = acc[v];
-            else atomicAdd(dbias + ((long)h * Nq + qrow) * Nk + key, acc[v]);
+            if (partial) dbias[(((long)slice * H + h) * Nq + qrow) * Nk + key] = acc[t][v];
+            else atomicAdd(dbias + ((long)h * Nq + qrow) * Nk + key, acc[t][v]);
         }
     }
 }
@@ -524,35 +599,58 @@ int launch_bwd(void* dq, void* dk, void* dv, float* dbias, float* lse, float* ds
                long Nk, float dq_scale, float dk_scale, OutMap mq, OutMap mk, int bias_pad, long dbias_parts, hipStream_t st) {
     const long QT = (Nq + 31) / 32, KT = (Nk + 31) / 32;
     const long part_q = B2 * H * QT * 1024, part_k = B2 * H * KT * 1024;
-    const long g1 = 8 * ((B2 * H * QT + 31) / 32), g2 = 8 * ((B2 * H * KT + 31) / 32);      // blocks of four waves, a multiple of 8
-    FFK_REQUIRE(g1 < (1L << 31) && g2 < (1L << 31), FFK_ERR_SHAPE, "ffk_attention_bwd: too many tiles for one launch");
-    if (bias_t) {
-        attention_bwd_dq_kernel<T, DP, true, STATS><<<(unsigned)g1, 256, 0, st>>>((T*)dq, lse, dsum, (const T*)q_qk, (const T*)k_qk,
-                                                                                (const T*)k_acc, (const T*)v_qk, (const T*)bias_t, keybias,
-                                                                                (const T*)do_qk, (const T*)o_qk, (int)B2, (int)H, (int)Nq,
-                                                                                (int)Nk, dq_scale, part_q, part_k, mq, bias_pad);
-    } else {
-        attention_bwd_dq_kernel<T, DP, false, STATS><<<(unsigned)g1, 256, 0, st>>>((T*)dq, lse, dsum, (const T*)q_qk, (const T*)k_qk,
-                                                                                 (const T*)k_acc, (const T*)v_qk, nullptr, keybias,
-                                                                                 (const T*)do_qk, (const T*)o_qk, (int)B2, (int)H, (int)Nq,
-                                                                                 (int)Nk, dq_scale, part_q, part_k, mq, 0);
-    }
-    int rc = ffk_check_launch("ffk_attention_bwd");
+    constexpr bool PAIRS = DP == 1 && sizeof(T) == 2;
+    auto blocks = [](long waves) { return 8 * ((waves + 31) / 32); };                       // of four waves, a multiple of 8
+    const long ns = !dbias ? 0 : (dbias_parts > 0 ? dbias_parts : dbias_slices(B2, H, QT, KT));
+    FFK_REQUIRE(blocks(B2 * H * QT) < (1L << 31) && blocks(B2 * H * KT) < (1L << 31) && blocks(ns * H * QT * KT) < (1L << 31), FFK_ERR_SHAPE,
+                "ffk_attention_bwd: too many tiles for one launch");
+    typedef std::integral_constant<int, 1> One;
+    typedef std::integral_constant<int, PAIRS ? 2 : 1> Two;
+    auto run_dq = [&](auto nt_c) {
+        constexpr int NT = decltype(nt_c)::value;
+        const unsigned g = (unsigned)blocks(B2 * H * ((QT + NT - 1) / NT));
+        if (bias_t)
+            attention_bwd_dq_kernel<T, DP, NT, true, STATS><<<g, 256, 0, st>>>((T*)dq, lse, dsum, (const T*)q_qk, (const T*)k_qk, (const T*)k_acc,
+                                                                             (const T*)v_qk, (const T*)bias_t, keybias, (const T*)do_qk,
+                                                                             (const T*)o_qk, (int)B2, (int)H, (int)Nq, (int)Nk, dq_scale, part_q,
+                                                                             part_k, mq, bias_pad);
+        else
+            attention_bwd_dq_kernel<T, DP, NT, false, STATS><<<g, 256, 0, st>>>((T*)dq, lse, dsum, (const T*)q_qk, (const T*)k_qk, (const T*)k_acc,
+                                                                              (const T*)v_qk, nullptr, keybias, (const T*)do_qk, (const T*)o_qk,
+                                                                              (int)B2, (int)H, (int)Nq, (int)Nk, dq_scale, part_q, part_k, mq, 0);
+        return ffk_check_launch("ffk_attention_bwd");
+    };
+    auto run_dkv = [&](auto nt_c) {
+        constexpr int NT = decltype(nt_c)::value;
+        attention_bwd_dkv_kernel<T, DP, NT><<<(unsigned)blocks(B2 * H * ((KT + NT - 1) / NT)), 256, 0, st>>>(
+            (T*)dk, (T*)dv, (const T*)q_qk, (const T*)q_acc, (const T*)k_qk, (const T*)v_qk, (const T*)bias_t, keybias, (const T*)do_qk,
+            (const T*)do_acc, lse, dsum, (int)B2, (int)H, (int)Nq, (int)Nk, dk_scale, part_q, part_k, mk, bias_pad);
+        return ffk_check_launch("ffk_attention_bwd");
+    };
+    auto run_dbias = [&](auto nt_c) {
+        constexpr int NT = decltype(nt_c)::value;
+        attention_bwd_dbias_kernel<T, DP, NT><<<(unsigned)blocks(ns * H * QT * ((KT + NT - 1) / NT)), 256, 0, st>>>(
+            dbias, (const T*)q_qk, (const T*)k_qk, (const T*)v_qk, (const T*)bias_t, keybias, (const T*)do_qk, lse, dsum, (int)B2, (int)H,
+            (int)Nq, (int)Nk, (int)ns, part_q, part_k, bias_pad, dbias_parts > 0 ? 1 : 0);
+        return ffk_check_launch("ffk_attention_bwd");
+    };
+    // Two tiles per wave (bf16, 32 channels) read what a step shares once for both and are two chains that cover each other, in
+    // registers for two waves per SIMD instead of three.  A launch takes about as long as the rounds of one wave on every SIMD that
+    // it is, and a round of pairs 1.4 (d bias, dk / dv) or 1.7 (dq) rounds of single tiles.  us, single tiles and pairs, 4 heads:
+    //   d bias  784 tiles 14.2, 19.3   1 536 20.3, 20.3   1 960 (seven a row) 22.0, 28.5   4 096 40.5, 31.8   8 192 76.7, 59.8
+    //   dk / dv 768 5.2, 6.6   1 280 8.1, 7.1   2 560 15.4, 15.5   4 096 29.5, 23.0   8 192 56.2, 45.6   16 384 121.4, 91.6
+    //   dq      2 560 18.5, 19.1   3 072 16.5, 17.5   3 584 19.1, 16.8   5 120 25.2, 26.3   6 144 30.4, 27.4   8 192 38.8, 34.7
+    auto rounds = [](long waves) { return (waves + 1023) / 1024; };
+    const bool pq = 4 * rounds(B2 * H * QT) >= 7 * rounds(B2 * H * ((QT + 1) / 2));
+    const bool pk = 2 * rounds(B2 * H * KT) >= 3 * rounds(B2 * H * ((KT + 1) / 2));
+    const bool pb = 2 * rounds(ns * H * QT * KT) >= 3 * rounds(ns * H * QT * ((KT + 1) / 2));
+    int rc;
+    if constexpr (STATS) rc = run_dq(One());
+    else rc = pq ? run_dq(Two()) : run_dq(One());
     if (rc != FFK_OK) return rc;
-    attention_bwd_dkv_kernel<T, DP><<<(unsigned)g2, 256, 0, st>>>((T*)dk, (T*)dv, (const T*)q_qk, (const T*)q_acc,
-                                                                (const T*)k_qk, (const T*)v_qk, (const T*)bias_t, keybias,
-                                                                (const T*)do_qk, (const T*)do_acc, lse, dsum, (int)B2, (int)H,
-                                                                (int)Nq, (int)Nk, dk_scale, part_q, part_k, mk, bias_pad);
-    rc = ffk_check_launch("ffk_attention_bwd");
+    rc = pk ? run_dkv(Two()) : run_dkv(One());
     if (rc != FFK_OK || !dbias) return rc;
-    const long ns = dbias_parts > 0 ? dbias_parts : dbias_slices(B2, H, QT, KT);
-    const long g3 = 8 * ((ns * H * QT * KT + 31) / 32);
-    FFK_REQUIRE(g3 < (1L << 31), FFK_ERR_SHAPE, "ffk_attention_bwd: too many tiles for one launch");
-    attention_bwd_dbias_kernel<T, DP><<<(unsigned)g3, 256, 0, st>>>(dbias, (const T*)q_qk, (const T*)k_qk, (const T*)v_qk,
-                                                                  (const T*)bias_t, keybias, (const T*)do_qk, lse, dsum,
-                                                                  (int)B2, (int)H, (int)Nq, (int)Nk, (int)ns, part_q, part_k, bias_pad,
-                                                                  dbias_parts > 0 ? 1 : 0);
-    return ffk_check_launch("ffk_attention_bwd");
+    return pb ? run_dbias(Two()) : run_dbias(One());
 }
 
 }  // namespace

@@ -399,6 +399,39 @@ def test_attention_bwd_entry_at_head_dimension_32(dev, dtype, tol, b2, n, use_bi
             assert _rel(_np(a), b.grad.numpy()) < tol, name
 
 
+@pytest.mark.parametrize("use_bias", [True, False])
+@pytest.mark.parametrize("B2,h,n,parts", [(128, 8, 40, 64), (128, 4, 96, 42), (64, 4, 200, 9), (150, 8, 20, 100)])
+def test_attention_backward_pairs_match_single_tiles(dev, B2, h, n, parts, use_bias):
+    """Launches of more tiles than SIMDs take two per wave (two, three and seven tiles a row; one a row stays single): the bits of
+    launches of a few batch rows, which do not - for the bias gradient of one launch per slice of the rows, rows in the same order."""
+    from fastfold_amd import _lib
+    nt, dt = (n + 31) // 32, torch.bfloat16
+    g = torch.Generator().manual_seed(n)
+    rn = lambda *s: (torch.randn(*s, generator=g) * 0.5).to(dev, dt)
+    tiles = [rn(B2, h, nt, 1024) for _ in range(7)]                      # q_t q_v k_t k_v v_t do_t do_v
+    bias = rn(h, nt, nt, 1024) if use_bias else None
+    lse = (torch.randn(B2, h, nt * 32, generator=g).abs() + 6).to(dev)
+    dsum = torch.randn(B2, h, nt * 32, generator=g).to(dev)
+    kb = torch.zeros(B2, nt * 32, device=dev)
+    kb[:, n:], kb[::3, 5:9] = -3.0e38, -1.4e9
+    def run(rows, parts):
+        x = [t[rows].contiguous() for t in tiles + [lse, dsum, kb]]
+        b = x[0].shape[0]
+        dq, dk, dv = (torch.full((b, n, h, 32), float("nan"), dtype=dt, device=dev) for _ in range(3))
+        db = torch.full((parts, h, n, n), float("nan"), device=dev) if use_bias else None
+        _lib.attention_bwd_rows(dq, dk, dv, db, x[7], x[8], *x[:5], bias, x[9], x[5], x[6], B2=b, H=h, N=n, s_b=n * h * 32, s_h=32,
+                                s_n=h * 32, dq_scale=0.17, dk_scale=1.5, dtype=dt, dbias_parts=parts if use_bias else 0)
+        return dq, dk, dv, db
+    whole = run(slice(None), parts)
+    step = 32 if h == 8 or nt < 7 else 16
+    small = [run(slice(i, i + step), 1) for i in range(0, B2, step)]
+    for k in range(3):
+        assert torch.isfinite(whole[k]).all() and torch.equal(whole[k], torch.cat([s[k] for s in small])), "qkv"[k]
+    if use_bias:
+        for s in range(0, parts, 5):
+            assert torch.equal(whole[3][s], run(slice(s, None, parts), 1)[3][0]), s
+
+
 def test_fused_attention_core_backward_fully_masked_rows(dev):
     """A batch row whose keys are all masked gives zero output in the forward pass and zero gradients here."""
     from fastfold_amd.model.fastnn.kernel import fused_attention_core
