@@ -79,7 +79,9 @@ def dtype_tag(dtype: torch.dtype) -> int:
 
 
 def stream_ptr() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device, as ``torch.cuda.current_stream().cuda_stream`` without the two objects in between
+    (every launch asks for it)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def ptr(t):
@@ -348,17 +350,20 @@ SIGNATURES["ffk_attention_pack"] = [ctypes.POINTER(PackDesc), _P]
 
 def attention_pack(jobs, *, B2, H, N, D, dtype, bias=None, bias_t=None, bias_scale=1.0):
     """``jobs``: tuples (src, scale, qk, acc, dsum, other); ``src`` and ``other`` are [B2, H, N, D] views with contiguous
-    channels, or ``src`` the [B2, H, ceil(N/32), 1024] FFK_TILE_QK tiles of an earlier call."""
+    channels, or ``src`` the [B2, H, ceil(N/32), 1024] FFK_TILE_QK tiles of an earlier call.  Either may be given as the address and
+    strides themselves, (address, s_b, s_h, s_n) or (address,) for tiles, and outputs as addresses."""
     d = PackDesc(bias=ptr(bias), bias_t=ptr(bias_t), bias_scale=bias_scale, n=len(jobs), B2=B2, H=H, N=N, D=D, dtype=dtype_tag(dtype))
-    for j, (src, scale, qk, acc, dsum, other) in zip(d.job, jobs):
-        tiled = src.shape[-1] == 1024
-        # raw pointers: the operands may be strided views (their strides go along), which ``ptr`` would refuse
-        j.src, j.qk, j.acc, j.dsum, j.scale, j.tiled = src.data_ptr(), ptr(qk), ptr(acc), ptr(dsum), scale, int(tiled)
-        if not tiled:
-            j.s_b, j.s_h, j.s_n = src.stride()[:3]
-        if other is not None:
-            j.other = other.data_ptr()
-            j.o_sb, j.o_sh, j.o_sn = other.stride()[:3]
+
+    def place(t):
+        # raw pointers: the operands may be strided views (their strides go along)
+        if isinstance(t, tuple):
+            return t
+        return (t.data_ptr(),) if t.shape[-1] == 1024 else (t.data_ptr(), *t.stride()[:3])
+
+    for i, (src, scale, qk, acc, dsum, other) in enumerate(jobs):
+        at = place(src)
+        to = (None, 0, 0, 0) if other is None else place(other)
+        d.job[i] = PackJob(at[0], ptr(qk), ptr(acc), to[0], ptr(dsum), *(at[1:] or (0, 0, 0)), *to[1:], scale, len(at) == 1)
     call("ffk_attention_pack", ctypes.byref(d), stream_ptr())
 
 
@@ -467,9 +472,10 @@ FFK_ACT_GATE_POS = 3
 FFK_LN_BWD_BLOCKS = 1024
 
 
-def attention_fwd_lse(out, lse, q_t, k_t, v_t, bias_t, keybias, tileflags, *, B2, H, N, bias_padded=False):
+def attention_fwd_lse(out, lse, q_t, k_t, v_t, bias_t, keybias, tileflags, *, B2, H, N, bias_padded=False, dtype=None):
     call("ffk_attention_fwd_lse", ptr(out), ptr(lse), ptr(q_t), ptr(k_t), ptr(v_t), ptr(bias_t), ptr(keybias), ptr(tileflags),
-         None, B2, H, N, N, 32, FFK_ATT_BIAS_PADDED if bias_padded else 0, dtype_tag(q_t.dtype), stream_ptr())
+         None, B2, H, N, N, 32, FFK_ATT_BIAS_PADDED if bias_padded else 0, dtype_tag(q_t.dtype if dtype is None else dtype),
+         stream_ptr())
 
 
 def attention_bwd_rows(dq, dk, dv, dbias, lse, dsum, q_t, q_v, k_t, k_v, v_t, bias_t, keybias, do_t, do_v, *, B2, H, N, s_b, s_h,

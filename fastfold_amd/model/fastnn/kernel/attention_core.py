@@ -60,6 +60,12 @@ def _attention_core_wide(q, k, v, mask, bias):
     return out
 
 
+def _at(t, i):
+    """Address and strides of element i of the first of the five dimensions of t."""
+    sb, *rest, _ = t.stride()
+    return (t.data_ptr() + i * sb * t.element_size(), *rest)
+
+
 def _attention_core(q, k, v, mask=None, bias=None, keep=False):
     """Head dims 8, 16 and 32.  ``keep``: also what the backward pass reads - the q and k tiles, the rows' log-sum-exp, the key
     bias of the mask and the bias tiles, one set per b1."""
@@ -76,18 +82,25 @@ def _attention_core(q, k, v, mask=None, bias=None, keep=False):
     fl = torch.empty(b2, nt, dtype=torch.int32, device=dev)
     lse = torch.empty(b1, b2 * h * nt * 32, dtype=torch.float32, device=dev) if keep else None
     q, k, v = (t if t.stride(-1) == 1 else t.contiguous() for t in (q, k, v))
+    mask = mask.to(dt).contiguous() if mask is not None else torch.ones(1, b2, n, dtype=dt, device=dev).expand(b1, b2, n)
+    bscale = 1.0
+    if bias is not None:                      # the kernel exponentiates in base 2
+        bias, bscale = ((bias.contiguous(), _lib.LOG2E) if bias.dtype == dt else ((bias.float() * _lib.LOG2E).to(dt).contiguous(), 1.0))
+    # addresses instead of views: a view of a tensor costs the host as much as a launch
+    es, tiles = q.element_size(), b2 * h * nt * 1024 * q.element_size()
     for i in range(b1):
         s = i if keep else 0
-        bi, bscale = None, 1.0
-        if bias is not None:                  # the kernel exponentiates in base 2
-            bi, bscale = ((bias[i].contiguous(), _lib.LOG2E) if bias.dtype == dt
-                          else ((bias[i].float() * _lib.LOG2E).to(dt).contiguous(), 1.0))
-        _key_bias(kb[s], fl, None if mask is None else mask[i], b2, n, dt, dev)
-        _lib.attention_pack([(q[i], _lib.LOG2E / math.sqrt(d), qk[s, 0], None, None, None), (k[i], 1.0, qk[s, 1], None, None, None),
-                             (v[i], 1.0, None, vt, None, None)],
-                            B2=b2, H=h, N=n, D=d, dtype=dt, bias=bi, bias_t=None if bt is None else bt[s], bias_scale=bscale)
-        _lib.attention_fwd_lse(out[i].view(b2 * n, h * 32), None if lse is None else lse[i], qk[s, 0], qk[s, 1], vt,
-                               None if bt is None else bt[s], kb[s], fl, B2=b2, H=h, N=n)
+        qt = qk.data_ptr() + 2 * s * tiles
+        kbi = kb.data_ptr() + s * b2 * nt * 128
+        bti = None if bt is None else bt.data_ptr() + s * h * nt * nt * 1024 * es
+        _lib.call("ffk_key_bias", kbi, fl.data_ptr(), mask.data_ptr() + i * mask.stride(0) * es, b2, n, n, 1, _lib.dtype_tag(dt),
+                  _lib.stream_ptr())
+        _lib.attention_pack([(_at(q, i), _lib.LOG2E / math.sqrt(d), qt, None, None, None), (_at(k, i), 1.0, qt + tiles, None, None, None),
+                             (_at(v, i), 1.0, None, vt, None, None)],
+                            B2=b2, H=h, N=n, D=d, dtype=dt, bias=None if bt is None else bias.data_ptr() + i * h * n * n * es, bias_t=bti,
+                            bias_scale=bscale)
+        _lib.attention_fwd_lse(out.data_ptr() + i * b2 * n * h * 32 * es, None if lse is None else lse.data_ptr() + i * b2 * h * nt * 128,
+                               qt, qt + tiles, vt, bti, kbi, fl, B2=b2, H=h, N=n, dtype=dt)
     if d < 32:
         out = out.view(b1, b2, n, h, 32)[..., :d].reshape(b1, b2, n, h * d)
     return (out, qk, kb, bt, lse) if keep else out
@@ -99,7 +112,9 @@ def _attention_core_backward(qk, v, kb, bt, lse, out, dout, need_dbias):
     dt, dev = v.dtype, v.device
     nt = layouts.n_tiles(n)
     dq, dk, dv = (torch.empty(b1, b2, h, n, 32, dtype=dt, device=dev) for _ in range(3))
-    q_acc, k_acc, v_qk, do_qk, do_acc = torch.empty(5, b2, h, nt, 1024, dtype=dt, device=dev)
+    es, tiles = v.element_size(), b2 * h * nt * 1024 * v.element_size()
+    work = torch.empty(5, b2, h, nt, 1024, dtype=dt, device=dev)
+    q_acc, k_acc, v_qk, do_qk, do_acc = (work.data_ptr() + j * tiles for j in range(5))
     dsum = torch.empty(b2 * h * nt * 32, dtype=torch.float32, device=dev)
     parts, dbias = 0, None
     if need_dbias and bt is not None:
@@ -108,14 +123,18 @@ def _attention_core_backward(qk, v, kb, bt, lse, out, dout, need_dbias):
         part = torch.empty(parts, h, n, n, dtype=torch.float32, device=dev)
         dbias = torch.empty(b1, h, n, n, dtype=dt, device=dev)
     v = v if v.stride(-1) == 1 else v.contiguous()
+    rows = (n * h * d, d, h * d)                                     # strides of dout and out as [b2, h, n, d]
     for i in range(b1):
-        do_ = dout[i].view(b2, n, h, d).permute(0, 2, 1, 3)          # [b2, h, n, d] views: re-tiled as they lie
-        o_ = out[i].view(b2, n, h, d).permute(0, 2, 1, 3)
-        _lib.attention_pack([(qk[i, 0], 1.0, None, q_acc, None, None), (qk[i, 1], 1.0, None, k_acc, None, None),
-                             (v[i], 1.0, v_qk, None, None, None), (do_, 1.0, do_qk, do_acc, dsum, o_)],
+        qt = qk.data_ptr() + 2 * i * tiles
+        off, grad = i * b2 * n * h * d * es, i * b2 * h * n * 32 * es
+        _lib.attention_pack([((qt,), 1.0, None, q_acc, None, None), ((qt + tiles,), 1.0, None, k_acc, None, None),
+                             (_at(v, i), 1.0, v_qk, None, None, None),
+                             ((dout.data_ptr() + off, *rows), 1.0, do_qk, do_acc, dsum, (out.data_ptr() + off, *rows))],
                             B2=b2, H=h, N=n, D=d, dtype=dt)
-        _lib.attention_bwd_rows(dq[i], dk[i], dv[i], part if parts else None, lse[i], dsum, qk[i, 0], q_acc, qk[i, 1], k_acc, v_qk,
-                                None if bt is None else bt[i], kb[i], do_qk, do_acc, B2=b2, H=h, N=n, s_b=h * n * 32, s_h=n * 32,
+        _lib.attention_bwd_rows(dq.data_ptr() + grad, dk.data_ptr() + grad, dv.data_ptr() + grad, part if parts else None,
+                                lse.data_ptr() + i * b2 * h * nt * 128, dsum, qt, q_acc, qt + tiles, k_acc, v_qk,
+                                None if bt is None else bt.data_ptr() + i * h * nt * nt * 1024 * es, kb.data_ptr() + i * b2 * nt * 128,
+                                do_qk, do_acc, B2=b2, H=h, N=n, s_b=h * n * 32, s_h=n * 32,
                                 s_n=32, dq_scale=1.0 / math.sqrt(d), dk_scale=1.0 / _lib.LOG2E, dtype=dt, dbias_parts=parts)
         if parts and h * n * n % 4 == 0:
             _lib.slice_sum(dbias[i], part, slices=parts, N=1, K=h * n * n, o_map=(1, 0, 0, 1), dtype=dt)

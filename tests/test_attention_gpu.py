@@ -432,6 +432,29 @@ def test_attention_backward_pairs_match_single_tiles(dev, B2, h, n, parts, use_b
             assert torch.equal(whole[3][s], run(slice(s, None, parts), 1)[3][0]), s
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b1,b2,h,n,d", [(2, 3, 4, 40, 32), (3, 2, 8, 33, 8)])
+def test_fused_attention_core_takes_views(dev, dtype, b1, b2, h, n, d):
+    """Operands as views of one projection, offset and strided, and a bias of another order: the bits of contiguous ones, forward and
+    backward, for every element of the first dimension."""
+    from fastfold_amd.model.fastnn.kernel import fused_attention_core
+    g = torch.Generator().manual_seed(n)
+    qkv = torch.randn(b1, b2, n, 3, h, d, generator=g).to(dev, dtype)
+    bias = torch.randn(n, n, h, b1, generator=g).to(dev, dtype)
+    mask = (torch.rand(b2, n, b1, generator=g) > 0.2).to(dev, dtype)
+    dout = torch.randn(b1, h * d, b2, n, generator=g).to(dev, dtype).permute(0, 2, 3, 1)
+    args = [qkv[:, :, :, j].permute(0, 1, 3, 2, 4) for j in range(3)] + [mask.permute(2, 0, 1), bias.permute(3, 2, 0, 1)]
+    res = []
+    for as_is in (True, False):
+        x = [(t if as_is else t.contiguous()).detach() for t in args]
+        for j in (0, 1, 2, 4):
+            x[j].requires_grad_(True)
+        out = fused_attention_core(*x)
+        res.append([out] + list(torch.autograd.grad(out, [x[0], x[1], x[2], x[4]], dout if as_is else dout.contiguous())))
+    for a, b in zip(*res):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
 def test_fused_attention_core_backward_fully_masked_rows(dev):
     """A batch row whose keys are all masked gives zero output in the forward pass and zero gradients here."""
     from fastfold_amd.model.fastnn.kernel import fused_attention_core
