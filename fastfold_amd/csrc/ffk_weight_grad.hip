@@ -13,8 +13,11 @@
 //          with the column index so that neither the stores (columns 8 apart) nor the fragment reads (adjacent columns) meet
 //          in one bank group.  The permutes cost a fifth of the MFMA time.
 //   fp32   v_mfma_f32_32x32x2_f32 takes one element per lane: rows stay as they are.
-// Bound: the reads of y and x (from HBM or the last-level cache).  65 536 x 640 by 65 536 x 128, bf16: library slab GEMM +
-// reduction 75 + 24 us, this pair 29 + 6 us.
+// Bound: the reads of y and x (from HBM or the last-level cache), in bf16; the matrix pipe in fp32.  The rows of a step are requested
+// before the products of the step before it and nothing looks at them in between: the rows past the end of a slice, which have to be
+// zeroed, are a step of their own behind the loop (as conditions of every load they made each step wait for its rows).
+// 65 536 rows, us of the first launch, before and after: 640 x 128 36.9, 26.1, 512 x 128 27.9, 23.5; 32 768 rows, 1 032 x 256 50.7,
+// 35.4; fp32 126.8, 113.3, 93.0, 86.3, 208, 187; the sums over the slices 5 .. 7 us.
 #include "ffk_common.h"
 #include <type_traits>
 
@@ -38,12 +41,57 @@ __device__ __forceinline__ long wg_row(unsigned m, unsigned inner, long so, long
     return (long)hi * so + (long)(m - hi * inner) * si;
 }
 
-template <typename T>
+// The rows m, m + RS, m + 2 RS .. of an operand that a thread fetches, a group every MB rows: no division and no multiplication per
+// row - the offset moves by a step the launch fixes, and by another one where the inner index wraps (FLAT: it never does; a kernel of
+// its own, because a branch between the two makes the compiler wait for the loads it merges).
+template <typename T, int RS, int MB, bool FLAT> struct RowWalk {
+    const T* p;                             // this thread's column in row 0
+    long off, row_inc, group_inc, wrap;     // of the group's first row; per row; per group; where lo passes inner
+    unsigned lo, inner, row_lo, group_lo;
+    __device__ __forceinline__ void init(const T* base, unsigned m, unsigned inner_, unsigned M, long so, long si) {
+        p = base;
+        inner = inner_ < M ? inner_ : 0x80000000u;          // rows and steps together stay below: no wrap
+        const unsigned hi = FLAT ? 0u : m / inner;
+        lo = m - hi * inner;
+        off = (long)hi * so + (long)lo * si;
+        row_lo = RS % inner;
+        group_lo = MB % inner;
+        row_inc = FLAT ? RS * si : (long)(RS / inner) * so + (long)row_lo * si;
+        group_inc = FLAT ? MB * si : (long)(MB / inner) * so + (long)group_lo * si;
+        wrap = so - (long)inner * si;
+    }
+    template <int N> __device__ __forceinline__ void fetch(Vec16<T>* v) {          // N rows of the group, on to the next group
+        long o = off;
+        unsigned l = lo;
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+            v[e] = ld16(p + (FLAT ? off + e * row_inc : o));
+            if (!FLAT) {
+                o += row_inc;
+                l += row_lo;
+                if (l >= inner) {
+                    l -= inner;
+                    o += wrap;
+                }
+            }
+        }
+        off += group_inc;
+        if (!FLAT) {
+            lo += group_lo;
+            if (lo >= inner) {
+                lo -= inner;
+                off += wrap;
+            }
+        }
+    }
+};
+
+template <typename T, bool FLAT>
 __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs a) {
     constexpr bool BF = std::is_same<T, bf16_t>::value;
     constexpr int MB = BF ? 64 : 32;                       // rows per step
     constexpr int BUF = BF ? WG_T * 128 : MB * 640;        // bytes of one operand's buffer
-    constexpr int NP = BF ? 8 : 4;                         // 16-byte loads per thread and step
+    constexpr int NP = BF ? 8 : 4;                         // 16-byte loads per thread, operand and step
     extern __shared__ __align__(16) unsigned char smem[];  // [2 buffers][y | x]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -55,43 +103,42 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
     const int n0 = (int)(item % tn) * WG_T, k0 = (int)((item / tn) % tk) * WG_T, slice = (int)(item / (tn * tk));
     const int m_begin = slice * a.rows_per_slice;
     const int m_end = m_begin + a.rows_per_slice < a.M ? m_begin + a.rows_per_slice : a.M;
-    const bool y_flat = a.y_inner >= (unsigned)a.M, x_flat = a.x_inner >= (unsigned)a.M;
 
-    // bf16: threads 0 .. 127 fetch y, 128 .. 255 x, an 8 x 8 block each.  fp32: every thread half of its vectors from each.
-    Vec16<T> pre[NP * (BF ? 1 : 2)];
+    // bf16: waves 0 and 1 fetch y, 2 and 3 x, an 8 x 8 block per thread.  fp32: every thread half of its vectors from each.
     const int bt = BF ? (tid & 127) : tid;
     const int cb = BF ? (bt & 15) : (bt & 31);             // column block (8 or 4 columns)
     const int rb = BF ? (bt >> 4) : (bt >> 5);             // row block
-    const bool is_x = BF && tid >= 128;
-    auto fetch = [&](int m0) {
-        if constexpr (BF) {
-            const T* base = (const T*)(is_x ? a.x : a.y);
-            int col = (is_x ? k0 : n0) + cb * 8;
-            const int cols = is_x ? a.K : a.N;
-            col = col < cols ? col : cols - 8;             // clamped columns are never stored
+    const bool is_x = BF && wave >= 2;                     // of the whole wave
+    constexpr int VEC = DT<T>::VEC, RS = BF ? 1 : 8;       // row e of a thread: first row + RS e
+    const unsigned r0 = BF ? rb * 8 : rb;
+    RowWalk<T, RS, MB, FLAT> wy, wx;                             // bf16: wy is the walk of the thread's one operand
+    auto column = [&](int first, int cols) {               // clamped columns are never stored
+        const int c = first + cb * VEC;
+        return c < cols ? c : cols - VEC;
+    };
+    if (is_x) wy.init((const T*)a.x + column(k0, a.K), m_begin + r0, a.x_inner, a.M, a.x_so, a.x_si);
+    else wy.init((const T*)a.y + column(n0, a.N), m_begin + r0, a.y_inner, a.M, a.y_so, a.y_si);
+    if (!BF) wx.init((const T*)a.x + column(k0, a.K), m_begin + r0, a.x_inner, a.M, a.x_so, a.x_si);
+    auto fetch_rows = [&](Vec16<T>* pre) __attribute__((always_inline)) {      // a whole step: requests only, nothing waits for them here
+        wy.template fetch<NP>(pre);
+        if (!BF) wx.template fetch<NP>(pre + (BF ? 0 : NP));
+    };
+    auto fetch_tail = [&](Vec16<T>* pre, int m0) __attribute__((always_inline)) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int m = m0 + rb * 8 + e;
-                const unsigned mc = (unsigned)(m < m_end ? m : m_end - 1);
-                const long off = is_x ? wg_row(mc, a.x_inner, a.x_so, a.x_si, x_flat) : wg_row(mc, a.y_inner, a.y_so, a.y_si, y_flat);
-                pre[e] = ld16(base + off + col);
-                if (m >= m_end && !is_x) pre[e] = Vec16<T>{};        // rows past the end add nothing
-            }
-        } else {
-            int cy = n0 + cb * 4, cx = k0 + cb * 4;
-            cy = cy < a.N ? cy : a.N - 4;
-            cx = cx < a.K ? cx : a.K - 4;
-#pragma unroll
-            for (int e = 0; e < NP; ++e) {
-                const int m = m0 + rb + 8 * e;
-                const unsigned mc = (unsigned)(m < m_end ? m : m_end - 1);
-                pre[e] = ld16((const T*)a.y + wg_row(mc, a.y_inner, a.y_so, a.y_si, y_flat) + cy);
-                pre[NP + e] = ld16((const T*)a.x + wg_row(mc, a.x_inner, a.x_so, a.x_si, x_flat) + cx);
+        for (int e = 0; e < NP; ++e) {                     // the last rows: clamped, and those past the end add nothing
+            const int m = m0 + r0 + RS * e;
+            const unsigned mc = (unsigned)(m < m_end ? m : m_end - 1);
+            if (BF) {
+                pre[e] = ld16(wy.p + (is_x ? wg_row(mc, a.x_inner, a.x_so, a.x_si, FLAT || a.x_inner >= (unsigned)a.M) : wg_row(mc, a.y_inner, a.y_so, a.y_si, FLAT || a.y_inner >= (unsigned)a.M)));
+                if (m >= m_end && !is_x) pre[e] = Vec16<T>{};
+            } else {
+                pre[e] = ld16(wy.p + wg_row(mc, a.y_inner, a.y_so, a.y_si, FLAT || a.y_inner >= (unsigned)a.M));
+                pre[(BF ? 0 : NP) + e] = ld16(wx.p + wg_row(mc, a.x_inner, a.x_so, a.x_si, FLAT || a.x_inner >= (unsigned)a.M));
                 if (m >= m_end) pre[e] = Vec16<T>{};
             }
         }
     };
-    auto commit = [&](int buf) {
+    auto commit = [&](const Vec16<T>* pre, int buf) __attribute__((always_inline)) {
         unsigned char* sb = smem + buf * 2 * BUF;
         if constexpr (BF) {
             unsigned char* so = sb + (is_x ? BUF : 0);
@@ -100,9 +147,9 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
                 u32x4 lo, hi;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const uint32_t r0 = reinterpret_cast<const u32x4*>(&pre[2 * j])[0][d], r1 = reinterpret_cast<const u32x4*>(&pre[2 * j + 1])[0][d];
-                    lo[j] = __builtin_amdgcn_perm(r1, r0, 0x05040100u);
-                    hi[j] = __builtin_amdgcn_perm(r1, r0, 0x07060302u);
+                    const uint32_t w0 = reinterpret_cast<const u32x4*>(&pre[2 * j])[0][d], w1 = reinterpret_cast<const u32x4*>(&pre[2 * j + 1])[0][d];
+                    lo[j] = __builtin_amdgcn_perm(w1, w0, 0x05040100u);
+                    hi[j] = __builtin_amdgcn_perm(w1, w0, 0x07060302u);
                 }
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
@@ -114,7 +161,7 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
 #pragma unroll
             for (int e = 0; e < NP; ++e) {
                 *reinterpret_cast<Vec16<T>*>(sb + (rb + 8 * e) * 640 + cb * 16) = pre[e];
-                *reinterpret_cast<Vec16<T>*>(sb + BUF + (rb + 8 * e) * 640 + cb * 16) = pre[NP + e];
+                *reinterpret_cast<Vec16<T>*>(sb + BUF + (rb + 8 * e) * 640 + cb * 16) = pre[(BF ? 0 : NP) + e];
             }
         }
     };
@@ -130,29 +177,29 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
 
-    fetch(m_begin);
-    commit(0);
-    lds_barrier();
-    int buf = 0;
-    for (int m0 = m_begin; m0 < m_end; m0 += MB) {
-        const bool more = m0 + MB < m_end;
-        if (more) fetch(m0 + MB);                          // in flight during the products
-        const unsigned char* sy = smem + buf * 2 * BUF;
+    // The products of a step.  The fragments of a K step are requested one K step ahead.
+    auto products = [&](const unsigned char* sy) __attribute__((always_inline)) {
         const unsigned char* sx = sy + BUF;
         if constexpr (BF) {
-#pragma unroll
-            for (int ks = 0; ks < MB / 16; ++ks) {
-                bf16x8 fy[2], fx[2];
+            bf16x8 fy[2][2], fx[2][2];
+            auto read = [&](int ks) __attribute__((always_inline)) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
                     const int n = wn * 64 + i * 32 + l32, k = wk * 64 + i * 32 + l32;
-                    fy[i] = *reinterpret_cast<const bf16x8*>(sy + n * 128 + ((((2 * ks + half) ^ n ^ (n >> 3)) & 7) << 4));
-                    fx[i] = *reinterpret_cast<const bf16x8*>(sx + k * 128 + ((((2 * ks + half) ^ k ^ (k >> 3)) & 7) << 4));
+                    fy[ks & 1][i] = *reinterpret_cast<const bf16x8*>(sy + n * 128 + ((((2 * ks + half) ^ n ^ (n >> 3)) & 7) << 4));
+                    fx[ks & 1][i] = *reinterpret_cast<const bf16x8*>(sx + k * 128 + ((((2 * ks + half) ^ k ^ (k >> 3)) & 7) << 4));
                 }
+            };
+            read(0);
+#pragma unroll
+            for (int ks = 0; ks < MB / 16; ++ks) {
+                if (ks + 1 < MB / 16) read(ks + 1);
+                const bf16x8* y2 = fy[ks & 1];
+                const bf16x8* x2 = fx[ks & 1];
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) Mma<bf16_t>::mma(acc[i][j], fy[i], fx[j]);
+                    for (int j = 0; j < 2; ++j) Mma<bf16_t>::mma(acc[i][j], y2[i], x2[j]);
                 if (sums) {
                     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
                     const bf16x2 ones = {(bf16_t)1.0f, (bf16_t)1.0f};
@@ -160,7 +207,7 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
                     for (int i = 0; i < 2; ++i)
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
-                            const bf16x2 pr = {fy[i][2 * e], fy[i][2 * e + 1]};
+                            const bf16x2 pr = {y2[i][2 * e], y2[i][2 * e + 1]};
                             cs[i] = __builtin_amdgcn_fdot2_f32_bf16(pr, ones, cs[i], false);
                         }
                 }
@@ -184,11 +231,31 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
                 }
             }
         }
-        if (!more) break;
-        commit(buf ^ 1);                                   // the other buffer: its last readers passed the barrier below
+    };
+
+    constexpr int NV = NP * (BF ? 1 : 2);
+    const int whole = (m_end - m_begin) / MB;
+    const bool tail = (m_end - m_begin) % MB != 0;
+    {
+        Vec16<T> pre[NV];
+        if (whole > 0) fetch_rows(pre);
+        else fetch_tail(pre, m_begin);
+        commit(pre, 0);
+    }
+    lds_barrier();
+    int buf = 0;
+    auto step = [&](auto tail_c) __attribute__((always_inline)) {          // products of one buffer while the rows of the next are on their way
+        Vec16<T> pre[NV];
+        if constexpr (decltype(tail_c)::value) fetch_tail(pre, m_begin + whole * MB);
+        else fetch_rows(pre);
+        products(smem + buf * 2 * BUF);
+        commit(pre, buf ^ 1);                              // its last readers passed the barrier below
         lds_barrier();
         buf ^= 1;
-    }
+    };
+    for (int i = 1; i < whole; ++i) step(std::false_type());
+    if (tail && whole > 0) step(std::true_type());
+    products(smem + buf * 2 * BUF);
     float* part = a.part + (long)slice * a.N * a.K;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -267,13 +334,18 @@ template <typename T>
 int launch_weight_grad(const WgArgs& a, void* out, long n_out, void* colsum, long cs_first, long cs_count, float* acc, long o_inner, long o_so, long o_si, long o_sk, int flags,
                        hipStream_t st) {
     const size_t smem = std::is_same<T, bf16_t>::value ? 4 * (size_t)WG_T * 128 : 4 * (size_t)32 * 640;
-    static FfkLdsReservation lds_reserved;
-    int rc = ffk_reserve_lds(lds_reserved, (const void*)weight_grad_kernel<T>, smem, "ffk_weight_grad");
-    if (rc != FFK_OK) return rc;
     const long items = (long)ffk_cdiv(a.N, WG_T) * ffk_cdiv(a.K, WG_T) * a.slices;
     FFK_REQUIRE(items < (1L << 31) - 8, FFK_ERR_SHAPE, "ffk_weight_grad: %ld workgroups exceed the grid limit", items);
-    weight_grad_kernel<T><<<(unsigned)(8 * ffk_cdiv(items, 8)), WG_THREADS, smem, st>>>(a);
-    rc = ffk_check_launch("ffk_weight_grad");
+    auto launch = [&](auto flat_c) {
+        constexpr bool FLAT = decltype(flat_c)::value;
+        static FfkLdsReservation lds_reserved;
+        const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)weight_grad_kernel<T, FLAT>, smem, "ffk_weight_grad");
+        if (rc_lds != FFK_OK) return rc_lds;
+        weight_grad_kernel<T, FLAT><<<(unsigned)(8 * ffk_cdiv(items, 8)), WG_THREADS, smem, st>>>(a);
+        return ffk_check_launch("ffk_weight_grad");
+    };
+    const bool flat = a.y_inner >= (unsigned)a.M && a.x_inner >= (unsigned)a.M;
+    const int rc = flat ? launch(std::true_type()) : launch(std::false_type());
     if (rc != FFK_OK) return rc;
     const long nk = (long)a.N * a.K;
     const SliceSum m = slice_sum(out, a.part, acc, n_out * a.K, a.K, o_inner, o_so, o_si, o_sk, nk);

@@ -44,17 +44,20 @@ def _rows(x, w, out, *, M, K, N, a_map=None, ln=None, bias=None, act=0, gate=Non
         _lib.fused_linear(x, w, tiles, M=M, K=K, a_inner=inner, a_so=so, a_si=si, ln=ln, w_row_off=w_row + t0 * 128)
 
 
-def _slices(M, N, K):
-    """Slices of the rows of a weight gradient: about two workgroups per CU over its 128 x 128 output tiles, at most 64 MB of
-    partial sums, whole 64-row steps."""
+def _slices(M, N, K, dtype):
+    """Slices of the rows of a weight gradient: two workgroups per CU over its 128 x 128 output tiles, at most 64 MB of partial sums,
+    whole 64-row steps and two of them at least.  Small outputs take half the slices: the sums over them cost more than the second
+    workgroup saves (us with 512 and 256 workgroups, bf16: 65 536 x 128 x 128 22.3, 18.3, 65 536 x 512 x 128 30.6, 29.1, but
+    65 536 x 640 x 128 33.1, 38.9; fp32: 38.2, 35.2, but 93.3, 101.1)."""
     tiles = ((N + 127) // 128) * ((K + 127) // 128)
     steps = (M + 63) // 64
-    s = max(1, min(512 // tiles, (64 << 20) // (4 * N * K), steps))
+    groups = 256 if tiles <= (4 if dtype == torch.bfloat16 else 1) else 512
+    s = max(1, min(groups // tiles, (64 << 20) // (4 * N * K), (steps + 1) // 2))
     return (steps + (steps + s - 1) // s - 1) // ((steps + s - 1) // s)
 
 
 def _wgrad(out, colsum, y, x, *, M, N, K, dtype, device, y_map=None, x_map=None, **kw):
-    s = _slices(M, N, K)
+    s = _slices(M, N, K, dtype)
     ws = alloc((s * N * (K + 1),), torch.float32, device)
     _lib.weight_grad(out, colsum, ws, y, x, M=M, N=N, K=K, slices=s, dtype=dtype, y_map=_plain(M, N) if y_map is None else y_map,
                      x_map=_plain(M, K) if x_map is None else x_map, **kw)

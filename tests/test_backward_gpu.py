@@ -43,6 +43,35 @@ def test_weight_grad(dev, dtype, M, N, K, slices):
 
 
 @pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("M,slices", [(63, 1), (64, 1), (65, 1), (640, 3), (1050, 4)])
+@pytest.mark.parametrize("yi,xi", [(1, None), (None, 3), (7, 31), (50, 70), (2, 35), (None, None)])
+def test_weight_grad_row_maps(dev, dtype, M, slices, yi, xi):
+    """Rows through maps whose inner index wraps within the rows of a thread, several times a row, between steps or never: the bits of
+    the same rows laid out one after the other."""
+    from fastfold_amd import _lib
+    N, K = 136, 264
+    g = torch.Generator().manual_seed(M)
+    out, cs = [], []
+    y, x = torch.randn(M, N, generator=g).to(dev, dtype), torch.randn(M, K, generator=g).to(dev, dtype)
+    ws = torch.empty(slices * N * (K + 1), device=dev)
+
+    def mapped(t, inner):                          # row m = hi * inner + lo of t at (lo, hi) of a [inner, outer] table with a gap
+        if inner is None:
+            return t, (M, 0, t.shape[1])
+        outer = (M + inner - 1) // inner
+        tab = torch.full((inner, outer, t.shape[1] + 8), float("nan"), device=dev, dtype=dtype)
+        m = torch.arange(M, device=dev)
+        tab[m % inner, m // inner, :t.shape[1]] = t
+        return tab, (inner, t.shape[1] + 8, outer * (t.shape[1] + 8))
+    for a, b in ((None, None), (yi, xi)):
+        (yt, ym), (xt, xm) = mapped(y, a), mapped(x, b)
+        out.append(torch.full((N, K), float("nan"), device=dev, dtype=dtype))
+        cs.append(torch.full((N,), float("nan"), device=dev, dtype=dtype))
+        _lib.weight_grad(out[-1], cs[-1], ws, yt, xt, M=M, N=N, K=K, slices=slices, dtype=dtype, y_map=ym, x_map=xm)
+    assert torch.isfinite(out[0]).all() and torch.equal(*out) and torch.equal(*cs)
+
+
+@pytest.mark.parametrize("dtype", DT)
 @pytest.mark.parametrize("rows,C", [(1, 64), (33, 128), (5000, 256), (70001, 128)])
 def test_layernorm_bwd_rows(dev, dtype, rows, C):
     from fastfold_amd import _lib
