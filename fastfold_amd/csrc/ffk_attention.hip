@@ -116,6 +116,11 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
     constexpr int NVL = (NTILES * TILE_VECS + ATT_THREADS - 1) / ATT_THREADS;   // vectors per thread per step
     extern __shared__ __align__(16) unsigned char att_smem[];
     constexpr int NSLOT = 3;                      // operand ring: the tile in use and two in flight behind it
+    // fp32: the bias is added to the scores as it is read (16 LDS reads and additions a lane and tile).  Through the matrix pipe, as
+    // in bf16, where it costs two products of 32 cycles, it was a third of all products: 16 of 64 cycles.  128 x 8 heads of 256 x 256:
+    // 121.8 -> 97.3 us, 391 x 391 355 -> 274.  Its tiles lie [query][key] transposed to what a lane needs (16 keys of one query); the 16-byte pieces of a tile go
+    // to LDS permuted, so that the lanes of a read - four adjacent queries to a piece - meet 16 pieces in 16 bank groups.
+    constexpr bool BIAS_ADD = HAS_BIAS && sizeof(T) == 4;
     T* lds = reinterpret_cast<T*>(att_smem);      // [NSLOT][NTILES][1024] operand slots, then [ATT_THREADS][16] gate values
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -223,7 +228,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
     }
 
     Frag ident[NF];
-    if (HAS_BIAS) {
+    if (HAS_BIAS && !BIAS_ADD) {
 #pragma unroll
         for (int i = 0; i < NF; ++i) ident[i] = identity_frag<T>(i, l32, half);
     }
@@ -249,6 +254,11 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
     // at the top of the loop is what orders them.
     const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)att_smem;
     const unsigned lane_off = lane * 16 * Ops16<T>::NV;   // byte offset of this lane's 16 elements; the base address is scalar
+    // piece c of lane L's 16 elements (key L % 32, queries 16 (L / 32) + 4 c ..) goes to place L ^ (c + 8 (L / 32)); a wave fetches one c
+    const unsigned bias_off = BIAS_ADD ? (lane ^ ((wave & 3) | half << 3)) * 16 * Ops16<T>::NV : lane_off;
+    static_assert(!BIAS_ADD || (TILE_VECS == 256 && ATT_THREADS == 512), "vectors of a wave's requests: number wave % 4 of every lane");
+    const int bq = (l32 & 15) >> 2, bhi = l32 >> 4;            // this lane's query: piece and half of the bias tile's rows
+    const T* bias_lane = lds + (4 + qsel) * 1024 + (bq * 64 + bhi * 32 + half * 4) * 4 + (l32 & 3);
     auto fetch = [&](int kt, int slot) {
 #pragma unroll
         for (int i = 0; i < NVL; ++i) {
@@ -256,7 +266,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
             const unsigned dst = lds_base + (slot * NTILES * TILE_VECS + wave * 64 + i * ATT_THREADS) * 16;
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(gp), "s"(dst)
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(BIAS_ADD && i * ATT_THREADS >= 4 * TILE_VECS ? bias_off : lane_off), "s"(gp), "s"(dst)
                          : "memory", "m0");
 #pragma clang diagnostic pop
         }
@@ -298,7 +308,15 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
             Ops16<T> kc, bc;
             if constexpr (HD == 32) kc.load_lds(buf + bsel * 1024, lane);
             else kc.v[0] = ld16(buf + bsel * 1024 + ((c0 >> 4) * 64 + lane) * VEC);
-            if (HAS_BIAS) bc.load_lds(buf + (4 + qsel) * 1024, lane);
+            if (HAS_BIAS && !BIAS_ADD) bc.load_lds(buf + (4 + qsel) * 1024, lane);
+            float ba[BIAS_ADD ? 16 : 1];
+            if constexpr (BIAS_ADD) {                          // key 8 g + 4 half + e of the tile, at place key ^ (bq + 8 bhi)
+                const T* bp = bias_lane + (buf - lds);
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) ba[4 * g + e] = (float)bp[((8 * g ^ 8 * bhi) + (e ^ bq)) * 4];
+            }
             s = negm;
             // FFK_ATT_HALF_K: elements 8 .. 15 of every lane's sixteen are zero padding in q and k (narrow heads): the
             // second half of the score product adds nothing and is skipped
@@ -308,7 +326,10 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
 #pragma unroll
                 for (int i = NF / 2; i < NF; ++i) MM::mma(s, kc.frag(i), qf.frag(i));
             }
-            if (HAS_BIAS) {
+            if constexpr (BIAS_ADD) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) s[v] += ba[v];
+            } else if (HAS_BIAS) {
 #pragma unroll
                 for (int i = 0; i < NF; ++i) MM::mma(s, bc.frag(i), ident[i]);
             }

@@ -24,13 +24,14 @@
 //                             the chip when H * QT * KT alone is a few hundred tiles) are left as partial sums the
 //                             caller adds up (ffk_attention_bwd_rows) or added with one fp32 atomic per element.
 // They take the pair bias from the same operand tiles as the forward kernel: added to the scores by a product with
-// an identity operand, in the last two with the roles of the two operands exchanged (rows = queries).
+// an identity operand, in the last two with the roles of the two operands exchanged (rows = queries); in fp32 dq and
+// dk / dv read its values in the order of the scores and add them.
 // Every operand arrives in the tile order its role needs.  Waves load their tiles straight from global memory, each
 // operand of the next step requested as soon as its registers are free, and no LDS is used: what bounds the kernels is
 // the latency of that chain and the exponentials, with three waves per SIMD to cover it, or two of two tiles each (NT = 2:
 // the operands of the walk are read once for both).  128 x 8 heads of 256 x 256 logits, bf16, one tile per wave and loads
 // that waited for each other, requested in time, two tiles per wave: dq 39.6, 38.8, 35.0 us, dk / dv 56.5, 56.2, 46.1,
-// d bias 41.5, 40.5, 32.1; fp32, the first two: dq 198, 174, dk / dv 232, 223, d bias 127, 121.
+// d bias 41.5, 40.5, 32.1; fp32, the first two: dq 198, 173, dk / dv 232, 229, d bias 127, 121.
 #include "ffk_common.h"
 #include <initializer_list>
 #include <type_traits>
@@ -97,6 +98,10 @@ __device__ __forceinline__ typename Mma<T>::Frag identity_frag(int i, int l32, i
     return f;
 }
 
+// fp32: the bias is added to the scores; through the matrix pipe, as in bf16, it was a product of 16 x 64 cycles beside the three (four)
+// that the walk is made of (128 x 8 heads of 256 x 256: dq 173 -> 150, dk / dv 229 -> 195 us).
+template <typename T> constexpr bool bias_add = sizeof(T) == 4;
+
 // Workgroup -> logical block.  The hardware hands consecutive workgroup ids to the eight XCDs in turn, each with its own
 // L2; the launches round their grids up to a multiple of eight and every XCD takes a contiguous eighth of the logical
 // order, so that the waves that walk the same k / v (or q / do) tiles run behind one L2.
@@ -130,6 +135,7 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? (NT == 1 ? 3 : 2) 
     int Nk, float dq_scale, long part_q, long part_k, OutMap om, int bias_pad) {
     typedef Mma<T> MM;
     typedef typename MM::Frag Frag;
+    constexpr bool BIAS_ADD = bias_add<T>;
     constexpr int NF = 16 / MM::KLANE;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l32 = lane & 31, half = lane >> 5;
@@ -240,6 +246,8 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? (NT == 1 ? 3 : 2) 
 #pragma unroll
     for (int t = 0; t < NT; ++t)
         bias_row[t] = HAS_BIAS ? bias_t + ((((long)h * QT + qtile(t)) * (KT + bias_pad)) << 10) + l32 * 16 : nullptr;
+    const T* bias_tile = HAS_BIAS ? bias_t + ((((long)h * QT + qt) * (KT + bias_pad)) << 10) + (4 * half + 32 * (l32 >> 4)) * 16 + (l32 & 15) : nullptr;
+    float ba[HAS_BIAS && BIAS_ADD ? 16 : 1];
     const long krow = (bh * KT) << 10;
     auto load_mask = [&](int kt) {
 #pragma unroll
@@ -251,7 +259,11 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? (NT == 1 ? 3 : 2) 
             kc[p].load_rows(k_qk + p * part_k + krow + ((long)kt << 10) + l32 * 16, half);
             vq[p].load_rows(v_qk + p * part_k + krow + ((long)kt << 10) + l32 * 16, half);
         }
-        if (HAS_BIAS) {
+        if constexpr (HAS_BIAS && BIAS_ADD) {                  // keys 8 g + 4 half + e of this lane's query
+            const T* bp = bias_tile + ((long)kt << 10);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) ba[v] = (float)bp[(8 * (v >> 2) + (v & 3)) * 16];
+        } else if (HAS_BIAS) {
 #pragma unroll
             for (int t = 0; t < NT; ++t) bc[t].load_rows(bias_row[t] + ((long)kt << 10), half);
         }
@@ -280,7 +292,10 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? (NT == 1 ? 3 : 2) 
 #pragma unroll
                 for (int i = 0; i < NF; ++i) MM::mma(dp[t], vq[p].frag(i), dof[t][p].frag(i));   // dP^T[key, q] = v[key] . do[q]
             }
-            if (HAS_BIAS) {
+            if constexpr (HAS_BIAS && BIAS_ADD) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) s[t][v] += ba[v];
+            } else if (HAS_BIAS) {
 #pragma unroll
                 for (int i = 0; i < NF; ++i) MM::mma(s[t], bc[t].frag(i), ident[i]);
             }
@@ -334,6 +349,7 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? (NT == 1 ? 3 : 2) 
     long part_q, long part_k, OutMap om, int bias_pad) {
     typedef Mma<T> MM;
     typedef typename MM::Frag Frag;
+    constexpr bool BIAS_ADD = bias_add<T>;
     constexpr int NF = 16 / MM::KLANE;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l32 = lane & 31, half = lane >> 5;
@@ -394,7 +410,15 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? (NT == 1 ? 3 : 2) 
         }
         if (bias_t) {
 #pragma unroll
-            for (int t = 0; t < NT; ++t) bc[t].load_rows(bias_col[t] + (((long)qt * (KT + bias_pad)) << 10), half);
+            for (int t = 0; t < NT; ++t) {
+                const T* bp = bias_col[t] + (((long)qt * (KT + bias_pad)) << 10);
+                if constexpr (BIAS_ADD) {                      // queries 8 g + 4 half .. of this lane's key
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) bc[t].v[g] = ld16(bp + (g >> 1) * 512 + 8 * (g & 1) + 4 * half);
+                } else {
+                    bc[t].load_rows(bp, half);
+                }
+            }
         }
     };
     auto load_acc = [&](int qt) {
@@ -424,9 +448,14 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? (NT == 1 ? 3 : 2) 
 #pragma unroll
                 for (int i = 0; i < NF; ++i) MM::mma(dp[t], doc[p].frag(i), vf[t][p].frag(i));     // dP[q, key] = do[q] . v[key]
             }
-            if (bias_t) {                                                           // S += I . bias (rows = queries)
+            if (bias_t) {                                                           // S += bias; bf16: I . bias (rows = queries)
+                if constexpr (BIAS_ADD) {
 #pragma unroll
-                for (int i = 0; i < NF; ++i) MM::mma(s[t], ident[i], bc[t].frag(i));
+                    for (int v = 0; v < 16; ++v) s[t][v] += bc[t].f(v);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < NF; ++i) MM::mma(s[t], ident[i], bc[t].frag(i));
+                }
             }
         }
         load_scores(next);
