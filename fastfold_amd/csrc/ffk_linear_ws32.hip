@@ -84,9 +84,7 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
             const float* p = A + (long)hi * d.a_so + (long)lo * d.a_si + (long)(tid / BM) * d.a_cs;
 #pragma unroll
             for (int i = 0; i < 4 * NP; ++i) pre[i >> 2][i & 3] = p[(long)(i * (G::THREADS / BM)) * d.a_cs];
-            return;
-        }
-        if (a_flat) {
+        } else if (a_flat) {
 #pragma unroll
             for (int i = 0; i < NP; ++i) {
                 const int m = slab * BM + r0 + RPP * i;

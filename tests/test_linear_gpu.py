@@ -719,3 +719,27 @@ def test_opm_workgroup_sizes_agree(dev, s):
         for r in (32, 128, 160):
             y, t = run(r, xt)
             assert torch.equal(y, whole[0][:r, :r]) and (not xt or torch.equal(t, whole[1][:r, :r])), (r, xt)
+
+
+@pytest.mark.parametrize("B,N", [(1, 1), (3, 37), (64, 64), (131, 96)])
+def test_fp32_channel_major_rows_masked(dev, B, N):
+    """A row mask with strides of its own on a channel-major operand, over 32 and 64 rows per workgroup and outputs of either
+    order: masked rows are zero, the others are the products (32-bit sums: 1e-5 of the largest)."""
+    from fastfold_amd import _lib
+    g = torch.Generator().manual_seed(B * N)
+    K, M, kp = 128, B * N, (N + 3) // 4 * 4
+    xt, w, b = torch.randn(K, B, kp, generator=g), torch.randn(128, K, generator=g) / K ** 0.5, torch.randn(128, generator=g)
+    ln, mask = (1 + 0.1 * torch.randn(K, generator=g), 0.1 * torch.randn(K, generator=g)), (torch.rand(N, B, generator=g) > 0.3).float()
+    x = xt[:, :, :N].reshape(K, M).t().numpy()
+    xt, w, b, mask, ln = xt.to(dev), w.to(dev), b.to(dev), mask.to(dev), tuple(t.to(dev) for t in ln)
+    for norm in (True, False):
+        out, cm = torch.full((M, 128), 7.0, device=dev), torch.full((128, B * kp), 7.0, device=dev)
+        mk = dict(rowmask=mask, m_so=1, m_si=B)
+        tiles = [_lib.make_tile(out, bias=b, inner=N, s_o=N * 128, s_i=128, **mk)]
+        if norm:
+            tiles.append(_lib.make_tile(cm, bias=b, inner=N, s_o=kp, s_i=1, s_h=32 * B * kp, s_d=B * kp, **mk))
+        _lib.fused_linear(xt, torch.cat([w, w]), tiles, M=M, K=K, a_inner=N, a_so=kp, a_si=1, a_chanmajor=True, a_cs=B * kp, ln=ln if norm else None)
+        ref = ops_np.linear(ops_np.layer_norm(x, *(t.cpu() for t in ln)) if norm else x, w.cpu(), b.cpu()) * _np(mask).T.reshape(M, 1)
+        assert np.abs(_np(out) - ref).max() <= 1e-5 * max(np.abs(ref).max(), 1.0)
+        if norm:
+            assert np.abs(_np(cm).reshape(128, B, kp)[:, :, :N].reshape(128, M).T - ref).max() <= 1e-5 * max(np.abs(ref).max(), 1.0)
