@@ -51,6 +51,9 @@ __host__ __device__ __forceinline__ bool w3_by_rows(const ffk_tile& t) {
     return t.kind == FFK_TILE_QK || t.kind == FFK_TILE_ACC || t.kind == FFK_TILE_BIAS || (t.kind == FFK_TILE_STRIDED && t.s_d == 1);
 }
 
+// 32-channel block of the output that unit u of its tile makes
+template <bool GLU> __device__ __forceinline__ int w3_sub(const ffk_tile& t, int u) { return GLU && t.glu ? (u & 3) >> 1 : u & 3; }
+
 // GLU: the launch has GLU tiles; the slots of a wave are then value and gate of one unit (a plain unit leaves the second empty)
 // CM: element (m, k) of the operand at a + k * a_cs + rowoffset(m) (ONE only)
 template <int K, bool GLU, bool ONE, int BM, bool CM>
@@ -183,7 +186,7 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
     auto store = [&](int u, const float* bias, const f32x16& acc, const f32x16& accg, int m0g, const float* sm, [[maybe_unused]] const f32x4 (&rv)[4]) __attribute__((always_inline)) {
         const ffk_tile& t = d.tiles[u >> 2];
         const bool by_rows = w3_by_rows(t), glu = GLU && t.glu != 0;
-        const int sub = glu ? (u & 3) >> 1 : u & 3, left = t.ncols - 32 * sub;        // 32-channel block of the output, channels left
+        const int sub = w3_sub<GLU>(t, u), left = t.ncols - 32 * sub;      // channels left
         // channels of this lane: by rows 16 half + v (through tau) or 8 a + 4 half + b (ACC); by columns l32
         const bool nat = t.kind == FFK_TILE_ACC;
         const float* bp = bias + (by_rows ? (nat ? 4 : 16) * half : l32);
@@ -354,10 +357,10 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
         f32x4 rv[4];
         if constexpr (ONE) {                             // the residual arrives behind the products
             const ffk_tile& t = d.tiles[u >> 2];
-            const int mrow = m0g + n32, left = t.ncols - 32 * (u & 3);
+            const int sub = w3_sub<GLU>(t, u), mrow = m0g + n32, left = t.ncols - 32 * sub;
             if (t.resid && mrow < M) {
                 const unsigned hi = t.inner < M ? (unsigned)mrow / (unsigned)t.inner : 0u, lo = (unsigned)mrow - hi * (unsigned)t.inner;
-                const float* r = (const float*)t.resid + (long)(u & 3) * t.s_h + (long)hi * t.s_o + (long)lo * t.s_i + 16 * half;
+                const float* r = (const float*)t.resid + (long)sub * t.s_h + (long)hi * t.s_o + (long)lo * t.s_i + 16 * half;
 #pragma unroll
                 for (int a = 0; a < 4; ++a)
                     if (16 * half + 4 * a < left) rv[a] = *reinterpret_cast<const f32x4*>(r + 4 * a);

@@ -743,3 +743,21 @@ def test_fp32_channel_major_rows_masked(dev, B, N):
         assert np.abs(_np(out) - ref).max() <= 1e-5 * max(np.abs(ref).max(), 1.0)
         if norm:
             assert np.abs(_np(cm).reshape(128, B, kp)[:, :, :N].reshape(128, M).T - ref).max() <= 1e-5 * max(np.abs(ref).max(), 1.0)
+
+
+@pytest.mark.parametrize("M,nt,ncols", [(33, 1, 64), (9000, 1, 36), (33000, 1, 64), (130000, 1, 20), (131041, 4, 64), (131041, 4, 44)])
+def test_fp32_glu_tile_with_residual(dev, M, nt, ncols):
+    """GLU channels stored [row][channel] onto a residual, in place, from 32 rows per workgroup to the persistent layout (four tiles):
+    the second unit of 32 channels takes the second half of the residual's (against float64; 2e-5 of the largest)."""
+    from fastfold_amd import _lib
+    g = torch.Generator().manual_seed(M + ncols)
+    K = 128
+    x, b = torch.randn(M, K, generator=g).to(dev), torch.randn(nt * 128, generator=g).to(dev)
+    w, out = (torch.randn(nt * 128, K, generator=g) / K ** 0.5).to(dev), torch.randn(M, nt * 64, generator=g).to(dev)
+    ref = out.double().view(M, nt, 64)
+    y = (x.double() @ w.double().t() + b).view(M, nt, 2, 2, 32)             # a tile: [p 0..31 | g 0..31 | p 32..63 | g 32..63]
+    ref[..., :ncols] += (y[..., 0, :] * torch.sigmoid(y[..., 1, :])).reshape(M, nt, 64)[..., :ncols]
+    tiles = [_lib.make_tile(out.data_ptr() + 256 * i, bias=b.data_ptr() + 512 * i, glu=1, ncols=ncols, resid=out.data_ptr() + 256 * i,
+                            inner=M, s_i=nt * 64) for i in range(nt)]
+    _lib.fused_linear(x, w, tiles, M=M, K=K)
+    assert float((out.view(M, nt, 64) - ref).abs().max()) <= 2e-5 * float(ref.abs().max())
