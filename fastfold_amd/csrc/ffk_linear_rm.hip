@@ -164,8 +164,9 @@ template <bool GLU>
 __device__ __forceinline__ void rm_value_cols(const RmSlot& t, const f32x16& acc, const f32x16& accg, const float* sb, const float* sm,
                                               int l32, int half, u32x4 (&y)[2]) {
     const float b = sb[l32], g = GLU ? sb[32 + l32] : 0.0f;
-    // the mask multiply is skipped for row groups without a masked row (the common case)
-    const bool masked = sm && t.kind != FFK_TILE_V && __builtin_amdgcn_ballot_w64(sm[l32] != 1.0f) != 0;
+    // the mask multiply is skipped for row groups without a masked row (the common case); V tiles have no mask here: their rows
+    // lie in another order, and carrying both costs every variant five to ten more spilled scalar registers
+    const bool masked = sm && __builtin_amdgcn_ballot_w64(sm[l32] != 1.0f) != 0;
     auto emit = [&](auto value) __attribute__((always_inline)) {
         if (masked || t.scale != 1.0f) {
 #pragma unroll
@@ -767,7 +768,7 @@ bool rm_tile_ok(const ffk_linear_desc& d, const ffk_tile& t) {
         return true;
     }
     if (t.resid || t.gate || t.xtail) return false;
-    if (t.kind == FFK_TILE_V) return t.inner % 32 == 0 && t.ncols % 32 == 0 && t.s_o % 8 == 0 && t.s_h % 8 == 0;
+    if (t.kind == FFK_TILE_V) return !t.rowmask && t.inner % 32 == 0 && t.ncols % 32 == 0 && t.s_o % 8 == 0 && t.s_h % 8 == 0;
     if (t.kind != FFK_TILE_STRIDED) return false;
     return d.M % 16 == 0 && t.inner % 16 == 0 && t.s_i == 1 && t.s_o % 8 == 0 && t.s_h % 8 == 0 && t.s_d % 8 == 0 && lane32(t.s_d);
 }

@@ -761,3 +761,18 @@ def test_fp32_glu_tile_with_residual(dev, M, nt, ncols):
                             inner=M, s_i=nt * 64) for i in range(nt)]
     _lib.fused_linear(x, w, tiles, M=M, K=K)
     assert float((out.view(M, nt, 64) - ref).abs().max()) <= 2e-5 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("K", [64, 128, 256])
+def test_value_tile_with_row_mask(dev, dtype, K):
+    """A row mask on the v tiles of an attention: masked keys have zeros."""
+    from fastfold_amd import _lib
+    from fastfold_amd.model.fastnn.kernel import layouts
+    B2, N = 5, 96
+    g = torch.Generator().manual_seed(K)
+    x, w = torch.randn(B2, N, K, generator=g).to(dev, dtype), (torch.randn(128, K, generator=g) / K ** 0.5).to(dev, dtype)
+    mask, v = (torch.rand(B2, N, generator=g) > 0.3).to(dev, dtype), torch.zeros(B2, 4, 3, 2, 32, 4, 4, dtype=dtype, device=dev)
+    _lib.fused_linear(x, w, [_lib.make_tile(v, kind=_lib.FFK_TILE_V, inner=N, s_o=4 * 3072, s_h=3072, rowmask=mask, m_so=N, m_si=1)], M=B2 * N, K=K)
+    ref = (ops_np.linear(_np(x), _np(w)) * _np(mask)[..., None]).reshape(B2, N, 4, 32).transpose(0, 2, 1, 3)
+    assert _rel(_np(layouts.untile_v(v, N)), ref) < TOL[dtype]
