@@ -719,7 +719,7 @@ bool ws_tile_ok(const ffk_linear_desc& d, const ffk_tile& t) {
         return true;
     }
     if (t.resid || t.gate || t.xtail) return false;
-    if (t.kind == FFK_TILE_V) return t.inner % 32 == 0 && t.ncols % 32 == 0 && t.s_o % 8 == 0 && t.s_h % 8 == 0;
+    if (t.kind == FFK_TILE_V) return d.M % 32 == 0 && t.inner % 32 == 0 && t.ncols % 32 == 0 && t.s_o % 8 == 0 && t.s_h % 8 == 0;
     if (t.kind != FFK_TILE_STRIDED) return false;
     return d.M % 16 == 0 && t.inner % 16 == 0 && t.s_i == 1 && t.s_o % 8 == 0 && t.s_h % 8 == 0 && t.s_d % 8 == 0;
 }

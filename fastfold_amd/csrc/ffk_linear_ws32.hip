@@ -232,7 +232,7 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
             }
         }
         float* out = (float*)t.out + (long)sub * t.s_h;
-        if (t.kind == FFK_TILE_V && inner % 32 != 0) {   // the rows of a group may lie in two key tiles
+        if (t.kind == FFK_TILE_V && (inner % 32 != 0 || (M & 31))) {         // the rows of a group may lie in two key tiles, or end in one
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int mrow = m0g + 8 * (v >> 2) + 4 * half + (v & 3);

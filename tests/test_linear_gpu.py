@@ -776,3 +776,22 @@ def test_value_tile_with_row_mask(dev, dtype, K):
     _lib.fused_linear(x, w, [_lib.make_tile(v, kind=_lib.FFK_TILE_V, inner=N, s_o=4 * 3072, s_h=3072, rowmask=mask, m_so=N, m_si=1)], M=B2 * N, K=K)
     ref = (ops_np.linear(_np(x), _np(w)) * _np(mask)[..., None]).reshape(B2, N, 4, 32).transpose(0, 2, 1, 3)
     assert _rel(_np(layouts.untile_v(v, N)), ref) < TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("K,chan", [(128, False), (256, False), (128, True)])
+@pytest.mark.parametrize("M", [40, 96 * 131 - 24])
+def test_value_tile_of_a_launch_that_ends_inside_it(dev, dtype, K, chan, M):
+    """Rows of a key tile behind the last row of the launch keep what they hold."""
+    from fastfold_amd import _lib
+    from fastfold_amd.model.fastnn.kernel import layouts
+    N = 96
+    B = (M + N - 1) // N
+    g = torch.Generator().manual_seed(K + M)
+    x, w = torch.randn(B * N, K, generator=g).to(dev, dtype), (torch.randn(128, K, generator=g) / K ** 0.5).to(dev, dtype)
+    v = torch.full((B, 4, 3, 2, 32, 4, 4), 7.0, dtype=dtype, device=dev)
+    kw = dict(a_chanmajor=True, a_inner=B * N, a_si=1, a_cs=B * N) if chan else {}
+    _lib.fused_linear(x.t().contiguous() if chan else x, w, [_lib.make_tile(v, kind=_lib.FFK_TILE_V, inner=N, s_o=4 * 3072, s_h=3072)], M=M, K=K, **kw)
+    got = _np(layouts.untile_v(v, N)).transpose(0, 2, 1, 3).reshape(B * N, 128)
+    ref = ops_np.linear(_np(x), _np(w))
+    assert _rel(got[:M], ref[:M]) < TOL[dtype] and (got[M:] == 7.0).all()
