@@ -208,9 +208,11 @@ __global__ __launch_bounds__(GA_THREADS, 2) void global_attention_kernel(
                     const float sc = exp_for<T>(mx[h] - mnew);
                     const float p = exp_for<T>(lv - mnew);
                     mx[h] = mnew;
-                    sm[h] = sm[h] * sc + p;
+                    sm[h] = __builtin_fmaf(sm[h], sc, p);
+                    // written out: left to the compiler, the product it rounds changes with the shape of the loop.  While the
+                    // maximum stands sc is one and this form rounds once.
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) y[h][e] = y[h][e] * sc + p * x[e];
+                    for (int e = 0; e < 8; ++e) y[h][e] = __builtin_fmaf(p, x[e], y[h][e] * sc);
                 }
             }
         }
