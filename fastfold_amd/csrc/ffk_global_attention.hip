@@ -16,13 +16,14 @@
 //
 // One workgroup of 256 threads per column.  A row of C channels is held by C / 8 adjacent lanes
 // (8 channels each, one 16-byte load for bf16); the 256 / (C / 8) lane groups of the workgroup walk
-// the rows of the column with stride, four rows in flight per group, each group keeping its own
+// the rows of the column with stride, four rows (fp32: two) in flight per group, each group keeping its own
 // running softmax state, merged at the end (within a wave by shuffles, across waves through LDS).
-// A column has four waves, one per SIMD, to cover the latency of its rows: they are requested a step of four
-// ahead, as they lie in memory, and the four are worked on by one copy of the code (unrolled, its 64 dot products
-// in flight left no registers for the requests).  1 024 x 384 rows, C = 64, 8 heads, bf16: 88.8 us with the
-// requests in front of their use, 71.3 us; fp32 105, 91.7; 5 120 x 384 395, 310.  The state moved once for two
-// or four rows instead of one: 81 us (spills).
+// A column has four waves, one per SIMD, to cover the latency of its rows: they are requested a step of four (two)
+// ahead, as they lie in memory, and the rows of a step are worked on by one copy of the code (unrolled, its 64 dot
+// products in flight left no registers for the requests).  1 024 x 384 rows, C = 64, 8 heads, bf16: 88.8 us with the
+// requests in front of their use, 71 us; 5 120 x 384 395, 307.  fp32: 105, 89 (four rows ahead 91.7 with one to four
+// registers spilled, three 92.2 without); 64 x 384 21.8 with four rows, 19.3 with two; 5 120 x 384 431, 420.  The
+// state moved once for two or four rows instead of one: 81 us (spills).
 #include "ffk_common.h"
 
 #include <math.h>
@@ -31,17 +32,17 @@ namespace {
 
 constexpr int GA_THREADS = 256;
 constexpr int GA_HMAX = 8;       // query heads held in registers
-constexpr int GA_UNR = 4;        // rows requested together per lane group, a step ahead
 constexpr int GA_QMAX = 128;     // H * D
 
-// UNR rows of a lane group as they lie in memory: eight channels and the mask value each.
+// UNR rows of a lane group as they lie in memory, requested together a step ahead: eight channels and the mask value each.
+// Two rows of fp32 are as many registers as four of bf16; four, with the state's 144, spilled (see above).
 template <typename T> struct GaRows {
-    static constexpr int NV = 8 / DT<T>::VEC;
-    Vec16<T> v[GA_UNR][NV];
-    T mk[GA_UNR];
+    static constexpr int NV = 8 / DT<T>::VEC, UNR = 4 / NV;
+    Vec16<T> v[UNR][NV];
+    T mk[UNR];
     __device__ __forceinline__ void shift() {               // row 0 is the next one
 #pragma unroll
-        for (int u = 0; u + 1 < GA_UNR; ++u) {
+        for (int u = 0; u + 1 < UNR; ++u) {
 #pragma unroll
             for (int i = 0; i < NV; ++i) v[u][i] = v[u + 1][i];
             mk[u] = mk[u + 1];
@@ -103,10 +104,10 @@ __global__ __launch_bounds__(GA_THREADS, 2) void global_attention_kernel(
         for (int e = 0; e < 8; ++e) x[e] = x[e] * rstd * gm[e] + bt[e];
     };
     // rows s0 + u * G + g, u = 0..UNR-1: loads issued together, a step ahead of their use; rows past the end are clamped
-    constexpr int STEP = G * GA_UNR;
+    constexpr int UNR = GaRows<T>::UNR, STEP = G * UNR;
     auto request = [&](int s0, GaRows<T>& r) {
 #pragma unroll
-        for (int u = 0; u < GA_UNR; ++u) {
+        for (int u = 0; u < UNR; ++u) {
             const int s = s0 + u * G + g;
             const int sc = s < S ? s : S - 1;
 #pragma unroll
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(GA_THREADS, 2) void global_attention_kernel(
             GaRows<T> next;
             request(s0 + STEP, next);
 #pragma unroll
-            for (int u = 0; u < GA_UNR; ++u) {
+            for (int u = 0; u < UNR; ++u) {
                 float x[8];
                 rows.get(u, x);
                 layer_norm(x);
@@ -186,7 +187,7 @@ __global__ __launch_bounds__(GA_THREADS, 2) void global_attention_kernel(
         GaRows<T> next;
         request(s0 + STEP, next);
 #pragma unroll 1
-        for (int u = 0; u < GA_UNR; ++u) {
+        for (int u = 0; u < UNR; ++u) {
             float x[8], l[GA_HMAX];
             rows.get(0, x);
             const float mk = DT<T>::to_f(rows.mk[0]);
