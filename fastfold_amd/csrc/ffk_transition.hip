@@ -40,17 +40,18 @@ __device__ __forceinline__ uint32_t tr_touch(const T* w1, const T* w2, int lines
     return x;
 }
 
-template <int C, int NS> struct TrGeo {
-    static constexpr int H = 4 * C;
+constexpr int TR_C = 128, TR_H = 4 * TR_C;
+template <int NS> struct TrGeo {
+    static constexpr int C = TR_C, H = TR_H;
     static constexpr int HC = 32;                   // hidden channels per chunk
     static constexpr int NCHUNK = H / HC;
-    static constexpr int W1SLOT = HC * C * 2;       // HC rows of 2 C bytes (16 KB)
-    static constexpr int W2SLOT = C * HC * 2;       // C rows of 2 HC bytes (16 KB)
+    static constexpr int W1SLOT = HC * C * 2;       // HC rows of 2 C bytes (8 KB)
+    static constexpr int W2SLOT = C * HC * 2;       // C rows of 2 HC bytes (8 KB)
     static constexpr int XP = C * 2 + 16;           // pitch of the normalised rows (set-up only)
     static constexpr int NC1 = C / 8;               // 16-byte columns of a W1 row
     static constexpr int NC2 = HC / 8;              // 16-byte columns of a W2 row
     static constexpr int RP2 = 256 / (HC * 2);      // W2 rows per 256 bytes of LDS: the swizzle period
-    static constexpr int KS1 = C / 16, KS2 = HC / 16, HT = HC / 32, CT = C / 32;
+    static constexpr int KS1 = C / 16, KS2 = HC / 16, CT = C / 32;
     static constexpr size_t SMEM_RINGS = NS * (size_t)W1SLOT + NS * W2SLOT + H * sizeof(float);
     static constexpr size_t SMEM_ROWS = (size_t)TR_BM * XP;
     static constexpr int NLD = W1SLOT / 16 / TR_THREADS;   // 16-byte requests per thread and ring slot
@@ -67,19 +68,19 @@ __device__ __forceinline__ void tr_load_lds(const T* src, unsigned char* dst_wav
                                      (__attribute__((address_space(3))) void*)dst_wave, 16, 0, 0);
 }
 
-// NS: slots of the weight rings.  Two slots (one chunk in flight) when two workgroups share a CU and cover each
+// NS: slots of the weight rings.  Two slots (one chunk in flight) when three workgroups share a CU and cover each
 // other's waits; four when the launch has at most one workgroup per CU and the chunk stream has to hide the whole
 // memory latency by itself (a chunk is multiplied in less than half a microsecond).
-template <int TR_C, int NS>
-__global__ __launch_bounds__(TR_THREADS, NS == 4 ? 1 : (TR_C == 128 ? 3 : 2)) void transition_fused_kernel(T* __restrict__ out, const T* __restrict__ x, int8_t* __restrict__ xtail,
+template <int NS>
+__global__ __launch_bounds__(TR_THREADS, NS == 4 ? 1 : 3) void transition_fused_kernel(T* __restrict__ out, const T* __restrict__ x, int8_t* __restrict__ xtail,
                                                                         const T* __restrict__ gamma, const T* __restrict__ beta,
                                                                         const T* __restrict__ w1, const T* __restrict__ b1,
                                                                         const T* __restrict__ w2, const T* __restrict__ b2,
                                                                         long M, float eps) {
     typedef Mma<T> MM;
-    typedef TrGeo<TR_C, NS> G;
+    typedef TrGeo<NS> G;
     constexpr int NLD = G::NLD;
-    constexpr int TR_H = G::H, TR_HC = G::HC, TR_NCHUNK = G::NCHUNK, TR_W1SLOT = G::W1SLOT, TR_W2SLOT = G::W2SLOT, TR_XP = G::XP;
+    constexpr int TR_HC = G::HC, TR_NCHUNK = G::NCHUNK, TR_W1SLOT = G::W1SLOT, TR_W2SLOT = G::W2SLOT, TR_XP = G::XP;
     extern __shared__ __align__(16) unsigned char smem[];
     unsigned char* s_w1 = smem;                           // [NS][HC][2 C bytes]
     unsigned char* s_w2 = smem + NS * TR_W1SLOT;          // [NS][C][2 HC bytes]
@@ -96,36 +97,33 @@ __global__ __launch_bounds__(TR_THREADS, NS == 4 ? 1 : (TR_C == 128 ? 3 : 2)) vo
         constexpr int LPR = TR_C / 8, RPP = TR_THREADS / LPR, NPASS = TR_BM / RPP;   // lanes per row, rows per pass
         const int c8 = tid % LPR, r0 = tid / LPR;
         const Vec16<T> g = ld16(gamma + c8 * 8), b = ld16(beta + c8 * 8);
+        Vec16<T> v[NPASS];
 #pragma unroll
-        for (int i0 = 0; i0 < NPASS; i0 += 8) {
-            Vec16<T> v[8];
+        for (int i = 0; i < NPASS; ++i) {
+            long m = m0 + r0 + RPP * i;
+            m = m < M ? m : M - 1;                        // clamped: rows past the end are never stored
+            v[i] = ld16(x + m * TR_C + c8 * 8);
+        }
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                long m = m0 + r0 + RPP * (i0 + i);
-                m = m < M ? m : M - 1;                    // clamped: rows past the end are never stored
-                v[i] = ld16(x + m * TR_C + c8 * 8);
+        for (int i = 0; i < NPASS; ++i) {
+            float f[8], s = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                f[e] = (float)v[i].e[e];
+                s += f[e];
             }
+            const float mu = group_sum(s, LPR) * (1.0f / TR_C);
+            float q = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                float f[8], s = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    f[e] = (float)v[i].e[e];
-                    s += f[e];
-                }
-                const float mu = group_sum(s, LPR) * (1.0f / TR_C);
-                float q = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    f[e] -= mu;
-                    q += f[e] * f[e];
-                }
-                const float rs = rsqrtf(group_sum(q, LPR) * (1.0f / TR_C) + eps);
-                Vec16<T> y;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) y.e[e] = (T)(f[e] * rs * (float)g.e[e] + (float)b.e[e]);
-                *reinterpret_cast<Vec16<T>*>(s_x + (r0 + RPP * (i0 + i)) * TR_XP + c8 * 16) = y;
+            for (int e = 0; e < 8; ++e) {
+                f[e] -= mu;
+                q += f[e] * f[e];
             }
+            const float rs = rsqrtf(group_sum(q, LPR) * (1.0f / TR_C) + eps);
+            Vec16<T> y;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y.e[e] = (T)(f[e] * rs * (float)g.e[e] + (float)b.e[e]);
+            *reinterpret_cast<Vec16<T>*>(s_x + (r0 + RPP * i) * TR_XP + c8 * 16) = y;
         }
     }
     lds_barrier();
@@ -137,14 +135,14 @@ __global__ __launch_bounds__(TR_THREADS, NS == 4 ? 1 : (TR_C == 128 ? 3 : 2)) vo
     for (int i = tid; i < TR_H; i += TR_THREADS) s_b1[i] = (float)b1[i];
 
     // ---- chunk loaders (direct to LDS; lane L of a wave lands at dst + 16 L) ----
-    // W1 chunk: LDS row rho (0..63) holds weight row 32 * (rho / 32) + sigma(rho % 32) of the chunk; 16 columns
+    // W1 chunk: LDS row rho (0..31) holds weight row sigma(rho) of the chunk; 16 columns
     const T* w1src[NLD];
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         const int v = i * TR_THREADS + tid, rho = v / G::NC1, c = v % G::NC1;
-        w1src[i] = w1 + (long)((rho & ~31) + tr_sigma(rho & 31)) * TR_C + ((c ^ (rho & 15)) * 8);
+        w1src[i] = w1 + (long)tr_sigma(rho) * TR_C + ((c ^ (rho & 15)) * 8);
     }
-    // W2 chunk: LDS row rho (0..127) holds weight row 32 * (rho / 32) + tau(rho % 32); 8 columns
+    // W2 chunk: LDS row rho (0..127) holds weight row 32 * (rho / 32) + tau(rho % 32); 4 columns
     const T* w2src[NLD];
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
@@ -172,11 +170,9 @@ __global__ __launch_bounds__(TR_THREADS, NS == 4 ? 1 : (TR_C == 128 ? 3 : 2)) vo
         }
     }
 
-    // W1 fragment of hidden tile 0: row l32, column 2 ks + half.  The swizzle touches the low four column bits only,
-    // so K steps 8 .. 15 (C = 256) are the first eight plus 256 bytes.
-    int w1off[8];
+    int w1off[G::KS1];                                     // W1 fragment: row l32, column 2 ks + half
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) w1off[ks] = l32 * (TR_C * 2) + (((2 * ks + half) ^ (l32 & 15)) << 4);
+    for (int ks = 0; ks < G::KS1; ++ks) w1off[ks] = l32 * (TR_C * 2) + (((2 * ks + half) ^ (l32 & 15)) << 4);
     int w2off[G::KS2];                                     // W2 fragment of c-tile 0: row l32, column 2 ks + half
 #pragma unroll
     for (int ks = 0; ks < G::KS2; ++ks) w2off[ks] = l32 * (TR_HC * 2) + (((2 * ks + half) ^ ((l32 / G::RP2) & (G::NC2 - 1))) << 4);
@@ -190,44 +186,40 @@ __global__ __launch_bounds__(TR_THREADS, NS == 4 ? 1 : (TR_C == 128 ? 3 : 2)) vo
         fetch(q + NS - 1);
         const unsigned char* wa = s_w1 + (q % NS) * TR_W1SLOT;
         const unsigned char* wb = s_w2 + (q % NS) * TR_W2SLOT;
-        bf16x8 hf[G::HT][2];                               // [hidden tile][K step]: the chunk's N operand
+        f32x16 h;
+        // registers 0..7: hidden 8 half + 0..7 of the chunk, registers 8..15: 16 + 8 half + 0..7
+        const float* bp = s_b1 + q * TR_HC + 8 * half;
 #pragma unroll
-        for (int ht = 0; ht < G::HT; ++ht) {
-            f32x16 h;
-            // registers 0..7: hidden 8 half + 0..7 of the tile, registers 8..15: 16 + 8 half + 0..7
-            const float* bp = s_b1 + q * TR_HC + ht * 32 + 8 * half;
+        for (int a = 0; a < 4; ++a) {
+            const f32x4 b4 = *reinterpret_cast<const f32x4*>(bp + (a >> 1) * 16 + (a & 1) * 4);
 #pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const f32x4 b4 = *reinterpret_cast<const f32x4*>(bp + (a >> 1) * 16 + (a & 1) * 4);
+            for (int b = 0; b < 4; ++b) h[4 * a + b] = b4[b];
+        }
 #pragma unroll
-                for (int b = 0; b < 4; ++b) h[4 * a + b] = b4[b];
+        for (int ks = 0; ks < G::KS1; ++ks) MM::mma(h, *reinterpret_cast<const bf16x8*>(wa + w1off[ks]), xf[ks]);
+        // relu after the rounding, on the packed bf16 bit patterns: a negative bf16 is a negative 16-bit integer, so
+        // one packed integer max per pair replaces one clamp per value (rounding is monotonic: same bits)
+        bf16x8 hf[2];                                      // [K step]: the chunk's N operand
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            typedef float f32x2 __attribute__((ext_vector_type(2)));
+            typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+            typedef short s16x2 __attribute__((ext_vector_type(2)));
+            const s16x2 zero = {0, 0};
+            u32x4 w;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {                  // one packed conversion and one packed max per pair
+                const f32x2 pr = {h[8 * j + 2 * t], h[8 * j + 2 * t + 1]};
+                const bf16x2 r = __builtin_convertvector(pr, bf16x2);
+                w[t] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(s16x2, r), zero));
             }
-#pragma unroll
-            for (int ks = 0; ks < G::KS1; ++ks)
-                MM::mma(h, *reinterpret_cast<const bf16x8*>(wa + ht * 32 * (TR_C * 2) + w1off[ks & 7] + (ks >> 3) * 256), xf[ks]);
-            // relu after the rounding, on the packed bf16 bit patterns: a negative bf16 is a negative 16-bit integer, so
-            // one packed integer max per pair replaces one clamp per value (rounding is monotonic: same bits)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                typedef float f32x2 __attribute__((ext_vector_type(2)));
-                typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-                typedef short s16x2 __attribute__((ext_vector_type(2)));
-                const s16x2 zero = {0, 0};
-                u32x4 w;
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {              // one packed conversion and one packed max per pair
-                    const f32x2 pr = {h[8 * j + 2 * t], h[8 * j + 2 * t + 1]};
-                    const bf16x2 r = __builtin_convertvector(pr, bf16x2);
-                    w[t] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(s16x2, r), zero));
-                }
-                hf[ht][j] = __builtin_bit_cast(bf16x8, w);
-            }
+            hf[j] = __builtin_bit_cast(bf16x8, w);
         }
 #pragma unroll
         for (int ks = 0; ks < G::KS2; ++ks)
 #pragma unroll
             for (int c = 0; c < G::CT; ++c)
-                MM::mma(acc2[c], *reinterpret_cast<const bf16x8*>(wb + c * 32 * (TR_HC * 2) + w2off[ks]), hf[ks >> 1][ks & 1]);
+                MM::mma(acc2[c], *reinterpret_cast<const bf16x8*>(wb + c * 32 * (TR_HC * 2) + w2off[ks]), hf[ks]);
     }
 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // the re-fetches past the last chunk
@@ -636,17 +628,15 @@ extern "C" int ffk_transition_fused(void* out, const void* x, void* xtail, const
     if (M <= 128 * 256) return wide(C128(), Two());
     const unsigned grid = (unsigned)ffk_cdiv(M, TR_BM);
     const bool deep = grid <= 256 + 128;                     // at most ~one workgroup on most CUs: four-slot rings
-#define FFK_TR_LAUNCH(CC, NS)                                                                                           \
-    do {                                                                                                                \
-        static FfkLdsReservation lds_reserved;                                                                          \
-        const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)transition_fused_kernel<CC, NS>, TrGeo<CC, NS>::SMEM, \
-                                           "ffk_transition_fused");                                                     \
-        if (rc_lds != FFK_OK) return rc_lds;                                                                            \
-        transition_fused_kernel<CC, NS><<<grid, TR_THREADS, TrGeo<CC, NS>::SMEM, (hipStream_t)stream>>>(                \
-            (T*)out, (const T*)x, (int8_t*)xtail, (const T*)gamma, (const T*)beta, (const T*)w1, (const T*)b1, (const T*)w2, \
-            (const T*)b2, (long)M, eps);                                                                                \
-    } while (0)
-    if (deep) FFK_TR_LAUNCH(128, 4); else FFK_TR_LAUNCH(128, 2);
-#undef FFK_TR_LAUNCH
-    return ffk_check_launch("ffk_transition_fused");
+    auto fused = [&](auto slots) {
+        constexpr int NS = decltype(slots)::value;
+        static FfkLdsReservation lds_reserved;
+        const int rc = ffk_reserve_lds(lds_reserved, (const void*)transition_fused_kernel<NS>, TrGeo<NS>::SMEM, "ffk_transition_fused");
+        if (rc != FFK_OK) return rc;
+        transition_fused_kernel<NS><<<grid, TR_THREADS, TrGeo<NS>::SMEM, (hipStream_t)stream>>>(
+            (T*)out, (const T*)x, (int8_t*)xtail, (const T*)gamma, (const T*)beta, (const T*)w1, (const T*)b1, (const T*)w2, (const T*)b2,
+            (long)M, eps);
+        return ffk_check_launch("ffk_transition_fused");
+    };
+    return deep ? fused(std::integral_constant<int, 4>()) : fused(Two());
 }
