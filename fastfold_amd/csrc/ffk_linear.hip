@@ -359,9 +359,9 @@ __global__ __launch_bounds__(THREADS, 4) void fused_linear_kernel(const LinArgs 
             const T* resid = (const T*)t.resid;
             int8_t* xtail = nullptr;                           // extended residual stream (bf16, with resid)
             if constexpr (XS_OK) xtail = (int8_t*)t.xtail;
-            const int c_last = ncols >= VEC ? ((ncols - VEC) / VEC) * VEC : 0;   // last full vector column
+            const int c_last = ((ncols - VEC) / VEC) * VEC;   // last full vector column
 #pragma unroll 1
-            for (int i0 = 0; i0 < N_IT; i0 += 4) {
+            for (int i0 = ncols >= VEC ? 0 : N_IT; i0 < N_IT; i0 += 4) {       // (fewer channels than a vector: the tail below alone)
                 Vec16<T> x[4], gv[4], rv[4];
                 u32x2 tv[4];
                 long o[4];

@@ -324,9 +324,9 @@ __global__ __launch_bounds__(THREADS, 2) void fused_linear_slab_kernel(const Lin
             const T* gate = (const T*)t.gate;
             const T* resid = (const T*)t.resid;
             int8_t* xtail = (int8_t*)t.xtail;                  // extended residual stream (with resid)
-            const int c_last = ncols >= VEC ? ((ncols - VEC) / VEC) * VEC : 0;   // last full vector column
+            const int c_last = ((ncols - VEC) / VEC) * VEC;   // last full vector column
 #pragma unroll 1
-            for (int i0 = 0; i0 < N_IT; i0 += 4) {
+            for (int i0 = ncols >= VEC ? 0 : N_IT; i0 < N_IT; i0 += 4) {       // (fewer channels than a vector: the tail below alone)
                 Vec16<T> x[4], gv[4], rv[4];
                 u32x2 tv[4];
                 long o[4];

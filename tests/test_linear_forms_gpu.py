@@ -62,7 +62,7 @@ def _form(r, bf16, K, chan):
         if r.random() < 0.3:
             t["mask"] = r.choice([(N, 1), (1, B), (0, 1)]) if not f["tiles"] or not same_mask else f["tiles"][0]["mask"] or (N, 1)
         if kind == STRIDED:
-            t["ncols"] = r.choice([wide, wide, wide - 8, 36, 32])
+            t["ncols"] = r.choice([wide, wide, wide - 8, 36, 32, 3])
             p, h = r.choice([(128, 32), (160, 32), (32, 32 * B * N)])
             t.update(r.choice([dict(inner=M, s_o=0, s_i=p, mask=t["mask"] and (0, 1)), dict(s_o=N * p, s_i=p), dict(s_o=p, s_i=B * p)]), s_h=h)
             if r.random() < 0.5:
