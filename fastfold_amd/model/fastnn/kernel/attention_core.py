@@ -183,7 +183,9 @@ class FusedAttenionCoreFunc(torch.autograd.Function):
         grads = any(t is not None and t.requires_grad for t in (q, k, v, bias))
         b1, b2, h, n, d = q.shape
         ctx.wide = d > 32
-        if q.numel() == 0:
+        ctx.empty = q.numel() == 0
+        if ctx.empty:
+            ctx.save_for_backward(q, k, v, bias)
             return torch.empty(b1, b2, n, h * d, dtype=q.dtype, device=q.device)
         if ctx.wide:
             out = _attention_core_wide(q, k, v, mask, bias)
@@ -198,6 +200,9 @@ class FusedAttenionCoreFunc(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout):
+        if ctx.empty:
+            dq, dk, dv, dbias = (None if t is None else torch.zeros_like(t) for t in ctx.saved_tensors)
+            return dq, dk, dv, None, dbias
         back = _attention_core_backward_wide if ctx.wide else _attention_core_backward
         saved = ctx.saved_tensors
         dq, dk, dv, dbias = back(*saved[:-1], saved[-1].contiguous(), dout.contiguous(), ctx.needs_input_grad[4])

@@ -71,9 +71,10 @@ class FusedLayerNormAffineFunction(torch.autograd.Function):
             return dx, dgb[0].view(shape), dgb[1].view(shape), None, None
         dgamma = torch.zeros(cols, dtype=torch.float32, device=input_.device)
         dbeta = torch.zeros(cols, dtype=torch.float32, device=input_.device)
-        _lib.call("ffk_layernorm_bwd", _lib.ptr(dx), _lib.ptr(dgamma), _lib.ptr(dbeta), _lib.ptr(g),
-                  _lib.ptr(input_), _lib.ptr(mean), _lib.ptr(rstd), _lib.ptr(weight_), rows, cols,
-                  _lib.dtype_tag(input_.dtype), _lib.stream_ptr())
+        if rows > 0:
+            _lib.call("ffk_layernorm_bwd", _lib.ptr(dx), _lib.ptr(dgamma), _lib.ptr(dbeta), _lib.ptr(g),
+                      _lib.ptr(input_), _lib.ptr(mean), _lib.ptr(rstd), _lib.ptr(weight_), rows, cols,
+                      _lib.dtype_tag(input_.dtype), _lib.stream_ptr())
         return dx, dgamma.to(weight_.dtype).view(shape), dbeta.to(weight_.dtype).view(shape), None, None
 
 

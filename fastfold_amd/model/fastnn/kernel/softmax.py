@@ -62,11 +62,12 @@ class FusedSoftmaxFunc(torch.autograd.Function):
         _lib.check_device(grad_output, output)
         grad_input = torch.empty_like(output)
         grad_bias = None
-        if not (ctx.use_bias and ctx.needs_input_grad[2]) or output.numel() == 0:
-            _lib.call("ffk_softmax_bwd", _lib.ptr(grad_input), _lib.ptr(grad_output), _lib.ptr(output),
-                      ctx.rows, ctx.cols, _lib.dtype_tag(output.dtype), _lib.stream_ptr())
+        if output.numel() == 0:
             if ctx.use_bias and ctx.needs_input_grad[2]:
                 grad_bias = torch.sum(grad_input, dim=1, keepdim=True)
+        elif not (ctx.use_bias and ctx.needs_input_grad[2]):
+            _lib.call("ffk_softmax_bwd", _lib.ptr(grad_input), _lib.ptr(grad_output), _lib.ptr(output),
+                      ctx.rows, ctx.cols, _lib.dtype_tag(output.dtype), _lib.stream_ptr())
         else:
             B1, B2, H, Nq, Nk = output.shape
             rows = B1 * H * Nq

@@ -276,3 +276,20 @@ def test_tied_parameters(dev):
             torch.autograd.backward(out, [torch.ones_like(t) for t in out])
             grads.append((x.grad, b.communication.linear_a.weight.grad, b.communication.linear_b.weight.grad))
         assert _rel(grads[1][0], grads[0][0]) < 3e-3 and _rel(grads[1][1], grads[0][1] + grads[0][2]) < 3e-3
+
+
+@pytest.mark.parametrize("b2,n", [(0, 5), (3, 0)])
+def test_operators_of_empty_tensors(dev, b2, n):
+    """No rows or no keys: gradients of the operands' shapes, zero where a parameter or a bias has elements."""
+    from fastfold_amd.model.fastnn.kernel import LayerNorm, fused_attention_core, fused_softmax
+
+    def leaf(*s):
+        return torch.randn(*s, device=dev, requires_grad=True)
+    norm, mask = LayerNorm(64).to(dev), torch.ones(1, b2, n, device=dev)
+    q, k, v = (leaf(1, b2, 4, n, 32) for _ in range(3))
+    pair, logits, bias, x = leaf(1, 4, n, n), leaf(1, b2, 4, n, n), leaf(1, 1, 4, n, n), leaf(b2, n, 64)
+    outs = [fused_attention_core(q, k, v, mask, pair), fused_softmax(logits, mask, bias), norm(x)]
+    assert [tuple(o.shape) for o in outs] == [(1, b2, n, 128), (1, b2, 4, n, n), (b2, n, 64)]
+    leaves = (q, k, v, pair, logits, bias, x, norm.weight, norm.bias)
+    for t, g in zip(leaves, torch.autograd.grad(outs, leaves, [torch.ones_like(o) for o in outs])):
+        assert g.shape == t.shape and not g.any()
