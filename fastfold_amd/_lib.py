@@ -78,10 +78,16 @@ def dtype_tag(dtype: torch.dtype) -> int:
         raise RuntimeError("fastfold_amd: unsupported dtype %s" % dtype)
 
 
+# Not a name torch promises to keep (seen with 2.10.0+rocm7.0); without it the public property serves.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_ptr() -> int:
     """The current stream of the current device, as ``torch.cuda.current_stream().cuda_stream`` without the two objects in between
     (every launch asks for it)."""
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def ptr(t):

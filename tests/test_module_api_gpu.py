@@ -276,6 +276,17 @@ def test_side_stream_matches_default_stream(dev):
     assert torch.equal(gm, rm) and torch.equal(gz, rz)
 
 
+def test_stream_of_a_launch(dev, monkeypatch):
+    """The handle a launch gets is the current stream's, with torch's own accessor and without it."""
+    from fastfold_amd import _lib
+    side = torch.cuda.Stream()
+    for accessor in (_lib._raw_stream, None):
+        monkeypatch.setattr(_lib, "_raw_stream", accessor)
+        assert _lib.stream_ptr() == torch.cuda.current_stream().cuda_stream
+        with torch.cuda.stream(side):
+            assert _lib.stream_ptr() == side.cuda_stream
+
+
 def test_block_forward_replays_from_a_captured_graph(dev):
     """One block forward captured in a HIP graph and replayed with new input contents, with eager work and
     synchronisations between the replays: every replay equals the eager result on the same inputs."""
