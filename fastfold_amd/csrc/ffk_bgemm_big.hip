@@ -29,8 +29,6 @@ constexpr int BG_THREADS = 512;
 constexpr int BG_BK = 32;                    // K elements per chunk: 64-byte rows, four 16-byte columns
 constexpr int BG_SLOTS = 4;                  // LDS ring depth: three chunks in flight behind the one in use
 
-__device__ __forceinline__ int bg_tau(int i) { return ((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3); }
-
 // One 16-byte column of a chunk row goes from global memory straight into LDS (no registers): the
 // hardware places lane L of the wave at  dst + 16 * L,  dst being wave-uniform.
 __device__ __forceinline__ void bg_load_lds(const T* src, unsigned char* dst_wave) {
@@ -135,7 +133,7 @@ __global__ __launch_bounds__(BG_THREADS, 2) void bgemm_big_kernel(const ffk_bgem
         }
     };
     // fragment addresses: A rows in natural order, B rows through tau; column (2 ks + half) un-swizzled
-    const int ra = wm * 64 + l32, rb = BM + wn * WTN + bg_tau(l32);
+    const int ra = wm * 64 + l32, rb = BM + wn * WTN + ffk_tau(l32);
     int fa_off[2], fb_off[2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {

@@ -329,6 +329,11 @@ template <> struct Mma<float> {
 // Row of the 32x32 accumulator tile held in register v by lane `lane`.
 __device__ __forceinline__ int acc_row(int v, int lane) { return 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3); }
 
+// Index permutation tau(8a + 4h + b) = 16h + 4a + b.  An accumulator register v = 4a + b of half-wave h holds row 8a + 4h + b of
+// the M operand (acc_row); loading M-operand row i from source row tau(i) therefore leaves source rows 16h .. 16h + 15 in
+// registers 0 .. 15: sixteen consecutive channels (or rows) per lane, whole vectors to store.
+__device__ __forceinline__ int ffk_tau(int i) { return ((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3); }
+
 static inline int ffk_cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 
 // ------------------------------------------------- attention operand tiles ----

@@ -41,7 +41,6 @@ template <int C> struct GoGeo {
     static constexpr size_t SMEM = SMEM_RINGS > SMEM_ROWS ? SMEM_RINGS : SMEM_ROWS;
 };
 
-__device__ __forceinline__ int go_tau(int i) { return ((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3); }
 // i = 8a + 4h + b  ->  16 (a / 2) + 8h + 4 (a % 2) + b
 __device__ __forceinline__ int go_sigma(int i) { return (i >> 4) * 16 + ((i >> 2) & 1) * 8 + ((i >> 3) & 1) * 4 + (i & 3); }
 
@@ -144,7 +143,7 @@ __global__ __launch_bounds__(GO_THREADS, GO_C == 128 ? 3 : 2) void gated_out_ker
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         const int v = i * GO_THREADS + tid, rho = v / G::NC2, c = v % G::NC2;
-        w2src[i] = w2 + (long)((rho & ~31) + go_tau(rho & 31)) * GO_H + ((c ^ ((rho / G::RP2) & (G::NC2 - 1))) * 8);
+        w2src[i] = w2 + (long)((rho & ~31) + ffk_tau(rho & 31)) * GO_H + ((c ^ ((rho / G::RP2) & (G::NC2 - 1))) * 8);
     }
     auto fetch = [&](int q) {                              // past the last chunk it is fetched again (into a free slot)
         const int qc = q < GO_NCHUNK ? q : GO_NCHUNK - 1;

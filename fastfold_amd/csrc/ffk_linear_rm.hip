@@ -103,11 +103,6 @@ __device__ __forceinline__ float rm_sigmoid_pre(float acc, float bs) {
     return fast_rcp(1.0f + fast_exp2(__builtin_fmaf(acc, -1.4426950408889634f, bs)));
 }
 
-// Index permutation tau(8a + 4h + b) = 16h + 4a + b.  An MFMA accumulator register v = 4a + b of half-wave h holds row
-// 8a + 4h + b of the M operand; loading M-operand row i from source row tau(i) therefore leaves source rows 16h .. 16h + 15 in
-// registers 0 .. 15: sixteen consecutive channels (or rows) per lane, i.e. 32 contiguous bytes to store.
-__host__ __device__ __forceinline__ int rm_tau(int i) { return ((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3); }
-
 __host__ __device__ __forceinline__ bool rm_by_rows(const ffk_tile& t) {
     return t.kind == FFK_TILE_QK || t.kind == FFK_TILE_ACC || (t.kind == FFK_TILE_STRIDED && t.s_d == 1);
 }
@@ -218,7 +213,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void linear_rm_kernel(const RmArgs
     const int slot0 = ((int)blockIdx.y * WAVES + wave) * NS;
 #pragma unroll
     for (int s = 0; s < NS; ++s) sp[s] = args.slot[slot0 + s];
-    const int n32 = d.row_perm ? rm_tau(l32) : l32;
+    const int n32 = d.row_perm ? ffk_tau(l32) : l32;
 
     // ---- slab streaming: thread -> (row tid / LPR + RPP * i, 8 channels starting at 8 * (tid % LPR)) ----
     const int c8 = tid % LPR, r0 = tid / LPR;
@@ -291,7 +286,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void linear_rm_kernel(const RmArgs
                     *reinterpret_cast<bf16x8*>(stage + row * (PW * 2) + ((lcol ^ (row & (LR - 1))) * 16)) = wf[sl][pc * NI + i];
                 }
                 // [row][channel] tiles take their weight rows through tau (16 consecutive channels per lane)
-                const int wl = (sp[sl].flags & RM_TAU) ? rm_tau(l32) : l32;
+                const int wl = (sp[sl].flags & RM_TAU) ? ffk_tau(l32) : l32;
 #pragma unroll
                 for (int k = 0; k < NI; ++k)
                     wf[sl][pc * NI + k] = *reinterpret_cast<const bf16x8*>(stage + wl * (PW * 2) + (((2 * k + half) ^ (wl & (LR - 1))) * 16));

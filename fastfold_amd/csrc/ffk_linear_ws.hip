@@ -54,7 +54,7 @@ struct WsSlot {
     signed char glu;         // 0 plain, 1 value half of a GLU unit (gate half in the next slot), 2 gate half
     bool has_bias, by_rows;
     signed char rg_first, rg_mask;   // row groups of a slab this wave takes for the slot: those with rg & rg_mask == rg_first
-    bool tau;                // weight rows through ws_tau
+    bool tau;                // weight rows through ffk_tau
     bool sig;                // bias pre-multiplied for ws_sigmoid_pre
 };
 
@@ -89,12 +89,6 @@ __device__ __forceinline__ void unpack4(const T* p, float (&f)[4]) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) f[e] = (float)h[e];
 }
-
-// Index permutation tau(8a + 4h + b) = 16h + 4a + b.  An MFMA accumulator register v = 4a + b of
-// half-wave h holds row 8a + 4h + b of the M operand; loading M-operand row i from source row tau(i)
-// therefore leaves source rows 16h .. 16h + 15 in registers 0 .. 15: sixteen consecutive channels
-// (or rows) per lane, i.e. 32 contiguous bytes to store.
-__device__ __forceinline__ int ws_tau(int i) { return ((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3); }
 
 __device__ __forceinline__ void unpack8(const T* p, float* f) {
     u32x4 raw = *reinterpret_cast<const u32x4*>(p);
@@ -393,7 +387,7 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
 #pragma unroll
     for (int s = 0; s < NS; ++s) sp[s] = args.slot[wave * NS + s];
     // launches with channel-major tiles read the rows of a group through tau (16 consecutive rows per lane)
-    const int n32 = args.row_perm ? ws_tau(l32) : l32;
+    const int n32 = args.row_perm ? ffk_tau(l32) : l32;
 
     // ---- slab streaming ----
     // DUAL launches carry both LayerNorms folded into the weights: ln_gamma is the fp32 table of row sums and
@@ -544,7 +538,7 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
                     *reinterpret_cast<bf16x8*>(stage + row * (PW * 2) + ((lcol ^ (row & (LR - 1))) * 16)) = wf[sl][pc * NI + i];
                 }
                 // [row][channel] tiles take their weight rows through tau (16 consecutive channels per lane)
-                const int wl = sp[sl].tau ? ws_tau(l32) : l32;
+                const int wl = sp[sl].tau ? ffk_tau(l32) : l32;
 #pragma unroll
                 for (int k = 0; k < NI; ++k)
                     wf[sl][pc * NI + k] = *reinterpret_cast<const bf16x8*>(

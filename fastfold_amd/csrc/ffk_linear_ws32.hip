@@ -45,8 +45,6 @@ struct W3Args {
     int mask_tile;                                       // tile whose row mask the launch uses, -1: none
 };
 
-__device__ __forceinline__ int w3_tau(int i) { return ((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3); }
-
 __host__ __device__ __forceinline__ bool w3_by_rows(const ffk_tile& t) {
     return t.kind == FFK_TILE_QK || t.kind == FFK_TILE_ACC || t.kind == FFK_TILE_BIAS || (t.kind == FFK_TILE_STRIDED && t.s_d == 1);
 }
@@ -140,7 +138,7 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         const ffk_tile& t = d.tiles[units[s] >= 0 ? units[s] >> 2 : 0];
-        const int wl = w3_by_rows(t) && t.kind != FFK_TILE_ACC ? w3_tau(l32) : l32;
+        const int wl = w3_by_rows(t) && t.kind != FFK_TILE_ACC ? ffk_tau(l32) : l32;
         unsigned char* stage = s_a + wave * 4096;
 #pragma unroll
         for (int p = 0; p < KF; p += 4) {
@@ -154,7 +152,7 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
         if (half == 0) s_bias[(wave * NS + s) * 32 + l32] = tb[s];
     }
     lds_barrier();                                       // every wave is done with the staging area
-    const int n32 = args.row_perm ? w3_tau(l32) : l32;
+    const int n32 = args.row_perm ? ffk_tau(l32) : l32;
 
     // ---- slab streaming ----
     if (!ONE && ln) {

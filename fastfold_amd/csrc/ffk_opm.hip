@@ -33,8 +33,6 @@ constexpr int OP_K2C = OP_EC * 32;               // k2 elements per chunk (64)
 constexpr int OP_PA = OP_K2C * 2 + 16;           // A2 row pitch in bytes (padded: written by ds_write)
 constexpr int OP_W2SLOT = 128 * OP_K2C * 2;      // W2 chunk: 128 rows of 128 bytes (16 KB)
 
-__device__ __forceinline__ int op_tau(int i) { return ((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3); }
-
 template <int KS1, int OP_TI, int WAVES>   // KS1: MFMA K steps of the outer product, spad / 16 (4 or 8)
 __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void opm_fused_kernel(T* __restrict__ out, const T* __restrict__ resid, int8_t* __restrict__ xtail,
                                                                  const T* __restrict__ at, const T* __restrict__ bt,
@@ -64,7 +62,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void opm_fused_kernel(T* __r
     // ---- a fragments of this wave's i (rows d through tau: registers of the result hold d = 16 half + v) ----
     bf16x8 af[KS1];
     {
-        const T* ap = at + ((long)(i0 + iw) * 32 + op_tau(l32)) * SPAD + half * 8;
+        const T* ap = at + ((long)(i0 + iw) * 32 + ffk_tau(l32)) * SPAD + half * 8;
 #pragma unroll
         for (int ks = 0; ks < KS1; ++ks) af[ks] = MM::ld(ap + ks * 16);
     }
@@ -83,7 +81,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void opm_fused_kernel(T* __r
 #pragma unroll
     for (int i = 0; i < WLD; ++i) {
         const int v = i * OP_THREADS + tid, rho = v >> 3, c = v & 7;
-        wsrc[i] = w2p + (long)((rho & ~31) + op_tau(rho & 31)) * 1024 + ((c ^ ((rho >> 1) & 7)) * 8);
+        wsrc[i] = w2p + (long)((rho & ~31) + ffk_tau(rho & 31)) * 1024 + ((c ^ ((rho >> 1) & 7)) * 8);
     }
     const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
     // asm: with loads to LDS that it knows of the compiler waits for every LDS read of the wave in front of each group of products

@@ -59,7 +59,6 @@ template <int NS> struct TrGeo {
     static constexpr size_t SMEM = SMEM_RINGS > SMEM_ROWS ? SMEM_RINGS : SMEM_ROWS;
 };
 
-__device__ __forceinline__ int tr_tau(int i) { return ((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3); }
 // i = 8a + 4h + b  ->  16 (a / 2) + 8h + 4 (a % 2) + b
 __device__ __forceinline__ int tr_sigma(int i) { return (i >> 4) * 16 + ((i >> 2) & 1) * 8 + ((i >> 3) & 1) * 4 + (i & 3); }
 
@@ -147,7 +146,7 @@ __global__ __launch_bounds__(TR_THREADS, NS == 4 ? 1 : 3) void transition_fused_
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         const int v = i * TR_THREADS + tid, rho = v / G::NC2, c = v % G::NC2;
-        w2src[i] = w2 + (long)((rho & ~31) + tr_tau(rho & 31)) * TR_H + ((c ^ ((rho / G::RP2) & (G::NC2 - 1))) * 8);
+        w2src[i] = w2 + (long)((rho & ~31) + ffk_tau(rho & 31)) * TR_H + ((c ^ ((rho / G::RP2) & (G::NC2 - 1))) * 8);
     }
     auto fetch = [&](int q) {                              // past the last chunk it is fetched again (into a free slot)
         const int qc = q < TR_NCHUNK ? q : TR_NCHUNK - 1;
@@ -323,7 +322,7 @@ __global__ __launch_bounds__(256 * RP, tw_occ(C, RP)) void transition_wide_kerne
         const int r = tid / NC1 + i * RPR;
         w1src[i] = w1 + (long)tr_sigma(r) * TW_C + (((tid % NC1) ^ (r & 15)) * 8);
     }
-    const T* w2src = w2 + (long)((tid / 8 & ~31) + tr_tau(tid / 8 & 31)) * TW_H + (((tid % 8) ^ ((tid / 16) & 7)) * 8);
+    const T* w2src = w2 + (long)((tid / 8 & ~31) + ffk_tau(tid / 8 & 31)) * TW_H + (((tid % 8) ^ ((tid / 16) & 7)) * 8);
     const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem;
     // asm: the compiler would order every later LDS read behind these loads
     auto dma = [&](const T* src, unsigned dst) __attribute__((always_inline)) {
