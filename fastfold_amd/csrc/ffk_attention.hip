@@ -362,12 +362,21 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
         // Only when some lane's sum exceeds that (or on the first tile, which sets the reference) is
         // the tile recomputed from its LDS slot, the reference moved to the row maximum and O / l rescaled.
         score_tile();
-        bool move_ref = first;
+        bool move_ref = first, fresh = first;
         if (!first) {
             prob_tile();
             if (CAREFUL) {
                 move_ref = __builtin_amdgcn_ballot_w64(!(tsum <= REF_LIMIT)) != 0;
-                if (move_ref) score_tile();
+                if (move_ref) {
+                    // A row that has met no key so far stands at the floor, beside which a score keeps three decimals: its
+                    // scores are taken again without a reference.
+                    fresh = negm[0] == -REF_FLOOR;
+                    if (fresh) {
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) negm[v] = 0.0f;
+                    }
+                    score_tile();
+                }
             }
         }
         if (move_ref) {
@@ -375,8 +384,8 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
 #pragma unroll
             for (int v = 2; v < 16; ++v) mt = fmaxf(mt, s[v]);
             const float mfull = fmaxf(mt, lane_xor<32>(mt));
-            const float delta = first ? fmaxf(mfull, REF_FLOOR) : fmaxf(mfull, 0.0f);
-            const float alpha = first ? 1.0f : fast_exp2(-delta);   // nothing accumulated before the first tile
+            const float delta = fmaxf(mfull, fresh ? REF_FLOOR : 0.0f);
+            const float alpha = first ? 1.0f : fast_exp2((fresh ? REF_FLOOR : 0.0f) - delta);   // nothing accumulated before the first tile
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 s[v] -= delta;

@@ -515,3 +515,27 @@ def test_attention_pack_matches_the_torch_layout_helpers(dev, dtype, b2, h, n, d
     assert torch.equal(bt.view(-1), layouts.tile_bias((bias.float() * 1.5).to(dtype)).reshape(-1))
     ref = (x.double() * y.double()).sum(-1)
     assert float((dsum[..., :n] - ref).abs().max()) < 1e-4 and float(dsum[..., n:].abs().sum()) == 0.0
+
+
+@pytest.mark.parametrize("by", ["mask", "bias"])
+@pytest.mark.parametrize("n,lead", [(100, 40), (160, 96), (257, 33)])
+def test_fp32_attention_behind_masked_leading_keys(dev, n, lead, by):
+    """The first key tiles hold no key, by the mask or by a bias of -1e9: the scores behind them keep their precision (fp32 sums and
+    exp2, 1e-5 of the norm; forward and gradients), in rows beside others that have all their keys."""
+    from fastfold_amd.model.fastnn.kernel import fused_attention_core
+    g = torch.Generator().manual_seed(n)
+    q, k, v, do = (torch.randn(1, 3, 4, n, 32, generator=g).to(dev).requires_grad_(True) for _ in range(4))
+    do = do.detach().transpose(2, 3).reshape(1, 3, n, 128).contiguous()
+    mask, bias = torch.ones(1, 3, n, device=dev), torch.randn(1, 4, n, n, generator=g).to(dev)
+    if by == "mask":
+        mask[:, 1, :lead] = 0
+    else:
+        bias[:, :, ::2, :lead] = -1e9
+    got = fused_attention_core(q, k, v, mask, bias.requires_grad_(True))
+    grads = torch.autograd.grad(got, (q, k, v, bias), do)
+    dq, dk, dv, db = (t.detach().double().requires_grad_(True) for t in (q, k, v, bias))
+    s = torch.matmul(dq * 32 ** -0.5, dk.transpose(-1, -2).contiguous()) + db[:, None]
+    s = torch.where(mask[:, :, None, None] == 0, -1e9, s)
+    ref = torch.matmul(s.softmax(-1), dv).transpose(2, 3).reshape(1, 3, n, 128)
+    for a, e in zip((got, *grads), (ref, *torch.autograd.grad(ref, (dq, dk, dv, db), do.double()))):
+        assert float((a - e).norm() / e.norm()) <= 1e-5
