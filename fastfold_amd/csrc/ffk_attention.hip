@@ -18,7 +18,6 @@
 
 namespace {
 
-constexpr int THREADS = 256;
 constexpr float NEG_BIG = -3.0e38f;
 
 template <typename T> struct Ops16 {   // the 16 elements one lane owns of a 1024-element tile
@@ -239,8 +238,7 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
     // directly.  m_ref is only moved (and O / l rescaled) when the probabilities of a tile show that
     // a score lies more than REF_SLACK above it, which bounds  p = exp2(s - m_ref) <= 2^REF_SLACK
     // in everything that is accumulated;  the first tile always sets it.
-    constexpr float REF_SLACK = 20.0f;
-    constexpr float REF_LIMIT = 1048576.0f;       // 2^REF_SLACK
+    constexpr float REF_LIMIT = 1048576.0f;       // 2^REF_SLACK, REF_SLACK = 20
     constexpr float REF_FLOOR = -1.0e4f;          // keeps m_ref small when the first tile is fully masked
     f32x16 o_acc, negm;
 #pragma unroll

@@ -516,7 +516,6 @@ __global__ __launch_bounds__(256, DP == 1 && sizeof(T) == 2 ? (NT == 1 ? 3 : 2) 
     const float* __restrict__ lse, const float* __restrict__ dsum, int B2, int H, int Nq, int Nk, int NS,
     long part_q, long part_k, int bias_pad, int partial) {
     typedef Mma<T> MM;
-    typedef typename MM::Frag Frag;
     constexpr int NF = 16 / MM::KLANE;
     constexpr bool PIN = DP == 1 && (sizeof(T) == 4 || NT == 1);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;

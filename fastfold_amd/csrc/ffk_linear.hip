@@ -567,11 +567,12 @@ extern "C" int ffk_fused_linear(const ffk_linear_desc* d, void* stream) {
                     FFK_ERR_UNSUPPORTED, "ffk_fused_linear: tile %d: a residual tail needs bf16, resid and a [row][channel] tile", i);
         FFK_REQUIRE(ffk_aligned16(t.xtail), FFK_ERR_ALIGN, "ffk_fused_linear: tile %d: residual tail alignment", i);
     }
-    // Two kernel variants.  Launches whose tiles are all stored channel-contiguous (plain, gated,
-    // residual and q/k tiles) use the slab-persistent kernel (128-row slabs, register prefetch of the
+    // The kernels with weights in registers are asked first.  What they refuse goes to one of two LDS-staged
+    // kernels: bf16 launches of row-major operands whose tiles are all stored channel-contiguous (plain, gated,
+    // residual and q/k tiles) to the slab-persistent one (128-row slabs, register prefetch of the
     // next slab and of whole weight tiles); launches with row-contiguous tiles (v / bias tiles,
-    // channel-major stores) use the 64-row kernel below, whose smaller LDS footprint keeps four
-    // workgroups per CU in flight and hides the longer store phase of those tiles.
+    // channel-major stores), channel-major operands and fp32 to the 64-row kernel below, whose smaller LDS footprint
+    // keeps four workgroups per CU in flight and hides the longer store phase of those tiles.
     bool all_c = d->dtype == FFK_BF16 && !d->a_chanmajor;
     for (int i = 0; i < d->n_tiles; ++i) {
         const ffk_tile& t = d->tiles[i];

@@ -1,7 +1,7 @@
 // Weights-in-registers variant of the fused linear layer for row-major operands (see ffk_fused_linear in include/ffk.h),
 // bf16, K = 64, 128 or 256: the projections of the MSA, pair, extra-MSA and template stacks and of their backward passes.
 //
-// A workgroup keeps the MFMA fragments of its weight units (32 output rows each, up to four per wave) in registers; rows of A
+// A workgroup keeps the MFMA fragments of its weight units (32 output rows each, one or two per wave) in registers; rows of A
 // stream through a double-buffered slab in LDS: global -> registers -> (LayerNorm in registers) -> LDS, the loads of slab i + 1
 // in flight while slab i is multiplied.  Each wave multiplies 32-row groups of the slab against its own units and finishes the
 // 32 x 32 blocks straight from the accumulators - bias, activation, GLU, row mask, gate, residual - and stores them:
@@ -11,8 +11,8 @@
 // What bounds it: a 32 x 32 block costs K / 16 matrix instructions of 32 cycles, and a vector instruction costs a SIMD 4 cycles
 // that no matrix instruction of it overlaps with.  So the loop is arranged for few vector instructions per block: the position
 // of a group in its output is scalar arithmetic (a multiplication by a reciprocal) and a store takes a scalar base and a 32-bit
-// lane offset fixed for the launch; what a unit's epilogue needs fits 48 bytes, so two or three units of a wave stay in scalar
-// registers; two units of a wave share the fragments of a row group, which are requested one step ahead.
+// lane offset fixed for the launch; what a unit's epilogue needs fits 48 bytes, so that of both units of a wave stays in scalar
+// registers; two units of a wave share the fragments of a row group (K <= 128), which are requested one step ahead.
 #include "ffk_common.h"
 #include <type_traits>
 

@@ -83,25 +83,11 @@ __host__ __device__ __forceinline__ bool ws_by_rows(const ffk_tile& t) {
     return t.kind == FFK_TILE_QK || t.kind == FFK_TILE_ACC || (t.kind == FFK_TILE_STRIDED && t.s_d == 1);
 }
 
-__device__ __forceinline__ void unpack4(const T* p, float (&f)[4]) {
-    u32x2 raw = *reinterpret_cast<const u32x2*>(p);
-    const T* h = reinterpret_cast<const T*>(&raw);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) f[e] = (float)h[e];
-}
-
-__device__ __forceinline__ void unpack8(const T* p, float* f) {
-    u32x4 raw = *reinterpret_cast<const u32x4*>(p);
-    const T* h = reinterpret_cast<const T*>(&raw);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = (float)h[e];
-}
-
 // ---- lane = row (n32 = its row within the group), registers = channels -----------------------
 // STRIDED tiles: weight rows were loaded through tau, registers hold channels 16*half + v.
 // ACC / QK tiles: natural weight order, registers hold channels 8a + 4*half + b.
 // sb: this slot's 32 (GLU: 64) bias values in LDS (fp32).
-template <bool GLU, bool XT, bool POS>
+template <bool GLU>
 __device__ __forceinline__ void ws_store_rows(const WsSlot& t, const f32x16& acc, const f32x16& accg, const float* sb,
                                               bool valid, unsigned mc, unsigned hi, unsigned lo, int half) {
     const bool strided = t.kind == FFK_TILE_STRIDED;
@@ -171,29 +157,6 @@ __device__ __forceinline__ void ws_store_rows(const WsSlot& t, const f32x16& acc
                 if (gate) gv[j] = *reinterpret_cast<const u32x4*>(gate + cj);
                 if (resid) rv[j] = *reinterpret_cast<const u32x4*>(resid + cj);
             }
-            if (XT && t.xtail) {     // extended residual stream (whole 16-channel runs: ncols % 16 == 0 with a tail)
-                const u32x4 tv = *reinterpret_cast<const u32x4*>(t.xtail + (ok1 ? off : off - cl));
-                u32x4 tn;
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {       // eight channels at a time (register budget)
-                    float f[8];
-                    xs_decode8(rv[j], tv[2 * j], tv[2 * j + 1], f);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        float u = (float)y[8 * j + e];
-                        if (gate) u = (float)(T)(u * gate_factor((float)reinterpret_cast<const T*>(&gv[j])[e], POS ? t.act : FFK_ACT_NONE));
-                        f[e] += u;
-                    }
-                    u32x4 hv;
-                    uint32_t ta, tb;
-                    xs_encode8(f, hv, ta, tb);
-                    tn[2 * j] = ta;
-                    tn[2 * j + 1] = tb;
-                    if (ok1) *reinterpret_cast<u32x4*>(out + off + 8 * j) = hv;
-                }
-                if (ok1) *reinterpret_cast<u32x4*>(t.xtail + off) = tn;
-                return;
-            }
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const T* gh = reinterpret_cast<const T*>(&gv[j]);
@@ -201,7 +164,7 @@ __device__ __forceinline__ void ws_store_rows(const WsSlot& t, const f32x16& acc
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     float f = (float)y[8 * j + e];
-                    if (gate) f = (float)(T)(f * gate_factor((float)gh[e], POS ? t.act : FFK_ACT_NONE));
+                    if (gate) f = (float)(T)(f * gate_factor((float)gh[e], t.act));
                     if (resid) f += (float)rh[e];
                     y[8 * j + e] = (T)f;
                 }
@@ -356,13 +319,12 @@ __device__ __forceinline__ void ws_store_rows_folded(const WsSlot& t, const f32x
 // DUAL: the gate halves of the GLU units multiply a second operand (row-major rows, own LayerNorm).  Its
 // slab goes from global memory straight into LDS (unpadded 256-byte rows, 16-byte columns XOR-swizzled
 // with the row index) one slab ahead and is normalised in place by the threads that requested it.
-// XT: the launch has tiles with a residual tail (extended residual stream); only those instantiations carry its code
+// XT (with DUAL): the launch has tiles with a residual tail (extended residual stream); only that instantiation carries its code
 template <int WS_K, bool DUAL, bool XT>
 __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs args) {
     typedef Mma<T> MM;
     typedef WsGeo<WS_K> G;
     constexpr int WS_KS = G::KS, WS_AP = G::AP, WS_BM = G::BM, WS_RG = G::RG;
-    constexpr bool POS = !XT;                              // variants that take FFK_ACT_GATE_POS (the others have no register for it)
     constexpr int NS = WS_NS, AFC = WS_K == 128 ? 8 : 4;   // AFC: A fragments held at a time (register budget)
     const WsArgs& d = args;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -682,8 +644,8 @@ __global__ __launch_bounds__(WS_THREADS, 2) void linear_ws_kernel(const WsArgs a
                         }
                         ws_store_rows_folded<XT>(t, acc, accg, sb, s_c1 + sp[s].wrow, rstd, -rstd * mean, rstd_g, -rstd_g * mean_g,
                                              valid, c_hi, c_lo, half, a2r, a2v, n32 & 15);
-                    } else if (glu) ws_store_rows<true, XT, POS>(t, acc, accg, sb, valid, mc, c_hi, c_lo, half);
-                    else ws_store_rows<false, XT, POS>(t, acc, accg, sb, valid, mc, c_hi, c_lo, half);
+                    } else if (glu) ws_store_rows<true>(t, acc, accg, sb, valid, mc, c_hi, c_lo, half);
+                    else ws_store_rows<false>(t, acc, accg, sb, valid, mc, c_hi, c_lo, half);
                 } else {
                     if (glu) ws_store_cols<true>(t, acc, accg, sb, m0g, M, l32, half);
                     else ws_store_cols<false>(t, acc, accg, sb, m0g, M, l32, half);
