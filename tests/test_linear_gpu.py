@@ -185,8 +185,8 @@ def test_bias_tiles(dev, dtype, r, H):
 
 @pytest.mark.parametrize("r,H", [(45, 4), (64, 3), (33, 1)])
 def test_bias_tile_rides_on_a_projection_launch(dev, r, H):
-    """A trailing FFK_TILE_BIAS tile in a launch of the weights-stationary kernel (bf16, K = 128, <= 4 heads): computed
-    on the vector pipe from the slab rows, no weight slot.  Checked against numpy, against the staged kernels on the
+    """A trailing FFK_TILE_BIAS tile in a launch of the weights-in-registers kernel (bf16, K = 128, <= 4 heads): computed
+    by small products on the slab rows, no weight slot.  Checked against numpy, against the staged kernels on the
     same descriptor, in both traversal orders; the other tile of the launch is unaffected and the padding of ragged
     bias tiles stays zero."""
     from fastfold_amd import _lib
@@ -761,6 +761,24 @@ def test_fp32_glu_tile_with_residual(dev, M, nt, ncols):
                             inner=M, s_i=nt * 64) for i in range(nt)]
     _lib.fused_linear(x, w, tiles, M=M, K=K)
     assert float((out.view(M, nt, 64) - ref).abs().max()) <= 2e-5 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("r", [362, 411])
+def test_fp32_gated_projection_persistent_layout(dev, r):
+    """The GLU projection of a triangle multiplication (channel-major outputs, row mask) at rows enough for the persistent layout
+    (131 044: eight units on 256 workgroups of eight waves) and a ragged last slab, against the staged kernel."""
+    from fastfold_amd import _lib
+    M, K, nt = r * r, 128, 4
+    g = torch.Generator(device=dev).manual_seed(r)
+    x, w, b = (torch.randn(*sh, device=dev, generator=g) for sh in ((M, K), (nt * 128, K), (nt * 128,)))
+    w, ln, mask = w / K ** 0.5, torch.randn(2, K, device=dev, generator=g), (torch.rand(r, device=dev, generator=g) > 0.3).float()
+    got = []
+    for staged in (True, False):
+        got.append(torch.full((256, M), 7.0, device=dev))
+        tiles = [_lib.make_tile(got[-1].data_ptr() + 256 * i * M, inner=r, s_o=r, s_i=1, s_h=32 * M, s_d=M, glu=1, ncols=64, bias=b.data_ptr() + 512 * i,
+                                rowmask=mask, m_so=1) for i in range(nt)]
+        _lib.fused_linear(x, w, tiles, M=M, K=K, ln=(ln[0], ln[1]), staged=staged)
+    assert float((got[0] - got[1]).abs().max()) <= 1e-5 * float(got[0].abs().max())
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
