@@ -710,7 +710,7 @@ constexpr int rm_occ(int K, int waves, int ns, int np, bool res) {      // waves
 // 65 536 rows 28.1 / 29.1 / 32.0, 1 048 576 rows 315 / 345 / 560.
 struct RmVariant { int K, waves, ns, np; bool res; };
 constexpr RmVariant RM_VARIANTS[] = {
-    {64, 8, 1, 4, false},  {64, 8, 2, 4, false},  {64, 4, 1, 2, false},  {64, 4, 2, 2, false},  {64, 8, 1, 4, true},  {64, 4, 1, 2, true},
+    {64, 8, 2, 4, false},  {64, 4, 1, 2, false},  {64, 4, 2, 2, false},  {64, 8, 1, 4, true},  {64, 4, 1, 2, true},
     {128, 8, 1, 4, false}, {128, 8, 2, 4, false}, {128, 4, 1, 2, false}, {128, 4, 2, 2, false}, {128, 4, 2, 4, false},
     {128, 8, 1, 4, true},  {128, 4, 1, 2, true},  {128, 4, 1, 4, true},
     {256, 8, 1, 4, false}, {256, 8, 2, 4, false}, {256, 4, 1, 4, false}, {256, 8, 1, 4, true},  {256, 4, 1, 4, true},
