@@ -627,6 +627,33 @@ def test_row_major_layouts(dev, K, B2, N):
         assert torch.isfinite(a.float()).all() and _rel(_np(a), _np(c)) < 2 ** -7, i
 
 
+@pytest.mark.parametrize("K,units,M,kind", [(64, 12, 32763, "tail"), (64, 12, 32763, "resid"), (64, 20, 32763, "plain"), (128, 6, 32763, "tail"),
+                                            (128, 3, 32763, "plain"), (128, 2, 9211, "glu"), (128, 12, 16379, "glu"), (256, 24, 16379, "plain")])
+def test_row_major_layouts_of_many_units(dev, K, units, M, kind):
+    """Launches that take the layouts of eight waves and of two units per wave, and of four waves over 64 rows, with a ragged last
+    slab, against the LDS-staged kernels (the same products, rounded once)."""
+    from fastfold_amd import _lib
+    bf = torch.bfloat16
+    g = torch.Generator(device=dev).manual_seed(K + units)
+
+    def rnd(*s):
+        return torch.randn(*s, device=dev, generator=g).to(bf)
+    C = 64 if kind == "glu" else 128                  # channels per tile
+    nt, N = -(-units * 32 // C), units * 32
+    x, w, b, ln = rnd(M, K), rnd(nt * 128, K) / K ** 0.5, rnd(nt * 128), (1 + 0.1 * rnd(K), 0.1 * rnd(K))
+    init, tail = rnd(M, nt * C), torch.randint(-128, 128, (M, nt * C), device=dev, generator=g).to(torch.int8)
+    init[init == 0] = 1.0
+    got = []
+    for staged in (False, True):
+        y, t = init.clone(), tail.clone()
+        at = lambda p, i: p.data_ptr() + i * C * p.element_size()
+        tiles = [_lib.make_tile(at(y, i), bias=b.data_ptr() + 256 * i, inner=M, s_i=nt * C, glu=int(kind == "glu"), ncols=min(C, N - i * C),
+                                resid=at(y, i) if kind in ("resid", "tail") else None, xtail=at(t, i) if kind == "tail" else None) for i in range(nt)]
+        _lib.fused_linear(x, w, tiles, M=M, K=K, ln=ln, staged=staged)
+        got.append(((y.view(torch.int16).int() << 16) + (t.int() << 8)).view(torch.float32) if kind == "tail" else y)
+    assert torch.isfinite(got[0].float()).all() and float((got[0].float() - got[1].float()).abs().max()) < 2 ** -7 * float(got[1].float().abs().max())
+
+
 @pytest.mark.parametrize("K", [128, 256])
 @pytest.mark.parametrize("B,N", [(1, 1), (3, 37), (64, 64), (131, 96), (260, 128)])
 def test_fp32_row_layouts(dev, K, B, N):

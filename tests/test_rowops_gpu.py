@@ -183,3 +183,47 @@ def test_errors_raise_runtime_error(dev):
         fused_softmax(x, torch.ones(1, 2, 5, device=dev))                          # wrong mask shape
     with pytest.raises(RuntimeError):
         fused_softmax(x.double())                                                  # unsupported dtype
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("accesses", [1, 7, 8, 13, 16, 25, 32, 51, 64, 101, 128, 201, 256, 301, 512, 701])
+def test_row_kernels_at_every_geometry(dev, dtype, accesses):
+    """Rows of so many 16-byte, two-element and one-element accesses: the lanes and accesses per lane the row kernels are built
+    with, whole and partly filled, forward and backward, against float64 on the GPU (one or two roundings to the type)."""
+    from fastfold_amd.model.fastnn.kernel import LayerNorm, bias_dropout_add, bias_ele_dropout_residual, bias_sigmod_ele, fused_softmax
+    vec = 4 if dtype == torch.float32 else 8
+    tol = {torch.float32: 5e-6, torch.bfloat16: 1.5e-2, torch.float16: 2e-3}[dtype]
+    g = torch.Generator(device=dev).manual_seed(accesses)
+
+    def rnd(*s):
+        return torch.randn(*s, device=dev, generator=g).to(dtype)
+
+    def check(got, ref, what):
+        for a, e in zip(got, ref):
+            assert float(((a.double() - e).norm() / e.norm().clamp_min(1e-3)).detach()) <= tol, what
+    for cols in {vec * accesses, 2 * accesses, accesses}:
+        x, bias, dy = rnd(1, 3, 2, 5, cols).requires_grad_(True), rnd(1, 1, 2, 5, cols).requires_grad_(True), rnd(1, 3, 2, 5, cols)
+        mask = (torch.rand(1, 3, cols, device=dev, generator=g) > 0.2).to(dtype)
+        mask[..., -1] = 1
+        xr, br = (t.detach().double().requires_grad_(True) for t in (x, bias))
+        s = torch.where(mask[:, :, None, None] == 0, -1e9, xr + br).softmax(-1)
+        ref = torch.autograd.grad(s, (xr, br), dy.double())
+        y = fused_softmax(x, mask, bias)
+        check((y, *torch.autograd.grad(y, (x, bias), dy)), (s, *ref), cols)
+        check(torch.autograd.grad(fused_softmax(x, mask, bias.detach()), (x,), dy), ref[:1], cols)
+        if cols == 1:
+            continue                                     # a row of one element has no variance
+        norm = LayerNorm(cols).to(dev, dtype)
+        with torch.no_grad():
+            norm.weight.copy_(1 + 0.2 * rnd(cols))
+            norm.bias.copy_(0.1 * rnd(cols))
+        x, dy = rnd(70, cols).requires_grad_(True), rnd(70, cols)
+        xr, wr, br = (t.detach().double().requires_grad_(True) for t in (x, norm.weight, norm.bias))
+        yr = torch.nn.functional.layer_norm(xr, (cols,), wr, br, norm.eps)
+        y = norm(x)
+        check((y, *torch.autograd.grad(y, (x, norm.weight, norm.bias), dy)), (yr, *torch.autograd.grad(yr, (xr, wr, br), dy.double())), cols)
+        a, z, r, b, dm = rnd(1, 4, 3, cols), rnd(1, 4, 3, cols), rnd(1, 4, 3, cols), rnd(cols), rnd(1, 1, 3, cols)
+        ad, zd, rd, bd, dd = (t.double() for t in (a, z, r, b, dm))
+        check((bias_sigmod_ele(a, b, z), bias_dropout_add(a, b, dm, r, prob=0.25, training=False),
+               bias_ele_dropout_residual(a, b, z, dm, r, prob=0.25, training=False)),
+              (torch.sigmoid(ad + bd) * zd, rd + (ad + bd) * dd, rd + dd * (zd * (ad + bd))), cols)
