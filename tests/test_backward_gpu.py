@@ -293,3 +293,20 @@ def test_operators_of_empty_tensors(dev, b2, n):
     leaves = (q, k, v, pair, logits, bias, x, norm.weight, norm.bias)
     for t, g in zip(leaves, torch.autograd.grad(outs, leaves, [torch.ones_like(o) for o in outs])):
         assert g.shape == t.shape and not g.any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d,n", [(64, 45), (128, 33)])
+def test_wide_heads_without_a_bias(dev, dtype, d, n):
+    """Forward and gradients of the attention core at head dimensions 64 and 128, masked, no pair bias, against float64."""
+    from fastfold_amd.model.fastnn.kernel import fused_attention_core
+    g = torch.Generator(device=dev).manual_seed(d)
+    q, k, v = (torch.randn(1, 3, 2, n, d, device=dev, generator=g).to(dtype).requires_grad_(True) for _ in range(3))
+    mask, do = (torch.rand(1, 3, n, device=dev, generator=g) > 0.2).to(dtype), torch.randn(1, 3, n, 2 * d, device=dev, generator=g).to(dtype)
+    mask[..., 0] = 1
+    o = fused_attention_core(q, k, v, mask, None)
+    dq, dk, dv = (t.detach().double().requires_grad_(True) for t in (q, k, v))
+    s = torch.matmul(dq * d ** -0.5, dk.transpose(-1, -2).contiguous())
+    ref = torch.matmul(torch.where(mask[:, :, None, None] == 0, -1e9, s).softmax(-1), dv).transpose(2, 3).reshape(1, 3, n, 2 * d)
+    for a, e in zip((o, *torch.autograd.grad(o, (q, k, v), do)), (ref, *torch.autograd.grad(ref, (dq, dk, dv), do.double()))):
+        assert float(((a.double() - e).norm() / e.norm()).detach()) <= (1e-5 if dtype == torch.float32 else 2e-2)

@@ -227,3 +227,19 @@ def test_row_kernels_at_every_geometry(dev, dtype, accesses):
         check((bias_sigmod_ele(a, b, z), bias_dropout_add(a, b, dm, r, prob=0.25, training=False),
                bias_ele_dropout_residual(a, b, z, dm, r, prob=0.25, training=False)),
               (torch.sigmoid(ad + bd) * zd, rd + (ad + bd) * dd, rd + dd * (zd * (ad + bd))), cols)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("cols", [32, 64, 128, 256, 512])
+def test_layernorm_bwd_entry_point(dev, dtype, cols):
+    """ffk_layernorm_bwd at the lengths whose module goes to ffk_layernorm_bwd_rows: column sums by one atomic per column and block."""
+    from fastfold_amd import _lib
+    rows, g = 203, torch.Generator(device=dev).manual_seed(cols)
+    x, dy, w = (torch.randn(*s, device=dev, generator=g).to(dtype) for s in ((rows, cols), (rows, cols), (cols,)))
+    xr, wr, br = x.double().requires_grad_(True), w.double().requires_grad_(True), torch.zeros(cols, device=dev, dtype=torch.double).requires_grad_(True)
+    ref = torch.autograd.grad(torch.nn.functional.layer_norm(xr, (cols,), wr, br), (xr, wr, br), dy.double())
+    mean, rstd = x.float().mean(-1), (x.double().var(-1, unbiased=False) + 1e-5).rsqrt().float()
+    dx, dw, db = torch.empty_like(x), torch.zeros(cols, device=dev), torch.zeros(cols, device=dev)
+    _lib.call("ffk_layernorm_bwd", *(_lib.ptr(t) for t in (dx, dw, db, dy, x, mean, rstd, w)), rows, cols, _lib.dtype_tag(dtype), _lib.stream_ptr())
+    for a, e, tol in zip((dx, dw, db), ref, ({torch.float32: 1e-5, torch.bfloat16: 1e-2, torch.float16: 2e-3}[dtype], 1e-5, 1e-5)):
+        assert float((a.double() - e).norm() / e.norm()) <= tol
