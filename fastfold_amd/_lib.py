@@ -415,6 +415,17 @@ def gated_out_fused(out, x, gamma, beta, wg, bg, o, wo, bo, *, M, C, inner, s_o,
          M, C, inner, s_o, s_i, eps, dtype_tag(o.dtype), stream_ptr())
 
 
+SIGNATURES["ffk_attention_block"] = [_P] * 12 + [_L] * 7 + [_F, _I, _P]
+
+
+def attention_block(out, x, gamma, beta, w, bg, bo, bias_t, keybias, tileflags, *, B2, N, C, D, s_row, s_tok, bias_pitch=0,
+                    eps=1e-5, xtail=None, drop=None, dtype=None):
+    """A gated attention from the rows of x to the updated rows in one kernel (see include/ffk.h)."""
+    call("ffk_attention_block", ptr(out), ptr(x), ptr(xtail), ptr(gamma), ptr(beta), ptr(w), ptr(bg), ptr(bo), ptr(bias_t),
+         ptr(keybias), ptr(tileflags), ptr(drop), B2, N, C, D, s_row, s_tok, bias_pitch, eps,
+         dtype_tag(dtype if dtype is not None else x.dtype), stream_ptr())
+
+
 def key_bias(keybias, tileflags, mask, *, B, N, mask_sb=0, mask_sn=1):
     call("ffk_key_bias", ptr(keybias), ptr(tileflags), ptr(mask), B, N, mask_sb, mask_sn,
          dtype_tag(mask.dtype) if mask is not None else FFK_F32, stream_ptr())

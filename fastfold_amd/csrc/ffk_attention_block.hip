@@ -1,0 +1,798 @@
+// A whole gated attention sub-module in one kernel (see ffk_attention_block in include/ffk.h), bf16, as many hidden as input channels:
+//     out = x + Wo . ( sigmoid( Wg . y + bg ) * softmax( q . k^T + bias ) v ) + bo,     q, k, v = Wq y, Wk y, Wv y,  y = LayerNorm(x)
+//
+// A workgroup of eight waves owns one batch row - the N tokens that attend to each other - from the rows of x to the updated rows.
+// A wave owns a head (or a block of 32 channels: two heads of 16) of some or all of the tiles of 32 tokens, so that a weight fragment
+// is fetched once for several products: with a wave per token tile, every wave fetching all the weights, the projections of 256 rows of
+// 128 tokens at 256 channels took 42 us of a launch of 86, as many bytes out of the second-level cache as it delivers.  The phases:
+//   rows -> LayerNorm -> LDS;  barrier
+//   q, k, v and the gate of the wave's tiles, packed as the MFMA operands they are next, in registers
+//   attention over the key tiles (k, v of all tokens in LDS, or in registers where one wave has all of a head's)
+//   gated outputs -> LDS;  barrier;  output projection, a wave 32 output channels;  updates -> LDS;  barrier;  rows updated
+// Nothing is transposed on the way: the accumulator of Wk y^T is the score product's A operand as it stands, that of Wq y^T its B
+// operand, that of y Wv^T the A operand of the weighted sum, and the gated outputs are the B operand of the output projection, whose
+// weight columns are packed in the accumulator's order.
+//
+// What bounds it: the matrix and vector instructions of a SIMD, which do not overlap (ffk_attention.hip), at two waves per SIMD.  At
+// 256 rows of 256 tokens, 128 channels, of 37 us: rows and LayerNorm 4, projections 6, attention 15 (240 ns per wave and 32 x 32 scores;
+// its instructions take 230 at the 2 GHz the clock falls to), barriers and exchanges 7, output projection and update 4.
+// What it replaces moves q, k, v, the gate and the heads' outputs through memory and fills and drains the chip three times.
+// us per sub-module, launches of their own -> here (both with the launch that computes the pair bias):
+//   128 channels in 4 heads, N rows of N tokens:  N = 64 17.7 -> 15.0, 96 24.6 -> 19.6, 128 29.4 -> 22.8, 192 49 -> 33.5, 256 62 -> 48
+//   64 channels in 4 heads:  N = 64 18.6 -> 11.1, 128 26.0 -> 15.0, 256 50.5 -> 32, 320 79 -> 77, 512 184 -> 171
+//   256 channels in 8 heads, rows of 128 tokens, no bias:  64 rows 33.5 -> 27.8, 256 69 -> 34, 416 109 -> 59, 1 024 266 -> 125
+//                            with a pair bias:  128 rows of 96 tokens 45 -> 29, of 128 tokens 51 -> 36
+// Longer rows do not fit: at 128 channels, k and v of more than 256 tokens go into LDS in two passes only (heads two by two, rows
+// normalised twice), which was built and is slower (288 tokens 122 us against 92, 416 235 against 189).
+#include "ffk_common.h"
+#include <type_traits>
+
+namespace {
+
+typedef bf16_t T;
+typedef Mma<T> MM;
+
+struct AbArgs {
+    T* out;
+    const T* x;
+    int8_t* xtail;
+    const T *gamma, *beta;
+    const T* w;              // [5][C / 32][C / 16][64][8]: q, k, v, gate, output projection
+    const T *bg, *bo;
+    const T* bias_t;         // [H][NT][bias_pitch] key x query tiles
+    const float* keybias;    // [B2][32 NT]
+    const int* flags;        // [B2][NT]
+    const T* drop;           // [N][C] multipliers of the update, or nullptr
+    long s_row, s_tok;
+    int B2, N, bias_pitch;
+    float qscale, eps;
+};
+
+// The lane number anew, so that the addresses made from it are not kept in registers from one end of a kernel to the other.
+__device__ __forceinline__ int ab_lane(int lane) {
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
+// Computed here: the compiler would otherwise move the packing to the value's use and keep the unpacked numbers in twice the registers.
+__device__ __forceinline__ void ab_pin(bf16x8& f) { asm volatile("" : "+v"(*reinterpret_cast<u32x4*>(&f))); }
+
+__device__ __forceinline__ bf16x8 ab_pack8(const f32x16& a, int v0, float scale) {
+    bf16x8 r;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) r[t] = (T)(a[v0 + t] * scale);
+    return r;
+}
+
+// What the rows take: eight waves, C / 8 lanes to a row, so that a request of a wave is 1 KB of whole rows.
+template <int C, int NT_MAX> struct AbRows {
+    static constexpr int LPR = C / 8, RPI = 64 / LPR, NI = NT_MAX * 32 / (8 * RPI), XP = C * 2 + 16;
+    // rows i of all waves lie before row 32 NT, or none (half of them: 64 channels and an odd NT)
+    static __device__ __forceinline__ bool past(int i, int NT) { return i * 8 * RPI >= NT * 32; }
+    static __device__ __forceinline__ int row(int i, int wave, int lane) { return (i * 8 + wave) * RPI + lane / LPR; }
+};
+
+// Rows of the batch row -> LayerNorm -> LDS (row-major, 16 bytes of padding); rows past the end repeat the last one.
+template <int C, int NT_MAX>
+__device__ __forceinline__ void ab_normalise(const AbArgs& a, const T* xrow, unsigned char* s_x, int NT, int wave, int lane) {
+    typedef AbRows<C, NT_MAX> R;
+    const int c8 = lane % R::LPR;
+    const Vec16<T> g = ld16(a.gamma + c8 * 8), b = ld16(a.beta + c8 * 8);
+    Vec16<T> r[R::NI];
+#pragma unroll
+    for (int i = 0; i < R::NI; ++i) {
+        if (R::past(i, NT)) break;
+        const int tok = R::row(i, wave, lane);
+        r[i] = ld16(xrow + (long)(tok < a.N ? tok : a.N - 1) * a.s_tok + c8 * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < R::NI; ++i) {
+        if (R::past(i, NT)) break;
+        float f[8], s = 0.0f, q = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            f[e] = (float)r[i].e[e];
+            s += f[e];
+        }
+        const float mu = group_sum(s, R::LPR) * (1.0f / C);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            f[e] -= mu;
+            q = __builtin_fmaf(f[e], f[e], q);
+        }
+        const float rs = rsqrtf(group_sum(q, R::LPR) * (1.0f / C) + a.eps);
+        bf16x8 y;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = (T)__builtin_fmaf(f[e] * rs, (float)g.e[e], (float)b.e[e]);
+        const int row = R::row(i, wave, lane);
+        if (row < NT * 32) *reinterpret_cast<bf16x8*>(s_x + row * R::XP + c8 * 16) = y;
+    }
+}
+
+// The update of a 32 x 32 block (lane: token l32, channels 16 half ..), rounded, to its place in the rows of updates in LDS.
+__device__ __forceinline__ void ab_put(unsigned char* p, f32x16& acc, const T* bo) {
+    if (bo) {
+        const Vec16<T> b0 = ld16(bo), b1 = ld16(bo + 8);
+#pragma unroll
+        for (int v = 0; v < 8; ++v) {
+            acc[v] += (float)b0.e[v];
+            acc[8 + v] += (float)b1.e[v];
+        }
+    }
+    *reinterpret_cast<bf16x8*>(p) = ab_pack8(acc, 0, 1.0f);
+    *reinterpret_cast<bf16x8*>(p + 16) = ab_pack8(acc, 8, 1.0f);
+}
+
+// out = x + update (times its dropout multipliers).  The rows are requested (`fetch`) before the barrier that completes the updates:
+// a lane with a token's 16 channels, as the accumulators have them, would touch 32 lines per request and the epilogue take twice as long.
+template <int C, int NT_MAX> struct AbUpdate {
+    typedef AbRows<C, NT_MAX> R;
+    u32x4 h[R::NI];
+    u32x2 t[R::NI];
+    __device__ __forceinline__ void fetch(const AbArgs& a, long row_off, int NT, int wave, int lane) {
+#pragma unroll
+        for (int i = 0; i < R::NI; ++i) {
+            if (R::past(i, NT)) break;
+            const int tok = R::row(i, wave, lane);
+            const long off = row_off + (long)(tok < a.N ? tok : a.N - 1) * a.s_tok + (lane % R::LPR) * 8;
+            h[i] = *reinterpret_cast<const u32x4*>(a.x + off);
+            if (a.xtail) t[i] = *reinterpret_cast<const u32x2*>(a.xtail + off);
+        }
+    }
+    __device__ __forceinline__ void store(const AbArgs& a, const unsigned char* s_u, long row_off, int NT, int wave, int lane) const {
+        const int c8 = lane % R::LPR;
+#pragma unroll
+        for (int i = 0; i < R::NI; ++i) {
+            if (R::past(i, NT)) break;
+            const int tok = R::row(i, wave, lane);
+            if (tok >= a.N) continue;
+            const bf16x8 u = *reinterpret_cast<const bf16x8*>(s_u + tok * R::XP + c8 * 16);
+            float upd[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) upd[e] = (float)u[e];
+            if (a.drop) {
+                const Vec16<T> d = ld16(a.drop + (long)tok * C + c8 * 8);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) upd[e] = (float)(T)(upd[e] * (float)d.e[e]);
+            }
+            const long off = row_off + (long)tok * a.s_tok + c8 * 8;
+            u32x4 hn;
+            if (a.xtail) {
+                float f[8];
+                u32x2 tn;
+                xs_decode8(h[i], t[i][0], t[i][1], f);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) f[e] += upd[e];
+                xs_encode8(f, hn, tn);
+                *reinterpret_cast<u32x2*>(a.xtail + off) = tn;
+            } else {
+                const bf16x8 x = __builtin_bit_cast(bf16x8, h[i]);
+                bf16x8 y;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) y[e] = (T)(upd[e] + (float)x[e]);
+                hn = __builtin_bit_cast(u32x4, y);
+            }
+            *reinterpret_cast<u32x4*>(a.out + off) = hn;
+        }
+    }
+};
+
+// Geometry of the kernel for 64 and 128 channels: eight waves, 8 / NB of them to a block of 32 channels (one head of 32, two of 16),
+// each with every (8 / NB)-th tile of 32 tokens, at most TPW of them.
+template <int C, int D, int TPW> struct AbGeo {
+    static constexpr int KS = C / 16;               // K steps of a projection
+    static constexpr int NB = C / 32;               // 32-channel blocks
+    static constexpr int HPB = 32 / D;              // heads per block
+    static constexpr int WPB = 8 / NB;              // waves per block
+    static constexpr int NT_MAX = WPB * TPW;
+    static constexpr int XP = C * 2 + 16;           // pitch of the normalised rows (bytes)
+    static constexpr size_t smem(long NT) {         // rows, then k and v, then the gated outputs and the updates
+        const size_t rows = (size_t)NT * 32 * XP, kv = (size_t)NT * NB * 4096, o = (size_t)NT * NB * 2048;
+        return rows + o > kv ? rows + o : kv;
+    }
+};
+
+template <int C, int D, int TPW>
+__global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a) {
+    typedef AbGeo<C, D, TPW> G;
+    constexpr int KS = G::KS, NB = G::NB, HPB = G::HPB, WPB = G::WPB, XP = G::XP;
+    constexpr float NEG_FLOOR = -1.0e4f;             // reference of a row that has met no key (see ffk_attention.hip)
+    extern __shared__ __align__(16) unsigned char ab_smem[];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, half = lane >> 5;
+    const int NT = (a.N + 31) >> 5;
+    // consecutive workgroup ids go to the eight XCDs in turn: each takes a contiguous eighth of the batch rows
+    const unsigned per_xcd = (unsigned)(a.B2 + 7) >> 3;
+    const unsigned b2 = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (b2 >= (unsigned)a.B2) return;                // whole workgroup
+    const int blk = wave % NB, t_first = wave / NB;  // block of hidden (at the end: output) channels, first tile of this wave
+    unsigned char* s_x = ab_smem;                    // [32 NT][XP]
+    T* s_k = reinterpret_cast<T*>(ab_smem);          // [NB][NT][2][64][8]
+    T* s_v = s_k + (size_t)NB * NT * 1024;           // the same
+    T* s_o = s_k;                                    // [NT][NB][2][64][8]
+    const T* xrow = a.x + (long)b2 * a.s_row;
+
+    // key tiles with a masked key; trailing tiles without a valid one are left out
+    const int fl = lane < NT ? a.flags[(long)b2 * NT + lane] : 2;
+    const unsigned long long m_some = __builtin_amdgcn_ballot_w64(fl != 0), m_live = __builtin_amdgcn_ballot_w64(fl != 2);
+    const int kt_end = m_live ? 64 - __builtin_clzll(m_live) : 1;
+    const float* kb = a.keybias + (long)b2 * NT * 32 + 4 * half;
+
+    bf16x8 ident[2];                                 // identity as B operand of the bias (see ffk_attention.hip)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ident[i][e] = (T)(16 * half + 8 * i + e == l32 ? 1.0f : 0.0f);
+
+    // weight fragments of block b of weight `which` (0 q, 1 k, 2 v, 3 gate, 4 output)
+    auto wptr = [&](int which, int b) { return a.w + ((long)which * NB + b) * (KS * 512) + lane * 8; };
+    // tile i of this wave; past the end the last tile again, whose products nobody uses
+    auto tile = [&](int i) { return t_first + WPB * i < NT ? t_first + WPB * i : NT - 1; };
+    // acc = W y^T (or y W^T) over this wave's tiles; fragments of `next` are requested on the way
+    bf16x8 w[KS];
+    auto request = [&](const T* p) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < KS; ++i) w[i] = MM::ld(p + i * 512);
+    };
+    auto project = [&](auto swap, const T* next, f32x16 (&acc)[TPW]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < TPW; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][v] = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const bf16x8 c = w[ks];
+#pragma unroll
+            for (int i = 0; i < TPW; ++i) {
+                const bf16x8 x = *reinterpret_cast<const bf16x8*>(s_x + (tile(i) * 32 + l32) * XP + ks * 32 + half * 16);
+                if (decltype(swap)::value) MM::mma(acc[i], x, c);
+                else MM::mma(acc[i], c, x);
+            }
+            if (next) w[ks] = MM::ld(next + ks * 512);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    // ---- one head of one query tile over all key tiles; o: its D normalised channels, in accumulator order.  bias: tiles 0 and 1
+    // have been requested; those of the next call (bp_next) are requested in the last two steps ----
+    bf16x8 bias[2][2];
+    auto bias_load = [&](const T* p, bf16x8 (&b)[2]) __attribute__((always_inline)) {
+        b[0] = MM::ld(p);
+        b[1] = MM::ld(p + 8);
+    };
+    auto attend = [&](int sub, const T* bp, const T* bp_next, const bf16x8& q0, const bf16x8& q1, f32x16& acc, float& inv) __attribute__((always_inline)) {
+        const T* kp = s_k + (size_t)blk * NT * 1024 + lane * 8;
+        const T* vp = s_v + (size_t)blk * NT * 1024 + lane * 8;
+        f32x16 negm, s;
+        float l_run;
+        auto bias_req = [&](int kt, bf16x8 (&b)[2]) __attribute__((always_inline)) {
+            const int past = kt - kt_end < kt_end ? kt - kt_end : 0;
+            bias_load(kt < kt_end ? bp + (long)kt * 1024 : bp_next + (long)past * 1024, b);
+        };
+        bf16x8 kf[2], vf[2], p[2];
+        auto k_req = [&](int kt) __attribute__((always_inline)) {
+            const T* q = kp + (kt < kt_end ? kt : kt_end - 1) * 1024;
+            if (D == 32) {
+                kf[0] = MM::ld(q);
+                kf[1] = MM::ld(q + 512);
+            } else {
+                kf[0] = MM::ld(q + sub * 512);
+            }
+        };
+        auto v_req = [&](int kt) __attribute__((always_inline)) {
+            vf[0] = MM::ld(vp + kt * 1024);
+            vf[1] = MM::ld(vp + kt * 1024 + 512);
+        };
+        auto score = [&](int kt, const bf16x8 (&b)[2]) __attribute__((always_inline)) {
+            s = negm;
+            if (D == 32) {
+                MM::mma(s, kf[0], q0);
+                MM::mma(s, kf[1], q1);
+            } else {
+                MM::mma(s, kf[0], sub ? q1 : q0);
+            }
+            MM::mma(s, b[0], ident[0]);
+            MM::mma(s, b[1], ident[1]);
+            if ((m_some >> kt) & 1) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const f32x4 mk = *reinterpret_cast<const f32x4*>(kb + kt * 32 + 8 * g);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[4 * g + e] += mk[e];
+                }
+            }
+        };
+        auto prob = [&]() __attribute__((always_inline)) -> float {
+            typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+            const bf16x2 ones = {(T)1.0f, (T)1.0f};
+            float sum = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+#pragma unroll
+                for (int t = 0; t < 8; ++t) p[i][t] = (T)fast_exp2(s[8 * i + t]);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const bf16x2 pr = {p[i][2 * t], p[i][2 * t + 1]};
+                    sum = __builtin_amdgcn_fdot2_f32_bf16(pr, ones, sum, false);
+                }
+            }
+            return sum;
+        };
+        auto weigh = [&]() __attribute__((always_inline)) {
+            MM::mma(acc, vf[0], p[0]);
+            MM::mma(acc, vf[1], p[1]);
+        };
+        // The reference is set by the first tile; a second walk moves it where a row sum shows that a later score lay far above it
+        // (see ffk_attention.hip).
+        for (int careful = 0; careful < 2; ++careful) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[v] = negm[v] = 0.0f;
+            if (careful) {
+                bias_req(0, bias[0]);
+                bias_req(1, bias[1]);
+            }
+            k_req(0);
+            score(0, bias[0]);
+            bias_req(2, bias[0]);
+            v_req(0);
+            k_req(1);
+            asm volatile("" ::: "memory");           // requested here, not at their first use
+            float mt = fmaxf(s[0], s[1]);
+#pragma unroll
+            for (int v = 2; v < 16; ++v) mt = fmaxf(mt, s[v]);
+            const float m0 = fmaxf(fmaxf(mt, lane_xor<32>(mt)), NEG_FLOOR);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                s[v] -= m0;
+                negm[v] = -m0;
+            }
+            l_run = prob();
+            weigh();
+            auto step = [&](int kt, bf16x8 (&b)[2]) __attribute__((always_inline)) {
+                v_req(kt);
+                score(kt, b);
+                if (!careful) {
+                    k_req(kt + 1);
+                    bias_req(kt + 2, b);
+                }
+                asm volatile("" ::: "memory");
+                float sum = prob();
+                if (careful) {
+                    if (__builtin_amdgcn_ballot_w64(!(sum <= 1048576.0f)) != 0) {
+                        const bool fresh = negm[0] == -NEG_FLOOR;
+                        if (fresh) {
+#pragma unroll
+                            for (int v = 0; v < 16; ++v) negm[v] = 0.0f;
+                        }
+                        score(kt, b);
+                        float mx = fmaxf(s[0], s[1]);
+#pragma unroll
+                        for (int v = 2; v < 16; ++v) mx = fmaxf(mx, s[v]);
+                        const float delta = fmaxf(fmaxf(mx, lane_xor<32>(mx)), fresh ? NEG_FLOOR : 0.0f);
+                        const float alpha = fast_exp2((fresh ? NEG_FLOOR : 0.0f) - delta);
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) {
+                            s[v] -= delta;
+                            negm[v] -= delta;
+                            acc[v] *= alpha;
+                        }
+                        l_run *= alpha;
+                        sum = prob();
+                    }
+                    k_req(kt + 1);
+                    bias_req(kt + 2, b);
+                }
+                l_run += sum;
+                weigh();
+            };
+            int kt = 1;
+            for (; kt + 1 < kt_end; kt += 2) {
+                step(kt, bias[1]);
+                step(kt + 1, bias[0]);
+            }
+            if (kt < kt_end) step(kt, bias[1]);
+            // probabilities are not negative: a finite sum shows that none overflowed
+            if (careful || __builtin_amdgcn_ballot_w64(!(l_run <= 1.8446744e19f)) == 0) break;
+        }
+        if (kt_end == 1) {                           // nothing of the next call has been requested in place
+            bias_load(bp_next, bias[0]);
+        } else if (kt_end & 1) {                     // the next call's tiles 0 and 1 lie in the other order
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const bf16x8 t = bias[0][i];
+                bias[0][i] = bias[1][i];
+                bias[1][i] = t;
+            }
+        }
+        const float l_tot = l_run + lane_xor<32>(l_run);
+        inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;              // all keys masked: zero
+    };
+
+    bf16x8 of[TPW][2];                       // gate, then gated outputs
+    request(wptr(1, blk));
+    ab_normalise<C, G::NT_MAX>(a, xrow, s_x, NT, wave, lane);
+    lds_barrier();
+    // ---- projections of this wave's tiles ----
+    bf16x8 qf[TPW][2];
+    {
+        bf16x8 kf[TPW][2], vf[TPW][2];
+        f32x16 acc[TPW];
+        project(std::false_type(), wptr(2, blk), acc);
+#pragma unroll
+        for (int i = 0; i < TPW; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                kf[i][j] = ab_pack8(acc[i], 8 * j, 1.0f);
+                ab_pin(kf[i][j]);
+            }
+        project(std::true_type(), wptr(0, blk), acc);
+#pragma unroll
+        for (int i = 0; i < TPW; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                vf[i][j] = ab_pack8(acc[i], 8 * j, 1.0f);
+                ab_pin(vf[i][j]);
+            }
+        project(std::false_type(), wptr(3, blk), acc);
+#pragma unroll
+        for (int i = 0; i < TPW; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                qf[i][j] = ab_pack8(acc[i], 8 * j, a.qscale);
+                ab_pin(qf[i][j]);
+            }
+        bf16x4 bg[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            bg[g] = __builtin_bit_cast(bf16x4, *reinterpret_cast<const u32x2*>(a.bg + blk * 32 + 4 * half + 8 * g));
+        project(std::false_type(), (const T*)nullptr, acc);
+#pragma unroll
+        for (int i = 0; i < TPW; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) of[i][j][e] = (T)sigmoid_f(acc[i][8 * j + e] + (float)bg[2 * j + (e >> 2)][e & 3]);
+                ab_pin(of[i][j]);
+            }
+        lds_barrier();                           // nobody reads the rows any more
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) {
+            if (t_first + WPB * i < NT) {
+                T* d = s_k + ((size_t)blk * NT + t_first + WPB * i) * 1024 + lane * 8;
+                T* e = s_v + ((size_t)blk * NT + t_first + WPB * i) * 1024 + lane * 8;
+                *reinterpret_cast<bf16x8*>(d) = kf[i][0];
+                *reinterpret_cast<bf16x8*>(d + 512) = kf[i][1];
+                *reinterpret_cast<bf16x8*>(e) = vf[i][0];
+                *reinterpret_cast<bf16x8*>(e + 512) = vf[i][1];
+            }
+        }
+    }
+    auto bias_row = [&](int i, int sub) {        // bias tiles of a call: tile i, head sub of the block
+        return a.bias_t + ((long)(blk * HPB + sub) * NT + tile(i)) * a.bias_pitch * 1024 + lane * 16;
+    };
+    bias_load(bias_row(0, 0), bias[0]);
+    bias_load(bias_row(0, 0) + (kt_end > 1 ? 1024 : 0), bias[1]);
+    lds_barrier();
+    // ---- attention ----
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+        if (t_first + WPB * i < NT) {
+#pragma unroll
+            for (int sub = 0; sub < HPB; ++sub) {
+                f32x16 acc;
+                float inv;
+                const T* next = sub + 1 < HPB ? bias_row(i, sub + 1) : bias_row(i + 1 < TPW ? i + 1 : i, 0);
+                attend(sub, bias_row(i, sub), next, qf[i][0], qf[i][1], acc, inv);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    if (D == 16 && j != sub) continue;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) of[i][j][e] = (T)(acc[8 * j + e] * inv * (float)of[i][j][e]);
+                    ab_pin(of[i][j]);
+                }
+            }
+        }
+    }
+    lds_barrier();                               // nobody reads k and v any more
+
+    // ---- gated outputs to LDS; output projection: 32 channels of the wave's tiles ----
+    request(wptr(4, blk));
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+        if (t_first + WPB * i < NT) {
+            T* d = s_o + ((size_t)(t_first + WPB * i) * NB + blk) * 1024 + lane * 8;
+            *reinterpret_cast<bf16x8*>(d) = of[i][0];
+            *reinterpret_cast<bf16x8*>(d + 512) = of[i][1];
+        }
+    }
+    unsigned char* s_u = ab_smem + (size_t)NT * NB * 2048;         // [32 NT][XP]
+    AbUpdate<C, G::NT_MAX> rows;
+    rows.fetch(a, (long)b2 * a.s_row, NT, wave, ab_lane(lane));
+    lds_barrier();
+    const T* bo = a.bo ? a.bo + blk * 32 + 16 * half : nullptr;
+    f32x16 acc[TPW];
+#pragma unroll
+    for (int i = 0; i < TPW; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][v] = 0.0f;
+#pragma unroll
+    for (int f = 0; f < KS; ++f)
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) MM::mma(acc[i], w[f], MM::ld(s_o + ((size_t)tile(i) * KS + f) * 512 + lane * 8));
+#pragma unroll
+    for (int i = 0; i < TPW; ++i)                    // past the end: the last tile's update once more
+        ab_put(s_u + (tile(i) * 32 + l32) * XP + blk * 64 + half * 32, acc[i], bo);
+    lds_barrier();
+    rows.store(a, s_u, (long)b2 * a.s_row, NT, wave, ab_lane(lane));
+}
+
+// 256 channels in eight heads, rows of at most 128 tokens: a wave owns a head, its q, k, v and gate of all NT token tiles stay in its
+// registers, and no weight is read by two waves.  The normalised rows lie in LDS (row-major, 16 bytes of padding), the gated outputs
+// of the heads beside them, in the order of the output projection's fragments; there a wave owns 32 output channels of all tokens.
+constexpr int AW_C = 256, AW_KS = 16, AW_XP = AW_C * 2 + 16;
+template <int NT> constexpr size_t aw_smem() { return (size_t)NT * 32 * AW_XP + (size_t)NT * 8 * 2048; }
+
+template <int NT, bool BIAS>
+__global__ __launch_bounds__(512, 2) void attention_block_wide_kernel(const AbArgs a) {
+    constexpr int C = AW_C, KS = AW_KS, XP = AW_XP;
+    constexpr int AHEAD = 4;                         // weight fragments requested ahead, of each of two weights
+    extern __shared__ __align__(16) unsigned char ab_smem[];
+    unsigned char* s_x = ab_smem;                    // [32 NT][XP]
+    T* s_o = reinterpret_cast<T*>(ab_smem + NT * 32 * XP);   // [NT][8 heads][2][64][8]
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, half = lane >> 5;
+    const unsigned per_xcd = (unsigned)(a.B2 + 7) >> 3;      // see attention_block_kernel
+    const unsigned b2 = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (b2 >= (unsigned)a.B2) return;
+    const T* xrow = a.x + (long)b2 * a.s_row;
+
+    ab_normalise<C, NT>(a, xrow, s_x, NT, wave, lane);
+    const unsigned char* xp = s_x + l32 * XP + half * 16;
+    const T* wbase = a.w + (long)wave * KS * 512 + lane * 8;         // this head's block (output: this wave's channels)
+    auto wptr = [&](int which) { return wbase + (long)which * 8 * KS * 512; };
+
+    // two weights at a time over all tokens: acc[0] = W0 y^T, acc[1] = W1 y^T or (V1) y W1^T
+    auto project2 = [&](const T* w0, const T* w1, auto v1, f32x16 (&acc)[2][NT]) __attribute__((always_inline)) {
+        bf16x8 f0[AHEAD], f1[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            f0[i] = MM::ld(w0 + i * 512);
+            f1[i] = MM::ld(w1 + i * 512);
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[0][t][v] = acc[1][t][v] = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const bf16x8 c0 = f0[ks % AHEAD], c1 = f1[ks % AHEAD];
+            if (ks + AHEAD < KS) {
+                f0[ks % AHEAD] = MM::ld(w0 + (ks + AHEAD) * 512);
+                f1[ks % AHEAD] = MM::ld(w1 + (ks + AHEAD) * 512);
+            }
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const bf16x8 x = *reinterpret_cast<const bf16x8*>(xp + t * 32 * XP + ks * 32);
+                MM::mma(acc[0][t], c0, x);
+                if (decltype(v1)::value) MM::mma(acc[1][t], x, c1);
+                else MM::mma(acc[1][t], c1, x);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    bf16x8 qf[NT][2], kf[NT][2], vf[NT][2], gf[NT][2];
+    lds_barrier();
+    {
+        f32x16 acc[2][NT];
+        project2(wptr(0), wptr(1), std::false_type(), acc);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                qf[t][i] = ab_pack8(acc[0][t], 8 * i, a.qscale);
+                kf[t][i] = ab_pack8(acc[1][t], 8 * i, 1.0f);
+                ab_pin(qf[t][i]);
+                ab_pin(kf[t][i]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        project2(wptr(3), wptr(2), std::true_type(), acc);
+        bf16x4 bg[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            bg[g] = __builtin_bit_cast(bf16x4, *reinterpret_cast<const u32x2*>(a.bg + wave * 32 + 4 * half + 8 * g));
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                vf[t][i] = ab_pack8(acc[1][t], 8 * i, 1.0f);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) gf[t][i][e] = (T)sigmoid_f(acc[0][t][8 * i + e] + (float)bg[2 * i + (e >> 2)][e & 3]);
+                ab_pin(vf[t][i]);
+                ab_pin(gf[t][i]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+
+    // ---- the head's attention: the scores of a query tile with all keys fit the registers ----
+    const int fl = lane < NT ? a.flags[(long)b2 * NT + lane] : 0;
+    const unsigned some = (unsigned)__builtin_amdgcn_ballot_w64(fl != 0);
+    const float* kb = a.keybias + (long)b2 * NT * 32 + 4 * half;
+    bf16x8 ident[2];
+    if (BIAS) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ident[i][e] = (T)(16 * half + 8 * i + e == l32 ? 1.0f : 0.0f);
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        f32x16 s[NT];
+        float m = -1.0e4f;                           // a row without a key: every probability zero
+        bf16x8 bias[NT][2];
+        if (BIAS) {
+            const T* bp = a.bias_t + ((long)wave * NT + t) * a.bias_pitch * 1024 + lane * 16;
+#pragma unroll
+            for (int kt = 0; kt < NT; ++kt) {
+                bias[kt][0] = MM::ld(bp + kt * 1024);
+                bias[kt][1] = MM::ld(bp + kt * 1024 + 8);
+            }
+        }
+#pragma unroll
+        for (int kt = 0; kt < NT; ++kt) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) s[kt][v] = 0.0f;
+            MM::mma(s[kt], kf[kt][0], qf[t][0]);
+            MM::mma(s[kt], kf[kt][1], qf[t][1]);
+            if (BIAS) {
+                MM::mma(s[kt], bias[kt][0], ident[0]);
+                MM::mma(s[kt], bias[kt][1], ident[1]);
+            }
+        }
+        if (some) {                                  // some key of the row is masked or padding
+#pragma unroll
+            for (int kt = 0; kt < NT; ++kt)
+                if ((some >> kt) & 1) {
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        const f32x4 mk = *reinterpret_cast<const f32x4*>(kb + kt * 32 + 8 * g);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) s[kt][4 * g + e] += mk[e];
+                    }
+                }
+        }
+#pragma unroll
+        for (int kt = 0; kt < NT; ++kt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) m = fmaxf(m, s[kt][v]);
+        m = fmaxf(m, lane_xor<32>(m));
+        float l = 0.0f;
+        f32x16 o;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[v] = 0.0f;
+#pragma unroll
+        for (int kt = 0; kt < NT; ++kt) {
+            typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+            const bf16x2 ones = {(T)1.0f, (T)1.0f};
+            bf16x8 p[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) p[i][e] = (T)fast_exp2(s[kt][8 * i + e] - m);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const bf16x2 pr = {p[i][2 * e], p[i][2 * e + 1]};
+                    l = __builtin_amdgcn_fdot2_f32_bf16(pr, ones, l, false);
+                }
+                MM::mma(o, vf[kt][i], p[i]);
+            }
+        }
+        l += lane_xor<32>(l);
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            bf16x8 y;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y[e] = (T)(o[8 * i + e] * inv * (float)gf[t][i][e]);
+            *reinterpret_cast<bf16x8*>(s_o + ((t * 8 + wave) * 2 + i) * 512 + lane * 8) = y;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
+    // ---- output projection: 32 channels of all tokens ----
+    const T* wo = wptr(4);
+    bf16x8 w[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w[i] = MM::ld(wo + i * 512);
+    AbUpdate<C, NT> rows;
+    rows.fetch(a, (long)b2 * a.s_row, NT, wave, ab_lane(lane));
+    lds_barrier();
+    f32x16 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[t][v] = 0.0f;
+#pragma unroll
+    for (int f = 0; f < KS; ++f) {
+        const bf16x8 c = w[f % 8];
+        if (f + 8 < KS) w[f % 8] = MM::ld(wo + (f + 8) * 512);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) MM::mma(acc[t], c, MM::ld(s_o + (t * KS + f) * 512 + lane * 8));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)                     // the normalised rows are not read any more
+        ab_put(s_x + (t * 32 + l32) * XP + wave * 64 + half * 32, acc[t], a.bo ? a.bo + wave * 32 + 16 * half : nullptr);
+    lds_barrier();
+    rows.store(a, s_x, (long)b2 * a.s_row, NT, wave, ab_lane(lane));
+}
+
+template <int C, int D, int TPW> int ab_launch(const AbArgs& a, long NT, hipStream_t st) {
+    typedef AbGeo<C, D, TPW> G;
+    static FfkLdsReservation lds_reserved;
+    const int rc = ffk_reserve_lds(lds_reserved, (const void*)attention_block_kernel<C, D, TPW>, G::smem(G::NT_MAX), "ffk_attention_block");
+    if (rc != FFK_OK) return rc;
+    attention_block_kernel<C, D, TPW><<<dim3(8u * ffk_cdiv(a.B2, 8)), 512, G::smem(NT), st>>>(a);
+    return ffk_check_launch("ffk_attention_block");
+}
+template <int NT, bool BIAS> int aw_launch(const AbArgs& a, hipStream_t st) {
+    static FfkLdsReservation lds_reserved;
+    const int rc = ffk_reserve_lds(lds_reserved, (const void*)attention_block_wide_kernel<NT, BIAS>, aw_smem<NT>(), "ffk_attention_block");
+    if (rc != FFK_OK) return rc;
+    attention_block_wide_kernel<NT, BIAS><<<dim3(8u * ffk_cdiv(a.B2, 8)), 512, aw_smem<NT>(), st>>>(a);
+    return ffk_check_launch("ffk_attention_block");
+}
+template <bool BIAS> int aw_launch_nt(const AbArgs& a, long NT, hipStream_t st) {
+    switch (NT) {
+        case 1: return aw_launch<1, BIAS>(a, st);
+        case 2: return aw_launch<2, BIAS>(a, st);
+        case 3: return aw_launch<3, BIAS>(a, st);
+        default: return aw_launch<4, BIAS>(a, st);
+    }
+}
+
+}  // namespace
+
+extern "C" int ffk_attention_block(void* out, const void* x, void* xtail, const void* gamma, const void* beta, const void* w,
+                                   const void* bg, const void* bo, const void* bias_t, const float* keybias,
+                                   const int32_t* tileflags, const void* drop, int64_t B2, int64_t N, int64_t C, int64_t D,
+                                   int64_t s_row, int64_t s_tok, int64_t bias_pitch, float eps, int dtype, void* stream) {
+    FFK_REQUIRE(out && x && gamma && beta && w && bg && keybias && tileflags, FFK_ERR_NULL, "ffk_attention_block: null pointer");
+    FFK_REQUIRE(dtype == FFK_BF16, FFK_ERR_DTYPE, "ffk_attention_block: bf16 only (dtype tag %d)", dtype);
+    FFK_REQUIRE((C == 128 && D == 32) || (C == 64 && D == 16) || (C == 256 && D == 32), FFK_ERR_UNSUPPORTED,
+                "ffk_attention_block: built for 128 or 256 channels in heads of 32 and 64 in heads of 16, got %ld / %ld", (long)C, (long)D);
+    FFK_REQUIRE(C == 256 || bias_t, FFK_ERR_UNSUPPORTED, "ffk_attention_block: built with a pair bias for 64 and 128 channels");
+    FFK_REQUIRE(B2 > 0 && B2 < (1L << 31) - 64 && N > 0, FFK_ERR_SHAPE, "ffk_attention_block: bad shape B2=%ld N=%ld", (long)B2, (long)N);
+    FFK_REQUIRE(s_row % 16 == 0 && s_tok % 16 == 0, FFK_ERR_ALIGN, "ffk_attention_block: row strides must be multiples of 16 elements");
+    FFK_REQUIRE(ffk_aligned16(out) && ffk_aligned16(x) && ffk_aligned16(xtail) && ffk_aligned16(gamma) && ffk_aligned16(beta) &&
+                    ffk_aligned16(w) && ffk_aligned16(bg) && ffk_aligned16(bo) && ffk_aligned16(bias_t) && ffk_aligned16(keybias) &&
+                    ffk_aligned16(drop),
+                FFK_ERR_ALIGN, "ffk_attention_block: buffers must be 16-byte aligned");
+    const long NT = (N + 31) / 32;
+    FFK_REQUIRE(NT <= (C == 256 ? 4 : C == 128 ? 8 : 16), FFK_ERR_UNSUPPORTED,
+                "ffk_attention_block: rows of %ld tokens are too long for %ld channels", (long)N, (long)C);
+    FFK_REQUIRE(!bias_t || bias_pitch >= NT, FFK_ERR_SHAPE, "ffk_attention_block: bias rows of %ld tiles, %ld needed", (long)bias_pitch, NT);
+    AbArgs a = {(T*)out, (const T*)x, (int8_t*)xtail, (const T*)gamma, (const T*)beta, (const T*)w, (const T*)bg, (const T*)bo,
+                (const T*)bias_t, keybias, (const int*)tileflags, (const T*)drop, (long)s_row, (long)s_tok, (int)B2, (int)N,
+                (int)bias_pitch, 1.4426950408889634f / sqrtf((float)D), eps};
+    hipStream_t st = (hipStream_t)stream;
+    if (C == 256) return bias_t ? aw_launch_nt<true>(a, NT, st) : aw_launch_nt<false>(a, NT, st);
+    if (C == 64) {
+        switch ((NT + 3) / 4) {
+            case 1: return ab_launch<64, 16, 1>(a, NT, st);
+            case 2: return ab_launch<64, 16, 2>(a, NT, st);
+            case 3: return ab_launch<64, 16, 3>(a, NT, st);
+            default: return ab_launch<64, 16, 4>(a, NT, st);
+        }
+    }
+    switch ((NT + 1) / 2) {
+        case 1: return ab_launch<128, 32, 1>(a, NT, st);
+        case 2: return ab_launch<128, 32, 2>(a, NT, st);
+        case 3: return ab_launch<128, 32, 3>(a, NT, st);
+        default: return ab_launch<128, 32, 4>(a, NT, st);
+    }
+}

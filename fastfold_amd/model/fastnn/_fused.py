@@ -45,7 +45,7 @@ def alloc(shape, dtype, device, zero=False):
 def switches():
     """Everything besides shapes and dtypes that the launch sequences below depend on."""
     return (_WS_BUDGET_DEFAULT, _WS_BUDGET_CHUNKED, _FUSED_TRANSITION, _TRIMUL_CHAN_PAD, _PAIR_BIAS_RIDES, _BIAS_ROW_PAD,
-            _GATE_IN_OUT_STAGE, _GATE_IN_OUT_MIN_N, _GATE_IN_OUT_WIDTHS)
+            _GATE_IN_OUT_STAGE, _GATE_IN_OUT_MIN_N, _GATE_IN_OUT_WIDTHS, _ATTENTION_BLOCK)
 
 
 def pack_rows(mats, dtype, device):
@@ -248,6 +248,29 @@ def key_bias(mask, device, *, B2, N, mask_sb, mask_sn):
     return build() if mask is None else _mask_derived(mask, ("key_bias", B2, N, mask_sb, mask_sn), build)
 
 
+def attention_block_tokens(dtype, H, c, d_in, d_out):
+    """Longest row of tokens that ``ffk_attention_block`` takes at these widths, 0 where it is not built for them.  It is the faster
+    path at every length it takes (timings of both sides in csrc/ffk_attention_block.hip)."""
+    if dtype != torch.bfloat16 or d_in != d_out or H * c != d_in:
+        return 0
+    return {(128, 32): 256, (64, 16): 512, (256, 32): 128}.get((d_in, c), 0)
+
+
+def pack_attention_block(qkv_w, gate_w, out_w, dtype, device):
+    """The weights of a gated attention in the fragment order of ``ffk_attention_block``: [q, k, v, gate, out][C/32][C/16][64][8]."""
+    C = gate_w.shape[0]
+    nb, ks = C // 32, C // 16
+    ws = torch.cat([qkv_w.detach(), gate_w.detach()], 0).to(device=device, dtype=dtype)
+    ws = ws.view(4, nb, 32, ks, 2, 8).permute(0, 1, 3, 4, 2, 5).reshape(-1)          # lane = 32 * (channel half) + row
+    tau = torch.tensor([((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3) for i in range(32)], device=device)
+    wo = out_w.detach().to(device=device, dtype=dtype).view(nb, 32, ks, 2, 2, 4)[:, tau]     # [ct][row][step][quad][half][4]
+    return torch.cat([ws, wo.permute(0, 2, 4, 1, 3, 5).reshape(-1)]).contiguous()
+
+
+# False: every attention runs as projection, core and output stage (tests compare the two)
+_ATTENTION_BLOCK = True
+
+
 def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_pk, out_bias_pk, c_out,
               mask, mask_sb, mask_sn, bias_t=None, bias_in_launch=False, pb_scratch=None, head_dim=32, budget=None, o_map=None, xtail=None,
               drop=None):
@@ -283,6 +306,20 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     # With bf16, 128 input channels and whole key tiles the projection runs on the weights-stationary
     # kernel, which writes q, k and the gate in accumulator order straight from its registers.
     acc_order = dt == torch.bfloat16 and C in (64, 128, 256) and N % 32 == 0
+    # Short rows: one kernel from the rows of x to the updated rows.
+    if (_ATTENTION_BLOCK and acc_order and hasattr(w_pk, "block") and N <= attention_block_tokens(dt, H, head_dim, C, c_out)
+            and ln is not None and resid is not None and resid.data_ptr() == x.data_ptr() and o_map is None
+            and a_so % 16 == 0 and a_si % 16 == 0 and (C == 256 or bias_t is not None or bias_in_launch)
+            and (drop is None or drop.shape[0] == N)):
+        if bias_in_launch:
+            bias_t = alloc((H, NT, NT, 1024), dt, dev)
+            _pair_bias_launch(bias_t, x, ln, w_pk[4 * ((H * 32 + 127) // 128) * 128:], pb_scratch, N=N, C=C, H=H, a_inner=a_inner,
+                              a_so=a_so, a_si=a_si, scale=LOG2E)
+        kb, flags = key_bias(mask, dev, B2=B2, N=N, mask_sb=mask_sb, mask_sn=mask_sn)
+        w, bg = w_pk.block
+        _lib.attention_block(out, x, ln[0], ln[1], w, bg, out_bias_pk, bias_t, kb, flags, B2=B2, N=N, C=C, D=head_dim,
+                             s_row=a_so if a_inner == N else N * a_si, s_tok=a_si, bias_pitch=NT, xtail=xtail, drop=drop)
+        return out
     qk_kind = FFK_TILE_ACC if acc_order else FFK_TILE_QK
     # Packed heads: nothing is written or read for padding (extra-MSA stack, 8 heads of 8 channels: a quarter of the operand
     # bytes; template stack, 4 heads of 16: half of them).

@@ -570,6 +570,9 @@ class SelfAttention(nn.Module, _PackMixin):
                                             + ([] if extra_rows is None else [extra])).contiguous(),
                                   F_.pack_vec([self.gating_bias], dtype, device),
                                   F_.pack_rows([self.o_linear.weight], dtype, device))
+            if F_.attention_block_tokens(dtype, H, c, self.qkv_dim, self.out_dim):
+                w.block = (F_.pack_attention_block(self.to_qkv.weight, self.gating_linear.weight, self.o_linear.weight, dtype, device),
+                           F_.pack_vec([self.gating_bias], dtype, device))
             return (w, F_.pack_vec([_pad_heads(self.gating_bias, H, c, 0)], dtype, device),
                     F_.pack_rows([_pad_heads(self.o_linear.weight, H, c, 1)], dtype, device))
         return self._packed(key, params, build)

@@ -442,6 +442,25 @@ int ffk_gated_out_fused(void* out, const void* x, void* xtail, const void* gamma
                         const void* bg, const void* o, const void* wo, const void* bo, int64_t M, int64_t C,
                         int64_t inner, int64_t s_o, int64_t s_i, float eps, int dtype, void* stream);
 
+/* A gated attention over short rows as one kernel (bf16): each of B2 batch rows of N tokens attends within itself,
+ *     out = x + (Wo . ( sigmoid(Wg y + bg) * attention(Wq y, Wk y, Wv y) ) + bo) * drop,    y = LayerNorm(x; gamma, beta, eps)
+ * C hidden and C output channels, built for C = 128 in heads of D = 32 and C = 64 in heads of 16 (both with a pair bias) and C = 256
+ * in heads of 32 (with or without one), N at most 256, 512 and 128 (what fits the LDS and the registers of a CU).
+ * x, out : token n of batch row b at b * s_row + n * s_tok (elements, multiples of 16; C contiguous channels; may alias);
+ * xtail : NULL or the tail bytes of x / out as an extended residual stream (addressed like x);
+ * w : the five weights in fragment order, [q, k, v, gate, output][C / 32][C / 16][64][8]: element e of lane l in step s of block b
+ *   is row 32 b + l % 32, column 16 s + 8 (l / 32) + e of the [C, C] weight; of the output projection it is row
+ *   32 b + tau(l % 32), tau(8 a + 4 h + c) = 16 h + 4 a + c, and column 16 s + 8 (e / 4) + 4 (l / 32) + e % 4;
+ * bg : [C]; bo : [C] or NULL; drop : [N, C] multipliers of the update of token n, or NULL;
+ * bias_t : [H][NT][bias_pitch] bias tiles (ffk_pair_bias with scale = log2 e; bias_pitch = NT = ceil(N / 32) there); NULL (C = 256): no bias;
+ * keybias, tileflags : of ffk_key_bias for the B2 rows.
+ * Replaces: SelfAttention.forward between the LayerNorm and the residual update of its callers
+ * (fastfold/model/fastnn/ops.py:289-331, 655-670; msa.py:92-104; triangle.py:156-173, 202-222). */
+int ffk_attention_block(void* out, const void* x, void* xtail, const void* gamma, const void* beta, const void* w,
+                        const void* bg, const void* bo, const void* bias_t, const float* keybias, const int32_t* tileflags,
+                        const void* drop, int64_t B2, int64_t N, int64_t C, int64_t D, int64_t s_row, int64_t s_tok,
+                        int64_t bias_pitch, float eps, int dtype, void* stream);
+
 /* Global column attention core of the extra-MSA stack: one query per residue column (the masked mean
  * of the normalised rows), one key / value head of width D shared by the H query heads.
  *     x_s = LayerNorm(m[s, j, :]; gamma, beta, ln_eps)
@@ -590,7 +609,8 @@ enum {
     FFK_OP_TRANSITION_FUSED = 5, FFK_OP_GATED_OUT_FUSED = 6, FFK_OP_GLOBAL_ATTENTION_CORE = 7, FFK_OP_LAYERNORM_FWD = 8,
     FFK_OP_FILL_ZERO = 9, FFK_OP_ATTENTION_FWD_LSE = 10, FFK_OP_ATTENTION_BWD_ROWS = 11, FFK_OP_TRANSPOSE_BATCHED = 12,
     FFK_OP_WEIGHT_GRAD = 13, FFK_OP_LAYERNORM_BWD_ROWS = 14, FFK_OP_SCALE_ROWS = 15, FFK_OP_ATT_GATE_BWD = 16,
-    FFK_OP_TRIMUL_GATE_BWD = 17, FFK_OP_GLU_BWD = 18, FFK_OP_BIAS_COLS = 19, FFK_OP_SLICE_SUM = 20, FFK_OP_COUNT = 21
+    FFK_OP_TRIMUL_GATE_BWD = 17, FFK_OP_GLU_BWD = 18, FFK_OP_BIAS_COLS = 19, FFK_OP_SLICE_SUM = 20,
+    FFK_OP_ATTENTION_BLOCK = 21, FFK_OP_COUNT = 22
 };
 int ffk_run_plan(const void* plan, int64_t bytes, const uint64_t* bases, int64_t n_bases, void* stream);
 

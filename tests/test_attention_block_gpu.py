@@ -1,0 +1,138 @@
+"""ffk_attention_block (a gated attention from the rows of x to the updated rows in one kernel) through the C ABI against float64
+(fastfold/model/fastnn/ops.py:289-331), at the edges of its tiles, waves and layouts."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+LOG2E = math.log2(math.e)
+
+
+def _case(dev, C, D, B2, N, seed, transposed=False, bias=True):
+    g = torch.Generator().manual_seed(seed)
+    H = C // D
+
+    def rnd(*shape, scale=1.0, shift=0.0):
+        return (torch.randn(*shape, generator=g) * scale + shift).to(dev, BF)
+    p = dict(C=C, D=D, H=H, B2=B2, N=N, qkv=rnd(3 * C, C, scale=C ** -0.5), wg=rnd(C, C, scale=C ** -0.5),
+             bg=rnd(C), wo=rnd(C, C, scale=C ** -0.5), gam=rnd(C, scale=0.1, shift=1.0), bet=rnd(C, scale=0.1))
+    p["x"] = rnd(N, B2, C, scale=1.5, shift=0.3).transpose(0, 1) if transposed else rnd(B2, N, C, scale=1.5, shift=0.3)
+    p["bias"] = rnd(H, N, N, scale=1.5) if bias else None   # in the kernel's unit, log2: the same rounded numbers on both sides
+    mask = torch.ones(B2, N)
+    mask[0, N - N // 3:] = 0                                  # a masked tail
+    if B2 > 1:
+        mask[1] = (torch.rand(N, generator=g) > 0.3).float()  # masked keys in every tile
+    if B2 > 2:
+        mask[2] = 0                                           # no key at all
+    if B2 > 3:
+        mask[3, :min(32, N - 1)] = 0                          # a first tile without one
+    p["mask"] = mask.to(dev, BF)
+    return p
+
+
+def _update(p, drop=None, bo=None):
+    """The update in float64 from the rounded rows and operands that the kernel multiplies."""
+    x = p["x"].double().cpu()
+    mu = x.mean(-1, keepdim=True)
+    y = (x - mu) / torch.sqrt(((x - mu) ** 2).mean(-1, keepdim=True) + 1e-5) * p["gam"].double().cpu() + p["bet"].double().cpu()
+    y = y.to(BF).double()
+    B2, N, C, H, D = (p[k] for k in ("B2", "N", "C", "H", "D"))
+    q, k, v = (t.view(B2, N, H, D).transpose(1, 2) for t in (y @ p["qkv"].double().cpu().t()).split(C, -1))
+    s = (q * D ** -0.5) @ k.transpose(-1, -2)
+    if p["bias"] is not None:
+        s = s + p["bias"].double().cpu() / LOG2E
+    mask = p["mask"].double().cpu()
+    s = s.masked_fill(mask[:, None, None, :] == 0, -1e9)
+    o = (torch.softmax(s, -1) @ v).transpose(1, 2).reshape(B2, N, C)
+    upd = (torch.sigmoid(y @ p["wg"].double().cpu().t() + p["bg"].double().cpu()) * o) @ p["wo"].double().cpu().t()
+    upd = upd + (0 if bo is None else bo.double().cpu())
+    return upd * (1 if drop is None else drop.double().cpu())
+
+
+def _run(p, x, out, bo=None, drop=None, xtail=None):
+    from fastfold_amd import _lib
+    from fastfold_amd.model.fastnn import _fused as F_
+    from fastfold_amd.model.fastnn.kernel import layouts
+    dev, B2, N, C = x.device, p["B2"], p["N"], p["C"]
+    w = F_.pack_attention_block(p["qkv"], p["wg"], p["wo"], BF, dev)
+    bias = None if p["bias"] is None else layouts.tile_bias(p["bias"])
+    kb, flags = F_.key_bias(p["mask"], dev, B2=B2, N=N, mask_sb=N, mask_sn=1)
+    _lib.attention_block(out, x, p["gam"], p["bet"], w, p["bg"], bo, bias, kb, flags, B2=B2, N=N, C=C, D=p["D"],
+                         s_row=x.stride(0), s_tok=x.stride(1), bias_pitch=(N + 31) // 32, xtail=xtail, drop=drop)
+    torch.cuda.synchronize()
+
+
+def _stream(h, tail):
+    """The 24-bit values of an extended residual stream."""
+    return ((h.view(torch.int16).to(torch.int32) << 16) + (tail.to(torch.int32) << 8)).view(torch.float32)
+
+
+def _err(got, p, upd, live=slice(None)):
+    d = (got.double().cpu() - p["x"].double().cpu())[live] - upd[live]
+    return float(d.norm() / upd[live].norm())
+
+
+# Six roundings to bf16 in a chain (q or k, v, p, o, gated o, update), each by at most 2^-9 of a value.  The result is read at 24 bits:
+# its rounding to bf16 would be one of the stream, which is several times as large as the update.
+TOL = 6 * 2.0 ** -9
+
+
+# One tile per wave with its heads divided by four, two and not at all; several tiles per wave; ragged rows; more batch rows than
+# a multiple of eight.
+@pytest.mark.parametrize("C,D,N", [(128, 32, n) for n in (1, 32, 50, 64, 96, 128, 129, 160, 224, 256)]
+                         + [(64, 16, n) for n in (32, 77, 128, 160, 256, 288, 320, 500, 512)]
+                         + [(256, 32, n) for n in (5, 32, 64, 65, 96, 128)] + [(256, -32, n) for n in (32, 50, 96, 128)])
+def test_attention_block_against_float64(dev, C, D, N):
+    p = _case(dev, C, abs(D), 9, N, seed=C + N, transposed=N % 3 == 0, bias=C != 256 or D < 0)
+    out = torch.empty_like(p["x"])                            # keeps the strides
+    tail = torch.empty_like(out, dtype=torch.int8).zero_()
+    _run(p, p["x"], out, xtail=tail)
+    live = [0, 1] + list(range(3, 9))                         # all keys masked: what the reference averages over is arbitrary
+    assert _err(_stream(out, tail), p, _update(p), live) < TOL
+    # ... and the heads are zero here, so that the row stays as it was
+    assert torch.equal(out[2], p["x"][2])
+
+
+@pytest.mark.parametrize("C,D,N", [(128, 32, 96), (128, 32, 256), (64, 16, 320), (256, 32, 128)])
+def test_attention_block_residual_forms(dev, C, D, N):
+    """Output bias, dropout multipliers, in place, and the tail of an extended residual stream."""
+    p = _case(dev, C, D, 3, N, seed=N, bias=C != 256)
+    p["mask"][2] = 1
+    g = torch.Generator().manual_seed(1)
+    bo = torch.randn(C, generator=g).to(dev, BF)
+    drop = ((torch.rand(N, C, generator=g) > 0.25).float() / 0.75).to(dev, BF)
+    want = _update(p, drop, bo)
+    plain = torch.empty_like(p["x"])
+    _run(p, p["x"], plain, bo, drop)
+    x2, tail = p["x"].clone(), torch.zeros(p["x"].shape, dtype=torch.int8, device=dev)
+    _run(p, x2, x2, bo, drop, tail)
+    # half up against half to even: one bf16 step at most
+    assert float(((x2.float() - plain.float()).abs() / plain.float().abs().clamp_min(1e-3)).max()) <= 2.0 ** -7
+    assert _err(_stream(x2, tail), p, want) < TOL
+
+
+def test_attention_block_moving_reference(dev):
+    """Scores that rise far above those of the first tile: the second walk, with the reference moved tile by tile."""
+    p = _case(dev, 128, 32, 4, 256, seed=2)
+    p["mask"][:] = 1
+    rise = torch.arange(8, device=dev).repeat_interleave(32).float() * 80.0
+    p["bias"] = (p["bias"].float() + rise[None, None, :]).to(BF)
+    p["bias"][:, 100:140] = p["bias"][:, 100:140].flip(-1)    # ... and falling ones in the same tiles of queries
+    out = p["x"].clone()
+    tail = torch.zeros(out.shape, dtype=torch.int8, device=dev)
+    _run(p, out, out, xtail=tail)
+    assert _err(_stream(out, tail), p, _update(p)) < TOL
+
+
+def test_attention_block_refuses(dev):
+    p = _case(dev, 256, 32, 2, 129, seed=0)
+    with pytest.raises(RuntimeError, match="too long"):
+        _run(p, p["x"], torch.empty_like(p["x"]))
+    p = _case(dev, 128, 32, 2, 257, seed=0)
+    with pytest.raises(RuntimeError, match="too long"):
+        _run(p, p["x"], torch.empty_like(p["x"]))
+    p = _case(dev, 128, 32, 2, 64, seed=0, bias=False)
+    with pytest.raises(RuntimeError, match="pair bias"):
+        _run(p, p["x"], torch.empty_like(p["x"]))
