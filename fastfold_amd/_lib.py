@@ -426,6 +426,15 @@ def attention_block(out, x, gamma, beta, w, bg, bo, bias_t, keybias, tileflags, 
          dtype_tag(dtype if dtype is not None else x.dtype), stream_ptr())
 
 
+SIGNATURES["ffk_attention_heads"] = [_P] * 9 + [_L] * 7 + [_F, _I, _P]
+
+
+def attention_heads(o, x, gamma, beta, w, bg, bias_t, keybias, tileflags, *, B2, N, C, D, s_row, s_tok, bias_pitch, eps=1e-5):
+    """The gated outputs of an attention's heads from the rows of x (see include/ffk.h)."""
+    call("ffk_attention_heads", ptr(o), ptr(x), ptr(gamma), ptr(beta), ptr(w), ptr(bg), ptr(bias_t), ptr(keybias), ptr(tileflags),
+         B2, N, C, D, s_row, s_tok, bias_pitch, eps, dtype_tag(o.dtype), stream_ptr())
+
+
 def key_bias(keybias, tileflags, mask, *, B, N, mask_sb=0, mask_sn=1):
     call("ffk_key_bias", ptr(keybias), ptr(tileflags), ptr(mask), B, N, mask_sb, mask_sn,
          dtype_tag(mask.dtype) if mask is not None else FFK_F32, stream_ptr())

@@ -22,7 +22,9 @@
 //   64 channels in 4 heads:  N = 64 18.6 -> 11.1, 128 26.0 -> 15.0, 256 50.5 -> 32, 320 79 -> 77, 512 184 -> 171
 //   256 channels in 8 heads, rows of 128 tokens, no bias:  64 rows 33.5 -> 27.8, 256 69 -> 34, 416 109 -> 59, 1 024 266 -> 125
 //                            with a pair bias:  128 rows of 96 tokens 45 -> 29, of 128 tokens 51 -> 36
-// Longer rows do not fit: at 128 channels, k and v of more than 256 tokens go into LDS in two passes only (heads two by two, rows
+//   the same to the gated heads, output projection apart (k and v of four heads of 256 tokens fill the LDS: two workgroups to a row):
+//                            128 rows of 160 tokens 67 -> 49, 192 74 -> 53, 256 87 -> 72;  512 rows of 256 296 -> 228
+// From how many rows on: attention_block_rows in model/fastnn/_fused.py.  Longer rows do not fit: at 128 channels, k and v of more than 256 tokens go into LDS in two passes only (heads two by two, rows
 // normalised twice), which was built and is slower (288 tokens 122 us against 92, 416 235 against 189).
 #include "ffk_common.h"
 #include <type_traits>
@@ -176,25 +178,29 @@ template <int C, int NT_MAX> struct AbUpdate {
     }
 };
 
-// Geometry of the kernel for 64 and 128 channels: eight waves, 8 / NB of them to a block of 32 channels (one head of 32, two of 16),
-// each with every (8 / NB)-th tile of 32 tokens, at most TPW of them.
+// Geometry: eight waves, WB blocks of 32 channels (one head of 32, two of 16) to a workgroup, 8 / WB waves to a block, each with every
+// (8 / WB)-th tile of 32 tokens, at most TPW of them.  64 and 128 channels: all blocks.  256 channels: half of them, k and v of more
+// would not fit; the output projection, which needs all heads, is a launch of its own (HEADS: `out` takes the gated outputs).
 template <int C, int D, int TPW> struct AbGeo {
+    static constexpr bool HEADS = C == 256;
     static constexpr int KS = C / 16;               // K steps of a projection
     static constexpr int NB = C / 32;               // 32-channel blocks
+    static constexpr int WB = HEADS ? NB / 2 : NB;  // ... of a workgroup
     static constexpr int HPB = 32 / D;              // heads per block
-    static constexpr int WPB = 8 / NB;              // waves per block
+    static constexpr int WPB = 8 / WB;              // waves per block
     static constexpr int NT_MAX = WPB * TPW;
     static constexpr int XP = C * 2 + 16;           // pitch of the normalised rows (bytes)
-    static constexpr size_t smem(long NT) {         // rows, then k and v, then the gated outputs and the updates
-        const size_t rows = (size_t)NT * 32 * XP, kv = (size_t)NT * NB * 4096, o = (size_t)NT * NB * 2048;
-        return rows + o > kv ? rows + o : kv;
+    static constexpr int HP = WB * 64 + 16;         // HEADS: pitch of the gated outputs
+    static constexpr size_t smem(long NT) {         // rows, then k and v, then the gated outputs (and the updates)
+        const size_t rows = (size_t)NT * 32 * XP, kv = (size_t)NT * WB * 4096, end = HEADS ? 0 : rows + (size_t)NT * NB * 2048;
+        return rows > kv ? (rows > end ? rows : end) : (kv > end ? kv : end);
     }
 };
 
 template <int C, int D, int TPW>
 __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a) {
     typedef AbGeo<C, D, TPW> G;
-    constexpr int KS = G::KS, NB = G::NB, HPB = G::HPB, WPB = G::WPB, XP = G::XP;
+    constexpr int KS = G::KS, NB = G::NB, WB = G::WB, HPB = G::HPB, WPB = G::WPB, XP = G::XP, PARTS = NB / WB;
     constexpr float NEG_FLOOR = -1.0e4f;             // reference of a row that has met no key (see ffk_attention.hip)
     extern __shared__ __align__(16) unsigned char ab_smem[];
 
@@ -203,13 +209,15 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
     const int l32 = lane & 31, half = lane >> 5;
     const int NT = (a.N + 31) >> 5;
     // consecutive workgroup ids go to the eight XCDs in turn: each takes a contiguous eighth of the batch rows
-    const unsigned per_xcd = (unsigned)(a.B2 + 7) >> 3;
-    const unsigned b2 = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (b2 >= (unsigned)a.B2) return;                // whole workgroup
-    const int blk = wave % NB, t_first = wave / NB;  // block of hidden (at the end: output) channels, first tile of this wave
+    const unsigned per_xcd = (unsigned)(a.B2 * PARTS + 7) >> 3;
+    const unsigned item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (item >= (unsigned)a.B2 * PARTS) return;      // whole workgroup
+    const unsigned b2 = item / PARTS;
+    const int wb = wave % WB, t_first = wave / WB;   // block within the workgroup, first tile of this wave
+    const int blk = (int)(item % PARTS) * WB + wb;   // block of hidden (at the end: output) channels
     unsigned char* s_x = ab_smem;                    // [32 NT][XP]
-    T* s_k = reinterpret_cast<T*>(ab_smem);          // [NB][NT][2][64][8]
-    T* s_v = s_k + (size_t)NB * NT * 1024;           // the same
+    T* s_k = reinterpret_cast<T*>(ab_smem);          // [WB][NT][2][64][8]
+    T* s_v = s_k + (size_t)WB * NT * 1024;           // the same
     T* s_o = s_k;                                    // [NT][NB][2][64][8]
     const T* xrow = a.x + (long)b2 * a.s_row;
 
@@ -262,8 +270,8 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
         b[1] = MM::ld(p + 8);
     };
     auto attend = [&](int sub, const T* bp, const T* bp_next, const bf16x8& q0, const bf16x8& q1, f32x16& acc, float& inv) __attribute__((always_inline)) {
-        const T* kp = s_k + (size_t)blk * NT * 1024 + lane * 8;
-        const T* vp = s_v + (size_t)blk * NT * 1024 + lane * 8;
+        const T* kp = s_k + (size_t)wb * NT * 1024 + lane * 8;
+        const T* vp = s_v + (size_t)wb * NT * 1024 + lane * 8;
         f32x16 negm, s;
         float l_run;
         auto bias_req = [&](int kt, bf16x8 (&b)[2]) __attribute__((always_inline)) {
@@ -459,8 +467,8 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
 #pragma unroll
         for (int i = 0; i < TPW; ++i) {
             if (t_first + WPB * i < NT) {
-                T* d = s_k + ((size_t)blk * NT + t_first + WPB * i) * 1024 + lane * 8;
-                T* e = s_v + ((size_t)blk * NT + t_first + WPB * i) * 1024 + lane * 8;
+                T* d = s_k + ((size_t)wb * NT + t_first + WPB * i) * 1024 + lane * 8;
+                T* e = s_v + ((size_t)wb * NT + t_first + WPB * i) * 1024 + lane * 8;
                 *reinterpret_cast<bf16x8*>(d) = kf[i][0];
                 *reinterpret_cast<bf16x8*>(d + 512) = kf[i][1];
                 *reinterpret_cast<bf16x8*>(e) = vf[i][0];
@@ -495,6 +503,26 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
         }
     }
     lds_barrier();                               // nobody reads k and v any more
+
+    if constexpr (G::HEADS) {                        // gated outputs -> LDS -> their rows, WB * 64 bytes at a time
+        constexpr int LPR = WB * 4, RPI = 64 / LPR;
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) {
+            if (t_first + WPB * i < NT) {
+                unsigned char* p = ab_smem + ((t_first + WPB * i) * 32 + l32) * G::HP + wb * 64 + half * 8;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {        // channels 8 j + 4 half ..
+                    const u32x4 y = *reinterpret_cast<const u32x4*>(&of[i][j >> 1]);
+                    *reinterpret_cast<u32x2*>(p + j * 16) = u32x2{y[2 * (j & 1)], y[2 * (j & 1) + 1]};
+                }
+            }
+        }
+        lds_barrier();
+        T* orow = a.out + (long)b2 * a.N * C + (item % PARTS) * (WB * 32) + (lane % LPR) * 8;
+        for (int tok = wave * RPI + lane / LPR; tok < a.N; tok += 8 * RPI)
+            st16(orow + (long)tok * C, *reinterpret_cast<const Vec16<T>*>(ab_smem + tok * G::HP + (lane % LPR) * 16));
+        return;
+    }
 
     // ---- gated outputs to LDS; output projection: 32 channels of the wave's tiles ----
     request(wptr(4, blk));
@@ -548,20 +576,22 @@ __global__ __launch_bounds__(512, 2) void attention_block_wide_kernel(const AbAr
     const unsigned b2 = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (b2 >= (unsigned)a.B2) return;
     const T* xrow = a.x + (long)b2 * a.s_row;
-
-    ab_normalise<C, NT>(a, xrow, s_x, NT, wave, lane);
-    const unsigned char* xp = s_x + l32 * XP + half * 16;
     const T* wbase = a.w + (long)wave * KS * 512 + lane * 8;         // this head's block (output: this wave's channels)
     auto wptr = [&](int which) { return wbase + (long)which * 8 * KS * 512; };
-
-    // two weights at a time over all tokens: acc[0] = W0 y^T, acc[1] = W1 y^T or (V1) y W1^T
-    auto project2 = [&](const T* w0, const T* w1, auto v1, f32x16 (&acc)[2][NT]) __attribute__((always_inline)) {
-        bf16x8 f0[AHEAD], f1[AHEAD];
+    bf16x8 f0[AHEAD], f1[AHEAD];
+    auto request = [&](const T* w0, const T* w1) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i) {
             f0[i] = MM::ld(w0 + i * 512);
             f1[i] = MM::ld(w1 + i * 512);
         }
+    };
+    request(wptr(0), wptr(1));
+    ab_normalise<C, NT>(a, xrow, s_x, NT, wave, lane);
+    const unsigned char* xp = s_x + l32 * XP + half * 16;
+
+    // two weights at a time over all tokens, their first fragments requested: acc[0] = W0 y^T, acc[1] = W1 y^T or (V1) y W1^T
+    auto project2 = [&](const T* w0, const T* w1, auto v1, f32x16 (&acc)[2][NT]) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -588,6 +618,7 @@ __global__ __launch_bounds__(512, 2) void attention_block_wide_kernel(const AbAr
     {
         f32x16 acc[2][NT];
         project2(wptr(0), wptr(1), std::false_type(), acc);
+        request(wptr(3), wptr(2));
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
 #pragma unroll
@@ -736,7 +767,7 @@ template <int C, int D, int TPW> int ab_launch(const AbArgs& a, long NT, hipStre
     static FfkLdsReservation lds_reserved;
     const int rc = ffk_reserve_lds(lds_reserved, (const void*)attention_block_kernel<C, D, TPW>, G::smem(G::NT_MAX), "ffk_attention_block");
     if (rc != FFK_OK) return rc;
-    attention_block_kernel<C, D, TPW><<<dim3(8u * ffk_cdiv(a.B2, 8)), 512, G::smem(NT), st>>>(a);
+    attention_block_kernel<C, D, TPW><<<dim3(8u * ffk_cdiv((long)a.B2 * (G::NB / G::WB), 8)), 512, G::smem(NT), st>>>(a);
     return ffk_check_launch("ffk_attention_block");
 }
 template <int NT, bool BIAS> int aw_launch(const AbArgs& a, hipStream_t st) {
@@ -776,7 +807,7 @@ extern "C" int ffk_attention_block(void* out, const void* x, void* xtail, const 
     FFK_REQUIRE(NT <= (C == 256 ? 4 : C == 128 ? 8 : 16), FFK_ERR_UNSUPPORTED,
                 "ffk_attention_block: rows of %ld tokens are too long for %ld channels", (long)N, (long)C);
     FFK_REQUIRE(!bias_t || bias_pitch >= NT, FFK_ERR_SHAPE, "ffk_attention_block: bias rows of %ld tiles, %ld needed", (long)bias_pitch, NT);
-    AbArgs a = {(T*)out, (const T*)x, (int8_t*)xtail, (const T*)gamma, (const T*)beta, (const T*)w, (const T*)bg, (const T*)bo,
+    const AbArgs a = {(T*)out, (const T*)x, (int8_t*)xtail, (const T*)gamma, (const T*)beta, (const T*)w, (const T*)bg, (const T*)bo,
                 (const T*)bias_t, keybias, (const int*)tileflags, (const T*)drop, (long)s_row, (long)s_tok, (int)B2, (int)N,
                 (int)bias_pitch, 1.4426950408889634f / sqrtf((float)D), eps};
     hipStream_t st = (hipStream_t)stream;
@@ -794,5 +825,32 @@ extern "C" int ffk_attention_block(void* out, const void* x, void* xtail, const 
         case 2: return ab_launch<128, 32, 2>(a, NT, st);
         case 3: return ab_launch<128, 32, 3>(a, NT, st);
         default: return ab_launch<128, 32, 4>(a, NT, st);
+    }
+}
+
+extern "C" int ffk_attention_heads(void* o, const void* x, const void* gamma, const void* beta, const void* w, const void* bg,
+                                   const void* bias_t, const float* keybias, const int32_t* tileflags, int64_t B2, int64_t N,
+                                   int64_t C, int64_t D, int64_t s_row, int64_t s_tok, int64_t bias_pitch, float eps, int dtype,
+                                   void* stream) {
+    FFK_REQUIRE(o && x && gamma && beta && w && bg && bias_t && keybias && tileflags, FFK_ERR_NULL, "ffk_attention_heads: null pointer");
+    FFK_REQUIRE(dtype == FFK_BF16, FFK_ERR_DTYPE, "ffk_attention_heads: bf16 only (dtype tag %d)", dtype);
+    FFK_REQUIRE(C == 256 && D == 32, FFK_ERR_UNSUPPORTED, "ffk_attention_heads: built for 256 channels in heads of 32, got %ld / %ld", (long)C, (long)D);
+    FFK_REQUIRE(B2 > 0 && B2 < (1L << 30) - 64 && N > 0, FFK_ERR_SHAPE, "ffk_attention_heads: bad shape B2=%ld N=%ld", (long)B2, (long)N);
+    FFK_REQUIRE(N <= 256, FFK_ERR_UNSUPPORTED, "ffk_attention_heads: rows of %ld tokens are too long", (long)N);
+    FFK_REQUIRE(s_row % 8 == 0 && s_tok % 8 == 0, FFK_ERR_ALIGN, "ffk_attention_heads: row strides must be multiples of 8 elements");
+    FFK_REQUIRE(ffk_aligned16(o) && ffk_aligned16(x) && ffk_aligned16(gamma) && ffk_aligned16(beta) && ffk_aligned16(w) &&
+                    ffk_aligned16(bg) && ffk_aligned16(bias_t) && ffk_aligned16(keybias),
+                FFK_ERR_ALIGN, "ffk_attention_heads: buffers must be 16-byte aligned");
+    const long NT = (N + 31) / 32;
+    FFK_REQUIRE(bias_pitch >= NT, FFK_ERR_SHAPE, "ffk_attention_heads: bias rows of %ld tiles, %ld needed", (long)bias_pitch, NT);
+    const AbArgs a = {(T*)o, (const T*)x, nullptr, (const T*)gamma, (const T*)beta, (const T*)w, (const T*)bg, nullptr, (const T*)bias_t,
+                      keybias, (const int*)tileflags, nullptr, (long)s_row, (long)s_tok, (int)B2, (int)N, (int)bias_pitch,
+                      1.4426950408889634f / sqrtf((float)D), eps};
+    hipStream_t st = (hipStream_t)stream;
+    switch ((NT + 1) / 2) {
+        case 1: return ab_launch<256, 32, 1>(a, NT, st);
+        case 2: return ab_launch<256, 32, 2>(a, NT, st);
+        case 3: return ab_launch<256, 32, 3>(a, NT, st);
+        default: return ab_launch<256, 32, 4>(a, NT, st);
     }
 }

@@ -256,6 +256,15 @@ def attention_block_tokens(dtype, H, c, d_in, d_out):
     return {(128, 32): 256, (64, 16): 512, (256, 32): 128}.get((d_in, c), 0)
 
 
+def attention_block_rows(C, N, biased):
+    """Fewest batch rows from which ``ffk_attention_block`` and ``ffk_attention_heads`` are taken.  Their time does not depend on the
+    number of rows up to one per CU, and 256 channels keep a CU busy for long: us per sub-module, one kernel / launches of their own,
+    rows with a bias of N = 64: 8 rows 21 / 22; 96: 16 rows 27 / 25, 32 27 / 28; 128: 32 rows 35 / 31, 48 35 / 38; 160: 32 rows
+    37 / 37, 48 38 / 40; 192: 48 rows 47 / 46, 64 48 / 49; 256: 64 rows 60 / 57, 96 65 / 75; without one: 96: 32 rows 20 / 21, 128: 32
+    rows 27 / 24, 64 28 / 34.  The narrower kernels have as many rows as tokens and win at every size."""
+    return 0 if C < 256 or N <= 64 else N // 3 if biased else N // 4
+
+
 def pack_attention_block(qkv_w, gate_w, out_w, dtype, device):
     """The weights of a gated attention in the fragment order of ``ffk_attention_block``: [q, k, v, gate, out][C/32][C/16][64][8]."""
     C = gate_w.shape[0]
@@ -266,6 +275,8 @@ def pack_attention_block(qkv_w, gate_w, out_w, dtype, device):
     wo = out_w.detach().to(device=device, dtype=dtype).view(nb, 32, ks, 2, 2, 4)[:, tau]     # [ct][row][step][quad][half][4]
     return torch.cat([ws, wo.permute(0, 2, 4, 1, 3, 5).reshape(-1)]).contiguous()
 
+
+ATTENTION_HEADS_TOKENS = 256     # longest row of ffk_attention_heads
 
 # False: every attention runs as projection, core and output stage (tests compare the two)
 _ATTENTION_BLOCK = True
@@ -307,7 +318,8 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     # kernel, which writes q, k and the gate in accumulator order straight from its registers.
     acc_order = dt == torch.bfloat16 and C in (64, 128, 256) and N % 32 == 0
     # Short rows: one kernel from the rows of x to the updated rows.
-    if (_ATTENTION_BLOCK and acc_order and hasattr(w_pk, "block") and N <= attention_block_tokens(dt, H, head_dim, C, c_out)
+    enough = B2 >= attention_block_rows(C, N, bias_t is not None or bias_in_launch)
+    if (_ATTENTION_BLOCK and enough and acc_order and hasattr(w_pk, "block") and N <= attention_block_tokens(dt, H, head_dim, C, c_out)
             and ln is not None and resid is not None and resid.data_ptr() == x.data_ptr() and o_map is None
             and a_so % 16 == 0 and a_si % 16 == 0 and (C == 256 or bias_t is not None or bias_in_launch)
             and (drop is None or drop.shape[0] == N)):
@@ -329,12 +341,13 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     HC = H * head_dim if packed else H * 32
     if HC % 128 != 0 and not packed:
         raise RuntimeError("attention: n_head * 32 must be a multiple of 128 (got %d heads)" % H)
+    # Rows of 256 channels too long for that, with a pair bias: one kernel up to the gated heads, the output projection behind it.
+    heads = (_ATTENTION_BLOCK and enough and acc_order and hasattr(w_pk, "block") and C == 256 and head_dim == 32 and HC == C
+             and N <= ATTENTION_HEADS_TOKENS and ln is not None and bias_t is not None and not bias_in_launch)
     HT = HC // 32                                  # operand tiles per batch row and 32 tokens
     per_row = 5 * HT * NT * 1024 * es
     slab = B2 if budget is None else min(B2, max(2, (budget // per_row) // 2 * 2))
-    q_t = alloc((slab, HT, NT, 1024), dt, dev, zero)
-    k_t = alloc((slab, HT, NT, 1024), dt, dev, zero)
-    v_t = alloc((slab, HT, NT, 1024), dt, dev, zero)
+    q_t, k_t, v_t = (alloc((slab, HT, NT, 1024), dt, dev, zero) for _ in range(3)) if not heads else (None,) * 3
     # Where the update goes back into the tensor the gate is computed from (every attention of the Evoformer block),
     # the gate is not a tensor at all: the output stage computes sigmoid(Wg LN(x) + bg) from the rows of x it reads as
     # residual anyway and multiplies the heads' outputs by it on their way into the output projection
@@ -347,9 +360,9 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     # batch rows: a subset of the batch rows must give the bits of the full call.
     gate_in_out = (_GATE_IN_OUT_STAGE and drop is None and N >= _GATE_IN_OUT_MIN_N and C in _GATE_IN_OUT_WIDTHS and acc_order
                    and ln is not None and not packed and HC == C and c_out == C and resid is not None and o_map is None
-                   and resid.data_ptr() == x.data_ptr() and a_so % 16 == 0 and a_si % 16 == 0)
+                   and resid.data_ptr() == x.data_ptr() and a_so % 16 == 0 and a_si % 16 == 0 and not heads)
     gate = None
-    if not gate_in_out:
+    if not gate_in_out and not heads:
         gate = alloc((slab, HT, NT, 1024) if acc_order else (slab * N, HC), dt, dev)
     o = alloc((slab * N, HC), dt, dev)
     tpg = (HC + 127) // 128
@@ -400,11 +413,15 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
         # rows b0 * N ... of the map: a shifted base, and an inner extent that still covers the slab
         off, inner = (b0 * N * a_si, Ms) if a_inner == M else (b0 * a_so, N)
         o_off = b0 * N * o_si if a_inner == M else b0 * o_so
+        if heads:
+            w, bg = w_pk.block
+            _lib.attention_heads(o, x.data_ptr() + off * es, ln[0], ln[1], w, bg, bias_t, kb[b0:b0 + nb], flags[b0:b0 + nb], B2=nb,
+                                 N=N, C=C, D=head_dim, s_row=a_so if a_inner == N else N * a_si, s_tok=a_si, bias_pitch=NT)
         tiles = []
-        for buf, kind, scale in ((q_t, qk_kind, qscale), (k_t, qk_kind, 1.0), (v_t, FFK_TILE_V, 1.0)):
+        for buf, kind, scale in () if heads else ((q_t, qk_kind, qscale), (k_t, qk_kind, 1.0), (v_t, FFK_TILE_V, 1.0)):
             for t in range(tpg):
                 tiles.append(make_tile(buf.data_ptr() + t * 4 * NT * 1024 * es, kind=kind, scale=scale, **tkw))
-        for t in range(0 if gate_in_out else tpg):
+        for t in range(0 if gate_in_out or heads else tpg):
             if acc_order:
                 tiles.append(make_tile(gate.data_ptr() + t * 4 * NT * 1024 * es, kind=FFK_TILE_ACC,
                                        bias=gate_bias_pk.data_ptr() + t * 128 * es, act=FFK_ACT_SIGMOID, **tkw))
@@ -419,9 +436,10 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
             wp = w_pk.without_gate if (gate_in_out and bias_tile is not None) else w_pk
             _lib.fused_linear(x, wp, tiles[t0:t0 + per], M=Ms, K=C, a_inner=inner, a_so=a_so, a_si=a_si, ln=ln,
                               w_row_off=t0 * 128, a_off=off)
-        _lib.attention_fwd(o, q_t, k_t, v_t, bias_t, kb[b0:b0 + nb], flags[b0:b0 + nb], gate, B2=nb, H=H, Nq=N, Nk=N,
-                           gate_tiled=acc_order, bias_padded=bias_padded,
-                           D=head_dim if packed else 32, half_k=not packed and head_dim <= (16 if acc_order else 8))
+        if not heads:
+            _lib.attention_fwd(o, q_t, k_t, v_t, bias_t, kb[b0:b0 + nb], flags[b0:b0 + nb], gate, B2=nb, H=H, Nq=N, Nk=N,
+                               gate_tiled=acc_order, bias_padded=bias_padded,
+                               D=head_dim if packed else 32, half_k=not packed and head_dim <= (16 if acc_order else 8))
         if gate_in_out:
             # packed rows of w_pk: q, k, v, gate blocks of HC rows each; o holds the slab's rows in logical order
             _lib.gated_out_fused(out.data_ptr() + o_off * es, x.data_ptr() + off * es, ln[0], ln[1],

@@ -461,6 +461,14 @@ int ffk_attention_block(void* out, const void* x, void* xtail, const void* gamma
                         const void* drop, int64_t B2, int64_t N, int64_t C, int64_t D, int64_t s_row, int64_t s_tok,
                         int64_t bias_pitch, float eps, int dtype, void* stream);
 
+/* The same up to the gated outputs of the heads, for rows whose operands leave no room for the output projection (bf16, C = 256 in
+ * heads of D = 32, with a pair bias, N at most 256):
+ *     o[b * N + n] = sigmoid(Wg y + bg) * attention(Wq y, Wk y, Wv y),    [B2 * N, C] contiguous
+ * Arguments as above; of w the first four weights are read.  x and o must not overlap. */
+int ffk_attention_heads(void* o, const void* x, const void* gamma, const void* beta, const void* w, const void* bg,
+                        const void* bias_t, const float* keybias, const int32_t* tileflags, int64_t B2, int64_t N, int64_t C,
+                        int64_t D, int64_t s_row, int64_t s_tok, int64_t bias_pitch, float eps, int dtype, void* stream);
+
 /* Global column attention core of the extra-MSA stack: one query per residue column (the masked mean
  * of the normalised rows), one key / value head of width D shared by the H query heads.
  *     x_s = LayerNorm(m[s, j, :]; gamma, beta, ln_eps)
@@ -610,7 +618,7 @@ enum {
     FFK_OP_FILL_ZERO = 9, FFK_OP_ATTENTION_FWD_LSE = 10, FFK_OP_ATTENTION_BWD_ROWS = 11, FFK_OP_TRANSPOSE_BATCHED = 12,
     FFK_OP_WEIGHT_GRAD = 13, FFK_OP_LAYERNORM_BWD_ROWS = 14, FFK_OP_SCALE_ROWS = 15, FFK_OP_ATT_GATE_BWD = 16,
     FFK_OP_TRIMUL_GATE_BWD = 17, FFK_OP_GLU_BWD = 18, FFK_OP_BIAS_COLS = 19, FFK_OP_SLICE_SUM = 20,
-    FFK_OP_ATTENTION_BLOCK = 21, FFK_OP_COUNT = 22
+    FFK_OP_ATTENTION_BLOCK = 21, FFK_OP_ATTENTION_HEADS = 22, FFK_OP_COUNT = 23
 };
 int ffk_run_plan(const void* plan, int64_t bytes, const uint64_t* bases, int64_t n_bases, void* stream);
 

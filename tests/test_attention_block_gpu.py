@@ -32,8 +32,8 @@ def _case(dev, C, D, B2, N, seed, transposed=False, bias=True):
     return p
 
 
-def _update(p, drop=None, bo=None):
-    """The update in float64 from the rounded rows and operands that the kernel multiplies."""
+def _heads(p):
+    """The gated heads in float64 from the rounded rows and operands that the kernel multiplies."""
     x = p["x"].double().cpu()
     mu = x.mean(-1, keepdim=True)
     y = (x - mu) / torch.sqrt(((x - mu) ** 2).mean(-1, keepdim=True) + 1e-5) * p["gam"].double().cpu() + p["bet"].double().cpu()
@@ -46,7 +46,11 @@ def _update(p, drop=None, bo=None):
     mask = p["mask"].double().cpu()
     s = s.masked_fill(mask[:, None, None, :] == 0, -1e9)
     o = (torch.softmax(s, -1) @ v).transpose(1, 2).reshape(B2, N, C)
-    upd = (torch.sigmoid(y @ p["wg"].double().cpu().t() + p["bg"].double().cpu()) * o) @ p["wo"].double().cpu().t()
+    return torch.sigmoid(y @ p["wg"].double().cpu().t() + p["bg"].double().cpu()) * o
+
+
+def _update(p, drop=None, bo=None):
+    upd = _heads(p) @ p["wo"].double().cpu().t()
     upd = upd + (0 if bo is None else bo.double().cpu())
     return upd * (1 if drop is None else drop.double().cpu())
 
@@ -124,6 +128,24 @@ def test_attention_block_moving_reference(dev):
     tail = torch.zeros(out.shape, dtype=torch.int8, device=dev)
     _run(p, out, out, xtail=tail)
     assert _err(_stream(out, tail), p, _update(p)) < TOL
+
+
+@pytest.mark.parametrize("N", [32, 100, 129, 160, 192, 225, 256])
+def test_attention_heads_against_float64(dev, N):
+    from fastfold_amd import _lib
+    from fastfold_amd.model.fastnn import _fused as F_
+    from fastfold_amd.model.fastnn.kernel import layouts
+    p = _case(dev, 256, 32, 5, N, seed=N, transposed=N % 2 == 1)
+    kb, flags = F_.key_bias(p["mask"], dev, B2=5, N=N, mask_sb=N, mask_sn=1)
+    o = torch.full((5, N, 256), float("nan"), device=dev, dtype=BF)
+    _lib.attention_heads(o, p["x"], p["gam"], p["bet"], F_.pack_attention_block(p["qkv"], p["wg"], p["wo"], BF, dev), p["bg"],
+                         layouts.tile_bias(p["bias"]), kb, flags, B2=5, N=N, C=256, D=32, s_row=p["x"].stride(0),
+                         s_tok=p["x"].stride(1), bias_pitch=(N + 31) // 32)
+    torch.cuda.synchronize()
+    want = _heads(p)
+    live = [0, 1, 3, 4]
+    assert float((o.double().cpu() - want)[live].norm() / want[live].norm()) < TOL
+    assert float(o[2].abs().max()) == 0.0                     # no key at all
 
 
 def test_attention_block_refuses(dev):
