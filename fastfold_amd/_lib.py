@@ -406,6 +406,15 @@ def transition_fused(out, x, gamma, beta, w1, b1, w2, b2, *, M, C, hidden, eps=1
          hidden, eps, dtype_tag(x.dtype), stream_ptr())
 
 
+SIGNATURES["ffk_transition_block"] = [_P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _L, _L, _F, _I, _P]
+
+
+def transition_block(out, x, gamma, beta, w1, b1, w2, b2, *, M, C, hidden, eps=1e-5, xtail=None, dtype=None):
+    """As ``transition_fused`` with the weights in fragment order (see include/ffk.h)."""
+    call("ffk_transition_block", ptr(out), ptr(x), ptr(xtail), ptr(gamma), ptr(beta), ptr(w1), ptr(b1), ptr(w2), ptr(b2), M, C,
+         hidden, eps, dtype_tag(x.dtype if dtype is None else dtype), stream_ptr())
+
+
 SIGNATURES["ffk_gated_out_fused"] = [_P] * 10 + [_L, _L, _L, _L, _L, _F, _I, _P]
 
 

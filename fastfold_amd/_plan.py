@@ -27,7 +27,7 @@ OPS = ["ffk_fused_linear", "ffk_bgemm_nt", "ffk_attention_fwd", "ffk_pair_bias",
        "ffk_gated_out_fused", "ffk_global_attention_core", "ffk_layernorm_fwd", "ffk_fill_zero", "ffk_attention_fwd_lse",
        "ffk_attention_bwd_rows", "ffk_transpose_batched", "ffk_weight_grad", "ffk_layernorm_bwd_rows", "ffk_scale_rows",
        "ffk_att_gate_bwd", "ffk_trimul_gate_bwd", "ffk_glu_bwd", "ffk_bias_cols", "ffk_slice_sum",
-       "ffk_attention_block", "ffk_attention_heads"]   # order of FFK_OP_*
+       "ffk_attention_block", "ffk_attention_heads", "ffk_transition_block"]   # order of FFK_OP_*
 _CODE = {name: i for i, name in enumerate(OPS)}
 _MAX_PLANS = 16               # per module: shapes in use at a time
 _ALIGN = 512                  # of scratch buffers, as torch's allocator aligns its blocks

@@ -26,156 +26,20 @@
 //                            128 rows of 160 tokens 67 -> 49, 192 74 -> 53, 256 87 -> 72;  512 rows of 256 296 -> 228
 // From how many rows on: attention_block_rows in model/fastnn/_fused.py.  Longer rows do not fit: at 128 channels, k and v of more than 256 tokens go into LDS in two passes only (heads two by two, rows
 // normalised twice), which was built and is slower (288 tokens 122 us against 92, 416 235 against 189).
-#include "ffk_common.h"
+#include "ffk_rowblock.h"
 #include <type_traits>
 
 namespace {
 
-typedef bf16_t T;
-typedef Mma<T> MM;
-
-struct AbArgs {
-    T* out;
-    const T* x;
-    int8_t* xtail;
-    const T *gamma, *beta;
+struct AbArgs : RbRows {
     const T* w;              // [5][C / 32][C / 16][64][8]: q, k, v, gate, output projection
     const T *bg, *bo;
     const T* bias_t;         // [H][NT][bias_pitch] key x query tiles
     const float* keybias;    // [B2][32 NT]
     const int* flags;        // [B2][NT]
-    const T* drop;           // [N][C] multipliers of the update, or nullptr
-    long s_row, s_tok;
-    int B2, N, bias_pitch;
-    float qscale, eps;
-};
-
-// The lane number anew, so that the addresses made from it are not kept in registers from one end of a kernel to the other.
-__device__ __forceinline__ int ab_lane(int lane) {
-    asm volatile("" : "+v"(lane));
-    return lane;
-}
-// Computed here: the compiler would otherwise move the packing to the value's use and keep the unpacked numbers in twice the registers.
-__device__ __forceinline__ void ab_pin(bf16x8& f) { asm volatile("" : "+v"(*reinterpret_cast<u32x4*>(&f))); }
-
-__device__ __forceinline__ bf16x8 ab_pack8(const f32x16& a, int v0, float scale) {
-    bf16x8 r;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) r[t] = (T)(a[v0 + t] * scale);
-    return r;
-}
-
-// What the rows take: eight waves, C / 8 lanes to a row, so that a request of a wave is 1 KB of whole rows.
-template <int C, int NT_MAX> struct AbRows {
-    static constexpr int LPR = C / 8, RPI = 64 / LPR, NI = NT_MAX * 32 / (8 * RPI), XP = C * 2 + 16;
-    // rows i of all waves lie before row 32 NT, or none (half of them: 64 channels and an odd NT)
-    static __device__ __forceinline__ bool past(int i, int NT) { return i * 8 * RPI >= NT * 32; }
-    static __device__ __forceinline__ int row(int i, int wave, int lane) { return (i * 8 + wave) * RPI + lane / LPR; }
-};
-
-// Rows of the batch row -> LayerNorm -> LDS (row-major, 16 bytes of padding); rows past the end repeat the last one.
-template <int C, int NT_MAX>
-__device__ __forceinline__ void ab_normalise(const AbArgs& a, const T* xrow, unsigned char* s_x, int NT, int wave, int lane) {
-    typedef AbRows<C, NT_MAX> R;
-    const int c8 = lane % R::LPR;
-    const Vec16<T> g = ld16(a.gamma + c8 * 8), b = ld16(a.beta + c8 * 8);
-    Vec16<T> r[R::NI];
-#pragma unroll
-    for (int i = 0; i < R::NI; ++i) {
-        if (R::past(i, NT)) break;
-        const int tok = R::row(i, wave, lane);
-        r[i] = ld16(xrow + (long)(tok < a.N ? tok : a.N - 1) * a.s_tok + c8 * 8);
-    }
-#pragma unroll
-    for (int i = 0; i < R::NI; ++i) {
-        if (R::past(i, NT)) break;
-        float f[8], s = 0.0f, q = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            f[e] = (float)r[i].e[e];
-            s += f[e];
-        }
-        const float mu = group_sum(s, R::LPR) * (1.0f / C);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            f[e] -= mu;
-            q = __builtin_fmaf(f[e], f[e], q);
-        }
-        const float rs = rsqrtf(group_sum(q, R::LPR) * (1.0f / C) + a.eps);
-        bf16x8 y;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) y[e] = (T)__builtin_fmaf(f[e] * rs, (float)g.e[e], (float)b.e[e]);
-        const int row = R::row(i, wave, lane);
-        if (row < NT * 32) *reinterpret_cast<bf16x8*>(s_x + row * R::XP + c8 * 16) = y;
-    }
-}
-
-// The update of a 32 x 32 block (lane: token l32, channels 16 half ..), rounded, to its place in the rows of updates in LDS.
-__device__ __forceinline__ void ab_put(unsigned char* p, f32x16& acc, const T* bo) {
-    if (bo) {
-        const Vec16<T> b0 = ld16(bo), b1 = ld16(bo + 8);
-#pragma unroll
-        for (int v = 0; v < 8; ++v) {
-            acc[v] += (float)b0.e[v];
-            acc[8 + v] += (float)b1.e[v];
-        }
-    }
-    *reinterpret_cast<bf16x8*>(p) = ab_pack8(acc, 0, 1.0f);
-    *reinterpret_cast<bf16x8*>(p + 16) = ab_pack8(acc, 8, 1.0f);
-}
-
-// out = x + update (times its dropout multipliers).  The rows are requested (`fetch`) before the barrier that completes the updates:
-// a lane with a token's 16 channels, as the accumulators have them, would touch 32 lines per request and the epilogue take twice as long.
-template <int C, int NT_MAX> struct AbUpdate {
-    typedef AbRows<C, NT_MAX> R;
-    u32x4 h[R::NI];
-    u32x2 t[R::NI];
-    __device__ __forceinline__ void fetch(const AbArgs& a, long row_off, int NT, int wave, int lane) {
-#pragma unroll
-        for (int i = 0; i < R::NI; ++i) {
-            if (R::past(i, NT)) break;
-            const int tok = R::row(i, wave, lane);
-            const long off = row_off + (long)(tok < a.N ? tok : a.N - 1) * a.s_tok + (lane % R::LPR) * 8;
-            h[i] = *reinterpret_cast<const u32x4*>(a.x + off);
-            if (a.xtail) t[i] = *reinterpret_cast<const u32x2*>(a.xtail + off);
-        }
-    }
-    __device__ __forceinline__ void store(const AbArgs& a, const unsigned char* s_u, long row_off, int NT, int wave, int lane) const {
-        const int c8 = lane % R::LPR;
-#pragma unroll
-        for (int i = 0; i < R::NI; ++i) {
-            if (R::past(i, NT)) break;
-            const int tok = R::row(i, wave, lane);
-            if (tok >= a.N) continue;
-            const bf16x8 u = *reinterpret_cast<const bf16x8*>(s_u + tok * R::XP + c8 * 16);
-            float upd[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) upd[e] = (float)u[e];
-            if (a.drop) {
-                const Vec16<T> d = ld16(a.drop + (long)tok * C + c8 * 8);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) upd[e] = (float)(T)(upd[e] * (float)d.e[e]);
-            }
-            const long off = row_off + (long)tok * a.s_tok + c8 * 8;
-            u32x4 hn;
-            if (a.xtail) {
-                float f[8];
-                u32x2 tn;
-                xs_decode8(h[i], t[i][0], t[i][1], f);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) f[e] += upd[e];
-                xs_encode8(f, hn, tn);
-                *reinterpret_cast<u32x2*>(a.xtail + off) = tn;
-            } else {
-                const bf16x8 x = __builtin_bit_cast(bf16x8, h[i]);
-                bf16x8 y;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) y[e] = (T)(upd[e] + (float)x[e]);
-                hn = __builtin_bit_cast(u32x4, y);
-            }
-            *reinterpret_cast<u32x4*>(a.out + off) = hn;
-        }
-    }
+    long s_row;
+    int B2, bias_pitch;
+    float qscale;
 };
 
 // Geometry: eight waves, WB blocks of 32 channels (one head of 32, two of 16) to a workgroup, 8 / WB waves to a block, each with every
@@ -207,7 +71,7 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
-    const int NT = (a.N + 31) >> 5;
+    const int NT = (a.n + 31) >> 5;
     // consecutive workgroup ids go to the eight XCDs in turn: each takes a contiguous eighth of the batch rows
     const unsigned per_xcd = (unsigned)(a.B2 * PARTS + 7) >> 3;
     const unsigned item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
@@ -419,7 +283,7 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
 
     bf16x8 of[TPW][2];                       // gate, then gated outputs
     request(wptr(1, blk));
-    ab_normalise<C, G::NT_MAX>(a, xrow, s_x, NT, wave, lane);
+    rb_normalise<C, G::NT_MAX>(a, xrow, s_x, NT, wave, lane);
     lds_barrier();
     // ---- projections of this wave's tiles ----
     bf16x8 qf[TPW][2];
@@ -431,24 +295,24 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
         for (int i = 0; i < TPW; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                kf[i][j] = ab_pack8(acc[i], 8 * j, 1.0f);
-                ab_pin(kf[i][j]);
+                kf[i][j] = rb_pack8(acc[i], 8 * j, 1.0f);
+                rb_pin(kf[i][j]);
             }
         project(std::true_type(), wptr(0, blk), acc);
 #pragma unroll
         for (int i = 0; i < TPW; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                vf[i][j] = ab_pack8(acc[i], 8 * j, 1.0f);
-                ab_pin(vf[i][j]);
+                vf[i][j] = rb_pack8(acc[i], 8 * j, 1.0f);
+                rb_pin(vf[i][j]);
             }
         project(std::false_type(), wptr(3, blk), acc);
 #pragma unroll
         for (int i = 0; i < TPW; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                qf[i][j] = ab_pack8(acc[i], 8 * j, a.qscale);
-                ab_pin(qf[i][j]);
+                qf[i][j] = rb_pack8(acc[i], 8 * j, a.qscale);
+                rb_pin(qf[i][j]);
             }
         bf16x4 bg[4];
 #pragma unroll
@@ -461,7 +325,7 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
             for (int j = 0; j < 2; ++j) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) of[i][j][e] = (T)sigmoid_f(acc[i][8 * j + e] + (float)bg[2 * j + (e >> 2)][e & 3]);
-                ab_pin(of[i][j]);
+                rb_pin(of[i][j]);
             }
         lds_barrier();                           // nobody reads the rows any more
 #pragma unroll
@@ -497,7 +361,7 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
                     if (D == 16 && j != sub) continue;
 #pragma unroll
                     for (int e = 0; e < 8; ++e) of[i][j][e] = (T)(acc[8 * j + e] * inv * (float)of[i][j][e]);
-                    ab_pin(of[i][j]);
+                    rb_pin(of[i][j]);
                 }
             }
         }
@@ -518,8 +382,8 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
             }
         }
         lds_barrier();
-        T* orow = a.out + (long)b2 * a.N * C + (item % PARTS) * (WB * 32) + (lane % LPR) * 8;
-        for (int tok = wave * RPI + lane / LPR; tok < a.N; tok += 8 * RPI)
+        T* orow = a.out + (long)b2 * a.n * C + (item % PARTS) * (WB * 32) + (lane % LPR) * 8;
+        for (int tok = wave * RPI + lane / LPR; tok < a.n; tok += 8 * RPI)
             st16(orow + (long)tok * C, *reinterpret_cast<const Vec16<T>*>(ab_smem + tok * G::HP + (lane % LPR) * 16));
         return;
     }
@@ -535,8 +399,8 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
         }
     }
     unsigned char* s_u = ab_smem + (size_t)NT * NB * 2048;         // [32 NT][XP]
-    AbUpdate<C, G::NT_MAX> rows;
-    rows.fetch(a, (long)b2 * a.s_row, NT, wave, ab_lane(lane));
+    RbUpdate<C, G::NT_MAX> rows;
+    rows.fetch(a, (long)b2 * a.s_row, NT, wave, rb_lane(lane));
     lds_barrier();
     const T* bo = a.bo ? a.bo + blk * 32 + 16 * half : nullptr;
     f32x16 acc[TPW];
@@ -550,9 +414,9 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
         for (int i = 0; i < TPW; ++i) MM::mma(acc[i], w[f], MM::ld(s_o + ((size_t)tile(i) * KS + f) * 512 + lane * 8));
 #pragma unroll
     for (int i = 0; i < TPW; ++i)                    // past the end: the last tile's update once more
-        ab_put(s_u + (tile(i) * 32 + l32) * XP + blk * 64 + half * 32, acc[i], bo);
+        rb_put(s_u + (tile(i) * 32 + l32) * XP + blk * 64 + half * 32, acc[i], bo);
     lds_barrier();
-    rows.store(a, s_u, (long)b2 * a.s_row, NT, wave, ab_lane(lane));
+    rows.store(a, s_u, (long)b2 * a.s_row, NT, wave, rb_lane(lane));
 }
 
 // 256 channels in eight heads, rows of at most 128 tokens: a wave owns a head, its q, k, v and gate of all NT token tiles stay in its
@@ -587,7 +451,7 @@ __global__ __launch_bounds__(512, 2) void attention_block_wide_kernel(const AbAr
         }
     };
     request(wptr(0), wptr(1));
-    ab_normalise<C, NT>(a, xrow, s_x, NT, wave, lane);
+    rb_normalise<C, NT>(a, xrow, s_x, NT, wave, lane);
     const unsigned char* xp = s_x + l32 * XP + half * 16;
 
     // two weights at a time over all tokens, their first fragments requested: acc[0] = W0 y^T, acc[1] = W1 y^T or (V1) y W1^T
@@ -623,10 +487,10 @@ __global__ __launch_bounds__(512, 2) void attention_block_wide_kernel(const AbAr
         for (int t = 0; t < NT; ++t) {
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                qf[t][i] = ab_pack8(acc[0][t], 8 * i, a.qscale);
-                kf[t][i] = ab_pack8(acc[1][t], 8 * i, 1.0f);
-                ab_pin(qf[t][i]);
-                ab_pin(kf[t][i]);
+                qf[t][i] = rb_pack8(acc[0][t], 8 * i, a.qscale);
+                kf[t][i] = rb_pack8(acc[1][t], 8 * i, 1.0f);
+                rb_pin(qf[t][i]);
+                rb_pin(kf[t][i]);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -639,11 +503,11 @@ __global__ __launch_bounds__(512, 2) void attention_block_wide_kernel(const AbAr
         for (int t = 0; t < NT; ++t) {
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                vf[t][i] = ab_pack8(acc[1][t], 8 * i, 1.0f);
+                vf[t][i] = rb_pack8(acc[1][t], 8 * i, 1.0f);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) gf[t][i][e] = (T)sigmoid_f(acc[0][t][8 * i + e] + (float)bg[2 * i + (e >> 2)][e & 3]);
-                ab_pin(vf[t][i]);
-                ab_pin(gf[t][i]);
+                rb_pin(vf[t][i]);
+                rb_pin(gf[t][i]);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -739,8 +603,8 @@ __global__ __launch_bounds__(512, 2) void attention_block_wide_kernel(const AbAr
     bf16x8 w[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) w[i] = MM::ld(wo + i * 512);
-    AbUpdate<C, NT> rows;
-    rows.fetch(a, (long)b2 * a.s_row, NT, wave, ab_lane(lane));
+    RbUpdate<C, NT> rows;
+    rows.fetch(a, (long)b2 * a.s_row, NT, wave, rb_lane(lane));
     lds_barrier();
     f32x16 acc[NT];
 #pragma unroll
@@ -757,9 +621,9 @@ __global__ __launch_bounds__(512, 2) void attention_block_wide_kernel(const AbAr
     }
 #pragma unroll
     for (int t = 0; t < NT; ++t)                     // the normalised rows are not read any more
-        ab_put(s_x + (t * 32 + l32) * XP + wave * 64 + half * 32, acc[t], a.bo ? a.bo + wave * 32 + 16 * half : nullptr);
+        rb_put(s_x + (t * 32 + l32) * XP + wave * 64 + half * 32, acc[t], a.bo ? a.bo + wave * 32 + 16 * half : nullptr);
     lds_barrier();
-    rows.store(a, s_x, (long)b2 * a.s_row, NT, wave, ab_lane(lane));
+    rows.store(a, s_x, (long)b2 * a.s_row, NT, wave, rb_lane(lane));
 }
 
 template <int C, int D, int TPW> int ab_launch(const AbArgs& a, long NT, hipStream_t st) {
@@ -807,9 +671,9 @@ extern "C" int ffk_attention_block(void* out, const void* x, void* xtail, const 
     FFK_REQUIRE(NT <= (C == 256 ? 4 : C == 128 ? 8 : 16), FFK_ERR_UNSUPPORTED,
                 "ffk_attention_block: rows of %ld tokens are too long for %ld channels", (long)N, (long)C);
     FFK_REQUIRE(!bias_t || bias_pitch >= NT, FFK_ERR_SHAPE, "ffk_attention_block: bias rows of %ld tiles, %ld needed", (long)bias_pitch, NT);
-    const AbArgs a = {(T*)out, (const T*)x, (int8_t*)xtail, (const T*)gamma, (const T*)beta, (const T*)w, (const T*)bg, (const T*)bo,
-                (const T*)bias_t, keybias, (const int*)tileflags, (const T*)drop, (long)s_row, (long)s_tok, (int)B2, (int)N,
-                (int)bias_pitch, 1.4426950408889634f / sqrtf((float)D), eps};
+    const AbArgs a = {{(T*)out, (const T*)x, (int8_t*)xtail, (const T*)gamma, (const T*)beta, (const T*)drop, (long)s_tok, (int)N, eps},
+                      (const T*)w, (const T*)bg, (const T*)bo, (const T*)bias_t, keybias, (const int*)tileflags, (long)s_row, (int)B2,
+                      (int)bias_pitch, 1.4426950408889634f / sqrtf((float)D)};
     hipStream_t st = (hipStream_t)stream;
     if (C == 256) return bias_t ? aw_launch_nt<true>(a, NT, st) : aw_launch_nt<false>(a, NT, st);
     if (C == 64) {
@@ -843,9 +707,9 @@ extern "C" int ffk_attention_heads(void* o, const void* x, const void* gamma, co
                 FFK_ERR_ALIGN, "ffk_attention_heads: buffers must be 16-byte aligned");
     const long NT = (N + 31) / 32;
     FFK_REQUIRE(bias_pitch >= NT, FFK_ERR_SHAPE, "ffk_attention_heads: bias rows of %ld tiles, %ld needed", (long)bias_pitch, NT);
-    const AbArgs a = {(T*)o, (const T*)x, nullptr, (const T*)gamma, (const T*)beta, (const T*)w, (const T*)bg, nullptr, (const T*)bias_t,
-                      keybias, (const int*)tileflags, nullptr, (long)s_row, (long)s_tok, (int)B2, (int)N, (int)bias_pitch,
-                      1.4426950408889634f / sqrtf((float)D), eps};
+    const AbArgs a = {{(T*)o, (const T*)x, nullptr, (const T*)gamma, (const T*)beta, nullptr, (long)s_tok, (int)N, eps},
+                      (const T*)w, (const T*)bg, nullptr, (const T*)bias_t, keybias, (const int*)tileflags, (long)s_row, (int)B2,
+                      (int)bias_pitch, 1.4426950408889634f / sqrtf((float)D)};
     hipStream_t st = (hipStream_t)stream;
     switch ((NT + 1) / 2) {
         case 1: return ab_launch<256, 32, 1>(a, NT, st);

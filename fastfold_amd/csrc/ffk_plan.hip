@@ -73,6 +73,7 @@ const OpEntry OPS[] = {
     args_op<ffk_slice_sum>(),
     args_op<ffk_attention_block>(),
     args_op<ffk_attention_heads>(),
+    args_op<ffk_transition_block>(),
 };
 constexpr int N_OPS = (int)(sizeof(OPS) / sizeof(OPS[0]));
 static_assert(N_OPS == FFK_OP_COUNT, "one entry per operation code");

@@ -210,12 +210,23 @@ def xtail_ptr(xtail, off=0):
 _FUSED_TRANSITION = True
 
 
-def transition(x, out, *, ln, w1_pk, b1_pk, w2, b2, hidden, budget, xtail=None):
-    """out = x + W2 relu(W1 LN(x) + b1) + b2 over rows of x [M, C]; out may alias x.  ``xtail`` (here and in the
+
+
+def transition_block_rows(C):
+    """Most rows ``ffk_transition_block`` is taken for (timings of both sides in csrc/ffk_transition_block.hip)."""
+    return 16384 if C == 128 else 1 << 36
+
+
+def transition(x, out, *, ln, w1_pk, b1_pk, w2, b2, hidden, budget, xtail=None, w_block=None):
+    """out = x + W2 relu(W1 LN(x) + b1) + b2 over rows of x [M, C]; out may alias x.  ``w_block``: the weights as
+    ``pack_transition_block`` lays them out, or None.  ``xtail`` (here and in the
     other sub-modules): int8 tensor of x's shape holding the tail bytes of x / out as an extended residual stream."""
     M, C = x.shape
     dt, dev = x.dtype, x.device
     es = es_of(dt)
+    if w_block is not None and ln is not None and _FUSED_TRANSITION and M <= transition_block_rows(C):
+        _lib.transition_block(out, x, ln[0], ln[1], w_block[0], b1_pk, w_block[1], b2, M=M, C=C, hidden=hidden, xtail=xtail)
+        return out
     if dt == torch.bfloat16 and C in (128, 256) and hidden == 4 * C and ln is not None and _FUSED_TRANSITION:
         # both layers in one kernel, hidden activation kept on chip
         _lib.transition_fused(out, x, ln[0], ln[1], w1_pk, b1_pk, w2, b2, M=M, C=C, hidden=hidden, xtail=xtail)
@@ -267,16 +278,34 @@ def attention_block_rows(C, N, biased):
 
 def pack_attention_block(qkv_w, gate_w, out_w, dtype, device):
     """The weights of a gated attention in the fragment order of ``ffk_attention_block``: [q, k, v, gate, out][C/32][C/16][64][8]."""
-    C = gate_w.shape[0]
-    nb, ks = C // 32, C // 16
-    ws = torch.cat([qkv_w.detach(), gate_w.detach()], 0).to(device=device, dtype=dtype)
-    ws = ws.view(4, nb, 32, ks, 2, 8).permute(0, 1, 3, 4, 2, 5).reshape(-1)          # lane = 32 * (channel half) + row
+    return torch.cat([pack_fragments(torch.cat([qkv_w.detach(), gate_w.detach()], 0), dtype, device),
+                      pack_fragments_of_accumulators(out_w, dtype, device)]).contiguous()
+
+
+def pack_fragments(w, dtype, device):
+    """[n, K] -> [n/32][K/16][64][8]: what each lane of a wave gives to the matrix instructions that multiply by 32 rows of w."""
+    w = w.detach().to(device=device, dtype=dtype)
+    return w.view(w.shape[0] // 32, 32, w.shape[1] // 16, 2, 8).permute(0, 2, 3, 1, 4).reshape(-1)      # lane = 32 * (half) + row
+
+
+def pack_fragments_of_accumulators(w, dtype, device):
+    """The same for a weight that multiplies accumulators as they stand: columns in their order, and rows so that a lane's results are
+    16 consecutive channels."""
+    w = w.detach().to(device=device, dtype=dtype)
     tau = torch.tensor([((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3) for i in range(32)], device=device)
-    wo = out_w.detach().to(device=device, dtype=dtype).view(nb, 32, ks, 2, 2, 4)[:, tau]     # [ct][row][step][quad][half][4]
-    return torch.cat([ws, wo.permute(0, 2, 4, 1, 3, 5).reshape(-1)]).contiguous()
+    w = w.view(w.shape[0] // 32, 32, w.shape[1] // 16, 2, 2, 4)[:, tau]                  # [block][row][step][quad][half][4]
+    return w.permute(0, 2, 4, 1, 3, 5).reshape(-1)
 
 
 ATTENTION_HEADS_TOKENS = 256     # longest row of ffk_attention_heads
+
+def pack_transition_block(w1, w2, dtype, device):
+    """The weights of a transition in the fragment order of ``ffk_transition_block``; None at widths it is not built for."""
+    hidden, C = w1.shape
+    if dtype != torch.bfloat16 or (C, hidden) not in ((64, 128), (64, 256), (128, 512), (256, 1024)):
+        return None
+    return pack_fragments(w1, dtype, device), pack_fragments_of_accumulators(w2, dtype, device)
+
 
 # False: every attention runs as projection, core and output stage (tests compare the two)
 _ATTENTION_BLOCK = True

@@ -429,6 +429,14 @@ int ffk_transition_fused(void* out, const void* x, void* xtail, const void* gamm
                          const void* b1, const void* w2, const void* b2, int64_t M, int64_t C,
                          int64_t hidden, float eps, int dtype, void* stream);
 
+/* The same with the weights in fragment order, built for C = 64, 128 and 256 with hidden = 4 C and for 64 -> 128 -> 64 (bf16):
+ * w1 : [hidden / 32][C / 16][64][8], element e of lane l in step s of block b is row 32 b + l % 32, column 16 s + 8 (l / 32) + e of W1;
+ * w2 : [C / 32][hidden / 16][64][8], the same element is row 32 b + tau(l % 32), tau(8 a + 4 h + c) = 16 h + 4 a + c, column
+ *   16 s + 8 (e / 4) + 4 (l / 32) + e % 4 of W2;  b1 : [hidden];  b2 : [C]. */
+int ffk_transition_block(void* out, const void* x, void* xtail, const void* gamma, const void* beta, const void* w1,
+                         const void* b1, const void* w2, const void* b2, int64_t M, int64_t C, int64_t hidden, float eps,
+                         int dtype, void* stream);
+
 /* Gated output stage of a gated attention (bf16; C = 128 or 256 channels, H * 32 = C gate channels):
  *     out[row m] = x[row m] + Wo . ( sigmoid( Wg . LayerNorm(x[row m]; gamma, beta, eps) + bg ) * o[m] ) + bo
  * x, out : the tensor the attention updates, logical row m at (m / inner) * s_o + (m % inner) * s_i (elements, C
@@ -618,7 +626,8 @@ enum {
     FFK_OP_FILL_ZERO = 9, FFK_OP_ATTENTION_FWD_LSE = 10, FFK_OP_ATTENTION_BWD_ROWS = 11, FFK_OP_TRANSPOSE_BATCHED = 12,
     FFK_OP_WEIGHT_GRAD = 13, FFK_OP_LAYERNORM_BWD_ROWS = 14, FFK_OP_SCALE_ROWS = 15, FFK_OP_ATT_GATE_BWD = 16,
     FFK_OP_TRIMUL_GATE_BWD = 17, FFK_OP_GLU_BWD = 18, FFK_OP_BIAS_COLS = 19, FFK_OP_SLICE_SUM = 20,
-    FFK_OP_ATTENTION_BLOCK = 21, FFK_OP_ATTENTION_HEADS = 22, FFK_OP_COUNT = 23
+    FFK_OP_ATTENTION_BLOCK = 21, FFK_OP_ATTENTION_HEADS = 22, FFK_OP_TRANSITION_BLOCK = 23,
+    FFK_OP_COUNT = 24
 };
 int ffk_run_plan(const void* plan, int64_t bytes, const uint64_t* bases, int64_t n_bases, void* stream);
 
