@@ -20,11 +20,14 @@
 // us per sub-module, launches of their own -> here (both with the launch that computes the pair bias):
 //   128 channels in 4 heads, N rows of N tokens:  N = 64 17.7 -> 15.0, 96 24.6 -> 19.6, 128 29.4 -> 22.8, 192 49 -> 33.5, 256 62 -> 48
 //   64 channels in 4 heads:  N = 64 18.6 -> 11.1, 128 26.0 -> 15.0, 256 50.5 -> 32, 320 79 -> 77, 512 184 -> 171
+//     (row sums of the probabilities as the matrix product's idle rows instead of eight dot instructions a tile: 320 77 -> 71, 512 171 -> 157)
+//   64 channels in 8 heads, 1 024 rows of N tokens:  N = 64 68 -> 39, 160 147 -> 96, 256 196 -> 157, 384 376 -> 320
+//     (more than 384 tokens: four tiles a wave with four heads each do not fit the registers, 512 593 -> 2 583)
 //   256 channels in 8 heads, rows of 128 tokens, no bias:  64 rows 33.5 -> 27.8, 256 69 -> 34, 416 109 -> 59, 1 024 266 -> 125
 //                            with a pair bias:  128 rows of 96 tokens 45 -> 29, of 128 tokens 51 -> 36
 //   the same to the gated heads, output projection apart (k and v of four heads of 256 tokens fill the LDS: two workgroups to a row):
 //                            128 rows of 160 tokens 67 -> 49, 192 74 -> 53, 256 87 -> 72;  512 rows of 256 296 -> 228
-// From how many rows on: attention_block_rows in model/fastnn/_fused.py.  Longer rows do not fit: at 128 channels, k and v of more than 256 tokens go into LDS in two passes only (heads two by two, rows
+// For which numbers of rows: attention_block_pays in model/fastnn/_fused.py.  Longer rows do not fit: at 128 channels, k and v of more than 256 tokens go into LDS in two passes only (heads two by two, rows
 // normalised twice), which was built and is slower (288 tokens 122 us against 92, 416 235 against 189).
 #include "ffk_rowblock.h"
 #include <type_traits>
@@ -42,7 +45,7 @@ struct AbArgs : RbRows {
     float qscale;
 };
 
-// Geometry: eight waves, WB blocks of 32 channels (one head of 32, two of 16) to a workgroup, 8 / WB waves to a block, each with every
+// Geometry: eight waves, WB blocks of 32 channels (one head of 32, two of 16, four of 8) to a workgroup, 8 / WB waves to a block, each with every
 // (8 / WB)-th tile of 32 tokens, at most TPW of them.  64 and 128 channels: all blocks.  256 channels: half of them, k and v of more
 // would not fit; the output projection, which needs all heads, is a launch of its own (HEADS: `out` takes the gated outputs).
 template <int C, int D, int TPW> struct AbGeo {
@@ -55,8 +58,9 @@ template <int C, int D, int TPW> struct AbGeo {
     static constexpr int NT_MAX = WPB * TPW;
     static constexpr int XP = C * 2 + 16;           // pitch of the normalised rows (bytes)
     static constexpr int HP = WB * 64 + 16;         // HEADS: pitch of the gated outputs
-    static constexpr size_t smem(long NT) {         // rows, then k and v, then the gated outputs (and the updates)
-        const size_t rows = (size_t)NT * 32 * XP, kv = (size_t)NT * WB * 4096, end = HEADS ? 0 : rows + (size_t)NT * NB * 2048;
+    static constexpr bool ONES = D < 32;            // row sums through the weighted sum's product (see attend)
+    static constexpr size_t smem(long NT) {         // rows, then k and v (and a tile of ones), then the gated outputs (and the updates)
+        const size_t rows = (size_t)NT * 32 * XP, kv = (size_t)NT * WB * 4096 + (ONES ? 2048 : 0), end = HEADS ? 0 : rows + (size_t)NT * NB * 2048;
         return rows > kv ? (rows > end ? rows : end) : (kv > end ? kv : end);
     }
 };
@@ -82,6 +86,7 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
     unsigned char* s_x = ab_smem;                    // [32 NT][XP]
     T* s_k = reinterpret_cast<T*>(ab_smem);          // [WB][NT][2][64][8]
     T* s_v = s_k + (size_t)WB * NT * 1024;           // the same
+    T* s_one = s_v + (size_t)WB * NT * 1024;         // ONES: a tile of ones
     T* s_o = s_k;                                    // [NT][NB][2][64][8]
     const T* xrow = a.x + (long)b2 * a.s_row;
 
@@ -135,7 +140,20 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
     };
     auto attend = [&](int sub, const T* bp, const T* bp_next, const bf16x8& q0, const bf16x8& q1, f32x16& acc, float& inv) __attribute__((always_inline)) {
         const T* kp = s_k + (size_t)wb * NT * 1024 + lane * 8;
-        const T* vp = s_v + (size_t)wb * NT * 1024 + lane * 8;
+        // D < 32: what v's tile holds of other heads is read as ones, so that the product's other rows are the row sums of the
+        // probabilities, in every lane for all keys
+        const bool own = !G::ONES || l32 / D == sub;
+        const T* vp = (own ? s_v + (size_t)wb * NT * 1024 : s_one) + lane * 8;
+        const int vstep = own ? 1024 : 0;
+        constexpr int REGS = D / 2;                  // accumulator registers of a head
+        const int lreg = sub == 0 ? REGS & 15 : 0;
+        bf16x8 qs = q0;                              // D < 32: the fragment with the head's channels, the others' cleared
+        if (sub * REGS >= 8) qs = q1;
+        if (D == 8) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if ((e >> 2) != (sub & 1)) qs[e] = (T)0.0f;
+        }
         f32x16 negm, s;
         float l_run;
         auto bias_req = [&](int kt, bf16x8 (&b)[2]) __attribute__((always_inline)) {
@@ -149,12 +167,13 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
                 kf[0] = MM::ld(q);
                 kf[1] = MM::ld(q + 512);
             } else {
-                kf[0] = MM::ld(q + sub * 512);
+                kf[0] = MM::ld(q + sub * REGS / 8 * 512);
             }
         };
         auto v_req = [&](int kt) __attribute__((always_inline)) {
-            vf[0] = MM::ld(vp + kt * 1024);
-            vf[1] = MM::ld(vp + kt * 1024 + 512);
+            const T* q = vp + kt * vstep;
+            vf[0] = MM::ld(q);
+            vf[1] = MM::ld(q + 512);
         };
         auto score = [&](int kt, const bf16x8 (&b)[2]) __attribute__((always_inline)) {
             s = negm;
@@ -162,7 +181,7 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
                 MM::mma(s, kf[0], q0);
                 MM::mma(s, kf[1], q1);
             } else {
-                MM::mma(s, kf[0], sub ? q1 : q0);
+                MM::mma(s, kf[0], qs);
             }
             MM::mma(s, b[0], ident[0]);
             MM::mma(s, b[1], ident[1]);
@@ -175,20 +194,23 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
                 }
             }
         };
-        auto prob = [&]() __attribute__((always_inline)) -> float {
+        auto prob = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int t = 0; t < 8; ++t) p[i][t] = (T)fast_exp2(s[8 * i + t]);
+        };
+        auto row_sum = [&]() __attribute__((always_inline)) -> float {         // of this lane's keys
             typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
             const bf16x2 ones = {(T)1.0f, (T)1.0f};
             float sum = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-#pragma unroll
-                for (int t = 0; t < 8; ++t) p[i][t] = (T)fast_exp2(s[8 * i + t]);
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const bf16x2 pr = {p[i][2 * t], p[i][2 * t + 1]};
                     sum = __builtin_amdgcn_fdot2_f32_bf16(pr, ones, sum, false);
                 }
-            }
             return sum;
         };
         auto weigh = [&]() __attribute__((always_inline)) {
@@ -219,7 +241,8 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
                 s[v] -= m0;
                 negm[v] = -m0;
             }
-            l_run = prob();
+            prob();
+            l_run = G::ONES ? 0.0f : row_sum();
             weigh();
             auto step = [&](int kt, bf16x8 (&b)[2]) __attribute__((always_inline)) {
                 v_req(kt);
@@ -229,8 +252,10 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
                     bias_req(kt + 2, b);
                 }
                 asm volatile("" ::: "memory");
-                float sum = prob();
+                prob();
+                float sum = G::ONES ? 0.0f : row_sum();
                 if (careful) {
+                    if (G::ONES) sum = row_sum();
                     if (__builtin_amdgcn_ballot_w64(!(sum <= 1048576.0f)) != 0) {
                         const bool fresh = negm[0] == -NEG_FLOOR;
                         if (fresh) {
@@ -250,12 +275,13 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
                             acc[v] *= alpha;
                         }
                         l_run *= alpha;
-                        sum = prob();
+                        prob();
+                        sum = row_sum();
                     }
                     k_req(kt + 1);
                     bias_req(kt + 2, b);
                 }
-                l_run += sum;
+                if (!G::ONES) l_run += sum;
                 weigh();
             };
             int kt = 1;
@@ -264,6 +290,7 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
                 step(kt + 1, bias[0]);
             }
             if (kt < kt_end) step(kt, bias[1]);
+            if (G::ONES) l_run = acc[lreg];
             // probabilities are not negative: a finite sum shows that none overflowed
             if (careful || __builtin_amdgcn_ballot_w64(!(l_run <= 1.8446744e19f)) == 0) break;
         }
@@ -277,7 +304,7 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
                 bias[1][i] = t;
             }
         }
-        const float l_tot = l_run + lane_xor<32>(l_run);
+        const float l_tot = G::ONES ? l_run : l_run + lane_xor<32>(l_run);
         inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;              // all keys masked: zero
     };
 
@@ -328,6 +355,7 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
                 rb_pin(of[i][j]);
             }
         lds_barrier();                           // nobody reads the rows any more
+        if (G::ONES && tid < 128) *reinterpret_cast<u32x4*>(s_one + tid * 8) = u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
 #pragma unroll
         for (int i = 0; i < TPW; ++i) {
             if (t_first + WPB * i < NT) {
@@ -358,9 +386,10 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
                 attend(sub, bias_row(i, sub), next, qf[i][0], qf[i][1], acc, inv);
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
-                    if (D == 16 && j != sub) continue;
+                    if (8 * j + 7 < sub * (D / 2) || 8 * j >= (sub + 1) * (D / 2)) continue;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) of[i][j][e] = (T)(acc[8 * j + e] * inv * (float)of[i][j][e]);
+                    for (int e = 0; e < 8; ++e)      // the head's registers
+                        if ((8 * j + e) / (D / 2) == sub) of[i][j][e] = (T)(acc[8 * j + e] * inv * (float)of[i][j][e]);
                     rb_pin(of[i][j]);
                 }
             }
@@ -658,8 +687,8 @@ extern "C" int ffk_attention_block(void* out, const void* x, void* xtail, const 
                                    int64_t s_row, int64_t s_tok, int64_t bias_pitch, float eps, int dtype, void* stream) {
     FFK_REQUIRE(out && x && gamma && beta && w && bg && keybias && tileflags, FFK_ERR_NULL, "ffk_attention_block: null pointer");
     FFK_REQUIRE(dtype == FFK_BF16, FFK_ERR_DTYPE, "ffk_attention_block: bf16 only (dtype tag %d)", dtype);
-    FFK_REQUIRE((C == 128 && D == 32) || (C == 64 && D == 16) || (C == 256 && D == 32), FFK_ERR_UNSUPPORTED,
-                "ffk_attention_block: built for 128 or 256 channels in heads of 32 and 64 in heads of 16, got %ld / %ld", (long)C, (long)D);
+    FFK_REQUIRE((C == 128 && D == 32) || (C == 64 && (D == 16 || D == 8)) || (C == 256 && D == 32), FFK_ERR_UNSUPPORTED,
+                "ffk_attention_block: built for 128 or 256 channels in heads of 32 and 64 in heads of 16 or 8, got %ld / %ld", (long)C, (long)D);
     FFK_REQUIRE(C == 256 || bias_t, FFK_ERR_UNSUPPORTED, "ffk_attention_block: built with a pair bias for 64 and 128 channels");
     FFK_REQUIRE(B2 > 0 && B2 < (1L << 31) - 64 && N > 0, FFK_ERR_SHAPE, "ffk_attention_block: bad shape B2=%ld N=%ld", (long)B2, (long)N);
     FFK_REQUIRE(s_row % 16 == 0 && s_tok % 16 == 0, FFK_ERR_ALIGN, "ffk_attention_block: row strides must be multiples of 16 elements");
@@ -668,7 +697,7 @@ extern "C" int ffk_attention_block(void* out, const void* x, void* xtail, const 
                     ffk_aligned16(drop),
                 FFK_ERR_ALIGN, "ffk_attention_block: buffers must be 16-byte aligned");
     const long NT = (N + 31) / 32;
-    FFK_REQUIRE(NT <= (C == 256 ? 4 : C == 128 ? 8 : 16), FFK_ERR_UNSUPPORTED,
+    FFK_REQUIRE(NT <= (C == 256 ? 4 : C == 128 ? 8 : D == 16 ? 16 : 12), FFK_ERR_UNSUPPORTED,
                 "ffk_attention_block: rows of %ld tokens are too long for %ld channels", (long)N, (long)C);
     FFK_REQUIRE(!bias_t || bias_pitch >= NT, FFK_ERR_SHAPE, "ffk_attention_block: bias rows of %ld tiles, %ld needed", (long)bias_pitch, NT);
     const AbArgs a = {{(T*)out, (const T*)x, (int8_t*)xtail, (const T*)gamma, (const T*)beta, (const T*)drop, (long)s_tok, (int)N, eps},
@@ -676,6 +705,13 @@ extern "C" int ffk_attention_block(void* out, const void* x, void* xtail, const 
                       (int)bias_pitch, 1.4426950408889634f / sqrtf((float)D)};
     hipStream_t st = (hipStream_t)stream;
     if (C == 256) return bias_t ? aw_launch_nt<true>(a, NT, st) : aw_launch_nt<false>(a, NT, st);
+    if (C == 64 && D == 8) {
+        switch ((NT + 3) / 4) {
+            case 1: return ab_launch<64, 8, 1>(a, NT, st);
+            case 2: return ab_launch<64, 8, 2>(a, NT, st);
+            default: return ab_launch<64, 8, 3>(a, NT, st);
+        }
+    }
     if (C == 64) {
         switch ((NT + 3) / 4) {
             case 1: return ab_launch<64, 16, 1>(a, NT, st);

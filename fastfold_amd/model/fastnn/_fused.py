@@ -260,20 +260,37 @@ def key_bias(mask, device, *, B2, N, mask_sb, mask_sn):
 
 
 def attention_block_tokens(dtype, H, c, d_in, d_out):
-    """Longest row of tokens that ``ffk_attention_block`` takes at these widths, 0 where it is not built for them.  It is the faster
-    path at every length it takes (timings of both sides in csrc/ffk_attention_block.hip)."""
+    """Longest row of tokens that ``ffk_attention_block`` takes at these widths, 0 where it is not built for them (timings of both
+    sides in csrc/ffk_attention_block.hip and below)."""
     if dtype != torch.bfloat16 or d_in != d_out or H * c != d_in:
         return 0
-    return {(128, 32): 256, (64, 16): 512, (256, 32): 128}.get((d_in, c), 0)
+    return {(128, 32): 256, (64, 16): 512, (64, 8): 384, (256, 32): 128}.get((d_in, c), 0)
 
 
-def attention_block_rows(C, N, biased):
-    """Fewest batch rows from which ``ffk_attention_block`` and ``ffk_attention_heads`` are taken.  Their time does not depend on the
-    number of rows up to one per CU, and 256 channels keep a CU busy for long: us per sub-module, one kernel / launches of their own,
-    rows with a bias of N = 64: 8 rows 21 / 22; 96: 16 rows 27 / 25, 32 27 / 28; 128: 32 rows 35 / 31, 48 35 / 38; 160: 32 rows
-    37 / 37, 48 38 / 40; 192: 48 rows 47 / 46, 64 48 / 49; 256: 64 rows 60 / 57, 96 65 / 75; without one: 96: 32 rows 20 / 21, 128: 32
-    rows 27 / 24, 64 28 / 34.  The narrower kernels have as many rows as tokens and win at every size."""
-    return 0 if C < 256 or N <= 64 else N // 3 if biased else N // 4
+def attention_block_pays(C, head_dim, N, B2, biased):
+    """Whether ``ffk_attention_block`` (``ffk_attention_heads``) beats launches of their own for B2 rows of N tokens.  One row keeps a
+    CU busy, whatever the others do (two CUs where the heads are split), so what counts is how full the last round of rows is.
+    us per sub-module, one kernel / launches of their own:
+      256 channels, no bias: 128 tokens, 32 rows 27 / 24, 40 28 / 30, 64 28 / 34, 260 57 / 82; 96 tokens, 24 rows 20 / 21
+      256 channels with a bias: 128 tokens, 32 rows 35 / 31, 48 35 / 38, 260 69 / 92; 96 tokens, 16 rows 27 / 25, 32 27 / 28;
+        heads apart: 160 tokens, 32 rows 37 / 37, 130 69 / 75; 192, 60 rows 47 / 49, 130 80 / 83; 224, 60 rows 55 / 54, 130 95 / 88,
+        200 102 / 119; 256, 60 rows 61 / 57, 90 65 / 74, 130 109 / 101, 180 115 / 114, 200 117 / 135
+      64 channels in heads of 8: 96 tokens, 80 rows 18 / 24, 260 29 / 39; 160, 64 rows 31 / 29, 140 31 / 41; 256, 140 rows 46 / 51,
+        200 47 / 63, 300 83 / 78, 380 84 / 89; 320, 380 rows 133 / 129, 600 193 / 189, 700 193 / 216; 384, 600 rows 244 / 223, 700 244 / 253
+    The other widths have as many rows as tokens, and it wins at every length it takes."""
+    cus = 256
+    wgs = B2 * 2 if C == 256 and N > 128 else B2
+    rounds = -(-wgs // cus)
+    fill = wgs / (cus * rounds)
+    if C == 64 and head_dim == 8:
+        return N <= 96 or fill >= 0.35 + 0.56 * (N - 96) / 288
+    if C < 256:
+        return True
+    if rounds > 1:
+        return N <= 192 or fill >= 0.75
+    if N > 128:
+        return fill >= N / 384
+    return N <= 64 or B2 >= N // (3 if biased else 4)
 
 
 def pack_attention_block(qkv_w, gate_w, out_w, dtype, device):
@@ -347,7 +364,7 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     # kernel, which writes q, k and the gate in accumulator order straight from its registers.
     acc_order = dt == torch.bfloat16 and C in (64, 128, 256) and N % 32 == 0
     # Short rows: one kernel from the rows of x to the updated rows.
-    enough = B2 >= attention_block_rows(C, N, bias_t is not None or bias_in_launch)
+    enough = attention_block_pays(C, head_dim, N, B2, bias_t is not None or bias_in_launch)
     if (_ATTENTION_BLOCK and enough and acc_order and hasattr(w_pk, "block") and N <= attention_block_tokens(dt, H, head_dim, C, c_out)
             and ln is not None and resid is not None and resid.data_ptr() == x.data_ptr() and o_map is None
             and a_so % 16 == 0 and a_si % 16 == 0 and (C == 256 or bias_t is not None or bias_in_launch)

@@ -452,8 +452,8 @@ int ffk_gated_out_fused(void* out, const void* x, void* xtail, const void* gamma
 
 /* A gated attention over short rows as one kernel (bf16): each of B2 batch rows of N tokens attends within itself,
  *     out = x + (Wo . ( sigmoid(Wg y + bg) * attention(Wq y, Wk y, Wv y) ) + bo) * drop,    y = LayerNorm(x; gamma, beta, eps)
- * C hidden and C output channels, built for C = 128 in heads of D = 32 and C = 64 in heads of 16 (both with a pair bias) and C = 256
- * in heads of 32 (with or without one), N at most 256, 512 and 128 (what fits the LDS and the registers of a CU).
+ * C hidden and C output channels, built for C = 128 in heads of D = 32 and C = 64 in heads of 16 or 8 (all with a pair bias) and C = 256
+ * in heads of 32 (with or without one), N at most 256, 512, 384 and 128 (what fits the LDS and the registers of a CU).
  * x, out : token n of batch row b at b * s_row + n * s_tok (elements, multiples of 16; C contiguous channels; may alias);
  * xtail : NULL or the tail bytes of x / out as an extended residual stream (addressed like x);
  * w : the five weights in fragment order, [q, k, v, gate, output][C / 32][C / 16][64][8]: element e of lane l in step s of block b

@@ -87,6 +87,7 @@ TOL = 6 * 2.0 ** -9
 # a multiple of eight.
 @pytest.mark.parametrize("C,D,N", [(128, 32, n) for n in (1, 32, 50, 64, 96, 128, 129, 160, 224, 256)]
                          + [(64, 16, n) for n in (32, 77, 128, 160, 256, 288, 320, 500, 512)]
+                         + [(64, 8, n) for n in (20, 32, 96, 128, 200, 256, 257, 384)]
                          + [(256, 32, n) for n in (5, 32, 64, 65, 96, 128)] + [(256, -32, n) for n in (32, 50, 96, 128)])
 def test_attention_block_against_float64(dev, C, D, N):
     p = _case(dev, C, abs(D), 9, N, seed=C + N, transposed=N % 3 == 0, bias=C != 256 or D < 0)
@@ -99,7 +100,7 @@ def test_attention_block_against_float64(dev, C, D, N):
     assert torch.equal(out[2], p["x"][2])
 
 
-@pytest.mark.parametrize("C,D,N", [(128, 32, 96), (128, 32, 256), (64, 16, 320), (256, 32, 128)])
+@pytest.mark.parametrize("C,D,N", [(128, 32, 96), (128, 32, 256), (64, 16, 320), (64, 8, 160), (256, 32, 128)])
 def test_attention_block_residual_forms(dev, C, D, N):
     """Output bias, dropout multipliers, in place, and the tail of an extended residual stream."""
     p = _case(dev, C, D, 3, N, seed=N, bias=C != 256)
@@ -117,9 +118,10 @@ def test_attention_block_residual_forms(dev, C, D, N):
     assert _err(_stream(x2, tail), p, want) < TOL
 
 
-def test_attention_block_moving_reference(dev):
+@pytest.mark.parametrize("C,D", [(128, 32), (64, 16), (64, 8)])
+def test_attention_block_moving_reference(dev, C, D):
     """Scores that rise far above those of the first tile: the second walk, with the reference moved tile by tile."""
-    p = _case(dev, 128, 32, 4, 256, seed=2)
+    p = _case(dev, C, D, 4, 256, seed=2)
     p["mask"][:] = 1
     rise = torch.arange(8, device=dev).repeat_interleave(32).float() * 80.0
     p["bias"] = (p["bias"].float() + rise[None, None, :]).to(BF)
@@ -158,3 +160,52 @@ def test_attention_block_refuses(dev):
     p = _case(dev, 128, 32, 2, 64, seed=0, bias=False)
     with pytest.raises(RuntimeError, match="pair bias"):
         _run(p, p["x"], torch.empty_like(p["x"]))
+
+
+def _modules(dev):
+    from fastfold_amd.model.fastnn.msa import MSAColumnAttention, MSARowAttentionWithPairBias
+    from fastfold_amd.model.fastnn.ops import ChunkTriangleAttentionEndingNode, ChunkTriangleAttentionStartingNode
+
+    def pair(r, c, **kw):
+        z, pm = torch.randn(1, r, r, c, device=dev).to(BF), torch.ones(1, r, r, device=dev, dtype=BF)
+        pm[:, -5:] = 0
+        pm[:, :, -5:] = 0
+        return z, pm
+
+    def msa(s, r, c):
+        m, mm = torch.randn(1, s, r, c, device=dev).to(BF), torch.ones(1, s, r, device=dev, dtype=BF)
+        mm[:, :, -5:] = 0
+        return m, mm
+    for r, c, d in ((64, 128, 32), (160, 128, 32), (96, 64, 16)):
+        for cls in (ChunkTriangleAttentionStartingNode, ChunkTriangleAttentionEndingNode):
+            yield cls(c, 0.25, c=d, n_head=4), pair(r, c)
+    for s, r, c, d in ((64, 96, 256, 32), (60, 160, 256, 32), (40, 96, 64, 8)):
+        m, mm = msa(s, r, c)
+        yield MSARowAttentionWithPairBias(c, 128, c=d, n_head=8), (m, pair(r, 128)[0], mm)
+    yield MSAColumnAttention(256), msa(96, 64, 256)
+
+
+def test_modules_take_the_block_and_match_the_separate_launches(dev, monkeypatch):
+    """Every attention module at sizes that go to the one kernel, against the same module as projection, core and output stage: the two
+    differ by their own bf16 roundings only (six of 2^-9 on either side)."""
+    from fastfold_amd import _lib
+    from fastfold_amd.model.fastnn import _fused as F_
+    torch.manual_seed(4)
+    names, call = [], _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *a: (names.append(name), call(name, *a))[1])
+    for mod, args in _modules(dev):
+        with torch.no_grad():
+            for n, p in mod.named_parameters():
+                p.copy_(1 + 0.1 * torch.randn_like(p) if "layernorm" in n and n.endswith("weight")
+                        else torch.randn_like(p) * (0.3 if p.dim() == 1 else p.shape[-1] ** -0.5))
+        mod = mod.to(dev, BF).eval()
+        outs = []
+        for on in (True, False):
+            monkeypatch.setattr(F_, "_ATTENTION_BLOCK", on)
+            del names[:]
+            with torch.no_grad():
+                outs.append(mod(*args).float())
+            assert on == any(n in ("ffk_attention_block", "ffk_attention_heads") for n in names), (type(mod).__name__, names)
+        upd = outs[1] - args[0].float()
+        err = float((outs[0] - outs[1]).norm() / upd.norm())
+        assert float(upd.norm()) > 1.0 and err < 2 * TOL, (type(mod).__name__, args[0].shape, err)
