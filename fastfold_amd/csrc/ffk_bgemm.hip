@@ -6,9 +6,14 @@
 //   128 x 128, chunks of 128 bytes, 64 x 64 per wave       (four 32 x 32 products per two fragments of each operand)
 //    64 x  64, chunks of 256 bytes, 32 x 32 per wave
 //    32 x  32, chunks of 4 x 128 bytes, each wave takes one quarter of K (fp32, K >= 512)
+// fp32 products are six bf16 products of the operands' parts (split4), which are cut on the way to LDS, one slot of it.  Against the
+// fp32 instructions, us: 128 products of 256 x 256 x 256 48 -> 35, of 384 x 384 x 384 169 -> 108; 65 536 x 128, K = 1 024 149 -> 110,
+// K = 512 80 -> 56; 32 768 x 256, K = 1 024 147 -> 97; 8 192 x 8 192, K = 128 193 -> 141; 4 096 x 128, K = 1 024, where the launch waits for one
+// chunk after the other and cutting lengthens that chain, 17.7 -> 19.1.
 // Every tile gives the same bits (callers cut their rows into pieces as memory allows, and pieces take other tiles): products are
 // added in ascending order of K, for fp32 and K >= 512 within quarters of K, as ((q0 + q1) + q2) + q3.
 #include "ffk_common.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -29,14 +34,17 @@ __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_de
     constexpr bool QUARTERS = std::is_same<T, float>::value;    // sums in quarters of K possible
     constexpr int BKB = 128 * 128 / BT;            // bytes of K per row and chunk
     constexpr int BK = BKB / ES;
-    constexpr int P = BKB + 16;                    // ring row pitch (bytes)
+    // fp32: operands lie in LDS as their three bf16 parts (see split4), [K step of 16][part][16] per row, one slot of each
+    constexpr bool SPLIT = std::is_same<T, float>::value;
+    constexpr int NSLOT = SPLIT ? 1 : 2;
+    constexpr int P = (SPLIT ? BKB / 2 * 3 : BKB) + 16;        // row pitch of a slot (bytes)
     constexpr int SLOT = BT * P;
     constexpr int CP = BT * OES + 16;              // staged C pitch [m][n]
     constexpr int NV = BT * (BK / VEC) / THREADS;  // 16-byte vectors per thread per operand chunk (= 4)
 
     extern __shared__ __align__(16) unsigned char smem[];
-    unsigned char* sA = smem;                      // 2 slots
-    unsigned char* sB = smem + 2 * SLOT;           // 2 slots
+    unsigned char* sA = smem;                      // NSLOT slots
+    unsigned char* sB = smem + NSLOT * SLOT;       // NSLOT slots
     unsigned char* sC = smem;                      // aliases the ring after the K loop
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -93,8 +101,18 @@ __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_de
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) xa.e[e] = xb.e[e] = DT<T>::from_f(0.0f);
             }
-            *reinterpret_cast<Vec16<T>*>(sA + slot * SLOT + r * P + c * 16) = xa;
-            *reinterpret_cast<Vec16<T>*>(sB + slot * SLOT + r * P + c * 16) = xb;
+            if constexpr (SPLIT) {
+                const int o = r * P + (c >> 2) * 96 + (c & 3) * 8;
+                const Split4 a3 = split4(*reinterpret_cast<const f32x4*>(&xa)), b3 = split4(*reinterpret_cast<const f32x4*>(&xb));
+#pragma unroll
+                for (int p = 0; p < 3; ++p) {
+                    *reinterpret_cast<u32x2*>(sA + o + p * 32) = a3.p[p];
+                    *reinterpret_cast<u32x2*>(sB + o + p * 32) = b3.p[p];
+                }
+            } else {
+                *reinterpret_cast<Vec16<T>*>(sA + slot * SLOT + r * P + c * 16) = xa;
+                *reinterpret_cast<Vec16<T>*>(sB + slot * SLOT + r * P + c * 16) = xb;
+            }
         }
     };
 
@@ -131,25 +149,60 @@ __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_de
                         for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
             }
         }
-        const int slot = kc & 1;
+        const int slot = kc & (NSLOT - 1);
+        if (SPLIT && kc) lds_barrier();            // nobody reads the chunk before any more
         commit(slot, kc);
         lds_barrier();
         if (kc + 1 < kchunks) fetch(kc + 1);
-        const unsigned char* pa = sA + slot * SLOT + (wm * WT * 32 + l32) * P + half * (MM::KLANE * ES);
-        const unsigned char* pb = sB + slot * SLOT + (wn * WT * 32 + l32) * P + half * (MM::KLANE * ES);
+        if constexpr (SPLIT) {
+            constexpr int STEPS = BK / 16 / (KSPLIT ? 4 : 1);
+            const unsigned char* pa = sA + (wm * WT * 32 + l32) * P + (KSPLIT ? wave * STEPS * 96 : 0) + half * 16;
+            const unsigned char* pb = sB + (wn * WT * 32 + l32) * P + (KSPLIT ? wave * STEPS * 96 : 0) + half * 16;
+            constexpr int FB = WT == 1 ? 2 : 1;    // fragments a step ahead, where the registers hold them
+            bf16x8 fa[FB][WT][3], fb[FB][WT][3];
+            auto frags = [&](int ks, bf16x8 (&fa)[WT][3], bf16x8 (&fb)[WT][3]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k0 = 0; k0 < BK / MM::KSTEP / (KSPLIT ? 4 : 1); ++k0) {
-            const int ks = KSPLIT ? wave * (BK / MM::KSTEP / 4) + k0 : k0;
-            typename MM::Frag fa[WT], fb[WT];
+                for (int i = 0; i < WT; ++i)
 #pragma unroll
-            for (int i = 0; i < WT; ++i) {
-                fa[i] = *reinterpret_cast<const typename MM::Frag*>(pa + i * 32 * P + ks * MM::KSTEP * ES);
-                fb[i] = *reinterpret_cast<const typename MM::Frag*>(pb + i * 32 * P + ks * MM::KSTEP * ES);
+                    for (int p = 0; p < 3; ++p) {
+                        fa[i][p] = *reinterpret_cast<const bf16x8*>(pa + i * 32 * P + ks * 96 + p * 32);
+                        fb[i][p] = *reinterpret_cast<const bf16x8*>(pb + i * 32 * P + ks * 96 + p * 32);
+                    }
+            };
+            frags(0, fa[0], fb[0]);
+#pragma unroll
+            for (int ks = 0; ks < STEPS; ++ks) {
+                if (FB == 2) {
+                    if (ks + 1 < STEPS) frags(ks + 1, fa[(ks + 1) % FB], fb[(ks + 1) % FB]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int t = 0; t < 6; ++t)
+#pragma unroll
+                    for (int ni = 0; ni < WT; ++ni)
+#pragma unroll
+                        for (int mi = 0; mi < WT; ++mi)
+                            Mma<bf16_t>::mma(acc[ni][mi], fb[ks % FB][ni][SPLIT_B[t]], fa[ks % FB][mi][SPLIT_A[t]]);
+                if (FB == 1 && ks + 1 < STEPS) frags(ks + 1, fa[0], fb[0]);
+                if (FB == 2) __builtin_amdgcn_sched_barrier(0);
             }
+        } else {
+            const unsigned char* pa = sA + slot * SLOT + (wm * WT * 32 + l32) * P + half * (MM::KLANE * ES);
+            const unsigned char* pb = sB + slot * SLOT + (wn * WT * 32 + l32) * P + half * (MM::KLANE * ES);
 #pragma unroll
-            for (int ni = 0; ni < WT; ++ni)
+            for (int k0 = 0; k0 < BK / MM::KSTEP / (KSPLIT ? 4 : 1); ++k0) {
+                const int ks = KSPLIT ? wave * (BK / MM::KSTEP / 4) + k0 : k0;
+                typename MM::Frag fa[WT], fb[WT];
 #pragma unroll
-                for (int mi = 0; mi < WT; ++mi) MM::mma(acc[ni][mi], fb[ni], fa[mi]);
+                for (int i = 0; i < WT; ++i) {
+                    fa[i] = *reinterpret_cast<const typename MM::Frag*>(pa + i * 32 * P + ks * MM::KSTEP * ES);
+                    fb[i] = *reinterpret_cast<const typename MM::Frag*>(pb + i * 32 * P + ks * MM::KSTEP * ES);
+                }
+#pragma unroll
+                for (int ni = 0; ni < WT; ++ni)
+#pragma unroll
+                    for (int mi = 0; mi < WT; ++mi) MM::mma(acc[ni][mi], fb[ni], fa[mi]);
+            }
         }
     }
     if constexpr (QUARTERS && !KSPLIT) {
@@ -174,6 +227,30 @@ __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_de
             for (int v = 0; v < 16; ++v) acc[0][0][v] = ((acc[0][0][v] + red[v * 64 + lane]) + red[(16 + v) * 64 + lane]) + red[(32 + v) * 64 + lane];
         }
         lds_barrier();
+    }
+
+    if constexpr (SPLIT) {                         // infinite operands, whose parts make NaN of every product: anew, product by product
+#pragma unroll
+        for (int ni = 0; ni < WT; ++ni)
+#pragma unroll
+            for (int mi = 0; mi < WT; ++mi) {
+                float x = acc[ni][mi][0];
+#pragma unroll
+                for (int v = 1; v < 16; ++v) x += acc[ni][mi][v];
+                if (__builtin_expect(!__any(x - x != 0.0f), 1)) continue;
+                const long m = m0 + wm * WT * 32 + mi * 32 + l32, nb = n0 + wn * WT * 32 + ni * 32;
+                const T* pa = A + (m < M ? m : M - 1) * d.lda;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    if (acc[ni][mi][v] == acc[ni][mi][v]) continue;
+                    const long n = nb + acc_row(v, lane);
+                    const T* pb = B + (n < N ? n : N - 1) * d.ldb;
+                    float y = 0.0f;
+#pragma unroll 1
+                    for (int k = 0; k < K; ++k) y = fmaf(pa[k], pb[k], y);
+                    acc[ni][mi][v] = y;
+                }
+            }
     }
 
     // row offsets of this tile, one integer division per row (kept in LDS for phase 2)
@@ -320,7 +397,7 @@ __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_de
 
 template <typename T, typename OT, int BT>
 int launch_tile(const ffk_bgemm_desc& d, hipStream_t st) {
-    size_t ring = 4 * (size_t)BT * (128 * 128 / BT + 16);
+    const size_t ring = sizeof(T) == 4 ? 2 * (size_t)BT * (128 * 192 / BT + 16) : 4 * (size_t)BT * (128 * 128 / BT + 16);
     size_t ct = (size_t)BT * (BT * sizeof(OT) + 16);
     const size_t smem = ring > ct ? ring : ct;
     static FfkLdsReservation lds_reserved;
@@ -335,23 +412,27 @@ int launch_tile(const ffk_bgemm_desc& d, hipStream_t st) {
     return ffk_check_launch("ffk_bgemm_nt");
 }
 
-// Which tile: the launch takes about  start + rounds * (each + per_k * K)  microseconds, rounds = tiles / 256 CUs rounded up.  The
-// constants are fitted to measured launches of 32 .. 24 576 rows, 32 .. 5 120 columns and K = 16 .. 1 024: a small tile pays its
-// latencies over less work, but a large one leaves CUs without a tile (fp32, 2 048 x 256, K = 1 024: 81 us with 16 tiles of 128,
-// 28 us with 128 of 64, 18.7 us with 512 of 32; bf16: 14.0 us with 16 of 256 x 128, 9.8 us with 128 of 64) or works on padding
-// (128 products of 64 x 64 x 64 in fp32: 12.4, 5.7, 6.3 us).  0: the large tiles of the other kernel, if it takes the launch.
+// Which tile: the launch takes about  start + rounds * (each + per_k * K)  microseconds, rounds = tiles / 256 CUs.  The constants are
+// fitted to measured launches of 32 .. 65 536 rows, 32 .. 8 192 columns and K = 16 .. 1 024: a small tile pays its latencies over less
+// work, but a large one leaves CUs without a tile or works on padding.  bf16, rounds rounded up: 2 048 x 256, K = 1 024 14.0 us with 16
+// tiles of 256 x 128, 9.8 us with 128 of 64.  fp32, where the start grows with K and two or three of the smaller tiles share a CU (128 /
+// 64 / 32, us): 4 096 x 128, K = 1 024 75 / 30 / 20.7; 9 000 rows 76 / 37 / 40; 13 689 76 / 41 / 56; 65 536 114 / 148 / 219; K = 512, 4 096 rows
+// 41 / 17.6 / 12.5, 16 384 44 / 24.5 / 34, 65 536 59 / 77 / 121; 128 products of K = 64, 64 x 64: 12.2 / 5.7 / -, of 256 x 256 x 256
+// 36 / 45 / -.  0: the large tiles of the other kernel, if it takes the launch.
 int pick_tile(const ffk_bgemm_desc& d, bool large) {
-    auto cost = [&](int bm, int bn, double start, double each, double per_k) {
-        return start + ffk_cdiv((long)ffk_cdiv(d.M, bm) * ffk_cdiv(d.N, bn) * d.batch, 256) * (each + per_k * d.K);
-    };
-    const bool f = d.dtype == FFK_F32;
-    const double c128 = f ? cost(128, 128, 2.0, 6.8, 0.0645) : cost(128, 128, 3.5, 5.0, 0.0060);
-    const double c64 = f ? cost(64, 64, 3.0, 2.3, 0.0182) : cost(64, 64, 3.0, 1.9, 0.0035);
-    if (large && (c64 >= c128 || c64 >= cost(256, d.N <= 128 ? 128 : 256, 4.7, 0.0, 0.0095))) return 0;
-    if (f && d.K >= BG_QUARTERS) {
-        const double c32 = cost(32, 32, 2.5, 2.1, 0.0060);
-        if (c32 < c64 && c32 < c128) return 32;
+    auto tiles = [&](int bm, int bn) { return (long)ffk_cdiv(d.M, bm) * ffk_cdiv(d.N, bn) * d.batch; };
+    if (d.dtype == FFK_F32) {
+        auto rounds = [&](int t) { return std::max(1.0, tiles(t, t) / 256.0); };
+        const double c128 = 8.0 + 0.0245 * d.K + ffk_cdiv(tiles(128, 128), 256) * (2.0 + 0.04 * d.K);
+        const double c64 = 3.0 + 0.009 * d.K + rounds(64) * (0.5 + 0.0165 * d.K);
+        const double c32 = 3.0 + 0.005 * d.K + rounds(32) * (0.6 + 0.0059 * d.K);
+        return d.K >= BG_QUARTERS && c32 < c64 && c32 < c128 ? 32 : c64 < c128 ? 64 : 128;
     }
+    auto cost = [&](int bm, int bn, double start, double each, double per_k) {
+        return start + ffk_cdiv(tiles(bm, bn), 256) * (each + per_k * d.K);
+    };
+    const double c128 = cost(128, 128, 3.5, 5.0, 0.0060), c64 = cost(64, 64, 3.0, 1.9, 0.0035);
+    if (large && (c64 >= c128 || c64 >= cost(256, d.N <= 128 ? 128 : 256, 4.7, 0.0, 0.0095))) return 0;
     return c64 < c128 ? 64 : 128;
 }
 

@@ -326,6 +326,50 @@ template <> struct Mma<float> {
     static __device__ __forceinline__ Frag ld(const float* p) { return *reinterpret_cast<const Frag*>(p); }
 };
 
+// fp32 products on the bf16 matrix pipe.  An fp32 number is the sum of three bf16 numbers of eight bits each, cut off one after
+// the other (x = x1 + x2 + x3 exactly, but for what lies below the smallest normal number), and
+//     x y = x1 y3 + x3 y1 + x2 y2 + x1 y2 + x2 y1 + x1 y1      up to 2^-24 |x y|,
+// added from the smallest to the largest term in the fp32 accumulator.  Six v_mfma_f32_32x32x16_bf16 take 196 cycles for a K step of 16,
+// eight v_mfma_f32_32x32x2_f32 512, and the bf16 ones let the vector instructions of other waves run beside them.  Relative error
+// (2-norm) of 32 x 32 sums of K products of normal numbers against float64, fp32 instructions -> this:  K = 64 1.6e-7 -> 1.3e-7,
+// 128 2.0e-7 -> 1.8e-7, 256 2.9e-7 -> 2.5e-7, 512 3.8e-7 -> 3.3e-7, 1 024 5.7e-7 -> 4.8e-7; of positive numbers 1.3e-7 -> 1.0e-7 and
+// 5.0e-7 -> 5.0e-7: sixteen products are added per rounding of the accumulator, not two.  The
+// parts of an infinite operand make NaN of its products: a kernel that finds one in its sums takes the fp32 instructions for them.
+struct Split4 {              // four numbers, part by part
+    u32x2 p[3];
+};
+__device__ __forceinline__ Split4 split4(const f32x4& x, uint32_t mask = 0xFFFF0000u, uint32_t high = 0x07060302u) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    Split4 r;
+    const u32x4 b = __builtin_bit_cast(u32x4, x);
+    float q[4];
+    uint32_t m[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {        // (what is left by a dot product with -1 instead of the mask and a subtraction: no faster)
+        const uint32_t h = b[i] & mask;
+        const float r1 = x[i] - __builtin_bit_cast(float, h);
+        m[i] = __builtin_bit_cast(uint32_t, r1);
+        const uint32_t h1 = m[i] & mask;
+        q[i] = r1 - __builtin_bit_cast(float, h1);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        r.p[0][j] = __builtin_amdgcn_perm(b[2 * j + 1], b[2 * j], high);
+        r.p[1][j] = __builtin_amdgcn_perm(m[2 * j + 1], m[2 * j], high);
+        r.p[2][j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{q[2 * j], q[2 * j + 1]}, bf16x2));
+    }
+    return r;
+}
+// eight numbers: part p as a fragment
+__device__ __forceinline__ bf16x8 split_frag(const Split4& a, const Split4& b, int p) {
+    return __builtin_bit_cast(bf16x8, u32x4{a.p[p][0], a.p[p][1], b.p[p][0], b.p[p][1]});
+}
+// the number whose parts these are; an infinite one has parts that are no numbers
+__device__ __forceinline__ float split_sum(float a, float b, float c) { return a - a == 0.0f ? a + b + c : a; }
+// The parts of a product in the order they are added: operand a's part, operand b's
+constexpr int SPLIT_A[6] = {0, 2, 1, 0, 1, 0}, SPLIT_B[6] = {2, 0, 1, 1, 0, 0};
+
 // Row of the 32x32 accumulator tile held in register v by lane `lane`.
 __device__ __forceinline__ int acc_row(int v, int lane) { return 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3); }
 

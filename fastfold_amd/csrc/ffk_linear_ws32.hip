@@ -1,39 +1,43 @@
 // Weights-stationary variant of the fused linear layer in fp32 (see ffk_fused_linear in include/ffk.h), K = 128 or 256.
 //
-// v_mfma_f32_32x32x2_f32 does 64 multiply-adds per cycle and SIMD, and it does not overlap with vector instructions of other
-// waves (a SIMD given 491 us of one and 617 us of the other takes 1 050 us; with bf16 products they hide each other).  So what
-// bounds a launch is products plus vector instructions, and the kernel is arranged to need few of the latter per product: a
-// row is normalised once for up to 16 weight units of 32 rows, weights stay in registers (two units per wave at K = 128, value
-// and gate of a GLU unit, one at K = 256), activations stream through a double-buffered slab of 64 rows in LDS whose 16-byte
-// fragments feed four products each, and a wave stores its blocks straight from registers (exchanging pieces between lanes
-// for wider stores cost 30 % of the launch).  Measured against the LDS-staged kernel: 32 768 rows, 256 -> 1 024: 263 -> 168 us
-// (102 TFLOP/s); 65 536 rows, 128 -> 1 024: 234 -> 181 us; 128 -> 128: 42.5 -> 39.7 us.
+// Products are six bf16 products of the operands' parts (split4): 196 cycles for a 32 x 32 block and a K step of 16, where
+// v_mfma_f32_32x32x2_f32 takes 512 and no vector instruction of another wave runs beside it.  Rows are cut once, behind their
+// LayerNorm and on the way to LDS, for up to eight weight units of 32 rows; weights stay in registers, at K = 128 as parts (96
+// registers a unit), else (GLU units, K = 256) as they are and cut for every use, one step ahead of the products where the registers
+// allow.  Against the fp32 instructions, us: 65 536 rows, 128 -> 1 024 173 -> 135, 128 -> 512 91 -> 70, 128 -> 128 34 -> 26, GLU 256 + 128
+// channels 134 -> 100; 32 768 rows, 256 -> 1 024 161 -> 122, 256 -> 256 52 -> 36; 4 096 rows, 128 -> 512 12.4 -> 10.4.  A launch of
+// 65 536 rows, 128 -> 512, is 35 us of memory traffic, 23 us of products and as many of vector instructions, which overlap in part:
+// without its stores it takes 52 us, without its products 55.  Stores go through LDS, 128 bytes of eight lanes side by side (by a lane's own
+// 16-byte pieces: 91 us), and the upper four waves prepare the next slab ahead of their products, the lower four behind them (all
+// behind: 2 to 4 % more).
 //
 // Persistent workgroups of eight waves, one per CU: the units of a launch are dealt to groups (blockIdx.y), each with workgroups of
-// its own over all rows; unit i of a group goes to wave i % 8, or, in a group of up to four, to waves i and i + 4, which take one
-// half of the slab each - so the SIMDs have equal shares of any multiple of four units.  Few rows take workgroups of four waves
-// with one slab and one unit per wave (ONE): what such a launch waits for is the weights, which come as whole lines while the rows
-// are normalised, and the residual, which is requested before the products.  1 024 rows, 256 -> 256: 21.5 us on the staged
-// kernel, 10.8 us; 4 096 rows, 128 -> 128 from channel-major rows: 20.6 -> 9.7 us.
+// its own over all rows; unit i of a group goes to wave i % 8, or, in a group of up to four with slabs of 64 rows, to waves i and i + 4,
+// which take one half of the slab each - so the SIMDs have equal shares of any multiple of four units.  Few rows, GLU units and
+// channel-major rows take workgroups of four waves with one slab and one unit per wave (ONE): what few rows wait for is the weights, which
+// come as whole lines while the rows are normalised, and the residual, which is requested before the products.
 //   by rows   (plain, q / k tiles, pair-bias tiles): product W . A^T, a lane owns one row and 16 consecutive channels
 //             (64 bytes; weight rows are taken through tau, except for accumulator-order tiles)
 //   by columns (v tiles, channel-major outputs): A . W^T, a lane owns one channel and 16 rows
 #include "ffk_common.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace {
 
 constexpr int W3_MAXU = FFK_MAX_TILES * 4, W3_CUS = 256;
 
-// ONE: every workgroup has one slab of BM rows; else workgroups are persistent and the slab is double-buffered
+// ONE: every workgroup has one slab of BM rows; else workgroups are persistent and the slab is double-buffered (32 rows at K = 256, else 64)
 template <int K, bool GLU, bool ONE, int BM_> struct W3Geo {
     static constexpr int WAVES = ONE ? 4 : 8, THREADS = 64 * WAVES, BM = BM_, RG = BM / 32;
-    static constexpr int KF = K / 8;                     // fragments (four MFMAs each) per unit
-    static constexpr int AP = K * 4 + 16;                // LDS row pitch in bytes
+    static constexpr int KF = K / 8;                     // 16-byte pieces per unit and lane, two to a K step of 16
+    static constexpr int AP = K * 6 + 16;                // LDS row pitch in bytes: [K step of 16][part][16] (see split4)
+    static constexpr int OP = 65 * 64 + 64 * 8;          // LDS of a wave's outputs
     static constexpr int LPR = K / 4;                    // lanes per row
     static constexpr int RPP = THREADS / LPR;            // rows fetched per pass
     static constexpr int NP = BM / RPP;                  // passes: 4, 8 or 16
-    static constexpr int SLOTS = K == 128 && (GLU || !ONE) ? 2 : 1;       // weight units in a wave's registers
+    static constexpr int SLOTS = GLU ? 2 : 1;            // weight units in a wave's registers
+    static constexpr bool CUT = K == 128 && !GLU;        // the weights' parts in the registers, not the weights
     static constexpr int NBUF = ONE ? 1 : 2;
 };
 
@@ -55,15 +59,16 @@ template <bool GLU> __device__ __forceinline__ int w3_sub(const ffk_tile& t, int
 // GLU: the launch has GLU tiles; the slots of a wave are then value and gate of one unit (a plain unit leaves the second empty)
 // CM: element (m, k) of the operand at a + k * a_cs + rowoffset(m) (ONE only)
 template <int K, bool GLU, bool ONE, int BM, bool CM>
-__global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W3Args args) {
+__global__ __launch_bounds__(ONE ? 256 : 512, K == 128 && !GLU && BM == 32 ? 3 : 2) void linear_ws32_kernel(const W3Args args) {
     typedef W3Geo<K, GLU, ONE, BM> G;
-    constexpr int NS = G::SLOTS, KF = G::KF, AP = G::AP, LPR = G::LPR, RPP = G::RPP, NP = G::NP, PF = 3;
+    constexpr int NS = G::SLOTS, KF = G::KF, AP = G::AP, LPR = G::LPR, RPP = G::RPP, NP = G::NP;
     constexpr int W3_WAVES = G::WAVES, W3_RG = G::RG;
     const ffk_linear_desc& d = args.d;
     extern __shared__ __align__(16) unsigned char smem[];
     unsigned char* s_a = smem;                                                  // [NBUF][BM][AP]
-    float* s_mask = reinterpret_cast<float*>(smem + G::NBUF * BM * AP);         // [NBUF][BM]
-    float* s_bias = s_mask + G::NBUF * BM;                                            // [wave][slot][32]
+    unsigned char* s_out = smem + G::NBUF * BM * AP;                            // [wave][OP]
+    float* s_mask = reinterpret_cast<float*>(s_out + G::WAVES * G::OP);         // [parity of the slab][BM]
+    float* s_bias = s_mask + 2 * BM;                                            // [wave][slot][32]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
@@ -125,8 +130,8 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
     float tb[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int i = halves ? wave % (W3_WAVES / W3_RG) : wave + (GLU ? 0 : s * W3_WAVES);
-        int u = i < n_u && !(halves && s && !GLU) ? args.unit[u0 + i] : -1;
+        const int i = halves ? wave % (W3_WAVES / W3_RG) : wave;
+        int u = i < n_u ? args.unit[u0 + i] : -1;
         if (GLU && s) u = u >= 0 && d.tiles[u >> 2].glu ? u + 1 : -1;
         units[s] = u;
         const ffk_tile& t = d.tiles[u >= 0 ? u >> 2 : 0];
@@ -147,9 +152,18 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
                 *reinterpret_cast<f32x4*>(stage + i * 1024 + (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 3)) * 16)) = wf[s][p + i];
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                wf[s][p + i] = *reinterpret_cast<const f32x4*>(stage + wl * 128 + (((2 * i + half) ^ (wl & 7)) * 16));
+                wf[s][p + i] = *reinterpret_cast<const f32x4*>(stage + wl * 128 + (((4 * (i >> 1) + 2 * half + (i & 1)) ^ (wl & 7)) * 16));
         }
         if (half == 0) s_bias[(wave * NS + s) * 32 + l32] = tb[s];
+    }
+    bf16x8 wp[G::CUT ? KF / 2 : 1][3];
+    if constexpr (G::CUT) {
+#pragma unroll
+        for (int g = 0; g < KF / 2; ++g) {
+            const Split4 a = split4(wf[0][2 * g]), b = split4(wf[0][2 * g + 1]);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) wp[g][p] = split_frag(a, b, p);
+        }
     }
     lds_barrier();                                       // every wave is done with the staging area
     const int n32 = args.row_perm ? ffk_tau(l32) : l32;
@@ -159,23 +173,26 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
         gam = *reinterpret_cast<const f32x4*>((const float*)d.ln_gamma + c4 * 4);
         bet = *reinterpret_cast<const f32x4*>((const float*)d.ln_beta + c4 * 4);
     }
-    auto commit = [&](int buf) __attribute__((always_inline)) {
-        unsigned char* sa = s_a + buf * (BM * AP);
+    auto commit = [&](int buf) __attribute__((always_inline)) {        // buf: parity of the slab
+        unsigned char* sa = s_a + (G::NBUF == 2 ? buf : 0) * (BM * AP);
         if constexpr (CM) {                              // transposed through LDS; rows are whole only there
 #pragma unroll
             for (int i = 0; i < 4 * NP; ++i)
                 *reinterpret_cast<float*>(sa + (tid & (BM - 1)) * AP + (tid / BM + i * (G::THREADS / BM)) * 4) = pre[i >> 2][i & 3];
-            if (rm && tid < BM) s_mask[buf * BM + tid] = pm;
-            if (!ln) return;
             lds_barrier();
 #pragma unroll
             for (int i = 0; i < NP; ++i) pre[i] = *reinterpret_cast<const f32x4*>(sa + (r0 + RPP * i) * AP + c4 * 16);
+            lds_barrier();
         }
 #pragma unroll
         for (int i = 0; i < NP; i += 4) {
             if (ln) ffk_ln_rows4<LPR>(pre + i, gam, bet, d.ln_eps);
 #pragma unroll
-            for (int j = i; j < i + 4; ++j) *reinterpret_cast<f32x4*>(sa + (r0 + RPP * j) * AP + c4 * 16) = pre[j];
+            for (int j = i; j < i + 4; ++j) {
+                const Split4 x = split4(pre[j]);
+#pragma unroll
+                for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(sa + (r0 + RPP * j) * AP + (c4 >> 2) * 96 + p * 32 + (c4 & 3) * 8) = x.p[p];
+            }
         }
         if (rm && tid < BM) s_mask[buf * BM + tid] = pm;
     };
@@ -257,19 +274,32 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
         }
         // row of this lane (by rows), of its key tile (V) or first of its sixteen (channel-major: they never straddle `inner`)
         const int mrow = m0g + (by_rows ? n32 : t.kind == FFK_TILE_V ? 0 : 16 * half);
-        if (mrow >= M) return;
         unsigned hi = 0, lo = (unsigned)mrow;
         if (t.inner < M) {
             hi = lo / inner;
             lo -= hi * inner;
         }
+        // The 64 bytes of every lane (null: none), four lanes side by side: by a lane's own 16-byte pieces every 64 bytes are four
+        // requests to L2, and they, not the products, bound the launch.
         auto put = [&](float* p) __attribute__((always_inline)) {
+            unsigned char* to = s_out + wave * G::OP;
 #pragma unroll
-            for (int a = 0; a < 4; ++a) *reinterpret_cast<f32x4*>(p + 4 * a) = f32x4{x[4 * a], x[4 * a + 1], x[4 * a + 2], x[4 * a + 3]};
+            for (int a = 0; a < 4; ++a)
+                *reinterpret_cast<f32x4*>(to + (lane + half) * 64 + ((a ^ (lane >> 2)) & 3) * 16) = f32x4{x[4 * a], x[4 * a + 1], x[4 * a + 2], x[4 * a + 3]};
+            *reinterpret_cast<float**>(to + 65 * 64 + lane * 8) = p;
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {                // rows (channels) 8 j .. 8 j + 7 and their other sixteen values
+                const int h = lane >> 2 & 1, from = 8 * j + (lane >> 3) + 32 * h;
+                const f32x4 y = *reinterpret_cast<const f32x4*>(to + (from + h) * 64 + ((lane ^ (from >> 2)) & 3) * 16);
+                float* q = *reinterpret_cast<float* const*>(to + 65 * 64 + from * 8);
+                if (q) *reinterpret_cast<f32x4*>(q + 4 * (lane & 3)) = y;
+            }
+            __builtin_amdgcn_wave_barrier();
         };
         if (t.kind == FFK_TILE_BIAS) {
             float* p = out + (long)(hi >> 5) * t.s_o + (long)(lo >> 5) * 1024 + qk_tile_off((int)(lo & 31), (int)(hi & 31));
-            if (half == 0) {
+            if (half == 0 && mrow < M) {
 #pragma unroll
                 for (int v = 0; v < 16; ++v)
                     if (v < t.ncols) p[(long)v * t.s_h] = x[v];
@@ -278,15 +308,15 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
         }
         out += (long)hi * t.s_o;
         if (t.kind != FFK_TILE_STRIDED) {
-            put(out + (long)(lo >> 5) * 1024 + (t.kind == FFK_TILE_QK ? half * 512 + (int)(lo & 31) * 16 : (half * 32 + (by_rows ? (int)(lo & 31) : l32)) * 16));
+            put(mrow >= M ? nullptr : out + (long)(lo >> 5) * 1024 + (t.kind == FFK_TILE_QK ? half * 512 + (int)(lo & 31) * 16 : (half * 32 + (by_rows ? (int)(lo & 31) : l32)) * 16));
             return;
         }
         if (!by_rows) {
-            if (l32 < left) put(out + lo + (long)l32 * t.s_d);
+            put(l32 < left && mrow < M ? out + lo + (long)l32 * t.s_d : nullptr);
             return;
         }
         const long off = (long)lo * t.s_i + 16 * half;
-        if (t.gate) {
+        if (t.gate && mrow < M) {
             const float* gate = (const float*)t.gate + (long)(t.gate_rows > 0 ? mrow % t.gate_rows : mrow) * t.gate_ld + 32 * sub + 16 * half;
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
@@ -296,7 +326,7 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
                 for (int e = 0; e < 4; ++e) x[4 * a + e] *= gate_factor(g[e], t.act);
             }
         }
-        if (t.resid) {
+        if (t.resid && mrow < M) {
             [[maybe_unused]] const float* r = (const float*)t.resid + (out - (float*)t.out) + off;
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
@@ -309,9 +339,10 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
             }
         }
         if (left >= 32) {
-            put(out + off);
+            put(mrow < M ? out + off : nullptr);
             return;
         }
+        if (mrow >= M) return;
 #pragma unroll
         for (int a = 0; a < 4; ++a) {                    // ncols is a multiple of 4
             if (16 * half + 4 * a >= left) break;
@@ -319,92 +350,185 @@ __global__ __launch_bounds__(ONE ? 256 : 512, 2) void linear_ws32_kernel(const W
         }
     };
 
-    // products of one row group with slots S0 .. S0 + N - 1, rows: W . A^T
-    auto products = [&](f32x16* acc, const unsigned char* ap, auto rows, auto s0, auto n) __attribute__((always_inline)) {
+    // products of R row groups with the first N slots, rows: W . A^T.  The weights are cut into their parts as they are used.
+    auto products = [&](f32x16* acc, const unsigned char* ap, auto rows, auto n, auto rt) __attribute__((always_inline)) {
+        constexpr int N = decltype(n)::value, R = decltype(rt)::value;
+        // constants the compiler cannot follow: it would cut all weights ahead of the loop over slabs, and their parts do not fit
+        // in the registers
+        uint32_t mask = 0xFFFF0000u, high = 0x07060302u;
+        asm volatile("" : "+s"(mask), "+s"(high));
 #pragma unroll
-        for (int s = 0; s < n.value; ++s)
+        for (int s = 0; s < N * R; ++s)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[s][v] = 0.0f;
-        f32x4 af[PF];                                    // fragments in flight
+        constexpr bool AHEAD = N * R == 1;     // the next step's operands are read and cut beside this step's products
+        bf16x8 xf[2][R][3], w[2][N][3];
+        auto rows_at = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
-        for (int f = 0; f < PF; ++f) af[f] = *reinterpret_cast<const f32x4*>(ap + f * 32);
-        __builtin_amdgcn_sched_group_barrier(0x100, PF, 0);
+            for (int i = 0; i < R; ++i)
 #pragma unroll
-        for (int f = 0; f < KF; ++f) {
-            const f32x4 x = af[f % PF];
+                for (int p = 0; p < 3; ++p) xf[g & 1][i][p] = *reinterpret_cast<const bf16x8*>(ap + i * 32 * AP + g * 96 + p * 32);
+        };
+        auto weights_at = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+            for (int s = 0; s < N; ++s) {
+                if constexpr (G::CUT) {
 #pragma unroll
-                for (int s = 0; s < n.value; ++s) {
-                    const float w = wf[s0.value + s][f][e];
-                    if constexpr (rows.value) acc[s] = __builtin_amdgcn_mfma_f32_32x32x2f32(w, x[e], acc[s], 0, 0, 0);
-                    else acc[s] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], w, acc[s], 0, 0, 0);
+                    for (int p = 0; p < 3; ++p) w[g & 1][s][p] = wp[g][p];
+                    continue;
                 }
-            __builtin_amdgcn_sched_group_barrier(0x008, 4 * n.value, 0);
-            if (f + PF < KF) {
-                af[f % PF] = *reinterpret_cast<const f32x4*>(ap + (f + PF) * 32);
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                const Split4 a = split4(wf[s][2 * g], mask, high), b = split4(wf[s][2 * g + 1], mask, high);
+#pragma unroll
+                for (int p = 0; p < 3; ++p) w[g & 1][s][p] = split_frag(a, b, p);
             }
+        };
+        if (AHEAD) {
+            rows_at(0);
+            weights_at(0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int g = 0; g < K / 16; ++g) {
+            if (!AHEAD) {
+                rows_at(g);
+                weights_at(g);
+            } else if (g + 1 < K / 16) {
+                rows_at(g + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                weights_at(g + 1);
+            }
+#pragma unroll
+            for (int t = 0; t < 6; ++t)
+#pragma unroll
+                for (int s = 0; s < N; ++s)
+#pragma unroll
+                    for (int i = 0; i < R; ++i) {
+                        if constexpr (rows.value) Mma<bf16_t>::mma(acc[s * R + i], w[g & 1][s][SPLIT_A[t]], xf[g & 1][i][SPLIT_B[t]]);
+                        else Mma<bf16_t>::mma(acc[s * R + i], xf[g & 1][i][SPLIT_B[t]], w[g & 1][s][SPLIT_A[t]]);
+                        if (AHEAD && !G::CUT) {
+                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+                        }
+                    }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // infinite operands, whose parts make NaN of every product: with the fp32 instructions
+        float sum = acc[0][0];
+#pragma unroll
+        for (int v = 1; v < 16 * N * R; ++v) sum += acc[v >> 4][v & 15];
+        if (__builtin_expect(__any(sum - sum != 0.0f), 0)) {
+#pragma unroll
+            for (int s = 0; s < N; ++s)
+#pragma unroll
+                for (int i = 0; i < R; ++i) {
+                    f32x16& y = acc[s * R + i];
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) y[v] = 0.0f;
+#pragma unroll
+                    for (int g = 0; g < K / 16; ++g) {
+                        const unsigned char* xp = ap + i * 32 * AP + g * 96;
+                        [[maybe_unused]] bf16x8 wq[3];
+                        if constexpr (G::CUT) {
+#pragma unroll
+                            for (int p = 0; p < 3; ++p) {
+                                u32x4 q = __builtin_bit_cast(u32x4, wp[g][p]);
+                                asm volatile("" : "+v"(q));      // whatever is made of it stays here
+                                wq[p] = __builtin_bit_cast(bf16x8, q);
+                            }
+                        }
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+                            const float x = split_sum(reinterpret_cast<const bf16_t*>(xp)[e], reinterpret_cast<const bf16_t*>(xp + 32)[e], reinterpret_cast<const bf16_t*>(xp + 64)[e]);
+                            float w;
+                            if constexpr (G::CUT) w = split_sum(wq[0][e], wq[1][e], wq[2][e]);
+                            else w = wf[s][2 * g + (e >> 2)][e & 3];
+                            if constexpr (rows.value) y = __builtin_amdgcn_mfma_f32_32x32x2f32(w, x, y, 0, 0, 0);
+                            else y = __builtin_amdgcn_mfma_f32_32x32x2f32(x, w, y, 0, 0, 0);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
         }
     };
-    // One row group against one unit.  With the last one of a slab the next slab comes: its loads are issued before the products
+    const int nslabs = (M + BM - 1) / BM;
+    const bool early = !ONE && wave >= G::WAVES / 2;
+    // R row groups against one unit.  With the last ones of a slab the next slab comes: its loads are issued before the products
     // and normalised and written to LDS after them, ahead of this block's stores - a wait for loads is a wait for the stores
-    // issued after them.
-    auto block = [&](int u, const unsigned char* ap, int m0g, const float* sm, auto s0, auto n, int next, int nbuf) __attribute__((always_inline)) {
-        f32x16 acc[n.value];
-        f32x4 rv[4];
+    // issued before them.  The waves of `early` do that ahead of the products, with loads of the iteration before, so that the two
+    // waves of a SIMD are not at their vector instructions at the same time.
+    auto block = [&](int u, const unsigned char* ap, int m0g, const float* sm, auto n, auto rt, int next, int nbuf) __attribute__((always_inline)) {
+        constexpr int N = decltype(n)::value, R = decltype(rt)::value;
+        f32x16 acc[N * R];
+        f32x4 rv[R][4];
         if constexpr (ONE) {                             // the residual arrives behind the products
             const ffk_tile& t = d.tiles[u >> 2];
-            const int sub = w3_sub<GLU>(t, u), mrow = m0g + n32, left = t.ncols - 32 * sub;
-            if (t.resid && mrow < M) {
-                const unsigned hi = t.inner < M ? (unsigned)mrow / (unsigned)t.inner : 0u, lo = (unsigned)mrow - hi * (unsigned)t.inner;
-                const float* r = (const float*)t.resid + (long)sub * t.s_h + (long)hi * t.s_o + (long)lo * t.s_i + 16 * half;
+            const int sub = w3_sub<GLU>(t, u), left = t.ncols - 32 * sub;
 #pragma unroll
-                for (int a = 0; a < 4; ++a)
-                    if (16 * half + 4 * a < left) rv[a] = *reinterpret_cast<const f32x4*>(r + 4 * a);
+            for (int i = 0; i < R; ++i) {
+                const int mrow = m0g + 32 * i + n32;
+                if (t.resid && mrow < M) {
+                    const unsigned hi = t.inner < M ? (unsigned)mrow / (unsigned)t.inner : 0u, lo = (unsigned)mrow - hi * (unsigned)t.inner;
+                    const float* r = (const float*)t.resid + (long)sub * t.s_h + (long)hi * t.s_o + (long)lo * t.s_i + 16 * half;
+#pragma unroll
+                    for (int a = 0; a < 4; ++a)
+                        if (16 * half + 4 * a < left) rv[i][a] = *reinterpret_cast<const f32x4*>(r + 4 * a);
+                }
             }
         }
-        if (next >= 0) fetch(next);
-        if (w3_by_rows(d.tiles[u >> 2])) products(acc, ap, std::true_type{}, s0, n);
-        else products(acc, ap, std::false_type{}, s0, n);
-        if (next >= 0) commit(nbuf);
-        store(u, s_bias + (wave * NS + s0.value) * 32, acc[0], acc[n.value - 1], m0g, sm, rv);
+        if (next >= 0) {
+            if (early) commit(nbuf);
+            const int n2 = early ? next + (int)gridDim.x : next;
+            if (n2 < nslabs) fetch(n2);
+        }
+        if (w3_by_rows(d.tiles[u >> 2])) products(acc, ap, std::true_type{}, n, rt);
+        else products(acc, ap, std::false_type{}, n, rt);
+        if (next >= 0 && !early) commit(nbuf);
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            if (i == 0 || m0g + 32 * i < M)
+                store(u, s_bias + (wave * NS) * 32, acc[i], acc[(N - 1) * R + i], m0g + 32 * i, sm + 32 * i, rv[i]);
     };
 
-    const int nslabs = (M + BM - 1) / BM;
     int slab = blockIdx.x;                               // grid.x <= nslabs
     if (!ONE) fetch(slab);
     commit(0);
     if (!ONE) __builtin_amdgcn_s_waitcnt(0x0f70);        // vmcnt(0): the products of the loop wait for no weights
+    if (early && slab + (int)gridDim.x < nslabs) fetch(slab + gridDim.x);
     lds_barrier();
     int buf = 0;
-    typedef std::integral_constant<int, 0> I0;
     typedef std::integral_constant<int, 1> I1;
+    constexpr int PAIR = GLU ? 1 : W3_RG;                // row groups multiplied together
+    typedef std::integral_constant<int, PAIR> IR;
     for (; slab < nslabs; slab += gridDim.x) {
         const int next = !ONE && slab + (int)gridDim.x < nslabs ? slab + (int)gridDim.x : -1;
+        const int nbuf = buf ^ 1;
         if (units[0] < 0 && next >= 0) {
-            fetch(next);
-            commit(buf ^ 1);
+            if (!early) fetch(next);
+            commit(nbuf);
+            if (early && next + (int)gridDim.x < nslabs) fetch(next + (int)gridDim.x);
         }
-        const int rg_end = halves && wave < W3_WAVES / W3_RG ? 1 : W3_RG;
-        for (int rg = halves ? wave / (W3_WAVES / W3_RG) : 0; rg < rg_end && units[0] >= 0; ++rg) {
-            const int m0g = slab * BM + rg * 32;
-            if (m0g >= M) break;                         // in the last slab only
-            const int nx = rg + 1 == rg_end ? next : -1;
-            const unsigned char* ap = s_a + buf * (BM * AP) + (rg * 32 + n32) * AP + half * 16;
-            const float* sm = s_mask + buf * BM + rg * 32;
-            if constexpr (GLU) {
-                if (units[NS - 1] >= 0) block(units[0], ap, m0g, sm, I0{}, std::integral_constant<int, NS>{}, nx, buf ^ 1);
-                else block(units[0], ap, m0g, sm, I0{}, I1{}, nx, buf ^ 1);
-            } else {
-                block(units[0], ap, m0g, sm, I0{}, I1{}, units[NS - 1] >= 0 && NS == 2 ? -1 : nx, buf ^ 1);
-                if constexpr (NS == 2)
-                    if (units[1] >= 0) block(units[1], ap, m0g, sm, I1{}, I1{}, nx, buf ^ 1);
+        const int m0 = slab * BM;
+        auto rows_of = [&](int rg) { return s_a + (G::NBUF == 2 ? buf : 0) * (BM * AP) + (rg * 32 + n32) * AP + half * 16; };
+        const float* sm = s_mask + buf * BM;
+        const int rg = halves ? wave / (W3_WAVES / W3_RG) : 0;
+        if (units[0] < 0) {
+        } else if (halves && W3_RG > 1) {                // this wave's half of the slab
+            if (m0 + rg * 32 < M) {
+                if (NS == 2 && units[NS - 1] >= 0) block(units[0], rows_of(rg), m0 + rg * 32, sm + rg * 32, std::integral_constant<int, NS>{}, I1{}, next, nbuf);
+                else block(units[0], rows_of(rg), m0 + rg * 32, sm + rg * 32, I1{}, I1{}, next, nbuf);
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < W3_RG; g += PAIR) {
+                if (m0 + g * 32 >= M) break;             // in the last slab only
+                const int nx = g + PAIR == W3_RG ? next : -1;
+                if (NS == 2 && units[NS - 1] >= 0) block(units[0], rows_of(g), m0 + g * 32, sm + g * 32, std::integral_constant<int, NS>{}, IR{}, nx, nbuf);
+                else block(units[0], rows_of(g), m0 + g * 32, sm + g * 32, I1{}, IR{}, nx, nbuf);
             }
         }
         if (next < 0) break;
         lds_barrier();
-        buf ^= 1;
+        buf = nbuf;
     }
 }
 
@@ -424,7 +548,7 @@ bool w3_tile_ok(const ffk_linear_desc& d, const ffk_tile& t) {
 template <int K, bool GLU, bool ONE, int BM, bool CM = false>
 int w3_launch(const W3Args& a, int gx, int groups, hipStream_t st) {
     typedef W3Geo<K, GLU, ONE, BM> G;
-    const size_t smem = G::NBUF * (size_t)BM * G::AP + (G::NBUF * BM + G::WAVES * G::SLOTS * 32) * sizeof(float);
+    const size_t smem = G::NBUF * (size_t)BM * G::AP + G::WAVES * G::OP + (2 * BM + G::WAVES * G::SLOTS * 32) * sizeof(float);
     static FfkLdsReservation lds_reserved;
     const int rc = ffk_reserve_lds(lds_reserved, (const void*)linear_ws32_kernel<K, GLU, ONE, BM, CM>, smem, "ffk_fused_linear");
     if (rc != FFK_OK) return rc;
@@ -466,48 +590,49 @@ int ffk_linear_ws32_try(const ffk_linear_desc* d, hipStream_t st, int* status) {
     if (chan_major && v_tiles) return 0;                 // they need different row orders within a group
     a.row_perm = chan_major ? 1 : 0;
     a.d = *d;
-    // Persistent workgroups of eight waves, or one slab per workgroup of four waves with a unit each (two to four workgroups per CU):
-    // the latter starts sooner, spreads few rows over more CUs and is alone built for channel-major operands.  In microseconds:
-    //   one slab: a start of 2 to 6.5, then for every workgroup of a CU about twice its products, which take 2 048 cycles per 32 x 32
-    //     block of K = 64 (2.05 x for 32 rows, 1.9 x for 64, 1.6 x for 64 rows of GLU units, whose products are twice as many)
-    //   persistent: a start of 7 to 10, then at 1 800 cycles per us, per slab, 2 x 2 048 per 64 x 32 block of K = 64 with four units (one
-    //     per SIMD) as the grain, LayerNorm and staging 12 per row and K = 64, and 3 000 for what is in flight at the slab's
-    //     barrier; fewer groups normalise the rows less often, more groups spread few rows over the CUs.
-    // Measured, staged kernel before / one slab of 32 / of 64 rows / persistent: 2 048 rows, 256 -> 1 024: 28.3 / 18.0 / 19.7 / 19.8 us;
-    // 256 -> 256: 22.5 / 11.2 / 16.3 / 17.2; 4 096 rows, 128 -> 512: 16.9 / 11.8 / 12.9 / 15.2; 36 864 rows 89.6 / 65.0 / 65.9 / 65.5;
-    // 65 536 rows, GLU 256 + 128 channels: - / 166 / 134 / 147; 128 -> 512: - / 102.8 / 108.6 / 95.2.
-    const int nslabs = ffk_cdiv(d->M, 64), kk = d->K / 64;
-    constexpr double US_PER_BLOCK = 2048.0 / 2350;
-    const int quads = ffk_cdiv(a.n_units, 4);
-    const double blk = US_PER_BLOCK * kk * (glu ? 2 : 1);
-    const double c32 = (glu ? 2.0 : 3.5) + ffk_cdiv((long)ffk_cdiv(d->M, 32) * quads, W3_CUS) * blk * 2.05;
-    const double c64 = (glu ? 6.5 : 4.0) + ffk_cdiv((long)nslabs * quads, W3_CUS) * blk * 2 * (glu ? 1.6 : 1.9);
-    const int cap = 8 * (glu || d->K == 256 ? 1 : 2);
+    // Persistent workgroups of eight waves, or one slab per workgroup of four waves with a unit each (two or three workgroups per CU):
+    // the latter starts sooner, spreads few rows over more CUs and is alone built for channel-major operands and for GLU units.  In
+    // microseconds, with a round = one workgroup per CU:
+    //   one slab of 32 rows: K = 128 4 + 3.4 per round (GLU 5 + 5), K = 256 3 + 5.7; of 64 rows (K = 128): 5 + 5.5 per round (GLU
+    //     4 + 7.8), 0.6 of it with fewer units than waves;
+    //   persistent: 8 to 8.5, then per slab (64 rows at K = 128, 32 at K = 256) 1.6 (0.7) and 3.0 (3.2) for every four units: one per SIMD.
+    // Measured, one slab of 32 / of 64 rows / persistent, K = 128: 65 536 rows, 1 024 channels 220 / 179 / 130 us, 512 111 / 91 / 68, 128
+    // 30.7 / 26.6 / 25.9, 32 23.2 / 18.3 / 22.7; 36 864 rows, 512 channels 66 / 54 / 45; 13 689 28.3 / 27.0 / 22.4; 8 192 17.6 / 14.7 / 15.9;
+    // 4 096 10.4 / 11.5 / 12.1; GLU 256 + 128 channels, 65 536 rows 127 / 99 / 146, 8 192 19.8 / 17.8 / 24.8, 4 096 12.5 / 15.3 / 18.2.
+    // K = 256, 1 024 channels: 32 768 rows 186 / - / 122, 8 192 49.5 / - / 36.5, 4 096 26.3 / - / 21.7, 2 048 14.3 / - / 16.1; 256 channels:
+    // 32 768 46.9 / - / 35.2, 8 192 13.4 / - / 14.8.
+    const int quads = ffk_cdiv(a.n_units, 4), sl32 = ffk_cdiv(d->M, 32), sl64 = ffk_cdiv(d->M, 64);
+    const long r32 = ffk_cdiv((long)sl32 * quads, W3_CUS), r64 = ffk_cdiv((long)sl64 * quads, W3_CUS);
+    const double few = a.n_units < 4 ? 0.6 : 1.0;
+    const double c32 = d->K == 256 ? 3 + 5.7 * r32 : glu ? 5 + 5.0 * r32 : 4 + 3.4 * r32;
+    const double c64 = d->K == 256 ? 1e30 : glu ? std::max(15.0, 4 + 7.8 * r64) : std::max(11.0, 5 + 5.5 * few * r64);
     int gx = 1, groups = 1;
     double best = 1e30;
-    for (int per = cap; per >= 4; per -= 4) {
-        const int g = ffk_cdiv(a.n_units, per), each = ffk_cdiv(a.n_units, g);
-        int x = W3_CUS / g;
-        x = x < nslabs ? x : nslabs;
-        const double cost = (d->K == 128 ? 10.0 : 7.0) + ffk_cdiv(nslabs, x) * (ffk_cdiv(each, 4) * 4096.0 * kk * (glu ? 2 : 1) + 64 * 12.0 * kk + 3000.0) / 1800;
-        if (cost < best) {
-            best = cost;
-            gx = x;
-            groups = ffk_cdiv(a.n_units, each);
-            a.per_group = each;
+    if (!glu && !d->a_chanmajor) {
+        const int nslabs = d->K == 256 ? sl32 : sl64;
+        for (int per = 8; per >= 4; per -= 4) {
+            const int g = ffk_cdiv(a.n_units, per), each = ffk_cdiv(a.n_units, g);
+            int x = W3_CUS / g;
+            x = x < nslabs ? x : nslabs;
+            const double grain = ffk_cdiv(each, 4), cost = d->K == 256 ? 8.5 + ffk_cdiv(nslabs, x) * (0.7 + 3.2 * grain) : 8 + ffk_cdiv(nslabs, x) * (1.6 + 3.0 * grain);
+            if (cost < best) {
+                best = cost;
+                gx = x;
+                groups = ffk_cdiv(a.n_units, each);
+                a.per_group = each;
+            }
         }
     }
-    if (d->a_chanmajor || c32 <= best || c64 <= best) {
+    if (c32 <= best || c64 <= best) {
         a.per_group = 4;
         const bool small = c32 <= c64;
-        gx = ffk_cdiv(d->M, small ? 32 : 64);
+        gx = small ? sl32 : sl64;
         if (d->a_chanmajor) *status = small ? w3_launch<128, false, true, 32, true>(a, gx, quads, st) : w3_launch<128, false, true, 64, true>(a, gx, quads, st);
-        else if (d->K == 256) *status = small ? w3_launch<256, false, true, 32>(a, gx, quads, st) : w3_launch<256, false, true, 64>(a, gx, quads, st);
+        else if (d->K == 256) *status = w3_launch<256, false, true, 32>(a, gx, quads, st);
         else if (glu) *status = small ? w3_launch<128, true, true, 32>(a, gx, quads, st) : w3_launch<128, true, true, 64>(a, gx, quads, st);
         else *status = small ? w3_launch<128, false, true, 32>(a, gx, quads, st) : w3_launch<128, false, true, 64>(a, gx, quads, st);
         return 1;
     }
-    if (d->K == 256) *status = w3_launch<256, false, false, 64>(a, gx, groups, st);
-    else *status = glu ? w3_launch<128, true, false, 64>(a, gx, groups, st) : w3_launch<128, false, false, 64>(a, gx, groups, st);
+    *status = d->K == 256 ? w3_launch<256, false, false, 32>(a, gx, groups, st) : w3_launch<128, false, false, 64>(a, gx, groups, st);
     return 1;
 }

@@ -1,0 +1,55 @@
+"""fp32 products as six products of bf16 parts (ffk_fused_linear and ffk_bgemm_nt in fp32) against float64: error bounds, edges of
+the tiles, infinite and undefined operands."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+INF = float("inf")
+
+
+def _run(x, w):
+    from fastfold_amd import _lib
+    from fastfold_amd.model.fastnn import _fused as F_
+    (M, K), N = x.shape, w.shape[0]
+    o = torch.empty(M, N, device=x.device)
+    if K in (128, 256):
+        F_.linear(x, torch.cat([w, w.new_zeros((-N) % 128, K)]), None, N, out=o)
+    else:
+        _lib.bgemm_nt(x, w, o, M=M, N=N, K=K, lda=K, ldb=K, s_i=N)
+    return o.double()
+
+
+# every kernel of the two entry points: one slab of 32 or 64 rows and persistent workgroups; tiles of 32, 64 and 128; K that ends
+# inside a step of 16, and the quarters of K
+SHAPES = [(M, 128, N) for M in (1, 33, 1000) for N in (32, 36, 512)] + [(13689, 128, 512), (20001, 128, 128)] \
+    + [(M, 256, N) for M in (1, 65, 4097) for N in (64, 256)] + [(8200, 256, 1024)] \
+    + [(1, 36, 4), (63, 20, 33), (129, 64, 65), (4000, 40, 300), (33, 512, 128), (300, 1024, 100), (16400, 512, 128), (30000, 1024, 129)]
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+@pytest.mark.parametrize("sx,sw", [(1.0, 1.0), (1e-25, 1e20)])
+def test_error_of_products(dev, M, K, N, sx, sw):
+    g = torch.Generator().manual_seed(M + K + N)
+    x, w = (torch.randn(M, K, generator=g) * sx).to(dev), (torch.randn(N, K, generator=g) * sw).to(dev)
+    got, want, size = _run(x, w), x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    # what is left out of a product: x2 y3 + x3 y2 + x3 y3, at most 2^-23 of it; roundings of the sum: six for a step of 16 and three for
+    # the quarters, each at most 2^-23 (cut off) of the sums of magnitudes
+    err = (got - want).abs()
+    assert bool((err <= (1 + 6 * ((K + 15) // 16) + 3) * 2.0 ** -23 * size).all())
+    # independent roundings add up as a random walk: at most what one rounding of 2^-24 for every product of the sum would give
+    assert float(err.norm() / want.norm()) <= max(K, 32) ** 0.5 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("M,K,N", [(100, 128, 256), (5000, 128, 512), (40000, 128, 512), (100, 256, 256), (20000, 256, 1024),
+                                   (300, 1024, 128), (30000, 512, 128), (300, 64, 64), (3000, 64, 300)])
+def test_infinite_and_undefined_operands(dev, M, K, N):
+    g = torch.Generator().manual_seed(M + K + N)
+    x, w = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g)
+    x[3, 5], x[M // 2, 1], x[M - 1, 0], w[7, 9], w[N - 1, 5] = INF, -INF, float("nan"), INF, -INF
+    x, w = x.to(dev), w.to(dev)
+    got, want = _run(x, w), x.double() @ w.double().t()
+    assert torch.equal(got.isnan(), want.isnan())
+    inf = want.isinf()
+    assert torch.equal(got[inf], want[inf]) and bool(got[want.isfinite()].isfinite().all())
+    ok = want.isfinite()
+    assert float((got[ok] - want[ok]).norm() / want[ok].norm()) <= max(K, 32) ** 0.5 * 2.0 ** -24
