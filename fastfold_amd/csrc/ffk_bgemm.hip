@@ -5,13 +5,16 @@
 // 4 consecutive n of one row m, and the tile is staged through LDS for 16-byte stores.  Three tiles (see launch_tile):
 //   128 x 128, chunks of 128 bytes, 64 x 64 per wave       (four 32 x 32 products per two fragments of each operand)
 //    64 x  64, chunks of 256 bytes, 32 x 32 per wave
-//    32 x  32, chunks of 4 x 128 bytes, each wave takes one quarter of K (fp32, K >= 512)
+//    32 x  32, chunks of 4 x 128 bytes, each wave takes one piece of K in four (fp32, K >= 512)
 // fp32 products are six bf16 products of the operands' parts (split4), which are cut on the way to LDS, one slot of it.  Against the
 // fp32 instructions, us: 128 products of 256 x 256 x 256 48 -> 35, of 384 x 384 x 384 169 -> 108; 65 536 x 128, K = 1 024 149 -> 110,
 // K = 512 80 -> 56; 32 768 x 256, K = 1 024 147 -> 97; 8 192 x 8 192, K = 128 193 -> 141; 4 096 x 128, K = 1 024, where the launch waits for one
 // chunk after the other and cutting lengthens that chain, 17.7 -> 19.1.
 // Every tile gives the same bits (callers cut their rows into pieces as memory allows, and pieces take other tiles): products are
-// added in ascending order of K, for fp32 and K >= 512 within quarters of K, as ((q0 + q1) + q2) + q3.
+// added in ascending order of K, for fp32 and K >= 512 within pieces of K (quarters up to K = 1 024, then 256), the pieces as
+// ((p0 + p1) + p2) + p3 ..  The bf16 instructions cut off what the sum has no room for, towards minus infinity: in long chains, of
+// numbers of one sign above all, that would add up to more than the roundings (K = 8 192 in four pieces 3.3e-6 of the sum), so a
+// piece ends after 256 and every other one has its sign turned.
 #include "ffk_common.h"
 #include <algorithm>
 #include <type_traits>
@@ -19,7 +22,7 @@
 namespace {
 
 constexpr int THREADS = 256;
-constexpr int BG_QUARTERS = 512;                   // K from which fp32 products are added in quarters of K
+constexpr int BG_PIECES = 512;                   // K from which fp32 products are added in pieces of K
 
 template <typename T, typename OT, int BT>
 __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_desc d) {
@@ -31,7 +34,7 @@ __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_de
     constexpr bool XS_OK = std::is_same<OT, bf16_t>::value;     // outputs that may carry a residual tail
     constexpr int WT = BT == 128 ? 2 : 1;          // 32 x 32 blocks per wave and dimension
     constexpr bool KSPLIT = BT == 32;
-    constexpr bool QUARTERS = std::is_same<T, float>::value;    // sums in quarters of K possible
+    constexpr bool PIECES = std::is_same<T, float>::value;    // sums in pieces of K possible
     constexpr int BKB = 128 * 128 / BT;            // bytes of K per row and chunk
     constexpr int BK = BKB / ES;
     // fp32: operands lie in LDS as their three bf16 parts (see split4), [K step of 16][part][16] per row, one slot of each
@@ -68,10 +71,14 @@ __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_de
     const T* A = (const T*)d.a + (long)bz * d.a_bs;
     const T* B = (const T*)d.b + (long)bz * d.b_bs;
 
-    const int kq = QUARTERS && K >= BG_QUARTERS ? (K + 255) / 256 * 64 : K;     // length of a quarter (whole chunks)
+    const int kq = PIECES && K >= BG_PIECES ? (K > 1024 ? 256 : (K + 255) / 256 * 64) : K;     // length of a piece (whole chunks)
+    auto round_of = [&](int kc) { return K > 1024 ? kc >> 3 : 0; };
     auto k_of = [&](int kc, int c) {               // K index of vector c of a chunk row
-        return KSPLIT ? c / (BK / VEC / 4) * kq + kc * (BK / 4) + c % (BK / VEC / 4) * VEC : kc * BK + c * VEC;
+        if (!KSPLIT) return kc * BK + c * VEC;
+        const int round = round_of(kc);            // four pieces at a time
+        return (4 * round + c / (BK / VEC / 4)) * kq + (kc - 8 * round) * (BK / 4) + c % (BK / VEC / 4) * VEC;
     };
+    int piece = 0;                               // finished pieces
     Vec16<T> ra[NV], rb[NV];
     auto fetch = [&](int kc) {
 #pragma unroll
@@ -103,6 +110,10 @@ __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_de
             }
             if constexpr (SPLIT) {
                 const int o = r * P + (c >> 2) * 96 + (c & 3) * 8;
+                const uint32_t sign = K >= BG_PIECES ? (uint32_t)(KSPLIT ? c / (BK / VEC / 4) : piece) << 31 : 0u;
+                u32x4& bits = *reinterpret_cast<u32x4*>(&xa);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bits[e] ^= sign;
                 const Split4 a3 = split4(*reinterpret_cast<const f32x4*>(&xa)), b3 = split4(*reinterpret_cast<const f32x4*>(&xb));
 #pragma unroll
                 for (int p = 0; p < 3; ++p) {
@@ -124,23 +135,40 @@ __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_de
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
 
-    f32x16 sum[QUARTERS && !KSPLIT ? WT : 1][QUARTERS && !KSPLIT ? WT : 1];       // of the finished quarters
-    int quarter = 0;
-    auto end_quarter = [&]() {
+    f32x16 sum[PIECES ? WT : 1][PIECES ? WT : 1];       // of the finished pieces
+    auto end_piece = [&]() {
 #pragma unroll
         for (int a = 0; a < WT; ++a)
 #pragma unroll
             for (int b = 0; b < WT; ++b)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) sum[a][b][v] = quarter ? sum[a][b][v] + acc[a][b][v] : acc[a][b][v];
-        ++quarter;
+                for (int v = 0; v < 16; ++v) sum[a][b][v] = piece == 0 ? acc[a][b][v] : piece & 1 ? sum[a][b][v] - acc[a][b][v] : sum[a][b][v] + acc[a][b][v];
+        ++piece;
     };
-    const int kchunks = KSPLIT ? kq / (BK / 4) : (K + BK - 1) / BK;
+    // KSPLIT: wave 0 adds the four pieces
+    [[maybe_unused]] auto end_round = [&]() {
+        float* red = reinterpret_cast<float*>(smem);
+        if (wave) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) red[((wave - 1) * 16 + v) * 64 + lane] = acc[0][0][v];
+        }
+        lds_barrier();
+        if (wave == 0) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const float p0 = piece ? sum[0][0][v] + acc[0][0][v] : acc[0][0][v];
+                sum[0][0][v] = ((p0 - red[v * 64 + lane]) + red[(16 + v) * 64 + lane]) - red[(32 + v) * 64 + lane];
+            }
+        }
+        lds_barrier();
+        piece = 1;
+    };
+    const int kchunks = KSPLIT ? (K + 4 * kq - 1) / (4 * kq) * (kq / (BK / 4)) : (K + BK - 1) / BK;
     fetch(0);
     for (int kc = 0; kc < kchunks; ++kc) {
-        if constexpr (QUARTERS && !KSPLIT) {
-            if (kc * BK == (quarter + 1) * kq) {
-                end_quarter();
+        if constexpr (PIECES && !KSPLIT) {
+            if (kc * BK == (piece + 1) * kq) {
+                end_piece();
 #pragma unroll
                 for (int a = 0; a < WT; ++a)
 #pragma unroll
@@ -151,6 +179,13 @@ __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_de
         }
         const int slot = kc & (NSLOT - 1);
         if (SPLIT && kc) lds_barrier();            // nobody reads the chunk before any more
+        if constexpr (KSPLIT) {
+            if (kc && kc == 8 * round_of(kc)) {
+                end_round();
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[0][0][v] = 0.0f;
+            }
+        }
         commit(slot, kc);
         lds_barrier();
         if (kc + 1 < kchunks) fetch(kc + 1);
@@ -205,9 +240,9 @@ __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_de
             }
         }
     }
-    if constexpr (QUARTERS && !KSPLIT) {
-        if (quarter) {
-            end_quarter();
+    if constexpr (PIECES && !KSPLIT) {
+        if (piece) {
+            end_piece();
 #pragma unroll
             for (int a = 0; a < WT; ++a)
 #pragma unroll
@@ -215,18 +250,9 @@ __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_de
         }
     }
     lds_barrier();
-    if constexpr (KSPLIT) {                        // wave 0 adds the quarters
-        float* red = reinterpret_cast<float*>(smem);
-        if (wave) {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) red[((wave - 1) * 16 + v) * 64 + lane] = acc[0][0][v];
-        }
-        lds_barrier();
-        if (wave == 0) {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[0][0][v] = ((acc[0][0][v] + red[v * 64 + lane]) + red[(16 + v) * 64 + lane]) + red[(32 + v) * 64 + lane];
-        }
-        lds_barrier();
+    if constexpr (KSPLIT) {
+        end_round();
+        if (wave == 0) acc[0][0] = sum[0][0];
     }
 
     if constexpr (SPLIT) {                         // infinite operands, whose parts make NaN of every product: anew, product by product
@@ -426,7 +452,7 @@ int pick_tile(const ffk_bgemm_desc& d, bool large) {
         const double c128 = 8.0 + 0.0245 * d.K + ffk_cdiv(tiles(128, 128), 256) * (2.0 + 0.04 * d.K);
         const double c64 = 3.0 + 0.009 * d.K + rounds(64) * (0.5 + 0.0165 * d.K);
         const double c32 = 3.0 + 0.005 * d.K + rounds(32) * (0.6 + 0.0059 * d.K);
-        return d.K >= BG_QUARTERS && c32 < c64 && c32 < c128 ? 32 : c64 < c128 ? 64 : 128;
+        return d.K >= BG_PIECES && c32 < c64 && c32 < c128 ? 32 : c64 < c128 ? 64 : 128;
     }
     auto cost = [&](int bm, int bn, double start, double each, double per_k) {
         return start + ffk_cdiv(tiles(bm, bn), 256) * (each + per_k * d.K);

@@ -53,3 +53,13 @@ def test_infinite_and_undefined_operands(dev, M, K, N):
     assert torch.equal(got[inf], want[inf]) and bool(got[want.isfinite()].isfinite().all())
     ok = want.isfinite()
     assert float((got[ok] - want[ok]).norm() / want[ok].norm()) <= max(K, 32) ** 0.5 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("M,K,N", [(40, 2048, 100), (700, 4096, 300), (4000, 4112, 2100), (64, 16384, 40)])
+def test_long_sums_of_one_sign(dev, M, K, N):
+    """What the instructions cut off has the sign of the sum: pieces of 256 with turned signs keep it from adding up."""
+    g = torch.Generator().manual_seed(K)
+    x, w = torch.rand(M, K, generator=g).to(dev), torch.rand(N, K, generator=g).to(dev)
+    got, want = _run(x, w), x.double() @ w.double().t()
+    # one rounding of the sum per piece of 256, at most 2^-24 of it each, adding up as a random walk, and 2^-23 for a piece's own products
+    assert float((got - want).norm() / want.norm()) <= (K / 256) ** 0.5 * 2.0 ** -24 + 2.0 ** -23
