@@ -12,8 +12,10 @@
 //          stores eight columns of eight rows; in LDS a column is 64 rows = 128 bytes, its eight 16-byte chunks XOR-swizzled
 //          with the column index so that neither the stores (columns 8 apart) nor the fragment reads (adjacent columns) meet
 //          in one bank group.  The permutes cost a fifth of the MFMA time.
-//   fp32   v_mfma_f32_32x32x2_f32 takes one element per lane: rows stay as they are.
-// Bound: the reads of y and x (from HBM or the last-level cache), in bf16; the matrix pipe in fp32.  The rows of a step are requested
+//   fp32   rows stay as they are; a lane reads eight rows of its column and cuts them into bf16 parts (split4) for six bf16 products.
+//          Against the fp32 instructions, which the matrix pipe bounded, with
+//          the sums over the slices: 13 689 rows, 640 x 128 42 -> 34 us, 14 976 rows, 1 024 x 256 92 -> 73, 65 536 rows, 512 x 128 95 -> 77.
+// Bound: the reads of y and x (from HBM or the last-level cache), in bf16; the vector instructions of the cuts in fp32.  The rows of a step are requested
 // before the products of the step before it and nothing looks at them in between: the rows past the end of a slice, which have to be
 // zeroed, are a step of their own behind the loop (as conditions of every load they made each step wait for its rows).
 // 65 536 rows, us of the first launch, before and after: 640 x 128 36.9, 26.1, 512 x 128 27.9, 23.5; 32 768 rows, 1 032 x 256 50.7,
@@ -116,9 +118,11 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
         const int c = first + cb * VEC;
         return c < cols ? c : cols - VEC;
     };
-    if (is_x) wy.init((const T*)a.x + column(k0, a.K), m_begin + r0, a.x_inner, a.M, a.x_so, a.x_si);
-    else wy.init((const T*)a.y + column(n0, a.N), m_begin + r0, a.y_inner, a.M, a.y_so, a.y_si);
-    if (!BF) wx.init((const T*)a.x + column(k0, a.K), m_begin + r0, a.x_inner, a.M, a.x_so, a.x_si);
+    auto start = [&]() __attribute__((always_inline)) {
+        if (is_x) wy.init((const T*)a.x + column(k0, a.K), m_begin + r0, a.x_inner, a.M, a.x_so, a.x_si);
+        else wy.init((const T*)a.y + column(n0, a.N), m_begin + r0, a.y_inner, a.M, a.y_so, a.y_si);
+        if (!BF) wx.init((const T*)a.x + column(k0, a.K), m_begin + r0, a.x_inner, a.M, a.x_so, a.x_si);
+    };
     auto fetch_rows = [&](Vec16<T>* pre) __attribute__((always_inline)) {      // a whole step: requests only, nothing waits for them here
         wy.template fetch<NP>(pre);
         if (!BF) wx.template fetch<NP>(pre + (BF ? 0 : NP));
@@ -138,6 +142,7 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
             }
         }
     };
+    [[maybe_unused]] uint32_t sign = (uint32_t)slice << 31;       // fp32: of the piece the next commit belongs to
     auto commit = [&](const Vec16<T>* pre, int buf) __attribute__((always_inline)) {
         unsigned char* sb = smem + buf * 2 * BUF;
         if constexpr (BF) {
@@ -160,7 +165,10 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
         } else {
 #pragma unroll
             for (int e = 0; e < NP; ++e) {
-                *reinterpret_cast<Vec16<T>*>(sb + (rb + 8 * e) * 640 + cb * 16) = pre[e];
+                u32x4 y = *reinterpret_cast<const u32x4*>(&pre[e]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) y[j] ^= sign;
+                *reinterpret_cast<u32x4*>(sb + (rb + 8 * e) * 640 + cb * 16) = y;
                 *reinterpret_cast<Vec16<T>*>(sb + BUF + (rb + 8 * e) * 640 + cb * 16) = pre[(BF ? 0 : NP) + e];
             }
         }
@@ -169,6 +177,7 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
     const int wn = wave >> 1, wk = wave & 1;               // the wave's 64 x 64 quarter of the tile
     const bool sums = a.csum != nullptr && k0 == 0 && wk == 0;
     float cs[2] = {0.0f, 0.0f};
+    [[maybe_unused]] float turn = slice & 1 ? -1.0f : 1.0f;        // fp32: sign of the products of this piece
     f32x16 acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -178,7 +187,7 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
 
     // The products of a step.  The fragments of a K step are requested one K step ahead.
-    auto products = [&](const unsigned char* sy) __attribute__((always_inline)) {
+    auto products = [&](const unsigned char* sy, [[maybe_unused]] auto plain) __attribute__((always_inline)) {
         const unsigned char* sx = sy + BUF;
         if constexpr (BF) {
             bf16x8 fy[2][2], fx[2][2];
@@ -212,8 +221,33 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
                         }
                 }
             }
+        } else if constexpr (!plain.value) {
+#pragma unroll
+            for (int ks = 0; ks < MB / 16; ++ks) {         // rows 16 ks + 8 half .. + 7 of a column per lane
+                bf16x8 fy[2][3];
+                auto cut = [&](bf16x8 (&f)[3], const unsigned char* p, float* c) __attribute__((always_inline)) {
+                    f32x4 x[2];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) x[e >> 2][e & 3] = *reinterpret_cast<const float*>(p + (16 * ks + 8 * half + e) * 640);
+                    const Split4 lo = split4(x[0]), hi = split4(x[1]);
+#pragma unroll
+                    for (int t = 0; t < 3; ++t) f[t] = split_frag(lo, hi, t);
+                    if (c) *c += turn * (((x[0][0] + x[0][1]) + (x[0][2] + x[0][3])) + ((x[1][0] + x[1][1]) + (x[1][2] + x[1][3])));
+                };
+#pragma unroll
+                for (int i = 0; i < 2; ++i) cut(fy[i], sy + (wn * 64 + i * 32 + l32) * 4, sums ? &cs[i] : nullptr);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    bf16x8 fx[3];
+                    cut(fx, sx + (wk * 64 + j * 32 + l32) * 4, nullptr);
+#pragma unroll
+                    for (int t = 0; t < 6; ++t)
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) Mma<bf16_t>::mma(acc[i][j], fy[i][SPLIT_A[t]], fx[SPLIT_B[t]]);
+                }
+            }
         } else {
-#pragma unroll 4
+#pragma unroll 1
             for (int ks = 0; ks < MB / 2; ++ks) {
                 float fy[2], fx[2];
 #pragma unroll
@@ -225,10 +259,6 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
                     for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fy[i], fx[j], acc[i][j], 0, 0, 0);
-                if (sums) {
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) cs[i] += fy[i];
-                }
             }
         }
     };
@@ -236,26 +266,77 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
     constexpr int NV = NP * (BF ? 1 : 2);
     const int whole = (m_end - m_begin) / MB;
     const bool tail = (m_end - m_begin) % MB != 0;
-    {
-        Vec16<T> pre[NV];
-        if (whole > 0) fetch_rows(pre);
-        else fetch_tail(pre, m_begin);
-        commit(pre, 0);
-    }
-    lds_barrier();
-    int buf = 0;
-    auto step = [&](auto tail_c) __attribute__((always_inline)) {          // products of one buffer while the rows of the next are on their way
-        Vec16<T> pre[NV];
-        if constexpr (decltype(tail_c)::value) fetch_tail(pre, m_begin + whole * MB);
-        else fetch_rows(pre);
-        products(smem + buf * 2 * BUF);
-        commit(pre, buf ^ 1);                              // its last readers passed the barrier below
-        lds_barrier();
-        buf ^= 1;
+    // fp32: the sums of every PIECE steps (256 rows) by themselves, and y's sign turned for every other piece and every other slice: the
+    // bf16 instructions cut off towards minus infinity, which in a long chain or the sum of many is more than its roundings.  Relative
+    // error (2-norm), fp32 instructions -> one chain per slice, no turns -> this: 65 536 rows in 64 slices 5.8e-7 -> 6.4e-7 -> 2.6e-7, in 256
+    // 3.2e-7 -> 3.7e-7 -> 2.5e-7.
+    constexpr int PIECE = 8;
+    f32x16 sum[BF ? 1 : 2][BF ? 1 : 2];
+#pragma unroll
+    for (auto& s : sum)
+#pragma unroll
+        for (f32x16& t : s) t = acc[0][0];
+    [[maybe_unused]] auto end_piece = [&]() __attribute__((always_inline)) {
+        if constexpr (!BF) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        sum[i][j][v] = fmaf(turn, acc[i][j][v], sum[i][j][v]);
+                        acc[i][j][v] = 0.0f;
+                    }
+            turn = -turn;
+        }
     };
-    for (int i = 1; i < whole; ++i) step(std::false_type());
-    if (tail && whole > 0) step(std::true_type());
-    products(smem + buf * 2 * BUF);
+    auto walk = [&](auto plain) __attribute__((always_inline)) {
+        start();
+        {
+            Vec16<T> pre[NV];
+            if (whole > 0) fetch_rows(pre);
+            else fetch_tail(pre, m_begin);
+            commit(pre, 0);
+        }
+        lds_barrier();
+        int buf = 0, steps = 1;                            // committed steps
+        auto step = [&](auto tail_c) __attribute__((always_inline)) {      // products of one buffer while the rows of the next are on their way
+            Vec16<T> pre[NV];
+            if constexpr (decltype(tail_c)::value) fetch_tail(pre, m_begin + whole * MB);
+            else fetch_rows(pre);
+            products(smem + buf * 2 * BUF, plain);
+            if (!BF && !plain.value && steps % PIECE == 0) {
+                end_piece();
+                sign ^= 0x80000000u;
+            }
+            ++steps;
+            commit(pre, buf ^ 1);                          // its last readers passed the barrier below
+            lds_barrier();
+            buf ^= 1;
+        };
+        for (int i = 1; i < whole; ++i) step(std::false_type());
+        if (tail && whole > 0) step(std::true_type());
+        products(smem + buf * 2 * BUF, plain);
+        if (!BF && !plain.value) end_piece();
+    };
+    walk(std::false_type());
+    if constexpr (!BF) {                                   // infinite operands, whose parts make NaN of every product: with the fp32 instructions
+        float t = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 64; ++v) t += acc[v >> 5][(v >> 4) & 1][v & 15] = sum[v >> 5][(v >> 4) & 1][v & 15];
+        int* bad = reinterpret_cast<int*>(smem);
+        lds_barrier();
+        if (lane == 0) bad[wave] = 0;
+        if (t - t != 0.0f) bad[wave] = 1;
+        lds_barrier();
+        if (__builtin_expect(bad[0] | bad[1] | bad[2] | bad[3], 0)) {
+            lds_barrier();
+#pragma unroll
+            for (int v = 0; v < 64; ++v) acc[v >> 5][(v >> 4) & 1][v & 15] = 0.0f;
+            sign = 0;
+            walk(std::true_type());
+        }
+    }
     float* part = a.part + (long)slice * a.N * a.K;
 #pragma unroll
     for (int i = 0; i < 2; ++i)

@@ -1,4 +1,4 @@
-"""fp32 products as six products of bf16 parts (ffk_fused_linear and ffk_bgemm_nt in fp32) against float64: error bounds, edges of
+"""fp32 products as six products of bf16 parts (ffk_fused_linear, ffk_bgemm_nt and ffk_weight_grad in fp32) against float64: error bounds, edges of
 the tiles, infinite and undefined operands."""
 import pytest
 import torch
@@ -63,3 +63,27 @@ def test_long_sums_of_one_sign(dev, M, K, N):
     got, want = _run(x, w), x.double() @ w.double().t()
     # one rounding of the sum per piece of 256, at most 2^-24 of it each, adding up as a random walk, and 2^-23 for a piece's own products
     assert float((got - want).norm() / want.norm()) <= (K / 256) ** 0.5 * 2.0 ** -24 + 2.0 ** -23
+
+
+@pytest.mark.parametrize("one_sign", [False, True])
+@pytest.mark.parametrize("M,slices", [(31, 1), (256, 1), (257, 1), (600, 1), (5000, 3), (65536, 64), (65536, 1024)])
+def test_error_of_weight_gradients(dev, M, slices, one_sign):
+    from fastfold_amd import _lib
+    g, N, K = torch.Generator().manual_seed(M), 136, 40
+    y, x = ((torch.rand(M, C, generator=g) if one_sign else torch.randn(M, C, generator=g)).to(dev) for C in (N, K))
+    ws, out, cs = torch.empty(slices * N * (K + 1), device=dev), torch.empty(N, K, device=dev), torch.empty(N, device=dev)
+
+    def run():
+        _lib.weight_grad(out, cs, ws, y, x, M=M, N=N, K=K, slices=slices, dtype=torch.float32, y_map=(M, 0, N), x_map=(M, 0, K))
+        return out.double().cpu(), y.double().cpu().t() @ x.double().cpu()
+    got, want = run()
+    rel = lambda a, b: float((a - b).norm() / b.norm())
+    # as above; the sums over the slices add slices / 4 + 3 roundings
+    walk = (max(M / slices, 256) / 256 + slices / 4 + 3) ** 0.5 * 2.0 ** -24 + 2.0 ** -23
+    assert rel(got, want) <= (walk if one_sign else 16 * 2.0 ** -24 + walk)       # of both signs: a piece's roundings against a sum that stays small
+    assert rel(cs.double(), y.double().sum(0)) <= (M / slices + slices) ** 0.5 * 2.0 ** -24
+    y[M // 2, 5], x[M // 3, 7], x[0, 9] = INF, -INF, float("nan")
+    got, want = run()
+    fin = want.isfinite()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[want.isinf()], want[want.isinf()])
+    assert rel(got[fin], want[fin]) <= (M / slices + slices) ** 0.5 * 2.0 ** -24
