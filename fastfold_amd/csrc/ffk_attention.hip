@@ -459,6 +459,379 @@ __global__ __launch_bounds__(ATT_THREADS, sizeof(T) == 2 ? 4 : 2) void attention
     }
 }
 
+constexpr int PAIR_THREADS = 256;
+
+// bf16 heads of 32 channels with a bias: a wave owns 32 queries of one head in TWO batch rows, two waves per SIMD.  The kernel above
+// takes the sum of its matrix and vector instructions (its waves leave a barrier together and then all wait for scores, all for
+// exp2), although one hides the other where both are at hand: six products, 18 exp2 and 24 other vector instructions of a wave in
+// turns take 133 ns, one kind after the other 203.  So here the scores of step kt + 1 are made while step kt is exponentiated, one
+// row's products beside the other row's exponentials, in an order that is written down; K and the bias of a step are read a step
+// ahead of V (four ring slots), and products go first where two waves ask (s_setprio: 2 %).  The bias tile is multiplied by the
+// identity once for both rows: its accumulator is the C operand of their scores (five products per tile, not six), which leaves no
+// place for a row's reference, so the reference is zero: sums of exp2 within OPT_LOW .. OPT_HIGH prove that nothing over- or
+// underflowed; a workgroup without that proof walks again with a running maximum.
+// Before -> after, us: 64 rows x 4 heads of 4 096 queries 888 -> 780, 1 024 x 4 of 1 024 984 -> 920, 391 x 4 of 391 99 -> 94, 320 x 4 of 320
+// 53.0 -> 49.0.  Of the 190 ns a tile takes at 4 096 queries its instructions take 148, LDS 14, the barrier 7 and
+// the ring's requests the rest.  Without a bias (212 -> 213 us, 128 x 8 of 1 024) the kernel above stays.  Workgroup = 2 batch rows x 4
+// query tiles, two per CU (one of 4 x 4 leaves the CU idle at its start and end: 985 us at 1 024 queries).
+__global__ __launch_bounds__(PAIR_THREADS, 2) void attention_pair_kernel(
+    bf16_t* __restrict__ out, const bf16_t* __restrict__ q_t, const bf16_t* __restrict__ k_t, const bf16_t* __restrict__ v_t,
+    const bf16_t* __restrict__ bias_t, const float* __restrict__ keybias, const int* __restrict__ tileflags,
+    const bf16_t* __restrict__ gate, int B2, int H, int Nq, int Nk, int flags) {
+    typedef Mma<bf16_t> MM;
+    constexpr int NTILES = 8;                     // operand tiles per key step: K0 K1 V0 V1 B0 .. B3
+    constexpr int NVL = 4, NSLOT = 4;             // 16-byte vectors per thread and step
+    constexpr float OPT_HIGH = 1.2676506e30f, OPT_LOW = 8.2718061e-25f;        // 2^100, 2^-80
+    constexpr float REF_FLOOR = -1.0e4f;
+    extern __shared__ __align__(16) unsigned char att_smem[];
+    bf16_t* lds = reinterpret_cast<bf16_t*>(att_smem);       // [NSLOT][NTILES][1024]
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, half = lane >> 5;
+    const int QT = (Nq + 31) >> 5, KT = (Nk + 31) >> 5;
+    const int NQG = (QT + 3) >> 2, NZ = (B2 + 1) >> 1;
+    const unsigned total = (unsigned)NQG * H * NZ, per_xcd = (total + 7) >> 3;
+    const unsigned item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);      // as above
+    if (item >= total) return;                    // whole workgroup leaves together
+    // (head, eight query groups, row pair, query group): the 64 workgroups an XCD holds share the bias of eight groups and the keys of
+    // eight pairs.  With all query groups of a pair first, 4 096 queries read their bias anew for every two pairs.
+    const int h = item / (NQG * NZ), in_head = item - h * (NQG * NZ), qb = in_head / (8 * NZ) * 8, in_block = in_head - qb * NZ;
+    const int width = NQG - qb < 8 ? NQG - qb : 8, wg_z = in_block / width, wg_q = qb + in_block - wg_z * width;
+    const int qt_raw = wg_q * 4 + wave, qt = qt_raw < QT ? qt_raw : QT - 1;
+    const int q = qt * 32 + l32, qc = q < Nq ? q : Nq - 1;
+    int b2[2];
+    bool live[2];                                 // of the wave; dead ones still help loading and keep the barriers
+    long bh[2], rowo[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const int raw = wg_z * 2 + r;
+        live[r] = raw < B2 && qt_raw < QT;
+        b2[r] = raw < B2 ? raw : B2 - 1;
+        bh[r] = (long)b2[r] * H + h;
+        rowo[r] = ((long)b2[r] * Nq + qc) * (H * 32) + h * 32 + 4 * half;
+    }
+
+    const bf16_t* src[NVL];                       // wave-uniform: start of the wave's 64 vectors in key tile 0 (see above)
+#pragma unroll
+    for (int i = 0; i < NVL; ++i) {
+        const int v = wave * 64 + i * PAIR_THREADS, tile = v >> 7, wv = v & 127;
+        const bf16_t* base;
+        if (tile < 4) {
+            int bb = wg_z * 2 + (tile & 1);
+            bb = bb < B2 ? bb : B2 - 1;
+            base = (tile < 2 ? k_t : v_t) + ((((long)bb * H + h) * KT) << 10);
+        } else {
+            int qq = wg_q * 4 + (tile - 4);
+            qq = qq < QT ? qq : QT - 1;
+            base = bias_t + ((((long)h * QT + qq) * (KT + ((flags >> 1) & 1))) << 10);
+        }
+        src[i] = base + (wv >> 6) * 512;
+    }
+
+    // from an asm statement for the reason given above
+    const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)att_smem;
+    // A request fetches 1 KB, and sixteen lanes 256 bytes of it side by side (by 16-byte pieces 32 bytes apart, as above, every line is
+    // asked for twice).  Of a lane's two pieces one lies in the first half of its sixteen places, the other in the second, the other
+    // way round in every other group of eight lanes: the sixteen lanes of a read meet sixteen places in sixteen bank groups.
+    const unsigned lane_off = ((lane >> 4) * 8 + (lane & 7)) * 32 + ((lane >> 3 ^ lane >> 4) & 1) * 16;
+    const int piece0 = (lane >> 5) * 512 + ((lane >> 3 & 3) * 16 + (lane & 7) + 8 * (lane >> 3 & 1)) * 8, piece1 = piece0 ^ 64;
+    auto operand = [&](const bf16_t* tile) __attribute__((always_inline)) {
+        Ops16<bf16_t> o;
+        o.v[0] = ld16(tile + piece0);
+        o.v[1] = ld16(tile + piece1);
+        return o;
+    };
+    auto fetch = [&](int kt, int slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NVL; ++i) {
+            const bf16_t* gp = src[i] + ((long)kt << 10);
+            const unsigned dst = lds_base + (slot * NTILES * 128 + wave * 64 + i * PAIR_THREADS) * 16;
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(gp), "s"(dst)
+                         : "memory", "m0");
+#pragma clang diagnostic pop
+        }
+    };
+    // the first steps (all masked or not), then what the wave itself needs
+    fetch(0, 0);
+    fetch(KT > 1 ? 1 : 0, 1);
+    fetch(KT > 2 ? 2 : KT - 1, 2);
+
+    Ops16<bf16_t> qf[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) qf[r].load(q_t + ((bh[r] * QT + qt) << 10) + lane * 16);
+
+    bf16_t gv[2][4][4];                           // this lane's gate values, fetched now
+    if (gate) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            if (flags & FFK_ATT_GATE_TILED) {
+                const bf16_t* gp = gate + ((bh[r] * QT + qt) << 10) + lane * 16;
+                *reinterpret_cast<u32x4*>(&gv[r][0][0]) = *reinterpret_cast<const u32x4*>(gp);
+                *reinterpret_cast<u32x4*>(&gv[r][2][0]) = *reinterpret_cast<const u32x4*>(gp + 8);
+            } else {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) *reinterpret_cast<u32x2*>(&gv[r][g][0]) = *reinterpret_cast<const u32x2*>(gate + rowo[r] + 8 * g);
+            }
+        }
+    }
+
+    // trailing key tiles that are completely masked in all batch rows contribute exactly zero
+    int kt_end = KT;
+    {
+        auto masked = [&](int kt) {
+            bool m = true;
+#pragma unroll
+            for (int r = 0; r < 2; ++r) m = m && tileflags[(long)b2[r] * KT + kt] == 2;
+            return m;
+        };
+        while (kt_end > 1 && masked(kt_end - 1)) --kt_end;
+    }
+    const int* fl0 = tileflags + (long)b2[0] * KT;
+    const int* fl1 = tileflags + (long)b2[1] * KT;
+    int first_flag = KT;                          // from here on some key may be masked or padding
+    for (int k0 = 0; k0 < KT; k0 += 64) {
+        const int k = k0 + lane < KT ? k0 + lane : KT - 1;
+        const unsigned long long f = __builtin_amdgcn_ballot_w64((fl0[k] | fl1[k]) != 0);
+        if (f) {
+            first_flag = k0 + __builtin_ctzll(f);
+            break;
+        }
+    }
+
+    bf16x8 ident[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) ident[i] = identity_frag<bf16_t>(i, l32, half);
+    f32x16 o_acc[2];
+    float l_run[2] = {0.0f, 0.0f}, ref[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o_acc[0][v] = o_acc[1][v] = 0.0f;
+
+    auto landed = [&](auto steps) __attribute__((always_inline)) {             // all but the newest `steps` requests of this thread
+        static_assert(NVL == 4);
+        if constexpr (decltype(steps)::value == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        else if constexpr (decltype(steps)::value == 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        lds_barrier();
+    };
+    typedef std::integral_constant<int, 0> I0;
+    typedef std::integral_constant<int, 1> I1;
+    typedef std::integral_constant<int, 2> I2;
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) asm volatile("" : "+v"(*reinterpret_cast<u32x4*>(&qf[r].v[i])));
+
+    auto bias_tile = [&](const bf16_t* buf) __attribute__((always_inline)) {
+        f32x16 c;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) c[v] = 0.0f;
+        const Ops16<bf16_t> bc = operand(buf + (4 + wave) * 1024);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) MM::mma(c, bc.frag(i), ident[i]);
+        return c;
+    };
+    auto scores = [&](const bf16_t* buf, int r, const f32x16& c) __attribute__((always_inline)) {
+        const Ops16<bf16_t> kc = operand(buf + r * 1024);
+        f32x16 s = c;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) MM::mma(s, kc.frag(i), qf[r].frag(i));
+        return s;
+    };
+    auto add_keybias = [&](f32x16 (&s)[2], int kt) __attribute__((always_inline)) {          // some key of this tile is masked or padding
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const float* mp = keybias + ((long)b2[r] * KT + kt) * 32 + 4 * half;
+            f32x4 mk[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) mk[g] = *reinterpret_cast<const f32x4*>(mp + 8 * g);
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[r][4 * g + e] += mk[g][e];
+        }
+    };
+    auto exponentiate = [&](const f32x16& s, bf16x8 (&pf)[2]) __attribute__((always_inline)) {        // and the sum of the rounded values
+        float p[16], t = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) p[v] = fast_exp2(s[v]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            pf[i] = PFrag<bf16_t>::make(p + i * 8);
+            t = PFrag<bf16_t>::add_sum(pf[i], t);
+        }
+        return t;
+    };
+
+    {
+        const int last = kt_end - 1;
+        landed(I2{});
+        f32x16 s[2], n[2];
+        {
+            const f32x16 c = bias_tile(lds);
+#pragma unroll
+            for (int r = 0; r < 2; ++r) s[r] = scores(lds, r, c);
+            if (first_flag == 0) add_keybias(s, 0);
+        }
+        int slot = 0;
+        auto step = [&](int kt, f32x16 (&s)[2], f32x16 (&n)[2]) __attribute__((always_inline)) {
+            landed(I1{});                         // step kt + 1; and everyone is done with step kt - 1
+            fetch(kt + 3 < kt_end ? kt + 3 : last, (slot + 3) & 3);
+            const bf16_t* buf = lds + slot * NTILES * 1024;
+            slot = (slot + 1) & 3;
+            const bf16_t* ahead = lds + slot * NTILES * 1024;
+            // everything is read at once; then a product to every four exponentials, in this order
+            Ops16<bf16_t> kc[2], vc[2], bc;
+            bc = operand(ahead + (4 + wave) * 1024);
+#pragma unroll
+            for (int r = 0; r < 2; ++r) kc[r] = operand(ahead + r * 1024);
+#pragma unroll
+            for (int r = 0; r < 2; ++r) vc[r] = operand(buf + (2 + r) * 1024);
+            __builtin_amdgcn_sched_barrier(0);
+            f32x16 c;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) c[v] = 0.0f;
+            float p[2][16], t[2] = {0.0f, 0.0f};
+            bf16x8 pf[2][2];
+            auto e4 = [&](int r, int g) __attribute__((always_inline)) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) p[r][4 * g + e] = fast_exp2(s[r][4 * g + e]);
+                if (g & 1) pf[r][g >> 1] = PFrag<bf16_t>::make(p[r] + 8 * (g >> 1));
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto score = [&](int r, int i) __attribute__((always_inline)) {
+                if (i == 0) n[r] = c;
+                __builtin_amdgcn_s_setprio(1);
+                MM::mma(n[r], kc[r].frag(i), qf[r].frag(i));
+                __builtin_amdgcn_s_setprio(0);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto value = [&](int r, int i) __attribute__((always_inline)) {
+                __builtin_amdgcn_s_setprio(1);
+                MM::mma(o_acc[r], vc[r].frag(i), pf[r][i]);
+                __builtin_amdgcn_s_setprio(0);
+                t[r] = PFrag<bf16_t>::add_sum(pf[r][i], t[r]);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto bias = [&](int i) __attribute__((always_inline)) {
+                MM::mma(c, bc.frag(i), ident[i]);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            e4(0, 0);
+            bias(0);
+            e4(0, 1);
+            bias(1);
+            e4(0, 2);
+            value(0, 0);
+            e4(0, 3);
+            score(0, 0);
+            e4(1, 0);
+            value(0, 1);
+            e4(1, 1);
+            score(0, 1);
+            e4(1, 2);
+            score(1, 0);
+            value(1, 0);
+            e4(1, 3);
+            score(1, 1);
+            value(1, 1);
+            l_run[0] += t[0];
+            l_run[1] += t[1];
+            if (kt + 1 >= first_flag && kt < last) add_keybias(n, kt + 1);
+        };
+        int kt = 0;
+#pragma unroll 1
+        for (; kt < last; kt += 2) {
+            step(kt, s, n);
+            step(kt + 1, n, s);
+        }
+        if (kt == last) step(kt, s, n);
+        landed(I0{});
+    }
+
+    float l_tot[2];
+    {
+        int* redo = reinterpret_cast<int*>(lds + NSLOT * NTILES * 1024);
+        bool bad = false;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            l_tot[r] = l_run[r] + lane_xor<32>(l_run[r]);
+            bool out_of_range = live[r] && q < Nq && !(l_tot[r] <= OPT_HIGH && l_tot[r] >= OPT_LOW);
+            if (__builtin_amdgcn_ballot_w64(out_of_range) != 0) {
+                bool any = false;                 // a row without keys has a sum of zero, and zeros for its result
+                for (int kt = 0; kt < KT; ++kt) any = any || (r ? fl1 : fl0)[kt] != 2;
+                bad = bad || any;
+            }
+        }
+        if (tid == 0) *redo = 0;
+        lds_barrier();
+        if (bad && lane == 0) *redo = 1;
+        lds_barrier();
+        if (*redo != 0) {                         // workgroup-uniform
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                l_run[r] = 0.0f;
+                ref[r] = REF_FLOOR;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) o_acc[r][v] = 0.0f;
+            }
+#pragma unroll 1
+            for (int kt = 0; kt < kt_end; ++kt) {
+                lds_barrier();
+                fetch(kt, 0);
+                landed(I0{});
+                const f32x16 c = bias_tile(lds);
+                f32x16 sc[2];
+#pragma unroll
+                for (int r = 0; r < 2; ++r) sc[r] = scores(lds, r, c);
+                if (kt >= first_flag) add_keybias(sc, kt);
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    f32x16& s = sc[r];
+                    float m = s[0];
+#pragma unroll
+                    for (int v = 1; v < 16; ++v) m = fmaxf(m, s[v]);
+                    m = fmaxf(m, lane_xor<32>(m));
+                    m = fmaxf(m, ref[r]);
+                    const float alpha = fast_exp2(ref[r] - m);
+                    ref[r] = m;
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        s[v] -= m;
+                        o_acc[r][v] *= alpha;
+                    }
+                    bf16x8 pf[2];
+                    l_run[r] = l_run[r] * alpha + exponentiate(s, pf);
+                    const Ops16<bf16_t> vc = operand(lds + (2 + r) * 1024);
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) MM::mma(o_acc[r], vc.frag(i), pf[i]);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 2; ++r) l_tot[r] = l_run[r] + lane_xor<32>(l_run[r]);
+        }
+    }
+
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const float inv = l_tot[r] > 0.0f ? 1.0f / l_tot[r] : 0.0f;
+        if (!live[r] || q >= Nq) continue;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            bf16_t r4[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float x = o_acc[r][4 * g + e] * inv;
+                if (gate) x *= (float)gv[r][g][e];
+                r4[e] = (bf16_t)x;
+            }
+            *reinterpret_cast<u32x2*>(out + rowo[r] + 8 * g) = *reinterpret_cast<const u32x2*>(r4);
+        }
+    }
+}
+
 // Head dimensions 64 and 128 (the widths the reference's attention core also accepts; no module of the Evoformer
 // uses them): the head is cut into DP = D / 32 parts of 32 channels, each part an operand tile of its own
 // (part-major: part p of every tensor lies p * part elements behind part 0), so a score tile is the sum of DP
@@ -622,6 +995,20 @@ int launch_attention_b(void* out, const void* q, const void* k, const void* v, c
     return ffk_check_launch("ffk_attention_fwd");
 }
 
+int launch_attention_pair(void* out, const void* q, const void* k, const void* v, const void* bias, const float* kb, const int* flags,
+                          const void* gate, long B2, long H, long Nq, long Nk, int aflags, hipStream_t st) {
+    const size_t smem = 4 * (size_t)8 * 2048 + 16;             // operand ring + redo flag
+    static FfkLdsReservation lds_reserved;
+    const int rc_lds = ffk_reserve_lds(lds_reserved, (const void*)attention_pair_kernel, smem, "ffk_attention_fwd");
+    if (rc_lds != FFK_OK) return rc_lds;
+    const long items = (long)ffk_cdiv((Nq + 31) / 32, 4) * H * ffk_cdiv(B2, 2);
+    FFK_REQUIRE(items < (1L << 31) - 8, FFK_ERR_SHAPE, "ffk_attention_fwd: %ld workgroups exceed the grid limit", items);
+    attention_pair_kernel<<<dim3((unsigned)(8 * ffk_cdiv(items, 8))), PAIR_THREADS, smem, st>>>(
+        (bf16_t*)out, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)bias, kb, flags, (const bf16_t*)gate, (int)B2,
+        (int)H, (int)Nq, (int)Nk, aflags);
+    return ffk_check_launch("ffk_attention_fwd");
+}
+
 template <typename T, int HD = 32>
 int launch_attention(void* out, const void* q, const void* k, const void* v, const void* bias, const float* kb,
                      const int* flags, const void* gate, float* lse, long B2, long H, long Nq, long Nk, int aflags,
@@ -669,7 +1056,13 @@ extern "C" int ffk_attention_fwd_lse(void* out, float* lse, const void* q_t, con
         return ffk_fail(FFK_ERR_DTYPE, "ffk_attention_fwd: unsupported dtype tag %d", dtype);
     }
     switch (dtype) {
-        case FFK_BF16: return launch_attention<bf16_t>(out, q_t, k_t, v_t, bias_t, keybias, tileflags, gate, lse, B2, H, Nq, Nk, flags, st);
+        case FFK_BF16:
+            // Two rows per wave (FFK_ATT_HALF_K or not: the padding adds nothing) for a bias and more than 256 keys, one row / two, us:
+            // 256 x 4 heads of 256 queries 26.8 / 28.0, 320 x 4 of 320 53.0 / 49.0, 128 x 4 of 512 41 / 38, and see there.  With the
+            // log-sum-exp, from sums of probabilities that were not rounded against a zero reference, 256 x 4 of 256 27.0 / 29.3,
+            // 391 x 4 of 391 102 / 102: one row.
+            if (bias_t && !lse && Nk > 256) return launch_attention_pair(out, q_t, k_t, v_t, bias_t, keybias, tileflags, gate, B2, H, Nq, Nk, flags, st);
+            return launch_attention<bf16_t>(out, q_t, k_t, v_t, bias_t, keybias, tileflags, gate, lse, B2, H, Nq, Nk, flags, st);
         case FFK_F32: return launch_attention<float>(out, q_t, k_t, v_t, bias_t, keybias, tileflags, gate, lse, B2, H, Nq, Nk, flags, st);
         default: return ffk_fail(FFK_ERR_DTYPE, "ffk_attention_fwd: unsupported dtype tag %d", dtype);
     }
