@@ -326,38 +326,38 @@ template <> struct Mma<float> {
     static __device__ __forceinline__ Frag ld(const float* p) { return *reinterpret_cast<const Frag*>(p); }
 };
 
-// fp32 products on the bf16 matrix pipe.  An fp32 number is the sum of three bf16 numbers of eight bits each, cut off one after
-// the other (x = x1 + x2 + x3 exactly, but for what lies below the smallest normal number), and
+// fp32 products on the bf16 matrix pipe.  An fp32 number is the sum of three bf16 numbers (x = x1 + x2 + x3 exactly, but for what lies
+// below the smallest normal number): the first cut off, so that a finite number has finite parts, the others rounded, so that what is
+// left out has either sign; and
 //     x y = x1 y3 + x3 y1 + x2 y2 + x1 y2 + x2 y1 + x1 y1      up to 2^-24 |x y|,
 // added from the smallest to the largest term in the fp32 accumulator.  Six v_mfma_f32_32x32x16_bf16 take 196 cycles for a K step of 16,
-// eight v_mfma_f32_32x32x2_f32 512, and the bf16 ones let the vector instructions of other waves run beside them.  Relative error
-// (2-norm) of 32 x 32 sums of K products of normal numbers against float64, fp32 instructions -> this:  K = 64 1.6e-7 -> 1.3e-7,
-// 128 2.0e-7 -> 1.8e-7, 256 2.9e-7 -> 2.5e-7, 512 3.8e-7 -> 3.3e-7, 1 024 5.7e-7 -> 4.8e-7; of positive numbers 1.3e-7 -> 1.0e-7 and
-// 5.0e-7 -> 5.0e-7: sixteen products are added per rounding of the accumulator, not two.  The
+// eight v_mfma_f32_32x32x2_f32 512, and the bf16 ones let the vector instructions of other waves run beside them.  The error of a sum is
+// lower than by the fp32 instructions (sixteen products are added per rounding, not two).  Relative error (2-norm) against float64, fp32
+// instructions -> this, as ffk_bgemm_nt adds them: normal numbers, K = 64 1.44e-7 -> 1.12e-7, 128 2.03e-7 -> 1.65e-7, 256 2.88e-7 -> 2.38e-7,
+// 496 3.99e-7 -> 3.38e-7; positive numbers, 64 1.22e-7 -> 0.90e-7, 256 2.47e-7 -> 2.06e-7, 496 3.43e-7 -> 2.87e-7.  Longer chains are for
+// the callers to cut: the instruction cuts off towards minus infinity what the accumulator has no room for.  The
 // parts of an infinite operand make NaN of its products: a kernel that finds one in its sums takes the fp32 instructions for them.
 struct Split4 {              // four numbers, part by part
     u32x2 p[3];
 };
-__device__ __forceinline__ Split4 split4(const f32x4& x, uint32_t mask = 0xFFFF0000u, uint32_t high = 0x07060302u) {
+// PIN: not to be moved out of a loop
+template <bool PIN = false> __device__ __forceinline__ Split4 split4(const f32x4& x) {
     typedef float f32x2 __attribute__((ext_vector_type(2)));
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
     Split4 r;
-    const u32x4 b = __builtin_bit_cast(u32x4, x);
-    float q[4];
-    uint32_t m[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {        // (what is left by a dot product with -1 instead of the mask and a subtraction: no faster)
-        const uint32_t h = b[i] & mask;
-        const float r1 = x[i] - __builtin_bit_cast(float, h);
-        m[i] = __builtin_bit_cast(uint32_t, r1);
-        const uint32_t h1 = m[i] & mask;
-        q[i] = r1 - __builtin_bit_cast(float, h1);
-    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        r.p[0][j] = __builtin_amdgcn_perm(b[2 * j + 1], b[2 * j], high);
-        r.p[1][j] = __builtin_amdgcn_perm(m[2 * j + 1], m[2 * j], high);
-        r.p[2][j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{q[2 * j], q[2 * j + 1]}, bf16x2));
+        float a = x[2 * j], b = x[2 * j + 1];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            uint32_t h;
+            if (PIN && p == 0) asm volatile("v_perm_b32 %0, %1, %2, %3" : "=v"(h) : "v"(b), "v"(a), "s"(0x07060302u));
+            else if (p == 0) h = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
+            else h = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+            r.p[p][j] = h;
+            a -= __builtin_bit_cast(float, h << 16);
+            b -= __builtin_bit_cast(float, h & 0xFFFF0000u);
+        }
     }
     return r;
 }

@@ -353,10 +353,6 @@ __global__ __launch_bounds__(ONE ? 256 : 512, K == 128 && !GLU && BM == 32 ? 3 :
     // products of R row groups with the first N slots, rows: W . A^T.  The weights are cut into their parts as they are used.
     auto products = [&](f32x16* acc, const unsigned char* ap, auto rows, auto n, auto rt) __attribute__((always_inline)) {
         constexpr int N = decltype(n)::value, R = decltype(rt)::value;
-        // constants the compiler cannot follow: it would cut all weights ahead of the loop over slabs, and their parts do not fit
-        // in the registers
-        uint32_t mask = 0xFFFF0000u, high = 0x07060302u;
-        asm volatile("" : "+s"(mask), "+s"(high));
 #pragma unroll
         for (int s = 0; s < N * R; ++s)
 #pragma unroll
@@ -377,7 +373,7 @@ __global__ __launch_bounds__(ONE ? 256 : 512, K == 128 && !GLU && BM == 32 ? 3 :
                     for (int p = 0; p < 3; ++p) w[g & 1][s][p] = wp[g][p];
                     continue;
                 }
-                const Split4 a = split4(wf[s][2 * g], mask, high), b = split4(wf[s][2 * g + 1], mask, high);
+                const Split4 a = split4<true>(wf[s][2 * g]), b = split4<true>(wf[s][2 * g + 1]);     // all ahead of the loop over slabs they would not fit
 #pragma unroll
                 for (int p = 0; p < 3; ++p) w[g & 1][s][p] = split_frag(a, b, p);
             }

@@ -32,7 +32,7 @@ def test_error_of_products(dev, M, K, N, sx, sw):
     g = torch.Generator().manual_seed(M + K + N)
     x, w = (torch.randn(M, K, generator=g) * sx).to(dev), (torch.randn(N, K, generator=g) * sw).to(dev)
     got, want, size = _run(x, w), x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
-    # what is left out of a product: x2 y3 + x3 y2 + x3 y3, at most 2^-23 of it; roundings of the sum: six for a step of 16 and three for
+    # what is left out of a product: x2 y3 + x3 y2 + x3 y3, less than 2^-23 of it; roundings of the sum: six for a step of 16 and three for
     # the quarters, each at most 2^-23 (cut off) of the sums of magnitudes
     err = (got - want).abs()
     assert bool((err <= (1 + 6 * ((K + 15) // 16) + 3) * 2.0 ** -23 * size).all())
