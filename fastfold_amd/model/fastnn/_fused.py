@@ -295,26 +295,37 @@ def attention_block_pays(C, head_dim, N, B2, biased):
 
 def pack_attention_block(qkv_w, gate_w, out_w, dtype, device):
     """The weights of a gated attention in the fragment order of ``ffk_attention_block``: [q, k, v, gate, out][C/32][C/16][64][8]."""
-    return torch.cat([pack_fragments(torch.cat([qkv_w.detach(), gate_w.detach()], 0), dtype, device),
-                      pack_fragments_of_accumulators(out_w, dtype, device)]).contiguous()
+    w = torch.empty(qkv_w.numel() + gate_w.numel() + out_w.numel(), dtype=dtype, device=device)
+    at = 0
+    for part in (fragments(qkv_w), fragments(gate_w), fragments_of_accumulators(out_w)):       # one launch each
+        w[at:at + part.numel()].view(part.shape).copy_(part)
+        at += part.numel()
+    return w
+
+
+def fragments(w):
+    """[n, K] as [n/32][K/16][half][row][8]: what each lane of a wave gives to the matrix instructions that multiply by 32 rows of w."""
+    w = w.detach()
+    return w.reshape(w.shape[0] // 32, 32, w.shape[1] // 16, 2, 8).permute(0, 2, 3, 1, 4)
+
+
+def fragments_of_accumulators(w):
+    """The same for a weight that multiplies accumulators as they stand: columns in their order ([quad][half][4] of a step), and rows
+    (8 a + 4 h + b from 16 h + 4 a + b) so that a lane's results are 16 consecutive channels."""
+    w = w.detach()
+    return w.reshape(w.shape[0] // 32, 2, 4, 4, w.shape[1] // 16, 2, 2, 4).permute(0, 4, 6, 2, 1, 3, 5, 7)
 
 
 def pack_fragments(w, dtype, device):
-    """[n, K] -> [n/32][K/16][64][8]: what each lane of a wave gives to the matrix instructions that multiply by 32 rows of w."""
-    w = w.detach().to(device=device, dtype=dtype)
-    return w.view(w.shape[0] // 32, 32, w.shape[1] // 16, 2, 8).permute(0, 2, 3, 1, 4).reshape(-1)      # lane = 32 * (half) + row
+    return fragments(w).to(device=device, dtype=dtype).reshape(-1)
 
 
 def pack_fragments_of_accumulators(w, dtype, device):
-    """The same for a weight that multiplies accumulators as they stand: columns in their order, and rows so that a lane's results are
-    16 consecutive channels."""
-    w = w.detach().to(device=device, dtype=dtype)
-    tau = torch.tensor([((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3) for i in range(32)], device=device)
-    w = w.view(w.shape[0] // 32, 32, w.shape[1] // 16, 2, 2, 4)[:, tau]                  # [block][row][step][quad][half][4]
-    return w.permute(0, 2, 4, 1, 3, 5).reshape(-1)
+    return fragments_of_accumulators(w).to(device=device, dtype=dtype).reshape(-1)
 
 
 ATTENTION_HEADS_TOKENS = 256     # longest row of ffk_attention_heads
+
 
 def pack_transition_block(w1, w2, dtype, device):
     """The weights of a transition in the fragment order of ``ffk_transition_block``; None at widths it is not built for."""
