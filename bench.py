@@ -37,7 +37,7 @@ def attention_traffic(profile):
     """HBM bytes per launch of the biased attention kernel, averaged over the launches the roofline object covers
     (triangle and MSA-row attention, weighted by their launch counts).  Hardware counters cannot be read inside a
     timed run: the figure is taken from the committed summary of the rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs
-    of this script (rows ``attention_kernel<bf16, true>  workgroups  n  read MB  written MB`` of its table, already
+    of this script (rows ``attention_pair_kernel  workgroups  n  read MB  written MB`` of its table, already
     scaled by the calibration the file states); None when the file or its rows are missing."""
     if profile is None:
         return None
@@ -47,9 +47,9 @@ def attention_traffic(profile):
         return None
     tot, n = 0.0, 0
     for ln in lines:
-        if not ln.startswith("attention_kernel<bf16, true>"):
+        f = ln.split()
+        if not f or f.pop(0) != "attention_pair_kernel":
             continue
-        f = ln.split(">", 1)[1].split()
         try:
             launches, rd, wr = int(f[1]), float(f[2]), float(f[3])
         except (IndexError, ValueError):
@@ -379,7 +379,7 @@ def main():
     # HIP events bracket every attention launch of the first timed step only: an event pair costs the
     # stream about 10 us per launch, which the other steps do not have to carry
     rec = _lib.time_kernel("ffk_attention_fwd")
-    others = {name: _lib.time_kernel(name) for name in ("ffk_bgemm_nt", "ffk_transition_fused", "ffk_opm_fused")}
+    others = {name: _lib.time_kernel(name) for name in ("ffk_bgemm_nt", "ffk_transition_fused", "ffk_transition_block", "ffk_opm_fused")}
     t0 = time.perf_counter()
     for i in range(args.steps):
         out = step()
@@ -401,7 +401,7 @@ def main():
         ms += e0.elapsed_time(e1)
         n += 1
     ach = flops / (ms * 1e-3) / 1e12 if ms > 0 else 0.0
-    roofline = {"bound": "mfma", "kernel": "attention_kernel<bf16, bias> (ffk_attention_fwd)",
+    roofline = {"bound": "mfma", "kernel": "attention_pair_kernel (ffk_attention_fwd, bf16, bias)",
                 "achieved": round(ach, 2), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                 "frac": round(ach / PEAK_BF16_TFLOPS, 4), "traffic": attention_traffic(wl["traffic_profile"]),
                 "traffic_unit": "bytes/launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, see profiles/)",
@@ -431,8 +431,8 @@ def main():
         return None
     kernels = {}
     kernels.update(summarise(others["ffk_bgemm_nt"], bgemm_kind))
-    kernels.update(summarise(others["ffk_transition_fused"],
-                             lambda a: ("transition_fused_C%d" % a[10], 4.0 * a[9] * a[10] * a[11] / 1e9)))
+    for name in ("transition_fused", "transition_block"):
+        kernels.update(summarise(others["ffk_" + name], lambda a: ("%s_C%d" % (name, a[10]), 4.0 * a[9] * a[10] * a[11] / 1e9)))
     kernels.update(summarise(others["ffk_opm_fused"],
                              lambda a: ("opm_fused", 2.0 * r * r * (32 * 32 * s + 1024 * 128) / 1e9)))
 
