@@ -448,7 +448,11 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     # it finds x as warm as before - the other way round the projection's output (four times the size of x)
     # has pushed x out by the time the bias pass reads it (measured: -0.65 % block time at N = 1024).
     if rides:
-        pass
+        if pb_scratch is not None and not pb_scratch.ready:
+            # The weight operand of the bias pass that short rows take, made with the other weights: made in the first pass of
+            # another size it keeps that pass from being recorded.  The bias of one row, thrown away.
+            _pair_bias_launch(alloc((H, 1, 1, 1024), dt, dev), x, ln, w_pk[4 * tpg * 128:], pb_scratch, N=1, C=C, H=H, a_inner=1,
+                              a_so=0, a_si=C, scale=LOG2E)
     elif can_ride and N < 1024:
         # In slabs: the same kernel with the bias as its only tile, so that slabs change no bit of the result.  Longer rows
         # keep the bias pass of its own, which streams x twice as fast (16 M rows at N = 4096: 0.9 against 1.9 ms).

@@ -209,3 +209,18 @@ def test_modules_take_the_block_and_match_the_separate_launches(dev, monkeypatch
         upd = outs[1] - args[0].float()
         err = float((outs[0] - outs[1]).norm() / upd.norm())
         assert float(upd.norm()) > 1.0 and err < 2 * TOL, (type(mod).__name__, args[0].shape, err)
+
+
+def test_weights_of_short_rows_are_laid_out_with_the_others(dev):
+    """The first pass of a triangle attention lays out all weights: the first pass at a length that takes another route builds
+    nothing, so a stack can record it."""
+    from fastfold_amd import _plan
+    from fastfold_amd.model.fastnn.ops import ChunkTriangleAttentionStartingNode
+    torch.manual_seed(0)
+    att = ChunkTriangleAttentionStartingNode(128, 32).to(dev, BF).eval()
+    with torch.no_grad():
+        for i, r in enumerate((288, 64, 256)):
+            z = torch.randn(1, r, r, 128, device=dev, dtype=BF)
+            before = _plan.builds
+            out = att(z, torch.ones(1, r, r, device=dev, dtype=BF))
+            assert bool(out.isfinite().all()) and (i == 0 or _plan.builds == before)
