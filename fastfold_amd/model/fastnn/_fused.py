@@ -379,6 +379,7 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     if (_ATTENTION_BLOCK and enough and acc_order and hasattr(w_pk, "block") and N <= attention_block_tokens(dt, H, head_dim, C, c_out)
             and ln is not None and resid is not None and resid.data_ptr() == x.data_ptr() and o_map is None
             and a_so % 16 == 0 and a_si % 16 == 0 and (C == 256 or bias_t is not None or bias_in_launch)
+            and not (bias_in_launch and C == 256)          # ffk_pair_bias, which makes that bias, is built for 64 and 128 channels
             and (drop is None or drop.shape[0] == N)):
         if bias_in_launch:
             bias_t = alloc((H, NT, NT, 1024), dt, dev)
