@@ -141,6 +141,12 @@ def _pair_bias_launch(bias_t, x, ln, w, scratch, **kw):
     scratch.ready = True
 
 
+def aligned16(*ts):
+    """Whether 16-byte loads may read the tensors from their first element.  Parameters come as they are (slices of a flat buffer, say);
+    the kernels that need whole vectors of them are taken only then."""
+    return all(t.data_ptr() % 16 == 0 for t in ts)
+
+
 def fits_fused(K, dtype):
     return K <= 256 and K % 32 == 0
 
@@ -224,7 +230,7 @@ def transition(x, out, *, ln, w1_pk, b1_pk, w2, b2, hidden, budget, xtail=None, 
     M, C = x.shape
     dt, dev = x.dtype, x.device
     es = es_of(dt)
-    if w_block is not None and ln is not None and _FUSED_TRANSITION and M <= transition_block_rows(C):
+    if w_block is not None and ln is not None and _FUSED_TRANSITION and M <= transition_block_rows(C) and aligned16(*ln, b2):
         _lib.transition_block(out, x, ln[0], ln[1], w_block[0], b1_pk, w_block[1], b2, M=M, C=C, hidden=hidden, xtail=xtail)
         return out
     if dt == torch.bfloat16 and C in (128, 256) and hidden == 4 * C and ln is not None and _FUSED_TRANSITION:
@@ -376,8 +382,9 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     acc_order = dt == torch.bfloat16 and C in (64, 128, 256) and N % 32 == 0
     # Short rows: one kernel from the rows of x to the updated rows.
     enough = attention_block_pays(C, head_dim, N, B2, bias_t is not None or bias_in_launch)
-    if (_ATTENTION_BLOCK and enough and acc_order and hasattr(w_pk, "block") and N <= attention_block_tokens(dt, H, head_dim, C, c_out)
-            and ln is not None and resid is not None and resid.data_ptr() == x.data_ptr() and o_map is None
+    short = _ATTENTION_BLOCK and enough and acc_order and hasattr(w_pk, "block") and ln is not None and aligned16(*ln)
+    if (short and N <= attention_block_tokens(dt, H, head_dim, C, c_out)
+            and resid is not None and resid.data_ptr() == x.data_ptr() and o_map is None
             and a_so % 16 == 0 and a_si % 16 == 0 and (C == 256 or bias_t is not None or bias_in_launch)
             and not (bias_in_launch and C == 256)          # ffk_pair_bias, which makes that bias, is built for 64 and 128 channels
             and (drop is None or drop.shape[0] == N)):
@@ -400,8 +407,8 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     if HC % 128 != 0 and not packed:
         raise RuntimeError("attention: n_head * 32 must be a multiple of 128 (got %d heads)" % H)
     # Rows of 256 channels too long for that, with a pair bias: one kernel up to the gated heads, the output projection behind it.
-    heads = (_ATTENTION_BLOCK and enough and acc_order and hasattr(w_pk, "block") and C == 256 and head_dim == 32 and HC == C
-             and N <= ATTENTION_HEADS_TOKENS and ln is not None and bias_t is not None and not bias_in_launch)
+    heads = (short and C == 256 and head_dim == 32 and HC == C and N <= ATTENTION_HEADS_TOKENS and bias_t is not None
+             and not bias_in_launch)
     HT = HC // 32                                  # operand tiles per batch row and 32 tokens
     per_row = 5 * HT * NT * 1024 * es
     slab = B2 if budget is None else min(B2, max(2, (budget // per_row) // 2 * 2))

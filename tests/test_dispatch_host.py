@@ -4,6 +4,7 @@ import torch
 
 from fastfold_amd import _lib
 from fastfold_amd.model.fastnn import _fused as F_
+from fastfold_amd.model.fastnn.kernel import LayerNorm
 
 BF = torch.bfloat16
 
@@ -15,6 +16,9 @@ def calls(monkeypatch):
     def call(name, *args):
         if name == "ffk_pair_bias" and args[7] not in (64, 128):
             raise RuntimeError("ffk_pair_bias: built for 64 or 128 pair channels, got %d" % args[7])
+        at = {"ffk_attention_block": (3, 4), "ffk_attention_heads": (2, 3), "ffk_transition_block": (3, 4, 8)}.get(name, ())
+        if any(args[i] % 16 for i in at):                     # gamma, beta (and the transition's second bias)
+            raise RuntimeError("%s: buffers must be 16-byte aligned" % name)
         seen.append(name)
     monkeypatch.setattr(_lib, "call", call)
     monkeypatch.setattr(_lib, "stream_ptr", lambda: 0)
@@ -35,3 +39,40 @@ def test_triangle_attention_of_256_channels_is_taken_at_every_length(calls, r, e
     with torch.no_grad():
         mod(torch.zeros(1, r, r, 256, dtype=BF), torch.ones(1, r, r, dtype=BF))
     assert "ffk_attention_fwd" in calls and "ffk_attention_block" not in calls
+
+
+def _modules():
+    from fastfold_amd.model.fastnn import msa, ops
+
+    def pair(r, c):
+        return torch.zeros(1, r, r, c, dtype=BF), torch.ones(1, r, r, dtype=BF)
+
+    def seqs(s, r, c):
+        return torch.zeros(1, s, r, c, dtype=BF), torch.ones(1, s, r, dtype=BF)
+    yield ops.ChunkTriangleAttentionStartingNode(128, 0.25, c=32, n_head=4), pair(64, 128)
+    yield ops.ChunkTriangleAttentionEndingNode(64, 0.25, c=16, n_head=4), pair(96, 64)
+    for r in (96, 160):
+        m, mask = seqs(128, r, 256)
+        yield msa.MSARowAttentionWithPairBias(256, 128, c=32, n_head=8), (m, pair(r, 128)[0], mask)
+    m, mask = seqs(128, 96, 64)
+    yield msa.MSARowAttentionWithPairBias(64, 128, c=8, n_head=8), (m, pair(96, 128)[0], mask)
+    yield msa.MSAColumnAttention(256), seqs(128, 96, 256)
+    yield ops.Transition(64), (torch.zeros(1, 40, 96, 64, dtype=BF),)
+
+
+@pytest.mark.parametrize("i", range(7))
+def test_normalisation_weights_may_lie_anywhere(calls, i):
+    """Parameters that are slices of one flat buffer need not begin on 16 bytes: the launches that read them element by element take
+    them, as they take every other module whose kernel wants them aligned."""
+    mod, args = list(_modules())[i]
+    mod = mod.to(BF).eval()
+    for aligned in (True, False):
+        del calls[:]
+        for m in mod.modules():
+            if isinstance(m, LayerNorm) and not aligned:
+                for p in (m.weight, m.bias):
+                    p.data = torch.ones(p.numel() + 8, dtype=BF)[1:p.numel() + 1]
+        with torch.no_grad():
+            mod(*args)
+        short = [n for n in calls if n in ("ffk_attention_block", "ffk_attention_heads", "ffk_transition_block")]
+        assert bool(short) == aligned, calls
