@@ -326,6 +326,18 @@ template <> struct Mma<float> {
     static __device__ __forceinline__ Frag ld(const float* p) { return *reinterpret_cast<const Frag*>(p); }
 };
 
+// f - mean over eight numbers of a row, and the sum of their squares, each square and sum rounded once in this order: left to the
+// compiler, which of two products is rounded ahead of their sum differs from kernel to kernel, and with it the bits of a row.
+__device__ __forceinline__ float centre8(float (&f)[8], float mean) {
+    float q = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        f[e] -= mean;
+        q = __builtin_fmaf(f[e], f[e], q);
+    }
+    return q;
+}
+
 // fp32 products on the bf16 matrix pipe.  An fp32 number is the sum of three bf16 numbers (x = x1 + x2 + x3 exactly, but for what lies
 // below the smallest normal number): the first cut off, so that a finite number has finite parts, the others rounded, so that what is
 // left out has either sign; and

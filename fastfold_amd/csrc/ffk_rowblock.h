@@ -58,18 +58,13 @@ __device__ __forceinline__ void rb_normalise(const RbRows& a, const T* xrow, uns
 #pragma unroll
     for (int i = 0; i < R::NI; ++i) {
         if (R::past(i, NT)) break;
-        float f[8], s = 0.0f, q = 0.0f;
+        float f[8], s = 0.0f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             f[e] = (float)r[i].e[e];
             s += f[e];
         }
-        const float mu = group_sum(s, R::LPR) * (1.0f / C);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            f[e] -= mu;
-            q = __builtin_fmaf(f[e], f[e], q);
-        }
+        const float q = centre8(f, group_sum(s, R::LPR) * (1.0f / C));
         const float rs = rsqrtf(group_sum(q, R::LPR) * (1.0f / C) + a.eps);
         bf16x8 y;
 #pragma unroll

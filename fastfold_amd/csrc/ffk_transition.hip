@@ -111,17 +111,11 @@ __global__ __launch_bounds__(TR_THREADS, NS == 4 ? 1 : 3) void transition_fused_
                 f[e] = (float)v[i].e[e];
                 s += f[e];
             }
-            const float mu = group_sum(s, LPR) * (1.0f / TR_C);
-            float q = 0.0f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                f[e] -= mu;
-                q += f[e] * f[e];
-            }
+            const float q = centre8(f, group_sum(s, LPR) * (1.0f / TR_C));
             const float rs = rsqrtf(group_sum(q, LPR) * (1.0f / TR_C) + eps);
             Vec16<T> y;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) y.e[e] = (T)(f[e] * rs * (float)g.e[e] + (float)b.e[e]);
+            for (int e = 0; e < 8; ++e) y.e[e] = (T)__builtin_fmaf(f[e] * rs, (float)g.e[e], (float)b.e[e]);
             *reinterpret_cast<Vec16<T>*>(s_x + (r0 + RPP * i) * TR_XP + c8 * 16) = y;
         }
     }
@@ -361,17 +355,11 @@ __global__ __launch_bounds__(256 * RP, tw_occ(C, RP)) void transition_wide_kerne
                 f[e] = (float)v[i].e[e];
                 s += f[e];
             }
-            const float mu = group_sum(s, NC1) * (1.0f / TW_C);
-            float q = 0.0f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                f[e] -= mu;
-                q += f[e] * f[e];
-            }
+            const float q = centre8(f, group_sum(s, NC1) * (1.0f / TW_C));
             const float rs = rsqrtf(group_sum(q, NC1) * (1.0f / TW_C) + eps);
             Vec16<T> y;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) y.e[e] = (T)(f[e] * rs * (float)g.e[e] + (float)b.e[e]);
+            for (int e = 0; e < 8; ++e) y.e[e] = (T)__builtin_fmaf(f[e] * rs, (float)g.e[e], (float)b.e[e]);
             *reinterpret_cast<Vec16<T>*>(s_x + (r0 + RPR * i) * TW_XP + c8 * 16) = y;
         }
         asm volatile("" ::"v"(touched));

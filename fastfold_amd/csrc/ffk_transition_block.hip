@@ -6,7 +6,8 @@
 // where there are fewer blocks than waves, several waves own one and divide the row tiles.  A weight fragment goes from the cache into
 // the registers of the wave that multiplies by it, requested a layer of a chunk ahead (16 KB a wave, 128 KB a CU in flight); only
 // the rows and the hidden chunk are read from LDS.  The accumulators of the first layer are the second's operand as they stand (the
-// weight columns are packed in their order), so the hidden values cross LDS in whole fragments.
+// rows of W1 are packed so that a lane's are consecutive hidden channels), so the hidden values cross LDS in whole fragments.  Sums are
+// begun and added as in ffk_transition_fused, to the bit: a caller may cut its rows anywhere, whichever kernel a piece goes to.
 //
 // What bounds it: at 256 channels the weights - 1 MB a workgroup, which a CU gets at 60 KB/us where the second-level cache has them and at
 // half that where it does not; 64 rows are multiplied by them in 8 us, 128 in 16.  At 64 channels, memory (393 216 rows: 151 MB with
@@ -68,22 +69,29 @@ __global__ __launch_bounds__(512, OCC) void transition_block_kernel(TbArgs a) {
     rb_normalise<C, RT>(a, a.x + m0 * C, s_x, RT, wave, lane);
     lds_barrier();
 
-    f32x16 acc2[T2];
+    f32x16 acc2[T2];                                 // from b2 on
+    {
+        const Vec16<T> v0 = ld16(a.b2 + ob * 32 + 16 * half), v1 = ld16(a.b2 + ob * 32 + 16 * half + 8);
 #pragma unroll
-    for (int t = 0; t < T2; ++t)
+        for (int t = 0; t < T2; ++t)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc2[t][v] = 0.0f;
+            for (int v = 0; v < 8; ++v) {
+                acc2[t][v] = (float)v0.e[v];
+                acc2[t][8 + v] = (float)v1.e[v];
+            }
+    }
     const unsigned char* xp = s_x + (t1 * 32 + l32) * XP + half * 16;
 #pragma unroll
     for (int q = 0; q < NCH; ++q) {
         // ---- first layer; the second layer's fragments are requested meanwhile ----
         f32x16 h[T1];
         {
-            const float* bp = s_b1 + (q * CB + hb) * 32 + 4 * half;
+            // registers 0 .. 7: hidden 8 half + 0 .. 7 of the block, registers 8 .. 15: 16 + 8 half + 0 .. 7
+            const float* bp = s_b1 + (q * CB + hb) * 32 + 8 * half;
             f32x16 bias;
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const f32x4 b = *reinterpret_cast<const f32x4*>(bp + 8 * g);
+                const f32x4 b = *reinterpret_cast<const f32x4*>(bp + (g >> 1) * 16 + (g & 1) * 4);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) bias[4 * g + e] = b[e];
             }
@@ -140,7 +148,7 @@ __global__ __launch_bounds__(512, OCC) void transition_block_kernel(TbArgs a) {
     RbUpdate<C, RT> rows;
     rows.fetch(a, m0 * C, RT, wave, rb_lane(lane));
 #pragma unroll
-    for (int t = 0; t < T2; ++t) rb_put(s_x + ((t2 + t) * 32 + l32) * XP + ob * 64 + half * 32, acc2[t], a.b2 + ob * 32 + 16 * half);
+    for (int t = 0; t < T2; ++t) rb_put(s_x + ((t2 + t) * 32 + l32) * XP + ob * 64 + half * 32, acc2[t], nullptr);
     lds_barrier();
     rows.store(a, s_x, m0 * C, RT, wave, rb_lane(lane));
 }

@@ -216,10 +216,9 @@ def xtail_ptr(xtail, off=0):
 _FUSED_TRANSITION = True
 
 
-
-
 def transition_block_rows(C):
-    """Most rows ``ffk_transition_block`` is taken for (timings of both sides in csrc/ffk_transition_block.hip)."""
+    """Most rows ``ffk_transition_block`` is taken for (timings of both sides in csrc/ffk_transition_block.hip).  The kernel behind the line
+    gives the same bits: a rank's share of the rows, or a piece of them, gets those of the full call."""
     return 16384 if C == 128 else 1 << 36
 
 
@@ -338,7 +337,12 @@ def pack_transition_block(w1, w2, dtype, device):
     hidden, C = w1.shape
     if dtype != torch.bfloat16 or (C, hidden) not in ((64, 128), (64, 256), (128, 512), (256, 1024)):
         return None
-    return pack_fragments(w1, dtype, device), pack_fragments_of_accumulators(w2, dtype, device)
+    w1, w2 = w1.detach(), w2.detach()
+    # rows of w1 in the order (16 a + 8 c + 4 h + b from 16 a + 8 h + 4 c + b) in which a lane's sums are consecutive hidden channels,
+    # the second layer's operand in the order of ffk_transition_fused; rows of w2 as in fragments_of_accumulators
+    f1 = w1.reshape(hidden // 32, 2, 2, 2, 4, C // 16, 2, 8).permute(0, 5, 6, 1, 3, 2, 4, 7)
+    f2 = w2.reshape(C // 32, 2, 4, 4, hidden // 16, 2, 8).permute(0, 4, 5, 2, 1, 3, 6)
+    return tuple(f.to(device=device, dtype=dtype).reshape(-1) for f in (f1, f2))
 
 
 # False: every attention runs as projection, core and output stage (tests compare the two)

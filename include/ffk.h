@@ -429,10 +429,11 @@ int ffk_transition_fused(void* out, const void* x, void* xtail, const void* gamm
                          const void* b1, const void* w2, const void* b2, int64_t M, int64_t C,
                          int64_t hidden, float eps, int dtype, void* stream);
 
-/* The same with the weights in fragment order, built for C = 64, 128 and 256 with hidden = 4 C and for 64 -> 128 -> 64 (bf16):
- * w1 : [hidden / 32][C / 16][64][8], element e of lane l in step s of block b is row 32 b + l % 32, column 16 s + 8 (l / 32) + e of W1;
+/* The same, to the bit, with the weights in fragment order, built for C = 64, 128 and 256 with hidden = 4 C and for 64 -> 128 -> 64 (bf16):
+ * w1 : [hidden / 32][C / 16][64][8], element e of lane l in step s of block b is row 32 b + sigma(l % 32),
+ *   sigma(16 a + 8 c + 4 h + d) = 16 a + 8 h + 4 c + d, column 16 s + 8 (l / 32) + e of W1;
  * w2 : [C / 32][hidden / 16][64][8], the same element is row 32 b + tau(l % 32), tau(8 a + 4 h + c) = 16 h + 4 a + c, column
- *   16 s + 8 (e / 4) + 4 (l / 32) + e % 4 of W2;  b1 : [hidden];  b2 : [C]. */
+ *   16 s + 8 (l / 32) + e of W2;  b1 : [hidden];  b2 : [C]. */
 int ffk_transition_block(void* out, const void* x, void* xtail, const void* gamma, const void* beta, const void* w1,
                          const void* b1, const void* w2, const void* b2, int64_t M, int64_t C, int64_t hidden, float eps,
                          int dtype, void* stream);

@@ -28,3 +28,19 @@ def test_attention_block_weights_are_five_of_one_size(C):
     for i, part in enumerate((*qkv.split(C), gate)):
         assert torch.equal(w[i], F_.pack_fragments(part, torch.bfloat16, "cpu"))
     assert torch.equal(w[4], F_.pack_fragments_of_accumulators(out, torch.bfloat16, "cpu"))
+
+
+@pytest.mark.parametrize("C,hidden", [(64, 128), (64, 256), (128, 512)])
+def test_transition_weights_against_their_definition(C, hidden):
+    w1, w2 = (torch.randn(*n, generator=torch.Generator().manual_seed(C)).bfloat16() for n in ((hidden, C), (C, hidden)))
+    p1, p2 = F_.pack_transition_block(w1, w2, torch.bfloat16, "cpu")
+    lane = torch.arange(64)
+    row, half = lane % 32, lane // 32
+    sigma = 16 * (row >> 4) + 8 * (row >> 2 & 1) + 4 * (row >> 3 & 1) + (row & 3)
+    tau = 16 * (row >> 2 & 1) + 4 * (row >> 3) + (row & 3)
+    for w, p, perm in ((w1, p1, sigma), (w2, p2, tau)):
+        n, K = w.shape
+        p = p.view(n // 32, K // 16, 64, 8)
+        for b in range(n // 32):
+            for s in range(K // 16):
+                assert torch.equal(p[b, s], w[(32 * b + perm)[:, None], 16 * s + 8 * half[:, None] + torch.arange(8)])

@@ -49,3 +49,27 @@ def test_transition_block_refuses(dev):
         _lib.transition_block(x, x, v, v, x, v, x, v, M=64, C=128, hidden=256)
     with pytest.raises(RuntimeError, match="bf16"):
         _lib.transition_block(x.float(), x.float(), v, v, x, v, x, v, M=64, C=64, hidden=256)
+
+
+@pytest.mark.parametrize("C,M", [(C, M) for C in (128, 256) for M in (1, 63, 1000, 16384 - 40, 16384 + 40, 40000)])
+@pytest.mark.parametrize("tail", [False, True])
+def test_both_kernels_of_a_transition_give_the_same_bits(dev, C, M, tail):
+    """Rows go to one or the other by their number, and a piece of the rows has to get the bits of all of them."""
+    from fastfold_amd import _lib
+    from fastfold_amd.model.fastnn import _fused as F_
+    g = torch.Generator().manual_seed(C + M)
+    H = 4 * C
+
+    def rnd(*shape, scale=1.0, shift=0.0):
+        return (torch.randn(*shape, generator=g) * scale + shift).to(dev, BF)
+    x = rnd(M, C, scale=1.5, shift=0.3)
+    gam, bet, b1, b2 = rnd(C, scale=0.1, shift=1.0), rnd(C, scale=0.1), rnd(H), rnd(C)
+    w1, w2 = rnd(H, C, scale=C ** -0.5), rnd(C, H, scale=H ** -0.5)
+    p1, p2 = F_.pack_transition_block(w1, w2, BF, dev)
+    tails = [torch.randint(-100, 100, (M, C), generator=g, dtype=torch.int8).to(dev)] * 2 if tail else [None, None]
+    tails = [t if t is None else t.clone() for t in tails]
+    outs = [torch.empty_like(x), torch.empty_like(x)]
+    _lib.transition_fused(outs[0], x, gam, bet, w1, b1, w2, b2, M=M, C=C, hidden=H, xtail=tails[0])
+    _lib.transition_block(outs[1], x, gam, bet, p1, b1, p2, b2, M=M, C=C, hidden=H, xtail=tails[1])
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and (not tail or torch.equal(tails[0], tails[1]))
