@@ -27,7 +27,7 @@
 //                            with a pair bias:  128 rows of 96 tokens 45 -> 29, of 128 tokens 51 -> 36
 //   the same to the gated heads, output projection apart (k and v of four heads of 256 tokens fill the LDS: two workgroups to a row):
 //                            128 rows of 160 tokens 67 -> 49, 192 74 -> 53, 256 87 -> 72;  512 rows of 256 296 -> 228
-// For which numbers of rows: attention_block_pays in model/fastnn/_fused.py.  Longer rows do not fit: at 128 channels, k and v of more than 256 tokens go into LDS in two passes only (heads two by two, rows
+// Other numbers of rows: attention_block_tokens in model/fastnn/_fused.py.  Longer rows do not fit: at 128 channels, k and v of more than 256 tokens go into LDS in two passes only (heads two by two, rows
 // normalised twice), which was built and is slower (288 tokens 122 us against 92, 416 235 against 189).
 #include "ffk_rowblock.h"
 #include <type_traits>

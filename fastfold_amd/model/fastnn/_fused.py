@@ -265,37 +265,25 @@ def key_bias(mask, device, *, B2, N, mask_sb, mask_sn):
 
 
 def attention_block_tokens(dtype, H, c, d_in, d_out):
-    """Longest row of tokens that ``ffk_attention_block`` takes at these widths, 0 where it is not built for them (timings of both
-    sides in csrc/ffk_attention_block.hip and below)."""
+    """Longest row of tokens that ``ffk_attention_block`` takes at these widths, 0 where it is not built for them.
+
+    Rows go to it by their length and width only, never by how many there are: a subset of the batch rows must give the bits of the
+    full call.  One row keeps a CU busy whatever the others do, so it loses where few long rows leave CUs idle or the last round of
+    rows is nearly empty.  us per sub-module, one kernel / launches of their own:
+      128 channels in heads of 32, N rows of N tokens: 32 13.4 / 14.0, 96 19.3 / 24.5, 160 28 / 43, 224 42 / 64, 256 49 / 67
+      64 channels in heads of 16, the same: 64 11.0 / 18.5, 256 31 / 52, 288 68 / 71, 320 76 / 83, 352 92 / 94, 384 98 / 104, 512 161 / 191
+      64 channels in heads of 8, 64 / 256 / 384 / 1 024 rows: 96 tokens 18 / 22, 19 / 36, 30 / 47, 54 / 79; 160 31 / 29, 32 / 55, 53 / 70,
+        99 / 150; 256 46 / 34, 49 / 69, 86 / 91, 163 / 205; 384 92 / 47, 96 / 114, 170 / 154, 327 / 397 (of the 64 rows that a stack of
+        extra sequences hardly has, more than 192 tokens lose; from 192 rows on all lengths win but at 384 rows)
+      256 channels without a bias, 32 / 64 / 256 / 1 024 rows: 64 tokens 14 / 19, 15 / 23, 18 / 47, 66 / 132; 96 20.5 / 21.8, 21 / 31, 27 / 61,
+        101 / 213; 128 27.5 / 24.0, 28 / 34, 34 / 72, 126 / 276
+      256 channels with one, 32 / 64 / 128 / 512 rows: 96 tokens 27 / 28, 27 / 37, 28 / 47, 61 / 106; 128 35 / 31, 35 / 39, 36 / 55, 77 / 135
+      the heads apart (``ATTENTION_HEADS_TOKENS``), 32 / 64 / 128 / 160 / 512 rows: 160 tokens 36.7 / 36.8, 42 / 48, 49 / 68, 71 / 82, 142 / 190;
+        192 42 / 38, 47 / 50, 54 / 75, 80 / 87, 164 / 233; 224 51 / 39, 55 / 56, 66 / 85, 99 / 100, 203 / 271; 256 57 / 40, 61 / 58, 73 / 89,
+        110 / 104, 232 / 303"""
     if dtype != torch.bfloat16 or d_in != d_out or H * c != d_in:
         return 0
     return {(128, 32): 256, (64, 16): 512, (64, 8): 384, (256, 32): 128}.get((d_in, c), 0)
-
-
-def attention_block_pays(C, head_dim, N, B2, biased):
-    """Whether ``ffk_attention_block`` (``ffk_attention_heads``) beats launches of their own for B2 rows of N tokens.  One row keeps a
-    CU busy, whatever the others do (two CUs where the heads are split), so what counts is how full the last round of rows is.
-    us per sub-module, one kernel / launches of their own:
-      256 channels, no bias: 128 tokens, 32 rows 27 / 24, 40 28 / 30, 64 28 / 34, 260 57 / 82; 96 tokens, 24 rows 20 / 21
-      256 channels with a bias: 128 tokens, 32 rows 35 / 31, 48 35 / 38, 260 69 / 92; 96 tokens, 16 rows 27 / 25, 32 27 / 28;
-        heads apart: 160 tokens, 32 rows 37 / 37, 130 69 / 75; 192, 60 rows 47 / 49, 130 80 / 83; 224, 60 rows 55 / 54, 130 95 / 88,
-        200 102 / 119; 256, 60 rows 61 / 57, 90 65 / 74, 130 109 / 101, 180 115 / 114, 200 117 / 135
-      64 channels in heads of 8: 96 tokens, 80 rows 18 / 24, 260 29 / 39; 160, 64 rows 31 / 29, 140 31 / 41; 256, 140 rows 46 / 51,
-        200 47 / 63, 300 83 / 78, 380 84 / 89; 320, 380 rows 133 / 129, 600 193 / 189, 700 193 / 216; 384, 600 rows 244 / 223, 700 244 / 253
-    The other widths have as many rows as tokens, and it wins at every length it takes."""
-    cus = 256
-    wgs = B2 * 2 if C == 256 and N > 128 else B2
-    rounds = -(-wgs // cus)
-    fill = wgs / (cus * rounds)
-    if C == 64 and head_dim == 8:
-        return N <= 96 or fill >= 0.35 + 0.56 * (N - 96) / 288
-    if C < 256:
-        return True
-    if rounds > 1:
-        return N <= 192 or fill >= 0.75
-    if N > 128:
-        return fill >= N / 384
-    return N <= 64 or B2 >= N // (3 if biased else 4)
 
 
 def pack_attention_block(qkv_w, gate_w, out_w, dtype, device):
@@ -385,8 +373,7 @@ def attention(x, out, resid, *, B2, N, C, H, a_map, ln, w_pk, gate_bias_pk, wo_p
     # kernel, which writes q, k and the gate in accumulator order straight from its registers.
     acc_order = dt == torch.bfloat16 and C in (64, 128, 256) and N % 32 == 0
     # Short rows: one kernel from the rows of x to the updated rows.
-    enough = attention_block_pays(C, head_dim, N, B2, bias_t is not None or bias_in_launch)
-    short = _ATTENTION_BLOCK and enough and acc_order and hasattr(w_pk, "block") and ln is not None and aligned16(*ln)
+    short = _ATTENTION_BLOCK and acc_order and hasattr(w_pk, "block") and ln is not None and aligned16(*ln)
     if (short and N <= attention_block_tokens(dt, H, head_dim, C, c_out)
             and resid is not None and resid.data_ptr() == x.data_ptr() and o_map is None
             and a_so % 16 == 0 and a_si % 16 == 0 and (C == 256 or bias_t is not None or bias_in_launch)

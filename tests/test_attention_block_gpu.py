@@ -211,6 +211,30 @@ def test_modules_take_the_block_and_match_the_separate_launches(dev, monkeypatch
         assert float(upd.norm()) > 1.0 and err < 2 * TOL, (type(mod).__name__, args[0].shape, err)
 
 
+@pytest.mark.parametrize("rows,tokens,C,D", [(300, 128, 256, 0), (200, 96, 256, 32), (256, 256, 256, 32), (512, 256, 64, 8)])
+def test_a_subset_of_the_rows_gives_the_bits_of_all(dev, rows, tokens, C, D):
+    """Column attention (D = 0) and row attention of few rows, a single one and all of them."""
+    from fastfold_amd.model.fastnn.msa import MSAColumnAttention, MSARowAttentionWithPairBias
+    torch.manual_seed(tokens)
+    mod = MSAColumnAttention(C) if D == 0 else MSARowAttentionWithPairBias(C, 128, c=D, n_head=C // D)
+    with torch.no_grad():
+        for n, p in mod.named_parameters():
+            p.copy_(1 + 0.1 * torch.randn_like(p) if "layernorm" in n and n.endswith("weight")
+                    else torch.randn_like(p) * (0.3 if p.dim() == 1 else p.shape[-1] ** -0.5))
+    mod = mod.to(dev, BF).eval()
+    m = torch.randn(1, rows, tokens, C, device=dev).to(BF)
+    mask = (torch.rand(1, rows, tokens, device=dev) > 0.2).to(BF)
+    z = torch.randn(1, tokens, tokens, 128, device=dev).to(BF)
+
+    def run(m, mask):
+        with torch.no_grad():
+            return mod(m.transpose(1, 2).contiguous(), mask.transpose(1, 2).contiguous()).transpose(1, 2) if D == 0 else mod(m, z, mask)
+    full = run(m, mask)
+    assert float((full - m).float().abs().max()) > 0.1
+    for lo, hi in ((5, 36), (0, 1), (rows - 60, rows)):
+        assert torch.equal(run(m[:, lo:hi].contiguous(), mask[:, lo:hi].contiguous()), full[:, lo:hi]), (lo, hi)
+
+
 def test_weights_of_short_rows_are_laid_out_with_the_others(dev):
     """The first pass of a triangle attention lays out all weights: the first pass at a length that takes another route builds
     nothing, so a stack can record it."""

@@ -76,3 +76,23 @@ def test_normalisation_weights_may_lie_anywhere(calls, i):
             mod(*args)
         short = [n for n in calls if n in ("ffk_attention_block", "ffk_attention_heads", "ffk_transition_block")]
         assert bool(short) == aligned, calls
+
+
+@pytest.mark.parametrize("r", [32, 96, 128, 160, 224, 256, 384])
+def test_the_route_of_an_attention_does_not_depend_on_the_number_of_rows(calls, r):
+    """A share of the batch rows (a rank's, a caller's piece) gets the bits of the full call, so it takes the same launches."""
+    from fastfold_amd.model.fastnn import msa
+    row, ext, col = (_module(*a, **kw) for a, kw in (((msa.MSARowAttentionWithPairBias, 256, 128), dict(c=32, n_head=8)),
+                                                     ((msa.MSARowAttentionWithPairBias, 64, 128), dict(c=8, n_head=8)),
+                                                     ((msa.MSAColumnAttention, 256), {})))
+    z = torch.zeros(1, r, r, 128, dtype=BF)
+    for mod, c in ((row, 256), (ext, 64), (col, 256)):
+        routes = set()
+        for b2 in (1, 31, 33, 60, 130, 300):
+            m = torch.zeros(1, r, b2, c, dtype=BF) if mod is col else torch.zeros(1, b2, r, c, dtype=BF)
+            mask = torch.ones(m.shape[:3], dtype=BF)
+            del calls[:]
+            with torch.no_grad():
+                mod(m, mask) if mod is col else mod(m, z, mask)
+            routes.add(tuple(calls))
+        assert len(routes) == 1, routes
