@@ -468,8 +468,9 @@ constexpr int PAIR_THREADS = 256;
 // row's products beside the other row's exponentials, in an order that is written down; K and the bias of a step are read a step
 // ahead of V (four ring slots), and products go first where two waves ask (s_setprio: 2 %).  The bias tile is multiplied by the
 // identity once for both rows: its accumulator is the C operand of their scores (five products per tile, not six), which leaves no
-// place for a row's reference, so the reference is zero: sums of exp2 within OPT_LOW .. OPT_HIGH prove that nothing over- or
-// underflowed; a workgroup without that proof walks again with a running maximum.
+// place for a row's reference, so the reference is zero.  Sums of exp2 within OPT_LOW .. OPT_HIGH prove that no probability over- or
+// underflowed, weighted sums that are numbers and, where the row's sum is below one, not all below OUT_LOW that no product with v did
+// (large v beside a large sum, small v beside a small one); a workgroup without that proof walks again with a running maximum.
 // Before -> after, us: 64 rows x 4 heads of 4 096 queries 888 -> 780, 1 024 x 4 of 1 024 984 -> 920, 391 x 4 of 391 99 -> 94, 320 x 4 of 320
 // 53.0 -> 49.0.  Of the 190 ns a tile takes at 4 096 queries its instructions take 148, LDS 14, the barrier 7 and
 // the ring's requests the rest.  Without a bias (212 -> 213 us, 128 x 8 of 1 024) the kernel above stays.  Workgroup = 2 batch rows x 4
@@ -482,6 +483,7 @@ __global__ __launch_bounds__(PAIR_THREADS, 2) void attention_pair_kernel(
     constexpr int NTILES = 8;                     // operand tiles per key step: K0 K1 V0 V1 B0 .. B3
     constexpr int NVL = 4, NSLOT = 4;             // 16-byte vectors per thread and step
     constexpr float OPT_HIGH = 1.2676506e30f, OPT_LOW = 8.2718061e-25f;        // 2^100, 2^-80
+    constexpr unsigned OUT_LOW = 27u << 23;       // 2^-100
     constexpr float REF_FLOOR = -1.0e4f;
     extern __shared__ __align__(16) unsigned char att_smem[];
     bf16_t* lds = reinterpret_cast<bf16_t*>(att_smem);       // [NSLOT][NTILES][1024]
@@ -758,7 +760,14 @@ __global__ __launch_bounds__(PAIR_THREADS, 2) void attention_pair_kernel(
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
             l_tot[r] = l_run[r] + lane_xor<32>(l_run[r]);
-            bool out_of_range = live[r] && q < Nq && !(l_tot[r] <= OPT_HIGH && l_tot[r] >= OPT_LOW);
+            unsigned big = 0;                     // largest magnitude of the lane's outputs; infinities and NaN above all numbers
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const unsigned m = __builtin_bit_cast(unsigned, o_acc[r][v]) & 0x7FFFFFFFu;
+                big = big > m ? big : m;
+            }
+            const bool sound = l_tot[r] <= OPT_HIGH && l_tot[r] >= OPT_LOW && big < 0x7F800000u && (l_tot[r] >= 1.0f || big >= OUT_LOW);
+            const bool out_of_range = live[r] && q < Nq && !sound;
             if (__builtin_amdgcn_ballot_w64(out_of_range) != 0) {
                 bool any = false;                 // a row without keys has a sum of zero, and zeros for its result
                 for (int kt = 0; kt < KT; ++kt) any = any || (r ? fl1 : fl0)[kt] != 2;
@@ -1058,7 +1067,10 @@ extern "C" int ffk_attention_fwd_lse(void* out, float* lse, const void* q_t, con
     switch (dtype) {
         case FFK_BF16:
             // Two rows per wave (FFK_ATT_HALF_K or not: the padding adds nothing) for a bias and more than 256 keys, one row / two, us:
-            // 256 x 4 heads of 256 queries 26.8 / 28.0, 320 x 4 of 320 53.0 / 49.0, 128 x 4 of 512 41 / 38, and see there.  With the
+            // 256 x 4 heads of 256 queries 26.8 / 28.0, 320 x 4 of 320 53.0 / 49.0, 128 x 4 of 512 41 / 38, and see there.  Few rows (the
+            // one-row kernel with its log-sum-exp), 1 / 8 / 32 / 64 x 4 of 288: 8.1 / 8.0, 8.6 / 8.6, 9.1 / 9.0, 12.7 / 12.6; of 512: 11.4 / 10.8,
+            // 11.8 / 11.6, 13.0 / 12.8, 19.2 / 20.0; of 1 024: 19.2 / 17.6, 19.7 / 18.8, 31.2 / 31.3, 59 / 58; of 2 048: 34 / 32, 36 / 35, 110 / 105,
+            // 217 / 204.  With the
             // log-sum-exp, from sums of probabilities that were not rounded against a zero reference, 256 x 4 of 256 27.0 / 29.3,
             // 391 x 4 of 391 102 / 102: one row.
             if (bias_t && !lse && Nk > 256) return launch_attention_pair(out, q_t, k_t, v_t, bias_t, keybias, tileflags, gate, B2, H, Nq, Nk, flags, st);

@@ -9,12 +9,12 @@ pytestmark = pytest.mark.gpu
 BF = torch.bfloat16
 
 
-def _case(dev, B2, H, N, shift, mask):
+def _case(dev, B2, H, N, shift, mask, v_scale=1.0):
     from fastfold_amd import _lib
     from fastfold_amd.model.fastnn.kernel import layouts
     g = torch.Generator().manual_seed(N * 7 + B2)
     q, k, v = (torch.randn(B2, H, N, 32, generator=g).to(BF) for _ in range(3))
-    q = (q.float() * 0.25).to(BF)
+    q, v = (q.float() * 0.25).to(BF), (v.float() * v_scale).to(BF)
     bias = torch.randn(H, N, N, generator=g) * 2
     if shift is not None:                       # log2 units added to every score of a query: nothing changes
         bias = bias + torch.tensor(shift).repeat(N // len(shift) + 1)[:N][None, :, None]
@@ -38,7 +38,7 @@ def _case(dev, B2, H, N, shift, mask):
     # probabilities rounded to bf16, in the numerator and in the denominator, and the result: at most 2^-8 each of the mean of |v|
     size = torch.where(l > 0, (p @ v.double().abs()) / l.clamp_min(1e-300), torch.zeros(()).double()).permute(0, 2, 1, 3).reshape(B2, N, H * 32)
     err = (out.cpu().double() - want).abs()
-    assert bool((err <= 3 * 2.0 ** -8 * size + 1e-30).all()), float((err / size.clamp_min(1e-30)).max())
+    assert bool((err <= 3 * 2.0 ** -8 * size + 1e-30 * min(v_scale, 1.0)).all()), float((err / size.clamp_min(1e-30)).max())
 
 
 @pytest.mark.parametrize("B2,N", [(1, 257), (2, 288), (3, 289), (2, 320), (5, 321), (1, 384), (3, 385), (2, 500), (1, 1030), (2, 1152)])
@@ -50,6 +50,13 @@ def test_edges(dev, B2, N):
 @pytest.mark.parametrize("shift", [(60.0,), (-60.0,), (-100.0,), (120.0,), (2048.0,), (-2048.0,), (0.0, 0.0, -512.0, 0.0, 64.0, 512.0)])
 def test_scores_far_from_zero(dev, shift):
     _case(dev, 3, 2, 300, shift, None)
+
+
+# sums of probabilities within range whose products with v are not: beyond the largest number, and below the smallest normal one; and
+# values of the same size beside sums of the other kind
+@pytest.mark.parametrize("shift,v_scale", [((60.0,), 1e30), ((-60.0,), 1e-25), ((-75.0,), 1e-30), ((90.0, 0.0), 1e15), ((60.0,), 1e-30), ((-60.0,), 1e30)])
+def test_values_far_from_one(dev, shift, v_scale):
+    _case(dev, 3, 2, 300, shift, None, v_scale)
 
 
 @pytest.mark.parametrize("N", [270, 400])
