@@ -19,6 +19,8 @@
 // What it replaces moves q, k, v, the gate and the heads' outputs through memory and fills and drains the chip three times.
 // us per sub-module, launches of their own -> here (both with the launch that computes the pair bias):
 //   128 channels in 4 heads, N rows of N tokens:  N = 64 17.7 -> 15.0, 96 24.6 -> 19.6, 128 29.4 -> 22.8, 192 49 -> 33.5, 256 62 -> 48
+//     (the gate in fp32 until it multiplies: no slower with a fourth tile's in LDS, 48.1 -> 54.3 with registers spilled for it; relative
+//     error of the update against float64, launches of their own / gate in bf16 / in fp32: 5.00e-3 / 4.96e-3 / 4.77e-3)
 //   64 channels in 4 heads:  N = 64 18.6 -> 11.1, 128 26.0 -> 15.0, 256 50.5 -> 32, 320 79 -> 77, 512 184 -> 171
 //     (row sums of the probabilities as the matrix product's idle rows instead of eight dot instructions a tile: 320 77 -> 71, 512 171 -> 157)
 //   64 channels in 8 heads, 1 024 rows of N tokens:  N = 64 68 -> 39, 160 147 -> 96, 256 196 -> 157, 384 376 -> 320
@@ -59,8 +61,11 @@ template <int C, int D, int TPW> struct AbGeo {
     static constexpr int XP = C * 2 + 16;           // pitch of the normalised rows (bytes)
     static constexpr int HP = WB * 64 + 16;         // HEADS: pitch of the gated outputs
     static constexpr bool ONES = D < 32;            // row sums through the weighted sum's product (see attend)
-    static constexpr size_t smem(long NT) {         // rows, then k and v (and a tile of ones), then the gated outputs (and the updates)
-        const size_t rows = (size_t)NT * 32 * XP, kv = (size_t)NT * WB * 4096 + (ONES ? 2048 : 0), end = HEADS ? 0 : rows + (size_t)NT * NB * 2048;
+    static constexpr bool GATE32 = C == 128;        // the gate stays in fp32 until it multiplies, as in ffk_gated_out_fused,
+    static constexpr bool GATE_LDS = GATE32 && TPW == 4;       // that of a wave's fourth tile in LDS, behind k and v
+    static constexpr size_t smem(long NT) {         // rows, then k and v (and a tile of ones or of the gate), then the gated outputs (and the updates)
+        const size_t rows = (size_t)NT * 32 * XP, kv = (size_t)NT * WB * 4096 + (ONES ? 2048 : 0) + (GATE_LDS ? 32768 : 0),
+                     end = HEADS ? 0 : rows + (size_t)NT * NB * 2048;
         return rows > kv ? (rows > end ? rows : end) : (kv > end ? kv : end);
     }
 };
@@ -308,7 +313,9 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
         inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;              // all keys masked: zero
     };
 
-    bf16x8 of[TPW][2];                       // gate, then gated outputs
+    bf16x8 of[TPW][2];                       // gate (but for GATE32), then gated outputs
+    f32x16 gate[G::GATE32 ? TPW : 1];
+    f32x4* const s_gate = reinterpret_cast<f32x4*>(ab_smem + (size_t)NT * WB * 4096) + tid;        // [4][512], each lane its own
     request(wptr(1, blk));
     rb_normalise<C, G::NT_MAX>(a, xrow, s_x, NT, wave, lane);
     lds_barrier();
@@ -347,13 +354,24 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
             bg[g] = __builtin_bit_cast(bf16x4, *reinterpret_cast<const u32x2*>(a.bg + blk * 32 + 4 * half + 8 * g));
         project(std::false_type(), (const T*)nullptr, acc);
 #pragma unroll
-        for (int i = 0; i < TPW; ++i)
+        for (int i = 0; i < TPW; ++i) {
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) of[i][j][e] = (T)sigmoid_f(acc[i][8 * j + e] + (float)bg[2 * j + (e >> 2)][e & 3]);
-                rb_pin(of[i][j]);
+                for (int e = 0; e < 8; ++e) {
+                    const float y = sigmoid_f(acc[i][8 * j + e] + (float)bg[2 * j + (e >> 2)][e & 3]);
+                    if (G::GATE32) gate[i][8 * j + e] = y;
+                    else of[i][j][e] = (T)y;
+                }
+                if (!G::GATE32) rb_pin(of[i][j]);
             }
+            if constexpr (G::GATE32) asm volatile("" : "+v"(gate[i]));        // one tile after the other
+            if constexpr (G::GATE_LDS)
+                if (i == 3) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) s_gate[v * 512] = f32x4{gate[i][4 * v], gate[i][4 * v + 1], gate[i][4 * v + 2], gate[i][4 * v + 3]};
+                }
+        }
         lds_barrier();                           // nobody reads the rows any more
         if (G::ONES && tid < 128) *reinterpret_cast<u32x4*>(s_one + tid * 8) = u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
 #pragma unroll
@@ -384,12 +402,21 @@ __global__ __launch_bounds__(512, 2) void attention_block_kernel(const AbArgs a)
                 float inv;
                 const T* next = sub + 1 < HPB ? bias_row(i, sub + 1) : bias_row(i + 1 < TPW ? i + 1 : i, 0);
                 attend(sub, bias_row(i, sub), next, qf[i][0], qf[i][1], acc, inv);
+                if constexpr (G::GATE_LDS)
+                    if (i == 3) {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            const f32x4 y = s_gate[v * 512];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) gate[i][4 * v + e] = y[e];
+                        }
+                    }
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
                     if (8 * j + 7 < sub * (D / 2) || 8 * j >= (sub + 1) * (D / 2)) continue;
 #pragma unroll
                     for (int e = 0; e < 8; ++e)      // the head's registers
-                        if ((8 * j + e) / (D / 2) == sub) of[i][j][e] = (T)(acc[8 * j + e] * inv * (float)of[i][j][e]);
+                        if ((8 * j + e) / (D / 2) == sub) of[i][j][e] = (T)(acc[8 * j + e] * inv * (G::GATE32 ? gate[i][8 * j + e] : (float)of[i][j][e]));
                     rb_pin(of[i][j]);
                 }
             }

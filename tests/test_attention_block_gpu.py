@@ -150,6 +150,24 @@ def test_attention_heads_against_float64(dev, N):
     assert float(o[2].abs().max()) == 0.0                     # no key at all
 
 
+@pytest.mark.parametrize("N", [64, 96, 160, 200, 224, 256])
+def test_the_gate_of_128_channels_is_not_rounded_ahead_of_its_product(dev, N):
+    """Uniform attention over equal exact values and an output projection that is the identity: one rounding to bf16, of gate times
+    value, is all that happens."""
+    C, v = 128, 1.1015625
+    g = torch.Generator().manual_seed(N)
+    eye = torch.eye(C)
+    p = dict(C=C, D=32, H=4, B2=3, N=N, qkv=torch.cat([torch.zeros(2 * C, C), eye]).to(dev, BF), wg=torch.zeros(C, C, device=dev, dtype=BF),
+             bg=torch.randn(C, generator=g).to(dev, BF), wo=eye.to(dev, BF), gam=torch.zeros(C, device=dev, dtype=BF),
+             bet=torch.full((C,), v, device=dev, dtype=BF), x=torch.zeros(3, N, C, device=dev, dtype=BF),
+             bias=torch.zeros(4, N, N, device=dev, dtype=BF), mask=torch.ones(3, N, device=dev, dtype=BF))
+    out = torch.empty_like(p["x"])
+    _run(p, p["x"], out)
+    want = torch.sigmoid(p["bg"].double().cpu()) * v
+    # half a step of the result, and 2^-20 for the fp32 exponential, reciprocals and mean
+    assert bool(((out.double().cpu() - want).abs() <= (2.0 ** -9 + 2.0 ** -20) * 2.0 ** want.log2().floor() * 2).all())
+
+
 def test_attention_block_refuses(dev):
     p = _case(dev, 256, 32, 2, 129, seed=0)
     with pytest.raises(RuntimeError, match="too long"):
