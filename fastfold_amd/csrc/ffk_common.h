@@ -338,24 +338,30 @@ __device__ __forceinline__ float centre8(float (&f)[8], float mean) {
     return q;
 }
 
-// fp32 products on the bf16 matrix pipe.  An fp32 number is the sum of three bf16 numbers (x = x1 + x2 + x3 exactly, but for what lies
-// below the smallest normal number): the first cut off, so that a finite number has finite parts, the others rounded, so that what is
-// left out has either sign; and
-//     x y = x1 y3 + x3 y1 + x2 y2 + x1 y2 + x2 y1 + x1 y1      up to 2^-24 |x y|,
-// added from the smallest to the largest term in the fp32 accumulator.  Six v_mfma_f32_32x32x16_bf16 take 196 cycles for a K step of 16,
-// eight v_mfma_f32_32x32x2_f32 512, and the bf16 ones let the vector instructions of other waves run beside them.  The error of a sum is
-// lower than by the fp32 instructions (sixteen products are added per rounding, not two).  Relative error (2-norm) against float64, fp32
-// instructions -> this, as ffk_bgemm_nt adds them: normal numbers, K = 64 1.44e-7 -> 1.12e-7, 128 2.03e-7 -> 1.65e-7, 256 2.88e-7 -> 2.38e-7,
-// 496 3.99e-7 -> 3.38e-7; positive numbers, 64 1.22e-7 -> 0.90e-7, 256 2.47e-7 -> 2.06e-7, 496 3.43e-7 -> 2.87e-7.  Longer chains are for
-// the callers to cut: the instruction cuts off towards minus infinity what the accumulator has no room for.  The
-// parts of an infinite operand make NaN of its products: a kernel that finds one in its sums takes the fp32 instructions for them.
+// fp32 products on the bf16 matrix pipe.  An fp32 number is the sum of three bf16 numbers, each the rounded rest of the ones before
+// (x = x1 + x2 + x3 exactly, but for what lies below the smallest normal number); of a number in [2^e, 2^(e+1)) the second is at most
+// 2^(e-8) and the third at most 2^(e-17), so that in
+//     x y = x1 y3 + x3 y1 + x2 y2 + x1 y2 + x2 y1 + x1 y1
+// at most 2^-24 (1 + 2^-10) |x y| is left out, of either sign.  (With the first part cut off instead of rounded it would be up to 2^-22, and
+// of one sign for operands of like mantissas: sums of 384 products of numbers just below 1 + 2^-7 4.6e-7 -> 2.5e-7, 256 products 3.0e-7 ->
+// 1.8e-7.)  The terms are added from the smallest to the largest in the fp32 accumulator.  Six v_mfma_f32_32x32x16_bf16 take 196 cycles
+// for a K step of 16, eight v_mfma_f32_32x32x2_f32 512, and the bf16 ones let the vector instructions of other waves run beside them.
+// The error of a sum is no larger than by the fp32 instructions from four products on (sixteen products are added per rounding, not two).
+// Relative error (2-norm) against float64, fp32 instructions -> this, as ffk_bgemm_nt adds them: normal numbers, K = 4 3.99e-8 -> 3.26e-8,
+// 16 7.4e-8 -> 3.4e-8, 64 1.43e-7 -> 1.09e-7, 128 2.05e-7 -> 1.64e-7, 256 2.86e-7 -> 2.36e-7, 384 3.52e-7 -> 2.94e-7; positive numbers, 4
+// 3.66e-8 -> 2.91e-8, 64 1.22e-7 -> 0.89e-7, 256 2.45e-7 -> 1.98e-7, 384 2.67e-7 -> 2.17e-7.
+// Longer chains are for the callers to cut: the instruction cuts off towards minus infinity what the accumulator has no room for.  The
+// parts of an infinite operand (and of a finite one that rounds to infinity, unless BOUND) make NaN of its products: a kernel that finds
+// one in its sums takes the fp32 instructions for them.
 struct Split4 {              // four numbers, part by part
     u32x2 p[3];
 };
-// PIN: not to be moved out of a loop
-template <bool PIN = false> __device__ __forceinline__ Split4 split4(const f32x4& x) {
+// PIN: not to be moved out of a loop.  BOUND: the first part at most the largest bf16 number, so that the parts of every finite number are
+// finite and split_sum gives it back (one more instruction a number).
+template <bool PIN = false, bool BOUND = false> __device__ __forceinline__ Split4 split4(const f32x4& x) {
     typedef float f32x2 __attribute__((ext_vector_type(2)));
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    constexpr float TOP = 3.3895313892515355e38f;
     Split4 r;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -363,8 +369,9 @@ template <bool PIN = false> __device__ __forceinline__ Split4 split4(const f32x4
 #pragma unroll
         for (int p = 0; p < 3; ++p) {
             uint32_t h;
-            if (PIN && p == 0) asm volatile("v_perm_b32 %0, %1, %2, %3" : "=v"(h) : "v"(b), "v"(a), "s"(0x07060302u));
-            else if (p == 0) h = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
+            if (PIN && p == 0) asm volatile("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h) : "v"(a), "v"(b));
+            else if (BOUND && p == 0)
+                h = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{__builtin_amdgcn_fmed3f(a, -TOP, TOP), __builtin_amdgcn_fmed3f(b, -TOP, TOP)}, bf16x2));
             else h = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
             r.p[p][j] = h;
             a -= __builtin_bit_cast(float, h << 16);
@@ -377,8 +384,8 @@ template <bool PIN = false> __device__ __forceinline__ Split4 split4(const f32x4
 __device__ __forceinline__ bf16x8 split_frag(const Split4& a, const Split4& b, int p) {
     return __builtin_bit_cast(bf16x8, u32x4{a.p[p][0], a.p[p][1], b.p[p][0], b.p[p][1]});
 }
-// the number whose parts these are; an infinite one has parts that are no numbers
-__device__ __forceinline__ float split_sum(float a, float b, float c) { return a - a == 0.0f ? a + b + c : a; }
+// the number whose parts (BOUND) these are; of an infinite or undefined one the second part is all that is left
+__device__ __forceinline__ float split_sum(float a, float b, float c) { return b - b == 0.0f ? a + (b + c) : b; }
 // The parts of a product in the order they are added: operand a's part, operand b's
 constexpr int SPLIT_A[6] = {0, 2, 1, 0, 1, 0}, SPLIT_B[6] = {2, 0, 1, 1, 0, 0};
 

@@ -160,7 +160,7 @@ __global__ __launch_bounds__(ONE ? 256 : 512, K == 128 && !GLU && BM == 32 ? 3 :
     if constexpr (G::CUT) {
 #pragma unroll
         for (int g = 0; g < KF / 2; ++g) {
-            const Split4 a = split4(wf[0][2 * g]), b = split4(wf[0][2 * g + 1]);
+            const Split4 a = split4<false, true>(wf[0][2 * g]), b = split4<false, true>(wf[0][2 * g + 1]);
 #pragma unroll
             for (int p = 0; p < 3; ++p) wp[g][p] = split_frag(a, b, p);
         }
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(ONE ? 256 : 512, K == 128 && !GLU && BM == 32 ? 3 :
             if (ln) ffk_ln_rows4<LPR>(pre + i, gam, bet, d.ln_eps);
 #pragma unroll
             for (int j = i; j < i + 4; ++j) {
-                const Split4 x = split4(pre[j]);
+                const Split4 x = split4<false, true>(pre[j]);
 #pragma unroll
                 for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(sa + (r0 + RPP * j) * AP + (c4 >> 2) * 96 + p * 32 + (c4 & 3) * 8) = x.p[p];
             }

@@ -32,12 +32,40 @@ def test_error_of_products(dev, M, K, N, sx, sw):
     g = torch.Generator().manual_seed(M + K + N)
     x, w = (torch.randn(M, K, generator=g) * sx).to(dev), (torch.randn(N, K, generator=g) * sw).to(dev)
     got, want, size = _run(x, w), x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
-    # what is left out of a product: x2 y3 + x3 y2 + x3 y3, less than 2^-23 of it; roundings of the sum: six for a step of 16 and three for
-    # the quarters, each at most 2^-23 (cut off) of the sums of magnitudes
+    # what is left out of a product: x2 y3 + x3 y2 + x3 y3, at most 2^-24 (1 + 2^-10) of it (tests/test_fp32_parts.py); roundings of the sum:
+    # six for a step of 16 and three for the pieces, each at most 2^-23 (cut off) of the sums of magnitudes
     err = (got - want).abs()
     assert bool((err <= (1 + 6 * ((K + 15) // 16) + 3) * 2.0 ** -23 * size).all())
     # independent roundings add up as a random walk: at most what one rounding of 2^-24 for every product of the sum would give
     assert float(err.norm() / want.norm()) <= max(K, 32) ** 0.5 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("K", [4, 128, 256])
+def test_error_of_single_products(dev, K):
+    """Every product by itself, over two million pairs of mantissas: what is left out of one (2^-24 (1 + 2^-10)) and the sum's cutting off of
+    the terms below its last place (2^-23 for the largest of them, 2^-30 for those below 2^-7)."""
+    g = torch.Generator().manual_seed(K)
+    x, w = torch.zeros(2048, K), torch.zeros(1024, K)
+    x[:, K // 2], w[:, K // 2] = (1 + torch.rand(n, generator=g) for n in (2048, 1024))
+    # the mantissas whose parts are as large as they get, among them those of a first part that is cut off
+    x[:4, K // 2] = w[:4, K // 2] = torch.tensor([0x3F80FEFF, 0x3F807F7F, 0x3F80FF7F, 0x3F8080FF], dtype=torch.int32).view(torch.float32)
+    got, want = _run(x.to(dev), w.to(dev)).cpu(), x.double() @ w.double().t()
+    assert float(((got - want) / want).abs().max()) <= 2.0 ** -24 * (1 + 2.0 ** -10) + 2.0 ** -23 + 2.0 ** -28
+
+
+@pytest.mark.parametrize("M,K,N", [(100, 128, 256), (40000, 128, 512), (100, 256, 256), (20000, 256, 256), (300, 64, 64), (300, 1024, 128)])
+def test_operands_that_round_to_infinity_are_finite(dev, M, K, N):
+    """Numbers between the largest bf16 number and the largest fp32 number, on either side."""
+    g = torch.Generator().manual_seed(M)
+    x, w = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g) * 2.0 ** -20
+    top = torch.finfo(torch.float32).max
+    x[3, 5], x[M // 2, 1], x[M - 1, 0] = top, -top, top * (1 - 2.0 ** -9)
+    w[7], x[:, 2], w[:, 2] = 0.0, 0.0, 0.0
+    x[M // 3, 2], w[7, 2] = 2.0 ** -20, -top
+    x, w = x.to(dev), w.to(dev)
+    got, want = _run(x, w), x.double() @ w.double().t()
+    assert bool(got.isfinite().all())
+    assert bool(((got - want).abs().amax(1) <= K ** 0.5 * 2.0 ** -23 * want.abs().amax(1) + 1e-30).all())
 
 
 @pytest.mark.parametrize("M,K,N", [(100, 128, 256), (5000, 128, 512), (40000, 128, 512), (100, 256, 256), (20000, 256, 1024),
