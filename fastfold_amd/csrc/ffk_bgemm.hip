@@ -255,27 +255,36 @@ __global__ __launch_bounds__(THREADS, 2) void bgemm_nt_kernel(const ffk_bgemm_de
         if (wave == 0) acc[0][0] = sum[0][0];
     }
 
-    if constexpr (SPLIT) {                         // infinite operands, whose parts make NaN of every product: anew, product by product
+    // infinite operands, whose parts make NaN of every product: those sums by the fp32 instructions, the others keep their bits; and sums of
+    // fewer products than make up for the six roundings of one (one product 2.6e-8 -> 3.5e-8, two 3.1e-8 -> 3.4e-8, four 4.0e-8 -> 3.3e-8)
+    if constexpr (SPLIT) {
+        const bool few = K <= 4;
 #pragma unroll
         for (int ni = 0; ni < WT; ++ni)
 #pragma unroll
             for (int mi = 0; mi < WT; ++mi) {
+                if (KSPLIT && wave) continue;          // wave 0 has the sums
                 float x = acc[ni][mi][0];
 #pragma unroll
                 for (int v = 1; v < 16; ++v) x += acc[ni][mi][v];
-                if (__builtin_expect(!__any(x - x != 0.0f), 1)) continue;
-                const long m = m0 + wm * WT * 32 + mi * 32 + l32, nb = n0 + wn * WT * 32 + ni * 32;
+                if (__builtin_expect(!few && !__any(x - x != 0.0f), 1)) continue;
+                const long m = m0 + wm * WT * 32 + mi * 32 + l32, n = n0 + wn * WT * 32 + ni * 32 + l32;
                 const T* pa = A + (m < M ? m : M - 1) * d.lda;
+                const T* pb = B + (n < N ? n : N - 1) * d.ldb;
+                f32x16 y;
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    if (acc[ni][mi][v] == acc[ni][mi][v]) continue;
-                    const long n = nb + acc_row(v, lane);
-                    const T* pb = B + (n < N ? n : N - 1) * d.ldb;
-                    float y = 0.0f;
+                for (int v = 0; v < 16; ++v) y[v] = 0.0f;
 #pragma unroll 1
-                    for (int k = 0; k < K; ++k) y = fmaf(pa[k], pb[k], y);
-                    acc[ni][mi][v] = y;
+                for (int k = 4 * half; k - 4 * half < K; k += 8) {
+                    typename MM::Frag fa = {0, 0, 0, 0}, fb = {0, 0, 0, 0};
+                    if (k < K) {
+                        fa = *reinterpret_cast<const typename MM::Frag*>(pa + k);
+                        fb = *reinterpret_cast<const typename MM::Frag*>(pb + k);
+                    }
+                    MM::mma(y, fb, fa);
                 }
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[ni][mi][v] = !few && acc[ni][mi][v] == acc[ni][mi][v] ? acc[ni][mi][v] : y[v];
             }
     }
 

@@ -408,7 +408,7 @@ __global__ __launch_bounds__(ONE ? 256 : 512, K == 128 && !GLU && BM == 32 ? 3 :
                     }
             __builtin_amdgcn_sched_barrier(0);
         }
-        // infinite operands, whose parts make NaN of every product: with the fp32 instructions
+        // infinite operands, whose parts make NaN of every product: those sums with the fp32 instructions, the others keep their bits
         float sum = acc[0][0];
 #pragma unroll
         for (int v = 1; v < 16 * N * R; ++v) sum += acc[v >> 4][v & 15];
@@ -418,8 +418,14 @@ __global__ __launch_bounds__(ONE ? 256 : 512, K == 128 && !GLU && BM == 32 ? 3 :
 #pragma unroll
                 for (int i = 0; i < R; ++i) {
                     f32x16& y = acc[s * R + i];
+                    int l = lane;
+                    asm volatile("" : "+v"(l));              // no address of it kept in registers on the way here
+                    f32x4* const kept = reinterpret_cast<f32x4*>(s_out + wave * G::OP) + l;         // free between this wave's stores
+#pragma unroll
+                    for (int a = 0; a < 4; ++a) kept[a * 64] = f32x4{y[4 * a], y[4 * a + 1], y[4 * a + 2], y[4 * a + 3]};
 #pragma unroll
                     for (int v = 0; v < 16; ++v) y[v] = 0.0f;
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int g = 0; g < K / 16; ++g) {
                         const unsigned char* xp = ap + i * 32 * AP + g * 96;
@@ -442,6 +448,12 @@ __global__ __launch_bounds__(ONE ? 256 : 512, K == 128 && !GLU && BM == 32 ? 3 :
                             else y = __builtin_amdgcn_mfma_f32_32x32x2f32(x, w, y, 0, 0, 0);
                         }
                         __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                    for (int a = 0; a < 4; ++a) {
+                        const f32x4 k = kept[a * 64];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) y[4 * a + e] = k[e] == k[e] ? k[e] : y[4 * a + e];
                     }
                 }
         }

@@ -178,6 +178,8 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
     const bool sums = a.csum != nullptr && k0 == 0 && wk == 0;
     float cs[2] = {0.0f, 0.0f};
     [[maybe_unused]] float turn = slice & 1 ? -1.0f : 1.0f;        // fp32: sign of the products of this piece
+    // fp32: one or two rows by the fp32 instructions (one row 2.6e-8 -> 3.5e-8 by parts, two 3.1e-8 -> 3.4e-8, four 4.0e-8 -> 3.1e-8)
+    [[maybe_unused]] const bool few = m_end - m_begin <= 2;
     f32x16 acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -259,6 +261,10 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
                     for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fy[i], fx[j], acc[i][j], 0, 0, 0);
+                if (few && sums) {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) cs[i] += fy[i];
+                }
             }
         }
     };
@@ -319,22 +325,33 @@ __global__ __launch_bounds__(WG_THREADS, 2) void weight_grad_kernel(const WgArgs
         products(smem + buf * 2 * BUF, plain);
         if (!BF && !plain.value) end_piece();
     };
-    walk(std::false_type());
-    if constexpr (!BF) {                                   // infinite operands, whose parts make NaN of every product: with the fp32 instructions
-        float t = 0.0f;
-#pragma unroll
-        for (int v = 0; v < 64; ++v) t += acc[v >> 5][(v >> 4) & 1][v & 15] = sum[v >> 5][(v >> 4) & 1][v & 15];
+    if constexpr (BF) walk(std::false_type());
+    else {
         int* bad = reinterpret_cast<int*>(smem);
-        lds_barrier();
-        if (lane == 0) bad[wave] = 0;
-        if (t - t != 0.0f) bad[wave] = 1;
-        lds_barrier();
-        if (__builtin_expect(bad[0] | bad[1] | bad[2] | bad[3], 0)) {
-            lds_barrier();
+        if (!few) {
+            walk(std::false_type());
+            float t = 0.0f;
 #pragma unroll
-            for (int v = 0; v < 64; ++v) acc[v >> 5][(v >> 4) & 1][v & 15] = 0.0f;
+            for (int v = 0; v < 64; ++v) t += sum[v >> 5][(v >> 4) & 1][v & 15];
+            lds_barrier();
+            if (lane == 0) bad[wave] = 0;
+            if (t - t != 0.0f) bad[wave] = 1;
+            lds_barrier();
+        }
+        // infinite operands, whose parts make NaN of every product: those sums by the fp32 instructions, the others keep their bits
+        const bool again = few || (bad[0] | bad[1] | bad[2] | bad[3]);
+        if (__builtin_expect(again, 0)) {
+            lds_barrier();
             sign = 0;
             walk(std::true_type());
+#pragma unroll
+            for (int v = 0; v < 64; ++v) {
+                const float y = sum[v >> 5][(v >> 4) & 1][v & 15];
+                if (!few && y == y) acc[v >> 5][(v >> 4) & 1][v & 15] = y;
+            }
+        } else {
+#pragma unroll
+            for (int v = 0; v < 64; ++v) acc[v >> 5][(v >> 4) & 1][v & 15] = sum[v >> 5][(v >> 4) & 1][v & 15];
         }
     }
     float* part = a.part + (long)slice * a.N * a.K;

@@ -83,6 +83,36 @@ def test_infinite_and_undefined_operands(dev, M, K, N):
     assert float((got[ok] - want[ok]).norm() / want[ok].norm()) <= max(K, 32) ** 0.5 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("M,K,N", [(100, 128, 256), (5000, 128, 512), (40000, 128, 512), (100, 256, 256), (20000, 256, 1024),
+                                   (300, 1024, 128), (30000, 512, 128), (300, 64, 64), (3000, 64, 300)])
+def test_other_sums_keep_their_bits(dev, M, K, N):
+    """Infinite and undefined operands change the sums they belong to and no others."""
+    g = torch.Generator().manual_seed(M + K)
+    x, w = torch.randn(M, K, generator=g).to(dev), torch.randn(N, K, generator=g).to(dev)
+    clean = _run(x, w)
+    rows, cols = [3, M // 2, M - 1], [7, N - 1]
+    x[3, 5], x[M // 2, 1], x[M - 1, 0], w[7, 9], w[N - 1, 5] = INF, -INF, float("nan"), INF, -INF
+    got = _run(x, w)
+    clean[rows] = got[rows] = 0.0
+    clean[:, cols] = got[:, cols] = 0.0
+    assert torch.equal(got, clean)
+
+
+def test_single_products_are_rounded_once(dev):
+    """Sums of so few products are taken by the fp32 instructions: one product alone is the fp32 product."""
+    from fastfold_amd import _lib
+    g = torch.Generator().manual_seed(3)
+    x, w = torch.zeros(300, 4), torch.zeros(200, 4)
+    x[:, 2], w[:, 2] = torch.randn(300, generator=g), torch.randn(200, generator=g)
+    assert torch.equal(_run(x.to(dev), w.to(dev)).float().cpu(), x[:, 2, None] * w[None, :, 2])
+    for M in (1, 2):
+        y, x = torch.randn(M, 136, generator=g), torch.randn(M, 40, generator=g)
+        y[1:], x[1:] = 0.0, 0.0
+        ws, out, cs = torch.empty(136 * 41, device=dev), torch.empty(136, 40, device=dev), torch.empty(136, device=dev)
+        _lib.weight_grad(out, cs, ws, y.to(dev), x.to(dev), M=M, N=136, K=40, slices=1, dtype=torch.float32, y_map=(M, 0, 136), x_map=(M, 0, 40))
+        assert torch.equal(out.cpu(), y[0, :, None] * x[0, None]) and torch.equal(cs.cpu(), y[0])
+
+
 @pytest.mark.parametrize("M,K,N", [(40, 2048, 100), (700, 4096, 300), (4000, 4112, 2100), (64, 16384, 40)])
 def test_long_sums_of_one_sign(dev, M, K, N):
     """What the instructions cut off has the sign of the sum: pieces of 256 with turned signs keep it from adding up."""
@@ -110,8 +140,12 @@ def test_error_of_weight_gradients(dev, M, slices, one_sign):
     walk = (max(M / slices, 256) / 256 + slices / 4 + 3) ** 0.5 * 2.0 ** -24 + 2.0 ** -23
     assert rel(got, want) <= (walk if one_sign else 16 * 2.0 ** -24 + walk)       # of both signs: a piece's roundings against a sum that stays small
     assert rel(cs.double(), y.double().sum(0)) <= (M / slices + slices) ** 0.5 * 2.0 ** -24
+    clean = got
     y[M // 2, 5], x[M // 3, 7], x[0, 9] = INF, -INF, float("nan")
     got, want = run()
+    keep = torch.ones_like(clean, dtype=torch.bool)
+    keep[5], keep[:, 7], keep[:, 9] = False, False, False
+    assert torch.equal(got[keep], clean[keep])                # the other sums keep their bits
     fin = want.isfinite()
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[want.isinf()], want[want.isinf()])
     assert rel(got[fin], want[fin]) <= (M / slices + slices) ** 0.5 * 2.0 ** -24
