@@ -470,7 +470,8 @@ constexpr int PAIR_THREADS = 256;
 // identity once for both rows: its accumulator is the C operand of their scores (five products per tile, not six), which leaves no
 // place for a row's reference, so the reference is zero.  Sums of exp2 within OPT_LOW .. OPT_HIGH prove that no probability over- or
 // underflowed, weighted sums that are numbers and, where the row's sum is below one, not all below OUT_LOW that no product with v did
-// (large v beside a large sum, small v beside a small one); a workgroup without that proof walks again with a running maximum.
+// (large v beside a large sum, small v beside a small one); a workgroup with queries that lack that proof walks again with a running
+// maximum, for them alone.
 // Before -> after, us: 64 rows x 4 heads of 4 096 queries 888 -> 780, 1 024 x 4 of 1 024 984 -> 920, 391 x 4 of 391 99 -> 94, 320 x 4 of 320
 // 53.0 -> 49.0.  Of the 190 ns a tile takes at 4 096 queries its instructions take 148, LDS 14, the barrier 7 and
 // the ring's requests the rest.  Without a bias (212 -> 213 us, 128 x 8 of 1 024) the kernel above stays.  Workgroup = 2 batch rows x 4
@@ -756,7 +757,7 @@ __global__ __launch_bounds__(PAIR_THREADS, 2) void attention_pair_kernel(
     float l_tot[2];
     {
         int* redo = reinterpret_cast<int*>(lds + NSLOT * NTILES * 1024);
-        bool bad = false;
+        bool bad = false, again[2];               // some query of the wave, this lane's query: to be walked again
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
             l_tot[r] = l_run[r] + lane_xor<32>(l_run[r]);
@@ -768,10 +769,14 @@ __global__ __launch_bounds__(PAIR_THREADS, 2) void attention_pair_kernel(
             }
             const bool sound = l_tot[r] <= OPT_HIGH && l_tot[r] >= OPT_LOW && big < 0x7F800000u && (l_tot[r] >= 1.0f || big >= OUT_LOW);
             const bool out_of_range = live[r] && q < Nq && !sound;
-            if (__builtin_amdgcn_ballot_w64(out_of_range) != 0) {
+            unsigned long long which = __builtin_amdgcn_ballot_w64(out_of_range);
+            which |= which >> 32 | which << 32;   // both halves of a query
+            again[r] = false;
+            if (which != 0) {
                 bool any = false;                 // a row without keys has a sum of zero, and zeros for its result
                 for (int kt = 0; kt < KT; ++kt) any = any || (r ? fl1 : fl0)[kt] != 2;
                 bad = bad || any;
+                again[r] = any && (which >> lane & 1);
             }
         }
         if (tid == 0) *redo = 0;
@@ -779,10 +784,15 @@ __global__ __launch_bounds__(PAIR_THREADS, 2) void attention_pair_kernel(
         if (bad && lane == 0) *redo = 1;
         lds_barrier();
         if (*redo != 0) {                         // workgroup-uniform
+            // What the first walk has proven is kept, in the ring's other slots: a query's bits are its own
+            f32x4* const kept = reinterpret_cast<f32x4*>(lds + NTILES * 1024) + tid;
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
                 l_run[r] = 0.0f;
                 ref[r] = REF_FLOOR;
+#pragma unroll
+                for (int a = 0; a < 4; ++a)
+                    kept[(4 * r + a) * PAIR_THREADS] = f32x4{o_acc[r][4 * a], o_acc[r][4 * a + 1], o_acc[r][4 * a + 2], o_acc[r][4 * a + 3]};
 #pragma unroll
                 for (int v = 0; v < 16; ++v) o_acc[r][v] = 0.0f;
             }
@@ -819,7 +829,16 @@ __global__ __launch_bounds__(PAIR_THREADS, 2) void attention_pair_kernel(
                 }
             }
 #pragma unroll
-            for (int r = 0; r < 2; ++r) l_tot[r] = l_run[r] + lane_xor<32>(l_run[r]);
+            for (int r = 0; r < 2; ++r) {
+                const float l = l_run[r] + lane_xor<32>(l_run[r]);
+                l_tot[r] = again[r] ? l : l_tot[r];
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    const f32x4 k = kept[(4 * r + a) * PAIR_THREADS];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o_acc[r][4 * a + e] = again[r] ? o_acc[r][4 * a + e] : k[e];
+                }
+            }
         }
     }
 

@@ -59,6 +59,38 @@ def test_values_far_from_one(dev, shift, v_scale):
     _case(dev, 3, 2, 300, shift, None, v_scale)
 
 
+def test_a_second_walk_changes_the_queries_that_need_it_only(dev):
+    """Scores out of range in some queries and values too large for another batch row's sums: everyone else's bits stay."""
+    from fastfold_amd import _lib
+    from fastfold_amd.model.fastnn.kernel import layouts
+    g = torch.Generator().manual_seed(11)
+    B2, H, N = 4, 2, 300
+    q, k, v = (torch.randn(B2, H, N, 32, generator=g).to(BF).to(dev) for _ in range(3))
+    bias = (torch.randn(H, N, N, generator=g) * 2).to(BF).to(dev)
+    kb, fl = torch.empty(B2, layouts.n_tiles(N) * 32, device=dev), torch.empty(B2, layouts.n_tiles(N), dtype=torch.int32, device=dev)
+    _lib.key_bias(kb, fl, None, B=B2, N=N)
+
+    def run(v, bias):
+        out = torch.empty(B2, N, H, 32, dtype=BF, device=dev)
+        _lib.attention_fwd(out, layouts.tile_qk(q), layouts.tile_qk(k), layouts.tile_v(v), layouts.tile_bias(bias), kb, fl, None, B2=B2, H=H,
+                           Nq=N, Nk=N)
+        torch.cuda.synchronize()
+        return out
+    far = torch.zeros(N, dtype=torch.bool, device=dev)
+    far[[5, 40, 41, 131, 299]] = True
+    bias[:, far] = (bias[:, far] / 4).round() * 4               # 512 more or less of them is exact
+    first, v2, bias2 = run(v, bias), v.clone(), bias.clone()
+    bias2[0, far] = bias2[0, far] + 512.0
+    v2[3, 1] = v2[3, 1] * 2.0 ** 124                            # sums of a few hundred such values overflow
+    second = run(v2, bias2)
+    assert torch.equal(second[:, ~far, 0], first[:, ~far, 0]) and torch.equal(second[:3, :, 1], first[:3, :, 1])
+    # ... and those that were walked again are right: softmax takes no notice of what is added to a whole row
+    near = second[:, far, 0].float() - first[:, far, 0].float()
+    # (probabilities and results rounded to bf16 on either side, scores of 512 to 2^-14)
+    assert float(near.norm()) <= (2 * 2.0 ** -8 + 2.0 ** -13) * float(first[:, far, 0].float().norm())
+    assert bool(second.isfinite().all())
+
+
 @pytest.mark.parametrize("N", [270, 400])
 def test_masks(dev, N):
     g = torch.Generator().manual_seed(N)
