@@ -308,6 +308,61 @@ def test_attention_slabs_really_iterate(dev, tiny_budget, monkeypatch):
     assert len(calls) >= 3 and sum(calls) == 88 and calls[-1] != calls[0], calls
 
 
+def test_chunked_block_of_long_rows_equals_unchunked(dev, tiny_budget, monkeypatch):
+    """The same in bf16 at extents whose attentions have slabs (rows of more than 256 tokens, columns of more than 128): shorter ones are
+    one kernel, without scratch to bound.  The core's launches show that each of the four attentions is cut."""
+    from fastfold_amd import _lib
+    _, fast = _models(87, 1, dev, fan_in_scaled=True)
+    args = [_t(a, dev) for a in synth_inputs(87, 160, 288, mask_tail_frac=0.1)]
+    cores, real = [], _lib.attention_fwd
+    monkeypatch.setattr(_lib, "attention_fwd", lambda *a, **k: (cores.append((k["H"], k["Nq"], k["B2"])), real(*a, **k))[1])
+    whole, pieces = _run_both(lambda: fast.evoformer(*args, chunk_size=None))
+    for name, a, b in zip("mzs", whole, pieces):
+        assert torch.equal(a, b), name
+    for H, N, rows, calls in ((8, 288, 160, 1), (8, 160, 288, 1), (4, 288, 288, 2)):
+        b2 = [b for h, n, b in cores if (h, n) == (H, N)]
+        assert b2[:calls] == [rows] * calls and sum(b2[calls:]) == calls * rows and max(b2[calls:]) < rows // 3, (H, N, b2)
+
+
+@pytest.mark.parametrize("r", [160, 256])
+@pytest.mark.parametrize("dropout", [False, True])
+def test_slabs_of_row_attention_up_to_256_residues(dev, r, dropout, tiny_budget, monkeypatch):
+    """MSA row attention in one kernel up to the gated heads (ffk_attention_heads) and the output stage behind it: a few sequences at a
+    time - shifted rows, masks and tile flags - against all of them bit by bit, in place and not, with and without dropout
+    multipliers, and against launches of their own."""
+    from fastfold_amd import _lib
+    from fastfold_amd.model.fastnn import _fused
+    from fastfold_amd.model.fastnn.msa import MSARowAttentionWithPairBias
+    torch.manual_seed(r)
+    s, C = 37, 256
+    mod = MSARowAttentionWithPairBias(C, 128, c=32, n_head=8)
+    with torch.no_grad():
+        for n, p in mod.named_parameters():
+            p.copy_(1 + 0.1 * torch.randn_like(p) if "layernorm" in n and n.endswith("weight")
+                    else torch.randn_like(p) * (0.3 if p.dim() == 1 else p.shape[-1] ** -0.5))
+    mod = mod.to(dev, torch.bfloat16).eval()
+    m, z = torch.randn(1, s, r, C, device=dev).bfloat16(), torch.randn(1, r, r, 128, device=dev).bfloat16()
+    mask = (torch.rand(1, s, r, device=dev) > 0.3).bfloat16()          # another mask in every row
+    mask[:, 5], mask[:, 30, 40:] = 0, 0
+    drop = (torch.rand(1, 1, r, C, device=dev) > 0.25).bfloat16() / 0.75 if dropout else None
+    rows, real = [], _lib.attention_heads
+    monkeypatch.setattr(_lib, "attention_heads", lambda *a, **k: (rows.append(k["B2"]), real(*a, **k))[1])
+    whole, pieces = _run_both(lambda: mod._run(m, z, mask, torch.empty_like(m), drop=drop))
+    assert torch.equal(whole, pieces) and rows[0] == s and len(rows) > 4 and sum(rows[1:]) == s and rows[-1] != rows[1], rows
+    x = m.clone()
+    with torch.no_grad():
+        mod._run(x, z, mask, x, drop=drop)                             # in place, in slabs
+    assert torch.equal(x, whole)
+    monkeypatch.setattr(_fused, "_ATTENTION_BLOCK", False)
+    apart = _run_both(lambda: mod._run(m, z, mask, torch.empty_like(m), drop=drop))
+    assert torch.equal(*apart)
+    live = [i for i in range(s) if i != 5]
+    upd = (apart[0] - m).float()[:, live]
+    # six roundings to bf16 on either side, and that of the sum with the residual
+    assert float((whole - apart[0]).float()[:, live].norm()) <= 12 * 2.0 ** -9 * float(upd.norm()) + 2.0 ** -8 * float(m.float().norm())
+    assert float(upd.norm()) > 1.0
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_chunked_extra_msa_block_equals_unchunked(dev, dtype, tiny_budget, monkeypatch):
     """Extra-MSA block: the gate / output projection of the global column attention (20 or 10 of 72 sequences at a
