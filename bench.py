@@ -5,7 +5,7 @@
 One step = one forward pass of the 48-block Evoformer stack (bf16, N_seq=128, random-init
 weights ~N(0, 0.02^2), inputs ~N(0,1)) with inputs and weights resident in HBM.  The metric is
 the Evoformer-block latency (ms per block = step time / 48).  The same JSON line carries
-  roofline      the dominant kernel (flash attention core with bias: triangle + MSA-row attention),
+  roofline      the dominant kernel (attention with bias: triangle + MSA-row, by the kernel its launches took),
                 algorithmic FLOPs / HIP-event time of its launches inside the timed region,
   cpu_baseline  the CPU oracle (plain-PyTorch restatement of the reference's nn Evoformer block)
                 timed on this box's host cores on a bounded sample,
@@ -378,35 +378,50 @@ def main():
     torch.cuda.synchronize()
     # HIP events bracket every attention launch of the first timed step only: an event pair costs the
     # stream about 10 us per launch, which the other steps do not have to carry
-    rec = _lib.time_kernel("ffk_attention_fwd")
-    others = {name: _lib.time_kernel(name) for name in ("ffk_bgemm_nt", "ffk_transition_fused", "ffk_transition_block", "ffk_opm_fused")}
+    # (which entry points the biased attentions go to is a matter of their length)
+    attention = ("ffk_attention_fwd",) if r > 256 else ("ffk_attention_fwd", "ffk_attention_block", "ffk_attention_heads")
+    others = {name: _lib.time_kernel(name) for name in attention + ("ffk_bgemm_nt", "ffk_transition_fused", "ffk_transition_block",
+                                                                    "ffk_opm_fused")}
     t0 = time.perf_counter()
     for i in range(args.steps):
         out = step()
         if i == 0:
-            _lib.time_kernel("ffk_attention_fwd", enable=False)
             for name in others:
                 _lib.time_kernel(name, enable=False)
     torch.cuda.synchronize()
     ms_per_step = (time.perf_counter() - t0) * 1e3 / args.steps
     assert all(bool(torch.isfinite(t.float()).all()) for t in out), "non-finite output"
 
-    # dominant kernel: attention core launches that carry a bias (MSA row + triangle start/end)
-    flops, ms, n = 0.0, 0.0, 0
-    for e0, e1, a in rec:
-        if a[4] is None:       # bias_t == NULL: column attention (other kernel instantiation)
-            continue
-        B2, H, Nq, Nk = a[8], a[9], a[10], a[11]
-        flops += 4.0 * B2 * H * Nq * Nk * 32
-        ms += e0.elapsed_time(e1)
-        n += 1
-    ach = flops / (ms * 1e-3) / 1e12 if ms > 0 else 0.0
-    roofline = {"bound": "mfma", "kernel": "attention_pair_kernel (ffk_attention_fwd, bf16, bias)",
-                "achieved": round(ach, 2), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
-                "frac": round(ach / PEAK_BF16_TFLOPS, 4), "traffic": attention_traffic(wl["traffic_profile"]),
-                "traffic_unit": "bytes/launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, see profiles/)",
-                "launches": n, "avg_launch_ms": round(ms / max(n, 1), 4),
-                "flops_per_launch_avg": round(flops / max(n, 1) / 1e9, 2)}
+    # dominant kernel: of the kernels that attentions with a bias went to (MSA row + triangle start/end), the one with most time.
+    # Algorithmic flops: scores and weighted sum; where a launch makes its operands itself, its projections too.
+    def attention_kind(name, a):
+        if name == "ffk_attention_fwd":
+            if a[4] is None:       # bias_t == NULL: column attention (other kernel instantiation)
+                return None
+            B2, H, Nq, Nk = a[8], a[9], a[10], a[11]
+            return "%s (%s, bf16, bias)" % ("attention_pair_kernel" if Nk > 256 else "attention_kernel", name), 4.0 * B2 * H * Nq * Nk * 32
+        bias, (B2, N, C) = (a[8], a[12:15]) if name == "ffk_attention_block" else (a[6], a[9:12])
+        if bias is None:
+            return None
+        return "%s (bf16, bias)" % name, 4.0 * B2 * N * N * C + 2.0 * B2 * N * C * C * (5 if name == "ffk_attention_block" else 4)
+    cores = {}
+    for name in attention:
+        for e0, e1, a in others[name]:
+            kind = attention_kind(name, a)
+            if kind is not None:
+                t = cores.setdefault(kind[0], [0, 0.0, 0.0])
+                t[0] += 1
+                t[1] += e0.elapsed_time(e1)
+                t[2] += kind[1]
+    roofline = None
+    if cores:
+        name, (n, ms, flops) = max(cores.items(), key=lambda kv: kv[1][1])
+        ach = flops / (ms * 1e-3) / 1e12
+        roofline = {"bound": "mfma", "kernel": name, "achieved": round(ach, 2), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
+                    "frac": round(ach / PEAK_BF16_TFLOPS, 4),
+                    "traffic": attention_traffic(wl["traffic_profile"]) if name.startswith("attention_pair_kernel") else None,
+                    "traffic_unit": "bytes/launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, see profiles/)",
+                    "launches": n, "avg_launch_ms": round(ms / n, 4), "flops_per_launch_avg": round(flops / n / 1e9, 2)}
 
     # the other matrix-pipe kernels of the block, timed the same way (HIP events around their launches in the
     # first timed step): algorithmic flops of the launch / its duration, against the dense bf16 peak
@@ -445,9 +460,10 @@ def main():
                    "block_gflop": round(block_gflop(s, r), 1),
                    "stack_tflops": round(block_gflop(s, r) * args.blocks / ms_per_step, 1),
                    "residual_stream": "bf16" if args.plain_residual else "bf16 + int8 tail (24-bit)"},
-        "roofline": roofline,
         "kernels": kernels,
     }
+    if roofline is not None:
+        line["roofline"] = roofline
     if args.workload == "cfg4" and not args.no_micro:
         # the same stack at benchmark configuration 3 (N_res = 256), reported beside the headline number
         w3 = WORKLOADS["cfg3"]
