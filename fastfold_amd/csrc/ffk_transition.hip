@@ -254,6 +254,8 @@ __global__ __launch_bounds__(TR_THREADS, NS == 4 ? 1 : 3) void transition_fused_
     }
 }
 
+// (Modules: 128 channels from 16 385 to 32 768 rows.  256 channels and fewer rows of 128 are theirs in ffk_transition_block, with weights
+// in fragment order; here they serve callers with plain weights.)
 // The same computation, to the bit, with the two layers on different waves and 64 rows per wave: every launch of 256 channels, and
 // those of 128 that leave a CU at most two workgroups.  A fragment of the weights read from LDS feeds two products instead of one:
 // with 32 rows per wave the four SIMDs ask LDS for a kilobyte per product each, which is all it delivers.  A workgroup has RP row

@@ -179,7 +179,8 @@ extern "C" int ffk_transition_block(void* out, const void* x, void* xtail, const
     const TbArgs a = {{(T*)out, (const T*)x, (int8_t*)xtail, (const T*)gamma, (const T*)beta, nullptr, (long)C, 0, eps},
                       (const T*)w1, (const T*)b1, (const T*)w2, (const T*)b2, (long)M};
     hipStream_t st = (hipStream_t)stream;
-    // 64 rows a workgroup as long as every one has a CU, 128 from there on (fewer weights per row)
+    // 64 rows a workgroup as long as every one has a CU, 128 from there on (fewer weights per row).  The modules send more than 16 384 rows
+    // of 128 channels to ffk_transition_fused (figures above); a caller that holds only these weights is served as well
     if (C == 256) return M <= 64 * 256 ? tb_launch<256, 4, 2, 2>(a, st) : tb_launch<256, 4, 4, 2>(a, st);
     if (C == 128) return M <= 64 * 256 ? tb_launch<128, 4, 2, 2>(a, st) : tb_launch<128, 4, 4, 2>(a, st);
     return hidden == 256 ? tb_launch<64, 4, 4, 2>(a, st) : tb_launch<64, 2, 4, 4>(a, st);

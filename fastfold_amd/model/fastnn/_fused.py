@@ -233,7 +233,8 @@ def transition(x, out, *, ln, w1_pk, b1_pk, w2, b2, hidden, budget, xtail=None, 
         _lib.transition_block(out, x, ln[0], ln[1], w_block[0], b1_pk, w_block[1], b2, M=M, C=C, hidden=hidden, xtail=xtail)
         return out
     if dt == torch.bfloat16 and C in (128, 256) and hidden == 4 * C and ln is not None and _FUSED_TRANSITION:
-        # both layers in one kernel, hidden activation kept on chip
+        # both layers in one kernel, hidden activation kept on chip: many rows of 128 channels (256: ffk_transition_block takes all but
+        # parameters that are not aligned, which this kernel does not take either)
         _lib.transition_fused(out, x, ln[0], ln[1], w1_pk, b1_pk, w2, b2, M=M, C=C, hidden=hidden, xtail=xtail)
         return out
     rows = max(128, min(M, (budget // (hidden * es)) // 128 * 128))
