@@ -222,14 +222,18 @@ def transition_block_rows(C):
     return 16384 if C == 128 else 1 << 36
 
 
+def transition_takes_block(M, C, w_block, ln, b2):
+    return w_block is not None and ln is not None and _FUSED_TRANSITION and M <= transition_block_rows(C) and aligned16(*ln, b2)
+
+
 def transition(x, out, *, ln, w1_pk, b1_pk, w2, b2, hidden, budget, xtail=None, w_block=None):
     """out = x + W2 relu(W1 LN(x) + b1) + b2 over rows of x [M, C]; out may alias x.  ``w_block``: the weights as
-    ``pack_transition_block`` lays them out, or None.  ``xtail`` (here and in the
+    ``pack_transition_block`` lays them out, or None; ``w1_pk`` is needed where ``transition_takes_block`` is false.  ``xtail`` (here and in the
     other sub-modules): int8 tensor of x's shape holding the tail bytes of x / out as an extended residual stream."""
     M, C = x.shape
     dt, dev = x.dtype, x.device
     es = es_of(dt)
-    if w_block is not None and ln is not None and _FUSED_TRANSITION and M <= transition_block_rows(C) and aligned16(*ln, b2):
+    if transition_takes_block(M, C, w_block, ln, b2):
         _lib.transition_block(out, x, ln[0], ln[1], w_block[0], b1_pk, w_block[1], b2, M=M, C=C, hidden=hidden, xtail=xtail)
         return out
     if dt == torch.bfloat16 and C in (128, 256) and hidden == 4 * C and ln is not None and _FUSED_TRANSITION:

@@ -411,13 +411,17 @@ class Transition(nn.Module, _PackMixin):
         hidden = self.linear1.out_features
         if not F_.fits_fused(d, dt) or hidden % 128 != 0:
             raise RuntimeError("Transition: unsupported width %d" % d)
-        w1, b1, w2, b2, w_block = self._packed(("tr", dt, dev), [self.linear1.weight, self.linear1.bias,
-                                                                self.linear2.weight, self.linear2.bias], lambda: (
-            F_.pack_rows([self.linear1.weight], dt, dev), F_.pack_vec([self.linear1.bias], dt, dev),
+        b1, w2, b2, w_block = self._packed(("tr", dt, dev), [self.linear1.weight, self.linear1.bias,
+                                                            self.linear2.weight, self.linear2.bias], lambda: (
+            F_.pack_vec([self.linear1.bias], dt, dev),
             self.linear2.weight.detach().to(dt).contiguous(), self.linear2.bias.detach().to(dt).contiguous(),
             F_.pack_transition_block(self.linear1.weight, self.linear2.weight, dt, dev)))
+        ln = _ln_pair(self.norm, dt)
+        w1 = None                # row by row only where some number of rows goes to a kernel that reads it so
+        if not F_.transition_takes_block(1 << 35, d, w_block, ln, b2):
+            w1 = self._packed(("tr1", dt, dev), [self.linear1.weight], lambda: F_.pack_rows([self.linear1.weight], dt, dev))
         x = src.view(-1, d)
-        F_.transition(x, out.view(-1, d), ln=_ln_pair(self.norm, dt), w1_pk=w1, b1_pk=b1, w2=w2, b2=b2,
+        F_.transition(x, out.view(-1, d), ln=ln, w1_pk=w1, b1_pk=b1, w2=w2, b2=b2,
                       hidden=hidden, budget=_budget(), xtail=_check_tail(xtail, src), w_block=w_block)
         return out
 
