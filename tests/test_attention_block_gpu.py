@@ -266,3 +266,56 @@ def test_weights_of_short_rows_are_laid_out_with_the_others(dev):
             before = _plan.builds
             out = att(z, torch.ones(1, r, r, device=dev, dtype=BF))
             assert bool(out.isfinite().all()) and (i == 0 or _plan.builds == before)
+
+
+def test_modules_with_normalisation_weights_anywhere(dev):
+    """LayerNorm parameters that are slices of a flat buffer, not on 16 bytes: the same update by the launches that take them (six
+    roundings of 2^-9 on either side; a transition has three)."""
+    from fastfold_amd.model.fastnn.kernel import LayerNorm
+    from fastfold_amd.model.fastnn.ops import Transition
+    torch.manual_seed(5)
+    cases = list(_modules(dev)) + [(Transition(64), (torch.randn(1, 40, 96, 64, device=dev).to(BF),))]
+    for mod, args in cases:
+        with torch.no_grad():
+            for n, p in mod.named_parameters():
+                p.copy_(1 + 0.1 * torch.randn_like(p) if "norm" in n and n.endswith("weight")
+                        else torch.randn_like(p) * (0.3 if p.dim() == 1 else p.shape[-1] ** -0.5))
+        mod = mod.to(dev, BF).eval()
+        outs = []
+        for shift in (0, 1):
+            for m in mod.modules():
+                if isinstance(m, LayerNorm) and shift:
+                    for p in (m.weight, m.bias):
+                        flat = torch.zeros(p.numel() + 8, device=dev, dtype=BF)
+                        flat[1:p.numel() + 1] = p.detach()
+                        p.data = flat[1:p.numel() + 1]
+            with torch.no_grad():
+                outs.append(mod(*args).float())
+        upd = outs[0] - args[0].float()
+        assert float((outs[0] - outs[1]).norm() / upd.norm()) < 2 * TOL, (type(mod).__name__, args[0].shape)
+
+
+@pytest.mark.parametrize("r", [32, 96, 128])
+def test_triangle_attention_of_256_channels(dev, r):
+    """Its pair bias is made by no kernel of 64 or 128 channels: launches of their own, against float64."""
+    from fastfold_amd.model.fastnn.ops import ChunkTriangleAttentionStartingNode
+    torch.manual_seed(r)
+    mod = ChunkTriangleAttentionStartingNode(256, 0.25, c=32, n_head=8)
+    with torch.no_grad():
+        for n, p in mod.named_parameters():
+            p.copy_(1 + 0.1 * torch.randn_like(p) if "norm" in n and n.endswith("weight")
+                    else torch.randn_like(p) * (0.3 if p.dim() == 1 else p.shape[-1] ** -0.5))
+    mod = mod.to(dev, BF).eval()
+    z = torch.randn(1, r, r, 256, device=dev).to(BF)
+    with torch.no_grad():
+        got = mod(z, torch.ones(1, r, r, device=dev, dtype=BF)).double().cpu()
+    d = lambda t: t.detach().double().cpu()                   # noqa: E731
+    x = d(z)[0]
+    y = torch.nn.functional.layer_norm(x, (256,), d(mod.layernorm1.weight), d(mod.layernorm1.bias))
+    a = mod.attention
+    q, k, v = (t.view(r, r, 8, 32).transpose(1, 2) for t in (y @ d(a.to_qkv.weight).t()).split(256, -1))
+    s = q * 32 ** -0.5 @ k.transpose(-1, -2) + (y @ d(mod.linear_b.weight).t()).permute(2, 0, 1)
+    o = (torch.softmax(s, -1) @ v).transpose(1, 2).reshape(r, r, 256)
+    upd = (torch.sigmoid(y @ d(a.gating_linear.weight).t() + d(a.gating_bias)) * o) @ d(a.o_linear.weight).t() + d(mod.out_bias)
+    # seven roundings of the update (y among them) and that of the result
+    assert float((got[0] - x - upd).norm()) < 7 * 2.0 ** -9 * float(upd.norm()) + 2.0 ** -9 * float((x + upd).norm())
