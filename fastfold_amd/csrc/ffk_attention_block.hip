@@ -6,7 +6,7 @@
 // is fetched once for several products: with a wave per token tile, every wave fetching all the weights, the projections of 256 rows of
 // 128 tokens at 256 channels took 42 us of a launch of 86, as many bytes out of the second-level cache as it delivers.  The phases:
 //   rows -> LayerNorm -> LDS;  barrier
-//   q, k, v and the gate of the wave's tiles, packed as the MFMA operands they are next, in registers
+//   q, k, v and the gate of the wave's tiles in registers, packed as the MFMA operands they are next (the gate of 128 channels in fp32)
 //   attention over the key tiles (k, v of all tokens in LDS, or in registers where one wave has all of a head's)
 //   gated outputs -> LDS;  barrier;  output projection, a wave 32 output channels;  updates -> LDS;  barrier;  rows updated
 // Nothing is transposed on the way: the accumulator of Wk y^T is the score product's A operand as it stands, that of Wq y^T its B
@@ -29,8 +29,8 @@
 //                            with a pair bias:  128 rows of 96 tokens 45 -> 29, of 128 tokens 51 -> 36
 //   the same to the gated heads, output projection apart (k and v of four heads of 256 tokens fill the LDS: two workgroups to a row):
 //                            128 rows of 160 tokens 67 -> 49, 192 74 -> 53, 256 87 -> 72;  512 rows of 256 296 -> 228
-// Other numbers of rows: attention_block_tokens in model/fastnn/_fused.py.  Longer rows do not fit: at 128 channels, k and v of more than 256 tokens go into LDS in two passes only (heads two by two, rows
-// normalised twice), which was built and is slower (288 tokens 122 us against 92, 416 235 against 189).
+// Other numbers of rows: attention_block_tokens in model/fastnn/_fused.py.  Longer rows do not fit: at 128 channels, k and v of more than
+// 256 tokens go into LDS in two passes only (heads two by two, rows normalised twice), which was built and is slower (288 tokens 122 us against 92, 416 235 against 189).
 #include "ffk_rowblock.h"
 #include <type_traits>
 
